@@ -67,16 +67,29 @@ const char* mi355_moe_last_error(void);
  * llmtuner/models/common/linear.py:107-131,179-183.
  * x: (T,D) x_dtype row-major; w: (E,D) w_dtype; logit_bias: (E) fp32 or NULL.
  * workspace: mi355_router_gate_fwd_workspace_bytes(T,D,E) bytes (for the same T, D, E)
- * or NULL.  With a workspace, bf16 x, fp32 w and D, E multiples of 64, each fp32 weight
- * is written as three bf16 pieces (24 mantissa bits) and the product runs as three bf16
- * MFMAs with fp32 accumulation (from 1024 tokens on in 128-token tiles with the
- * contraction split over workgroups, partial sums added in a fixed order); otherwise the
- * strided fp32-MFMA kernel is used.
+ * or NULL.  With a workspace and 16-byte aligned operands: for fp32 w, bf16 x with D % 8 == 0 takes
+ * each fp32 weight as three bf16 pieces (24 mantissa bits) and runs the product as three bf16
+ * MFMAs with fp32 accumulation, fp32 x with D % 4 == 0 runs on fp32 MFMAs; the contraction is
+ * split over waves and workgroups, partial sums added in a fixed order.  Otherwise the strided
+ * fp32-MFMA kernel is used.
  */
 int64_t mi355_router_gate_fwd_workspace_bytes(int64_t T, int64_t D, int64_t E);
 int mi355_router_gate_fwd(const void* x, int x_dtype, const void* w, int w_dtype,
                           const float* logit_bias, float* logits_TE, void* workspace,
                           int64_t T, int64_t D, int64_t E, void* stream);
+
+/*
+ * The same product left as `splits` (T,E) partial sums, for a consumer that adds them itself
+ * (mi355_route_plan): mi355_router_gate_fwd_splits is their number, 0 where this form does not
+ * exist.  logit_bias goes in here when splits is 1 and is the consumer's to add otherwise.
+ * pieces: scratch of mi355_router_gate_fwd_pieces_bytes (NULL if that is 0); it holds the
+ * weight pieces afterwards and may be handed to mi355_router_gate_add_bwd.
+ */
+int mi355_router_gate_fwd_splits(int x_dtype, int w_dtype, int64_t T, int64_t D, int64_t E);
+int64_t mi355_router_gate_fwd_pieces_bytes(int x_dtype, int w_dtype, int64_t T, int64_t D, int64_t E);
+int mi355_router_gate_fwd_partial(const void* x, int x_dtype, const float* w, const float* logit_bias,
+                                  float* partial, void* pieces, int64_t T, int64_t D, int64_t E,
+                                  void* stream);
 
 /*
  * dx[t][d] = sum_e dlogits[t][e] * w[e][d]   (written in x_dtype; NULL = skip)
@@ -91,6 +104,12 @@ int mi355_router_gate_bwd(const float* dlogits_TE, const void* x, int x_dtype,
                           const void* w, int w_dtype, void* dx, void* dw,
                           void* workspace, int64_t T, int64_t D, int64_t E,
                           void* stream);
+/* The same with dx = (the gradient above, rounded to x_dtype) + addend (T,D, x_dtype, or NULL): what
+ * adding two tensors of that type gives.  pieces: the forward's weight pieces, or NULL. */
+int mi355_router_gate_add_bwd(const float* dlogits_TE, const void* x, int x_dtype,
+                              const void* w, int w_dtype, const void* pieces, const void* addend,
+                              void* dx, void* dw, void* workspace, int64_t T, int64_t D, int64_t E,
+                              void* stream);
 
 /*
  * Scores, expert choice, gather, norm and scale in one pass over the logits.
@@ -168,6 +187,13 @@ int mi355_router_select_bwd(const float* logits_TE, const int64_t* ids_TK,
                             float* dlogits_TE, int64_t T, int64_t E, int64_t K,
                             int score_func, int route_norm, float route_scale,
                             int select_mode, void* stream);
+/* The same for a plain top-k whose weights' gradient is still in pieces, as
+ * mi355_grouped_swiglu_combine_bwd leaves it: dweights[slot] = sum_i dot_partial[row_of_slot[slot]][i]. */
+int mi355_router_select_dots_bwd(const float* logits_TE, const int64_t* ids_TK, const float* dot_partial,
+                                 int64_t pieces, const int32_t* row_of_slot, int64_t row_capacity,
+                                 float* dlogits_TE, int64_t T, int64_t E, int64_t K, int score_func,
+                                 int route_norm, float route_scale, void* stream);
+
 
 /*
  * Per-forward load-balance loss on the dense score map and the routing map:
@@ -280,6 +306,29 @@ int mi355_segments_from_counts(const int32_t* counts, int64_t El, int64_t tile_m
                                int64_t row_capacity, int32_t* seg_offsets, int32_t* seg_counts,
                                int32_t* tile_expert, int32_t* tile_row0,
                                int32_t* num_tiles, int64_t tile_capacity, void* stream);
+/* The same for one dense segment of `rows` rows, without a count on the device. */
+int mi355_segments_dense(int64_t rows, int64_t tile_m, int32_t* seg_offsets, int32_t* seg_counts,
+                         int32_t* tile_expert, int32_t* tile_row0, int32_t* num_tiles,
+                         int64_t tile_capacity, void* stream);
+
+/*
+ * mi355_router_select_fwd (plain or group-limited top-k) and mi355_permute_plan in one pass, same
+ * results: partial (splits,T,E) logits are added in order (plus logit_bias if splits > 1), the sums
+ * written to logits_TE unless NULL, and additionally row_scale[row] = weights[slot of row] (0 for
+ * padding rows; NULL = skip).  Covers E <= 256, K <= 16, groups that are whole runs of E/16 experts
+ * (mi355_route_plan_covers); workspace of mi355_route_plan_workspace_bytes, T >= 1.
+ */
+int mi355_route_plan_covers(int64_t E, int64_t K, int num_groups, int select_mode);
+int64_t mi355_route_plan_workspace_bytes(int64_t T, int64_t K, int64_t E);
+int mi355_route_plan(const float* partial, int splits, const float* logit_bias, float* logits_TE,
+                     const float* expert_bias, int64_t T, int64_t E, int64_t K, int score_func,
+                     int route_norm, float route_scale, int num_groups, int num_limited, float* weights_TK,
+                     int64_t* ids_TK, int64_t lo, int64_t hi, int64_t align, int64_t tile_m,
+                     int32_t* counts_E, int32_t* seg_offsets, int32_t* seg_counts, int32_t* row_of_slot,
+                     int32_t* slot_of_row, int32_t* token_of_row, float* row_scale, int64_t row_capacity,
+                     int32_t* tile_expert, int32_t* tile_row0, int32_t* num_tiles, int64_t tile_capacity,
+                     void* workspace, void* stream);
+
 
 /*
  * rows[row_of_slot[t*K+k]] = x[t] for every slot with a row (each token row is read once
@@ -302,6 +351,10 @@ int mi355_permute_rows_fwd(const void* x, int dtype, const int32_t* row_of_slot,
  */
 int mi355_permute_rows_bwd(const void* drows, int dtype, const int32_t* row_of_slot,
                            void* dx, int64_t T, int64_t D, int64_t K, void* stream);
+/* The same plus addend (T,D, dtype, or NULL; not for fp64): added to the rounded sum and rounded again. */
+int mi355_permute_rows_add_bwd(const void* drows, int dtype, const int32_t* row_of_slot, const void* addend,
+                               void* dx, int64_t T, int64_t D, int64_t K, void* stream);
+
 
 /* ------------------------------------------------------------------ combine */
 
@@ -318,6 +371,11 @@ int mi355_permute_rows_bwd(const void* drows, int dtype, const int32_t* row_of_s
 int mi355_combine_fwd(const void* y, int dtype, const float* weights_TK,
                       const int32_t* row_of_slot, void* out, int64_t T, int64_t D,
                       int64_t K, int round_terms, void* stream);
+/* The same plus addend (T,D, dtype, or NULL; not for fp64): added to the rounded sum and rounded again. */
+int mi355_combine_add_fwd(const void* y, int dtype, const float* weights_TK, const int32_t* row_of_slot,
+                          const void* addend, void* out, int64_t T, int64_t D, int64_t K, int round_terms,
+                          void* stream);
+
 
 /*
  * dy[row] = weights[t][k] * dout[t]   for every slot with a row (rows that hold

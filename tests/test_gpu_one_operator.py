@@ -1,0 +1,76 @@
+"""The block as one operator (csrc/torch_block.cpp) and the kernels only it uses, at the edges of their
+tiles: against the stage operators (a forward hook on the router makes the block visible in stages),
+bit for bit, and the gate projection against fp64."""
+
+import pytest
+import torch
+
+from oracle import moe_ref as R
+from tests.helpers import build_block, make_params
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("dtype,T,D,E,K,F,kw", [
+    (torch.bfloat16, 1, 384, 128, 8, 384, {}),
+    (torch.bfloat16, 63, 384, 256, 16, 448, dict(groups=(8, 4))),
+    (torch.bfloat16, 64, 512, 60, 6, 384, dict(dispatcher="padded", pad_multiple=16)),
+    (torch.bfloat16, 65, 512, 64, 5, 384, dict(bias=True)),
+    (torch.bfloat16, 1023, 448, 128, 2, 384, dict(dispatcher="share", local=(32, 80))),
+    (torch.bfloat16, 1025, 512, 128, 8, 384, dict(shared=448)),
+    (torch.bfloat16, 16449, 384, 64, 2, 384, {}),  # two chunks of tokens per workgroup
+    (torch.bfloat16, 200, 72, 17, 3, 100, dict(shared=60)),
+    (torch.float32, 65, 100, 5, 2, 92, dict(dispatcher="padded", pad_multiple=8, shared=64)),
+    (torch.float32, 1, 36, 1, 1, 40, {}),
+    (torch.float32, 129, 33, 12, 4, 31, dict(gate_bias=True)),
+])
+def test_one_operator_equals_the_stages_bit_for_bit(dtype, T, D, E, K, F, kw):
+    print(f"one operator {dtype} T={T} D={D} E={E} K={K} F={F} {kw}", flush=True)
+    kw = dict(kw)
+    groups, shared, bias, gate_bias = kw.pop("groups", None), kw.pop("shared", None), kw.pop("bias", False), kw.pop("gate_bias", False)
+    spec = R.RouterSpec(E, K, score_func="sigmoid" if bias or groups else "softmax", route_norm=True,
+                        num_expert_groups=groups and groups[0], num_limited_groups=groups and groups[1])
+    El = kw["local"][1] - kw["local"][0] if "local" in kw else None
+    p = make_params(E, D, F, dtype, seed=T, std=0.05, shared_F=shared, El=El)
+    if bias:
+        p.expert_bias_E = torch.linspace(-0.1, 0.1, E)
+    g = torch.Generator().manual_seed(T + 1)
+    x = torch.randn(T, D, generator=g).to(dtype).to(DEV)
+    gout = torch.randn(T, D, generator=g).to(dtype).to(DEV)
+
+    def run(in_stages):
+        block = build_block(p, spec, D, F, dtype, DEV, load_balance_coeff=1e-3 if bias else None, **kw)
+        if gate_bias:
+            block.router.gate.bias = torch.nn.Parameter(torch.linspace(-1, 1, E, device=DEV))
+        block.train()
+        block.overlap_shared_experts = not in_stages  # (one stream: the stages' order of the three input gradients)
+        if in_stages:
+            block.router.register_forward_hook(lambda *a: None)
+        whole = block._forward_as_one(x)
+        assert (whole is None) == in_stages
+        xin = x.clone().requires_grad_()
+        out = block(xin)
+        out.backward(gout)
+        with torch.no_grad():
+            plain = block.eval()(x)
+        return [out.detach(), plain, xin.grad, block.tokens_per_expert_E] + [q.grad for q in block.parameters()]
+
+    for i, (a, b) in enumerate(zip(run(True), run(False))):
+        assert torch.equal(a, b), f"tensor {i} differs by {float((a.float() - b.float()).abs().max())}"
+
+
+@pytest.mark.parametrize("dtype,T,D,E", [
+    (torch.bfloat16, 1, 8, 1), (torch.bfloat16, 33, 2056, 33), (torch.bfloat16, 1000, 7168, 256), (torch.bfloat16, 32, 1024, 66),
+    (torch.float32, 1, 4, 3), (torch.float32, 31, 1028, 32), (torch.float32, 2000, 640, 10), (torch.float32, 4, 3000, 5)])
+def test_gate_projection_of_few_tokens_matches_fp64(dtype, T, D, E):
+    from torchllmtuner_amd import ops
+
+    print(f"gate {dtype} T={T} D={D} E={E}", flush=True)
+    g = torch.Generator().manual_seed(D)
+    x, w, b = torch.randn(T, D, generator=g).to(dtype), torch.randn(E, D, generator=g) * 0.05, torch.randn(E, generator=g)
+    want = x.double() @ w.double().T + b.double()
+    got = ops.router_gate_fwd(x.to(DEV), w.to(DEV), b.to(DEV)).cpu().double()
+    # fp32 sums of D products: the error of a plain fp32 dot product bounds it
+    scale = (x.double().abs() @ w.double().abs().T + b.double().abs()).max()
+    assert float((got - want).abs().max()) < 4e-7 * float(scale)

@@ -44,11 +44,20 @@ __device__ __forceinline__ float round_to<float>(float v) { return v; }
 template <>
 __device__ __forceinline__ float round_to<uint16_t>(float v) { return round_bf16(v); }
 
+// a = round(a) + v
+template <typename T>
+__device__ __forceinline__ void plus(float (&a)[Vec<T>::N], const uint4& v) {
+  float f[Vec<T>::N];
+  Vec<T>::unpack(v, f);
+#pragma unroll
+  for (int q = 0; q < Vec<T>::N; ++q) a[q] = round_to<T>(a[q]) + f[q];
+}
+
 // SMALL_K: K <= 8, the eight-row chunk below is the only one
 template <typename T, bool SMALL_K>
 __global__ __launch_bounds__(256) void combine_fwd_kernel(
     const T* __restrict__ y, const float* __restrict__ weights,
-    const int32_t* __restrict__ row_of_slot, T* __restrict__ out, int T_, int D, int K,
+    const int32_t* __restrict__ row_of_slot, const T* __restrict__ addend, T* __restrict__ out, int T_, int D, int K,
     int round_terms) {
   const int lane = threadIdx.x & 63;
   const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -56,6 +65,9 @@ __global__ __launch_bounds__(256) void combine_fwd_kernel(
   const int64_t s0 = static_cast<int64_t>(t) * K;
   const int row = lane < K ? row_of_slot[s0 + lane] : -1;
   const float w = lane < K ? weights[s0 + lane] : 0.0f;
+  // addend (the shared expert's output): added to the rounded sum and rounded again, as the separate
+  // addition of two tensors of this type would be
+  const T* add = addend ? addend + static_cast<int64_t>(t) * D : nullptr;
   // ascending-row visiting order (index_add's order): position of each valid slot
   int pos = 0;
   for (int j = 0; j < K; ++j) {
@@ -119,7 +131,10 @@ __global__ __launch_bounds__(256) void combine_fwd_kernel(
           for (int j = 0; j < B; ++j)
             if (j < nvalid) add_terms(a, v[j][g], ww[j]);
           const int i = base + g * kWave + lane;
-          if (i < nv) reinterpret_cast<uint4*>(dst)[i] = Vec<T>::pack(a);
+          if (i < nv) {
+            if (add) plus<T>(a, reinterpret_cast<const uint4*>(add)[i]);
+            reinterpret_cast<uint4*>(dst)[i] = Vec<T>::pack(a);
+          }
         }
       } else {
         float a[G][V];
@@ -141,7 +156,10 @@ __global__ __launch_bounds__(256) void combine_fwd_kernel(
 #pragma unroll
         for (int g = 0; g < G; ++g) {
           const int i = base + g * kWave + lane;
-          if (i < nv) reinterpret_cast<uint4*>(dst)[i] = Vec<T>::pack(a[g]);
+          if (i < nv) {
+            if (add) plus<T>(a[g], reinterpret_cast<const uint4*>(add)[i]);
+            reinterpret_cast<uint4*>(dst)[i] = Vec<T>::pack(a[g]);
+          }
         }
       }
     }
@@ -157,7 +175,7 @@ __global__ __launch_bounds__(256) void combine_fwd_kernel(
         const float term = load_as_f32(y + static_cast<int64_t>(r) * D + i) * ww;
         a += round_terms ? round_to<T>(term) : term;
       }
-      if (on) store_from_f32(dst + i, a);
+      if (on) store_from_f32(dst + i, add ? round_to<T>(a) + load_as_f32(add + i) : a);
     }
   }
 }
@@ -327,17 +345,18 @@ __global__ __launch_bounds__(256) void combine_bwd_f64_kernel(
 
 using namespace mi355;
 
-extern "C" int mi355_combine_fwd(const void* y, int dtype, const float* weights,
-                                 const int32_t* row_of_slot, void* out, int64_t T, int64_t D,
-                                 int64_t K, int round_terms, void* stream) {
+extern "C" int mi355_combine_add_fwd(const void* y, int dtype, const float* weights, const int32_t* row_of_slot,
+                                     const void* addend, void* out, int64_t T, int64_t D, int64_t K, int round_terms,
+                                     void* stream) {
   MI355_REQUIRE(T >= 0 && D >= 1 && K >= 1 && K <= 64 && T < (1ll << 31) && D < (1ll << 31),
                 "combine_fwd: bad shape (K must be <= 64)");
   if (T == 0) return MI355_OK;
   MI355_REQUIRE(weights && row_of_slot && out, "combine_fwd: null pointer");
+  MI355_REQUIRE(!addend || dtype != MI355_F64, "combine_fwd: no fp64 form with an addend");
   const dim3 grid((unsigned)((T + 3) / 4));
   auto launch = [&](auto kernel, auto* yp, auto* op) {
-    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, as_stream(stream), yp, weights, row_of_slot, op, (int)T, (int)D,
-                       (int)K, round_terms);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, as_stream(stream), yp, weights, row_of_slot,
+                       static_cast<decltype(yp)>(addend), op, (int)T, (int)D, (int)K, round_terms);
   };
   if (dtype == MI355_F32) {
     if (K <= 8) launch(combine_fwd_kernel<float, true>, static_cast<const float*>(y), static_cast<float*>(out));
@@ -351,6 +370,12 @@ extern "C" int mi355_combine_fwd(const void* y, int dtype, const float* weights,
   } else
     return fail(MI355_EINVAL, "combine_fwd: unknown dtype %d", dtype);
   return check_launch("combine_fwd");
+}
+
+extern "C" int mi355_combine_fwd(const void* y, int dtype, const float* weights,
+                                 const int32_t* row_of_slot, void* out, int64_t T, int64_t D,
+                                 int64_t K, int round_terms, void* stream) {
+  return mi355_combine_add_fwd(y, dtype, weights, row_of_slot, nullptr, out, T, D, K, round_terms, stream);
 }
 
 extern "C" int mi355_combine_bwd(const void* dout, const void* y, int dtype, const float* weights,

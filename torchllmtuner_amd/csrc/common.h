@@ -27,6 +27,7 @@ int check_launch(const char* what);
     if (!(cond)) return mi355::fail(MI355_EINVAL, __VA_ARGS__); \
   } while (0)
 
+inline bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
 // One-time set-up per device (kernel attributes are per device): `needed()` is true until

@@ -22,6 +22,7 @@ struct GemmArgs {
   const void* B;
   void* C;
   const float* bias;  // per output column, fp32, may be null
+  const void* addend; // DENSE, no split: C = round(result) + addend, in C's dtype and layout; may be null
   int64_t a_rs, a_cs; // A(m,k) = A[m*a_rs + k*a_cs]
   int64_t b_rs, b_cs; // B(k,n) = B[k*b_rs + n*b_cs]
   int64_t ldc;
@@ -51,14 +52,20 @@ dim3 gemm_grid_kseg(int M, int N, int El);
 int launch_splitk_reduce(const float* partial, void* out, int out_dtype, int64_t MN,
                          int ksplit, hipStream_t stream);
 
-// Router projections as three bf16 MFMAs per fp32 product (router_gemm.hip): bf16 tokens,
-// fp32 weights, D and E multiples of 64.
+// Router projections (router_gemm.hip).  Backward: three bf16 MFMAs per fp32 product, for bf16
+// tokens, fp32 weights, D and E multiples of 64.
 bool router_x3_ok(int x_dtype, int w_dtype, int64_t D, int64_t E);
-int64_t router_x3_fwd_workspace(int64_t T, int64_t D, int64_t E);
 int64_t router_x3_bwd_workspace(int64_t T, int64_t D, int64_t E);
-int router_x3_fwd(const void* x, const float* w, const float* bias, float* logits, void* workspace,
-                  int64_t T, int64_t D, int64_t E, hipStream_t s);
-int router_x3_bwd(const float* dlogits, const void* x, const float* w, void* dx, float* dw,
-                  void* workspace, int64_t T, int64_t D, int64_t E, hipStream_t s);
+// Forward: `splits` (T, E) partial sums of the contraction, to be added in order (with the bias,
+// unless splits is 1: then it is added already and the one partial is the logits); 0 = no kernel
+// of that file serves the case.  `pieces` is scratch of router_fwd_pieces_bytes.
+int router_fwd_splits(int x_dtype, int w_dtype, int64_t T, int64_t D, int64_t E);
+int64_t router_fwd_pieces_bytes(int x_dtype, int w_dtype, int64_t T, int64_t D, int64_t E);
+int router_fwd_partial(const void* x, int x_dtype, const float* w, const float* bias, float* partial, void* pieces,
+                       int64_t T, int64_t D, int64_t E, hipStream_t s);
+int router_logits_reduce(const float* partial, const float* bias, float* logits, int64_t T, int64_t E, int splits,
+                         hipStream_t s);
+int router_x3_bwd(const float* dlogits, const void* x, const float* w, const void* pieces, const void* addend,
+                  void* dx, float* dw, void* workspace, int64_t T, int64_t D, int64_t E, hipStream_t s);
 
 }  // namespace mi355

@@ -40,6 +40,14 @@ __device__ __forceinline__ void store_op(T* p, CT v) {
   else store_from_f32(p, v);
 }
 
+// v rounded to the result's type, plus an element of that type
+template <typename TC>
+__device__ __forceinline__ float plus_rounded(float v, const TC* add) {
+  TC r;
+  store_from_f32(&r, v);
+  return load_as_f32(&r) + load_as_f32(add);
+}
+
 constexpr int TM = 64, TN = 64, TK = 16, PITCH = 65;
 
 template <typename TA, typename TB, typename TC>
@@ -205,7 +213,7 @@ __global__ __launch_bounds__(256) void ggemm_kernel(GemmArgs g) {
     } else {
       float v = acc[i] + bias;
       if (g.accumulate) v += load_as_f32(C + off);
-      store_from_f32(C + off, v);
+      store_from_f32(C + off, g.addend ? plus_rounded(v, static_cast<const TC*>(g.addend) + off) : v);
     }
   }
 }
@@ -307,7 +315,8 @@ __global__ __launch_bounds__(256) void dense_vec_kernel(GemmArgs g) {
     if (m >= g.M) continue;
     const int64_t off = static_cast<int64_t>(m) * g.ldc + n;
     if (Cpartial) Cpartial[off] = acc[i];
-    else store_from_f32(C + off, acc[i] + bias);
+    else store_from_f32(C + off, g.addend ? plus_rounded(acc[i] + bias, static_cast<const TC*>(g.addend) + off)
+                                          : acc[i] + bias);
   }
 }
 

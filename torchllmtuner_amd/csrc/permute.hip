@@ -15,6 +15,8 @@
 //   3. plan_rows    row = segment offset + workgroups-before + rank-in-workgroup,
 //                   written both ways (row_of_slot, slot_of_row).
 // The row movers are pure bandwidth kernels: one wave per token, 16-byte lanes.
+#include <algorithm>
+
 #include "common.h"
 
 namespace mi355 {
@@ -393,13 +395,16 @@ __device__ __forceinline__ uint4 pack_vec<uint16_t>(const float (&a)[8]) {
 
 template <typename T>
 __global__ __launch_bounds__(256) void permute_rows_bwd_kernel(
-    const T* __restrict__ drows, const int32_t* __restrict__ row_of_slot, T* __restrict__ dx, int T_,
-    int D, int K) {
+    const T* __restrict__ drows, const int32_t* __restrict__ row_of_slot, const T* __restrict__ addend,
+    T* __restrict__ dx, int T_, int D, int K) {
   const int lane = threadIdx.x & 63;
   const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (t >= T_) return;
   constexpr int V = 16 / sizeof(T);
   T* dst = dx + static_cast<int64_t>(t) * D;
+  // addend (the shared expert's input gradient): added to the rounded sum and rounded again, as the
+  // separate addition of two tensors of this type would be
+  const T* add = addend ? addend + static_cast<int64_t>(t) * D : nullptr;
   const int my_row = lane < K ? row_of_slot[static_cast<int64_t>(t) * K + lane] : -1;  // K <= 64
   // Loops are uniform across the wave (shuffles need every lane); lanes past the
   // end of the row just skip their loads and stores.
@@ -436,7 +441,18 @@ __global__ __launch_bounds__(256) void permute_rows_bwd_kernel(
 #pragma unroll
       for (int g = 0; g < G; ++g) {
         const int i = base + g * kWave + lane;
-        if (i < nv) reinterpret_cast<uint4*>(dst)[i] = pack_vec<T>(a[g]);
+        if (i < nv) {
+          uint4 sum = pack_vec<T>(a[g]);
+          if (add) {
+            float r[V];
+#pragma unroll
+            for (int q = 0; q < V; ++q) r[q] = 0.0f;
+            acc_vec<T>(r, sum);
+            acc_vec<T>(r, reinterpret_cast<const uint4*>(add)[i]);
+            sum = pack_vec<T>(r);
+          }
+          reinterpret_cast<uint4*>(dst)[i] = sum;
+        }
       }
     }
   } else {
@@ -448,7 +464,10 @@ __global__ __launch_bounds__(256) void permute_rows_bwd_kernel(
         const int row = __shfl(my_row, k, kWave);
         if (row >= 0 && on) a += load_as_f32(drows + static_cast<int64_t>(row) * D + i);
       }
-      if (on) store_from_f32(dst + i, a);
+      if (on) {
+        store_from_f32(dst + i, a);
+        if (add) store_from_f32(dst + i, load_as_f32(dst + i) + load_as_f32(add + i));
+      }
     }
   }
 }
@@ -633,20 +652,22 @@ extern "C" int mi355_permute_rows_fwd(const void* x, int dtype, const int32_t* r
   return check_launch("permute_rows_fwd");
 }
 
-extern "C" int mi355_permute_rows_bwd(const void* drows, int dtype, const int32_t* row_of_slot,
-                                      void* dx, int64_t T, int64_t D, int64_t K, void* stream) {
+extern "C" int mi355_permute_rows_add_bwd(const void* drows, int dtype, const int32_t* row_of_slot,
+                                          const void* addend, void* dx, int64_t T, int64_t D, int64_t K,
+                                          void* stream) {
   MI355_REQUIRE(D >= 1 && K >= 1 && K <= 64 && T >= 0 && T < (1ll << 31) && D < (1ll << 31),
                 "permute_rows_bwd: bad shape (K must be <= 64)");
   if (T == 0) return MI355_OK;
   MI355_REQUIRE(row_of_slot && dx, "permute_rows_bwd: null pointer");
+  MI355_REQUIRE(!addend || dtype != MI355_F64, "permute_rows_bwd: no fp64 form with an addend");
   const dim3 grid((unsigned)((T + 3) / 4));
   if (dtype == MI355_F32)
     hipLaunchKernelGGL(permute_rows_bwd_kernel<float>, grid, dim3(256), 0, as_stream(stream),
-                       static_cast<const float*>(drows), row_of_slot, static_cast<float*>(dx),
-                       (int)T, (int)D, (int)K);
+                       static_cast<const float*>(drows), row_of_slot, static_cast<const float*>(addend),
+                       static_cast<float*>(dx), (int)T, (int)D, (int)K);
   else if (dtype == MI355_BF16)
     hipLaunchKernelGGL(permute_rows_bwd_kernel<uint16_t>, grid, dim3(256), 0, as_stream(stream),
-                       static_cast<const uint16_t*>(drows), row_of_slot,
+                       static_cast<const uint16_t*>(drows), row_of_slot, static_cast<const uint16_t*>(addend),
                        static_cast<uint16_t*>(dx), (int)T, (int)D, (int)K);
   else if (dtype == MI355_F64)
     hipLaunchKernelGGL(permute_rows_bwd_f64_kernel, grid, dim3(256), 0, as_stream(stream),
@@ -655,6 +676,51 @@ extern "C" int mi355_permute_rows_bwd(const void* drows, int dtype, const int32_
   else
     return fail(MI355_EINVAL, "permute_rows_bwd: unknown dtype %d", dtype);
   return check_launch("permute_rows_bwd");
+}
+
+extern "C" int mi355_permute_rows_bwd(const void* drows, int dtype, const int32_t* row_of_slot,
+                                      void* dx, int64_t T, int64_t D, int64_t K, void* stream) {
+  return mi355_permute_rows_add_bwd(drows, dtype, row_of_slot, nullptr, dx, T, D, K, stream);
+}
+
+// Plan of one dense segment of `rows` rows (a shared expert): what segments_from_counts gives for the
+// single count, written by one launch that needs no count on the device.
+namespace mi355 {
+namespace {
+__global__ __launch_bounds__(256) void segments_dense_kernel(int rows, int tile_m, int32_t* __restrict__ seg_offsets,
+                                                             int32_t* __restrict__ seg_counts,
+                                                             int32_t* __restrict__ tile_expert,
+                                                             int32_t* __restrict__ tile_row0,
+                                                             int32_t* __restrict__ num_tiles, int nt) {
+  const int height = even_tile_rows(rows, tile_m);
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < nt; i += gridDim.x * 256) {
+    tile_expert[i] = 0;
+    tile_row0[i] = i * height;
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    seg_offsets[0] = 0;
+    seg_offsets[1] = rows;
+    seg_counts[0] = rows;
+    seg_counts[1] = 0;  // the order of the one expert
+    *num_tiles = nt;
+  }
+}
+}  // namespace
+}  // namespace mi355
+
+extern "C" int mi355_segments_dense(int64_t rows, int64_t tile_m, int32_t* seg_offsets, int32_t* seg_counts,
+                                    int32_t* tile_expert, int32_t* tile_row0, int32_t* num_tiles,
+                                    int64_t tile_capacity, void* stream) {
+  MI355_REQUIRE(rows >= 0 && rows < (1ll << 31) && tile_m >= 1 && tile_m < (1ll << 20),
+                "segments_dense: bad shape rows=%lld", (long long)rows);
+  const int64_t nt = (rows + tile_m - 1) / tile_m;
+  MI355_REQUIRE(tile_capacity >= nt, "segments_dense: tile capacity %lld below %lld", (long long)tile_capacity, (long long)nt);
+  MI355_REQUIRE(seg_offsets && seg_counts && num_tiles && (nt == 0 || (tile_expert && tile_row0)),
+                "segments_dense: null pointer");
+  hipLaunchKernelGGL(segments_dense_kernel, dim3((unsigned)std::max<int64_t>(1, (nt + 255) / 256)), dim3(256), 0,
+                     as_stream(stream), (int)rows, (int)tile_m, seg_offsets, seg_counts, tile_expert, tile_row0,
+                     num_tiles, (int)nt);
+  return check_launch("segments_dense");
 }
 
 extern "C" int mi355_segments_from_counts(const int32_t* counts, int64_t El, int64_t tile_m,

@@ -1,0 +1,340 @@
+// Expert choice and permutation plan in one pass: what mi355_router_select_fwd followed by
+// mi355_permute_plan compute, for the block's own path, in one launch (up to 64 tokens) or two.
+//
+//   1. route_rank   a workgroup of 1024 lanes takes 64 tokens at a time: each row of 16 lanes adds its
+//                   token's partial logits, selects its experts (select_rows.h) and leaves the ids
+//                   in LDS, where the workgroup ranks its slots among equal experts in slot order
+//                   (the wave's lanes by ballots over the bits of the id, the waves through
+//                   per-wave counts).  Emits weights, ids, ranks and the workgroup's histogram.
+//   2. route_rows   the same partition: every workgroup sums the histograms below its own for its
+//                   slots' offsets (all of them, for the segments), which costs it a read of a few
+//                   dozen KiB from L2 and saves the launch of a scan, and writes its slots' rows in
+//                   both directions; the first workgroup writes the plan's lists.
+// A single workgroup does both at once.  Bound by launches and dependent latency throughout: at 33
+// tokens of 128 experts the four launches this replaces took 29 us of GPU time, at 8192 tokens
+// (8 each) 39 us; here 9 and 21.
+#include <algorithm>
+
+#include "common.h"
+#include "select_rows.h"
+
+namespace mi355 {
+namespace {
+
+constexpr int kLanes = 1024, kRows = kLanes / 16, kWaves = kLanes / kWave;
+// 64 tokens of at most 16 choices are at most 1024 slots, one per lane; beyond this many workgroups
+// a workgroup takes several such chunks, so that the histograms everyone reads stay small
+constexpr int kMaxBlocks = 256;
+
+struct PlanOut {
+  int lo, hi, align, tile_m, row_capacity, tile_capacity;
+  int32_t *counts_E, *seg_offsets, *seg_counts, *row_of_slot, *slot_of_row, *token_of_row;
+  float* row_scale;
+  int32_t *tile_expert, *tile_row0, *num_tiles;
+};
+
+// Integer arrays in LDS for the layout step, E experts.
+struct LayoutLds {
+  int32_t *count, *before, *seg, *tile, *order;
+  __device__ LayoutLds(int32_t* base, int E)
+      : count(base), before(base + E), seg(base + 2 * E), tile(base + 3 * E + 1), order(base + 4 * E + 2) {}
+};
+constexpr int layout_words(int E) { return 5 * E + 3; }
+
+// counts -> padded segment offsets, tiles before each local expert, rank by descending count; left in
+// LDS for all lanes (ends on a barrier).  Each of the El + 1 sums is shared by several lanes.
+__device__ void plan_layout(const LayoutLds& s, const PlanOut& p, bool lists) {
+  const int El = p.hi - p.lo, tid = threadIdx.x;
+  for (int j = tid; j <= El; j += kLanes) s.seg[j] = s.tile[j] = s.order[j] = 0;
+  __syncthreads();
+  const int sums = El + 1;
+  const int lanes_per_sum = max(1, kLanes / sums);
+  const int slice = (El + lanes_per_sum - 1) / lanes_per_sum;
+  for (int idx = tid; idx < sums * lanes_per_sum; idx += kLanes) {
+    const int j = idx % sums, o0 = (idx / sums) * slice, o1 = min(El, o0 + slice);
+    const int c = j < El ? s.count[p.lo + j] : 0;
+    int off = 0, toff = 0, rank = 0;
+#pragma unroll 4
+    for (int o = o0; o < o1; ++o) {
+      const bool below = o < j;
+      const int co = s.count[p.lo + o];
+      off += below ? (co + p.align - 1) / p.align * p.align : 0;
+      toff += below ? (co + p.tile_m - 1) / p.tile_m : 0;
+      rank += (co > c || (co == c && below)) ? 1 : 0;
+    }
+    atomicAdd(&s.seg[j], off);
+    if (lists) {
+      atomicAdd(&s.tile[j], toff);
+      atomicAdd(&s.order[j], rank);
+    }
+  }
+  __syncthreads();
+}
+
+__device__ void write_lists(const LayoutLds& s, const PlanOut& p, int E) {
+  const int El = p.hi - p.lo, tid = threadIdx.x;
+  for (int e = tid; e < E; e += kLanes) p.counts_E[e] = s.count[e];
+  for (int j = tid; j <= El; j += kLanes) {
+    p.seg_offsets[j] = s.seg[j];
+    if (j == El) {
+      *p.num_tiles = min(s.tile[El], p.tile_capacity);
+      break;
+    }
+    const int c = s.count[p.lo + j];
+    p.seg_counts[j] = c;
+    p.seg_counts[El + s.order[j]] = j;
+    const int nt = (c + p.tile_m - 1) / p.tile_m, rows = even_tile_rows(c, p.tile_m);
+    for (int i = 0; i < nt; ++i) {
+      const int at = s.tile[j] + i;
+      if (at < p.tile_capacity) {
+        p.tile_expert[at] = j;
+        p.tile_row0[at] = s.seg[j] + i * rows;
+      }
+    }
+  }
+}
+
+__device__ __forceinline__ void place_slot(const LayoutLds& s, const PlanOut& p, int slot, int e, int rank, int K,
+                                           float weight) {
+  int row = -1;
+  if (e >= p.lo && e < p.hi) {
+    row = s.seg[e - p.lo] + s.before[e] + rank;
+    if (row < p.row_capacity) {
+      p.slot_of_row[row] = slot;
+      p.token_of_row[row] = slot / K;
+      if (p.row_scale) p.row_scale[row] = weight;
+    } else {
+      row = -1;
+    }
+  }
+  p.row_of_slot[slot] = row;
+}
+
+template <int VPR, bool FULL>
+__global__ __launch_bounds__(kLanes) void route_rank_kernel(
+    const float* __restrict__ partial, int splits, const float* __restrict__ logit_bias,
+    float* __restrict__ logits_out, SelectArgs sel, float* __restrict__ weights, int64_t* __restrict__ ids,
+    uint32_t* __restrict__ rank_in_block, int32_t* __restrict__ block_hist, int T, int chunks, int fill, PlanOut p) {
+  extern __shared__ int32_t lds[];
+  const int E = sel.E, K = sel.K;
+  int32_t* run = lds;                       // [E] slots of each expert so far
+  int32_t* cnt = lds + E;                   // [waves][E] slots of each expert in each wave of the chunk
+  int32_t* extra = cnt + kWaves * E;        // single workgroup: the layout arrays
+  __shared__ uint16_t id_sh[kLanes];
+  __shared__ float w_sh[kLanes];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l = tid & 15;
+  const bool single = gridDim.x == 1;
+  // rows that end up without a slot (padding, unused capacity) must read -1 and a zero scale
+  if (fill) {
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * kLanes + tid; i < p.row_capacity;
+         i += static_cast<int64_t>(gridDim.x) * kLanes) {
+      p.slot_of_row[i] = -1;
+      p.token_of_row[i] = -1;
+      if (p.row_scale) p.row_scale[i] = 0.0f;
+    }
+    if (single) __threadfence();  // before this workgroup's own rows, written below
+  }
+  for (int e = tid; e < E; e += kLanes) run[e] = 0;
+
+  int my_e = -1, my_rank = 0;
+  for (int c = 0; c < chunks; ++c) {
+    const int t0 = (blockIdx.x * chunks + c) * kRows;
+    if (t0 >= T) break;  // workgroup-uniform
+    for (int i = tid; i < kWaves * E; i += kLanes) cnt[i] = 0;
+    // ---- selection: one token per row of 16 lanes
+    {
+      const int t_raw = t0 + (tid >> 4);
+      const bool live = t_raw < T;
+      const int t = live ? t_raw : T - 1;
+      float x[VPR], s[VPR], cutoff;
+      load_row<VPR, FULL>(partial + static_cast<int64_t>(t) * E, l, E, x);
+      for (int z = 1; z < splits; ++z) {
+        float y[VPR];
+        load_row<VPR, FULL>(partial + (static_cast<int64_t>(z) * T + t) * E, l, E, y);
+#pragma unroll
+        for (int j = 0; j < VPR; ++j) x[j] += y[j];
+      }
+      if (splits > 1 && logit_bias) {
+#pragma unroll
+        for (int j = 0; j < VPR; ++j)
+          if (FULL || l * VPR + j < E) x[j] += logit_bias[l * VPR + j];
+      }
+      if (logits_out && live) {
+#pragma unroll
+        for (int j = 0; j < VPR; ++j)
+          if (FULL || l * VPR + j < E) logits_out[static_cast<int64_t>(t) * E + l * VPR + j] = x[j];
+      }
+      const RowChoice ch = select_row<VPR, FULL>(sel, x, l, false, s, cutoff);
+      if (l < K) {
+        const int at = (tid >> 4) * K + l;
+        id_sh[at] = static_cast<uint16_t>(live && ch.id >= 0 && ch.id < E ? ch.id : 0xffff);
+        w_sh[at] = ch.weight;
+        if (live) {
+          weights[static_cast<int64_t>(t) * K + l] = ch.weight;
+          ids[static_cast<int64_t>(t) * K + l] = ch.id;
+        }
+      }
+    }
+    __syncthreads();
+    // ---- rank of each slot among the chunk's earlier slots of its expert
+    const bool slot_here = tid < kRows * K;
+    const int e = slot_here ? id_sh[tid] : 0xffff;
+    const bool valid = e != 0xffff;
+    unsigned long long same = __ballot(valid);
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+      const bool bit = (e >> b) & 1;
+      const unsigned long long set = __ballot(bit);
+      same &= bit ? set : ~set;
+    }
+    const unsigned long long lower = (1ull << lane) - 1;
+    const int below = __popcll(same & lower);
+    if (valid && below == 0) cnt[wave * E + e] = __popcll(same);  // the lowest lane of each expert
+    __syncthreads();
+    for (int i = tid; i < E; i += kLanes) {
+      int r = run[i];
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) {
+        const int v = cnt[w * E + i];
+        cnt[w * E + i] = r;
+        r += v;
+      }
+      run[i] = r;
+    }
+    __syncthreads();
+    my_e = valid ? e : -1;
+    my_rank = valid ? cnt[wave * E + e] + below : 0;
+    const int slot = t0 * K + tid;
+    if (!single && slot_here && slot < T * K) rank_in_block[slot] = static_cast<uint32_t>(my_rank);
+    if (c + 1 < chunks) __syncthreads();  // cnt and id_sh are reused
+  }
+  if (!single) {
+    for (int e = tid; e < E; e += kLanes) block_hist[static_cast<int64_t>(blockIdx.x) * E + e] = run[e];
+    return;
+  }
+  const LayoutLds s(extra, E);
+  for (int e = tid; e < E; e += kLanes) {
+    s.count[e] = run[e];
+    s.before[e] = 0;
+  }
+  __syncthreads();
+  plan_layout(s, p, true);
+  write_lists(s, p, E);
+  if (tid < T * K && tid < kRows * K) place_slot(s, p, tid, my_e, my_rank, K, w_sh[tid]);
+}
+
+__global__ __launch_bounds__(kLanes) void route_rows_kernel(const float* __restrict__ weights,
+                                                            const int64_t* __restrict__ ids,
+                                                            const uint32_t* __restrict__ rank_in_block,
+                                                            const int32_t* __restrict__ block_hist, int T, int E, int K,
+                                                            int chunks, PlanOut p) {
+  extern __shared__ int32_t lds[];
+  const LayoutLds s(lds, E);
+  const int tid = threadIdx.x;
+  for (int e = tid; e < E; e += kLanes) s.count[e] = s.before[e] = 0;
+  __syncthreads();
+  // every expert's slots in all workgroups and in those before this one, a slice of the histograms
+  // per lane, sixteen loads in flight
+  const int parts = max(1, kLanes / E), nb = gridDim.x, per = (nb + parts - 1) / parts;
+  constexpr int kBatch = 16;
+  for (int idx = tid; idx < E * parts; idx += kLanes) {
+    const int e = idx % E, b0 = (idx / E) * per, b1 = min(nb, b0 + per);
+    int all = 0, before = 0;
+    for (int b = b0; b < b1; b += kBatch) {
+      int v[kBatch];
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) v[i] = b + i < b1 ? block_hist[static_cast<int64_t>(b + i) * E + e] : 0;
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        all += v[i];
+        before += b + i < static_cast<int>(blockIdx.x) ? v[i] : 0;
+      }
+    }
+    if (all) atomicAdd(&s.count[e], all);
+    if (before) atomicAdd(&s.before[e], before);
+  }
+  __syncthreads();
+  plan_layout(s, p, blockIdx.x == 0);
+  if (blockIdx.x == 0) write_lists(s, p, E);
+  const int first = blockIdx.x * chunks * kRows * K, last = min(T * K, first + chunks * kRows * K);
+  for (int slot = first + tid; slot < last; slot += kLanes) {
+    const int64_t e = ids[slot];
+    place_slot(s, p, slot, e >= 0 && e < E ? static_cast<int>(e) : -1, static_cast<int>(rank_in_block[slot]), K,
+               weights[slot]);
+  }
+}
+
+int route_chunks(int64_t T) {
+  const int64_t groups = (T + kRows - 1) / kRows;
+  return static_cast<int>((groups + kMaxBlocks - 1) / kMaxBlocks);
+}
+int64_t route_blocks(int64_t T) {
+  const int64_t per = static_cast<int64_t>(route_chunks(T)) * kRows;
+  return (T + per - 1) / per;
+}
+
+}  // namespace
+}  // namespace mi355
+
+using namespace mi355;
+
+extern "C" int mi355_route_plan_covers(int64_t E, int64_t K, int num_groups, int select_mode) {
+  return E >= 1 && K >= 1 && K <= E && select_row_covers(E, K, num_groups, select_mode) ? 1 : 0;
+}
+
+extern "C" int64_t mi355_route_plan_workspace_bytes(int64_t T, int64_t K, int64_t E) {
+  if (T <= kRows || K < 1 || E < 1) return 0;
+  return (T * K + route_blocks(T) * E) * (int64_t)sizeof(int32_t);
+}
+
+extern "C" int mi355_route_plan(const float* partial, int splits, const float* logit_bias, float* logits,
+                                const float* expert_bias, int64_t T, int64_t E, int64_t K, int score_func,
+                                int route_norm, float route_scale, int num_groups, int num_limited, float* weights,
+                                int64_t* ids, int64_t lo, int64_t hi, int64_t align, int64_t tile_m,
+                                int32_t* counts_E, int32_t* seg_offsets, int32_t* seg_counts, int32_t* row_of_slot,
+                                int32_t* slot_of_row, int32_t* token_of_row, float* row_scale, int64_t row_capacity,
+                                int32_t* tile_expert, int32_t* tile_row0, int32_t* num_tiles, int64_t tile_capacity,
+                                void* workspace, void* stream) {
+  MI355_REQUIRE(T >= 1 && T < (1ll << 26) && E >= 1 && K >= 1 && K <= E && T * K < (1ll << 30),
+                "route_plan: bad shape T=%lld E=%lld K=%lld", (long long)T, (long long)E, (long long)K);
+  if (!select_row_covers(E, K, num_groups, MI355_SELECT_TOPK))
+    return fail(MI355_EUNSUP, "route_plan: E=%lld K=%lld G=%d is not covered; use mi355_router_select_fwd and "
+                              "mi355_permute_plan", (long long)E, (long long)K, num_groups);
+  MI355_REQUIRE(score_func >= 0 && score_func <= 2, "route_plan: unknown score_func %d", score_func);
+  if (num_groups > 0)
+    MI355_REQUIRE(E % num_groups == 0 && E / num_groups >= 2 && num_limited >= 1 && num_limited <= num_groups &&
+                      K <= (int64_t)num_limited * (E / num_groups),
+                  "route_plan: bad group config G=%d L=%d", num_groups, num_limited);
+  MI355_REQUIRE(0 <= lo && lo < hi && hi <= E, "route_plan: bad local range [%lld,%lld)", (long long)lo, (long long)hi);
+  MI355_REQUIRE(align >= 1 && tile_m >= 1 && align < (1ll << 20) && tile_m < (1ll << 20), "route_plan: align and tile_m must be positive");
+  MI355_REQUIRE(row_capacity >= 1 && row_capacity < (1ll << 31) && tile_capacity >= 1 && tile_capacity < (1ll << 31),
+                "route_plan: bad capacity");
+  MI355_REQUIRE(partial && splits >= 1 && aligned16(partial) && weights && ids && counts_E && seg_offsets &&
+                    seg_counts && row_of_slot && slot_of_row && token_of_row && tile_expert && tile_row0 && num_tiles,
+                "route_plan: null or misaligned pointer");
+  MI355_REQUIRE(T <= kRows || workspace, "route_plan: workspace required");
+  hipStream_t s = as_stream(stream);
+  const SelectArgs sel{expert_bias, (int)E, (int)K, score_func, route_norm, route_scale, num_groups, num_limited};
+  const PlanOut p{(int)lo, (int)hi, (int)align, (int)tile_m, (int)row_capacity, (int)tile_capacity, counts_E,
+                  seg_offsets, seg_counts, row_of_slot, slot_of_row, token_of_row, row_scale, tile_expert, tile_row0,
+                  num_tiles};
+  const int chunks = route_chunks(T);
+  const int blocks = (int)route_blocks(T);
+  uint32_t* rank = static_cast<uint32_t*>(workspace);
+  int32_t* hist = reinterpret_cast<int32_t*>(rank + (blocks > 1 ? T * K : 0));
+  // every row has a slot when all experts are local and nothing is padded
+  const int fill = !(lo == 0 && hi == E && align == 1 && row_capacity == T * K);
+  const size_t lds = ((1 + kWaves) * E + (blocks == 1 ? layout_words((int)E) : 0)) * sizeof(int32_t);
+  with_row_shape(E, [&](auto vpr, auto full) {
+    hipLaunchKernelGGL((route_rank_kernel<decltype(vpr)::value, decltype(full)::value>), dim3(blocks), dim3(kLanes),
+                       lds, s, partial, splits, logit_bias, logits, sel, weights, ids, rank, hist, (int)T, chunks,
+                       fill, p);
+  });
+  if (int rc = check_launch("route_rank")) return rc;
+  if (blocks > 1) {
+    hipLaunchKernelGGL(route_rows_kernel, dim3(blocks), dim3(kLanes), layout_words((int)E) * sizeof(int32_t), s,
+                       weights, ids, rank, hist, (int)T, (int)E, (int)K, chunks, p);
+    return check_launch("route_rows");
+  }
+  return MI355_OK;
+}

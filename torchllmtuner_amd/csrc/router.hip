@@ -1,112 +1,20 @@
 // Router: fp32 gate projection and the fused score / top-k / gather / norm pass.
 //
-// Selection kernels: a token is owned by one row of 16 lanes (E = 64, 128 or 256: four tokens
-// per wavefront, lane l keeps experts l*E/16 ...) or by one 64-lane wavefront (any E up to 512:
+// Selection kernels: a token is owned by one row of 16 lanes (E <= 256: four tokens per
+// wavefront, lane l keeps consecutive experts) or by one 64-lane wavefront (any E up to 512:
 // lane l keeps experts l, l+64, l+128, ...).  The scores stay in registers, the softmax max /
 // sum and every arg-max are DPP reductions, and the K winners are written by lanes 0..K-1.  No
 // LDS, no atomics; HBM traffic is the (T,E) logits once plus the (T,K) outputs.
-#include <type_traits>
+#include <algorithm>
 
 #include "common.h"
 #include "gemm_generic.h"
+#include "select_rows.h"
 
 namespace mi355 {
 namespace {
 
 constexpr int kMaxVPL = 8;  // experts per lane -> E <= 512
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ float softplus_f32(float x) {
-  return x > 20.0f ? x : log1pf(expf(x));  // torch's threshold=20, beta=1
-}
-
-// Wave reductions of this file run on DPP row operations (VALU rate) plus four lane reads, not on
-// shuffles: a shuffle is an LDS permute, and a token's selection needs about a hundred of them --
-// with one wavefront per token the LDS pipe of a CU, not memory, was what the select kernels waited
-// for.  The four controls below exchange within a row of 16 lanes (pairs, quads, halves, the row),
-// so after them every lane holds its row's result; lanes 0, 16, 32, 48 then give the four rows.
-template <int CTRL>
-__device__ __forceinline__ float dpp_f32(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
-}
-template <int CTRL>
-__device__ __forceinline__ int dpp_i32(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, false);
-}
-constexpr int kDppPairs = 0xB1, kDppQuads = 0x4E, kDppHalfMirror = 0x141, kDppRowMirror = 0x140;
-
-__device__ __forceinline__ float lane_f32(float v, int l) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-}
-
-// sum over the wave, left in every lane
-__device__ __forceinline__ float wave_sum_dpp(float v) {
-  v += dpp_f32<kDppPairs>(v);
-  v += dpp_f32<kDppQuads>(v);
-  v += dpp_f32<kDppHalfMirror>(v);
-  v += dpp_f32<kDppRowMirror>(v);
-  return (lane_f32(v, 0) + lane_f32(v, 16)) + (lane_f32(v, 32) + lane_f32(v, 48));
-}
-__device__ __forceinline__ float wave_max_dpp(float v) {
-  v = fmaxf(v, dpp_f32<kDppPairs>(v));
-  v = fmaxf(v, dpp_f32<kDppQuads>(v));
-  v = fmaxf(v, dpp_f32<kDppHalfMirror>(v));
-  v = fmaxf(v, dpp_f32<kDppRowMirror>(v));
-  return fmaxf(fmaxf(lane_f32(v, 0), lane_f32(v, 16)), fmaxf(lane_f32(v, 32), lane_f32(v, 48)));
-}
-
-// the better of two (value, index) candidates: the larger value, ties to the lower index
-__device__ __forceinline__ void take_better(float& v, int& idx, float ov, int oi) {
-  if (ov > v || (ov == v && oi < idx)) { v = ov; idx = oi; }
-}
-
-// (value, index) arg-max across the wave, left in every lane; ties go to the lower index.
-__device__ __forceinline__ void wave_argmax(float& v, int& idx) {
-  { const float ov = dpp_f32<kDppPairs>(v); const int oi = dpp_i32<kDppPairs>(idx); take_better(v, idx, ov, oi); }
-  { const float ov = dpp_f32<kDppQuads>(v); const int oi = dpp_i32<kDppQuads>(idx); take_better(v, idx, ov, oi); }
-  { const float ov = dpp_f32<kDppHalfMirror>(v); const int oi = dpp_i32<kDppHalfMirror>(idx); take_better(v, idx, ov, oi); }
-  { const float ov = dpp_f32<kDppRowMirror>(v); const int oi = dpp_i32<kDppRowMirror>(idx); take_better(v, idx, ov, oi); }
-  float a = lane_f32(v, 0), b = lane_f32(v, 32);
-  int ai = __builtin_amdgcn_readlane(idx, 0), bi = __builtin_amdgcn_readlane(idx, 32);
-  take_better(a, ai, lane_f32(v, 16), __builtin_amdgcn_readlane(idx, 16));
-  take_better(b, bi, lane_f32(v, 48), __builtin_amdgcn_readlane(idx, 48));
-  take_better(a, ai, b, bi);
-  v = a;
-  idx = ai;
-}
-
-// the two largest of {a1 >= a2} and {b1 >= b2}, equal values counted as often as they occur
-__device__ __forceinline__ void merge_top2(float& a1, float& a2, float b1, float b2) {
-  const float lo = fminf(a1, b1);
-  a1 = fmaxf(a1, b1);
-  a2 = fmaxf(lo, fmaxf(a2, b2));
-}
-template <int CTRL>
-__device__ __forceinline__ void top2_dpp(float& m1, float& m2) {
-  const float o1 = dpp_f32<CTRL>(m1), o2 = dpp_f32<CTRL>(m2);
-  merge_top2(m1, m2, o1, o2);
-}
-// The two largest values held by the `width` lanes (a power of two, 2..64; wave-uniform) of every
-// aligned run of lanes, left in all of them.  Each step exchanges between two halves that already
-// agree among themselves, so the mirrors of the DPP controls are as good as a butterfly.
-__device__ __forceinline__ void run_top2(float& m1, float& m2, int width) {
-  top2_dpp<kDppPairs>(m1, m2);
-  if (width >= 4) top2_dpp<kDppQuads>(m1, m2);
-  if (width >= 8) top2_dpp<kDppHalfMirror>(m1, m2);
-  if (width >= 16) top2_dpp<kDppRowMirror>(m1, m2);
-  if (width >= 32) {
-    // lane ^ 16 within each half of the wave (swizzle bit mode: and 0x1f, or 0, xor 0x10)
-    const float o1 = __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(m1), 0x401f));
-    const float o2 = __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(m2), 0x401f));
-    merge_top2(m1, m2, o1, o2);
-  }
-  if (width >= 64) {
-    float a1 = lane_f32(m1, 0), a2 = lane_f32(m2, 0);
-    merge_top2(a1, a2, lane_f32(m1, 32), lane_f32(m2, 32));
-    m1 = a1;
-    m2 = a2;
-  }
-}
 
 template <int VPL>
 __device__ __forceinline__ float pick(const float (&a)[VPL], int j) {
@@ -327,212 +235,94 @@ __global__ __launch_bounds__(256) void select_fwd_kernel(
   }
 }
 
-// ---- the same selection with one token per row of 16 lanes -------------------------------------
-// For E = 64, 128 or 256, K <= 16 and 1, 2, 4, 8 or 16 expert groups (or none): four tokens per
-// wavefront, lane l of a row keeps experts l*VPR .. l*VPR + VPR - 1, so a group is a run of
-// 16 / num_groups whole lanes.  Every reduction is four
-// DPP steps inside the row and serves four tokens at once, where the wave-per-token kernel above
-// spends the same steps plus eight lane reads on one: the selection is bound by instruction
-// issue, not by memory, and this form issues about a third of the instructions per token.  The
-// choice (larger value, ties to the lower expert index) does not depend on the order of the
-// comparisons, so both kernels pick the same experts.
-__device__ __forceinline__ float row_max(float v) {
-  v = fmaxf(v, dpp_f32<kDppPairs>(v));
-  v = fmaxf(v, dpp_f32<kDppQuads>(v));
-  v = fmaxf(v, dpp_f32<kDppHalfMirror>(v));
-  return fmaxf(v, dpp_f32<kDppRowMirror>(v));
-}
-__device__ __forceinline__ float row_sum(float v) {
-  v += dpp_f32<kDppPairs>(v);
-  v += dpp_f32<kDppQuads>(v);
-  v += dpp_f32<kDppHalfMirror>(v);
-  return v + dpp_f32<kDppRowMirror>(v);
-}
-template <int CTRL>
-__device__ __forceinline__ void row_better(float& v, int& idx, float& carried) {
-  const float ov = dpp_f32<CTRL>(v), oc = dpp_f32<CTRL>(carried);
-  const int oi = dpp_i32<CTRL>(idx);
-  if (ov > v || (ov == v && oi < idx)) { v = ov; idx = oi; carried = oc; }
-}
-// (value, index) arg-max over a row, with a value carried along from the winner; left in all 16 lanes
-__device__ __forceinline__ void row_argmax(float& v, int& idx, float& carried) {
-  row_better<kDppPairs>(v, idx, carried);
-  row_better<kDppQuads>(v, idx, carried);
-  row_better<kDppHalfMirror>(v, idx, carried);
-  row_better<kDppRowMirror>(v, idx, carried);
-}
-
-template <int VPR>
+// ---- the same selection with one token per row of 16 lanes (select_rows.h) ----------------------
+template <int VPR, bool FULL>
 __global__ __launch_bounds__(256) void select_rows_kernel(
-    const float* __restrict__ logits, const float* __restrict__ expert_bias, float* __restrict__ weights,
+    const float* __restrict__ logits, SelectArgs p, float* __restrict__ weights,
     int64_t* __restrict__ ids, float* __restrict__ scores_out, uint8_t* __restrict__ map_out,
-    float* __restrict__ cutoff_out, int T, int K, int score_func, int route_norm, float route_scale,
-    int num_groups, int num_limited) {
-  constexpr int E = 16 * VPR;
+    float* __restrict__ cutoff_out, int T) {
+  const int E = p.E, K = p.K;
   const int l = threadIdx.x & 15;
   const int t_raw = blockIdx.x * 16 + (threadIdx.x >> 4);
   const bool live = t_raw < T;
   const int t = live ? t_raw : T - 1;  // a row past the end redoes the last token and stores nothing
   const int e0 = l * VPR;
-
-  float x[VPR], s[VPR];
-  const f32x4* src = reinterpret_cast<const f32x4*>(logits + static_cast<int64_t>(t) * E + e0);
+  float x[VPR], s[VPR], cutoff = 0.0f;
+  load_row<VPR, FULL>(logits + static_cast<int64_t>(t) * E, l, E, x);
+  const RowChoice c = select_row<VPR, FULL>(p, x, l, cutoff_out != nullptr, s, cutoff);
+  if (!live) return;
+  if (scores_out) {
+    float* dst = scores_out + static_cast<int64_t>(t) * E + e0;
+    if constexpr (FULL && VPR >= 4) {
 #pragma unroll
-  for (int q = 0; q < VPR / 4; ++q) {
-    const f32x4 v = src[q];
-    x[q * 4] = v[0]; x[q * 4 + 1] = v[1]; x[q * 4 + 2] = v[2]; x[q * 4 + 3] = v[3];
-  }
-  if (score_func == MI355_SCORE_SOFTMAX) {
-    float m = x[0];
+      for (int q = 0; q < VPR / 4; ++q) {
+        const f32x4 v = {s[q * 4], s[q * 4 + 1], s[q * 4 + 2], s[q * 4 + 3]};
+        reinterpret_cast<f32x4*>(dst)[q] = v;
+      }
+    } else {
 #pragma unroll
-    for (int j = 1; j < VPR; ++j) m = fmaxf(m, x[j]);
-    m = row_max(m);
-    float sum = 0.0f;
-#pragma unroll
-    for (int j = 0; j < VPR; ++j) {
-      s[j] = expf(x[j] - m);
-      sum += s[j];
-    }
-    sum = row_sum(sum);
-#pragma unroll
-    for (int j = 0; j < VPR; ++j) s[j] = s[j] / sum;
-  } else if (score_func == MI355_SCORE_SIGMOID) {
-#pragma unroll
-    for (int j = 0; j < VPR; ++j) s[j] = 1.0f / (1.0f + expf(-x[j]));
-  } else {
-#pragma unroll
-    for (int j = 0; j < VPR; ++j) s[j] = sqrtf(softplus_f32(x[j]));
-  }
-  if (scores_out && live) {
-    f32x4* dst = reinterpret_cast<f32x4*>(scores_out + static_cast<int64_t>(t) * E + e0);
-#pragma unroll
-    for (int q = 0; q < VPR / 4; ++q) {
-      const f32x4 v = {s[q * 4], s[q * 4 + 1], s[q * 4 + 2], s[q * 4 + 3]};
-      dst[q] = v;
+      for (int j = 0; j < VPR; ++j)
+        if (FULL || e0 + j < E) dst[j] = s[j];
     }
   }
-
-  // choice values: the logit itself when nothing but a monotone score function stands between
-  // it and the choice (exact: two exp() implementations can order two nearly equal scores
-  // differently, never two logits), else score (+ bias)
-  float c[VPR];
-  if (expert_bias) {
-    const f32x4* bsrc = reinterpret_cast<const f32x4*>(expert_bias + e0);
-#pragma unroll
-    for (int q = 0; q < VPR / 4; ++q) {
-      const f32x4 b = bsrc[q];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) c[q * 4 + i] = s[q * 4 + i] + b[i];
-    }
-  } else {
-#pragma unroll
-    for (int j = 0; j < VPR; ++j) c[j] = (num_groups > 0 || cutoff_out) ? s[j] : x[j];  // the cutoff is a score
+  if (cutoff_out && l == 0) cutoff_out[t] = cutoff;
+  if (l < K) {
+    weights[static_cast<int64_t>(t) * K + l] = c.weight;
+    ids[static_cast<int64_t>(t) * K + l] = c.id;
   }
-  if (num_groups > 0) {
-    // group score = sum of the group's two best choice values: each lane folds its own, the lanes
-    // of a group join them; every lane then counts the groups that beat its own (a higher score,
-    // or the same score and a lower index), seeing each other group's score by a row rotation,
-    // and a group beaten by num_limited others or more is masked
-    const int m = 16 / num_groups;  // lanes per group
-    float m1 = -INFINITY, m2 = -INFINITY;
+  if (map_out) {
+    // one-hot routing map of the token, one byte per expert: this lane's VPR experts
+    uint8_t* dst = map_out + static_cast<int64_t>(t) * E + e0;
+    if constexpr (FULL && VPR >= 4) {
 #pragma unroll
-    for (int j = 0; j < VPR; ++j) merge_top2(m1, m2, c[j], -INFINITY);
-    if (m >= 2) top2_dpp<kDppPairs>(m1, m2);
-    if (m >= 4) top2_dpp<kDppQuads>(m1, m2);
-    if (m >= 8) top2_dpp<kDppHalfMirror>(m1, m2);
-    if (m >= 16) top2_dpp<kDppRowMirror>(m1, m2);
-    const float gs = m1 + m2;
-    const int gid = l / m;
-    int beaten_by = 0;
-    auto other = [&](auto n_t) {
-      constexpr int n = decltype(n_t)::value;
-      if (n % m != 0) return;  // wave-uniform
-      const float og = dpp_f32<0x120 + n>(gs);  // row rotation by n lanes
-      const int oi = dpp_i32<0x120 + n>(gid);
-      beaten_by += (og > gs || (og == gs && oi < gid)) ? 1 : 0;
-    };
-    other(std::integral_constant<int, 1>{}); other(std::integral_constant<int, 2>{});
-    other(std::integral_constant<int, 3>{}); other(std::integral_constant<int, 4>{});
-    other(std::integral_constant<int, 5>{}); other(std::integral_constant<int, 6>{});
-    other(std::integral_constant<int, 7>{}); other(std::integral_constant<int, 8>{});
-    other(std::integral_constant<int, 9>{}); other(std::integral_constant<int, 10>{});
-    other(std::integral_constant<int, 11>{}); other(std::integral_constant<int, 12>{});
-    other(std::integral_constant<int, 13>{}); other(std::integral_constant<int, 14>{});
-    other(std::integral_constant<int, 15>{});
-    if (beaten_by >= num_limited) {
+      for (int q = 0; q < VPR / 4; ++q) {
+        const unsigned b = c.taken >> (q * 4);
+        reinterpret_cast<uint32_t*>(dst)[q] = (b & 1u) | ((b & 2u) << 7) | ((b & 4u) << 14) | ((b & 8u) << 21);
+      }
+    } else {
 #pragma unroll
-      for (int j = 0; j < VPR; ++j) c[j] = -INFINITY;
-    }
-  }
-
-  unsigned taken = 0;
-  float my_w = 0.0f;
-  int my_id = 0;
-  auto best_left = [&](float& bv, int& bi, float& bs) {
-    bv = -INFINITY;
-    bi = 0x7fffffff;
-    bs = 0.0f;
-#pragma unroll
-    for (int j = 0; j < VPR; ++j) {
-      if ((taken >> j) & 1u) continue;
-      if (bi == 0x7fffffff || c[j] > bv) { bv = c[j]; bi = e0 + j; bs = s[j]; }
-    }
-    row_argmax(bv, bi, bs);
-  };
-  for (int k = 0; k < K; ++k) {
-    float bv, bs;
-    int bi;
-    best_left(bv, bi, bs);
-    if (bi / VPR == l) taken |= 1u << (bi % VPR);
-    if (l == k) { my_w = bs; my_id = bi; }
-  }
-  if (cutoff_out) {
-    // the best choice value left after the K winners: the (K+1)-th of a sorted top-(K+1)
-    float bv, bs;
-    int bi;
-    best_left(bv, bi, bs);
-    if (l == 0 && live) cutoff_out[t] = bv;
-  }
-  if (route_norm) {
-    const float sum = row_sum(l < K ? my_w : 0.0f);
-    my_w = my_w / (sum + 1e-20f);
-  }
-  my_w = my_w * route_scale;
-  if (l < K && live) {
-    weights[static_cast<int64_t>(t) * K + l] = my_w;
-    ids[static_cast<int64_t>(t) * K + l] = my_id;
-  }
-  if (map_out && live) {
-    // one-hot routing map of the token, one byte per expert: this lane's VPR experts, four bytes a store
-    uint32_t* dst = reinterpret_cast<uint32_t*>(map_out + static_cast<int64_t>(t) * E + e0);
-#pragma unroll
-    for (int q = 0; q < VPR / 4; ++q) {
-      const unsigned b = taken >> (q * 4);
-      dst[q] = (b & 1u) | ((b & 2u) << 7) | ((b & 4u) << 14) | ((b & 8u) << 21);
+      for (int j = 0; j < VPR; ++j)
+        if (FULL || e0 + j < E) dst[j] = (c.taken >> j) & 1u;
     }
   }
 }
 
 // whether select_rows_kernel serves this call
-inline bool select_rows_ok(const float* logits, const float* bias, const float* scores, const uint8_t* map,
-                           int64_t E, int64_t K, int num_groups, int mode) {
-  return mode == MI355_SELECT_TOPK && (num_groups == 0 || (num_groups <= 16 && 16 % num_groups == 0)) && K <= 16 &&
-         (E == 64 || E == 128 || E == 256) &&
-         reinterpret_cast<uintptr_t>(logits) % 16 == 0 && reinterpret_cast<uintptr_t>(bias) % 16 == 0 &&
-         reinterpret_cast<uintptr_t>(scores) % 16 == 0 && reinterpret_cast<uintptr_t>(map) % 4 == 0;
+inline bool select_rows_ok(const float* logits, const float* scores, const uint8_t* map, int64_t E, int64_t K,
+                           int num_groups, int mode) {
+  return select_row_covers(E, K, num_groups, mode) && aligned16(logits) && aligned16(scores) &&
+         reinterpret_cast<uintptr_t>(map) % 4 == 0;
 }
-template <typename... Args>
-void launch_select_rows(int64_t E, int64_t T, hipStream_t s, Args... args) {
-  const dim3 grid((unsigned)((T + 15) / 16));
-  if (E == 64) hipLaunchKernelGGL(select_rows_kernel<4>, grid, dim3(256), 0, s, args...);
-  else if (E == 128) hipLaunchKernelGGL(select_rows_kernel<8>, grid, dim3(256), 0, s, args...);
-  else hipLaunchKernelGGL(select_rows_kernel<16>, grid, dim3(256), 0, s, args...);
+int launch_select_rows(const SelectArgs& p, const float* logits, float* weights, int64_t* ids, float* scores,
+                       uint8_t* map, float* cutoff, int64_t T, hipStream_t s, const char* what) {
+  with_row_shape(p.E, [&](auto vpr, auto full) {
+    hipLaunchKernelGGL((select_rows_kernel<decltype(vpr)::value, decltype(full)::value>), dim3((unsigned)((T + 15) / 16)),
+                       dim3(256), 0, s, logits, p, weights, ids, scores, map, cutoff, (int)T);
+  });
+  return check_launch(what);
+}
+
+// The weights' gradient as the folded expert backward leaves it: the sum, in order, of `pieces`
+// partial dot products of the slot's row (zero for a slot without one).  Added up here, by the one
+// reader, instead of by a launch of its own.
+struct DotPieces {
+  const float* partial;  // (rows, pieces) or null: dweights holds the sums
+  const int32_t* row_of_slot;
+  int pieces, rows;
+};
+__device__ __forceinline__ float slot_dweight(const DotPieces& d, const float* dweights, int64_t slot) {
+  if (!d.partial) return dweights[slot];
+  const int row = d.row_of_slot[slot];
+  float sum = 0.0f;
+  if (row >= 0 && row < d.rows)
+    for (int i = 0; i < d.pieces; ++i) sum += d.partial[static_cast<int64_t>(row) * d.pieces + i];
+  return sum;
 }
 
 template <int VPL>
 __global__ __launch_bounds__(256) void select_bwd_kernel(
     const float* __restrict__ logits, const int64_t* __restrict__ ids,
-    const float* __restrict__ dweights, const float* __restrict__ dscores,
+    const float* __restrict__ dweights, const float* __restrict__ dscores, DotPieces dots,
     float* __restrict__ dlogits, int T, int E, int K, int score_func, int route_norm,
     float route_scale, int mode) {
   extern __shared__ float lds[];  // per wave: sc[E], ds[E]
@@ -557,12 +347,12 @@ __global__ __launch_bounds__(256) void select_bwd_kernel(
   }
   __syncthreads();
 
-  if (mode != MI355_SELECT_FIXED && dweights) {
+  if (mode != MI355_SELECT_FIXED && (dweights || dots.partial)) {
     // lanes 0..K-1 own one selected expert each (K <= 64)
     int id = lane < K ? static_cast<int>(ids[static_cast<int64_t>(t) * K + lane]) : 0;
     id = min(max(id, 0), E - 1);
     const float sk = lane < K ? sc[id] : 0.0f;
-    const float dw = lane < K ? dweights[static_cast<int64_t>(t) * K + lane] : 0.0f;
+    const float dw = lane < K ? slot_dweight(dots, dweights, static_cast<int64_t>(t) * K + lane) : 0.0f;
     float g;
     if (route_norm) {
       const float denom = wave_sum_dpp(sk) + 1e-20f;
@@ -626,8 +416,13 @@ int check_router_args(int64_t T, int64_t E, int64_t K) {
 
 using namespace mi355;
 
+// Scratch of the forward for whatever dtypes follow: the weight pieces, then the partial sums.
 extern "C" int64_t mi355_router_gate_fwd_workspace_bytes(int64_t T, int64_t D, int64_t E) {
-  return (T >= 0 && D >= 1 && E >= 1 && router_x3_ok(MI355_BF16, MI355_F32, D, E)) ? router_x3_fwd_workspace(T, D, E) : 0;
+  if (T < 0 || D < 1 || E < 1) return 0;
+  const int64_t pieces = router_fwd_pieces_bytes(MI355_BF16, MI355_F32, T, D, E);
+  const int splits = std::max(router_fwd_splits(MI355_BF16, MI355_F32, T, D, E),
+                              router_fwd_splits(MI355_F32, MI355_F32, T, D, E));
+  return pieces + (splits > 1 ? splits * T * E * 4 : 0);
 }
 
 extern "C" int mi355_router_gate_fwd(const void* x, int x_dtype, const void* w, int w_dtype,
@@ -638,10 +433,15 @@ extern "C" int mi355_router_gate_fwd(const void* x, int x_dtype, const void* w, 
   MI355_REQUIRE(T < (1ll << 31) && D < (1ll << 31), "router_gate_fwd: shape exceeds int32");
   if (T == 0) return MI355_OK;
   MI355_REQUIRE(x && w && logits, "router_gate_fwd: null pointer");
-  // bf16 tokens against fp32 weights: three bf16 MFMAs per product, fp32-exact operands
-  if (workspace && router_x3_ok(x_dtype, w_dtype, D, E))
-    return router_x3_fwd(x, static_cast<const float*>(w), logit_bias, logits, workspace, T, D, E,
-                         as_stream(stream));
+  const int splits = aligned16(x) && aligned16(w) ? router_fwd_splits(x_dtype, w_dtype, T, D, E) : 0;
+  const int64_t pieces = splits ? router_fwd_pieces_bytes(x_dtype, w_dtype, T, D, E) : 0;
+  if (splits > 0 && (workspace || (splits == 1 && pieces == 0))) {
+    float* partial = splits > 1 ? reinterpret_cast<float*>(static_cast<char*>(workspace) + pieces) : logits;
+    if (int rc = router_fwd_partial(x, x_dtype, static_cast<const float*>(w), logit_bias, partial, workspace, T, D, E,
+                                    as_stream(stream)))
+      return rc;
+    return splits > 1 ? router_logits_reduce(partial, logit_bias, logits, T, E, splits, as_stream(stream)) : MI355_OK;
+  }
   GemmArgs g{};
   g.A = x; g.B = w; g.C = logits; g.bias = logit_bias;
   g.a_rs = D; g.a_cs = 1;
@@ -669,20 +469,20 @@ extern "C" int64_t mi355_router_gate_bwd_workspace_bytes(int64_t T, int64_t D, i
   return strided > x3 ? strided : x3;
 }
 
-extern "C" int mi355_router_gate_bwd(const float* dlogits, const void* x, int x_dtype,
-                                     const void* w, int w_dtype, void* dx, void* dw,
-                                     void* workspace, int64_t T, int64_t D, int64_t E,
-                                     void* stream) {
+extern "C" int mi355_router_gate_add_bwd(const float* dlogits, const void* x, int x_dtype, const void* w, int w_dtype,
+                                         const void* pieces, const void* addend, void* dx, void* dw, void* workspace,
+                                         int64_t T, int64_t D, int64_t E, void* stream) {
   MI355_REQUIRE(T >= 0 && D >= 1 && E >= 1 && T < (1ll << 31) && D < (1ll << 31),
                 "router_gate_bwd: bad shape");
   hipStream_t s = as_stream(stream);
   if (workspace && router_x3_ok(x_dtype, w_dtype, D, E)) {
     MI355_REQUIRE(dlogits && w && (x || !dw), "router_gate_bwd: null pointer");
-    return router_x3_bwd(dlogits, x, static_cast<const float*>(w), dx, static_cast<float*>(dw), workspace, T, D, E, s);
+    return router_x3_bwd(dlogits, x, static_cast<const float*>(w), pieces, addend, dx, static_cast<float*>(dw),
+                         workspace, T, D, E, s);
   }
   if (dx && T > 0) {
     GemmArgs g{};
-    g.A = dlogits; g.B = w; g.C = dx;
+    g.A = dlogits; g.B = w; g.C = dx; g.addend = addend;
     g.a_rs = E; g.a_cs = 1;
     g.b_rs = D; g.b_cs = 1;  // B(k=e, n=d) = w[e][d]
     g.ldc = D; g.M = (int)T; g.N = (int)D; g.K = (int)E;
@@ -706,6 +506,34 @@ extern "C" int mi355_router_gate_bwd(const float* dlogits, const void* x, int x_
       return launch_splitk_reduce(static_cast<const float*>(workspace), dw, w_dtype, E * D, split, s);
   }
   return MI355_OK;
+}
+
+extern "C" int mi355_router_gate_bwd(const float* dlogits, const void* x, int x_dtype,
+                                     const void* w, int w_dtype, void* dx, void* dw,
+                                     void* workspace, int64_t T, int64_t D, int64_t E,
+                                     void* stream) {
+  return mi355_router_gate_add_bwd(dlogits, x, x_dtype, w, w_dtype, nullptr, nullptr, dx, dw, workspace, T, D, E, stream);
+}
+
+extern "C" int mi355_router_gate_fwd_splits(int x_dtype, int w_dtype, int64_t T, int64_t D, int64_t E) {
+  return router_fwd_splits(x_dtype, w_dtype, T, D, E);
+}
+
+extern "C" int64_t mi355_router_gate_fwd_pieces_bytes(int x_dtype, int w_dtype, int64_t T, int64_t D, int64_t E) {
+  return T >= 1 && D >= 1 && E >= 1 ? router_fwd_pieces_bytes(x_dtype, w_dtype, T, D, E) : 0;
+}
+
+extern "C" int mi355_router_gate_fwd_partial(const void* x, int x_dtype, const float* w, const float* logit_bias,
+                                             float* partial, void* pieces, int64_t T, int64_t D, int64_t E,
+                                             void* stream) {
+  MI355_REQUIRE(T >= 1 && D >= 1 && E >= 1 && T < (1ll << 31) && D < (1ll << 31), "router_gate_fwd_partial: bad shape");
+  if (router_fwd_splits(x_dtype, MI355_F32, T, D, E) < 1)
+    return fail(MI355_EUNSUP, "router_gate_fwd_partial: dtype / width not covered; use mi355_router_gate_fwd");
+  MI355_REQUIRE(x && w && partial && aligned16(x) && aligned16(w) && aligned16(partial),
+                "router_gate_fwd_partial: null or misaligned pointer");
+  MI355_REQUIRE(pieces || router_fwd_pieces_bytes(x_dtype, MI355_F32, T, D, E) == 0,
+                "router_gate_fwd_partial: scratch for the weight pieces required");
+  return router_fwd_partial(x, x_dtype, w, logit_bias, partial, pieces, T, D, E, as_stream(stream));
 }
 
 #define DISPATCH_VPL(E, ...)                           \
@@ -734,12 +562,10 @@ extern "C" int mi355_router_select_fwd(const float* logits, const float* expert_
   }
   if (T == 0) return MI355_OK;
   MI355_REQUIRE(logits && weights && ids, "router_select_fwd: null pointer");
-  if (select_rows_ok(logits, expert_bias, scores_TE, routing_map_TE, E, K, num_groups, select_mode)) {
-    launch_select_rows(E, T, as_stream(stream), logits, expert_bias, weights, ids, scores_TE, routing_map_TE,
-                       static_cast<float*>(nullptr), (int)T, (int)K, score_func, route_norm, route_scale, num_groups,
-                       num_limited);
-    return check_launch("router_select_fwd");
-  }
+  if (select_rows_ok(logits, scores_TE, routing_map_TE, E, K, num_groups, select_mode))
+    return launch_select_rows({expert_bias, (int)E, (int)K, score_func, route_norm, route_scale, num_groups, num_limited},
+                              logits, weights, ids, scores_TE, routing_map_TE, nullptr, T, as_stream(stream),
+                              "router_select_fwd");
   const dim3 grid((unsigned)((T + 3) / 4));
   DISPATCH_VPL(E, hipLaunchKernelGGL(select_fwd_kernel<VPL>, grid, dim3(256), 0, as_stream(stream),
                                      logits, expert_bias, weights, ids, scores_TE, routing_map_TE,
@@ -760,12 +586,9 @@ extern "C" int mi355_router_select_cutoff_fwd(const float* logits, const float* 
                 (long long)K, (long long)E);
   if (T == 0) return MI355_OK;
   MI355_REQUIRE(logits && weights && ids && cutoff_T, "router_select_cutoff_fwd: null pointer");
-  if (select_rows_ok(logits, expert_bias, scores_TE, nullptr, E, K, 0, MI355_SELECT_TOPK) &&
-      reinterpret_cast<uintptr_t>(cutoff_T) % 4 == 0) {
-    launch_select_rows(E, T, as_stream(stream), logits, expert_bias, weights, ids, scores_TE,
-                       static_cast<uint8_t*>(nullptr), cutoff_T, (int)T, (int)K, score_func, route_norm, route_scale, 0, 0);
-    return check_launch("router_select_cutoff_fwd");
-  }
+  if (select_rows_ok(logits, scores_TE, nullptr, E, K, 0, MI355_SELECT_TOPK))
+    return launch_select_rows({expert_bias, (int)E, (int)K, score_func, route_norm, route_scale, 0, 0}, logits, weights,
+                              ids, scores_TE, nullptr, cutoff_T, T, as_stream(stream), "router_select_cutoff_fwd");
   const dim3 grid((unsigned)((T + 3) / 4));
   DISPATCH_VPL(E, hipLaunchKernelGGL(select_fwd_kernel<VPL>, grid, dim3(256), 0, as_stream(stream),
                                      logits, expert_bias, weights, ids, scores_TE,
@@ -775,11 +598,9 @@ extern "C" int mi355_router_select_cutoff_fwd(const float* logits, const float* 
   return check_launch("router_select_cutoff_fwd");
 }
 
-extern "C" int mi355_router_select_bwd(const float* logits, const int64_t* ids,
-                                       const float* dweights, const float* dscores_TE,
-                                       float* dlogits, int64_t T, int64_t E, int64_t K,
-                                       int score_func, int route_norm, float route_scale,
-                                       int select_mode, void* stream) {
+static int select_bwd(const float* logits, const int64_t* ids, const float* dweights, const float* dscores_TE,
+                      const DotPieces& dots, float* dlogits, int64_t T, int64_t E, int64_t K, int score_func,
+                      int route_norm, float route_scale, int select_mode, void* stream) {
   if (int rc = check_router_args(T, E, K)) return rc;
   MI355_REQUIRE(K <= 64, "router_select_bwd: top_k > 64 unsupported");
   if (T == 0) return MI355_OK;
@@ -787,7 +608,27 @@ extern "C" int mi355_router_select_bwd(const float* logits, const int64_t* ids,
   const dim3 grid((unsigned)((T + 3) / 4));
   const size_t lds = (size_t)4 * 2 * E * sizeof(float);
   DISPATCH_VPL(E, hipLaunchKernelGGL(select_bwd_kernel<VPL>, grid, dim3(256), lds, as_stream(stream),
-                                     logits, ids, dweights, dscores_TE, dlogits, (int)T, (int)E,
+                                     logits, ids, dweights, dscores_TE, dots, dlogits, (int)T, (int)E,
                                      (int)K, score_func, route_norm, route_scale, select_mode));
   return check_launch("router_select_bwd");
+}
+
+extern "C" int mi355_router_select_bwd(const float* logits, const int64_t* ids,
+                                       const float* dweights, const float* dscores_TE,
+                                       float* dlogits, int64_t T, int64_t E, int64_t K,
+                                       int score_func, int route_norm, float route_scale,
+                                       int select_mode, void* stream) {
+  return select_bwd(logits, ids, dweights, dscores_TE, DotPieces{}, dlogits, T, E, K, score_func, route_norm,
+                    route_scale, select_mode, stream);
+}
+
+extern "C" int mi355_router_select_dots_bwd(const float* logits, const int64_t* ids, const float* dot_partial,
+                                            int64_t pieces, const int32_t* row_of_slot, int64_t row_capacity,
+                                            float* dlogits, int64_t T, int64_t E, int64_t K, int score_func,
+                                            int route_norm, float route_scale, void* stream) {
+  MI355_REQUIRE(pieces >= 1 && pieces <= 4096 && row_capacity >= 0 && row_capacity < (1ll << 31),
+                "router_select_dots_bwd: bad shape");
+  MI355_REQUIRE(T == 0 || (dot_partial && row_of_slot), "router_select_dots_bwd: null pointer");
+  return select_bwd(logits, ids, nullptr, nullptr, DotPieces{dot_partial, row_of_slot, (int)pieces, (int)row_capacity},
+                    dlogits, T, E, K, score_func, route_norm, route_scale, MI355_SELECT_TOPK, stream);
 }

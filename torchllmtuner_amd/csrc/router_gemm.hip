@@ -12,6 +12,7 @@
 // Shapes: D and E multiples of 64; anything else stays on the strided fp32-MFMA kernels.
 #include <algorithm>
 #include <cstdint>
+#include <type_traits>
 
 #include "bf16_tiles.h"
 #include "common.h"
@@ -59,85 +60,127 @@ __global__ __launch_bounds__(256) void split_kernel(const float* __restrict__ w,
   if (nsplit > 2) *reinterpret_cast<u32x4*>(out + 2 * n + i) = lo;
 }
 
-// ---- logits(T,E) = x(T,D) . W(E,D)^T + bias --------------------------------------------
-// Tile 32 tokens x 128 experts, 4 waves each 32 x 32; per K step of 64: x tile KC (4 KiB)
-// and the three weight-piece tiles KC (48 KiB); two LDS stages.
-constexpr int F_BM = 32, F_BN = 128, F_NT = 256;
-constexpr int F_STAGE = (F_BM + 3 * F_BN) * BK;  // elements
+// ---- logits(T,E) = x(T,D) . W(E,D)^T + bias, few tokens or any widths --------------------
+// Bound by latency: at one token the product is one read of W (1 MB at 128 x 2048), which wants to
+// be in flight all at once and in as few launches as possible.  A workgroup takes 32 tokens x 32
+// experts and a slice of the contraction; its eight waves split that slice, and every wave reads
+// its operands straight into MFMA fragments (no LDS, no barrier in the loop; a weight is used by
+// one wave of one workgroup per 32 tokens), the fp32 weights becoming their three bf16 pieces in
+// registers on the way.  The eight partial tiles are added in wave order through LDS.  The order
+// of k inside a 32-wide step is a permutation (lane half h holds k = 16 h ..) that both operands
+// share, so that each lane reads whole 32- or 64-byte pieces of a row.
+// This replaces a kernel that walked the whole contraction in 128-expert tiles behind a separate
+// weight-splitting launch: 1 token of 2048 x 128 experts 34 -> 5 us, 1000 tokens 43 -> 14 us, 128
+// tokens of 7168 x 256 experts 131 -> 12 us.  From 1024 tokens on, with widths on its grid, the
+// 128-token kernel below reads the weights four times less often and is the faster one.
+constexpr int R_BM = 32, R_BN = 32, R_WAVES = 8, R_STEP = 32;
 
-__global__ __launch_bounds__(F_NT) void gate_fwd_kernel(const uint16_t* __restrict__ x,
-                                                        const uint16_t* __restrict__ ws,
-                                                        const float* __restrict__ bias,
-                                                        float* __restrict__ logits, int T, int D, int E) {
-  extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
+template <typename TX>
+__device__ __forceinline__ void load16_masked(const TX* p, int k, int k_end, f32x4 (&v)[4]) {
+  // fp32: four pieces of four, each inside the row or zero (D % 4 == 0)
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    v[j] = k + 4 * j < k_end ? *reinterpret_cast<const f32x4*>(p + k + 4 * j) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+}
+__device__ __forceinline__ void load16_masked(const uint16_t* p, int k, int k_end, u32x4 (&v)[2]) {
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+    v[j] = k + 8 * j < k_end ? *reinterpret_cast<const u32x4*>(p + k + 8 * j) : u32x4{0, 0, 0, 0};
+}
+
+template <typename TX>
+__global__ __launch_bounds__(64 * R_WAVES) void gate_rows_kernel(const TX* __restrict__ x,
+                                                                 const float* __restrict__ w,
+                                                                 const float* __restrict__ bias,
+                                                                 float* __restrict__ out, int T, int D, int E,
+                                                                 int k_per_wave) {
+  constexpr bool BF = sizeof(TX) == 2;
+  __shared__ __attribute__((aligned(16))) float red[R_WAVES][4][64][4];  // [wave][q][lane][i]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int t0 = blockIdx.x * F_BM, n0 = blockIdx.y * F_BN;
-  const int row = tid >> 3, chunk = tid & 7;
-  const int64_t ED = static_cast<int64_t>(E) * D;
-  const uint16_t* ap = x + static_cast<int64_t>(min(t0 + row, T - 1)) * D + chunk * 8;
-  const uint16_t* bp[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) bp[i] = ws + static_cast<int64_t>(min(n0 + row + 32 * i, E - 1)) * D + chunk * 8;
-  const int a_lds = kc_off(row, chunk);
-  u32x4 ra, rb[12];
-  auto fetch = [&](int k0) {
-    ra = *reinterpret_cast<const u32x4*>(ap + k0);
-#pragma unroll
-    for (int s = 0; s < 3; ++s)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) rb[s * 4 + i] = *reinterpret_cast<const u32x4*>(bp[i] + s * ED + k0);
-  };
-  auto park = [&](uint16_t* st) {
-    *reinterpret_cast<u32x4*>(st + a_lds) = ra;
-#pragma unroll
-    for (int s = 0; s < 3; ++s)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        *reinterpret_cast<u32x4*>(st + (F_BM + s * F_BN + 32 * i) * BK + a_lds) = rb[s * 4 + i];
-  };
+  const int t0 = blockIdx.x * R_BM, n0 = blockIdx.y * R_BN;
+  const int half = lane >> 5;
+  const TX* xp = x + static_cast<int64_t>(min(t0 + (lane & 31), T - 1)) * D;
+  const float* wp = w + static_cast<int64_t>(min(n0 + (lane & 31), E - 1)) * D;
+  const int k0 = (blockIdx.z * R_WAVES + wave) * k_per_wave;
+  const int k1 = min(k0 + k_per_wave, D);
   f32x16 acc;
 #pragma unroll
   for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
-  const int ksteps = D / BK;
-  fetch(0);
-  park(smem);
-  if (ksteps > 1) fetch(BK);
+  constexpr int B = 4;  // steps requested together: 128 of the contraction, 24 KiB (bf16 x) per wave
+  for (int kb = k0; kb < k1; kb += B * R_STEP) {
+    f32x4 wv[B][4];
+    std::conditional_t<BF, u32x4[B][2], f32x4[B][4]> xv;
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      const int k = kb + b * R_STEP + 16 * half;
+      load16_masked(wp, k, k1, wv[b]);
+      load16_masked(xp, k, k1, xv[b]);
+    }
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      if (kb + b * R_STEP >= k1) break;  // wave-uniform
+      if constexpr (BF) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          u32x4 hi, mid, lo;
+          split8(wv[b][2 * j], wv[b][2 * j + 1], hi, mid, lo);
+          const bf16x8 a = __builtin_bit_cast(bf16x8, xv[b][j]);
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, hi), a, acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, mid), a, acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, lo), a, acc, 0, 0, 0);
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(wv[b][j][i], xv[b][j][i], acc, 0, 0, 0);
+      }
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const f32x4 v = {acc[q * 4], acc[q * 4 + 1], acc[q * 4 + 2], acc[q * 4 + 3]};
+    *reinterpret_cast<f32x4*>(red[wave][q][lane]) = v;
+  }
   __syncthreads();
-  for (int ks = 0; ks < ksteps; ++ks) {
-    const uint16_t* As = smem + (ks & 1) * F_STAGE;
-    if (ks + 1 < ksteps) park(smem + ((ks + 1) & 1) * F_STAGE);
-    if (ks + 2 < ksteps) fetch((ks + 2) * BK);
+  if (tid >= 256) return;
+  // lane = token row (lane & 31); piece q = expert columns q * 8 + (lane >> 5) * 4 + 0..3
+  const int q = tid >> 6;
+  f32x4 v = *reinterpret_cast<const f32x4*>(red[0][q][lane]);
 #pragma unroll
-    for (int kk = 0; kk < BK / 16; ++kk) {
-      const bf16x8 af = frag_kc(As, 0, kk, lane);
+  for (int i = 1; i < R_WAVES; ++i) v += *reinterpret_cast<const f32x4*>(red[i][q][lane]);
+  const int t = t0 + (lane & 31), n = n0 + q * 8 + half * 4;
+  if (t >= T || n >= E) return;
+  float* dst = out + (static_cast<int64_t>(blockIdx.z) * T + t) * E + n;
+  if (bias) {
 #pragma unroll
-      for (int s = 0; s < 3; ++s) {
-        const bf16x8 bf = frag_kc(As + (F_BM + s * F_BN) * BK, wave * 32, kk, lane);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf, af, acc, 0, 0, 0);
-      }
-    }
-    __syncthreads();
+    for (int i = 0; i < 4; ++i)
+      if (n + i < E) v[i] += bias[n + i];
   }
-  // lane = token row (lane & 31); registers = expert columns (i>>2)*8 + (lane>>5)*4 + (i&3)
-  const int t = t0 + (lane & 31);
-  if (t < T) {
+  if (E % 4 == 0) {
+    *reinterpret_cast<f32x4*>(dst) = v;
+  } else {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int n = n0 + wave * 32 + q * 8 + (lane >> 5) * 4;
-      if (n < E) {  // E % 4 == 0
-        f32x4 v = {acc[q * 4], acc[q * 4 + 1], acc[q * 4 + 2], acc[q * 4 + 3]};
-        if (bias) v += *reinterpret_cast<const f32x4*>(bias + n);
-        *reinterpret_cast<f32x4*>(logits + static_cast<int64_t>(t) * E + n) = v;
-      }
-    }
+    for (int i = 0; i < 4; ++i)
+      if (n + i < E) dst[i] = v[i];
   }
+}
+
+// Splits of the contraction over workgroups: about 128 of it per wave (one batch of requests)
+// while that leaves the launch below four workgroups a CU; each split costs its consumer one
+// more read of the (T, E) partial sums.
+int rows_splits(int64_t T, int64_t D, int64_t E) {
+  const int64_t tiles = ((T + R_BM - 1) / R_BM) * ((E + R_BN - 1) / R_BN);
+  const int64_t want = (D + 128 * R_WAVES - 1) / (128 * R_WAVES);
+  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({want, 8, 1024 / tiles})));
 }
 
 // The same product for many tokens: 128 tokens x 128 experts per workgroup, 8 waves as 2 x 4
 // (each 64 tokens x 32 experts), the contraction split over gridDim.z so that the grid still
-// fills the chip.  The 32-token kernel above streams the three weight-piece tiles once per 32
-// tokens -- at T = 8192 that is 0.4 GB through L2 for a 37 MB problem, and all of its time;
-// this one streams them once per 128 tokens.  Partial sums go to the workspace and are added
+// fills the chip.  The kernel above reads the weights once per 32 tokens -- at T = 8192 that is
+// 0.25 GB through L2 and a conversion each time for a 37 MB problem; this one streams the weight
+// pieces, split beforehand, once per 128 tokens.  Partial sums go to the workspace and are added
 // (with the bias) in split order by logits_reduce_kernel; a single split writes logits itself.
 constexpr int G_BM = 128, G_BN = 128, G_NT = 512;
 constexpr int G_STAGE = (G_BM + 3 * G_BN) * BK;  // elements, 64 KiB
@@ -234,11 +277,23 @@ __global__ __launch_bounds__(256) void logits_reduce_kernel(const float* __restr
                                                             const float* __restrict__ bias,
                                                             float* __restrict__ logits, int64_t TE, int E,
                                                             int splits) {
-  const int64_t i = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
-  if (i >= TE) return;  // E % 4 == 0: a group of four never straddles a row
+  const int64_t first = static_cast<int64_t>(blockIdx.x) * 1024;
+  if (TE % 4) {  // (then E % 4 != 0 too, and the splits' rows are not 16-byte aligned)
+    for (int64_t i = first + threadIdx.x; i < min(first + 1024, TE); i += 256) {
+      float acc = partial[i];
+      for (int z = 1; z < splits; ++z) acc += partial[z * TE + i];
+      logits[i] = bias ? acc + bias[i % E] : acc;
+    }
+    return;
+  }
+  const int64_t i = first + threadIdx.x * 4;
+  if (i >= TE) return;
   f32x4 acc = *reinterpret_cast<const f32x4*>(partial + i);
   for (int z = 1; z < splits; ++z) acc += *reinterpret_cast<const f32x4*>(partial + z * TE + i);
-  if (bias) acc += *reinterpret_cast<const f32x4*>(bias + i % E);
+  if (bias) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] += bias[(i + j) % E];
+  }
   *reinterpret_cast<f32x4*>(logits + i) = acc;
 }
 
@@ -249,6 +304,7 @@ constexpr int X_BM = 128, X_BN = 128, X_NT = 512;
 
 __global__ __launch_bounds__(X_NT, 2) void gate_dx_kernel(const float* __restrict__ dlogits,
                                                          const uint16_t* __restrict__ ws,
+                                                         const uint16_t* __restrict__ addend,
                                                          uint16_t* __restrict__ dx, int T, int D, int E) {
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
   uint16_t* A_hi = smem;                    // [128][64] KC
@@ -327,9 +383,20 @@ __global__ __launch_bounds__(X_NT, 2) void gate_dx_kernel(const float* __restric
     const int idx = it * 64 + lane;
     const int m = idx >> 2, c = idx & 3;
     const int t = t0 + wm + m;
-    if (t < T)
-      *reinterpret_cast<u32x4*>(dx + static_cast<int64_t>(t) * D + n0 + wn + c * 8) =
-          *reinterpret_cast<const u32x4*>(st + m * S::PITCH + c * 8);
+    if (t < T) {
+      const int64_t at = static_cast<int64_t>(t) * D + n0 + wn + c * 8;
+      u32x4 v = *reinterpret_cast<const u32x4*>(st + m * S::PITCH + c * 8);
+      if (addend) {
+        // the gradient that came back along the tokens' other uses: added here instead of by a pass of
+        // its own over three (T, D) tensors (17 us at 8192 x 2048), with that pass's rounding
+        const u32x4 a = *reinterpret_cast<const u32x4*>(addend + at);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          v[i] = pack_bf16x2(__uint_as_float(v[i] << 16) + __uint_as_float(a[i] << 16),
+                             __uint_as_float(v[i] & 0xffff0000u) + __uint_as_float(a[i] & 0xffff0000u));
+      }
+      *reinterpret_cast<u32x4*>(dx + at) = v;
+    }
   }
 }
 
@@ -425,13 +492,11 @@ int set_dyn_lds(K kernel, int bytes) {
   return e == hipSuccess ? MI355_OK : fail(MI355_ELAUNCH, "hipFuncSetAttribute: %s", hipGetErrorString(e));
 }
 
-constexpr int F_LDS = 2 * F_STAGE * 2;                         // 106496
 constexpr int G_LDS = 2 * G_STAGE * 2;                         // 131072
 
 // Splits of the contraction for the 128-token forward kernel: enough workgroups for the chip,
-// at least four K steps each, whole K steps.  0 = use the 32-token kernel (few tokens).
+// at least four K steps each, whole K steps.
 int fwd_splits(int64_t T, int64_t D, int64_t E) {
-  if (T < 1024) return 0;
   const int64_t tiles = ((T + G_BM - 1) / G_BM) * ((E + G_BN - 1) / G_BN);
   int64_t s = 1;
   while (s < 8 && tiles * s < 256 && D % (2 * s * BK) == 0 && D / (2 * s) >= 4 * BK) s *= 2;
@@ -464,49 +529,67 @@ bool router_x3_ok(int x_dtype, int w_dtype, int64_t D, int64_t E) {
   return x_dtype == MI355_BF16 && w_dtype == MI355_F32 && D % 64 == 0 && E % 64 == 0 && D >= 128;
 }
 
-int64_t router_x3_fwd_workspace(int64_t T, int64_t D, int64_t E) {
-  const int s = fwd_splits(T, D, E);
-  return 3 * E * D * 2 + (s > 1 ? static_cast<int64_t>(s) * T * E * 4 : 0);
-}
-
 int64_t router_x3_bwd_workspace(int64_t T, int64_t D, int64_t E) {
   return 2 * E * D * 2 + static_cast<int64_t>(dw_splits(T, D, E)) * E * D * 4;
 }
 
-int router_x3_fwd(const void* x, const float* w, const float* bias, float* logits, void* workspace, int64_t T,
-                  int64_t D, int64_t E, hipStream_t s) {
-  static PerDeviceOnce configured;
-  if (configured.needed()) {
-    if (int rc = set_dyn_lds(gate_fwd_kernel, F_LDS)) return rc;
-    configured.done();
-  }
-  uint16_t* ws = static_cast<uint16_t*>(workspace);
-  const int64_t n = E * D;
-  hipLaunchKernelGGL(split_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, s, w, ws, n, 3);
-  if (const int splits = fwd_splits(T, D, E)) {
+// Which forward kernel serves a gate: the 128-token one (widths on its grid and tokens enough), the
+// 32-token one (fp32 weights, rows of whole 16-byte pieces), or neither (fp64, odd widths).
+static bool gate_wide(int x_dtype, int w_dtype, int64_t T, int64_t D, int64_t E) {
+  return T >= 1024 && router_x3_ok(x_dtype, w_dtype, D, E);
+}
+int router_fwd_splits(int x_dtype, int w_dtype, int64_t T, int64_t D, int64_t E) {
+  if (T < 1 || D < 1 || E < 1) return 0;
+  if (gate_wide(x_dtype, w_dtype, T, D, E)) return fwd_splits(T, D, E);
+  if (w_dtype != MI355_F32 || E > 65535 * R_BN) return 0;
+  if ((x_dtype == MI355_BF16 && D % 8 == 0) || (x_dtype == MI355_F32 && D % 4 == 0)) return rows_splits(T, D, E);
+  return 0;
+}
+
+int64_t router_fwd_pieces_bytes(int x_dtype, int w_dtype, int64_t T, int64_t D, int64_t E) {
+  return gate_wide(x_dtype, w_dtype, T, D, E) ? 3 * E * D * 2 : 0;
+}
+
+int router_fwd_partial(const void* x, int x_dtype, const float* w, const float* bias, float* partial, void* pieces,
+                       int64_t T, int64_t D, int64_t E, hipStream_t s) {
+  const int splits = router_fwd_splits(x_dtype, MI355_F32, T, D, E);
+  const float* in_kernel_bias = splits == 1 ? bias : nullptr;
+  if (gate_wide(x_dtype, MI355_F32, T, D, E)) {
     static PerDeviceOnce wide_configured;
     if (wide_configured.needed()) {
       if (int rc = set_dyn_lds(gate_fwd_wide_kernel, G_LDS)) return rc;
       wide_configured.done();
     }
-    float* partial = reinterpret_cast<float*>(ws + 3 * n);  // behind the weight pieces
+    uint16_t* ws = static_cast<uint16_t*>(pieces);
+    const int64_t n = E * D;
+    hipLaunchKernelGGL(split_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, s, w, ws, n, 3);
     const dim3 grid((unsigned)((T + G_BM - 1) / G_BM), (unsigned)((E + G_BN - 1) / G_BN), (unsigned)splits);
-    hipLaunchKernelGGL(gate_fwd_wide_kernel, grid, dim3(G_NT), G_LDS, s, static_cast<const uint16_t*>(x), ws, bias,
-                       splits > 1 ? partial : logits, (int)T, (int)D, (int)E, (int)(D / splits));
-    if (splits > 1) {
-      const int64_t te = T * E;
-      hipLaunchKernelGGL(logits_reduce_kernel, dim3((unsigned)((te / 4 + 255) / 256)), dim3(256), 0, s, partial, bias,
-                         logits, te, (int)E, splits);
-    }
+    hipLaunchKernelGGL(gate_fwd_wide_kernel, grid, dim3(G_NT), G_LDS, s, static_cast<const uint16_t*>(x), ws,
+                       in_kernel_bias, partial, (int)T, (int)D, (int)E, (int)(D / splits));
     return check_launch("router_gate_fwd");
   }
-  hipLaunchKernelGGL(gate_fwd_kernel, dim3((unsigned)((T + F_BM - 1) / F_BM), (unsigned)((E + F_BN - 1) / F_BN)),
-                     dim3(F_NT), F_LDS, s, static_cast<const uint16_t*>(x), ws, bias, logits, (int)T, (int)D, (int)E);
+  const int64_t per_wave = (D + splits * R_WAVES - 1) / (splits * R_WAVES);
+  const int k_per_wave = (int)((per_wave + R_STEP - 1) / R_STEP * R_STEP);
+  const dim3 grid((unsigned)((T + R_BM - 1) / R_BM), (unsigned)((E + R_BN - 1) / R_BN), (unsigned)splits);
+  if (x_dtype == MI355_BF16)
+    hipLaunchKernelGGL(gate_rows_kernel<uint16_t>, grid, dim3(64 * R_WAVES), 0, s, static_cast<const uint16_t*>(x), w,
+                       in_kernel_bias, partial, (int)T, (int)D, (int)E, k_per_wave);
+  else
+    hipLaunchKernelGGL(gate_rows_kernel<float>, grid, dim3(64 * R_WAVES), 0, s, static_cast<const float*>(x), w,
+                       in_kernel_bias, partial, (int)T, (int)D, (int)E, k_per_wave);
   return check_launch("router_gate_fwd");
 }
 
-int router_x3_bwd(const float* dlogits, const void* x, const float* w, void* dx, float* dw, void* workspace,
-                  int64_t T, int64_t D, int64_t E, hipStream_t s) {
+int router_logits_reduce(const float* partial, const float* bias, float* logits, int64_t T, int64_t E, int splits,
+                         hipStream_t s) {
+  const int64_t te = T * E;
+  hipLaunchKernelGGL(logits_reduce_kernel, dim3((unsigned)((te + 1023) / 1024)), dim3(256), 0, s, partial, bias,
+                     logits, te, (int)E, splits);
+  return check_launch("router_gate_fwd");
+}
+
+int router_x3_bwd(const float* dlogits, const void* x, const float* w, const void* pieces, const void* addend,
+                  void* dx, float* dw, void* workspace, int64_t T, int64_t D, int64_t E, hipStream_t s) {
   static PerDeviceOnce configured;
   if (configured.needed()) {
     if (int rc = set_dyn_lds(gate_dx_kernel, X_LDS)) return rc;
@@ -516,9 +599,12 @@ int router_x3_bwd(const float* dlogits, const void* x, const float* w, void* dx,
   uint16_t* ws = static_cast<uint16_t*>(workspace);
   const int64_t n = E * D;
   if (dx && T > 0) {
-    hipLaunchKernelGGL(split_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, s, w, ws, n, 2);
+    // (the forward's pieces, when its caller kept them: hi and mid come first there too)
+    if (!pieces)
+      hipLaunchKernelGGL(split_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, s, w, ws, n, 2);
     hipLaunchKernelGGL(gate_dx_kernel, dim3((unsigned)((T + X_BM - 1) / X_BM), (unsigned)((D + X_BN - 1) / X_BN)),
-                       dim3(X_NT), X_LDS, s, dlogits, ws, static_cast<uint16_t*>(dx), (int)T, (int)D, (int)E);
+                       dim3(X_NT), X_LDS, s, dlogits, pieces ? static_cast<const uint16_t*>(pieces) : ws,
+                       static_cast<const uint16_t*>(addend), static_cast<uint16_t*>(dx), (int)T, (int)D, (int)E);
     if (int rc = check_launch("router_gate_bwd dx")) return rc;
   }
   if (dw) {

@@ -15,106 +15,15 @@
 // tile_expert (tile_cap) | tile_row0 (tile_cap) | num_tiles (1) in one allocation;
 // seg_counts and expert_order must stay adjacent (the weight-gradient kernels read the
 // experts' order right behind the counts).
-#include <ATen/ATen.h>
-#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
-#include <c10/core/DeviceGuard.h>
 #include <torch/library.h>
 
-#include <hip/hip_runtime_api.h>
-
-#include <mutex>
-#include <optional>
 #include <tuple>
 
-#include "../../include/mi355_moe.h"
+#include "torch_common.h"
 
 namespace {
 
-// A second stream per device (default priority, not synchronising with the null stream) and the
-// two events of a fork / join around it.  The backward's weight gradients do not depend on its
-// input gradient: launched there, their workgroups fill the CUs that the last, partly filled
-// round of the other product's tiles leaves idle, and the bandwidth-bound row sum runs beside
-// matrix work instead of between two launches.  Created on first use; never under stream
-// capture (a caller who captures first runs a step uncaptured, as for every lazily built state);
-// nullptr means "stay on one stream".
-struct SideStream {
-  hipStream_t stream = nullptr;
-  hipEvent_t fork = nullptr, join = nullptr;
-  std::mutex order;  // an event is recorded and waited for as one step: host threads share the pair
-
-  // `to` waits for everything enqueued on `from` so far
-  bool chain(hipEvent_t event, hipStream_t from, hipStream_t to) {
-    std::lock_guard<std::mutex> lock(order);
-    return hipEventRecord(event, from) == hipSuccess && hipStreamWaitEvent(to, event, 0) == hipSuccess;
-  }
-};
-
-// which: 0 the weight gradients of the fused backward, 1 the shared expert (handed to the Python
-// layer as a raw pointer, see aux_stream below)
-SideStream* side_stream(int device, hipStream_t current, int which = 0) {
-  static std::mutex mu;
-  static SideStream streams[2][64];
-  static bool attempted[2][64];
-  if (device < 0 || device >= 64 || which < 0 || which > 1) return nullptr;
-  std::lock_guard<std::mutex> lock(mu);
-  SideStream& s = streams[which][device];
-  bool* tried = attempted[which];
-  if (!tried[device]) {
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(current, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone)
-      return nullptr;  // not now: try again on a later, uncaptured call
-    tried[device] = true;
-    if (hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking) != hipSuccess ||
-        hipEventCreateWithFlags(&s.fork, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&s.join, hipEventDisableTiming) != hipSuccess) {
-      (void)hipGetLastError();
-      s.stream = nullptr;
-    }
-  }
-  return s.stream ? &s : nullptr;
-}
-
-using at::Tensor;
-using OptTensor = std::optional<Tensor>;
-
-int dtype_code(const Tensor& t) {
-  if (t.scalar_type() == at::kFloat) return MI355_F32;
-  if (t.scalar_type() == at::kBFloat16) return MI355_BF16;
-  if (t.scalar_type() == at::kDouble) return MI355_F64;
-  TORCH_CHECK_TYPE(false, "MI355 MoE kernels support float32, bfloat16 and float64, got ", t.scalar_type());
-}
-
-void* ptr(const Tensor& t) { return (t.defined() && t.numel() > 0) ? t.data_ptr() : nullptr; }
-void* ptr(const OptTensor& t) { return t.has_value() ? ptr(*t) : nullptr; }
-const int32_t* iptr(const Tensor& t) { return static_cast<const int32_t*>(ptr(t)); }
-const int32_t* iptr(const OptTensor& t) { return static_cast<const int32_t*>(ptr(t)); }
-const float* fptr(const Tensor& t) { return static_cast<const float*>(ptr(t)); }
-const float* fptr(const OptTensor& t) { return static_cast<const float*>(ptr(t)); }
-
-// Device guard + the current stream of that device, for the duration of one operator.
-struct Launch {
-  c10::DeviceGuard guard;
-  void* stream;
-  explicit Launch(const Tensor& t)
-      : guard(t.device()),
-        stream(c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream()) {
-    TORCH_CHECK(t.is_cuda(), "MI355 MoE kernels need tensors on a HIP device (got ", t.device(),
-                "); there is no CPU implementation");
-  }
-};
-
-void check(int rc, const char* what) {
-  if (rc == MI355_OK) return;
-  const char* msg = mi355_moe_last_error();
-  TORCH_CHECK_VALUE(rc != MI355_EINVAL, what, " failed (", rc, "): ", msg);
-  TORCH_CHECK(false, what, " failed (", rc, "): ", msg);
-}
-
-Tensor cf(const Tensor& t) { return t.scalar_type() == at::kFloat ? t.contiguous() : t.to(at::kFloat).contiguous(); }
-Tensor bytes(int64_t n, const Tensor& like) {
-  return at::empty({n > 0 ? n : 1}, like.options().dtype(at::kByte));
-}
-Tensor none_like(const Tensor& like) { return at::empty({0}, like.options()); }
+using namespace mi355_torch;
 
 // ------------------------------------------------------------------ router
 Tensor router_gate_fwd(const Tensor& x_, const Tensor& w_, const OptTensor& bias_) {

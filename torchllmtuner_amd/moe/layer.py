@@ -20,13 +20,33 @@ import torch.nn as nn
 
 from .. import ops
 from .auxiliary_loss import in_checkpoint_recompute
-from .experts import RoutedExperts, _is_own_dispatcher
+from .experts import DenseSwiGLU, GroupedExperts, RoutedExperts, _is_own_dispatcher
+from .linear import RouterGateLinear
 from .routing import QuantileBalancedTopKRouter, TokenChoiceTopKRouter
 
 __all__ = ["MoE", "in_checkpoint_recompute"]
 
 # in_checkpoint_recompute is set by an activation-checkpointing wrapper while it replays a
 # forward; counter updates are skipped there (llmtuner/models/common/aux_loss.py:47-68).
+
+
+_BLOCK_DTYPES = (torch.bfloat16, torch.float32)
+
+
+def _plain(module: nn.Module, cls: type) -> bool:
+    """True when calling ``module`` is exactly ``cls.forward``: that very class, nothing patched onto the
+    instance, no hooks on it (the global hooks are the caller's to check)."""
+    if type(module) is not cls:
+        return False
+    d = module.__dict__
+    return not (d["_forward_hooks"] or d["_forward_pre_hooks"] or d["_backward_hooks"] or d["_backward_pre_hooks"]
+                or "forward" in d)
+
+
+def _global_hooks() -> bool:
+    m = nn.modules.module
+    return bool(m._global_forward_hooks or m._global_forward_pre_hooks or m._global_backward_hooks
+                or m._global_backward_pre_hooks)
 
 
 class MoE(nn.Module):
@@ -147,6 +167,72 @@ class MoE(nn.Module):
             shared_TD = self.shared_experts(tokens)
         return shared_TD, stream
 
+    def _shared_weights(self, dtype):
+        """``(gate, up, down)`` weights when the shared expert is a plain ``DenseSwiGLU`` of ``dtype``,
+        ``(None, None, None)`` when there is none, None when it is anything else."""
+        shared = self.shared_experts
+        if shared is None:
+            return None, None, None
+        if not _plain(shared, DenseSwiGLU):
+            return None
+        weights = []
+        for name in ("gate_proj", "up_proj", "down_proj"):
+            linear = shared._modules[name]
+            if not _plain(linear, nn.Linear) or linear._parameters["bias"] is not None:
+                return None
+            weights.append(linear._parameters["weight"])
+        return weights if all(w.dtype is dtype for w in weights) else None
+
+    def _forward_as_one(self, tokens: torch.Tensor):
+        """``(output, counts per expert)`` from the one operator that computes the whole block
+        (``mi355_moe::moe_block``), or None when a stage has to be visible or is not what it computes: a
+        hook or an override anywhere below, an observer, an auxiliary loss, another router, dispatcher,
+        activation or shared expert, fp64, no tokens, a tracing compiler.  Both ways give the same bits."""
+        if (
+            torch.compiler.is_compiling()
+            or type(tokens) not in (torch.Tensor, nn.Parameter)
+            or not tokens.is_cuda
+            or tokens.dtype not in _BLOCK_DTYPES
+            or tokens.shape[0] == 0
+            or _global_hooks()
+        ):
+            return None
+        modules = self._modules
+        router, routed = modules["router"], modules["routed_experts"]
+        if not _plain(router, TokenChoiceTopKRouter) or not _plain(routed, RoutedExperts):
+            return None
+        d = router.__dict__
+        if (
+            router.fixed_router
+            or router._debug_force_load_balance
+            or (router.aux_loss is not None and self.training)
+            or "_select" in d
+            or not ops.route_plan_covers(router.num_experts, router.top_k, router.num_expert_groups)
+        ):
+            return None
+        gate, experts = router._modules["gate"], routed._modules["inner_experts"]
+        if not _plain(gate, RouterGateLinear) or not _plain(experts, GroupedExperts) or "_grouped_mm" in experts.__dict__:
+            return None
+        observation = routed.dispatch_observation
+        if (observation is not None and observation.observer is not None) or "_compute" in experts.__dict__:
+            return None
+        dispatcher = routed.token_dispatcher
+        if not experts.fuses_activation() or not _is_own_dispatcher(dispatcher):
+            return None
+        dtype = tokens.dtype
+        p = experts._parameters
+        w1, w3, w2 = p["w1_EFD"], p["w3_EFD"], p["w2_EDF"]
+        gate_weight = gate._parameters["weight"]
+        shared = self._shared_weights(dtype)
+        if shared is None or w1.dtype is not dtype or w3.dtype is not dtype or w2.dtype is not dtype:
+            return None
+        lo, hi = dispatcher._local_range()
+        return ops.moe_block(
+            tokens, gate_weight, gate._parameters["bias"], self.expert_bias_E, w1, w3, w2, shared,
+            router.top_k, router.score_func, router.route_norm, router.route_scale, router.num_expert_groups,
+            router.num_limited_groups, lo, hi, dispatcher._align(), not dispatcher.accumulate_in_fp32,
+            self.overlap_shared_experts)
+
     def set_padding_mask(self, padding_mask: torch.Tensor | None) -> None:
         self._pending_padding_mask = padding_mask
 
@@ -165,6 +251,17 @@ class MoE(nn.Module):
                     "padding_mask_T must have shape matching the routing-map token axis, "
                     f"got {tuple(padding_mask.shape)} for {tokens.shape[0]} tokens."
                 )
+
+        if padding_mask is None:
+            whole = self._forward_as_one(tokens)
+            if whole is not None:
+                out_TD, num_tokens_per_expert_E = whole
+                if self.training and not in_checkpoint_recompute.get():
+                    with torch.no_grad():
+                        self.tokens_per_expert_E.add_(num_tokens_per_expert_E)
+                if restore_shape:
+                    out_TD = out_TD.reshape(*x.shape[:-1], out_TD.shape[-1])
+                return (out_TD, None) if self.returns_router_logits else out_TD
 
         shared_TD, shared_stream = self._start_shared_experts(tokens)
 

@@ -290,6 +290,12 @@ def _(dout, x, weights, w1, w3, w2, gate, up, token_of_row, slot_of_row, row_of_
             x.new_empty((x.shape[0], top_k), dtype=torch.float32))
 
 
+@_fake("moe_block")
+def _(x, gate_w, gate_bias, expert_bias, w1, w3, w2, shared_gate, shared_up, shared_down, top_k, score_func, route_norm,
+      route_scale, num_groups, num_limited, local_lo, local_hi, align, round_terms, overlap_shared):
+    return torch.empty_like(x), x.new_empty((gate_w.shape[0],), dtype=torch.int32)
+
+
 # ====================================================================== autograd formulas
 # Each differentiable operator's backward is the hand-written kernel for that stage (linear.py:133-151 is
 # the gate's formula).  The formulas are C++ autograd nodes registered for the operators' Autograd key in
@@ -669,6 +675,30 @@ def grouped_swiglu_combine_bwd(dout_TD, x_TD, weights_TK, w1_EFD, w3_EFD, w2_EDF
         dout_TD, x_TD, weights_TK, w1_EFD, w3_EFD, w2_EDF, gate, up, plan.token_of_row, plan.slot_of_row,
         plan.row_of_slot, *plan.segments(), plan.top_k, bool(need_dx), bool(need_dw))
     return _opt(dx, need_dx), _opt(dw1, need_dw), _opt(dw3, need_dw), _opt(dw2, need_dw), dweights
+
+
+# ====================================================================== the whole block
+_moe_block = _O.moe_block.default
+_COVERS: dict = {}
+
+
+def route_plan_covers(num_experts, top_k, num_groups) -> bool:
+    """Whether the one-pass selection + plan, and with it ``moe_block``, serves this router."""
+    key = (num_experts, top_k, num_groups)
+    covers = _COVERS.get(key)
+    if covers is None:
+        covers = _COVERS[key] = bool(
+            _lib.load().mi355_route_plan_covers(int(num_experts), int(top_k), int(num_groups or 0), SELECT_TOPK))
+    return covers
+
+
+def moe_block(x_TD, gate_w_ED, gate_bias_E, expert_bias_E, w1_EFD, w3_EFD, w2_EDF, shared, top_k, score_func, route_norm,
+              route_scale, num_groups, num_limited, local_lo, local_hi, align, round_terms, overlap_shared):
+    """The block of ``moe.MoE`` as one operator: ``(output, int32 counts per expert)``, differentiable in the
+    tokens and every weight.  ``shared``: the shared expert's (gate, up, down) weights or three Nones."""
+    return _moe_block(x_TD, gate_w_ED, gate_bias_E, expert_bias_E, w1_EFD, w3_EFD, w2_EDF, *shared, top_k,
+                      SCORE_FUNCS[score_func], route_norm, route_scale, num_groups or 0, num_limited or 0, local_lo,
+                      local_hi, align, round_terms, overlap_shared)
 
 
 # ====================================================================== profiling hooks
