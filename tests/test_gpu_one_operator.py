@@ -74,3 +74,28 @@ def test_gate_projection_of_few_tokens_matches_fp64(dtype, T, D, E):
     # fp32 sums of D products: the error of a plain fp32 dot product bounds it
     scale = (x.double().abs() @ w.double().abs().T + b.double().abs()).max()
     assert float((got - want).abs().max()) < 4e-7 * float(scale)
+
+
+@pytest.mark.parametrize("counts,D,F", [
+    ([1], 384, 384), ([0, 3, 0, 16], 448, 576), ([17, 0, 1, 15, 7], 512, 1024), ([2] * 40, 2048, 384), ([64], 384, 832)])
+def test_forward_experts_of_few_rows_match_fp32(counts, D, F):
+    """A handful of rows per expert (csrc/grouped_few.hip): one row, exactly 16 and one more, experts
+    without rows, contractions whose steps do not divide by the four waves."""
+    from torchllmtuner_amd import ops
+
+    print(f"few rows {counts} D={D} F={F}", flush=True)
+    g = torch.Generator().manual_seed(D + F)
+    R_, E = sum(counts), len(counts)
+    x = torch.randn(R_, D, generator=g).bfloat16()
+    w1, w3, w2 = (torch.randn(E, *s, generator=g).mul(0.05).bfloat16() for s in ((F, D), (F, D), (D, F)))
+    plan = ops.segments_from_counts(torch.tensor(counts, dtype=torch.int32, device=DEV), R_)
+    y, gate, up, h = ops.grouped_swiglu_fwd(x.to(DEV), w1.to(DEV), w3.to(DEV), w2.to(DEV), plan)
+    seg = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))
+    xf = x.float()
+    want_g = torch.stack([w1[e].float() @ xf[r] for r, e in enumerate(seg)])
+    want_u = torch.stack([w3[e].float() @ xf[r] for r, e in enumerate(seg)])
+    want_h = (torch.nn.functional.silu(want_g.bfloat16().float()).bfloat16().float() * want_u.bfloat16().float())
+    want_y = torch.stack([w2[e].float() @ h[r].float().cpu() for r, e in enumerate(seg)])
+    for name, got, want in (("gate", gate, want_g), ("up", up, want_u), ("h", h, want_h), ("y", y, want_y)):
+        err = float((got.float().cpu() - want).norm() / want.norm())
+        assert err < 4e-3, f"{name}: rel-L2 {err}"

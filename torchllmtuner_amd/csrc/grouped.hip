@@ -18,8 +18,8 @@ inline int tile_m_for(int dtype) { (void)dtype; return bf16_row_tile_m(); }
 int bf16_grouped_fwd(const void* rows, const int32_t* token_of_row, int64_t num_tokens, const void* w1,
                      const void* w3, const void* w2, const int32_t* seg_offsets, const int32_t* seg_counts,
                      const int32_t* tile_expert, const int32_t* tile_row0, const int32_t* num_tiles,
-                     int64_t tile_capacity, void* gate, void* up, void* h, void* y, int64_t D,
-                     int64_t F, int stages, hipStream_t s);
+                     int64_t tile_capacity, void* gate, void* up, void* h, void* y, int64_t El, int64_t D,
+                     int64_t F, int64_t row_capacity, int stages, hipStream_t s);
 int bf16_fused_dot_slots(int64_t F);
 int bf16_grouped_linear_dx(const void* dy, const void* w, const int32_t* seg_offsets, const int32_t* seg_counts,
                            const int32_t* tile_expert, const int32_t* tile_row0, const int32_t* num_tiles,
@@ -185,7 +185,7 @@ extern "C" int mi355_grouped_swiglu_fwd(const void* rows, const int32_t* token_o
   hipStream_t s = as_stream(stream);
   if (fast)
     return bf16_grouped_fwd(rows, token_of_row, num_tokens, w1, w3, w2, seg_offsets, seg_counts, tile_expert,
-                            tile_row0, num_tiles, tile_capacity, gate, up, h, y, D, F, 3, s);
+                            tile_row0, num_tiles, tile_capacity, gate, up, h, y, El, D, F, row_capacity, 3, s);
   if (token_of_row)
     return fail(MI355_EUNSUP, "grouped_swiglu_fwd: the token gather needs bf16 with D and F multiples of 64; "
                               "materialise the rows with mi355_permute_rows_fwd instead");
@@ -279,7 +279,7 @@ extern "C" int mi355_grouped_swiglu_stage(int stage, const void* dy, const void*
   hipStream_t s = as_stream(stream);
   if (stage <= 2)
     return bf16_grouped_fwd(rows, token_of_row, num_tokens, w1, w3, w2, seg_offsets, seg_counts, tile_expert,
-                            tile_row0, num_tiles, tile_capacity, gate, up, h, y, D, F, stage, s);
+                            tile_row0, num_tiles, tile_capacity, gate, up, h, y, El, D, F, row_capacity, stage, s);
   return bf16_grouped_bwd(
       dy, rows, token_of_row, num_tokens, w1, w3, w2, gate, up, h, nullptr, nullptr, seg_offsets, seg_counts,
       tile_expert, tile_row0, num_tiles, tile_capacity, dgate, dup, drows, dw1, dw3, dw2, El, D, F, stage, s);
@@ -299,7 +299,8 @@ extern "C" int mi355_grouped_linear_fwd(const void* x, const void* w, int dtype,
   if (dtype == MI355_BF16 && bf16_fast_path_ok(O, I))
     // the down projection's kernel is this product: rows (R, I) . w[e] (O, I)^T
     return bf16_grouped_fwd(nullptr, nullptr, 0, nullptr, nullptr, w, seg_offsets, seg_counts, tile_expert, tile_row0,
-                            num_tiles, tile_capacity, nullptr, nullptr, const_cast<void*>(x), y, O, I, 2, s);
+                            num_tiles, tile_capacity, nullptr, nullptr, const_cast<void*>(x), y, El, O, I, row_capacity, 2,
+                            s);
   const Seg sg{seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity};
   // B(k=i, n=o) = w[e][o][i]
   return rowseg(sg, x, I, w, 1, I, O * I, y, O, I, dtype, 0, s);

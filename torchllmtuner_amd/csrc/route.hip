@@ -35,37 +35,68 @@ struct PlanOut {
 
 // Integer arrays in LDS for the layout step, E experts.
 struct LayoutLds {
-  int32_t *count, *before, *seg, *tile, *order;
+  int32_t *count, *before, *seg, *tile, *order, *wave_sums;
   __device__ LayoutLds(int32_t* base, int E)
-      : count(base), before(base + E), seg(base + 2 * E), tile(base + 3 * E + 1), order(base + 4 * E + 2) {}
+      : count(base), before(base + E), seg(base + 2 * E), tile(base + 3 * E + 1), order(base + 4 * E + 2),
+        wave_sums(base + 5 * E + 2) {}
 };
-constexpr int layout_words(int E) { return 5 * E + 3; }
+constexpr int layout_words(int E) { return 5 * E + 2 + 8; }
+
+// inclusive sum over the wave
+__device__ __forceinline__ int wave_scan(int v, int lane) {
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const int below = __shfl_up(v, o, kWave);
+    v += lane >= o ? below : 0;
+  }
+  return v;
+}
 
 // counts -> padded segment offsets, tiles before each local expert, rank by descending count; left in
-// LDS for all lanes (ends on a barrier).  Each of the El + 1 sums is shared by several lanes.
+// LDS for all lanes (ends on a barrier).  One lane per local expert (at most 256: four waves) scans
+// rows and tiles; the ranks, one comparison per pair of experts, are shared by all lanes.
 __device__ void plan_layout(const LayoutLds& s, const PlanOut& p, bool lists) {
-  const int El = p.hi - p.lo, tid = threadIdx.x;
-  for (int j = tid; j <= El; j += kLanes) s.seg[j] = s.tile[j] = s.order[j] = 0;
-  __syncthreads();
-  const int sums = El + 1;
-  const int lanes_per_sum = max(1, kLanes / sums);
-  const int slice = (El + lanes_per_sum - 1) / lanes_per_sum;
-  for (int idx = tid; idx < sums * lanes_per_sum; idx += kLanes) {
-    const int j = idx % sums, o0 = (idx / sums) * slice, o1 = min(El, o0 + slice);
-    const int c = j < El ? s.count[p.lo + j] : 0;
-    int off = 0, toff = 0, rank = 0;
-#pragma unroll 4
-    for (int o = o0; o < o1; ++o) {
-      const bool below = o < j;
-      const int co = s.count[p.lo + o];
-      off += below ? (co + p.align - 1) / p.align * p.align : 0;
-      toff += below ? (co + p.tile_m - 1) / p.tile_m : 0;
-      rank += (co > c || (co == c && below)) ? 1 : 0;
+  const int El = p.hi - p.lo, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lanes = blockDim.x;
+  for (int j = tid; j < El; j += lanes) s.order[j] = 0;
+  int rows = 0, tiles = 0, rows_to = 0, tiles_to = 0;
+  if (wave < 4) {
+    const int c = tid < El ? s.count[p.lo + tid] : 0;
+    rows = p.align > 1 ? (c + p.align - 1) / p.align * p.align : c;
+    tiles = (c + p.tile_m - 1) / p.tile_m;
+    rows_to = wave_scan(rows, lane);
+    tiles_to = wave_scan(tiles, lane);
+    if (lane == 63) {
+      s.wave_sums[wave] = rows_to;
+      s.wave_sums[4 + wave] = tiles_to;
     }
-    atomicAdd(&s.seg[j], off);
-    if (lists) {
-      atomicAdd(&s.tile[j], toff);
-      atomicAdd(&s.order[j], rank);
+  }
+  __syncthreads();
+  if (wave < 4) {
+    for (int w = 0; w < wave; ++w) {
+      rows_to += s.wave_sums[w];
+      tiles_to += s.wave_sums[4 + w];
+    }
+    if (tid < El) {
+      s.seg[tid] = rows_to - rows;
+      s.tile[tid] = tiles_to - tiles;
+      if (tid == El - 1) {
+        s.seg[El] = rows_to;
+        s.tile[El] = tiles_to;
+      }
+    }
+  }
+  if (lists) {
+    const int shares = max(1, lanes / El), slice = (El + shares - 1) / shares;
+    for (int idx = tid; idx < El * shares; idx += lanes) {
+      const int j = idx % El, o0 = (idx / El) * slice, o1 = min(El, o0 + slice);
+      const int c = s.count[p.lo + j];
+      int rank = 0;
+#pragma unroll 4
+      for (int o = o0; o < o1; ++o) {
+        const int co = s.count[p.lo + o];
+        rank += (co > c || (co == c && o < j)) ? 1 : 0;
+      }
+      if (rank) atomicAdd(&s.order[j], rank);
     }
   }
   __syncthreads();
@@ -83,7 +114,7 @@ __device__ void write_lists(const LayoutLds& s, const PlanOut& p, int E) {
     const int c = s.count[p.lo + j];
     p.seg_counts[j] = c;
     p.seg_counts[El + s.order[j]] = j;
-    const int nt = (c + p.tile_m - 1) / p.tile_m, rows = even_tile_rows(c, p.tile_m);
+    const int nt = s.tile[j + 1] - s.tile[j], rows = even_tile_rows(c, p.tile_m);
     for (int i = 0; i < nt; ++i) {
       const int at = s.tile[j] + i;
       if (at < p.tile_capacity) {
@@ -141,8 +172,8 @@ __global__ __launch_bounds__(kLanes) void route_rank_kernel(
     const int t0 = (blockIdx.x * chunks + c) * kRows;
     if (t0 >= T) break;  // workgroup-uniform
     for (int i = tid; i < kWaves * E; i += kLanes) cnt[i] = 0;
-    // ---- selection: one token per row of 16 lanes
-    {
+    // ---- selection: one token per row of 16 lanes; waves without a token have nothing to select
+    if (t0 + (wave << 2) < T) {
       const int t_raw = t0 + (tid >> 4);
       const bool live = t_raw < T;
       const int t = live ? t_raw : T - 1;
@@ -176,8 +207,10 @@ __global__ __launch_bounds__(kLanes) void route_rank_kernel(
       }
     }
     __syncthreads();
+    // (the ids of the chunk's missing tokens were not written: their slots are past T * K)
     // ---- rank of each slot among the chunk's earlier slots of its expert
-    const bool slot_here = tid < kRows * K;
+    const int slot = t0 * K + tid;
+    const bool slot_here = tid < kRows * K && slot < T * K;
     const int e = slot_here ? id_sh[tid] : 0xffff;
     const bool valid = e != 0xffff;
     unsigned long long same = __ballot(valid);
@@ -204,8 +237,7 @@ __global__ __launch_bounds__(kLanes) void route_rank_kernel(
     __syncthreads();
     my_e = valid ? e : -1;
     my_rank = valid ? cnt[wave * E + e] + below : 0;
-    const int slot = t0 * K + tid;
-    if (!single && slot_here && slot < T * K) rank_in_block[slot] = static_cast<uint32_t>(my_rank);
+    if (!single && slot_here) rank_in_block[slot] = static_cast<uint32_t>(my_rank);
     if (c + 1 < chunks) __syncthreads();  // cnt and id_sh are reused
   }
   if (!single) {
