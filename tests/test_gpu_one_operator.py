@@ -99,3 +99,54 @@ def test_forward_experts_of_few_rows_match_fp32(counts, D, F):
     for name, got, want in (("gate", gate, want_g), ("up", up, want_u), ("h", h, want_h), ("y", y, want_y)):
         err = float((got.float().cpu() - want).norm() / want.norm())
         assert err < 4e-3, f"{name}: rel-L2 {err}"
+
+
+@pytest.mark.parametrize("dtype,counts,D,F", [
+    (torch.float32, [1, 0, 65], 4, 8), (torch.float32, [130, 3], 68, 36), (torch.float32, [200, 57, 300], 132, 260),
+    (torch.bfloat16, [1, 0, 65], 4, 8), (torch.bfloat16, [130, 3], 68, 36), (torch.bfloat16, [0, 257], 124, 380),
+    (torch.float32, [700] * 12, 640, 516), (torch.bfloat16, [700] * 12, 652, 644)])
+def test_experts_of_any_width_match_fp64(dtype, counts, D, F):
+    """csrc/grouped_any.hip, forward and backward: contractions and columns that end inside a tile, empty
+    experts, segments that end inside a row tile; the last two sizes take the large tiles."""
+    from torchllmtuner_amd import ops
+
+    print(f"any width {dtype} {counts[:4]} D={D} F={F}", flush=True)
+    g = torch.Generator().manual_seed(D + F)
+    R_, E = sum(counts), len(counts)
+    mk = lambda *s, std=0.05: torch.randn(*s, generator=g).mul(std).to(dtype)
+    x, dy = mk(R_, D, std=1.0), mk(R_, D, std=1.0)
+    w1, w3, w2 = mk(E, F, D), mk(E, F, D), mk(E, D, F)
+    dev = [t.to(DEV) for t in (x, w1, w3, w2)]
+    plan = ops.segments_from_counts(torch.tensor(counts, dtype=torch.int32, device=DEV), R_)
+    y, gate, up, h = ops.grouped_swiglu_fwd(*dev, plan)
+    dx, dw1, dw3, dw2 = ops.grouped_swiglu_bwd(dy.to(DEV), *dev, gate, up, h, plan)
+    only_dx = ops.grouped_swiglu_bwd(dy.to(DEV), *dev, gate, up, h, plan, need_dw=False)[0]
+    assert torch.equal(only_dx, dx)
+    ref = [t.double().requires_grad_() for t in (x, w1, w3, w2)]
+    out, r0 = [], 0
+    for e, c in enumerate(counts):
+        xe = ref[0][r0:r0 + c]
+        out.append((torch.nn.functional.silu(xe @ ref[1][e].T) * (xe @ ref[2][e].T)) @ ref[3][e].T)
+        r0 += c
+    want = torch.cat(out)
+    want.backward(dy.double())
+    tol = 2e-6 if dtype == torch.float32 else 1e-2
+    for name, got, exp in (("y", y.detach(), want.detach()), ("dx", dx, ref[0].grad), ("dw1", dw1, ref[1].grad), ("dw3", dw3, ref[2].grad),
+                           ("dw2", dw2, ref[3].grad)):
+        err = float((got.double().cpu() - exp).norm() / exp.norm())
+        assert err < tol, f"{name}: rel-L2 {err}"
+
+
+@pytest.mark.parametrize("dtype,T,D,E", [(torch.bfloat16, 1, 8, 2), (torch.bfloat16, 1531, 324, 17), (torch.float32, 33, 260, 32),
+                                         (torch.float32, 4097, 256, 8)])
+def test_gate_gradients_of_few_experts_match_fp64(dtype, T, D, E):
+    from torchllmtuner_amd import ops
+
+    print(f"gate backward {dtype} T={T} D={D} E={E}", flush=True)
+    g = torch.Generator().manual_seed(T)
+    x, w, dl = torch.randn(T, D, generator=g).to(dtype), torch.randn(E, D, generator=g), torch.randn(T, E, generator=g)
+    dx, dw = ops.router_gate_bwd(dl.to(DEV), x.to(DEV), w.to(DEV))
+    for name, got, exp, tol in (("dx", dx, dl.double() @ w.double(), 1e-6 if dtype == torch.float32 else 4e-3),
+                                ("dw", dw, dl.double().T @ x.double(), 1e-6)):
+        err = float((got.double().cpu() - exp).norm() / exp.norm())
+        assert err < tol, f"{name}: rel-L2 {err}"

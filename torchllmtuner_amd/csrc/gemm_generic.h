@@ -56,6 +56,11 @@ int launch_splitk_reduce(const float* partial, void* out, int out_dtype, int64_t
 // tokens, fp32 weights, D and E multiples of 64.
 bool router_x3_ok(int x_dtype, int w_dtype, int64_t D, int64_t E);
 int64_t router_x3_bwd_workspace(int64_t T, int64_t D, int64_t E);
+// Backward for few experts, fp32 weights, D a multiple of four: both gradients in one launch (dx, dw: null = skip).
+bool router_few_ok(int x_dtype, int w_dtype, int64_t D, int64_t E);
+int64_t router_few_bwd_workspace(int64_t T, int64_t D, int64_t E);
+int router_few_bwd(const float* dlogits, const void* x, int x_dtype, const float* w, const void* addend, void* dx, float* dw,
+                   void* workspace, int64_t T, int64_t D, int64_t E, hipStream_t s);
 // Forward: `splits` (T, E) partial sums of the contraction, to be added in order (with the bias,
 // unless splits is 1: then it is added already and the one partial is the logits); 0 = no kernel
 // of that file serves the case.  `pieces` is scratch of router_fwd_pieces_bytes.

@@ -326,7 +326,16 @@ __global__ void splitk_reduce_kernel(const float* __restrict__ partial, TC* __re
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= MN) return;
   float s = 0.0f;
-  for (int z = 0; z < ksplit; ++z) s += partial[z * MN + i];
+  constexpr int B = 8;  // loads in flight; added in split order all the same
+  int z = 0;
+  for (; z + B <= ksplit; z += B) {
+    float v[B];
+#pragma unroll
+    for (int b = 0; b < B; ++b) v[b] = partial[(z + b) * MN + i];
+#pragma unroll
+    for (int b = 0; b < B; ++b) s += v[b];
+  }
+  for (; z < ksplit; ++z) s += partial[z * MN + i];
   store_from_f32(out + i, s);
 }
 

@@ -1,11 +1,13 @@
 // Grouped SwiGLU experts: C entry points and the generic (any dtype, any shape)
-// path.  bf16 problems whose D and F are multiples of 64 go to the MFMA kernels of
-// grouped_bf16.hip; everything else (fp32, fp64, odd shapes) runs the strided GEMM of
-// gemm_generic.hip (fp32 MFMA; fp64 MFMA for fp64) plus two small elementwise kernels.
+// path.  bf16 problems whose D and F are multiples of 64 (>= 384) go to the MFMA kernels of
+// grouped_bf16.hip, other bf16 and fp32 problems with D and F multiples of 4 to grouped_any.hip;
+// the rest (fp64, odd widths) runs the strided GEMM of gemm_generic.hip (fp32 MFMA; fp64 MFMA for
+// fp64) plus two small elementwise kernels.
 #include <cstdlib>
 
 #include "common.h"
 #include "gemm_generic.h"
+#include "grouped_any.h"
 
 namespace mi355 {
 
@@ -189,6 +191,11 @@ extern "C" int mi355_grouped_swiglu_fwd(const void* rows, const int32_t* token_o
   if (token_of_row)
     return fail(MI355_EUNSUP, "grouped_swiglu_fwd: the token gather needs bf16 with D and F multiples of 64; "
                               "materialise the rows with mi355_permute_rows_fwd instead");
+  if (any_path_ok(dtype, D, F, row_capacity)) {
+    const AnySeg g{seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity, El};
+    if (int rc = any_gateup(g, dtype, rows, w1, w3, gate, up, h, D, F, row_capacity, s)) return rc;
+    return any_linear(g, dtype, h, w2, y, F, D, row_capacity, s);
+  }
   const Seg sg{seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity};
   // gate/up: B(k=d, n=f) = w[e][f][d]
   if (int rc = rowseg(sg, rows, D, w1, 1, D, F * D, gate, F, D, dtype, 0, s)) return rc;
@@ -234,6 +241,19 @@ extern "C" int mi355_grouped_swiglu_bwd(const void* dy, const void* rows,
   // (with no rows at all nothing is gathered: only the zero weight gradients remain to be written)
   if (token_of_row && row_capacity > 0 && tile_capacity > 0)
     return fail(MI355_EUNSUP, "grouped_swiglu_bwd: the token gather needs bf16 with D and F multiples of 64");
+  if (any_path_ok(dtype, D, F, row_capacity)) {
+    const AnySeg g{seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity, El};
+    const bool some = row_capacity > 0 && tile_capacity > 0;
+    if (some)
+      if (int rc = any_dh(g, dtype, dy, w2, gate, up, dgate, dup, D, F, row_capacity, s)) return rc;
+    // the weight gradients also cover the no-rows case: every expert's gradient is written (zeros)
+    AnyGrad grads[3];
+    int count = 0;
+    if (dw2) grads[count++] = {dy, h, dw2, D, F};
+    if (dw1) grads[count++] = {dgate, rows, dw1, F, D};
+    if (dw3) grads[count++] = {dup, rows, dw3, F, D};
+    return any_backward(g, dtype, dgate, dup, w1, w3, some ? drows : nullptr, D, F, grads, count, row_capacity, s);
+  }
   const Seg sg{seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity};
   if (row_capacity > 0 && tile_capacity > 0) {
     // dh = dy . w2[e]: B(k=d, n=f) = w2[e][d][f]   (lands in dgate, rewritten in place below)
@@ -301,6 +321,9 @@ extern "C" int mi355_grouped_linear_fwd(const void* x, const void* w, int dtype,
     return bf16_grouped_fwd(nullptr, nullptr, 0, nullptr, nullptr, w, seg_offsets, seg_counts, tile_expert, tile_row0,
                             num_tiles, tile_capacity, nullptr, nullptr, const_cast<void*>(x), y, El, O, I, row_capacity, 2,
                             s);
+  if (any_path_ok(dtype, I, O, row_capacity))
+    return any_linear({seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity, El}, dtype, x, w, y, I, O,
+                      row_capacity, s);
   const Seg sg{seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity};
   // B(k=i, n=o) = w[e][o][i]
   return rowseg(sg, x, I, w, 1, I, O * I, y, O, I, dtype, 0, s);
@@ -328,6 +351,13 @@ extern "C" int mi355_grouped_linear_bwd(const void* dy, const void* x, const voi
                               seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity, nullptr,
                               nullptr, nullptr, nullptr, nullptr, dw, El, O, I, 16, s);
     return MI355_OK;
+  }
+  if (any_path_ok(dtype, I, O, row_capacity)) {
+    const AnySeg g{seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity, El};
+    if (dx && rows)
+      if (int rc = any_linear_dx(g, dtype, dy, w, dx, I, O, row_capacity, s)) return rc;
+    const AnyGrad grad{dy, x, dw, O, I};
+    return any_backward(g, dtype, nullptr, nullptr, nullptr, nullptr, nullptr, I, O, &grad, dw ? 1 : 0, row_capacity, s);
   }
   // dx = dy . w[e]: B(k=o, n=i) = w[e][o][i]
   if (dx && rows)

@@ -1,0 +1,466 @@
+// Grouped expert products of any width: fp32, and bf16 whose widths are not on the 64-column grid (or
+// are below the 384 columns) of the kernels in grouped_bf16.hip.  Widths are multiples of four.
+//
+// One kernel template over the element type, the product and the tile: 256 lanes as 2 x 2 waves on a
+// TM x TN output tile, each wave (TM/2) x (TN/2) in 32x32 accumulators (v_mfma_f32_32x32x16_bf16, or
+// v_mfma_f32_32x32x2_f32 for fp32), 128 bytes of the contraction per step, two LDS stages, the next
+// step's operands held in registers.  Operands are fetched 16 bytes at a time whatever the width
+// (buffer loads: dword alignment suffices, and what lies past a matrix reads as zero); the tail of
+// the contraction is zeroed as it is parked.  LDS holds an operand as it lies in memory -- contraction
+// contiguous [row][128 B + 16] or strided [k][cols + pad], the pads chosen so that fragment reads
+// are free of bank conflicts -- and the fragment reads (b128, b32, or the transposing b64 for bf16)
+// make up for the difference.
+//   Products and their fused ends: gate and up in one pass with SwiGLU; down; dh with the SwiGLU
+// backward; drows as one contraction over both halves; all three weight gradients in one launch.
+//   What bounds them at the sizes they are for is latency: few tiles, short contractions.  Small tiles
+// (64 rows) are used until the large ones fill the chip.  Before, nine launches of a 64x64 tile fed by
+// scalar loads plus two elementwise passes did this: 512 tokens of 8 fp32 experts of 256 x 512, forward
+// and backward, 210 us of GPU time; 1531 tokens of 16 bf16 experts of 320 x 232, 543 us.
+#include <algorithm>
+#include <type_traits>
+
+#include "bf16_tiles.h"
+#include "common.h"
+#include "grouped_any.h"
+
+namespace mi355 {
+namespace {
+
+enum AnyMode { ANY_GATEUP, ANY_KC, ANY_DH, ANY_DX, ANY_KS, ANY_DW };
+
+struct AnyDw {  // c[e] (M, N) = a[segment e]^T (rows, M) . b[segment e] (rows, N)
+  const void *a, *b;
+  void* c;
+  int M, N, nt, first;  // column tiles; first block of the problem
+};
+
+struct AnyArgs {
+  const void *a0, *a1, *b0, *b1;  // rows; weights (El, ., .).  GATEUP: w1, w3; DX: dgate, dup and w1, w3
+  void *c0, *c1, *c2;             // GATEUP gate, up, h; DH dgate, dup
+  const void *gate, *up;          // DH
+  int K, N, ldb;                  // contraction (of one half), output columns, row length of the weights
+  int64_t rows, w_elems;          // rows of the buffers, elements of one expert's weights
+  const int32_t *seg_offsets, *seg_counts, *tile_expert, *tile_row0, *num_tiles;
+  int col_tiles;
+  AnyDw dw[3];
+  int num_dw;
+};
+
+template <typename T> struct El;
+template <> struct El<float> {
+  static constexpr int KS_PAD = 8;   // words: rows k and k + 4 half the banks apart
+  using V4 = f32x4;
+};
+template <> struct El<uint16_t> {
+  static constexpr int KS_PAD = 32;  // four consecutive k rows a quarter of the banks apart
+  using V4 = u32x2;
+};
+
+__device__ __forceinline__ f32x4 any_pack(float, float a, float b, float c, float d) { return {a, b, c, d}; }
+__device__ __forceinline__ u32x2 any_pack(uint16_t, float a, float b, float c, float d) { return {pack2(a, b), pack2(c, d)}; }
+__device__ __forceinline__ void any_unpack(const f32x4& v, float (&f)[4]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) f[i] = v[i];
+}
+__device__ __forceinline__ void any_unpack(const u32x2& v, float (&f)[4]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) f[i] = __uint_as_float(i & 1 ? v[i >> 1] & 0xffff0000u : v[i >> 1] << 16);
+}
+template <typename T>
+__device__ __forceinline__ float any_round(float v) {
+  if constexpr (sizeof(T) == 2) return round_bf16(v);
+  else return v;
+}
+
+// Buffer resource over [base, end) of a matrix, clipped to the 32-bit range of the offsets.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t any_rsrc(const void* base, int64_t bytes) {
+  const int64_t clipped = bytes < 0 ? 0 : bytes < 0xfffffffcll ? bytes : 0xfffffffcll;
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, static_cast<int>(static_cast<uint32_t>(clipped)), 0x00020000);
+}
+
+// One operand's tile: ROWS rows (or columns) of the output, one 128-byte step of the contraction.
+template <typename T, bool KS, int ROWS>
+struct Operand {
+  static constexpr int E = 16 / sizeof(T), BKE = 128 / sizeof(T);
+  static constexpr int PITCH = KS ? ROWS + El<T>::KS_PAD : BKE + E;
+  static constexpr int ELEMS = KS ? BKE * PITCH : ROWS * PITCH;
+  static constexpr int CPR = KS ? ROWS / E : 8;  // chunks per stored row
+  static constexpr int N = ROWS * 8 / 256;       // chunks per lane and step
+
+  static __device__ __forceinline__ int at(int tid, int i) {
+    const int q = tid + 256 * i;
+    return (q / CPR) * PITCH + (q % CPR) * E;
+  }
+  // keep what lies inside the contraction (kv of BKE elements); a multiple of four
+  static __device__ __forceinline__ u32x4 clip(const u32x4& v, int tid, int i, int kv) {
+    const int q = tid + 256 * i;
+    const int k = KS ? q / CPR : (q % CPR) * E;
+    u32x4 r = v;
+    const bool lo = k < kv, hi = KS || sizeof(T) == 4 ? lo : k + 4 < kv;
+    r[0] = lo ? r[0] : 0; r[1] = lo ? r[1] : 0;
+    r[2] = hi ? r[2] : 0; r[3] = hi ? r[3] : 0;
+    return r;
+  }
+};
+
+// Fragments of one 32-row block.  The weights' operand is the first of the MFMA, so that a lane holds four
+// consecutive columns of one output row.
+template <bool KS, int ROWS>
+__device__ __forceinline__ bf16x8 any_frag(const uint16_t* tile, int row, int kk, int lane) {
+  using O = Operand<uint16_t, KS, ROWS>;
+  if constexpr (!KS) {
+    return *reinterpret_cast<const bf16x8*>(tile + (row + (lane & 31)) * O::PITCH + kk * 16 + 8 * (lane >> 5));
+  } else {
+    const int g = lane >> 4, i = lane & 15;
+    const uint16_t* p = tile + (kk * 16 + 8 * (g >> 1) + (i >> 2)) * O::PITCH + row + 16 * (g & 1) + 4 * (i & 3);
+    const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(p));
+    const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(p + 4 * O::PITCH));
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  }
+}
+// fp32: the four values of k = 8 kk + 4 (lane / 32) ..
+template <bool KS, int ROWS>
+__device__ __forceinline__ f32x4 any_frag(const float* tile, int row, int kk, int lane) {
+  using O = Operand<float, KS, ROWS>;
+  const int k = 8 * kk + 4 * (lane >> 5);
+  if constexpr (!KS) return *reinterpret_cast<const f32x4*>(tile + (row + (lane & 31)) * O::PITCH + k);
+  f32x4 v;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v[j] = tile[(k + j) * O::PITCH + row + (lane & 31)];
+  return v;
+}
+__device__ __forceinline__ f32x16 any_mfma(const bf16x8& b, const bf16x8& a, const f32x16& acc) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, a, acc, 0, 0, 0);
+}
+__device__ __forceinline__ f32x16 any_mfma(const f32x4& b, const f32x4& a, f32x16 acc) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(b[j], a[j], acc, 0, 0, 0);
+  return acc;
+}
+
+// LDS of one instantiation
+template <typename T, int MODE, int TM, int TN>
+constexpr int any_lds() {
+  constexpr bool B_KS = MODE == ANY_DH || MODE == ANY_DX || MODE == ANY_KS || MODE == ANY_DW;
+  return 2 * (Operand<T, MODE == ANY_DW, TM>::ELEMS + Operand<T, B_KS, TN>::ELEMS);
+}
+
+template <typename T, int MODE, int TM, int TN>
+__device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
+  constexpr bool A_KS = MODE == ANY_DW, B_KS = MODE == ANY_DH || MODE == ANY_DX || MODE == ANY_KS || MODE == ANY_DW;
+  using OA = Operand<T, A_KS, TM>;
+  using OB = Operand<T, B_KS, TN>;
+  constexpr int BKE = OA::BKE, MI = TM / 64, NJ = TN / 64, KK = 128 / sizeof(T) / (sizeof(T) == 2 ? 16 : 8);
+  constexpr int STAGE = OA::ELEMS + OB::ELEMS;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm = (wave >> 1) * (TM / 2), wn = (wave & 1) * (TN / 2);
+
+  // ---- which tile
+  int m_valid, n0, N = p.N, M = 0, m0 = 0, K = p.K, k_rows = 0;
+  int64_t row0 = 0;
+  const T *A0, *A1 = nullptr, *B0, *B1 = nullptr;
+  T *C0 = static_cast<T*>(p.c0);
+  int lda = p.K, ldb = p.ldb;
+  int64_t a_bytes, b_bytes;
+  if constexpr (MODE == ANY_DW) {
+    int d = 0;
+    while (d + 1 < p.num_dw && block >= p.dw[d + 1].first) ++d;
+    const AnyDw& w = p.dw[d];
+    const int local = block - w.first;
+    const int mt = (w.M + TM - 1) / TM, per = mt * w.nt;
+    const int e = local / per, t = local - e * per;
+    M = w.M; N = w.N;
+    m0 = (t / w.nt) * TM;
+    n0 = (t % w.nt) * TN;
+    m_valid = min(TM, M - m0);
+    k_rows = p.seg_counts[e];
+    const int64_t first = p.seg_offsets[e];
+    lda = M; ldb = N; K = k_rows;
+    A0 = static_cast<const T*>(w.a) + first * M + m0;
+    B0 = static_cast<const T*>(w.b) + first * N + n0;
+    a_bytes = ((p.rows - first) * M - m0) * static_cast<int64_t>(sizeof(T));
+    b_bytes = ((p.rows - first) * N - n0) * static_cast<int64_t>(sizeof(T));
+    C0 = static_cast<T*>(w.c) + static_cast<int64_t>(e) * M * N;
+  } else {
+    constexpr int SUBS = 256 / TM;
+    const int slot = block / p.col_tiles, tile = slot / SUBS;
+    if (tile >= *p.num_tiles) return;
+    const int e = p.tile_expert[tile], cnt = p.seg_counts[e], seg0 = p.seg_offsets[e], top = p.tile_row0[tile];
+    const int end = min(top + even_tile_rows(cnt, 256), seg0 + cnt);
+    const int first = top + (slot % SUBS) * TM;
+    m_valid = min(TM, end - first);
+    if (m_valid <= 0) return;
+    row0 = first;
+    n0 = (block % p.col_tiles) * (MODE == ANY_GATEUP ? TN / 2 : TN);
+    A0 = static_cast<const T*>(p.a0) + row0 * lda;
+    a_bytes = (p.rows - row0) * lda * static_cast<int64_t>(sizeof(T));
+    if (MODE == ANY_DX) A1 = static_cast<const T*>(p.a1) + row0 * lda;
+    const int64_t w = e * p.w_elems + (B_KS ? n0 : static_cast<int64_t>(n0) * ldb);
+    B0 = static_cast<const T*>(p.b0) + w;
+    if (MODE == ANY_GATEUP || MODE == ANY_DX) B1 = static_cast<const T*>(p.b1) + w;
+    b_bytes = (p.w_elems - (w - e * p.w_elems)) * static_cast<int64_t>(sizeof(T));
+  }
+  const auto rsA0 = any_rsrc(A0, a_bytes), rsB0 = any_rsrc(B0, b_bytes);
+  const auto rsA1 = MODE == ANY_DX ? any_rsrc(A1, a_bytes) : rsA0;
+  const auto rsB1 = (MODE == ANY_GATEUP || MODE == ANY_DX) ? any_rsrc(B1, b_bytes) : rsB0;
+
+  // ---- operand offsets (bytes): fixed per lane, plus the step's
+  uint32_t offA[OA::N], offB[OB::N];
+#pragma unroll
+  for (int i = 0; i < OA::N; ++i) {
+    const int q = tid + 256 * i, r = q / OA::CPR, c = (q % OA::CPR) * OA::E;
+    offA[i] = (A_KS ? static_cast<uint32_t>(r) * lda + c : static_cast<uint32_t>(min(r, m_valid - 1)) * lda + c) * sizeof(T);
+  }
+  const int b_rows = (MODE == ANY_GATEUP ? TN / 2 : TN);  // KC: weight rows of the tile (of each of the two)
+#pragma unroll
+  for (int i = 0; i < OB::N; ++i) {
+    const int q = tid + 256 * i, r = q / OB::CPR, c = (q % OB::CPR) * OB::E;
+    offB[i] = (B_KS ? static_cast<uint32_t>(r) * ldb + c
+                    : static_cast<uint32_t>(min(r % b_rows, N - 1 - n0)) * ldb + c) * sizeof(T);
+  }
+  const int half_steps = (K + BKE - 1) / BKE, steps = MODE == ANY_DX ? 2 * half_steps : half_steps;
+  u32x4 ra[OA::N], rb[OB::N];
+  auto fetch = [&](int s) {
+    const bool second = MODE == ANY_DX && s >= half_steps;
+    const uint32_t k = static_cast<uint32_t>(second ? s - half_steps : s) * BKE;
+    const uint32_t ka = (A_KS ? k * lda : k) * sizeof(T), kb = (B_KS ? k * ldb : k) * sizeof(T);
+#pragma unroll
+    for (int i = 0; i < OA::N; ++i)
+      ra[i] = __builtin_amdgcn_raw_buffer_load_b128(second ? rsA1 : rsA0, offA[i] + ka, 0, 0);
+#pragma unroll
+    for (int i = 0; i < OB::N; ++i) {
+      const bool up = MODE == ANY_GATEUP && i >= OB::N / 2;
+      rb[i] = __builtin_amdgcn_raw_buffer_load_b128(second || up ? rsB1 : rsB0, offB[i] + kb, 0, 0);
+    }
+  };
+  auto park = [&](int s) {
+    T* As = smem + (s & 1) * STAGE;
+    T* Bs = As + OA::ELEMS;
+    const int kv = K - (MODE == ANY_DX && s >= half_steps ? s - half_steps : s) * BKE;
+    if (kv < BKE) {  // the tail: whatever was read past the contraction must not meet anything
+#pragma unroll
+      for (int i = 0; i < OA::N; ++i) ra[i] = OA::clip(ra[i], tid, i, kv);
+#pragma unroll
+      for (int i = 0; i < OB::N; ++i) rb[i] = OB::clip(rb[i], tid, i, kv);
+    }
+#pragma unroll
+    for (int i = 0; i < OA::N; ++i) *reinterpret_cast<u32x4*>(As + OA::at(tid, i)) = ra[i];
+#pragma unroll
+    for (int i = 0; i < OB::N; ++i) *reinterpret_cast<u32x4*>(Bs + OB::at(tid, i)) = rb[i];
+  };
+  // column block j of the wave: GATEUP's first half of the blocks are gate columns, the second the same of up
+  auto bcol = [&](int j) {
+    if constexpr (MODE == ANY_GATEUP) return (j < NJ / 2 ? 0 : TN / 2) + (wave & 1) * (TN / 4) + (j % (NJ / 2)) * 32;
+    else return wn + j * 32;
+  };
+  static_assert(MODE != ANY_GATEUP || NJ >= 2, "a wave of the gate/up product holds both of a column");
+
+  f32x16 acc[MI][NJ];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+  if (steps > 0) {
+    fetch(0);
+    park(0);
+    if (steps > 1) fetch(1);
+  }
+  __syncthreads();
+  for (int s = 0; s < steps; ++s) {
+    if (s + 1 < steps) park(s + 1);
+    if (s + 2 < steps) fetch(s + 2);
+    const T* As = smem + (s & 1) * STAGE;
+    const T* Bs = As + OA::ELEMS;
+#pragma unroll
+    for (int kk = 0; kk < KK; ++kk) {
+      decltype(any_frag<A_KS, TM>(As, 0, 0, 0)) af[MI];
+#pragma unroll
+      for (int i = 0; i < MI; ++i) af[i] = any_frag<A_KS, TM>(As, wm + i * 32, kk, lane);
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const auto bf = any_frag<B_KS, TN>(Bs, bcol(j), kk, lane);
+#pragma unroll
+        for (int i = 0; i < MI; ++i) acc[i][j] = any_mfma(bf, af[i], acc[i][j]);
+      }
+    }
+    __syncthreads();
+  }
+
+  // ---- epilogue: lane = output row lane & 31 of the block, four consecutive columns per q
+  using V4 = typename El<T>::V4;
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    const int m = wm + i * 32 + (lane & 31);
+    if (m >= m_valid) continue;
+#pragma unroll
+    for (int j = 0; j < (MODE == ANY_GATEUP ? NJ / 2 : NJ); ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int n = n0 + (MODE == ANY_GATEUP ? (wave & 1) * (TN / 4) : wn) + j * 32 + q * 8 + 4 * (lane >> 5);
+        if (n >= N) continue;  // N is a multiple of four
+        const int64_t at = (MODE == ANY_DW ? static_cast<int64_t>(m0 + m) : row0 + m) * N + n;
+        const f32x16& c = acc[i][j];
+        float v[4] = {c[q * 4], c[q * 4 + 1], c[q * 4 + 2], c[q * 4 + 3]};
+        if constexpr (MODE == ANY_GATEUP) {
+          const f32x16& cu = acc[i][j + NJ / 2];
+          float h[4], u[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            v[r] = any_round<T>(v[r]);
+            u[r] = any_round<T>(cu[q * 4 + r]);
+            h[r] = any_round<T>(v[r] / (1.0f + expf(-v[r]))) * u[r];
+          }
+          *reinterpret_cast<V4*>(C0 + at) = any_pack(T{}, v[0], v[1], v[2], v[3]);
+          *reinterpret_cast<V4*>(static_cast<T*>(p.c1) + at) = any_pack(T{}, u[0], u[1], u[2], u[3]);
+          *reinterpret_cast<V4*>(static_cast<T*>(p.c2) + at) = any_pack(T{}, h[0], h[1], h[2], h[3]);
+        } else if constexpr (MODE == ANY_DH) {
+          float g[4], u[4], dg[4], du[4];
+          any_unpack(*reinterpret_cast<const V4*>(static_cast<const T*>(p.gate) + at), g);
+          any_unpack(*reinterpret_cast<const V4*>(static_cast<const T*>(p.up) + at), u);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float dh = any_round<T>(v[r]);
+            const float sig = 1.0f / (1.0f + expf(-g[r]));
+            du[r] = dh * any_round<T>(g[r] * sig);
+            dg[r] = any_round<T>(dh * u[r]) * (sig * (1.0f + g[r] * (1.0f - sig)));
+          }
+          *reinterpret_cast<V4*>(C0 + at) = any_pack(T{}, dg[0], dg[1], dg[2], dg[3]);
+          *reinterpret_cast<V4*>(static_cast<T*>(p.c1) + at) = any_pack(T{}, du[0], du[1], du[2], du[3]);
+        } else {
+          *reinterpret_cast<V4*>(C0 + at) = any_pack(T{}, v[0], v[1], v[2], v[3]);
+        }
+      }
+  }
+}
+
+template <typename T, int MODE, int TM, int TN>
+__global__ __launch_bounds__(256) void any_kernel(AnyArgs p) {
+  __shared__ __attribute__((aligned(16))) T smem[any_lds<T, MODE, TM, TN>()];
+  any_tile<T, MODE, TM, TN>(p, blockIdx.x, smem);
+}
+
+// The input gradient and the weight gradients of a backward pass read the same buffers and write different
+// ones: with few tiles each they share a launch (at 512 fp32 tokens of 8 experts 26 + 16 us one after the
+// other).  The input gradient, the longer contraction, starts first.
+template <typename T, int TM>
+__global__ __launch_bounds__(256) void any_dx_dw_kernel(AnyArgs dx, AnyArgs dw, int dx_blocks) {
+  constexpr int A = any_lds<T, ANY_DX, TM, TM>(), B = any_lds<T, ANY_DW, TM, TM>();
+  __shared__ __attribute__((aligned(16))) T smem[A > B ? A : B];
+  if (static_cast<int>(blockIdx.x) < dx_blocks) any_tile<T, ANY_DX, TM, TM>(dx, blockIdx.x, smem);
+  else any_tile<T, ANY_DW, TM, TM>(dw, blockIdx.x - dx_blocks, smem);
+}
+
+template <int MODE, int TM, int TN>
+int launch_any(const AnyArgs& p, int dtype, int64_t blocks, hipStream_t s, const char* what) {
+  if (blocks <= 0) return MI355_OK;
+  if (dtype == MI355_F32) hipLaunchKernelGGL((any_kernel<float, MODE, TM, TN>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+  else hipLaunchKernelGGL((any_kernel<uint16_t, MODE, TM, TN>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+  return check_launch(what);
+}
+
+// Large tiles (128 x 128) once they give two workgroups for every CU; before that small ones (64 rows), whose
+// count is four times as large.
+bool rows_large(const AnyArgs& p, int64_t El, int64_t cols) {
+  return (p.rows / 128 + std::min(El, p.rows)) * ((cols + 127) / 128) >= 512;
+}
+
+template <int MODE>
+int launch_rows(AnyArgs& p, int dtype, int64_t tile_capacity, int64_t El, int64_t cols, hipStream_t s, const char* what) {
+  constexpr bool GU = MODE == ANY_GATEUP;
+  if (rows_large(p, El, cols)) {
+    p.col_tiles = (int)((cols + (GU ? 63 : 127)) / (GU ? 64 : 128));
+    return launch_any<MODE, 128, 128>(p, dtype, tile_capacity * 2 * p.col_tiles, s, what);
+  }
+  p.col_tiles = (int)((cols + 63) / 64);
+  return launch_any<MODE, 64, GU ? 128 : 64>(p, dtype, tile_capacity * 4 * p.col_tiles, s, what);
+}
+
+int64_t dw_tiles(AnyArgs& p, int64_t El, int tile) {
+  int64_t blocks = 0;
+  for (int d = 0; d < p.num_dw; ++d) {
+    AnyDw& w = p.dw[d];
+    w.nt = (w.N + tile - 1) / tile;
+    w.first = (int)blocks;
+    blocks += El * ((w.M + tile - 1) / tile) * w.nt;
+  }
+  return blocks;
+}
+
+}  // namespace
+
+// (a matrix of rows and an expert's weights within the 32-bit range of the operand offsets)
+bool any_path_ok(int dtype, int64_t D, int64_t F, int64_t R) {
+  return (dtype == MI355_F32 || dtype == MI355_BF16) && D % 4 == 0 && F % 4 == 0 &&
+         std::max(R * std::max(D, F), D * F) * (dtype == MI355_F32 ? 4 : 2) < (int64_t{1} << 32) - 4;
+}
+
+static AnyArgs any_args(const AnySeg& g, int64_t rows) {
+  AnyArgs p{};
+  p.rows = rows;
+  p.seg_offsets = g.seg_offsets; p.seg_counts = g.seg_counts; p.tile_expert = g.tile_expert;
+  p.tile_row0 = g.tile_row0; p.num_tiles = g.num_tiles;
+  return p;
+}
+
+int any_gateup(const AnySeg& g, int dtype, const void* rows, const void* w1, const void* w3, void* gate, void* up, void* h,
+               int64_t D, int64_t F, int64_t R, hipStream_t s) {
+  AnyArgs p = any_args(g, R);
+  p.a0 = rows; p.b0 = w1; p.b1 = w3; p.c0 = gate; p.c1 = up; p.c2 = h;
+  p.K = (int)D; p.N = (int)F; p.ldb = (int)D; p.w_elems = D * F;
+  return launch_rows<ANY_GATEUP>(p, dtype, g.tile_capacity, g.El, F, s, "grouped gate/up");
+}
+
+int any_linear(const AnySeg& g, int dtype, const void* x, const void* w, void* y, int64_t I, int64_t O, int64_t R,
+               hipStream_t s) {
+  AnyArgs p = any_args(g, R);
+  p.a0 = x; p.b0 = w; p.c0 = y;
+  p.K = (int)I; p.N = (int)O; p.ldb = (int)I; p.w_elems = I * O;
+  return launch_rows<ANY_KC>(p, dtype, g.tile_capacity, g.El, O, s, "grouped linear");
+}
+
+int any_linear_dx(const AnySeg& g, int dtype, const void* dy, const void* w, void* dx, int64_t I, int64_t O, int64_t R,
+                  hipStream_t s) {
+  AnyArgs p = any_args(g, R);
+  p.a0 = dy; p.b0 = w; p.c0 = dx;
+  p.K = (int)O; p.N = (int)I; p.ldb = (int)I; p.w_elems = I * O;
+  return launch_rows<ANY_KS>(p, dtype, g.tile_capacity, g.El, I, s, "grouped linear dx");
+}
+
+int any_dh(const AnySeg& g, int dtype, const void* dy, const void* w2, const void* gate, const void* up, void* dgate,
+           void* dup, int64_t D, int64_t F, int64_t R, hipStream_t s) {
+  AnyArgs p = any_args(g, R);
+  p.a0 = dy; p.b0 = w2; p.c0 = dgate; p.c1 = dup; p.gate = gate; p.up = up;
+  p.K = (int)D; p.N = (int)F; p.ldb = (int)F; p.w_elems = D * F;
+  return launch_rows<ANY_DH>(p, dtype, g.tile_capacity, g.El, F, s, "grouped dh");
+}
+
+int any_backward(const AnySeg& g, int dtype, const void* dgate, const void* dup, const void* w1, const void* w3, void* drows,
+                 int64_t D, int64_t F, const AnyGrad* grads, int count, int64_t R, hipStream_t s) {
+  AnyArgs p = any_args(g, R);
+  p.a0 = dgate; p.a1 = dup; p.b0 = w1; p.b1 = w3; p.c0 = drows;
+  p.K = (int)F; p.N = (int)D; p.ldb = (int)D; p.w_elems = D * F;
+  AnyArgs w = any_args(g, R);
+  for (int i = 0; i < count; ++i) w.dw[i] = {grads[i].a, grads[i].b, grads[i].c, (int)grads[i].M, (int)grads[i].N, 0, 0};
+  w.num_dw = count;
+  const bool dw_large = count && dw_tiles(w, g.El, 128) >= 512;
+  const int64_t tiles = count ? dw_tiles(w, g.El, dw_large ? 128 : 64) : 0;
+  MI355_REQUIRE(tiles < (1ll << 30), "grouped weight gradients: too many tiles");
+  if (drows && count && !dw_large && !rows_large(p, g.El, D)) {
+    p.col_tiles = (int)((D + 63) / 64);
+    const int64_t dx_blocks = g.tile_capacity * 4 * p.col_tiles;
+    MI355_REQUIRE(dx_blocks < (1ll << 30), "grouped drows: too many tiles");
+    const dim3 grid((unsigned)(dx_blocks + tiles));
+    if (dtype == MI355_F32) hipLaunchKernelGGL((any_dx_dw_kernel<float, 64>), grid, dim3(256), 0, s, p, w, (int)dx_blocks);
+    else hipLaunchKernelGGL((any_dx_dw_kernel<uint16_t, 64>), grid, dim3(256), 0, s, p, w, (int)dx_blocks);
+    return check_launch("grouped drows and weight gradients");
+  }
+  if (drows)
+    if (int rc = launch_rows<ANY_DX>(p, dtype, g.tile_capacity, g.El, D, s, "grouped drows")) return rc;
+  if (!count) return MI355_OK;
+  return dw_large ? launch_any<ANY_DW, 128, 128>(w, dtype, tiles, s, "grouped weight gradients")
+                  : launch_any<ANY_DW, 64, 64>(w, dtype, tiles, s, "grouped weight gradients");
+}
+
+}  // namespace mi355

@@ -13,8 +13,8 @@
 //     in kernels that hold the other operand anyway.
 // Every kernel and every rounding is the stage operators' own: both ways give the same bits.
 //
-// Memory.  Integers and fp32 of the plan and the router share one allocation (`meta`, kept for the
-// backward); everything else comes from PyTorch's allocator on the current stream.  Work on the
+// Memory.  From PyTorch's allocator on the current stream: the results one by one, what the backward
+// reads in one allocation, a pass's scratch in another.  Work on the
 // library's side streams is forked from the current stream and joined before the operator returns, so
 // buffers need no record_stream.
 #include <torch/csrc/autograd/custom_function.h>
@@ -55,6 +55,8 @@ struct Block {
   Config c;
   int64_t T, D, E, F, El, N, R, Fs, tile_m, tile_cap, shared_cap;
   int dt, gate_dt;
+  int splits;           // partial sums of the router's forward (0: the kernel without them)
+  int64_t piece_bytes;  // its weight pieces
   bool folded;         // the folded kernels (token gather, combine's backward inside the experts') serve the routed part
   bool shared_folded;  // the bf16 MFMA kernels serve the shared expert
 
@@ -69,45 +71,83 @@ struct Block {
     folded = mi355_grouped_combine_bwd_slots(dt, D, F) > 0 && T * D * 2 < (int64_t{1} << 32);
     Fs = sg.defined() ? sg.size(0) : 0;
     shared_cap = Fs > 0 ? (T + tile_m - 1) / tile_m : 0;
+    splits = mi355_router_gate_fwd_splits(dt, gate_dt, T, D, E);
+    piece_bytes = splits > 0 ? mi355_router_gate_fwd_pieces_bytes(dt, gate_dt, T, D, E) : 0;
     shared_folded = Fs > 0 && mi355_grouped_combine_bwd_slots(dt, D, Fs) > 0;
   }
 };
 
-// The plan's and the router's arrays inside `meta`.
-struct Meta {
+// Hands out 256-byte aligned pieces of one allocation.  With a null base it only measures.
+struct Carver {
+  char* base;
+  int64_t at = 0;
+  template <typename T>
+  T* take(int64_t n) {
+    T* p = reinterpret_cast<T*>(base + at);
+    at += (n * static_cast<int64_t>(sizeof(T)) + 255) / 256 * 256;
+    return base ? p : nullptr;
+  }
+  void* take(int64_t n, int64_t item) { return take<char>(n * item); }
+};
+
+// Runs `layout` twice, to measure and to hand out, around one allocation.
+template <typename Layout>
+Tensor carve(const Tensor& like, Layout layout) {
+  Carver measure{nullptr};
+  layout(measure);
+  Tensor t = bytes(measure.at, like);
+  Carver c{static_cast<char*>(t.data_ptr())};
+  layout(c);
+  return t;
+}
+
+// What the backward reads besides the inputs, in one allocation: the plan's and the router's arrays, the
+// activations, the shared expert's plan and activations.
+struct Kept {
   int64_t* ids;
   float *weights, *logits, *row_scale;
-  int32_t *counts, *seg_offsets, *seg_counts, *tile_expert, *tile_row0, *num_tiles, *row_of_slot, *slot_of_row,
-      *token_of_row;
+  int32_t *seg_offsets, *seg_counts, *tile_expert, *tile_row0, *num_tiles, *row_of_slot, *slot_of_row, *token_of_row;
   int32_t *s_offsets, *s_counts, *s_expert, *s_row0, *s_num;
-  int64_t bytes;
+  void *pieces = nullptr, *rows = nullptr, *gate = nullptr, *up = nullptr, *h = nullptr, *y = nullptr;
+  void *s_gate = nullptr, *s_up = nullptr, *s_h = nullptr;
 
-  Meta(const Block& b, void* base, int32_t* counts_E) : counts(counts_E) {
-    char* p = static_cast<char*>(base);
-    int64_t at = 0;
-    auto take = [&](auto*& out, int64_t n) {
-      using T = std::remove_reference_t<decltype(*out)>;
-      out = reinterpret_cast<T*>(p + at);
-      at += (n * static_cast<int64_t>(sizeof(T)) + 255) / 256 * 256;
-    };
-    take(ids, b.N);
-    take(weights, b.N);
-    take(logits, b.T * b.E);
-    take(row_scale, b.R);
-    take(row_of_slot, b.N);
-    take(slot_of_row, b.R);
-    take(token_of_row, b.R);
-    take(seg_offsets, b.El + 1);
-    take(seg_counts, 2 * b.El);
-    take(tile_expert, b.tile_cap);
-    take(tile_row0, b.tile_cap);
-    take(num_tiles, 1);
-    take(s_offsets, 2);
-    take(s_counts, 2);
-    take(s_expert, b.shared_cap);
-    take(s_row0, b.shared_cap);
-    take(s_num, 1);
-    bytes = at;
+  // save: someone will run the backward (else only what the forward itself needs is there)
+  void layout(Carver& c, const Block& b, bool save) {
+    const int64_t item = b.dt == MI355_F32 ? 4 : 2;
+    ids = c.take<int64_t>(b.N);
+    weights = c.take<float>(b.N);
+    logits = c.take<float>(b.T * b.E);
+    row_scale = c.take<float>(b.R);
+    row_of_slot = c.take<int32_t>(b.N);
+    slot_of_row = c.take<int32_t>(b.R);
+    token_of_row = c.take<int32_t>(b.R);
+    seg_offsets = c.take<int32_t>(b.El + 1);
+    seg_counts = c.take<int32_t>(2 * b.El);
+    tile_expert = c.take<int32_t>(b.tile_cap);
+    tile_row0 = c.take<int32_t>(b.tile_cap);
+    num_tiles = c.take<int32_t>(1);
+    if (b.piece_bytes > 0) pieces = c.take(b.piece_bytes, 1);
+    if (save || !b.folded) {  // (gate and up are the other kernels' own intermediates)
+      gate = c.take(b.R * b.F, item);
+      up = c.take(b.R * b.F, item);
+    }
+    if (!b.folded) {
+      rows = c.take(b.R * b.D, item);
+      h = c.take(b.R * b.F, item);
+      y = c.take(b.R * b.D, item);
+    }
+    if (b.Fs > 0) {
+      s_offsets = c.take<int32_t>(2);
+      s_counts = c.take<int32_t>(2);
+      s_expert = c.take<int32_t>(b.shared_cap);
+      s_row0 = c.take<int32_t>(b.shared_cap);
+      s_num = c.take<int32_t>(1);
+      s_h = c.take(b.T * b.Fs, item);
+      if (save || !b.shared_folded) {
+        s_gate = c.take(b.T * b.Fs, item);
+        s_up = c.take(b.T * b.Fs, item);
+      }
+    }
   }
 };
 
@@ -136,30 +176,40 @@ struct Fork {
   }
 };
 
-struct Kept {  // what the backward reads besides the inputs
-  Tensor meta, pieces, rows, gate, up, h, y, s_gate, s_up, s_h;
-};
-
-void shared_forward(const Block& b, const Meta& m, Kept& kept, const Tensor& y, bool save, void* stream) {
-  check(mi355_segments_dense(b.T, b.tile_m, m.s_offsets, m.s_counts, m.s_expert, m.s_row0, m.s_num, b.shared_cap, stream),
+void shared_forward(const Block& b, const Kept& k, void* y, void* stream) {
+  check(mi355_segments_dense(b.T, b.tile_m, k.s_offsets, k.s_counts, k.s_expert, k.s_row0, k.s_num, b.shared_cap, stream),
         "segments_dense");
-  // (gate and up are the generic kernels' own intermediates)
-  const bool gu = save || !b.shared_folded;
-  check(mi355_grouped_swiglu_fwd(ptr(b.x), nullptr, b.T, ptr(b.sg), ptr(b.su), ptr(b.sd), b.dt, m.s_offsets, m.s_counts,
-                                 m.s_expert, m.s_row0, m.s_num, b.shared_cap, gu ? ptr(kept.s_gate) : nullptr,
-                                 gu ? ptr(kept.s_up) : nullptr, ptr(kept.s_h), ptr(y), 1, b.D, b.Fs, b.T, stream),
+  check(mi355_grouped_swiglu_fwd(ptr(b.x), nullptr, b.T, ptr(b.sg), ptr(b.su), ptr(b.sd), b.dt, k.s_offsets, k.s_counts,
+                                 k.s_expert, k.s_row0, k.s_num, b.shared_cap, k.s_gate, k.s_up, k.s_h, y, 1, b.D, b.Fs,
+                                 b.T, stream),
         "shared expert");
 }
 
-std::tuple<Tensor, Tensor> block_forward(const Block& b, bool save, Kept& kept) {
+// (output, counts per expert, what the backward reads)
+std::tuple<Tensor, Tensor, Tensor> block_forward(const Block& b, bool save) {
   Launch L(b.x);
   const Config& c = b.c;
   const auto opts = b.x.options();
+  const int64_t item = b.dt == MI355_F32 ? 4 : 2;
   const hipStream_t main = static_cast<hipStream_t>(L.stream);
   Tensor counts = at::empty({b.E}, opts.dtype(at::kInt));
-  const int64_t meta_bytes = Meta(b, nullptr, nullptr).bytes;
-  kept.meta = bytes(meta_bytes, b.x);
-  const Meta m(b, kept.meta.data_ptr(), counts.data_ptr<int32_t>());
+  Tensor out = at::empty({b.T, b.D}, opts);
+  Kept k;
+  Tensor kept = carve(b.x, [&](Carver& cv) { k.layout(cv, b, save); });
+  // scratch of this call
+  const int64_t partial_bytes = b.splits > 1 ? b.splits * b.T * b.E * 4
+                                : b.splits == 0 ? mi355_router_gate_fwd_workspace_bytes(b.T, b.D, b.E) : 0;
+  const int64_t plan_bytes = mi355_route_plan_workspace_bytes(b.T, c.K, b.E);
+  void *gate_work = nullptr, *plan_work = nullptr, *y_shared = nullptr, *h = k.h, *y = k.y;
+  Tensor scratch = carve(b.x, [&](Carver& cv) {
+    if (partial_bytes > 0) gate_work = cv.take(partial_bytes, 1);
+    if (plan_bytes > 0) plan_work = cv.take(plan_bytes, 1);
+    if (b.Fs > 0) y_shared = cv.take(b.T * b.D, item);
+    if (b.folded) {
+      h = cv.take(b.R * b.F, item);
+      y = cv.take(b.R * b.D, item);
+    }
+  });
   Tensor gate_b, expert_b;
   if (b.gate_b.defined()) gate_b = cf(b.gate_b);
   if (b.expert_b.defined()) expert_b = cf(b.expert_b);
@@ -167,81 +217,44 @@ std::tuple<Tensor, Tensor> block_forward(const Block& b, bool save, Kept& kept) 
   // shared expert: beside the router and the routed experts when it may, else right before the sum
   SideStream* aux = b.Fs > 0 && c.overlap ? side_stream(b.x.device().index(), main, 1) : nullptr;
   Fork shared(aux, main);
-  Tensor y_shared;
-  if (b.Fs > 0) {
-    const bool gu = save || !b.shared_folded;
-    y_shared = at::empty({b.T, b.D}, opts);
-    kept.s_h = at::empty({b.T, b.Fs}, opts);
-    if (gu) {
-      kept.s_gate = at::empty({b.T, b.Fs}, opts);
-      kept.s_up = at::empty({b.T, b.Fs}, opts);
-    }
-    if (aux) {
-      shared.start();
-      shared_forward(b, m, kept, y_shared, save, aux->stream);
-    }
+  if (aux) {
+    shared.start();
+    shared_forward(b, k, y_shared, aux->stream);
   }
 
   // router: partial logits, then selection and plan
-  const int splits = mi355_router_gate_fwd_splits(b.dt, b.gate_dt, b.T, b.D, b.E);
-  const int64_t piece_bytes = splits > 0 ? mi355_router_gate_fwd_pieces_bytes(b.dt, b.gate_dt, b.T, b.D, b.E) : 0;
-  const int64_t partial_bytes = splits > 1 ? splits * b.T * b.E * 4
-                                : splits == 0 ? mi355_router_gate_fwd_workspace_bytes(b.T, b.D, b.E) : 0;
-  const int64_t plan_bytes = mi355_route_plan_workspace_bytes(b.T, c.K, b.E);
-  const int64_t plan_at = (partial_bytes + 255) / 256 * 256;
-  Tensor scratch;
-  if (partial_bytes + plan_bytes > 0) scratch = bytes(plan_at + plan_bytes, b.x);
-  char* work = scratch.defined() ? static_cast<char*>(scratch.data_ptr()) : nullptr;
-  if (piece_bytes > 0) kept.pieces = bytes(piece_bytes, b.x);
-  float* partial = splits > 1 ? reinterpret_cast<float*>(work) : m.logits;
-  if (splits > 0)
-    check(mi355_router_gate_fwd_partial(ptr(b.x), b.dt, fptr(b.gate_w), fptr(gate_b), partial, ptr(kept.pieces), b.T,
-                                        b.D, b.E, L.stream),
+  float* partial = b.splits > 1 ? static_cast<float*>(gate_work) : k.logits;
+  if (b.splits > 0)
+    check(mi355_router_gate_fwd_partial(ptr(b.x), b.dt, fptr(b.gate_w), fptr(gate_b), partial, k.pieces, b.T, b.D, b.E,
+                                        L.stream),
           "router_gate_fwd");
   else
-    check(mi355_router_gate_fwd(ptr(b.x), b.dt, ptr(b.gate_w), b.gate_dt, fptr(gate_b), m.logits,
-                                partial_bytes > 0 ? work : nullptr, b.T, b.D, b.E, L.stream),
+    check(mi355_router_gate_fwd(ptr(b.x), b.dt, ptr(b.gate_w), b.gate_dt, fptr(gate_b), k.logits, gate_work, b.T, b.D,
+                                b.E, L.stream),
           "router_gate_fwd");
-  check(mi355_route_plan(partial, splits > 1 ? splits : 1, fptr(gate_b), save && splits > 1 ? m.logits : nullptr,
+  check(mi355_route_plan(partial, b.splits > 1 ? b.splits : 1, fptr(gate_b), save && b.splits > 1 ? k.logits : nullptr,
                          fptr(expert_b), b.T, b.E, c.K, (int)c.score_func, (int)c.route_norm, (float)c.route_scale,
-                         (int)c.num_groups, (int)c.num_limited, m.weights, m.ids, c.lo, c.hi, c.align, b.tile_m,
-                         m.counts, m.seg_offsets, m.seg_counts, m.row_of_slot, m.slot_of_row, m.token_of_row,
-                         save && b.folded ? m.row_scale : nullptr, b.R, m.tile_expert, m.tile_row0, m.num_tiles,
-                         b.tile_cap, plan_bytes > 0 ? work + plan_at : nullptr, L.stream),
+                         (int)c.num_groups, (int)c.num_limited, k.weights, k.ids, c.lo, c.hi, c.align, b.tile_m,
+                         counts.data_ptr<int32_t>(), k.seg_offsets, k.seg_counts, k.row_of_slot, k.slot_of_row,
+                         k.token_of_row, save && b.folded ? k.row_scale : nullptr, b.R, k.tile_expert, k.tile_row0,
+                         k.num_tiles, b.tile_cap, plan_work, L.stream),
         "route_plan");
 
   // routed experts
-  Tensor y = at::empty({b.R, b.D}, opts), h = at::empty({b.R, b.F}, opts);
-  if (b.folded) {
-    if (save) {
-      kept.gate = at::empty({b.R, b.F}, opts);
-      kept.up = at::empty({b.R, b.F}, opts);
-    }
-    check(mi355_grouped_swiglu_fwd(ptr(b.x), m.token_of_row, b.T, ptr(b.w1), ptr(b.w3), ptr(b.w2), b.dt, m.seg_offsets,
-                                   m.seg_counts, m.tile_expert, m.tile_row0, m.num_tiles, b.tile_cap, ptr(kept.gate),
-                                   ptr(kept.up), ptr(h), ptr(y), b.El, b.D, b.F, b.R, L.stream),
-          "grouped_swiglu_fwd");
-  } else {
-    kept.rows = at::empty({b.R, b.D}, opts);
-    kept.gate = at::empty({b.R, b.F}, opts);
-    kept.up = at::empty({b.R, b.F}, opts);
-    check(mi355_permute_rows_fwd(ptr(b.x), b.dt, m.row_of_slot, c.align > 1 ? m.slot_of_row : nullptr,
-                                 m.seg_offsets + b.El, ptr(kept.rows), b.T, b.D, c.K, b.R, L.stream),
+  if (!b.folded)
+    check(mi355_permute_rows_fwd(ptr(b.x), b.dt, k.row_of_slot, c.align > 1 ? k.slot_of_row : nullptr,
+                                 k.seg_offsets + b.El, k.rows, b.T, b.D, c.K, b.R, L.stream),
           "permute_rows_fwd");
-    check(mi355_grouped_swiglu_fwd(ptr(kept.rows), nullptr, b.R, ptr(b.w1), ptr(b.w3), ptr(b.w2), b.dt, m.seg_offsets,
-                                   m.seg_counts, m.tile_expert, m.tile_row0, m.num_tiles, b.tile_cap, ptr(kept.gate),
-                                   ptr(kept.up), ptr(h), ptr(y), b.El, b.D, b.F, b.R, L.stream),
-          "grouped_swiglu_fwd");
-    kept.h = h;
-    kept.y = y;
-  }
-  if (b.Fs > 0 && !aux) shared_forward(b, m, kept, y_shared, save, L.stream);
+  check(mi355_grouped_swiglu_fwd(b.folded ? ptr(b.x) : k.rows, b.folded ? k.token_of_row : nullptr, b.folded ? b.T : b.R,
+                                 ptr(b.w1), ptr(b.w3), ptr(b.w2), b.dt, k.seg_offsets, k.seg_counts, k.tile_expert,
+                                 k.tile_row0, k.num_tiles, b.tile_cap, k.gate, k.up, h, y, b.El, b.D, b.F, b.R, L.stream),
+        "grouped_swiglu_fwd");
+  if (b.Fs > 0 && !aux) shared_forward(b, k, y_shared, L.stream);
   shared.join();
-  Tensor out = at::empty({b.T, b.D}, opts);
-  check(mi355_combine_add_fwd(ptr(y), b.dt, m.weights, m.row_of_slot, ptr(y_shared), ptr(out), b.T, b.D, c.K,
-                              (int)c.round_terms, L.stream),
+  check(mi355_combine_add_fwd(y, b.dt, k.weights, k.row_of_slot, y_shared, ptr(out), b.T, b.D, c.K, (int)c.round_terms,
+                              L.stream),
         "combine_fwd");
-  return {out, counts};
+  return {out, counts, kept};
 }
 
 struct Needs {
@@ -251,43 +264,80 @@ struct Grads {
   Tensor x, gate_w, gate_b, w1, w3, w2, sg, su, sd;
 };
 
-Grads block_backward(const Block& b, const Kept& k, const Tensor& dout_, const Needs& need) {
+Grads block_backward(const Block& b, const Tensor& kept, const Tensor& dout_, const Needs& need) {
   Launch L(b.x);
   const Config& c = b.c;
   const auto opts = b.x.options();
-  const auto f32 = opts.dtype(at::kFloat);
+  const int64_t item = b.dt == MI355_F32 ? 4 : 2;
   const hipStream_t main = static_cast<hipStream_t>(L.stream);
   const Tensor dout = (dout_.scalar_type() == b.x.scalar_type() ? dout_ : dout_.to(b.x.scalar_type())).contiguous();
-  const Meta m(b, k.meta.data_ptr(), nullptr);
+  Kept k;
+  Carver held{static_cast<char*>(kept.data_ptr())};
+  k.layout(held, b, true);
   const int device = b.x.device().index();
+  const bool gate = need.gate_w || need.gate_b, routed = need.x || gate || need.experts, logits = need.x || gate;
+  const bool run_shared = b.Fs > 0 && (need.x || need.shared);
+
   Grads g;
-  const bool gate = need.gate_w || need.gate_b, routed = need.x || gate || need.experts;
+  auto like = [](Tensor& out, const Tensor& t) { out = at::empty(t.sizes(), t.options()); };
+  if (need.x) like(g.x, b.x);
+  if (need.gate_w) like(g.gate_w, b.gate_w);
+  if (need.experts) {
+    like(g.w1, b.w1);
+    like(g.w3, b.w3);
+    like(g.w2, b.w2);
+  }
+  if (need.shared) {
+    like(g.sg, b.sg);
+    like(g.su, b.su);
+    like(g.sd, b.sd);
+  }
+  const int64_t slots = b.folded ? mi355_grouped_combine_bwd_slots(b.dt, b.D, b.F) : 0;
+  const int64_t gate_bytes = need.x || need.gate_w ? mi355_router_gate_bwd_workspace_bytes(b.T, b.D, b.E) : 0;
+  void *s_dgate = nullptr, *s_dup = nullptr, *dx_shared = nullptr, *dx_routed = nullptr, *dgate = nullptr, *dup = nullptr,
+       *drows = nullptr, *hs = nullptr, *dy = nullptr, *gate_work = nullptr;
+  float *dots = nullptr, *dlogits = nullptr;  // dots: pieces (R, slots), or whole (T, K)
+  Tensor dlogits_t;
+  if (need.gate_b) dlogits_t = at::empty({b.T, b.E}, opts.dtype(at::kFloat));
+  Tensor scratch = carve(b.x, [&](Carver& cv) {
+    if (run_shared) {
+      s_dgate = cv.take(b.T * b.Fs, item);
+      s_dup = cv.take(b.T * b.Fs, item);
+      if (need.x) dx_shared = cv.take(b.T * b.D, item);
+    }
+    if (!routed) return;
+    if (need.x) {
+      dx_routed = cv.take(b.T * b.D, item);
+      drows = cv.take(b.R * b.D, item);
+    }
+    dgate = cv.take(b.R * b.F, item);
+    dup = cv.take(b.R * b.F, item);
+    if (b.folded) {
+      hs = cv.take(b.R * b.F, item);
+      dots = cv.take<float>(b.R * slots);
+    } else {
+      dy = cv.take(b.R * b.D, item);
+      dots = cv.take<float>(b.N);
+    }
+    if (logits) dlogits = need.gate_b ? dlogits_t.data_ptr<float>() : cv.take<float>(b.T * b.E);
+    if (gate_bytes > 0) gate_work = cv.take(gate_bytes, 1);
+  });
 
   // ---- shared expert: dH and dX beside the routed part where they may be, its weight gradients in front
   // of the routed ones on the stream those use
-  Tensor dx_shared, s_dgate, s_dup;
-  const bool run_shared = b.Fs > 0 && (need.x || need.shared);
   SideStream* aux = run_shared && c.overlap && routed ? side_stream(device, main, 1) : nullptr;
   SideStream* side = routed && need.x && ((b.folded && need.experts) || (b.shared_folded && aux && need.shared))
                          ? side_stream(device, main, 0) : nullptr;
   Fork shared(aux, main), weights(side, main);
   if (run_shared) {
-    s_dgate = at::empty({b.T, b.Fs}, opts);
-    s_dup = at::empty({b.T, b.Fs}, opts);
-    if (need.x) dx_shared = at::empty({b.T, b.D}, opts);
-    if (need.shared) {
-      g.sg = at::empty_like(b.sg);
-      g.su = at::empty_like(b.su);
-      g.sd = at::empty_like(b.sd);
-    }
     if (aux) shared.start();
     void* stream = aux ? static_cast<void*>(aux->stream) : L.stream;
     if (b.shared_folded) {
       auto stage = [&](int s, void* on) {
-        check(mi355_grouped_swiglu_stage(s, ptr(dout), ptr(b.x), nullptr, b.T, ptr(b.sg), ptr(b.su), ptr(b.sd),
-                                         ptr(k.s_gate), ptr(k.s_up), ptr(k.s_h), nullptr, m.s_offsets, m.s_counts,
-                                         m.s_expert, m.s_row0, m.s_num, b.shared_cap, ptr(s_dgate), ptr(s_dup),
-                                         ptr(dx_shared), ptr(g.sg), ptr(g.su), ptr(g.sd), 1, b.D, b.Fs, b.T, on),
+        check(mi355_grouped_swiglu_stage(s, ptr(dout), ptr(b.x), nullptr, b.T, ptr(b.sg), ptr(b.su), ptr(b.sd), k.s_gate,
+                                         k.s_up, k.s_h, nullptr, k.s_offsets, k.s_counts, k.s_expert, k.s_row0, k.s_num,
+                                         b.shared_cap, s_dgate, s_dup, dx_shared, ptr(g.sg), ptr(g.su), ptr(g.sd), 1,
+                                         b.D, b.Fs, b.T, on),
               "shared expert backward");
       };
       stage(MI355_STAGE_DH, stream);
@@ -300,44 +350,27 @@ Grads block_backward(const Block& b, const Kept& k, const Tensor& dout_, const N
       if (need.shared)
         for (int s : {MI355_STAGE_DW2, MI355_STAGE_DW1, MI355_STAGE_DW3}) stage(s, weight_stream);
     } else {
-      check(mi355_grouped_swiglu_bwd(ptr(dout), ptr(b.x), nullptr, b.T, ptr(b.sg), ptr(b.su), ptr(b.sd), ptr(k.s_gate),
-                                     ptr(k.s_up), ptr(k.s_h), b.dt, m.s_offsets, m.s_counts, m.s_expert, m.s_row0,
-                                     m.s_num, b.shared_cap, ptr(s_dgate), ptr(s_dup), ptr(dx_shared), ptr(g.sg),
-                                     ptr(g.su), ptr(g.sd), 1, b.D, b.Fs, b.T, stream),
+      check(mi355_grouped_swiglu_bwd(ptr(dout), ptr(b.x), nullptr, b.T, ptr(b.sg), ptr(b.su), ptr(b.sd), k.s_gate, k.s_up,
+                                     k.s_h, b.dt, k.s_offsets, k.s_counts, k.s_expert, k.s_row0, k.s_num, b.shared_cap,
+                                     s_dgate, s_dup, dx_shared, ptr(g.sg), ptr(g.su), ptr(g.sd), 1, b.D, b.Fs, b.T, stream),
             "shared expert backward");
     }
   }
   if (!routed) return g;
 
   // ---- routed experts: dx_routed is the sum over a token's rows plus the shared expert's part
-  Tensor dx_routed, dlogits;
-  if (need.x) dx_routed = at::empty({b.T, b.D}, opts);
-  if (need.experts) {
-    g.w1 = at::empty_like(b.w1);
-    g.w3 = at::empty_like(b.w3);
-    g.w2 = at::empty_like(b.w2);
-  }
-  if (need.x || gate) dlogits = at::empty({b.T, b.E}, f32);
-  auto row_sum = [&](const Tensor& drows) {
+  auto row_sum = [&]() {
     if (!need.x) return;
     shared.join();
-    check(mi355_permute_rows_add_bwd(ptr(drows), b.dt, m.row_of_slot, ptr(dx_shared), ptr(dx_routed), b.T, b.D, c.K,
-                                     L.stream),
+    check(mi355_permute_rows_add_bwd(drows, b.dt, k.row_of_slot, dx_shared, dx_routed, b.T, b.D, c.K, L.stream),
           "permute_rows_bwd");
   };
-  Tensor dgate = at::empty_like(k.gate), dup = at::empty_like(k.up);
-  Tensor drows, hs, partial, dy, dweights;
-  if (need.x) drows = at::empty({b.R, b.D}, opts);
   if (b.folded) {
-    const int64_t slots = mi355_grouped_combine_bwd_slots(b.dt, b.D, b.F);
-    hs = at::empty_like(k.gate);
-    partial = at::empty({b.R, slots}, f32);
     auto run = [&](int stages, void* stream) {
-      check(mi355_grouped_swiglu_combine_bwd(
-                ptr(dout), ptr(b.x), m.token_of_row, b.T, m.row_scale, ptr(b.w1), ptr(b.w3), ptr(b.w2), ptr(k.gate),
-                ptr(k.up), b.dt, m.seg_offsets, m.seg_counts, m.tile_expert, m.tile_row0, m.num_tiles, b.tile_cap,
-                ptr(dgate), ptr(dup), ptr(hs), static_cast<float*>(ptr(partial)), ptr(drows), ptr(g.w1), ptr(g.w3),
-                ptr(g.w2), b.El, b.D, b.F, b.R, stages, stream),
+      check(mi355_grouped_swiglu_combine_bwd(ptr(dout), ptr(b.x), k.token_of_row, b.T, k.row_scale, ptr(b.w1), ptr(b.w3),
+                                             ptr(b.w2), k.gate, k.up, b.dt, k.seg_offsets, k.seg_counts, k.tile_expert,
+                                             k.tile_row0, k.num_tiles, b.tile_cap, dgate, dup, hs, dots, drows, ptr(g.w1),
+                                             ptr(g.w3), ptr(g.w2), b.El, b.D, b.F, b.R, stages, stream),
             "grouped_swiglu_combine_bwd");
     };
     constexpr int kWeights = MI355_STAGE_DW2 | MI355_STAGE_DW1 | MI355_STAGE_DW3;
@@ -349,44 +382,35 @@ Grads block_backward(const Block& b, const Kept& k, const Tensor& dout_, const N
       run(kWeights, side->stream);
     }
     if (need.x) run(MI355_STAGE_DX, L.stream);
-    row_sum(drows);
-    if (dlogits.defined())
-      check(mi355_router_select_dots_bwd(m.logits, m.ids, fptr(partial), slots, m.row_of_slot, b.R,
-                                         dlogits.data_ptr<float>(), b.T, b.E, c.K, (int)c.score_func,
-                                         (int)c.route_norm, (float)c.route_scale, L.stream),
+    row_sum();
+    if (logits)
+      check(mi355_router_select_dots_bwd(k.logits, k.ids, dots, slots, k.row_of_slot, b.R, dlogits, b.T, b.E, c.K,
+                                         (int)c.score_func, (int)c.route_norm, (float)c.route_scale, L.stream),
             "router_select_bwd");
     if (need.experts && !side) run(kWeights, L.stream);
   } else {
-    const int32_t* pad = c.align > 1 ? m.slot_of_row : nullptr;
-    dy = at::empty({b.R, b.D}, opts);
-    dweights = at::empty({b.T, c.K}, f32);
-    check(mi355_combine_bwd(ptr(dout), ptr(k.y), b.dt, m.weights, m.row_of_slot, pad, m.seg_offsets + b.El, ptr(dy),
-                            dweights.data_ptr<float>(), b.T, b.D, c.K, b.R, L.stream),
+    const int32_t* pad = c.align > 1 ? k.slot_of_row : nullptr;
+    check(mi355_combine_bwd(ptr(dout), k.y, b.dt, k.weights, k.row_of_slot, pad, k.seg_offsets + b.El, dy, dots, b.T, b.D,
+                            c.K, b.R, L.stream),
           "combine_bwd");
     if (need.x || need.experts)
-      check(mi355_grouped_swiglu_bwd(ptr(dy), ptr(k.rows), nullptr, b.R, ptr(b.w1), ptr(b.w3), ptr(b.w2), ptr(k.gate),
-                                     ptr(k.up), ptr(k.h), b.dt, m.seg_offsets, m.seg_counts, m.tile_expert, m.tile_row0,
-                                     m.num_tiles, b.tile_cap, ptr(dgate), ptr(dup), ptr(drows), ptr(g.w1), ptr(g.w3),
-                                     ptr(g.w2), b.El, b.D, b.F, b.R, L.stream),
+      check(mi355_grouped_swiglu_bwd(dy, k.rows, nullptr, b.R, ptr(b.w1), ptr(b.w3), ptr(b.w2), k.gate, k.up, k.h, b.dt,
+                                     k.seg_offsets, k.seg_counts, k.tile_expert, k.tile_row0, k.num_tiles, b.tile_cap,
+                                     dgate, dup, drows, ptr(g.w1), ptr(g.w3), ptr(g.w2), b.El, b.D, b.F, b.R, L.stream),
             "grouped_swiglu_bwd");
-    row_sum(drows);
-    if (dlogits.defined())
-      check(mi355_router_select_bwd(m.logits, m.ids, fptr(dweights), nullptr, dlogits.data_ptr<float>(), b.T, b.E, c.K,
-                                    (int)c.score_func, (int)c.route_norm, (float)c.route_scale, MI355_SELECT_TOPK,
-                                    L.stream),
+    row_sum();
+    if (logits)
+      check(mi355_router_select_bwd(k.logits, k.ids, dots, nullptr, dlogits, b.T, b.E, c.K, (int)c.score_func,
+                                    (int)c.route_norm, (float)c.route_scale, MI355_SELECT_TOPK, L.stream),
             "router_select_bwd");
   }
 
   // ---- router gate; the input gradient is complete with its part
-  if (need.x || need.gate_w) {
-    if (need.x) g.x = at::empty({b.T, b.D}, opts);
-    if (need.gate_w) g.gate_w = at::empty_like(b.gate_w);
-    Tensor ws = bytes(mi355_router_gate_bwd_workspace_bytes(b.T, b.D, b.E), b.x);
-    check(mi355_router_gate_add_bwd(fptr(dlogits), ptr(b.x), b.dt, ptr(b.gate_w), b.gate_dt, ptr(k.pieces),
-                                    ptr(dx_routed), ptr(g.x), ptr(g.gate_w), ptr(ws), b.T, b.D, b.E, L.stream),
+  if (need.x || need.gate_w)
+    check(mi355_router_gate_add_bwd(dlogits, ptr(b.x), b.dt, ptr(b.gate_w), b.gate_dt, k.pieces, dx_routed, ptr(g.x),
+                                    ptr(g.gate_w), gate_work, b.T, b.D, b.E, L.stream),
           "router_gate_bwd");
-  }
-  if (need.gate_b) g.gate_b = dlogits.sum(0).to(b.gate_b.scalar_type());
+  if (need.gate_b) g.gate_b = dlogits_t.sum(0).to(b.gate_b.scalar_type());
   weights.join();
   shared.join();
   return g;
@@ -402,10 +426,8 @@ struct MoeBlock : public torch::autograd::Function<MoeBlock> {
     at::AutoDispatchBelowADInplaceOrView below;
     Block b{x, gate_w, some(gate_b), some(expert_b), w1, w3, w2, some(sg), some(su), some(sd), c};
     b.sizes();
-    Kept k;
-    auto [out, counts] = block_forward(b, true, k);
-    ctx->save_for_backward({x, gate_w, b.gate_b, w1, w3, w2, b.sg, b.su, b.sd, k.meta, k.pieces, k.rows, k.gate, k.up, k.h, k.y,
-                            k.s_gate, k.s_up, k.s_h});
+    auto [out, counts, kept] = block_forward(b, true);
+    ctx->save_for_backward({x, gate_w, b.gate_b, w1, w3, w2, b.sg, b.su, b.sd, kept});
     auto packed = c.pack();
     packed.push_back(b.expert_b.defined());
     ctx->saved_data["config"] = packed;
@@ -420,14 +442,13 @@ struct MoeBlock : public torch::autograd::Function<MoeBlock> {
     const auto packed = ctx->saved_data["config"].toIntVector();
     Block b{s[0], s[1], s[2], Tensor(), s[3], s[4], s[5], s[6], s[7], s[8], Config::unpack(packed)};
     b.sizes();
-    const Kept k{s[9], s[10], s[11], s[12], s[13], s[14], s[15], s[16], s[17], s[18]};
     // needs_input_grad counts the tensors among the arguments: an absent one has no index
     const int gb = 2, w = gb + (b.gate_b.defined() ? 1 : 0) + (packed.back() ? 1 : 0), sh = w + 3;
     auto wants = [&](int i) { return ctx->needs_input_grad(i); };
     const bool shared = b.Fs > 0;
     const Needs need{wants(0), wants(1), b.gate_b.defined() && wants(gb), wants(w) || wants(w + 1) || wants(w + 2),
                      shared && (wants(sh) || wants(sh + 1) || wants(sh + 2))};
-    Grads g = block_backward(b, k, grads[0], need);
+    Grads g = block_backward(b, s[9], grads[0], need);
     auto put = [&](int argument, int tensor, const Tensor& t) {
       if (t.defined() && wants(tensor)) out[argument] = t;
     };
@@ -491,8 +512,8 @@ std::tuple<Tensor, Tensor> moe_block(const Tensor& x_, const Tensor& gate_w_, co
   at::AutoDispatchBelowADInplaceOrView below;
   Block b{x, gate_w, gate_b, expert_b, w1, w3, w2, sg, su, sd, c};
   b.sizes();
-  Kept k;
-  return block_forward(b, false, k);
+  auto [out, counts, kept] = block_forward(b, false);
+  return {out, counts};
 }
 
 }  // namespace

@@ -257,8 +257,7 @@ class MoE(nn.Module):
             if whole is not None:
                 out_TD, num_tokens_per_expert_E = whole
                 if self.training and not in_checkpoint_recompute.get():
-                    with torch.no_grad():
-                        self.tokens_per_expert_E.add_(num_tokens_per_expert_E)
+                    self.tokens_per_expert_E.add_(num_tokens_per_expert_E)  # (neither takes part in autograd)
                 if restore_shape:
                     out_TD = out_TD.reshape(*x.shape[:-1], out_TD.shape[-1])
                 return (out_TD, None) if self.returns_router_logits else out_TD
