@@ -188,9 +188,12 @@ int mi355_router_select_bwd(const float* logits_TE, const int64_t* ids_TK,
                             int score_func, int route_norm, float route_scale,
                             int select_mode, void* stream);
 /* The same for a plain top-k whose weights' gradient is still in pieces, as
- * mi355_grouped_swiglu_combine_bwd leaves it: dweights[slot] = sum_i dot_partial[row_of_slot[slot]][i]. */
-int mi355_router_select_dots_bwd(const float* logits_TE, const int64_t* ids_TK, const float* dot_partial,
+ * mi355_grouped_swiglu_combine_bwd leaves it: dweights[slot] = sum_i dots[row_of_slot[slot]][i]; with
+ * pieces = 0, dots is dweights_TK itself.  aux_f_E, aux_scale, padding_mask_T (all NULL: no loss): what
+ * mi355_route_plan_stats left of the load-balance loss, whose gradient is added to the scores'. */
+int mi355_router_select_dots_bwd(const float* logits_TE, const int64_t* ids_TK, const float* dots,
                                  int64_t pieces, const int32_t* row_of_slot, int64_t row_capacity,
+                                 const float* aux_f_E, const float* aux_scale, const uint8_t* padding_mask_T,
                                  float* dlogits_TE, int64_t T, int64_t E, int64_t K, int score_func,
                                  int route_norm, float route_scale, void* stream);
 
@@ -328,6 +331,27 @@ int mi355_route_plan(const float* partial, int splits, const float* logit_bias, 
                      int32_t* slot_of_row, int32_t* token_of_row, float* row_scale, int64_t row_capacity,
                      int32_t* tile_expert, int32_t* tile_row0, int32_t* num_tiles, int64_t tile_capacity,
                      void* workspace, void* stream);
+
+/*
+ * The same for a router that keeps statistics; each NULL = not wanted.  valid_counts_E: slots per
+ * expert of the tokens that are not padding.  scores_TE, cutoff_T: as mi355_router_select_cutoff_fwd
+ * gives them.  aux_f_E, aux_scale: the load-balance loss of mi355_balance_loss_fwd over those tokens
+ * and slots, as its backward wants it (aux_scale[0] = aux_coeff / max(aux_denominator[0], 1));
+ * aux_acc[0] (fp32 or bf16) += loss / max(aux_denominator[0], 1).  stats_workspace of
+ * mi355_route_stats_workspace_bytes (NULL without counts and loss).
+ */
+int64_t mi355_route_stats_workspace_bytes(int64_t T, int64_t E);
+int mi355_route_plan_stats(const float* partial, int splits, const float* logit_bias, float* logits_TE,
+                           const float* expert_bias, int64_t T, int64_t E, int64_t K, int score_func,
+                           int route_norm, float route_scale, int num_groups, int num_limited,
+                           float* weights_TK, int64_t* ids_TK, int64_t lo, int64_t hi, int64_t align,
+                           int64_t tile_m, int32_t* counts_E, int32_t* seg_offsets, int32_t* seg_counts,
+                           int32_t* row_of_slot, int32_t* slot_of_row, int32_t* token_of_row,
+                           float* row_scale, int64_t row_capacity, int32_t* tile_expert, int32_t* tile_row0,
+                           int32_t* num_tiles, int64_t tile_capacity, void* workspace,
+                           const uint8_t* padding_mask_T, int32_t* valid_counts_E, float* scores_TE,
+                           float* cutoff_T, float* aux_f_E, float* aux_scale, void* aux_acc,
+                           int aux_acc_dtype, const float* aux_denominator, float aux_coeff, void* stats_workspace, void* stream);
 
 
 /*

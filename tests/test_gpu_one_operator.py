@@ -60,6 +60,65 @@ def test_one_operator_equals_the_stages_bit_for_bit(dtype, T, D, E, K, F, kw):
         assert torch.equal(a, b), f"tensor {i} differs by {float((a.float() - b.float()).abs().max())}"
 
 
+@pytest.mark.parametrize("quantile,masked,T,E,K,groups", [
+    (True, True, 64, 64, 6, None), (True, False, 65, 24, 3, None), (False, True, 1000, 128, 8, (8, 4)), (False, True, 16500, 256, 2, None),
+    (False, False, 3, 5, 2, None)])
+def test_router_statistics_of_the_one_operator_match_the_stages(quantile, masked, T, E, K, groups):
+    """Histogram, counts without padding, the balance loss's metric and gradient: one operator against the
+    stages.  Counts and histogram are equal; the loss is the same sums in another order."""
+    from torchllmtuner_amd import moe
+
+    print(f"one operator statistics quantile={quantile} masked={masked} T={T} E={E} K={K}", flush=True)
+    D, F = 384, 384
+    p = make_params(E, D, F, torch.bfloat16, seed=T, std=0.05)
+    g = torch.Generator().manual_seed(T + 1)
+    x = torch.randn(T, D, generator=g).bfloat16().to(DEV)
+    gout = torch.randn(T, D, generator=g).bfloat16().to(DEV)
+    mask = (torch.rand(T, generator=g) < 0.2).to(DEV) if masked else None
+    denom = torch.tensor(float(T * K), device=DEV)
+
+    def run(in_stages):
+        aux = moe.MicrobatchWiseLoadBalanceLoss(coeff=2.0)
+        if quantile:
+            router = moe.QuantileBalancedTopKRouter(E, D, K, num_bins=500, route_norm=True, aux_loss=aux)
+        else:
+            router = moe.TokenChoiceTopKRouter(E, D, K, score_func="softmax", aux_loss=aux,
+                                               num_expert_groups=groups and groups[0], num_limited_groups=groups and groups[1])
+        block = moe.MoE(E, moe.RoutedExperts(moe.GroupedExperts(D, F, E), moe.LocalTokenDispatcher(E, K)), router,
+                        load_balance_coeff=None).to(torch.bfloat16)
+        router.gate.float()
+        aux.to(torch.bfloat16 if masked else torch.float32)
+        with torch.no_grad():
+            router.gate.weight.copy_(p.router_w_ED)
+            ie = block.routed_experts.inner_experts
+            ie.w1_EFD.copy_(p.w1_EFD); ie.w3_EFD.copy_(p.w3_EFD); ie.w2_EDF.copy_(p.w2_EDF)
+            if quantile:
+                block.expert_bias_E.copy_(torch.linspace(-0.05, 0.05, E))
+        block = block.to(DEV).train()
+        moe.AuxLoss.set_step_denominator(denom, model_parts=[block])
+        if in_stages:
+            router.register_forward_hook(lambda *a: None)
+        assert (block._forward_as_one(x, mask) is None) == in_stages
+        if not in_stages:  # (the call above kept statistics)
+            aux.instance_acc.zero_()
+            if quantile:
+                router.quantile_balancer.required_bias_histogram_EB.zero_()
+        xin = x.clone().requires_grad_()
+        out = block(xin, padding_mask=mask)
+        out.backward(gout)
+        exact = [out.detach(), block.tokens_per_expert_E] + [q.grad for q in ie.parameters()]
+        if quantile:
+            exact.append(router.quantile_balancer.required_bias_histogram_EB)
+        return exact, [aux.instance_acc, router.gate.weight.grad, xin.grad]
+
+    (exact_a, close_a), (exact_b, close_b) = run(True), run(False)
+    for i, (a, b) in enumerate(zip(exact_a, exact_b)):
+        assert torch.equal(a, b), f"tensor {i}"
+    for i, (a, b) in enumerate(zip(close_a, close_b)):
+        err = float((a.double() - b.double()).norm() / a.double().norm())
+        assert err < (2e-3 if i == 2 else 4e-3 if a.dtype == torch.bfloat16 else 2e-6), f"tensor {i}: {err}"
+
+
 @pytest.mark.parametrize("dtype,T,D,E", [
     (torch.bfloat16, 1, 8, 1), (torch.bfloat16, 33, 2056, 33), (torch.bfloat16, 1000, 7168, 256), (torch.bfloat16, 32, 1024, 66),
     (torch.float32, 1, 4, 3), (torch.float32, 31, 1028, 32), (torch.float32, 2000, 640, 10), (torch.float32, 4, 3000, 5)])

@@ -68,7 +68,13 @@ SIGNATURES = {
     "mi355_router_gate_fwd_pieces_bytes": (L, [I, I, L, L, L]),
     "mi355_router_gate_fwd_partial": (I, [P, I, P, P, P, P, L, L, L, P]),
     "mi355_router_gate_add_bwd": (I, [P, P, I, P, I, P, P, P, P, P, L, L, L, P]),
-    "mi355_router_select_dots_bwd": (I, [P, P, P, L, P, L, P, L, L, L, I, I, F, P]),
+    "mi355_router_select_dots_bwd": (I, [P, P, P, L, P, L, P, P, P, P, L, L, L, I, I, F, P]),
+    "mi355_route_stats_workspace_bytes": (L, [L, L]),
+    "mi355_route_plan_stats": (
+        I,
+        [P, I, P, P, P, L, L, L, I, I, F, I, I, P, P, L, L, L, L, P, P, P, P, P, P, P, L, P, P, P, L, P,
+         P, P, P, P, P, P, P, I, P, F, P, P],
+    ),
     "mi355_combine_add_fwd": (I, [P, I, P, P, P, P, L, L, L, I, P]),
     "mi355_permute_rows_add_bwd": (I, [P, I, P, P, P, L, L, L, P]),
     "mi355_segments_dense": (I, [L, L, P, P, P, P, P, L, P]),

@@ -33,6 +33,23 @@ struct PlanOut {
   int32_t *tile_expert, *tile_row0, *num_tiles;
 };
 
+// What a router that keeps statistics wants besides (all null: nothing).  valid_counts: every expert's slots
+// of the tokens that are not padding.  scores, cutoff: for the required-bias histogram.  f, scale, acc:
+// the load-balance loss sum_e f_e p_e of aux.hip over the tokens that are not padding: f_e and the
+// factor of its gradient for the backward, and the running mean metric it is added to.
+struct StatsOut {
+  const uint8_t* padding;  // (T), non-zero = padding
+  int32_t* valid_counts;
+  float *scores, *cutoff;
+  float *f, *scale;
+  void* acc;
+  int acc_dtype;
+  const float* denominator;
+  float coeff;
+  int32_t* block_valid;  // (blocks, E)
+  float* block_share;    // (blocks, E)
+};
+
 // Integer arrays in LDS for the layout step, E experts.
 struct LayoutLds {
   int32_t *count, *before, *seg, *tile, *order, *wave_sums;
@@ -141,18 +158,73 @@ __device__ __forceinline__ void place_slot(const LayoutLds& s, const PlanOut& p,
   p.row_of_slot[slot] = row;
 }
 
+// Sums the workgroups' valid counts and score shares (in order), and the loss from them; one workgroup.
+__device__ void finish_stats(const StatsOut& st, int E, int nb, float* red) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr float kEps = 1e-12f;  // F.normalize's clamp
+  constexpr int kBatch = 8;
+  int valid = 0;
+  float share = 0.0f;
+  if (tid < E) {
+    for (int b0 = 0; b0 < nb; b0 += kBatch) {
+      int v[kBatch];
+      float p[kBatch];
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        const int64_t at = static_cast<int64_t>(b0 + i) * E + tid;
+        v[i] = b0 + i < nb ? st.block_valid[at] : 0;
+        p[i] = st.f && b0 + i < nb ? st.block_share[at] : 0.0f;
+      }
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        valid += v[i];
+        share += p[i];
+      }
+    }
+    if (st.valid_counts) st.valid_counts[tid] = valid;
+  }
+  if (!st.f) return;
+  // E <= 256: four waves hold everything
+  auto total = [&](float v) {
+    v = wave_sum(v);
+    __syncthreads();
+    if (lane == 0 && wave < 4) red[wave] = v;
+    __syncthreads();
+    return (red[0] + red[1]) + (red[2] + red[3]);
+  };
+  const float all = total(static_cast<float>(valid));
+  const float f = static_cast<float>(valid) * (static_cast<float>(E) / fmaxf(all, kEps));
+  const float loss = total(f * share);
+  if (tid < E) st.f[tid] = f;
+  if (tid == 0) {
+    const float scale = 1.0f / fmaxf(*st.denominator, 1.0f);
+    *st.scale = st.coeff * scale;
+    if (st.acc && st.acc_dtype == MI355_BF16) {
+      uint16_t* acc = static_cast<uint16_t*>(st.acc);
+      *acc = f32_to_bf16(bf16_to_f32(*acc) + loss * scale);
+    } else if (st.acc) {
+      *static_cast<float*>(st.acc) += loss * scale;
+    }
+  }
+}
+
 template <int VPR, bool FULL>
 __global__ __launch_bounds__(kLanes) void route_rank_kernel(
     const float* __restrict__ partial, int splits, const float* __restrict__ logit_bias,
     float* __restrict__ logits_out, SelectArgs sel, float* __restrict__ weights, int64_t* __restrict__ ids,
-    uint32_t* __restrict__ rank_in_block, int32_t* __restrict__ block_hist, int T, int chunks, int fill, PlanOut p) {
+    uint32_t* __restrict__ rank_in_block, int32_t* __restrict__ block_hist, int T, int chunks, int fill, PlanOut p,
+    StatsOut st) {
   extern __shared__ int32_t lds[];
   const int E = sel.E, K = sel.K;
   int32_t* run = lds;                       // [E] slots of each expert so far
   int32_t* cnt = lds + E;                   // [waves][E] slots of each expert in each wave of the chunk
-  int32_t* extra = cnt + kWaves * E;        // single workgroup: the layout arrays
+  const bool stats = st.valid_counts != nullptr || st.f != nullptr;
+  int32_t* valid_run = cnt + kWaves * E;    // with statistics: [E] valid slots, [waves][E] score shares
+  float* share = reinterpret_cast<float*>(valid_run + E);
+  int32_t* extra = valid_run + (stats ? (1 + kWaves) * E : 0);  // single workgroup: the layout arrays
   __shared__ uint16_t id_sh[kLanes];
   __shared__ float w_sh[kLanes];
+  __shared__ float red_sh[4];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l = tid & 15;
   const bool single = gridDim.x == 1;
   // rows that end up without a slot (padding, unused capacity) must read -1 and a zero scale
@@ -166,12 +238,15 @@ __global__ __launch_bounds__(kLanes) void route_rank_kernel(
     if (single) __threadfence();  // before this workgroup's own rows, written below
   }
   for (int e = tid; e < E; e += kLanes) run[e] = 0;
+  if (stats)
+    for (int i = tid; i < (1 + kWaves) * E; i += kLanes) valid_run[i] = 0;  // (also the shares: 0.0f)
 
   int my_e = -1, my_rank = 0;
   for (int c = 0; c < chunks; ++c) {
     const int t0 = (blockIdx.x * chunks + c) * kRows;
     if (t0 >= T) break;  // workgroup-uniform
     for (int i = tid; i < kWaves * E; i += kLanes) cnt[i] = 0;
+    if (c == 0 && stats) __syncthreads();  // the shares are zero before a wave adds to its own
     // ---- selection: one token per row of 16 lanes; waves without a token have nothing to select
     if (t0 + (wave << 2) < T) {
       const int t_raw = t0 + (tid >> 4);
@@ -195,7 +270,28 @@ __global__ __launch_bounds__(kLanes) void route_rank_kernel(
         for (int j = 0; j < VPR; ++j)
           if (FULL || l * VPR + j < E) logits_out[static_cast<int64_t>(t) * E + l * VPR + j] = x[j];
       }
-      const RowChoice ch = select_row<VPR, FULL>(sel, x, l, false, s, cutoff);
+      const RowChoice ch = select_row<VPR, FULL>(sel, x, l, st.cutoff != nullptr, s, cutoff);
+      if (st.scores && live) {
+#pragma unroll
+        for (int j = 0; j < VPR; ++j)
+          if (FULL || l * VPR + j < E) st.scores[static_cast<int64_t>(t) * E + l * VPR + j] = s[j];
+      }
+      if (st.cutoff && live && l == 0) st.cutoff[t] = cutoff;
+      if (st.f) {
+        // the token's scores over their sum, added up over the wave's four rows, then the wave's tokens
+        float sum = 0.0f;
+#pragma unroll
+        for (int j = 0; j < VPR; ++j) sum += s[j];
+        sum = row_sum(sum);
+        const float inv = live && !(st.padding && st.padding[t]) ? 1.0f / fmaxf(sum, 1e-12f) : 0.0f;
+#pragma unroll
+        for (int j = 0; j < VPR; ++j) {
+          float v = s[j] * inv;
+          v += __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x401f));  // lane ^ 16
+          v += __shfl_xor(v, 32, kWave);
+          if (lane < 16 && (FULL || l * VPR + j < E)) share[wave * E + l * VPR + j] += v;
+        }
+      }
       if (l < K) {
         const int at = (tid >> 4) * K + l;
         id_sh[at] = static_cast<uint16_t>(live && ch.id >= 0 && ch.id < E ? ch.id : 0xffff);
@@ -223,6 +319,11 @@ __global__ __launch_bounds__(kLanes) void route_rank_kernel(
     const unsigned long long lower = (1ull << lane) - 1;
     const int below = __popcll(same & lower);
     if (valid && below == 0) cnt[wave * E + e] = __popcll(same);  // the lowest lane of each expert
+    if (stats) {
+      const bool counts = valid && !(st.padding && st.padding[slot / K]);
+      const int n = __popcll(same & __ballot(counts));
+      if (valid && below == 0 && n) atomicAdd(&valid_run[e], n);
+    }
     __syncthreads();
     for (int i = tid; i < E; i += kLanes) {
       int r = run[i];
@@ -240,10 +341,21 @@ __global__ __launch_bounds__(kLanes) void route_rank_kernel(
     if (!single && slot_here) rank_in_block[slot] = static_cast<uint32_t>(my_rank);
     if (c + 1 < chunks) __syncthreads();  // cnt and id_sh are reused
   }
+  if (stats) {
+    __syncthreads();
+    for (int e = tid; e < E; e += kLanes) {
+      st.block_valid[static_cast<int64_t>(blockIdx.x) * E + e] = valid_run[e];
+      float v = 0.0f;
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) v += share[w * E + e];
+      if (st.f) st.block_share[static_cast<int64_t>(blockIdx.x) * E + e] = v;
+    }
+  }
   if (!single) {
     for (int e = tid; e < E; e += kLanes) block_hist[static_cast<int64_t>(blockIdx.x) * E + e] = run[e];
     return;
   }
+  if (stats) finish_stats(st, E, 1, red_sh);  // (each lane reads back the counts it wrote)
   const LayoutLds s(extra, E);
   for (int e = tid; e < E; e += kLanes) {
     s.count[e] = run[e];
@@ -259,8 +371,9 @@ __global__ __launch_bounds__(kLanes) void route_rows_kernel(const float* __restr
                                                             const int64_t* __restrict__ ids,
                                                             const uint32_t* __restrict__ rank_in_block,
                                                             const int32_t* __restrict__ block_hist, int T, int E, int K,
-                                                            int chunks, PlanOut p) {
+                                                            int chunks, PlanOut p, StatsOut st) {
   extern __shared__ int32_t lds[];
+  __shared__ float red_sh[4];
   const LayoutLds s(lds, E);
   const int tid = threadIdx.x;
   for (int e = tid; e < E; e += kLanes) s.count[e] = s.before[e] = 0;
@@ -287,7 +400,10 @@ __global__ __launch_bounds__(kLanes) void route_rows_kernel(const float* __restr
   }
   __syncthreads();
   plan_layout(s, p, blockIdx.x == 0);
-  if (blockIdx.x == 0) write_lists(s, p, E);
+  if (blockIdx.x == 0) {
+    write_lists(s, p, E);
+    if (st.valid_counts || st.f) finish_stats(st, E, gridDim.x, red_sh);
+  }
   const int first = blockIdx.x * chunks * kRows * K, last = min(T * K, first + chunks * kRows * K);
   for (int slot = first + tid; slot < last; slot += kLanes) {
     const int64_t e = ids[slot];
@@ -318,15 +434,18 @@ extern "C" int64_t mi355_route_plan_workspace_bytes(int64_t T, int64_t K, int64_
   if (T <= kRows || K < 1 || E < 1) return 0;
   return (T * K + route_blocks(T) * E) * (int64_t)sizeof(int32_t);
 }
+extern "C" int64_t mi355_route_stats_workspace_bytes(int64_t T, int64_t E) {
+  return T < 1 || E < 1 ? 0 : 2 * route_blocks(T) * E * (int64_t)sizeof(int32_t);
+}
 
-extern "C" int mi355_route_plan(const float* partial, int splits, const float* logit_bias, float* logits,
+static int route_plan(const float* partial, int splits, const float* logit_bias, float* logits,
                                 const float* expert_bias, int64_t T, int64_t E, int64_t K, int score_func,
                                 int route_norm, float route_scale, int num_groups, int num_limited, float* weights,
                                 int64_t* ids, int64_t lo, int64_t hi, int64_t align, int64_t tile_m,
                                 int32_t* counts_E, int32_t* seg_offsets, int32_t* seg_counts, int32_t* row_of_slot,
                                 int32_t* slot_of_row, int32_t* token_of_row, float* row_scale, int64_t row_capacity,
                                 int32_t* tile_expert, int32_t* tile_row0, int32_t* num_tiles, int64_t tile_capacity,
-                                void* workspace, void* stream) {
+                                void* workspace, const StatsOut& st, void* stream) {
   MI355_REQUIRE(T >= 1 && T < (1ll << 26) && E >= 1 && K >= 1 && K <= E && T * K < (1ll << 30),
                 "route_plan: bad shape T=%lld E=%lld K=%lld", (long long)T, (long long)E, (long long)K);
   if (!select_row_covers(E, K, num_groups, MI355_SELECT_TOPK))
@@ -356,17 +475,56 @@ extern "C" int mi355_route_plan(const float* partial, int splits, const float* l
   int32_t* hist = reinterpret_cast<int32_t*>(rank + (blocks > 1 ? T * K : 0));
   // every row has a slot when all experts are local and nothing is padded
   const int fill = !(lo == 0 && hi == E && align == 1 && row_capacity == T * K);
-  const size_t lds = ((1 + kWaves) * E + (blocks == 1 ? layout_words((int)E) : 0)) * sizeof(int32_t);
+  const bool stats = st.valid_counts || st.f;
+  const size_t lds = ((1 + kWaves) * E * (stats ? 2 : 1) + (blocks == 1 ? layout_words((int)E) : 0)) * sizeof(int32_t);
   with_row_shape(E, [&](auto vpr, auto full) {
     hipLaunchKernelGGL((route_rank_kernel<decltype(vpr)::value, decltype(full)::value>), dim3(blocks), dim3(kLanes),
                        lds, s, partial, splits, logit_bias, logits, sel, weights, ids, rank, hist, (int)T, chunks,
-                       fill, p);
+                       fill, p, st);
   });
   if (int rc = check_launch("route_rank")) return rc;
   if (blocks > 1) {
     hipLaunchKernelGGL(route_rows_kernel, dim3(blocks), dim3(kLanes), layout_words((int)E) * sizeof(int32_t), s,
-                       weights, ids, rank, hist, (int)T, (int)E, (int)K, chunks, p);
+                       weights, ids, rank, hist, (int)T, (int)E, (int)K, chunks, p, st);
     return check_launch("route_rows");
   }
   return MI355_OK;
+}
+
+extern "C" int mi355_route_plan(const float* partial, int splits, const float* logit_bias, float* logits,
+                                const float* expert_bias, int64_t T, int64_t E, int64_t K, int score_func,
+                                int route_norm, float route_scale, int num_groups, int num_limited, float* weights,
+                                int64_t* ids, int64_t lo, int64_t hi, int64_t align, int64_t tile_m,
+                                int32_t* counts_E, int32_t* seg_offsets, int32_t* seg_counts, int32_t* row_of_slot,
+                                int32_t* slot_of_row, int32_t* token_of_row, float* row_scale, int64_t row_capacity,
+                                int32_t* tile_expert, int32_t* tile_row0, int32_t* num_tiles, int64_t tile_capacity,
+                                void* workspace, void* stream) {
+  return route_plan(partial, splits, logit_bias, logits, expert_bias, T, E, K, score_func, route_norm, route_scale,
+                    num_groups, num_limited, weights, ids, lo, hi, align, tile_m, counts_E, seg_offsets, seg_counts,
+                    row_of_slot, slot_of_row, token_of_row, row_scale, row_capacity, tile_expert, tile_row0, num_tiles,
+                    tile_capacity, workspace, StatsOut{}, stream);
+}
+
+extern "C" int mi355_route_plan_stats(
+    const float* partial, int splits, const float* logit_bias, float* logits, const float* expert_bias, int64_t T,
+    int64_t E, int64_t K, int score_func, int route_norm, float route_scale, int num_groups, int num_limited,
+    float* weights, int64_t* ids, int64_t lo, int64_t hi, int64_t align, int64_t tile_m, int32_t* counts_E,
+    int32_t* seg_offsets, int32_t* seg_counts, int32_t* row_of_slot, int32_t* slot_of_row, int32_t* token_of_row,
+    float* row_scale, int64_t row_capacity, int32_t* tile_expert, int32_t* tile_row0, int32_t* num_tiles,
+    int64_t tile_capacity, void* workspace, const uint8_t* padding_mask_T, int32_t* valid_counts_E, float* scores_TE,
+    float* cutoff_T, float* aux_f_E, float* aux_scale, void* aux_acc, int aux_acc_dtype, const float* aux_denominator, float aux_coeff,
+    void* stats_workspace, void* stream) {
+  MI355_REQUIRE(!cutoff_T || K < E, "route_plan_stats: top_k (%lld) must leave a (K+1)-th expert of %lld", (long long)K,
+                (long long)E);
+  MI355_REQUIRE(!aux_f_E || (aux_scale && aux_denominator), "route_plan_stats: the loss needs scale and denominator");
+  MI355_REQUIRE(!aux_acc || aux_acc_dtype == MI355_F32 || aux_acc_dtype == MI355_BF16, "route_plan_stats: aux_acc is fp32 or bf16");
+  MI355_REQUIRE((!aux_f_E && !valid_counts_E) || stats_workspace, "route_plan_stats: workspace required");
+  int32_t* block_valid = static_cast<int32_t*>(stats_workspace);
+  float* block_share = block_valid ? reinterpret_cast<float*>(block_valid + (T >= 1 ? route_blocks(T) : 0) * E) : nullptr;
+  const StatsOut st{padding_mask_T, valid_counts_E, scores_TE, cutoff_T, aux_f_E, aux_scale, aux_acc, aux_acc_dtype, aux_denominator,
+                    aux_coeff, block_valid, block_share};
+  return route_plan(partial, splits, logit_bias, logits, expert_bias, T, E, K, score_func, route_norm, route_scale,
+                    num_groups, num_limited, weights, ids, lo, hi, align, tile_m, counts_E, seg_offsets, seg_counts,
+                    row_of_slot, slot_of_row, token_of_row, row_scale, row_capacity, tile_expert, tile_row0, num_tiles,
+                    tile_capacity, workspace, st, stream);
 }

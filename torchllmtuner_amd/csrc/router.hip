@@ -319,10 +319,17 @@ __device__ __forceinline__ float slot_dweight(const DotPieces& d, const float* d
   return sum;
 }
 
+// The load-balance loss's part of the score gradient (aux.hip's formula), for the tokens that are not padding.
+struct BalanceGrad {
+  const float* f;  // (E) or null: no loss
+  const float* scale;
+  const uint8_t* padding;
+};
+
 template <int VPL>
 __global__ __launch_bounds__(256) void select_bwd_kernel(
     const float* __restrict__ logits, const int64_t* __restrict__ ids,
-    const float* __restrict__ dweights, const float* __restrict__ dscores, DotPieces dots,
+    const float* __restrict__ dweights, const float* __restrict__ dscores, DotPieces dots, BalanceGrad bal,
     float* __restrict__ dlogits, int T, int E, int K, int score_func, int route_norm,
     float route_scale, int mode) {
   extern __shared__ float lds[];  // per wave: sc[E], ds[E]
@@ -337,12 +344,30 @@ __global__ __launch_bounds__(256) void select_bwd_kernel(
   float s[VPL];
   float xs[VPL];
   compute_scores<VPL>(row, E, lane, score_func, s, xs);
+  float bal_mean = 0.0f, bal_inv = 0.0f;
+  if (bal.f && !(bal.padding && bal.padding[t])) {
+    float sum = 0.0f, dot = 0.0f;
+#pragma unroll
+    for (int j = 0; j < VPL; ++j) {
+      const int e = lane + j * kWave;
+      sum += e < E ? s[j] : 0.0f;
+      dot += e < E ? s[j] * bal.f[e] : 0.0f;
+    }
+    sum = wave_sum_dpp(sum);
+    dot = wave_sum_dpp(dot);
+    // below the clamp the normalised score is s / eps and the sum no longer enters
+    const float inv = 1.0f / fmaxf(sum, 1e-12f);
+    bal_mean = sum < 1e-12f ? 0.0f : dot * inv;
+    bal_inv = *bal.scale * inv;
+  }
 #pragma unroll
   for (int j = 0; j < VPL; ++j) {
     const int e = lane + j * kWave;
     if (e < E) {
       sc[e] = s[j];
-      ds[e] = dscores ? dscores[static_cast<int64_t>(t) * E + e] : 0.0f;
+      float d = dscores ? dscores[static_cast<int64_t>(t) * E + e] : 0.0f;
+      if (bal.f) d += (bal.f[e] - bal_mean) * bal_inv;
+      ds[e] = d;
     }
   }
   __syncthreads();
@@ -605,8 +630,8 @@ extern "C" int mi355_router_select_cutoff_fwd(const float* logits, const float* 
 }
 
 static int select_bwd(const float* logits, const int64_t* ids, const float* dweights, const float* dscores_TE,
-                      const DotPieces& dots, float* dlogits, int64_t T, int64_t E, int64_t K, int score_func,
-                      int route_norm, float route_scale, int select_mode, void* stream) {
+                      const DotPieces& dots, const BalanceGrad& bal, float* dlogits, int64_t T, int64_t E, int64_t K,
+                      int score_func, int route_norm, float route_scale, int select_mode, void* stream) {
   if (int rc = check_router_args(T, E, K)) return rc;
   MI355_REQUIRE(K <= 64, "router_select_bwd: top_k > 64 unsupported");
   if (T == 0) return MI355_OK;
@@ -614,7 +639,7 @@ static int select_bwd(const float* logits, const int64_t* ids, const float* dwei
   const dim3 grid((unsigned)((T + 3) / 4));
   const size_t lds = (size_t)4 * 2 * E * sizeof(float);
   DISPATCH_VPL(E, hipLaunchKernelGGL(select_bwd_kernel<VPL>, grid, dim3(256), lds, as_stream(stream),
-                                     logits, ids, dweights, dscores_TE, dots, dlogits, (int)T, (int)E,
+                                     logits, ids, dweights, dscores_TE, dots, bal, dlogits, (int)T, (int)E,
                                      (int)K, score_func, route_norm, route_scale, select_mode));
   return check_launch("router_select_bwd");
 }
@@ -624,17 +649,21 @@ extern "C" int mi355_router_select_bwd(const float* logits, const int64_t* ids,
                                        float* dlogits, int64_t T, int64_t E, int64_t K,
                                        int score_func, int route_norm, float route_scale,
                                        int select_mode, void* stream) {
-  return select_bwd(logits, ids, dweights, dscores_TE, DotPieces{}, dlogits, T, E, K, score_func, route_norm,
+  return select_bwd(logits, ids, dweights, dscores_TE, DotPieces{}, BalanceGrad{}, dlogits, T, E, K, score_func, route_norm,
                     route_scale, select_mode, stream);
 }
 
-extern "C" int mi355_router_select_dots_bwd(const float* logits, const int64_t* ids, const float* dot_partial,
+extern "C" int mi355_router_select_dots_bwd(const float* logits, const int64_t* ids, const float* dots,
                                             int64_t pieces, const int32_t* row_of_slot, int64_t row_capacity,
+                                            const float* aux_f_E, const float* aux_scale, const uint8_t* padding_mask_T,
                                             float* dlogits, int64_t T, int64_t E, int64_t K, int score_func,
                                             int route_norm, float route_scale, void* stream) {
-  MI355_REQUIRE(pieces >= 1 && pieces <= 4096 && row_capacity >= 0 && row_capacity < (1ll << 31),
+  MI355_REQUIRE(pieces >= 0 && pieces <= 4096 && row_capacity >= 0 && row_capacity < (1ll << 31),
                 "router_select_dots_bwd: bad shape");
-  MI355_REQUIRE(T == 0 || (dot_partial && row_of_slot), "router_select_dots_bwd: null pointer");
-  return select_bwd(logits, ids, nullptr, nullptr, DotPieces{dot_partial, row_of_slot, (int)pieces, (int)row_capacity},
-                    dlogits, T, E, K, score_func, route_norm, route_scale, MI355_SELECT_TOPK, stream);
+  MI355_REQUIRE(T == 0 || (dots && (pieces == 0 || row_of_slot)), "router_select_dots_bwd: null pointer");
+  MI355_REQUIRE(!aux_f_E || aux_scale, "router_select_dots_bwd: the loss needs its scale");
+  return select_bwd(logits, ids, pieces ? nullptr : dots, nullptr,
+                    pieces ? DotPieces{dots, row_of_slot, (int)pieces, (int)row_capacity} : DotPieces{},
+                    BalanceGrad{aux_f_E, aux_scale, padding_mask_T}, dlogits, T, E, K, score_func, route_norm, route_scale,
+                    MI355_SELECT_TOPK, stream);
 }

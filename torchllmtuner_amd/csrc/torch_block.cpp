@@ -35,23 +35,31 @@ using torch::autograd::variable_list;
 
 struct Config {
   int64_t K, score_func, route_norm, num_groups, num_limited, lo, hi, align, round_terms, overlap;
+  int64_t aux;  // the router injects a load-balance loss
   double route_scale;
 
   std::vector<int64_t> pack() const {
-    std::vector<int64_t> v{K, score_func, route_norm, num_groups, num_limited, lo, hi, align, round_terms, overlap, 0};
-    std::memcpy(&v[10], &route_scale, sizeof(double));
+    std::vector<int64_t> v{K, score_func, route_norm, num_groups, num_limited, lo, hi, align, round_terms, overlap, aux, 0};
+    std::memcpy(&v[11], &route_scale, sizeof(double));
     return v;
   }
   static Config unpack(const std::vector<int64_t>& v) {
-    Config c{v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9], 0.0};
-    std::memcpy(&c.route_scale, &v[10], sizeof(double));
+    Config c{v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9], v[10], 0.0};
+    std::memcpy(&c.route_scale, &v[11], sizeof(double));
     return c;
   }
 };
 
+// What a router that keeps statistics brings; undefined / zero where it keeps none.  Written in the forward.
+struct Stats {
+  Tensor histogram, aux_acc, aux_denominator;
+  double aux_coeff = 0.0;
+  Tensor mask;  // (T) bool, true = padding
+};
+
 // The block's tensors; undefined where the block has none.
 struct Block {
-  Tensor x, gate_w, gate_b, expert_b, w1, w3, w2, sg, su, sd;
+  Tensor x, gate_w, gate_b, expert_b, w1, w3, w2, sg, su, sd, mask;
   Config c;
   int64_t T, D, E, F, El, N, R, Fs, tile_m, tile_cap, shared_cap;
   int dt, gate_dt;
@@ -105,7 +113,7 @@ Tensor carve(const Tensor& like, Layout layout) {
 // activations, the shared expert's plan and activations.
 struct Kept {
   int64_t* ids;
-  float *weights, *logits, *row_scale;
+  float *weights, *logits, *row_scale, *aux_f = nullptr, *aux_scale = nullptr;
   int32_t *seg_offsets, *seg_counts, *tile_expert, *tile_row0, *num_tiles, *row_of_slot, *slot_of_row, *token_of_row;
   int32_t *s_offsets, *s_counts, *s_expert, *s_row0, *s_num;
   void *pieces = nullptr, *rows = nullptr, *gate = nullptr, *up = nullptr, *h = nullptr, *y = nullptr;
@@ -126,6 +134,10 @@ struct Kept {
     tile_expert = c.take<int32_t>(b.tile_cap);
     tile_row0 = c.take<int32_t>(b.tile_cap);
     num_tiles = c.take<int32_t>(1);
+    if (b.c.aux) {
+      aux_f = c.take<float>(b.E);
+      aux_scale = c.take<float>(1);
+    }
     if (b.piece_bytes > 0) pieces = c.take(b.piece_bytes, 1);
     if (save || !b.folded) {  // (gate and up are the other kernels' own intermediates)
       gate = c.take(b.R * b.F, item);
@@ -186,7 +198,7 @@ void shared_forward(const Block& b, const Kept& k, void* y, void* stream) {
 }
 
 // (output, counts per expert, what the backward reads)
-std::tuple<Tensor, Tensor, Tensor> block_forward(const Block& b, bool save) {
+std::tuple<Tensor, Tensor, Tensor> block_forward(const Block& b, const Stats& st, bool save) {
   Launch L(b.x);
   const Config& c = b.c;
   const auto opts = b.x.options();
@@ -200,10 +212,22 @@ std::tuple<Tensor, Tensor, Tensor> block_forward(const Block& b, bool save) {
   const int64_t partial_bytes = b.splits > 1 ? b.splits * b.T * b.E * 4
                                 : b.splits == 0 ? mi355_router_gate_fwd_workspace_bytes(b.T, b.D, b.E) : 0;
   const int64_t plan_bytes = mi355_route_plan_workspace_bytes(b.T, c.K, b.E);
+  const bool stats = b.mask.defined() || c.aux;
+  float *scores = nullptr, *cutoff = nullptr;
+  void* stats_work = nullptr;
+  int32_t* all_counts = nullptr;  // the plan's counts where `counts` leaves the padding out
   void *gate_work = nullptr, *plan_work = nullptr, *y_shared = nullptr, *h = k.h, *y = k.y;
   Tensor scratch = carve(b.x, [&](Carver& cv) {
     if (partial_bytes > 0) gate_work = cv.take(partial_bytes, 1);
     if (plan_bytes > 0) plan_work = cv.take(plan_bytes, 1);
+    if (stats) {
+      stats_work = cv.take(mi355_route_stats_workspace_bytes(b.T, b.E), 1);
+      all_counts = cv.take<int32_t>(b.E);
+    }
+    if (st.histogram.defined()) {
+      scores = cv.take<float>(b.T * b.E);
+      cutoff = cv.take<float>(b.T);
+    }
     if (b.Fs > 0) y_shared = cv.take(b.T * b.D, item);
     if (b.folded) {
       h = cv.take(b.R * b.F, item);
@@ -232,13 +256,21 @@ std::tuple<Tensor, Tensor, Tensor> block_forward(const Block& b, bool save) {
     check(mi355_router_gate_fwd(ptr(b.x), b.dt, ptr(b.gate_w), b.gate_dt, fptr(gate_b), k.logits, gate_work, b.T, b.D,
                                 b.E, L.stream),
           "router_gate_fwd");
-  check(mi355_route_plan(partial, b.splits > 1 ? b.splits : 1, fptr(gate_b), save && b.splits > 1 ? k.logits : nullptr,
-                         fptr(expert_b), b.T, b.E, c.K, (int)c.score_func, (int)c.route_norm, (float)c.route_scale,
-                         (int)c.num_groups, (int)c.num_limited, k.weights, k.ids, c.lo, c.hi, c.align, b.tile_m,
-                         counts.data_ptr<int32_t>(), k.seg_offsets, k.seg_counts, k.row_of_slot, k.slot_of_row,
-                         k.token_of_row, save && b.folded ? k.row_scale : nullptr, b.R, k.tile_expert, k.tile_row0,
-                         k.num_tiles, b.tile_cap, plan_work, L.stream),
+  const uint8_t* padding = static_cast<const uint8_t*>(ptr(b.mask));
+  check(mi355_route_plan_stats(
+            partial, b.splits > 1 ? b.splits : 1, fptr(gate_b), save && b.splits > 1 ? k.logits : nullptr, fptr(expert_b),
+            b.T, b.E, c.K, (int)c.score_func, (int)c.route_norm, (float)c.route_scale, (int)c.num_groups,
+            (int)c.num_limited, k.weights, k.ids, c.lo, c.hi, c.align, b.tile_m,
+            stats ? all_counts : counts.data_ptr<int32_t>(), k.seg_offsets, k.seg_counts, k.row_of_slot, k.slot_of_row,
+            k.token_of_row, save && b.folded ? k.row_scale : nullptr, b.R, k.tile_expert, k.tile_row0, k.num_tiles,
+            b.tile_cap, plan_work, padding, stats ? counts.data_ptr<int32_t>() : nullptr, scores, cutoff, k.aux_f,
+            k.aux_scale, ptr(st.aux_acc), st.aux_acc.defined() ? dtype_code(st.aux_acc) : MI355_F32, fptr(st.aux_denominator), (float)st.aux_coeff, stats_work,
+            L.stream),
         "route_plan");
+  if (st.histogram.defined())
+    check(mi355_quantile_observe(scores, cutoff, fptr(expert_b), padding, st.histogram.data_ptr<int64_t>(), b.T, b.E,
+                                 st.histogram.size(1), L.stream),
+          "quantile_observe");
 
   // routed experts
   if (!b.folded)
@@ -365,6 +397,12 @@ Grads block_backward(const Block& b, const Tensor& kept, const Tensor& dout_, co
     check(mi355_permute_rows_add_bwd(drows, b.dt, k.row_of_slot, dx_shared, dx_routed, b.T, b.D, c.K, L.stream),
           "permute_rows_bwd");
   };
+  auto select = [&]() {
+    check(mi355_router_select_dots_bwd(k.logits, k.ids, dots, slots, k.row_of_slot, b.R, k.aux_f, k.aux_scale,
+                                       static_cast<const uint8_t*>(ptr(b.mask)), dlogits, b.T, b.E, c.K,
+                                       (int)c.score_func, (int)c.route_norm, (float)c.route_scale, L.stream),
+          "router_select_bwd");
+  };
   if (b.folded) {
     auto run = [&](int stages, void* stream) {
       check(mi355_grouped_swiglu_combine_bwd(ptr(dout), ptr(b.x), k.token_of_row, b.T, k.row_scale, ptr(b.w1), ptr(b.w3),
@@ -383,10 +421,7 @@ Grads block_backward(const Block& b, const Tensor& kept, const Tensor& dout_, co
     }
     if (need.x) run(MI355_STAGE_DX, L.stream);
     row_sum();
-    if (logits)
-      check(mi355_router_select_dots_bwd(k.logits, k.ids, dots, slots, k.row_of_slot, b.R, dlogits, b.T, b.E, c.K,
-                                         (int)c.score_func, (int)c.route_norm, (float)c.route_scale, L.stream),
-            "router_select_bwd");
+    if (logits) select();
     if (need.experts && !side) run(kWeights, L.stream);
   } else {
     const int32_t* pad = c.align > 1 ? k.slot_of_row : nullptr;
@@ -399,10 +434,7 @@ Grads block_backward(const Block& b, const Tensor& kept, const Tensor& dout_, co
                                      dgate, dup, drows, ptr(g.w1), ptr(g.w3), ptr(g.w2), b.El, b.D, b.F, b.R, L.stream),
             "grouped_swiglu_bwd");
     row_sum();
-    if (logits)
-      check(mi355_router_select_bwd(k.logits, k.ids, dots, nullptr, dlogits, b.T, b.E, c.K, (int)c.score_func,
-                                    (int)c.route_norm, (float)c.route_scale, MI355_SELECT_TOPK, L.stream),
-            "router_select_bwd");
+    if (logits) select();
   }
 
   // ---- router gate; the input gradient is complete with its part
@@ -422,12 +454,13 @@ OptTensor opt(const Tensor& t) { return t.defined() ? OptTensor(t) : std::nullop
 struct MoeBlock : public torch::autograd::Function<MoeBlock> {
   static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& gate_w, const OptTensor& gate_b,
                                const OptTensor& expert_b, const Tensor& w1, const Tensor& w3, const Tensor& w2,
-                               const OptTensor& sg, const OptTensor& su, const OptTensor& sd, const Config& c) {
+                               const OptTensor& sg, const OptTensor& su, const OptTensor& sd, const Config& c,
+                               const Stats& st) {
     at::AutoDispatchBelowADInplaceOrView below;
-    Block b{x, gate_w, some(gate_b), some(expert_b), w1, w3, w2, some(sg), some(su), some(sd), c};
+    Block b{x, gate_w, some(gate_b), some(expert_b), w1, w3, w2, some(sg), some(su), some(sd), st.mask, c};
     b.sizes();
-    auto [out, counts, kept] = block_forward(b, true);
-    ctx->save_for_backward({x, gate_w, b.gate_b, w1, w3, w2, b.sg, b.su, b.sd, kept});
+    auto [out, counts, kept] = block_forward(b, st, true);
+    ctx->save_for_backward({x, gate_w, b.gate_b, w1, w3, w2, b.sg, b.su, b.sd, kept, b.mask});
     auto packed = c.pack();
     packed.push_back(b.expert_b.defined());
     ctx->saved_data["config"] = packed;
@@ -436,11 +469,11 @@ struct MoeBlock : public torch::autograd::Function<MoeBlock> {
     return {out, counts};
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    variable_list out(11);
+    variable_list out(12);
     if (!grads[0].defined()) return out;
     const auto s = ctx->get_saved_variables();
     const auto packed = ctx->saved_data["config"].toIntVector();
-    Block b{s[0], s[1], s[2], Tensor(), s[3], s[4], s[5], s[6], s[7], s[8], Config::unpack(packed)};
+    Block b{s[0], s[1], s[2], Tensor(), s[3], s[4], s[5], s[6], s[7], s[8], s[10], Config::unpack(packed)};
     b.sizes();
     // needs_input_grad counts the tensors among the arguments: an absent one has no index
     const int gb = 2, w = gb + (b.gate_b.defined() ? 1 : 0) + (packed.back() ? 1 : 0), sh = w + 3;
@@ -474,7 +507,9 @@ std::tuple<Tensor, Tensor> moe_block(const Tensor& x_, const Tensor& gate_w_, co
                                      const Tensor& w2_, const OptTensor& sg_, const OptTensor& su_,
                                      const OptTensor& sd_, int64_t K, int64_t score_func, bool route_norm,
                                      double route_scale, int64_t num_groups, int64_t num_limited, int64_t lo,
-                                     int64_t hi, int64_t align, bool round_terms, bool overlap_shared) {
+                                     int64_t hi, int64_t align, bool round_terms, bool overlap_shared,
+                                     const OptTensor& mask_, const OptTensor& histogram_,
+                                     const OptTensor& aux_denominator_, double aux_coeff, const OptTensor& aux_acc_) {
   const Tensor x = x_.contiguous(), gate_w = gate_w_.contiguous(), w1 = w1_.contiguous(), w3 = w3_.contiguous(),
                w2 = w2_.contiguous();
   const Tensor gate_b = contiguous(gate_b_), expert_b = contiguous(expert_b_), sg = contiguous(sg_),
@@ -504,15 +539,32 @@ std::tuple<Tensor, Tensor> moe_block(const Tensor& x_, const Tensor& gate_w_, co
   for (const Tensor* t : {&gate_w, &gate_b, &expert_b, &w1, &w3, &w2, &sg, &su, &sd})
     TORCH_CHECK(!t->defined() || t->device() == x.device(), "moe_block: tensors on different devices: ", x.device(),
                 " and ", t->device());
-  const Config c{K, score_func, route_norm, num_groups, num_limited, lo, hi, align, round_terms, overlap_shared, route_scale};
+  const Tensor mask = contiguous(mask_);
+  const Stats st{some(histogram_), some(aux_acc_), some(aux_denominator_), aux_coeff, mask};
+  TORCH_CHECK_VALUE(!mask.defined() || (mask.scalar_type() == at::kBool && mask.numel() == x.size(0) &&
+                                        mask.device() == x.device()),
+                    "padding mask: one bool per token on the tokens' device");
+  TORCH_CHECK_VALUE(!st.histogram.defined() ||
+                        (st.histogram.scalar_type() == at::kLong && st.histogram.is_contiguous() &&
+                         st.histogram.dim() == 2 && st.histogram.size(0) == gate_w.size(0) &&
+                         st.histogram.device() == x.device() && expert_b.defined()),
+                    "histogram: contiguous int64 (experts, bins) beside an expert bias");
+  auto scalar = [&](const Tensor& t) { return !t.defined() || (t.numel() == 1 && t.device() == x.device()); };
+  TORCH_CHECK_VALUE(scalar(st.aux_acc) && scalar(st.aux_denominator) &&
+                        (!st.aux_denominator.defined() || st.aux_denominator.scalar_type() == at::kFloat) &&
+                        (!st.aux_acc.defined() || st.aux_acc.scalar_type() == at::kFloat ||
+                         st.aux_acc.scalar_type() == at::kBFloat16),
+                    "auxiliary loss: scalars on the tokens' device, the denominator fp32, the metric fp32 or bf16");
+  const Config c{K, score_func, route_norm, num_groups, num_limited, lo, hi, align, round_terms, overlap_shared,
+                 st.aux_denominator.defined(), route_scale};
   if (torch::autograd::compute_requires_grad(x, gate_w, gate_b, w1, w3, w2, sg, su, sd)) {
-    auto r = MoeBlock::apply(x, gate_w, opt(gate_b), opt(expert_b), w1, w3, w2, opt(sg), opt(su), opt(sd), c);
+    auto r = MoeBlock::apply(x, gate_w, opt(gate_b), opt(expert_b), w1, w3, w2, opt(sg), opt(su), opt(sd), c, st);
     return {r[0], r[1]};
   }
   at::AutoDispatchBelowADInplaceOrView below;
-  Block b{x, gate_w, gate_b, expert_b, w1, w3, w2, sg, su, sd, c};
+  Block b{x, gate_w, gate_b, expert_b, w1, w3, w2, sg, su, sd, mask, c};
   b.sizes();
-  auto [out, counts, kept] = block_forward(b, false);
+  auto [out, counts, kept] = block_forward(b, st, false);
   return {out, counts};
 }
 
@@ -523,7 +575,8 @@ TORCH_LIBRARY_FRAGMENT(mi355_moe, m) {
       "moe_block(Tensor x, Tensor gate_w, Tensor? gate_bias, Tensor? expert_bias, Tensor w1, Tensor w3, Tensor w2, "
       "Tensor? shared_gate, Tensor? shared_up, Tensor? shared_down, int top_k, int score_func, bool route_norm, "
       "float route_scale, int num_groups, int num_limited, int local_lo, int local_hi, int align, bool round_terms, "
-      "bool overlap_shared) -> (Tensor, Tensor)");
+      "bool overlap_shared, Tensor? padding_mask, Tensor(a!)? histogram, Tensor? aux_denominator, float aux_coeff, "
+      "Tensor(b!)? aux_acc) -> (Tensor, Tensor)");
 }
 TORCH_LIBRARY_IMPL(mi355_moe, CUDA, m) { m.impl("moe_block", moe_block); }
 TORCH_LIBRARY_IMPL(mi355_moe, Autograd, m) { m.impl("moe_block", moe_block); }

@@ -19,10 +19,10 @@ import torch
 import torch.nn as nn
 
 from .. import ops
-from .auxiliary_loss import in_checkpoint_recompute
+from .auxiliary_loss import AuxLoss, MicrobatchWiseLoadBalanceLoss, in_checkpoint_recompute
 from .experts import DenseSwiGLU, GroupedExperts, RoutedExperts, _is_own_dispatcher
 from .linear import RouterGateLinear
-from .routing import QuantileBalancedTopKRouter, TokenChoiceTopKRouter
+from .routing import QuantileBalancedTopKRouter, QuantileBalancer, TokenChoiceTopKRouter
 
 __all__ = ["MoE", "in_checkpoint_recompute"]
 
@@ -183,11 +183,54 @@ class MoE(nn.Module):
             weights.append(linear._parameters["weight"])
         return weights if all(w.dtype is dtype for w in weights) else None
 
-    def _forward_as_one(self, tokens: torch.Tensor):
+    def _router_statistics(self, router, tokens):
+        """Keywords of ``ops.moe_block`` for what the router keeps in training -- the quantile router's
+        histogram, the load-balance loss -- or None when that is not this package's own, un-overridden."""
+        stats = {}
+        recompute = in_checkpoint_recompute.get()
+        if type(router) is QuantileBalancedTopKRouter:
+            balancer = router._modules["quantile_balancer"]
+            if (
+                type(balancer) is not QuantileBalancer
+                or "observe" in balancer.__dict__
+                or "_select_observing" in router.__dict__
+                or self.expert_bias_E.dtype is not torch.float32
+            ):
+                return None
+            if balancer.training and not recompute:
+                stats["histogram"] = balancer.required_bias_histogram_EB
+        aux = router.aux_loss
+        if aux is not None:
+            if (
+                not _plain(aux, MicrobatchWiseLoadBalanceLoss)
+                or "inject" in aux.__dict__
+                or aux.token_replication_size != 1
+            ):
+                return None
+            denominator = aux._runtime_denominator if aux._runtime_denominator is not None else AuxLoss._step_denominator
+            if (
+                denominator is None
+                or denominator.dtype is not torch.float32
+                or denominator.numel() != 1
+                or denominator.device != tokens.device
+                or denominator.requires_grad
+                or aux.instance_acc.dtype not in _BLOCK_DTYPES
+                or aux.instance_acc.device != tokens.device
+            ):
+                return None
+            stats["aux_denominator"] = denominator
+            stats["aux_coeff"] = float(aux.coeff)
+            if not recompute:
+                stats["aux_acc"] = aux.instance_acc
+        return stats
+
+    def _forward_as_one(self, tokens: torch.Tensor, padding_mask: torch.Tensor | None = None):
         """``(output, counts per expert)`` from the one operator that computes the whole block
         (``mi355_moe::moe_block``), or None when a stage has to be visible or is not what it computes: a
-        hook or an override anywhere below, an observer, an auxiliary loss, another router, dispatcher,
-        activation or shared expert, fp64, no tokens, a tracing compiler.  Both ways give the same bits."""
+        hook or an override anywhere below, an observer, another auxiliary loss, router, dispatcher,
+        activation or shared expert, fp64, no tokens, a tracing compiler.  Both ways give the same bits
+        (the load-balance loss: the same sums in another order).  In training the counts leave out the
+        tokens of ``padding_mask``."""
         if (
             torch.compiler.is_compiling()
             or type(tokens) not in (torch.Tensor, nn.Parameter)
@@ -199,13 +242,14 @@ class MoE(nn.Module):
             return None
         modules = self._modules
         router, routed = modules["router"], modules["routed_experts"]
-        if not _plain(router, TokenChoiceTopKRouter) or not _plain(routed, RoutedExperts):
+        if not (_plain(router, TokenChoiceTopKRouter) or _plain(router, QuantileBalancedTopKRouter)):
+            return None
+        if not _plain(routed, RoutedExperts):
             return None
         d = router.__dict__
         if (
             router.fixed_router
             or router._debug_force_load_balance
-            or (router.aux_loss is not None and self.training)
             or "_select" in d
             or not ops.route_plan_covers(router.num_experts, router.top_k, router.num_expert_groups)
         ):
@@ -226,12 +270,24 @@ class MoE(nn.Module):
         shared = self._shared_weights(dtype)
         if shared is None or w1.dtype is not dtype or w3.dtype is not dtype or w2.dtype is not dtype:
             return None
+        stats = {}
+        if router.training != self.training or (type(router) is QuantileBalancedTopKRouter and self.expert_bias_E is None):
+            return None
+        if self.training:
+            if router.aux_loss is not None or type(router) is QuantileBalancedTopKRouter:
+                stats = self._router_statistics(router, tokens)
+                if stats is None:
+                    return None
+            if padding_mask is not None:
+                if padding_mask.device != tokens.device:
+                    return None
+                stats["padding_mask"] = padding_mask
         lo, hi = dispatcher._local_range()
         return ops.moe_block(
             tokens, gate_weight, gate._parameters["bias"], self.expert_bias_E, w1, w3, w2, shared,
             router.top_k, router.score_func, router.route_norm, router.route_scale, router.num_expert_groups,
             router.num_limited_groups, lo, hi, dispatcher._align(), not dispatcher.accumulate_in_fp32,
-            self.overlap_shared_experts)
+            self.overlap_shared_experts, **stats)
 
     def set_padding_mask(self, padding_mask: torch.Tensor | None) -> None:
         self._pending_padding_mask = padding_mask
@@ -252,15 +308,14 @@ class MoE(nn.Module):
                     f"got {tuple(padding_mask.shape)} for {tokens.shape[0]} tokens."
                 )
 
-        if padding_mask is None:
-            whole = self._forward_as_one(tokens)
-            if whole is not None:
-                out_TD, num_tokens_per_expert_E = whole
-                if self.training and not in_checkpoint_recompute.get():
-                    self.tokens_per_expert_E.add_(num_tokens_per_expert_E)  # (neither takes part in autograd)
-                if restore_shape:
-                    out_TD = out_TD.reshape(*x.shape[:-1], out_TD.shape[-1])
-                return (out_TD, None) if self.returns_router_logits else out_TD
+        whole = self._forward_as_one(tokens, padding_mask)
+        if whole is not None:
+            out_TD, num_tokens_per_expert_E = whole
+            if self.training and not in_checkpoint_recompute.get():
+                self.tokens_per_expert_E.add_(num_tokens_per_expert_E)  # (neither takes part in autograd)
+            if restore_shape:
+                out_TD = out_TD.reshape(*x.shape[:-1], out_TD.shape[-1])
+            return (out_TD, None) if self.returns_router_logits else out_TD
 
         shared_TD, shared_stream = self._start_shared_experts(tokens)
 
