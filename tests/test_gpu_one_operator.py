@@ -119,6 +119,26 @@ def test_router_statistics_of_the_one_operator_match_the_stages(quantile, masked
         assert err < (2e-3 if i == 2 else 4e-3 if a.dtype == torch.bfloat16 else 2e-6), f"tensor {i}: {err}"
 
 
+@pytest.mark.parametrize("E,K,T", [(5, 5, 3), (16, 4, 65), (60, 16, 64), (128, 8, 130), (256, 1, 33)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_selection_among_equal_values_takes_the_lower_experts(E, K, T, bias):
+    """Integer keys of the choice values (csrc/select_rows.h): whole-number logits with many ties, both zeros,
+    -inf; with a bias (of zeros) the choice is by score, whose ties are the logits'."""
+    from torchllmtuner_amd import ops
+
+    print(f"selection ties E={E} K={K} T={T} bias={bias}", flush=True)
+    g = torch.Generator().manual_seed(E)
+    x = torch.randint(-2, 3, (T, E), generator=g).float()
+    x[x == 0] *= torch.where(torch.rand(int((x == 0).sum()), generator=g) < 0.5, -1.0, 1.0)
+    x[:, ::3] = torch.where(torch.rand(T, (E + 2) // 3, generator=g) < 0.2, float("-inf"), x[:, ::3])
+    if bias:  # scores of -inf and of logits far below are equal zeros or not: keep the ties exact
+        x = x.clamp(min=-2)
+    w, ids, _ = ops.router_select_fwd(x.to(DEV), torch.zeros(E, device=DEV) if bias else None, K, "sigmoid", False, 1.0)
+    want = torch.sort(x + 0.0, dim=1, descending=True, stable=True).indices[:, :K]
+    assert torch.equal(ids.cpu(), want)
+    assert torch.allclose(w.cpu(), torch.sigmoid(x).gather(1, want), rtol=1e-6, atol=0)
+
+
 @pytest.mark.parametrize("dtype,T,D,E", [
     (torch.bfloat16, 1, 8, 1), (torch.bfloat16, 33, 2056, 33), (torch.bfloat16, 1000, 7168, 256), (torch.bfloat16, 32, 1024, 66),
     (torch.float32, 1, 4, 3), (torch.float32, 31, 1028, 32), (torch.float32, 2000, 640, 10), (torch.float32, 4, 3000, 5)])

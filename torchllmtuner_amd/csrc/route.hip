@@ -1,7 +1,7 @@
 // Expert choice and permutation plan in one pass: what mi355_router_select_fwd followed by
 // mi355_permute_plan compute, for the block's own path, in one launch (up to 64 tokens) or two.
 //
-//   1. route_rank   a workgroup of 1024 lanes takes 64 tokens at a time: each row of 16 lanes adds its
+//   1. route_rank   a workgroup takes 32 or 64 tokens at a time: each row of 16 lanes adds its
 //                   token's partial logits, selects its experts (select_rows.h) and leaves the ids
 //                   in LDS, where the workgroup ranks its slots among equal experts in slot order
 //                   (the wave's lanes by ballots over the bits of the id, the waves through
@@ -10,10 +10,11 @@
 //                   slots' offsets (all of them, for the segments), which costs it a read of a few
 //                   dozen KiB from L2 and saves the launch of a scan, and writes its slots' rows in
 //                   both directions; the first workgroup writes the plan's lists.
-// A single workgroup does both at once.  Bound by launches and dependent latency throughout: at 33
+// A single workgroup does both at once.  Bound by launches, instruction issue and dependent latency throughout: at 33
 // tokens of 128 experts the four launches this replaces took 29 us of GPU time, at 8192 tokens
-// (8 each) 39 us; here 9 and 21.
+// (8 each) 39 us; here 12 and 23.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "select_rows.h"
@@ -21,9 +22,9 @@
 namespace mi355 {
 namespace {
 
-constexpr int kLanes = 1024, kRows = kLanes / 16, kWaves = kLanes / kWave;
-// 64 tokens of at most 16 choices are at most 1024 slots, one per lane; beyond this many workgroups
-// a workgroup takes several such chunks, so that the histograms everyone reads stay small
+// A workgroup of LANES takes LANES / 16 tokens at a time; of at most 16 choices they are at most LANES slots,
+// one per lane.  Beyond this many workgroups a workgroup takes several such chunks, so that the histograms
+// everyone reads stay small.
 constexpr int kMaxBlocks = 256;
 
 struct PlanOut {
@@ -59,13 +60,15 @@ struct LayoutLds {
 };
 constexpr int layout_words(int E) { return 5 * E + 2 + 8; }
 
-// inclusive sum over the wave
-__device__ __forceinline__ int wave_scan(int v, int lane) {
-#pragma unroll
-  for (int o = 1; o < kWave; o <<= 1) {
-    const int below = __shfl_up(v, o, kWave);
-    v += lane >= o ? below : 0;
-  }
+// inclusive sum over the wave: within the rows of 16 lanes, then lane 15 of each odd row's
+// predecessor, then lane 31 for the upper half
+__device__ __forceinline__ int wave_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
   return v;
 }
 
@@ -80,8 +83,8 @@ __device__ void plan_layout(const LayoutLds& s, const PlanOut& p, bool lists) {
     const int c = tid < El ? s.count[p.lo + tid] : 0;
     rows = p.align > 1 ? (c + p.align - 1) / p.align * p.align : c;
     tiles = (c + p.tile_m - 1) / p.tile_m;
-    rows_to = wave_scan(rows, lane);
-    tiles_to = wave_scan(tiles, lane);
+    rows_to = wave_scan(rows);
+    tiles_to = wave_scan(tiles);
     if (lane == 63) {
       s.wave_sums[wave] = rows_to;
       s.wave_sums[4 + wave] = tiles_to;
@@ -108,11 +111,8 @@ __device__ void plan_layout(const LayoutLds& s, const PlanOut& p, bool lists) {
       const int j = idx % El, o0 = (idx / El) * slice, o1 = min(El, o0 + slice);
       const int c = s.count[p.lo + j];
       int rank = 0;
-#pragma unroll 4
-      for (int o = o0; o < o1; ++o) {
-        const int co = s.count[p.lo + o];
-        rank += (co > c || (co == c && o < j)) ? 1 : 0;
-      }
+#pragma unroll 8
+      for (int o = o0; o < o1; ++o) rank += s.count[p.lo + o] > c - (o < j ? 1 : 0) ? 1 : 0;  // more, or as many and before it
       if (rank) atomicAdd(&s.order[j], rank);
     }
   }
@@ -120,9 +120,9 @@ __device__ void plan_layout(const LayoutLds& s, const PlanOut& p, bool lists) {
 }
 
 __device__ void write_lists(const LayoutLds& s, const PlanOut& p, int E) {
-  const int El = p.hi - p.lo, tid = threadIdx.x;
-  for (int e = tid; e < E; e += kLanes) p.counts_E[e] = s.count[e];
-  for (int j = tid; j <= El; j += kLanes) {
+  const int El = p.hi - p.lo, tid = threadIdx.x, lanes = blockDim.x;
+  for (int e = tid; e < E; e += lanes) p.counts_E[e] = s.count[e];
+  for (int j = tid; j <= El; j += lanes) {
     p.seg_offsets[j] = s.seg[j];
     if (j == El) {
       *p.num_tiles = min(s.tile[El], p.tile_capacity);
@@ -208,12 +208,13 @@ __device__ void finish_stats(const StatsOut& st, int E, int nb, float* red) {
   }
 }
 
-template <int VPR, bool FULL>
+template <int VPR, bool FULL, int kLanes>
 __global__ __launch_bounds__(kLanes) void route_rank_kernel(
     const float* __restrict__ partial, int splits, const float* __restrict__ logit_bias,
     float* __restrict__ logits_out, SelectArgs sel, float* __restrict__ weights, int64_t* __restrict__ ids,
     uint32_t* __restrict__ rank_in_block, int32_t* __restrict__ block_hist, int T, int chunks, int fill, PlanOut p,
     StatsOut st) {
+  constexpr int kRows = kLanes / 16, kWaves = kLanes / kWave;
   extern __shared__ int32_t lds[];
   const int E = sel.E, K = sel.K;
   int32_t* run = lds;                       // [E] slots of each expert so far
@@ -254,11 +255,16 @@ __global__ __launch_bounds__(kLanes) void route_rank_kernel(
       const int t = live ? t_raw : T - 1;
       float x[VPR], s[VPR], cutoff;
       load_row<VPR, FULL>(partial + static_cast<int64_t>(t) * E, l, E, x);
-      for (int z = 1; z < splits; ++z) {
-        float y[VPR];
-        load_row<VPR, FULL>(partial + (static_cast<int64_t>(z) * T + t) * E, l, E, y);
+      constexpr int kAhead = VPR >= 16 ? 2 : 4;  // partial sums requested together
+      for (int z0 = 1; z0 < splits; z0 += kAhead) {
+        float y[kAhead][VPR];
 #pragma unroll
-        for (int j = 0; j < VPR; ++j) x[j] += y[j];
+        for (int i = 0; i < kAhead; ++i)
+          load_row<VPR, FULL>(partial + (static_cast<int64_t>(min(z0 + i, splits - 1)) * T + t) * E, l, E, y[i]);
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i)
+#pragma unroll
+          for (int j = 0; j < VPR; ++j) x[j] = z0 + i < splits ? x[j] + y[i][j] : x[j];
       }
       if (splits > 1 && logit_bias) {
 #pragma unroll
@@ -270,7 +276,7 @@ __global__ __launch_bounds__(kLanes) void route_rank_kernel(
         for (int j = 0; j < VPR; ++j)
           if (FULL || l * VPR + j < E) logits_out[static_cast<int64_t>(t) * E + l * VPR + j] = x[j];
       }
-      const RowChoice ch = select_row<VPR, FULL>(sel, x, l, st.cutoff != nullptr, s, cutoff);
+      const RowChoice ch = select_row<VPR, FULL>(sel, x, l, st.scores || st.f, st.cutoff != nullptr, s, cutoff);
       if (st.scores && live) {
 #pragma unroll
         for (int j = 0; j < VPR; ++j)
@@ -326,12 +332,13 @@ __global__ __launch_bounds__(kLanes) void route_rank_kernel(
     }
     __syncthreads();
     for (int i = tid; i < E; i += kLanes) {
-      int r = run[i];
+      int r = run[i], v[kWaves];  // (all read before the first write: the compiler sees one array)
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) v[w] = cnt[w * E + i];
 #pragma unroll
       for (int w = 0; w < kWaves; ++w) {
-        const int v = cnt[w * E + i];
         cnt[w * E + i] = r;
-        r += v;
+        r += v[w];
       }
       run[i] = r;
     }
@@ -367,6 +374,7 @@ __global__ __launch_bounds__(kLanes) void route_rank_kernel(
   if (tid < T * K && tid < kRows * K) place_slot(s, p, tid, my_e, my_rank, K, w_sh[tid]);
 }
 
+template <int kLanes>
 __global__ __launch_bounds__(kLanes) void route_rows_kernel(const float* __restrict__ weights,
                                                             const int64_t* __restrict__ ids,
                                                             const uint32_t* __restrict__ rank_in_block,
@@ -404,7 +412,8 @@ __global__ __launch_bounds__(kLanes) void route_rows_kernel(const float* __restr
     write_lists(s, p, E);
     if (st.valid_counts || st.f) finish_stats(st, E, gridDim.x, red_sh);
   }
-  const int first = blockIdx.x * chunks * kRows * K, last = min(T * K, first + chunks * kRows * K);
+  const int per_block = chunks * (kLanes / 16) * K;
+  const int first = blockIdx.x * per_block, last = min(T * K, first + per_block);
   for (int slot = first + tid; slot < last; slot += kLanes) {
     const int64_t e = ids[slot];
     place_slot(s, p, slot, e >= 0 && e < E ? static_cast<int>(e) : -1, static_cast<int>(rank_in_block[slot]), K,
@@ -412,13 +421,25 @@ __global__ __launch_bounds__(kLanes) void route_rows_kernel(const float* __restr
   }
 }
 
+// Lanes per workgroup.  Selection is bound by instruction issue, so its tokens want to be spread over the
+// CUs; but every workgroup of route_rows reads all histograms, so there should not be more than two hundred
+// or so.  Both kernels together at 128 experts, 1024 / 512 / 256 lanes: 21 / 15 / 16 us at 1000 tokens, 22 / 19 / 26 at
+// 4096, 23 / 22 / 30 at 8192.  Up to 64 tokens one workgroup does everything.
+int route_lanes(int64_t T) { return T > 64 && T < 8192 ? 512 : 1024; }
 int route_chunks(int64_t T) {
-  const int64_t groups = (T + kRows - 1) / kRows;
+  const int64_t rows = route_lanes(T) / 16, groups = (T + rows - 1) / rows;
   return static_cast<int>((groups + kMaxBlocks - 1) / kMaxBlocks);
 }
 int64_t route_blocks(int64_t T) {
-  const int64_t per = static_cast<int64_t>(route_chunks(T)) * kRows;
+  const int64_t per = static_cast<int64_t>(route_chunks(T)) * (route_lanes(T) / 16);
   return (T + per - 1) / per;
+}
+// calls f(integral_constant lanes)
+template <typename Fn>
+void with_lanes(int64_t T, Fn f) {
+  const int lanes = route_lanes(T);
+  if (lanes == 512) f(std::integral_constant<int, 512>{});
+  else f(std::integral_constant<int, 1024>{});
 }
 
 }  // namespace
@@ -431,7 +452,7 @@ extern "C" int mi355_route_plan_covers(int64_t E, int64_t K, int num_groups, int
 }
 
 extern "C" int64_t mi355_route_plan_workspace_bytes(int64_t T, int64_t K, int64_t E) {
-  if (T <= kRows || K < 1 || E < 1) return 0;
+  if (K < 1 || E < 1 || T < 1 || route_blocks(T) == 1) return 0;
   return (T * K + route_blocks(T) * E) * (int64_t)sizeof(int32_t);
 }
 extern "C" int64_t mi355_route_stats_workspace_bytes(int64_t T, int64_t E) {
@@ -463,7 +484,7 @@ static int route_plan(const float* partial, int splits, const float* logit_bias,
   MI355_REQUIRE(partial && splits >= 1 && aligned16(partial) && weights && ids && counts_E && seg_offsets &&
                     seg_counts && row_of_slot && slot_of_row && token_of_row && tile_expert && tile_row0 && num_tiles,
                 "route_plan: null or misaligned pointer");
-  MI355_REQUIRE(T <= kRows || workspace, "route_plan: workspace required");
+  MI355_REQUIRE(route_blocks(T) == 1 || workspace, "route_plan: workspace required");
   hipStream_t s = as_stream(stream);
   const SelectArgs sel{expert_bias, (int)E, (int)K, score_func, route_norm, route_scale, num_groups, num_limited};
   const PlanOut p{(int)lo, (int)hi, (int)align, (int)tile_m, (int)row_capacity, (int)tile_capacity, counts_E,
@@ -476,16 +497,21 @@ static int route_plan(const float* partial, int splits, const float* logit_bias,
   // every row has a slot when all experts are local and nothing is padded
   const int fill = !(lo == 0 && hi == E && align == 1 && row_capacity == T * K);
   const bool stats = st.valid_counts || st.f;
-  const size_t lds = ((1 + kWaves) * E * (stats ? 2 : 1) + (blocks == 1 ? layout_words((int)E) : 0)) * sizeof(int32_t);
+  const int waves = route_lanes(T) / kWave;
+  const size_t lds = ((1 + waves) * E * (stats ? 2 : 1) + (blocks == 1 ? layout_words((int)E) : 0)) * sizeof(int32_t);
   with_row_shape(E, [&](auto vpr, auto full) {
-    hipLaunchKernelGGL((route_rank_kernel<decltype(vpr)::value, decltype(full)::value>), dim3(blocks), dim3(kLanes),
-                       lds, s, partial, splits, logit_bias, logits, sel, weights, ids, rank, hist, (int)T, chunks,
-                       fill, p, st);
+    with_lanes(T, [&](auto lanes) {
+      hipLaunchKernelGGL((route_rank_kernel<decltype(vpr)::value, decltype(full)::value, decltype(lanes)::value>), dim3(blocks),
+                         dim3(lanes), lds, s, partial, splits, logit_bias, logits, sel, weights, ids, rank, hist, (int)T,
+                         chunks, fill, p, st);
+    });
   });
   if (int rc = check_launch("route_rank")) return rc;
   if (blocks > 1) {
-    hipLaunchKernelGGL(route_rows_kernel, dim3(blocks), dim3(kLanes), layout_words((int)E) * sizeof(int32_t), s,
-                       weights, ids, rank, hist, (int)T, (int)E, (int)K, chunks, p, st);
+    with_lanes(T, [&](auto lanes) {
+      hipLaunchKernelGGL(route_rows_kernel<decltype(lanes)::value>, dim3(blocks), dim3(lanes), layout_words((int)E) * sizeof(int32_t),
+                         s, weights, ids, rank, hist, (int)T, (int)E, (int)K, chunks, p, st);
+    });
     return check_launch("route_rows");
   }
   return MI355_OK;

@@ -249,7 +249,7 @@ __global__ __launch_bounds__(256) void select_rows_kernel(
   const int e0 = l * VPR;
   float x[VPR], s[VPR], cutoff = 0.0f;
   load_row<VPR, FULL>(logits + static_cast<int64_t>(t) * E, l, E, x);
-  const RowChoice c = select_row<VPR, FULL>(p, x, l, cutoff_out != nullptr, s, cutoff);
+  const RowChoice c = select_row<VPR, FULL>(p, x, l, scores_out != nullptr, cutoff_out != nullptr, s, cutoff);
   if (!live) return;
   if (scores_out) {
     float* dst = scores_out + static_cast<int64_t>(t) * E + e0;
