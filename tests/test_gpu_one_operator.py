@@ -229,3 +229,36 @@ def test_gate_gradients_of_few_experts_match_fp64(dtype, T, D, E):
                                 ("dw", dw, dl.double().T @ x.double(), 1e-6)):
         err = float((got.double().cpu() - exp).norm() / exp.norm())
         assert err < tol, f"{name}: rel-L2 {err}"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("D,K,addend", [(2056, 8, True), (8, 1, False), (516, 11, True), (70, 3, True)])
+def test_combine_of_few_tokens_equals_that_of_many(dtype, D, K, addend):
+    """The combine deals a row's columns over waves below 4096 tokens: the tokens of a 4096-token call, bit for
+    bit, with absent slots, more than eight slots and rows that are not whole 16-byte pieces; and fp64 sums."""
+    from torchllmtuner_amd import _lib
+
+    print(f"combine {dtype} D={D} K={K}", flush=True)
+    lib, T, code = _lib.load(), 4096, 0 if dtype == torch.float32 else 1
+    g = torch.Generator().manual_seed(D)
+    y = torch.randn(500, D, generator=g).to(dtype).to(DEV)
+    add = torch.randn(T, D, generator=g).to(dtype).to(DEV) if addend else None
+    w = torch.rand(T, K, generator=g).to(DEV)
+    rows = torch.randint(-1, 500, (T, K), generator=g, dtype=torch.int32).to(DEV)
+
+    def run(n):
+        out = torch.full((n, D), float("nan"), dtype=dtype, device=DEV)
+        rc = lib.mi355_combine_add_fwd(y.data_ptr(), code, w.data_ptr(), rows.data_ptr(), add.data_ptr() if addend else None,
+                                       out.data_ptr(), n, D, K, 0, torch.cuda.current_stream().cuda_stream)
+        _lib.check(rc, "combine_fwd")
+        return out
+
+    many = run(T)
+    for n in (1, 5, 4095):
+        assert torch.equal(run(n), many[:n])
+    terms = torch.where((rows >= 0)[..., None], y.double()[rows.clamp(min=0).long()] * w.double()[..., None], 0.0)
+    want = terms.sum(1) + (add.double() if addend else 0.0)
+    # one rounding of the sum and one of the addition; fp32 sums of K terms
+    tol = (2 ** -8 * 2 if dtype == torch.bfloat16 else 2 ** -24 * (K + 2))
+    scale = terms.abs().sum(1) + (add.double().abs() if addend else 0.0)
+    assert bool(((many.double() - want).abs() <= tol * scale + 1e-30).all())

@@ -3,6 +3,9 @@
 // lanes along D, the K row indices and weights held in lanes 0..K-1 and broadcast
 // by shuffles.  No atomics: every output element has exactly one writer, so the
 // result is deterministic.
+#include <algorithm>
+#include <type_traits>
+
 #include "common.h"
 
 namespace mi355 {
@@ -53,8 +56,9 @@ __device__ __forceinline__ void plus(float (&a)[Vec<T>::N], const uint4& v) {
   for (int q = 0; q < Vec<T>::N; ++q) a[q] = round_to<T>(a[q]) + f[q];
 }
 
-// SMALL_K: K <= 8, the eight-row chunk below is the only one
-template <typename T, bool SMALL_K>
+// SMALL_K: K <= 8, the eight-row chunk below is the only one.  Pieces of G vectors per lane are dealt over
+// gridDim.y.
+template <typename T, bool SMALL_K, int G>
 __global__ __launch_bounds__(256) void combine_fwd_kernel(
     const T* __restrict__ y, const float* __restrict__ weights,
     const int32_t* __restrict__ row_of_slot, const T* __restrict__ addend, T* __restrict__ out, int T_, int D, int K,
@@ -88,10 +92,10 @@ __global__ __launch_bounds__(256) void combine_fwd_kernel(
   // Loops are uniform across the wave (shuffles need every lane).
   if (D % V == 0) {
     const int nv = D / V;
-    // G vectors per lane and pass (4 KiB of every row per wave) from eight rows at a time, all
+    // G vectors per lane and pass (4 KiB of every row per wave with G = 4) from eight rows at a time, all
     // requested before the first is used: 32 KiB in flight per wave.  Rows and weights are
     // wave-uniform; the terms are still added in visiting order.
-    constexpr int G = 4, B = 8;
+    constexpr int B = 8;
     auto request = [&](int base, int p0, uint4 (&v)[B][G], float (&ww)[B]) {
 #pragma unroll
       for (int j = 0; j < B; ++j) {
@@ -115,7 +119,7 @@ __global__ __launch_bounds__(256) void combine_fwd_kernel(
         a[q] += round_terms ? round_to<T>(term) : term;
       }
     };
-    for (int base = 0; base < nv; base += G * kWave) {
+    for (int base = blockIdx.y * G * kWave; base < nv; base += gridDim.y * G * kWave) {
       if constexpr (SMALL_K) {
         // one chunk: each vector is summed and stored on its own (8 live accumulators, not 32,
         // which is what lets three waves share a SIMD)
@@ -164,7 +168,7 @@ __global__ __launch_bounds__(256) void combine_fwd_kernel(
       }
     }
   } else {
-    for (int base = 0; base < D; base += kWave) {
+    for (int base = blockIdx.y * kWave; base < D; base += gridDim.y * kWave) {
       const int i = base + lane;
       const bool on = i < D;
       float a = 0.0f;
@@ -353,19 +357,28 @@ extern "C" int mi355_combine_add_fwd(const void* y, int dtype, const float* weig
   if (T == 0) return MI355_OK;
   MI355_REQUIRE(weights && row_of_slot && out, "combine_fwd: null pointer");
   MI355_REQUIRE(!addend || dtype != MI355_F64, "combine_fwd: no fp64 form with an addend");
-  const dim3 grid((unsigned)((T + 3) / 4));
+  // Few tokens: one wave a token leaves most of the chip idle and a wide row to several passes of one wave, so
+  // a wave takes 1 KiB of the row instead of 4.  4 KiB / 1 KiB a wave, eight rows of 2048 columns a token: 1 token 6.0 /
+  // 3.9 us, 33 7.7 / 5.0, 1000 12.7 / 10.8, 8192 52.5 / 54.5; 3000 tokens of 6 x 1024 15.0 / 11.5; 128 of 7168 columns
+  // 22.4 / 5.0.
+  const bool spread = T < 4096;
+  const int64_t pieces = (D * (dtype == MI355_F32 ? 4 : 2) + 1023) / 1024;  // 64 lanes of 16 bytes
+  const dim3 grid((unsigned)((T + 3) / 4), spread ? (unsigned)std::min<int64_t>(pieces, 1024) : 1);
   auto launch = [&](auto kernel, auto* yp, auto* op) {
     hipLaunchKernelGGL(kernel, grid, dim3(256), 0, as_stream(stream), yp, weights, row_of_slot,
                        static_cast<decltype(yp)>(addend), op, (int)T, (int)D, (int)K, round_terms);
   };
+  auto run = [&](auto* yp, auto* op) {
+    using E = std::remove_pointer_t<decltype(op)>;
+    if (K <= 8) launch(spread ? combine_fwd_kernel<E, true, 1> : combine_fwd_kernel<E, true, 4>, yp, op);
+    else launch(spread ? combine_fwd_kernel<E, false, 1> : combine_fwd_kernel<E, false, 4>, yp, op);
+  };
   if (dtype == MI355_F32) {
-    if (K <= 8) launch(combine_fwd_kernel<float, true>, static_cast<const float*>(y), static_cast<float*>(out));
-    else launch(combine_fwd_kernel<float, false>, static_cast<const float*>(y), static_cast<float*>(out));
+    run(static_cast<const float*>(y), static_cast<float*>(out));
   } else if (dtype == MI355_BF16) {
-    if (K <= 8) launch(combine_fwd_kernel<uint16_t, true>, static_cast<const uint16_t*>(y), static_cast<uint16_t*>(out));
-    else launch(combine_fwd_kernel<uint16_t, false>, static_cast<const uint16_t*>(y), static_cast<uint16_t*>(out));
+    run(static_cast<const uint16_t*>(y), static_cast<uint16_t*>(out));
   } else if (dtype == MI355_F64) {
-    hipLaunchKernelGGL(combine_fwd_f64_kernel, grid, dim3(256), 0, as_stream(stream), static_cast<const double*>(y),
+    hipLaunchKernelGGL(combine_fwd_f64_kernel, dim3(grid.x), dim3(256), 0, as_stream(stream), static_cast<const double*>(y),
                        weights, row_of_slot, static_cast<double*>(out), (int)T, (int)D, (int)K);
   } else
     return fail(MI355_EINVAL, "combine_fwd: unknown dtype %d", dtype);
