@@ -181,6 +181,7 @@ def test_forward_experts_of_few_rows_match_fp32(counts, D, F):
 
 
 @pytest.mark.parametrize("dtype,counts,D,F", [
+    (torch.float32, [33, 31, 0, 32, 1], 160, 1028), (torch.float32, [5], 36, 28), (torch.float32, [2100], 60, 68),
     (torch.float32, [1, 0, 65], 4, 8), (torch.float32, [130, 3], 68, 36), (torch.float32, [200, 57, 300], 132, 260),
     (torch.bfloat16, [1, 0, 65], 4, 8), (torch.bfloat16, [130, 3], 68, 36), (torch.bfloat16, [0, 257], 124, 380),
     (torch.float32, [700] * 12, 640, 516), (torch.bfloat16, [700] * 12, 652, 644)])

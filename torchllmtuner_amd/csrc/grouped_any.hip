@@ -12,10 +12,13 @@
 // make up for the difference.
 //   Products and their fused ends: gate and up in one pass with SwiGLU; down; dh with the SwiGLU
 // backward; drows as one contraction over both halves; all three weight gradients in one launch.
-//   What bounds them at the sizes they are for is latency: few tiles, short contractions.  Small tiles
-// (64 rows) are used until the large ones fill the chip.  Before, nine launches of a 64x64 tile fed by
-// scalar loads plus two elementwise passes did this: 512 tokens of 8 fp32 experts of 256 x 512, forward
-// and backward, 210 us of GPU time; 1531 tokens of 16 bf16 experts of 320 x 232, 543 us.
+//   What bounds them at the sizes they are for is latency and CUs without work: few tiles, short
+// contractions.  Small tiles are used until the large ones fill the chip: 64 rows, and for fp32 32 x 32, where
+// the four waves hold the same tile and split each step's contraction (their shares are added through LDS in
+// wave order) and four steps are requested ahead.
+//   512 tokens of 8 fp32 experts of 256 x 512, gate/up + down and the backward experts: 30 + 46 us on 64-row
+// tiles, 25 + 33 us now; 200 tokens of 16 of 640 x 1024, two each, 88 + 171 us, 49 + 97 now;
+// 1531 tokens of 16 bf16 experts of 320 x 232, 23 + 41 us.
 #include <algorithm>
 #include <type_traits>
 
@@ -138,11 +141,13 @@ __device__ __forceinline__ f32x16 any_mfma(const f32x4& b, const f32x4& a, f32x1
   return acc;
 }
 
-// LDS of one instantiation
+// LDS of one instantiation: two stages; on 32-row tiles also the four waves' partial tiles
 template <typename T, int MODE, int TM, int TN>
 constexpr int any_lds() {
   constexpr bool B_KS = MODE == ANY_DH || MODE == ANY_DX || MODE == ANY_KS || MODE == ANY_DW;
-  return 2 * (Operand<T, MODE == ANY_DW, TM>::ELEMS + Operand<T, B_KS, TN>::ELEMS);
+  constexpr int stages = 2 * (Operand<T, MODE == ANY_DW, TM>::ELEMS + Operand<T, B_KS, TN>::ELEMS);
+  constexpr int parts = TM == 32 ? 4 * 32 * TN * 4 / (int)sizeof(T) : 0;
+  return stages > parts ? stages : parts;
 }
 
 template <typename T, int MODE, int TM, int TN>
@@ -150,10 +155,15 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
   constexpr bool A_KS = MODE == ANY_DW, B_KS = MODE == ANY_DH || MODE == ANY_DX || MODE == ANY_KS || MODE == ANY_DW;
   using OA = Operand<T, A_KS, TM>;
   using OB = Operand<T, B_KS, TN>;
-  constexpr int BKE = OA::BKE, MI = TM / 64, NJ = TN / 64, KK = 128 / sizeof(T) / (sizeof(T) == 2 ? 16 : 8);
+  // 32-row tiles: every wave holds the whole tile and takes a quarter of each step's contraction
+  constexpr bool KSPLIT = TM == 32;
+  constexpr int BKE = OA::BKE, MI = KSPLIT ? 1 : TM / 64, NJ = KSPLIT ? TN / 32 : TN / 64;
+  constexpr int KK = 128 / sizeof(T) / (sizeof(T) == 2 ? 16 : 8);
+  static_assert(KK == 4, "a step's fragments are dealt to four waves");
+  constexpr int AHEAD = TM == 32 ? 4 : 1;  // steps requested ahead
   constexpr int STAGE = OA::ELEMS + OB::ELEMS;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave >> 1) * (TM / 2), wn = (wave & 1) * (TN / 2);
+  const int wm = KSPLIT ? 0 : (wave >> 1) * (TM / 2), wn = KSPLIT ? 0 : (wave & 1) * (TN / 2);
 
   // ---- which tile
   int m_valid, n0, N = p.N, M = 0, m0 = 0, K = p.K, k_rows = 0;
@@ -200,10 +210,6 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
     if (MODE == ANY_GATEUP || MODE == ANY_DX) B1 = static_cast<const T*>(p.b1) + w;
     b_bytes = (p.w_elems - (w - e * p.w_elems)) * static_cast<int64_t>(sizeof(T));
   }
-  const auto rsA0 = any_rsrc(A0, a_bytes), rsB0 = any_rsrc(B0, b_bytes);
-  const auto rsA1 = MODE == ANY_DX ? any_rsrc(A1, a_bytes) : rsA0;
-  const auto rsB1 = (MODE == ANY_GATEUP || MODE == ANY_DX) ? any_rsrc(B1, b_bytes) : rsB0;
-
   // ---- operand offsets (bytes): fixed per lane, plus the step's
   uint32_t offA[OA::N], offB[OB::N];
 #pragma unroll
@@ -219,38 +225,47 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
                     : static_cast<uint32_t>(min(r % b_rows, N - 1 - n0)) * ldb + c) * sizeof(T);
   }
   const int half_steps = (K + BKE - 1) / BKE, steps = MODE == ANY_DX ? 2 * half_steps : half_steps;
-  u32x4 ra[OA::N], rb[OB::N];
-  auto fetch = [&](int s) {
+  u32x4 ra[AHEAD][OA::N], rb[AHEAD][OB::N];
+  const auto rsA0 = any_rsrc(A0, a_bytes), rsB0 = any_rsrc(B0, b_bytes);
+  const auto rsA1 = MODE == ANY_DX ? any_rsrc(A1, a_bytes) : rsA0;
+  const auto rsB1 = (MODE == ANY_GATEUP || MODE == ANY_DX) ? any_rsrc(B1, b_bytes) : rsB0;
+  auto fetch = [&](int slot, int s) {
     const bool second = MODE == ANY_DX && s >= half_steps;
     const uint32_t k = static_cast<uint32_t>(second ? s - half_steps : s) * BKE;
     const uint32_t ka = (A_KS ? k * lda : k) * sizeof(T), kb = (B_KS ? k * ldb : k) * sizeof(T);
-#pragma unroll
-    for (int i = 0; i < OA::N; ++i)
-      ra[i] = __builtin_amdgcn_raw_buffer_load_b128(second ? rsA1 : rsA0, offA[i] + ka, 0, 0);
-#pragma unroll
-    for (int i = 0; i < OB::N; ++i) {
-      const bool up = MODE == ANY_GATEUP && i >= OB::N / 2;
-      rb[i] = __builtin_amdgcn_raw_buffer_load_b128(second || up ? rsB1 : rsB0, offB[i] + kb, 0, 0);
+    auto rsA = second ? rsA1 : rsA0, rsB = second ? rsB1 : rsB0, rsU = MODE == ANY_GATEUP ? rsB1 : rsB;
+    if constexpr (KSPLIT) {
+      // a step past the end reads as zero, without traffic, so that requests are unconditional and the
+      // compiler counts them exactly
+      const int64_t an = s < steps ? a_bytes : 0, bn = s < steps ? b_bytes : 0;
+      rsA = any_rsrc(second ? A1 : A0, an);
+      rsB = any_rsrc(second ? B1 : B0, bn);
+      rsU = MODE == ANY_GATEUP ? any_rsrc(B1, bn) : rsB;
     }
+#pragma unroll
+    for (int i = 0; i < OA::N; ++i) ra[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(rsA, offA[i] + ka, 0, 0);
+#pragma unroll
+    for (int i = 0; i < OB::N; ++i)
+      rb[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(i >= OB::N / 2 ? rsU : rsB, offB[i] + kb, 0, 0);
   };
-  auto park = [&](int s) {
+  auto park = [&](int slot, int s) {
     T* As = smem + (s & 1) * STAGE;
     T* Bs = As + OA::ELEMS;
     const int kv = K - (MODE == ANY_DX && s >= half_steps ? s - half_steps : s) * BKE;
     if (kv < BKE) {  // the tail: whatever was read past the contraction must not meet anything
 #pragma unroll
-      for (int i = 0; i < OA::N; ++i) ra[i] = OA::clip(ra[i], tid, i, kv);
+      for (int i = 0; i < OA::N; ++i) ra[slot][i] = OA::clip(ra[slot][i], tid, i, kv);
 #pragma unroll
-      for (int i = 0; i < OB::N; ++i) rb[i] = OB::clip(rb[i], tid, i, kv);
+      for (int i = 0; i < OB::N; ++i) rb[slot][i] = OB::clip(rb[slot][i], tid, i, kv);
     }
 #pragma unroll
-    for (int i = 0; i < OA::N; ++i) *reinterpret_cast<u32x4*>(As + OA::at(tid, i)) = ra[i];
+    for (int i = 0; i < OA::N; ++i) *reinterpret_cast<u32x4*>(As + OA::at(tid, i)) = ra[slot][i];
 #pragma unroll
-    for (int i = 0; i < OB::N; ++i) *reinterpret_cast<u32x4*>(Bs + OB::at(tid, i)) = rb[i];
+    for (int i = 0; i < OB::N; ++i) *reinterpret_cast<u32x4*>(Bs + OB::at(tid, i)) = rb[slot][i];
   };
   // column block j of the wave: GATEUP's first half of the blocks are gate columns, the second the same of up
   auto bcol = [&](int j) {
-    if constexpr (MODE == ANY_GATEUP) return (j < NJ / 2 ? 0 : TN / 2) + (wave & 1) * (TN / 4) + (j % (NJ / 2)) * 32;
+    if constexpr (MODE == ANY_GATEUP) return (j < NJ / 2 ? 0 : TN / 2) + (KSPLIT ? 0 : (wave & 1) * (TN / 4)) + (j % (NJ / 2)) * 32;
     else return wn + j * 32;
   };
   static_assert(MODE != ANY_GATEUP || NJ >= 2, "a wave of the gate/up product holds both of a column");
@@ -262,30 +277,70 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
     for (int j = 0; j < NJ; ++j)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-  if (steps > 0) {
-    fetch(0);
-    park(0);
-    if (steps > 1) fetch(1);
-  }
-  __syncthreads();
-  for (int s = 0; s < steps; ++s) {
-    if (s + 1 < steps) park(s + 1);
-    if (s + 2 < steps) fetch(s + 2);
-    const T* As = smem + (s & 1) * STAGE;
-    const T* Bs = As + OA::ELEMS;
+  auto multiply = [&](const T* As, const T* Bs, int kk) {
+    decltype(any_frag<A_KS, TM>(As, 0, 0, 0)) af[MI];
 #pragma unroll
-    for (int kk = 0; kk < KK; ++kk) {
-      decltype(any_frag<A_KS, TM>(As, 0, 0, 0)) af[MI];
+    for (int i = 0; i < MI; ++i) af[i] = any_frag<A_KS, TM>(As, wm + i * 32, kk, lane);
 #pragma unroll
-      for (int i = 0; i < MI; ++i) af[i] = any_frag<A_KS, TM>(As, wm + i * 32, kk, lane);
+    for (int j = 0; j < NJ; ++j) {
+      const auto bf = any_frag<B_KS, TN>(Bs, bcol(j), kk, lane);
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        const auto bf = any_frag<B_KS, TN>(Bs, bcol(j), kk, lane);
-#pragma unroll
-        for (int i = 0; i < MI; ++i) acc[i][j] = any_mfma(bf, af[i], acc[i][j]);
-      }
+      for (int i = 0; i < MI; ++i) acc[i][j] = any_mfma(bf, af[i], acc[i][j]);
+    }
+  };
+  if constexpr (!KSPLIT) {
+    if (steps > 0) {
+      fetch(0, 0);
+      park(0, 0);
+      if (steps > 1) fetch(0, 1);
     }
     __syncthreads();
+    for (int s = 0; s < steps; ++s) {
+      if (s + 1 < steps) park(0, s + 1);
+      if (s + 2 < steps) fetch(0, s + 2);
+      const T* As = smem + (s & 1) * STAGE;
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) multiply(As, As + OA::ELEMS, kk);
+      __syncthreads();
+    }
+  } else {
+    if (steps > 0) {
+#pragma unroll
+      for (int i = 0; i < AHEAD; ++i) fetch(i, i);
+      park(0, 0);
+      fetch(0, AHEAD);
+      phase_barrier();
+    }
+    for (int s0 = 0; s0 < steps; s0 += AHEAD) {
+#pragma unroll
+      for (int i = 0; i < AHEAD; ++i) {
+        const int s = s0 + i;
+        if (s >= steps) goto done;
+        if (s + 1 < steps) park((i + 1) % AHEAD, s + 1);
+        fetch((i + 1) % AHEAD, s + 1 + AHEAD);
+        const T* As = smem + (s & 1) * STAGE;
+        multiply(As, As + OA::ELEMS, wave);
+        phase_barrier();
+      }
+    }
+  done:
+    // quad q of every column block goes to wave q, which adds the four waves' shares in their order
+    f32x4* part = reinterpret_cast<f32x4*>(smem);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        part[((wave * NJ + j) * 4 + q) * 64 + lane] =
+            f32x4{acc[0][j][q * 4], acc[0][j][q * 4 + 1], acc[0][j][q * 4 + 2], acc[0][j][q * 4 + 3]};
+    phase_barrier();
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      f32x4 v = part[(j * 4 + wave) * 64 + lane];
+#pragma unroll
+      for (int w = 1; w < 4; ++w) v += part[((w * NJ + j) * 4 + wave) * 64 + lane];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[0][j][r] = v[r];
+    }
   }
 
   // ---- epilogue: lane = output row lane & 31 of the block, four consecutive columns per q
@@ -297,8 +352,8 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
 #pragma unroll
     for (int j = 0; j < (MODE == ANY_GATEUP ? NJ / 2 : NJ); ++j)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int n = n0 + (MODE == ANY_GATEUP ? (wave & 1) * (TN / 4) : wn) + j * 32 + q * 8 + 4 * (lane >> 5);
+      for (int q = 0; q < (KSPLIT ? 1 : 4); ++q) {
+        const int n = n0 + (KSPLIT ? wave * 8 : MODE == ANY_GATEUP ? (wave & 1) * (TN / 4) : wn) + j * 32 + q * 8 + 4 * (lane >> 5);
         if (n >= N) continue;  // N is a multiple of four
         const int64_t at = (MODE == ANY_DW ? static_cast<int64_t>(m0 + m) : row0 + m) * N + n;
         const f32x16& c = acc[i][j];
@@ -343,38 +398,49 @@ __global__ __launch_bounds__(256) void any_kernel(AnyArgs p) {
 
 // The input gradient and the weight gradients of a backward pass read the same buffers and write different
 // ones: with few tiles each they share a launch (at 512 fp32 tokens of 8 experts 26 + 16 us one after the
-// other).  The input gradient, the longer contraction, starts first.
-template <typename T, int TM>
-__global__ __launch_bounds__(256) void any_dx_dw_kernel(AnyArgs dx, AnyArgs dw, int dx_blocks) {
-  constexpr int A = any_lds<T, ANY_DX, TM, TM>(), B = any_lds<T, ANY_DW, TM, TM>();
+// other).  The longer contraction starts first.
+template <typename T, int TX, int TW>
+__global__ __launch_bounds__(256) void any_dx_dw_kernel(AnyArgs dx, AnyArgs dw, int dx_blocks, int dw_blocks, int dw_first) {
+  constexpr int A = any_lds<T, ANY_DX, TX, TX>(), B = any_lds<T, ANY_DW, TW, TW>();
   __shared__ __attribute__((aligned(16))) T smem[A > B ? A : B];
-  if (static_cast<int>(blockIdx.x) < dx_blocks) any_tile<T, ANY_DX, TM, TM>(dx, blockIdx.x, smem);
-  else any_tile<T, ANY_DW, TM, TM>(dw, blockIdx.x - dx_blocks, smem);
+  const int block = static_cast<int>(blockIdx.x) - (dw_first ? dw_blocks : 0);  // of dx
+  if (block >= 0 && block < dx_blocks) any_tile<T, ANY_DX, TX, TX>(dx, block, smem);
+  else any_tile<T, ANY_DW, TW, TW>(dw, dw_first ? blockIdx.x : block - dx_blocks, smem);
 }
 
 template <int MODE, int TM, int TN>
 int launch_any(const AnyArgs& p, int dtype, int64_t blocks, hipStream_t s, const char* what) {
   if (blocks <= 0) return MI355_OK;
-  if (dtype == MI355_F32) hipLaunchKernelGGL((any_kernel<float, MODE, TM, TN>), dim3((unsigned)blocks), dim3(256), 0, s, p);
-  else hipLaunchKernelGGL((any_kernel<uint16_t, MODE, TM, TN>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+  if (TM == 32 || dtype == MI355_F32) hipLaunchKernelGGL((any_kernel<float, MODE, TM, TN>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+  else if constexpr (TM != 32) hipLaunchKernelGGL((any_kernel<uint16_t, MODE, TM, TN>), dim3((unsigned)blocks), dim3(256), 0, s, p);
   return check_launch(what);
 }
 
-// Large tiles (128 x 128) once they give two workgroups for every CU; before that small ones (64 rows), whose
-// count is four times as large.
-bool rows_large(const AnyArgs& p, int64_t El, int64_t cols) {
-  return (p.rows / 128 + std::min(El, p.rows)) * ((cols + 127) / 128) >= 512;
+// Large tiles (128 x 128) once they give two workgroups for every CU; before that 64-row ones.  fp32 products
+// run on 32 x 32 tiles where 64-row ones leave CUs without work or, with few rows per expert, are mostly
+// padding: an fp32 step of a 64-row tile is 0.9 us of MFMA time on four waves, full or not.  Experts' forward
+// / backward in us, 64 against 32:
+//   few tiles: 40-80 (64 tokens of 8 experts, 256 x 512) 27 / 38 against 18 / 25, 96-192 29 / 44 against
+//     25 / 33, 216-432 (375 rows per expert) 40 / 61 against 48 / 74;
+//   16 experts of 640 x 1024: 25 rows each 88 / 171 against 49 / 97, 64 rows 90 / 201 against 74 / 153, 160 rows
+//     152 / 287 against 134 / 269, 225 rows 152 / 319 against 165 / 332.
+// bf16 steps are 16 times shorter and gain nothing (14 / 17 against 14 / 18, slower with more tiles).
+int row_tile(const AnyArgs& p, int dtype, int64_t El, int64_t cols) {
+  auto tiles = [&](int64_t t) { return (p.rows / t + std::min(El, p.rows)) * ((cols + t - 1) / t); };
+  if (dtype == MI355_F32 && (p.rows <= 160 * El || tiles(64) < 200)) return 32;
+  return tiles(128) >= 512 ? 128 : 64;
 }
 
 template <int MODE>
 int launch_rows(AnyArgs& p, int dtype, int64_t tile_capacity, int64_t El, int64_t cols, hipStream_t s, const char* what) {
   constexpr bool GU = MODE == ANY_GATEUP;
-  if (rows_large(p, El, cols)) {
-    p.col_tiles = (int)((cols + (GU ? 63 : 127)) / (GU ? 64 : 128));
-    return launch_any<MODE, 128, 128>(p, dtype, tile_capacity * 2 * p.col_tiles, s, what);
-  }
-  p.col_tiles = (int)((cols + 63) / 64);
-  return launch_any<MODE, 64, GU ? 128 : 64>(p, dtype, tile_capacity * 4 * p.col_tiles, s, what);
+  const int t = row_tile(p, dtype, El, cols), width = GU && t == 128 ? 64 : t;
+  p.col_tiles = (int)((cols + width - 1) / width);
+  const int64_t blocks = tile_capacity * (256 / t) * p.col_tiles;
+  MI355_REQUIRE(blocks < (1ll << 30), "%s: too many tiles", what);
+  if (t == 128) return launch_any<MODE, 128, 128>(p, dtype, blocks, s, what);
+  return t == 64 ? launch_any<MODE, 64, GU ? 128 : 64>(p, dtype, blocks, s, what)
+                 : launch_any<MODE, 32, GU ? 64 : 32>(p, dtype, blocks, s, what);
 }
 
 int64_t dw_tiles(AnyArgs& p, int64_t El, int tile) {
@@ -445,20 +511,29 @@ int any_backward(const AnySeg& g, int dtype, const void* dgate, const void* dup,
   for (int i = 0; i < count; ++i) w.dw[i] = {grads[i].a, grads[i].b, grads[i].c, (int)grads[i].M, (int)grads[i].N, 0, 0};
   w.num_dw = count;
   const bool dw_large = count && dw_tiles(w, g.El, 128) >= 512;
-  const int64_t tiles = count ? dw_tiles(w, g.El, dw_large ? 128 : 64) : 0;
+  int64_t tiles = count ? dw_tiles(w, g.El, dw_large ? 128 : 64) : 0;
+  const bool dw_small = dtype == MI355_F32 && tiles < 256;  // as in row_tile
+  if (dw_small) tiles = dw_tiles(w, g.El, 32);
   MI355_REQUIRE(tiles < (1ll << 30), "grouped weight gradients: too many tiles");
-  if (drows && count && !dw_large && !rows_large(p, g.El, D)) {
-    p.col_tiles = (int)((D + 63) / 64);
-    const int64_t dx_blocks = g.tile_capacity * 4 * p.col_tiles;
+  const int t = row_tile(p, dtype, g.El, D);
+  if (drows && count && !dw_large && t < 128) {
+    p.col_tiles = (int)((D + t - 1) / t);
+    const int64_t dx_blocks = g.tile_capacity * (256 / t) * p.col_tiles;
     MI355_REQUIRE(dx_blocks < (1ll << 30), "grouped drows: too many tiles");
     const dim3 grid((unsigned)(dx_blocks + tiles));
-    if (dtype == MI355_F32) hipLaunchKernelGGL((any_dx_dw_kernel<float, 64>), grid, dim3(256), 0, s, p, w, (int)dx_blocks);
-    else hipLaunchKernelGGL((any_dx_dw_kernel<uint16_t, 64>), grid, dim3(256), 0, s, p, w, (int)dx_blocks);
+    const int dw_first = R / g.El > 2 * F;
+    auto run = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, p, w, (int)dx_blocks, (int)tiles, dw_first);
+    };
+    if (dtype == MI355_BF16) run(any_dx_dw_kernel<uint16_t, 64, 64>);
+    else if (dw_small) run(t == 64 ? any_dx_dw_kernel<float, 64, 32> : any_dx_dw_kernel<float, 32, 32>);
+    else run(t == 64 ? any_dx_dw_kernel<float, 64, 64> : any_dx_dw_kernel<float, 32, 64>);
     return check_launch("grouped drows and weight gradients");
   }
   if (drows)
     if (int rc = launch_rows<ANY_DX>(p, dtype, g.tile_capacity, g.El, D, s, "grouped drows")) return rc;
   if (!count) return MI355_OK;
+  if (dw_small) return launch_any<ANY_DW, 32, 32>(w, dtype, tiles, s, "grouped weight gradients");
   return dw_large ? launch_any<ANY_DW, 128, 128>(w, dtype, tiles, s, "grouped weight gradients")
                   : launch_any<ANY_DW, 64, 64>(w, dtype, tiles, s, "grouped weight gradients");
 }
