@@ -263,3 +263,31 @@ def test_combine_of_few_tokens_equals_that_of_many(dtype, D, K, addend):
     tol = (2 ** -8 * 2 if dtype == torch.bfloat16 else 2 ** -24 * (K + 2))
     scale = terms.abs().sum(1) + (add.double().abs() if addend else 0.0)
     assert bool(((many.double() - want).abs() <= tol * scale + 1e-30).all())
+
+
+@pytest.mark.parametrize("dtype,rows,D", [
+    (torch.bfloat16, 1, 8), (torch.bfloat16, 5, 520), (torch.bfloat16, 513, 2048), (torch.bfloat16, 1, 2056),
+    (torch.bfloat16, 1030, 4096), (torch.bfloat16, 7, 4104), (torch.bfloat16, 515, 8192), (torch.bfloat16, 3, 8200),
+    (torch.bfloat16, 2, 16392), (torch.bfloat16, 9, 2051), (torch.float32, 1, 4), (torch.float32, 514, 1024),
+    (torch.float32, 3, 1028), (torch.float32, 600, 2052), (torch.float32, 1030, 5000), (torch.float32, 2, 8192),
+    (torch.float32, 5, 8196)])
+def test_rms_norm_rows_in_registers_match_fp64(dtype, rows, D):
+    """csrc/rmsnorm.hip at the ends of its row widths: one wave to a row, four, rows in memory."""
+    from torchllmtuner_amd import ops
+
+    print(f"rms {dtype} {rows} x {D}", flush=True)
+    g = torch.Generator().manual_seed(D)
+    x, dy = torch.randn(rows, D, generator=g).to(dtype), torch.randn(rows, D, generator=g).to(dtype)
+    w = (1 + 0.1 * torch.randn(D, generator=g)).to(dtype)
+    y, rstd = ops.rms_norm_fwd(x.to(DEV), w.to(DEV), 1e-6)
+    dx, dw = ops.rms_norm_bwd(dy.to(DEV), x.to(DEV), w.to(DEV), rstd)
+    ref = [t.double().requires_grad_() for t in (x, w)]
+    want = ref[0] * torch.rsqrt(ref[0].square().mean(-1, keepdim=True) + 1e-6) * ref[1]
+    want.backward(dy.double())
+    # one rounding to bf16 (half an ulp: 2^-9) per result; fp32 sums of D or of rows terms, relative to their norms
+    tol = 2 ** -8 if dtype == torch.bfloat16 else 2e-6
+    for name, got, exp in (("y", y, want.detach()), ("dx", dx, ref[0].grad), ("dw", dw, ref[1].grad)):
+        err = float((got.double().cpu() - exp).norm() / exp.norm())
+        assert err < tol, f"{name}: rel-L2 {err}"
+    only_dw = ops.rms_norm_bwd(dy.to(DEV), x.to(DEV), w.to(DEV), rstd, need_dx=False)[1]
+    assert torch.equal(only_dw, dw)

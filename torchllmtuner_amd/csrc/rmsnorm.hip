@@ -8,19 +8,18 @@
 // torch's CPU routine does for bf16 inputs.  Backward, with g = dy * w and xh = x * r:
 //   dx[t][d] = r_t * (g[t][d] - xh[t][d] * mean_d(g[t][.] * xh[t][.]))
 //   dw[d]    = sum_t dy[t][d] * xh[t][d]
-// HBM-bound: one wavefront per row for y and dx (16-byte lanes, the second pass over the
-// row comes from cache); dw as per-workgroup column sums over a run of rows, combined by a
-// second kernel in a fixed order (no atomics, deterministic).
+// HBM-bound: a row is held in registers by one wave or by four, read once, and reduced there; dw as
+// per-workgroup column sums over a run of rows, combined by a second kernel in a fixed order (no
+// atomics, deterministic).  Rows too wide for that, or not in whole 16-byte pieces, are read again.
 #include <algorithm>
 #include <initializer_list>
 #include <type_traits>
 
+#include "bf16_tiles.h"
 #include "common.h"
 
 namespace mi355 {
 namespace {
-
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // N consecutive elements as floats; N = 16 bytes' worth uses one 16-byte access
 template <typename T, int N>
@@ -65,6 +64,33 @@ struct Pack<uint16_t, 8> {
 template <typename T>
 constexpr int kVec = 16 / sizeof(T);
 
+// 16 bytes of T as N floats and back
+template <typename T, int N>
+__device__ __forceinline__ void unpack16(const u32x4& q, float (&v)[N]) {
+  if constexpr (std::is_same<T, float>::value) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = __uint_as_float(q[j]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      v[2 * j] = __uint_as_float(q[j] << 16);
+      v[2 * j + 1] = __uint_as_float(q[j] & 0xffff0000u);
+    }
+  }
+}
+template <typename T, int N>
+__device__ __forceinline__ u32x4 pack16(const float (&v)[N]) {
+  u32x4 q;
+  if constexpr (std::is_same<T, float>::value) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) q[j] = __float_as_uint(v[j]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) q[j] = pack_bf16x2(v[2 * j], v[2 * j + 1]);
+  }
+  return q;
+}
+
 template <typename T, int N>
 __device__ __forceinline__ float row_sumsq(const T* xr, int D, int lane) {
   float ss = 0.0f;
@@ -102,6 +128,66 @@ __global__ __launch_bounds__(256) void rms_fwd_kernel(const T* __restrict__ x, c
   const float ss = wave_sum(vec ? row_sumsq<T, kVec<T>>(xr, D, lane) : row_sumsq<T, 1>(xr, D, lane));
   const float r = 1.0f / sqrtf(ss / static_cast<float>(D) + eps);
   if (vec) row_scale<T, kVec<T>>(xr, w, yr, r, D, lane); else row_scale<T, 1>(xr, w, yr, r, D, lane);
+  if (lane == 0 && rstd) rstd[row] = r;
+}
+
+// Sum over a workgroup of four waves, in all lanes; `slot` alternates between calls, which makes one barrier
+// a call enough.  Global loads stay in flight across it.
+__device__ __forceinline__ float group_sum(float v, float (*red)[4], int slot) {
+  v = wave_sum(v);
+  if ((threadIdx.x & 63) == 0) red[slot][threadIdx.x >> 6] = v;
+  phase_barrier();
+  const float* r = red[slot];
+  return (r[0] + r[1]) + (r[2] + r[3]);
+}
+
+// The same with the row in registers between the sum and the scaling, requested at once: WAVES (1 or 4) to a
+// row, ITER sixteen-byte groups per lane.  Reading the row again for the scaling kept the kernel at 4.2-4.5 TB/s
+// (8192 / 32768 rows of 2048 bf16: 15.9 / 60 us, 12.6 / 41 now); four waves to a row once one would hold more than
+// four groups a lane.
+template <typename T, int WAVES, int ITER>
+__global__ __launch_bounds__(256) void rms_fwd_row_in_registers_kernel(const T* __restrict__ x, const T* __restrict__ w,
+                                                                       T* __restrict__ y, float* __restrict__ rstd,
+                                                                       int rows, int D, float eps) {
+  constexpr int N = kVec<T>, LANES = WAVES * kWave;
+  __shared__ float red[1][4];
+  const int lane = threadIdx.x % LANES;
+  const int row = blockIdx.x * (4 / WAVES) + threadIdx.x / LANES;
+  if (row >= rows) return;  // (four waves to a row: the grid has no such workgroup)
+  const int64_t o = static_cast<int64_t>(row) * D;
+  const u32x4 zero = {0, 0, 0, 0};
+  u32x4 q[ITER], g[ITER];
+#pragma unroll
+  for (int k = 0; k < ITER; ++k) {
+    const int i = (k * LANES + lane) * N;
+    q[k] = i < D ? *reinterpret_cast<const u32x4*>(x + o + i) : zero;
+  }
+#pragma unroll
+  for (int k = 0; k < ITER; ++k) {
+    const int i = (k * LANES + lane) * N;
+    g[k] = i < D ? *reinterpret_cast<const u32x4*>(w + i) : zero;
+  }
+  float ss = 0.0f;
+#pragma unroll
+  for (int k = 0; k < ITER; ++k) {
+    float v[N];
+    unpack16<T, N>(q[k], v);
+#pragma unroll
+    for (int j = 0; j < N; ++j) ss += v[j] * v[j];
+  }
+  ss = WAVES == 1 ? wave_sum(ss) : group_sum(ss, red, 0);
+  const float r = 1.0f / sqrtf(ss / static_cast<float>(D) + eps);
+#pragma unroll
+  for (int k = 0; k < ITER; ++k) {
+    const int i = (k * LANES + lane) * N;
+    if (i >= D) break;
+    float v[N], gv[N], out[N];
+    unpack16<T, N>(q[k], v);
+    unpack16<T, N>(g[k], gv);
+#pragma unroll
+    for (int j = 0; j < N; ++j) out[j] = (v[j] * r) * gv[j];
+    *reinterpret_cast<u32x4*>(y + o + i) = pack16<T, N>(out);
+  }
   if (lane == 0 && rstd) rstd[row] = r;
 }
 
@@ -149,95 +235,92 @@ __global__ __launch_bounds__(256) void rms_dx_kernel(const T* __restrict__ dy, c
 }
 
 // dx and the column sums of dweight in one pass over dy and x: a workgroup walks a run of
-// rows, one wavefront per row; a lane keeps the dweight partial sums of the columns it owns
-// in registers across its rows (ITER 16-byte groups per lane), the four waves add theirs up
-// through LDS at the end and the workgroup writes one row of partial sums.
+// rows and writes one row of partial sums.
 constexpr int kFusedBlocks = 2048;  // at most; 512 until a workgroup would get more than 32 rows
 
+// Four waves to a row, ITER sixteen-byte groups per lane: the row of dy and x is held in registers and the next
+// one requested before it is reduced (one barrier a row); a lane keeps the dweight sums of the columns it owns.
+// One wave to a row read the row twice and had too few in flight: 32768 rows of 4096 / 8192 bf16
+// 283 / 520 us, 144 / 334 now; fp32 rows beyond 4096 columns took two passes (16384 of 5000: 418, 204 now).
 template <typename T, int ITER>
-__global__ __launch_bounds__(256) void rms_bwd_fused_kernel(const T* __restrict__ dy, const T* __restrict__ x,
-                                                            const T* __restrict__ w,
-                                                            const float* __restrict__ rstd, T* __restrict__ dx,
-                                                            float* __restrict__ partial, int rows, int D,
-                                                            int rows_per_block) {
+__global__ __launch_bounds__(256) void rms_bwd_row_per_group_kernel(
+    const T* __restrict__ dy, const T* __restrict__ x, const T* __restrict__ w, const float* __restrict__ rstd,
+    T* __restrict__ dx, float* __restrict__ partial, int rows, int D, int rows_per_block) {
   constexpr int N = kVec<T>;
-  extern __shared__ float colsum[];  // [D]
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  __shared__ float red[2][4];
+  const u32x4 zero = {0, 0, 0, 0};
   float acc[ITER][N];
+  u32x4 g[ITER], cdy[ITER], cx[ITER];
+  auto at = [&](int k) { return (k * 256 + static_cast<int>(threadIdx.x)) * N; };
 #pragma unroll
-  for (int k = 0; k < ITER; ++k)
+  for (int k = 0; k < ITER; ++k) {
+    g[k] = at(k) < D ? *reinterpret_cast<const u32x4*>(w + at(k)) : zero;
 #pragma unroll
     for (int j = 0; j < N; ++j) acc[k][j] = 0.0f;
-  const int r0 = blockIdx.x * rows_per_block;
-  const int r1 = min(r0 + rows_per_block, rows);
-  for (int row = r0 + wave; row < r1; row += 4) {
+  }
+  auto fetch = [&](int row, u32x4 (&a)[ITER], u32x4 (&b)[ITER]) {
     const int64_t o = static_cast<int64_t>(row) * D;
-    const float r = rstd[row];
-    const float c = wave_sum(row_dot<T, N>(dy + o, x + o, w, r, D, lane)) / static_cast<float>(D);
 #pragma unroll
     for (int k = 0; k < ITER; ++k) {
-      const int i = (k * kWave + lane) * N;
-      if (i < D) {
-        float a[N], b[N], g[N], out[N];
-        Pack<T, N>::load(dy + o + i, a);
-        Pack<T, N>::load(x + o + i, b);
-        Pack<T, N>::load(w + i, g);
-#pragma unroll
-        for (int j = 0; j < N; ++j) {
-          const float xh = b[j] * r;
-          out[j] = r * (a[j] * g[j] - xh * c);
-          acc[k][j] += a[j] * xh;
-        }
-        if (dx) Pack<T, N>::store(dx + o + i, out);
+      a[k] = b[k] = zero;
+      if (at(k) < D) {
+        a[k] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(dy + o + at(k)));
+        b[k] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(x + o + at(k)));
       }
     }
-  }
-  for (int turn = 0; turn < 4; ++turn) {
-    if (wave == turn) {
+  };
+  const int r0 = blockIdx.x * rows_per_block, r1 = min(r0 + rows_per_block, rows);
+  if (r0 < r1) fetch(r0, cdy, cx);
+  for (int row = r0; row < r1; ++row) {
+    u32x4 ndy[ITER], nx[ITER];
+    const bool more = row + 1 < r1;
+    if (more) fetch(row + 1, ndy, nx);
+    const float r = rstd[row];
+    float dot = 0.0f;
+#pragma unroll
+    for (int k = 0; k < ITER; ++k) {
+      float a[N], b[N], gv[N];
+      unpack16<T, N>(cdy[k], a);
+      unpack16<T, N>(cx[k], b);
+      unpack16<T, N>(g[k], gv);
+#pragma unroll
+      for (int j = 0; j < N; ++j) dot += (a[j] * gv[j]) * (b[j] * r);
+    }
+    const float c = group_sum(dot, red, row & 1) / static_cast<float>(D);
+    const int64_t o = static_cast<int64_t>(row) * D;
+#pragma unroll
+    for (int k = 0; k < ITER; ++k) {
+      float a[N], b[N], gv[N], out[N];
+      unpack16<T, N>(cdy[k], a);
+      unpack16<T, N>(cx[k], b);
+      unpack16<T, N>(g[k], gv);
+#pragma unroll
+      for (int j = 0; j < N; ++j) {
+        const float xh = b[j] * r;
+        out[j] = r * (a[j] * gv[j] - xh * c);
+        acc[k][j] += a[j] * xh;
+      }
+      if (dx && at(k) < D) *reinterpret_cast<u32x4*>(dx + o + at(k)) = pack16<T, N>(out);
+    }
+    if (more) {
 #pragma unroll
       for (int k = 0; k < ITER; ++k) {
-        const int i = (k * kWave + lane) * N;
-        if (i < D) {
-#pragma unroll
-          for (int j = 0; j < N; ++j) colsum[i + j] = turn == 0 ? acc[k][j] : colsum[i + j] + acc[k][j];
-        }
+        cdy[k] = ndy[k];
+        cx[k] = nx[k];
       }
     }
-    __syncthreads();
   }
-  for (int d = threadIdx.x; d < D; d += 256) partial[static_cast<int64_t>(blockIdx.x) * D + d] = colsum[d];
+#pragma unroll
+  for (int k = 0; k < ITER; ++k)
+    if (at(k) < D)
+#pragma unroll
+      for (int j = 0; j < N; j += 4)
+        *reinterpret_cast<float4*>(partial + static_cast<int64_t>(blockIdx.x) * D + at(k) + j) =
+            make_float4(acc[k][j], acc[k][j + 1], acc[k][j + 2], acc[k][j + 3]);
 }
 
-// 16 bytes of T as N floats and back
-template <typename T, int N>
-__device__ __forceinline__ void unpack16(const u32x4& q, float (&v)[N]) {
-  if constexpr (std::is_same<T, float>::value) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = __uint_as_float(q[j]);
-  } else {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      v[2 * j] = __uint_as_float(q[j] << 16);
-      v[2 * j + 1] = __uint_as_float(q[j] & 0xffff0000u);
-    }
-  }
-}
-template <typename T, int N>
-__device__ __forceinline__ u32x4 pack16(const float (&v)[N]) {
-  u32x4 q;
-  if constexpr (std::is_same<T, float>::value) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) q[j] = __float_as_uint(v[j]);
-  } else {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) q[j] = pack_bf16x2(v[2 * j], v[2 * j + 1]);
-  }
-  return q;
-}
-
-// The same pass for rows of at most 4 x 64 sixteen-byte groups (2048 bf16 or 1024 fp32 columns): a
-// wave holds its row of dy and x in registers, so the row is read from memory once (the kernel
-// above reads it for the row's dot product and again, from cache, for dx), the weights stay in
+// The same with one wave to a row, for rows of at most 4 x 64 sixteen-byte groups (2048 bf16 or 1024 fp32
+// columns): a workgroup's four waves add their column sums up through LDS at the end, the weights stay in
 // registers across the rows, and the next row of the wave is requested before the current one is
 // reduced -- with one row in flight per wave the kernel waited out a memory round trip per row.
 template <typename T, int ITER>
@@ -410,14 +493,31 @@ extern "C" int mi355_rms_norm_fwd(const void* x, const void* weight, int dtype, 
   MI355_REQUIRE(x && weight && y, "rms_norm_fwd: null pointer");
   const dim3 grid((unsigned)((rows + 3) / 4));
   const int vec = rows_are_16_byte_aligned(D, dtype, {x, weight, y});
-  if (dtype == MI355_F32)
-    hipLaunchKernelGGL(rms_fwd_kernel<float>, grid, dim3(256), 0, as_stream(stream), static_cast<const float*>(x),
-                       static_cast<const float*>(weight), static_cast<float*>(y), rstd, (int)rows, (int)D, epsilon,
-                       vec);
-  else
-    hipLaunchKernelGGL(rms_fwd_kernel<uint16_t>, grid, dim3(256), 0, as_stream(stream),
-                       static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(weight),
-                       static_cast<uint16_t*>(y), rstd, (int)rows, (int)D, epsilon, vec);
+  auto run = [&](auto tag) {
+    using T = decltype(tag);
+    const int64_t groups = (D / kVec<T> + kWave - 1) / kWave;  // 16-byte groups per lane
+    const T *xp = static_cast<const T*>(x), *wp = static_cast<const T*>(weight);
+    T* yp = static_cast<T*>(y);
+    auto launch = [&](auto waves, auto iter) {
+      constexpr int W = decltype(waves)::value;
+      hipLaunchKernelGGL((rms_fwd_row_in_registers_kernel<T, W, decltype(iter)::value>), W == 1 ? grid : dim3((unsigned)rows),
+                         dim3(256), 0, as_stream(stream), xp, wp, yp, rstd, (int)rows, (int)D, epsilon);
+    };
+    const std::integral_constant<int, 1> i1;
+    const std::integral_constant<int, 2> i2;
+    const std::integral_constant<int, 4> i4;
+    const std::integral_constant<int, 8> i8;
+    if (vec && groups <= 1) launch(i1, i1);
+    else if (vec && groups <= 2) launch(i1, i2);
+    else if (vec && groups <= 4) launch(i1, i4);
+    else if (vec && groups <= 8) launch(i4, i2);
+    else if (vec && groups <= 16) launch(i4, i4);
+    else if (vec && groups <= 32) launch(i4, i8);
+    else
+      hipLaunchKernelGGL(rms_fwd_kernel<T>, grid, dim3(256), 0, as_stream(stream), xp, wp, yp, rstd, (int)rows, (int)D,
+                         epsilon, vec);
+  };
+  if (dtype == MI355_F32) run(float{}); else run(uint16_t{});
   return check_launch("rms_norm_fwd");
 }
 
@@ -444,29 +544,24 @@ extern "C" int mi355_rms_norm_bwd(const void* dy, const void* x, const void* wei
     // one pass for both when rows are 16-byte aligned and a lane's columns fit in registers
     constexpr int N = 16 / sizeof(T);
     const int64_t groups = (D / N + kWave - 1) / kWave;  // 16-byte groups per lane
-    if (dweight && rows > 0 && groups <= 16 && D * 4 <= 64 * 1024 &&
-        rows_are_16_byte_aligned(D, dtype, {dy, x, weight, dx})) {
+    const bool one_wave = groups <= 4;
+    if (dweight && rows > 0 && (groups <= 16 || (groups <= 32 && dtype == MI355_F32)) &&
+        rows_are_16_byte_aligned(D, dtype, {dy, x, weight, dx, workspace})) {
       const int blocks = (int)std::min<int64_t>(std::min<int64_t>(kFusedBlocks, std::max<int64_t>(512, rows / 32)),
-                                                (rows + 3) / 4);
+                                                one_wave ? (rows + 3) / 4 : rows);
       const int rpb = (int)((rows + blocks - 1) / blocks);
       const int used = (int)((rows + rpb - 1) / rpb);
-      auto launch = [&](auto iter) {
-        constexpr int ITER = decltype(iter)::value;
-        if constexpr (ITER <= 4) {
-          hipLaunchKernelGGL((rms_bwd_rows_in_registers_kernel<T, ITER>), dim3(used), dim3(256), (size_t)D * 4, s,
-                             static_cast<const T*>(dy), static_cast<const T*>(x), static_cast<const T*>(weight), rstd,
-                             static_cast<T*>(dx), static_cast<float*>(workspace), (int)rows, (int)D, rpb);
-          return;
-        }
-        hipLaunchKernelGGL((rms_bwd_fused_kernel<T, ITER>), dim3(used), dim3(256), (size_t)D * 4, s,
-                           static_cast<const T*>(dy), static_cast<const T*>(x), static_cast<const T*>(weight), rstd,
-                           static_cast<T*>(dx), static_cast<float*>(workspace), (int)rows, (int)D, rpb);
+      auto launch = [&](auto kernel, size_t lds) {
+        hipLaunchKernelGGL(kernel, dim3(used), dim3(256), lds, s, static_cast<const T*>(dy), static_cast<const T*>(x),
+                           static_cast<const T*>(weight), rstd, static_cast<T*>(dx), static_cast<float*>(workspace),
+                           (int)rows, (int)D, rpb);
       };
-      if (groups <= 1) launch(std::integral_constant<int, 1>{});
-      else if (groups <= 2) launch(std::integral_constant<int, 2>{});
-      else if (groups <= 4) launch(std::integral_constant<int, 4>{});
-      else if (groups <= 8) launch(std::integral_constant<int, 8>{});
-      else launch(std::integral_constant<int, 16>{});
+      if (groups <= 1) launch(rms_bwd_rows_in_registers_kernel<T, 1>, (size_t)D * 4);
+      else if (groups <= 2) launch(rms_bwd_rows_in_registers_kernel<T, 2>, (size_t)D * 4);
+      else if (groups <= 4) launch(rms_bwd_rows_in_registers_kernel<T, 4>, (size_t)D * 4);
+      else if (groups <= 8) launch(rms_bwd_row_per_group_kernel<T, 2>, 0);
+      else if (groups <= 16) launch(rms_bwd_row_per_group_kernel<T, 4>, 0);
+      else if constexpr (sizeof(T) == 4) launch(rms_bwd_row_per_group_kernel<T, 8>, 0);
       hipLaunchKernelGGL(rms_dw_final_kernel<T>, fgrid, dim3(256), 0, s, static_cast<const float*>(workspace),
                          static_cast<T*>(dweight), used, (int)D);
       return;
