@@ -424,8 +424,9 @@ __global__ __launch_bounds__(kLanes) void route_rows_kernel(const float* __restr
 // Lanes per workgroup.  Selection is bound by instruction issue, so its tokens want to be spread over the
 // CUs; but every workgroup of route_rows reads all histograms, so there should not be more than two hundred
 // or so.  Both kernels together at 128 experts, 1024 / 512 / 256 lanes: 21 / 15 / 16 us at 1000 tokens, 22 / 19 / 26 at
-// 4096, 23 / 22 / 30 at 8192.  Up to 64 tokens one workgroup does everything.
-int route_lanes(int64_t T) { return T > 64 && T < 8192 ? 512 : 1024; }
+// 4096, 23 / 22 / 30 at 8192.  Up to 64 tokens one workgroup does everything, up to 32 with 512 lanes: fewer
+// waves to clear counters for and to meet at barriers (8 tokens 9.9 us with 1024, 9.6 with 512; 32 tokens 11.5 / 10.9).
+int route_lanes(int64_t T) { return T <= 32 || (T > 64 && T < 8192) ? 512 : 1024; }
 int route_chunks(int64_t T) {
   const int64_t rows = route_lanes(T) / 16, groups = (T + rows - 1) / rows;
   return static_cast<int>((groups + kMaxBlocks - 1) / kMaxBlocks);
