@@ -10,26 +10,21 @@
 // Conventions shared with ops.py: an output that was not asked for is an empty (0,) tensor; a
 // gradient that is not needed is returned undefined; incoming gradients are not materialised, so
 // an output nobody differentiated arrives undefined.
-#include <ATen/ATen.h>
-#include <ATen/core/dispatch/Dispatcher.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/library.h>
 
-#include <optional>
 #include <tuple>
+
+#include "torch_common.h"
 
 namespace {
 
-using at::Tensor;
-using OptTensor = std::optional<Tensor>;
+using mi355_torch::OptTensor;
+using mi355_torch::Tensor;
+using mi355_torch::typed_op;
 using torch::autograd::AutogradContext;
 using torch::autograd::variable_list;
-
-template <class Sig>
-auto typed_op(const char* name) {
-  return c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<Sig>();
-}
 
 OptTensor opt(const Tensor& t) { return t.defined() ? OptTensor(t) : std::nullopt; }
 Tensor keep(const Tensor& t, bool wanted) { return wanted ? t : Tensor(); }

@@ -1,9 +1,17 @@
 // The whole MoE block as one operator: router, plan, routed experts, combine and (when there is one)
 // the dense shared expert, with one autograd node whose backward is written out below.
 //
+//   moe_block       what callers use.  Its Autograd kernel passes on to the two below when an input asks for
+//                   a gradient, and to its own device kernel otherwise.
+//   moe_block_fwd   the forward that also returns what the backward reads
+//   moe_block_bwd   the backward
+// All three are reached through the dispatcher, also from inside the autograd node: whatever stands in its
+// way -- a tracing mode, fake tensors, a function transform -- sees an operator with its inputs and
+// outputs and never this file's allocations.
+//
 // The stage operators of torch_ext.cpp compute the same things one at a time, for callers that
-// look between the stages (hooks, other dispatchers, other routers, tracing); MoE.forward comes here
-// when nothing hangs on the stages.  What the single operator saves:
+// look between the stages (hooks, other dispatchers, other routers, tracing, dispatch modes); MoE.forward
+// comes here when nothing hangs on the stages.  What the single operator saves:
 //   * host time: a forward pass is one trip through the dispatcher and about ten C calls instead of four
 //     operators, a plan object and its views (83 -> 35 us at one token), a training step has one autograd
 //     node instead of three to five;
@@ -21,8 +29,9 @@
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/library.h>
 
-#include <cstring>
+#include <string>
 #include <tuple>
+#include <utility>
 #include <vector>
 
 #include "torch_common.h"
@@ -37,29 +46,18 @@ struct Config {
   int64_t K, score_func, route_norm, num_groups, num_limited, lo, hi, align, round_terms, overlap;
   int64_t aux;  // the router injects a load-balance loss
   double route_scale;
-
-  std::vector<int64_t> pack() const {
-    std::vector<int64_t> v{K, score_func, route_norm, num_groups, num_limited, lo, hi, align, round_terms, overlap, aux, 0};
-    std::memcpy(&v[11], &route_scale, sizeof(double));
-    return v;
-  }
-  static Config unpack(const std::vector<int64_t>& v) {
-    Config c{v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[9], v[10], 0.0};
-    std::memcpy(&c.route_scale, &v[11], sizeof(double));
-    return c;
-  }
 };
 
 // What a router that keeps statistics brings; undefined / zero where it keeps none.  Written in the forward.
 struct Stats {
   Tensor histogram, aux_acc, aux_denominator;
   double aux_coeff = 0.0;
-  Tensor mask;  // (T) bool, true = padding
 };
 
 // The block's tensors; undefined where the block has none.
 struct Block {
-  Tensor x, gate_w, gate_b, expert_b, w1, w3, w2, sg, su, sd, mask;
+  Tensor x, gate_w, gate_b, expert_b, w1, w3, w2, sg, su, sd;
+  Tensor mask;  // (T) bool, true = padding
   Config c;
   int64_t T, D, E, F, El, N, R, Fs, tile_m, tile_cap, shared_cap;
   int dt, gate_dt;
@@ -451,50 +449,67 @@ Grads block_backward(const Block& b, const Tensor& kept, const Tensor& dout_, co
 Tensor some(const OptTensor& t) { return t.has_value() ? *t : Tensor(); }
 OptTensor opt(const Tensor& t) { return t.defined() ? OptTensor(t) : std::nullopt; }
 
+// The arguments of moe_block and moe_block_fwd, once as parameters and once to pass on.
+#define BLOCK_PARAMS                                                                                               \
+  const Tensor &x, const Tensor &gate_w, const OptTensor &gate_b, const OptTensor &expert_b, const Tensor &w1,     \
+      const Tensor &w3, const Tensor &w2, const OptTensor &sg, const OptTensor &su, const OptTensor &sd, int64_t K, \
+      int64_t score_func, bool route_norm, double route_scale, int64_t num_groups, int64_t num_limited, int64_t lo, \
+      int64_t hi, int64_t align, bool round_terms, bool overlap_shared, const OptTensor &mask,                     \
+      const OptTensor &histogram, const OptTensor &aux_denominator, double aux_coeff, const OptTensor &aux_acc
+#define BLOCK_ARGS                                                                                                 \
+  x, gate_w, gate_b, expert_b, w1, w3, w2, sg, su, sd, K, score_func, route_norm, route_scale, num_groups,         \
+      num_limited, lo, hi, align, round_terms, overlap_shared, mask, histogram, aux_denominator, aux_coeff, aux_acc
+
+using BlockSig = std::tuple<Tensor, Tensor>(BLOCK_PARAMS);
+using BlockFwdSig = std::tuple<Tensor, Tensor, Tensor>(BLOCK_PARAMS);
+using NineTensors = std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor>;
+using BlockBwdSig = NineTensors(const Tensor&, const Tensor&, const Tensor&, const OptTensor&, const Tensor&,
+                                const Tensor&, const Tensor&, const OptTensor&, const OptTensor&, const OptTensor&,
+                                const Tensor&, const OptTensor&, int64_t, int64_t, bool, double, int64_t, int64_t,
+                                int64_t, bool, bool, bool, bool, bool, bool, bool);
+
 struct MoeBlock : public torch::autograd::Function<MoeBlock> {
-  static variable_list forward(AutogradContext* ctx, const Tensor& x, const Tensor& gate_w, const OptTensor& gate_b,
-                               const OptTensor& expert_b, const Tensor& w1, const Tensor& w3, const Tensor& w2,
-                               const OptTensor& sg, const OptTensor& su, const OptTensor& sd, const Config& c,
-                               const Stats& st) {
+  static variable_list forward(AutogradContext* ctx, BLOCK_PARAMS) {
     at::AutoDispatchBelowADInplaceOrView below;
-    Block b{x, gate_w, some(gate_b), some(expert_b), w1, w3, w2, some(sg), some(su), some(sd), st.mask, c};
-    b.sizes();
-    auto [out, counts, kept] = block_forward(b, st, true);
-    ctx->save_for_backward({x, gate_w, b.gate_b, w1, w3, w2, b.sg, b.su, b.sd, kept, b.mask});
-    auto packed = c.pack();
-    packed.push_back(b.expert_b.defined());
-    ctx->saved_data["config"] = packed;
+    static auto op = typed_op<BlockFwdSig>("mi355_moe::moe_block_fwd");
+    auto [out, counts, kept] = op.call(BLOCK_ARGS);
+    ctx->save_for_backward({x, gate_w, some(gate_b), w1, w3, w2, some(sg), some(su), some(sd), kept, some(mask)});
+    ctx->saved_data["config"] = std::vector<int64_t>{K, score_func, route_norm, lo, hi, align, overlap_shared,
+                                                     some(aux_denominator).defined(), some(expert_b).defined()};
+    ctx->saved_data["route_scale"] = route_scale;
     ctx->set_materialize_grads(false);
     ctx->mark_non_differentiable({counts});
     return {out, counts};
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    variable_list out(12);
+    variable_list out(26);
     if (!grads[0].defined()) return out;
     const auto s = ctx->get_saved_variables();
-    const auto packed = ctx->saved_data["config"].toIntVector();
-    Block b{s[0], s[1], s[2], Tensor(), s[3], s[4], s[5], s[6], s[7], s[8], s[10], Config::unpack(packed)};
-    b.sizes();
+    const auto c = ctx->saved_data["config"].toIntVector();
     // needs_input_grad counts the tensors among the arguments: an absent one has no index
-    const int gb = 2, w = gb + (b.gate_b.defined() ? 1 : 0) + (packed.back() ? 1 : 0), sh = w + 3;
+    const int gb = 2, w = gb + (s[2].defined() ? 1 : 0) + (c.back() ? 1 : 0), sh = w + 3;
     auto wants = [&](int i) { return ctx->needs_input_grad(i); };
-    const bool shared = b.Fs > 0;
-    const Needs need{wants(0), wants(1), b.gate_b.defined() && wants(gb), wants(w) || wants(w + 1) || wants(w + 2),
-                     shared && (wants(sh) || wants(sh + 1) || wants(sh + 2))};
-    Grads g = block_backward(b, s[9], grads[0], need);
+    const bool shared = s[6].defined();
+    at::AutoDispatchBelowADInplaceOrView below;
+    static auto op = typed_op<BlockBwdSig>("mi355_moe::moe_block_bwd");
+    auto [dx, dgate_w, dgate_b, dw1, dw3, dw2, dsg, dsu, dsd] =
+        op.call(grads[0], s[0], s[1], opt(s[2]), s[3], s[4], s[5], opt(s[6]), opt(s[7]), opt(s[8]), s[9], opt(s[10]), c[0],
+                c[1], c[2] != 0, ctx->saved_data["route_scale"].toDouble(), c[3], c[4], c[5], c[6] != 0, c[7] != 0,
+                wants(0), wants(1), s[2].defined() && wants(gb), wants(w) || wants(w + 1) || wants(w + 2),
+                shared && (wants(sh) || wants(sh + 1) || wants(sh + 2)));
     auto put = [&](int argument, int tensor, const Tensor& t) {
       if (t.defined() && wants(tensor)) out[argument] = t;
     };
-    put(0, 0, g.x);
-    put(1, 1, g.gate_w);
-    if (need.gate_b) out[2] = g.gate_b;
-    put(4, w, g.w1);
-    put(5, w + 1, g.w3);
-    put(6, w + 2, g.w2);
+    put(0, 0, dx);
+    put(1, 1, dgate_w);
+    out[2] = dgate_b;  // (undefined unless it was asked for)
+    put(4, w, dw1);
+    put(5, w + 1, dw3);
+    put(6, w + 2, dw2);
     if (shared) {
-      put(7, sh, g.sg);
-      put(8, sh + 1, g.su);
-      put(9, sh + 2, g.sd);
+      put(7, sh, dsg);
+      put(8, sh + 1, dsu);
+      put(9, sh + 2, dsd);
     }
     return out;
   }
@@ -502,32 +517,23 @@ struct MoeBlock : public torch::autograd::Function<MoeBlock> {
 
 Tensor contiguous(const OptTensor& t) { return t.has_value() && t->defined() ? t->contiguous() : Tensor(); }
 
-std::tuple<Tensor, Tensor> moe_block(const Tensor& x_, const Tensor& gate_w_, const OptTensor& gate_b_,
-                                     const OptTensor& expert_b_, const Tensor& w1_, const Tensor& w3_,
-                                     const Tensor& w2_, const OptTensor& sg_, const OptTensor& su_,
-                                     const OptTensor& sd_, int64_t K, int64_t score_func, bool route_norm,
-                                     double route_scale, int64_t num_groups, int64_t num_limited, int64_t lo,
-                                     int64_t hi, int64_t align, bool round_terms, bool overlap_shared,
-                                     const OptTensor& mask_, const OptTensor& histogram_,
-                                     const OptTensor& aux_denominator_, double aux_coeff, const OptTensor& aux_acc_) {
-  const Tensor x = x_.contiguous(), gate_w = gate_w_.contiguous(), w1 = w1_.contiguous(), w3 = w3_.contiguous(),
-               w2 = w2_.contiguous();
-  const Tensor gate_b = contiguous(gate_b_), expert_b = contiguous(expert_b_), sg = contiguous(sg_),
-               su = contiguous(su_), sd = contiguous(sd_);
-  TORCH_CHECK_VALUE(x.dim() == 2 && x.size(0) >= 1 && gate_w.dim() == 2 && gate_w.size(1) == x.size(1), "gate weight ",
-                    gate_w.sizes(), " does not match input ", x.sizes());
-  TORCH_CHECK_VALUE(w1.dim() == 3 && w1.size(2) == x.size(1) && w3.sizes() == w1.sizes() && w2.dim() == 3 &&
+void check_weights(const Block& b) {
+  const Tensor &x = b.x, &w1 = b.w1, &w2 = b.w2;
+  TORCH_CHECK_VALUE(x.dim() == 2 && x.size(0) >= 1 && b.gate_w.dim() == 2 && b.gate_w.size(1) == x.size(1), "gate weight ",
+                    b.gate_w.sizes(), " does not match input ", x.sizes());
+  TORCH_CHECK_VALUE(w1.dim() == 3 && w1.size(2) == x.size(1) && b.w3.sizes() == w1.sizes() && w2.dim() == 3 &&
                         w2.size(0) == w1.size(0) && w2.size(1) == w1.size(2) && w2.size(2) == w1.size(1),
                     "expert weight shapes do not match (E,F,D)/(E,F,D)/(E,D,F)");
-  TORCH_CHECK_VALUE(lo >= 0 && hi - lo == w1.size(0) && hi <= gate_w.size(0) && align >= 1,
-                    "local expert range [", lo, ",", hi, ") does not match the weights");
+  TORCH_CHECK_VALUE(b.c.lo >= 0 && b.c.hi - b.c.lo == w1.size(0) && b.c.hi <= b.gate_w.size(0) && b.c.align >= 1,
+                    "local expert range [", b.c.lo, ",", b.c.hi, ") does not match the weights");
   const auto type = x.scalar_type();
   TORCH_CHECK_TYPE((type == at::kFloat || type == at::kBFloat16) && w1.scalar_type() == type &&
-                       w3.scalar_type() == type && w2.scalar_type() == type,
+                       b.w3.scalar_type() == type && w2.scalar_type() == type,
                    "expert weights and rows must share one dtype, float32 or bfloat16");
-  TORCH_CHECK_VALUE((!gate_b.defined() || gate_b.numel() == gate_w.size(0)) &&
-                        (!expert_b.defined() || expert_b.numel() == gate_w.size(0)),
+  TORCH_CHECK_VALUE((!b.gate_b.defined() || b.gate_b.numel() == b.gate_w.size(0)) &&
+                        (!b.expert_b.defined() || b.expert_b.numel() == b.gate_w.size(0)),
                     "a bias does not match the number of experts");
+  const Tensor &sg = b.sg, &su = b.su, &sd = b.sd;
   TORCH_CHECK_VALUE(sg.defined() == su.defined() && sg.defined() == sd.defined(), "shared expert: three weights or none");
   if (sg.defined()) {
     TORCH_CHECK_VALUE(sg.dim() == 2 && sg.size(1) == x.size(1) && su.sizes() == sg.sizes() && sd.dim() == 2 &&
@@ -536,47 +542,137 @@ std::tuple<Tensor, Tensor> moe_block(const Tensor& x_, const Tensor& gate_w_, co
     TORCH_CHECK_TYPE(sg.scalar_type() == type && su.scalar_type() == type && sd.scalar_type() == type,
                      "shared expert weights and tokens must share one dtype");
   }
-  for (const Tensor* t : {&gate_w, &gate_b, &expert_b, &w1, &w3, &w2, &sg, &su, &sd})
+  for (const Tensor* t : {&b.gate_w, &b.gate_b, &b.expert_b, &b.w1, &b.w3, &b.w2, &sg, &su, &sd})
     TORCH_CHECK(!t->defined() || t->device() == x.device(), "moe_block: tensors on different devices: ", x.device(),
                 " and ", t->device());
-  const Tensor mask = contiguous(mask_);
-  const Stats st{some(histogram_), some(aux_acc_), some(aux_denominator_), aux_coeff, mask};
-  TORCH_CHECK_VALUE(!mask.defined() || (mask.scalar_type() == at::kBool && mask.numel() == x.size(0) &&
-                                        mask.device() == x.device()),
+  TORCH_CHECK_VALUE(!b.mask.defined() || (b.mask.scalar_type() == at::kBool && b.mask.numel() == x.size(0) &&
+                                          b.mask.device() == x.device()),
                     "padding mask: one bool per token on the tokens' device");
+}
+
+void check_stats(const Block& b, const Stats& st) {
   TORCH_CHECK_VALUE(!st.histogram.defined() ||
                         (st.histogram.scalar_type() == at::kLong && st.histogram.is_contiguous() &&
-                         st.histogram.dim() == 2 && st.histogram.size(0) == gate_w.size(0) &&
-                         st.histogram.device() == x.device() && expert_b.defined()),
+                         st.histogram.dim() == 2 && st.histogram.size(0) == b.gate_w.size(0) &&
+                         st.histogram.device() == b.x.device() && b.expert_b.defined()),
                     "histogram: contiguous int64 (experts, bins) beside an expert bias");
-  auto scalar = [&](const Tensor& t) { return !t.defined() || (t.numel() == 1 && t.device() == x.device()); };
+  auto scalar = [&](const Tensor& t) { return !t.defined() || (t.numel() == 1 && t.device() == b.x.device()); };
   TORCH_CHECK_VALUE(scalar(st.aux_acc) && scalar(st.aux_denominator) &&
                         (!st.aux_denominator.defined() || st.aux_denominator.scalar_type() == at::kFloat) &&
                         (!st.aux_acc.defined() || st.aux_acc.scalar_type() == at::kFloat ||
                          st.aux_acc.scalar_type() == at::kBFloat16),
                     "auxiliary loss: scalars on the tokens' device, the denominator fp32, the metric fp32 or bf16");
-  const Config c{K, score_func, route_norm, num_groups, num_limited, lo, hi, align, round_terms, overlap_shared,
-                 st.aux_denominator.defined(), route_scale};
+}
+
+// The block of a forward call, checked.
+std::pair<Block, Stats> block_of(BLOCK_PARAMS) {
+  const Stats st{some(histogram), some(aux_acc), some(aux_denominator), aux_coeff};
+  Block b{x.contiguous(), gate_w.contiguous(), contiguous(gate_b), contiguous(expert_b), w1.contiguous(),
+          w3.contiguous(), w2.contiguous(), contiguous(sg), contiguous(su), contiguous(sd), contiguous(mask),
+          Config{K, score_func, route_norm, num_groups, num_limited, lo, hi, align, round_terms, overlap_shared,
+                 st.aux_denominator.defined(), route_scale}};
+  check_weights(b);
+  check_stats(b, st);
+  b.sizes();
+  return {b, st};
+}
+
+std::tuple<Tensor, Tensor> moe_block(BLOCK_PARAMS) {
+  const auto [b, st] = block_of(BLOCK_ARGS);
+  auto [out, counts, kept] = block_forward(b, st, false);
+  return {out, counts};
+}
+
+std::tuple<Tensor, Tensor, Tensor> moe_block_fwd(BLOCK_PARAMS) {
+  const auto [b, st] = block_of(BLOCK_ARGS);
+  return block_forward(b, st, true);
+}
+
+// shapes only (fake and meta tensors)
+std::tuple<Tensor, Tensor, Tensor> moe_block_fwd_meta(BLOCK_PARAMS) {
+  const auto [b, st] = block_of(BLOCK_ARGS);
+  Carver measure{nullptr};
+  Kept{}.layout(measure, b, true);
+  return {at::empty({b.T, b.D}, b.x.options()), at::empty({b.E}, b.x.options().dtype(at::kInt)), bytes(measure.at, b.x)};
+}
+
+#define BLOCK_BWD_PARAMS                                                                                              \
+  const Tensor &dout, const Tensor &x, const Tensor &gate_w, const OptTensor &gate_b, const Tensor &w1,               \
+      const Tensor &w3, const Tensor &w2, const OptTensor &sg, const OptTensor &su, const OptTensor &sd,              \
+      const Tensor &kept, const OptTensor &mask, int64_t K, int64_t score_func, bool route_norm, double route_scale,  \
+      int64_t lo, int64_t hi, int64_t align, bool overlap_shared, bool aux, bool need_x, bool need_gate_w,            \
+      bool need_gate_b, bool need_experts, bool need_shared
+#define BLOCK_BWD_ARGS                                                                                                \
+  dout, x, gate_w, gate_b, w1, w3, w2, sg, su, sd, kept, mask, K, score_func, route_norm, route_scale, lo, hi, align, \
+      overlap_shared, aux, need_x, need_gate_w, need_gate_b, need_experts, need_shared
+
+// The block and what is asked of a backward call, checked.
+std::pair<Block, Needs> block_bwd_of(BLOCK_BWD_PARAMS) {
+  Block b{x.contiguous(), gate_w.contiguous(), contiguous(gate_b), Tensor(), w1.contiguous(), w3.contiguous(),
+          w2.contiguous(), contiguous(sg), contiguous(su), contiguous(sd), contiguous(mask),
+          Config{K, score_func, route_norm, 0, 0, lo, hi, align, 0, overlap_shared, aux, route_scale}};
+  check_weights(b);
+  b.sizes();
+  Carver measure{nullptr};
+  Kept{}.layout(measure, b, true);
+  TORCH_CHECK_VALUE(kept.scalar_type() == at::kByte && kept.is_contiguous() && kept.numel() >= measure.at &&
+                        kept.device() == b.x.device(),
+                    "moe_block_bwd: not what moe_block_fwd kept for this block");
+  TORCH_CHECK_VALUE(dout.sizes() == b.x.sizes() && dout.device() == b.x.device(), "moe_block_bwd: gradient ", dout.sizes(),
+                    " does not match the output ", b.x.sizes());
+  return {b, Needs{need_x, need_gate_w, need_gate_b && b.gate_b.defined(), need_experts, need_shared && b.Fs > 0}};
+}
+
+NineTensors moe_block_bwd(BLOCK_BWD_PARAMS) {
+  const auto [b, need] = block_bwd_of(BLOCK_BWD_ARGS);
+  Grads g = block_backward(b, kept, dout, need);
+  return {g.x, g.gate_w, g.gate_b, g.w1, g.w3, g.w2, g.sg, g.su, g.sd};
+}
+
+NineTensors moe_block_bwd_meta(BLOCK_BWD_PARAMS) {
+  const auto [b, need] = block_bwd_of(BLOCK_BWD_ARGS);
+  auto like = [](bool wanted, const Tensor& t) { return wanted ? at::empty(t.sizes(), t.options()) : Tensor(); };
+  return {like(need.x, b.x),           like(need.gate_w, b.gate_w), like(need.gate_b, b.gate_b),
+          like(need.experts, b.w1),    like(need.experts, b.w3),    like(need.experts, b.w2),
+          like(need.shared, b.sg),     like(need.shared, b.su),     like(need.shared, b.sd)};
+}
+
+std::tuple<Tensor, Tensor> moe_block_autograd(BLOCK_PARAMS) {
   if (torch::autograd::compute_requires_grad(x, gate_w, gate_b, w1, w3, w2, sg, su, sd)) {
-    auto r = MoeBlock::apply(x, gate_w, opt(gate_b), opt(expert_b), w1, w3, w2, opt(sg), opt(su), opt(sd), c, st);
+    auto r = MoeBlock::apply(BLOCK_ARGS);
     return {r[0], r[1]};
   }
   at::AutoDispatchBelowADInplaceOrView below;
-  Block b{x, gate_w, gate_b, expert_b, w1, w3, w2, sg, su, sd, mask, c};
-  b.sizes();
-  auto [out, counts, kept] = block_forward(b, st, false);
-  return {out, counts};
+  static auto op = typed_op<BlockSig>("mi355_moe::moe_block");
+  return op.call(BLOCK_ARGS);
 }
 
 }  // namespace
 
 TORCH_LIBRARY_FRAGMENT(mi355_moe, m) {
-  m.def(
-      "moe_block(Tensor x, Tensor gate_w, Tensor? gate_bias, Tensor? expert_bias, Tensor w1, Tensor w3, Tensor w2, "
+  const std::string args =
+      "(Tensor x, Tensor gate_w, Tensor? gate_bias, Tensor? expert_bias, Tensor w1, Tensor w3, Tensor w2, "
       "Tensor? shared_gate, Tensor? shared_up, Tensor? shared_down, int top_k, int score_func, bool route_norm, "
       "float route_scale, int num_groups, int num_limited, int local_lo, int local_hi, int align, bool round_terms, "
       "bool overlap_shared, Tensor? padding_mask, Tensor(a!)? histogram, Tensor? aux_denominator, float aux_coeff, "
-      "Tensor(b!)? aux_acc) -> (Tensor, Tensor)");
+      "Tensor(b!)? aux_acc)";
+  m.def(("moe_block" + args + " -> (Tensor, Tensor)").c_str());
+  m.def(("moe_block_fwd" + args + " -> (Tensor, Tensor, Tensor)").c_str());
+  // a gradient that is not asked for is undefined (None)
+  m.def(
+      "moe_block_bwd(Tensor dout, Tensor x, Tensor gate_w, Tensor? gate_bias, Tensor w1, Tensor w3, Tensor w2, "
+      "Tensor? shared_gate, Tensor? shared_up, Tensor? shared_down, Tensor kept, Tensor? padding_mask, int top_k, "
+      "int score_func, bool route_norm, float route_scale, int local_lo, int local_hi, int align, bool overlap_shared, "
+      "bool aux, bool need_x, bool need_gate_w, bool need_gate_bias, bool need_experts, bool need_shared) -> "
+      "(Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor)");
 }
-TORCH_LIBRARY_IMPL(mi355_moe, CUDA, m) { m.impl("moe_block", moe_block); }
-TORCH_LIBRARY_IMPL(mi355_moe, Autograd, m) { m.impl("moe_block", moe_block); }
+TORCH_LIBRARY_IMPL(mi355_moe, CUDA, m) {
+  m.impl("moe_block", moe_block);
+  m.impl("moe_block_fwd", moe_block_fwd);
+  m.impl("moe_block_bwd", moe_block_bwd);
+}
+TORCH_LIBRARY_IMPL(mi355_moe, Meta, m) {
+  m.impl("moe_block_fwd", moe_block_fwd_meta);
+  m.impl("moe_block_bwd", moe_block_bwd_meta);
+}
+TORCH_LIBRARY_IMPL(mi355_moe, Autograd, m) { m.impl("moe_block", moe_block_autograd); }

@@ -2,6 +2,7 @@
 // pointers, error translation, the launch context and the library's side streams.
 #pragma once
 #include <ATen/ATen.h>
+#include <ATen/core/dispatch/Dispatcher.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
 
@@ -60,6 +61,12 @@ inline SideStream* side_stream(int device, hipStream_t current, int which = 0) {
 
 using at::Tensor;
 using OptTensor = std::optional<Tensor>;
+
+// A registered operator, to be called through the dispatcher.
+template <class Sig>
+auto typed_op(const char* name) {
+  return c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<Sig>();
+}
 
 inline int dtype_code(const Tensor& t) {
   if (t.scalar_type() == at::kFloat) return MI355_F32;

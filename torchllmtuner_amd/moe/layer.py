@@ -31,6 +31,13 @@ __all__ = ["MoE", "in_checkpoint_recompute"]
 
 
 _BLOCK_DTYPES = (torch.bfloat16, torch.float32)
+_PLAIN_TENSORS = (torch.Tensor, nn.Parameter)
+
+
+def _intercepted() -> bool:
+    """True inside a dispatch mode (a tracer, a selective-checkpoint policy, a flop counter: they look at the
+    operators, by name) or a function transform (vmap cannot batch an operator that updates statistics)."""
+    return torch._C._len_torch_dispatch_stack() > 0 or torch._C._functorch.peek_interpreter_stack() is not None
 
 
 def _plain(module: nn.Module, cls: type) -> bool:
@@ -181,7 +188,7 @@ class MoE(nn.Module):
             if not _plain(linear, nn.Linear) or linear._parameters["bias"] is not None:
                 return None
             weights.append(linear._parameters["weight"])
-        return weights if all(w.dtype is dtype for w in weights) else None
+        return weights if all(type(w) in _PLAIN_TENSORS and w.dtype is dtype for w in weights) else None
 
     def _router_statistics(self, router, tokens):
         """Keywords of ``ops.moe_block`` for what the router keeps in training -- the quantile router's
@@ -228,12 +235,14 @@ class MoE(nn.Module):
         """``(output, counts per expert)`` from the one operator that computes the whole block
         (``mi355_moe::moe_block``), or None when a stage has to be visible or is not what it computes: a
         hook or an override anywhere below, an observer, another auxiliary loss, router, dispatcher,
-        activation or shared expert, fp64, no tokens, a tracing compiler.  Both ways give the same bits
+        activation or shared expert, a weight of a tensor subclass, fp64, no tokens, a tracing compiler, a
+        dispatch mode or a function transform.  Both ways give the same bits
         (the load-balance loss: the same sums in another order).  In training the counts leave out the
         tokens of ``padding_mask``."""
         if (
             torch.compiler.is_compiling()
-            or type(tokens) not in (torch.Tensor, nn.Parameter)
+            or _intercepted()
+            or type(tokens) not in _PLAIN_TENSORS
             or not tokens.is_cuda
             or tokens.dtype not in _BLOCK_DTYPES
             or tokens.shape[0] == 0
@@ -266,7 +275,12 @@ class MoE(nn.Module):
         dtype = tokens.dtype
         p = experts._parameters
         w1, w3, w2 = p["w1_EFD"], p["w3_EFD"], p["w2_EDF"]
-        gate_weight = gate._parameters["weight"]
+        gate_weight, gate_bias = gate._parameters["weight"], gate._parameters["bias"]
+        for w in (w1, w3, w2, gate_weight):
+            if type(w) not in _PLAIN_TENSORS:
+                return None
+        if gate_bias is not None and type(gate_bias) not in _PLAIN_TENSORS:
+            return None
         shared = self._shared_weights(dtype)
         if shared is None or w1.dtype is not dtype or w3.dtype is not dtype or w2.dtype is not dtype:
             return None
@@ -284,7 +298,7 @@ class MoE(nn.Module):
                 stats["padding_mask"] = padding_mask
         lo, hi = dispatcher._local_range()
         return ops.moe_block(
-            tokens, gate_weight, gate._parameters["bias"], self.expert_bias_E, w1, w3, w2, shared,
+            tokens, gate_weight, gate_bias, self.expert_bias_E, w1, w3, w2, shared,
             router.top_k, router.score_func, router.route_norm, router.route_scale, router.num_expert_groups,
             router.num_limited_groups, lo, hi, dispatcher._align(), not dispatcher.accumulate_in_fp32,
             self.overlap_shared_experts, **stats)
