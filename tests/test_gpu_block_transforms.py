@@ -185,3 +185,22 @@ def test_weights_of_a_tensor_subclass_are_unwrapped_by_their_own_rules(which):
             module._parameters[name] = Wrapped(module._parameters[name].data)
         assert block._forward_as_one(x) is None
         _equal([block(x)], [want])
+
+
+@pytest.mark.parametrize("which", ["experts", "gate", "gate bias", "shared"])
+def test_weights_that_are_plain_attributes(which):
+    """What a wrapper that owns the parameters leaves in their place: a tensor set as an attribute."""
+    for dtype, D, F, _ in SHAPES:
+        block = _block(dtype, D, F, 64)
+        block.overlap_shared_experts = False
+        gate, shared = block.router.gate, block.shared_experts
+        if which == "gate bias":
+            gate.bias = torch.nn.Parameter(torch.linspace(-1, 1, E, device=DEV))
+        x = _x(1, dtype, D)
+        want = block(x)
+        for module in dict(experts=[block.routed_experts.inner_experts], gate=[gate], shared=[
+                shared.gate_proj, shared.up_proj, shared.down_proj]).get(which.split()[0]):
+            for name in ["bias"] if which == "gate bias" else [n for n, p in module._parameters.items() if p is not None]:
+                object.__setattr__(module, name, module._parameters.pop(name).detach().requires_grad_())
+        assert block._forward_as_one(x) is None
+        _equal([block(x)], [want])

@@ -185,9 +185,10 @@ class MoE(nn.Module):
         weights = []
         for name in ("gate_proj", "up_proj", "down_proj"):
             linear = shared._modules[name]
-            if not _plain(linear, nn.Linear) or linear._parameters["bias"] is not None:
+            p = linear._parameters
+            if not _plain(linear, nn.Linear) or p.get("bias", linear) is not None:
                 return None
-            weights.append(linear._parameters["weight"])
+            weights.append(p.get("weight"))
         return weights if all(type(w) in _PLAIN_TENSORS and w.dtype is dtype for w in weights) else None
 
     def _router_statistics(self, router, tokens):
@@ -235,8 +236,8 @@ class MoE(nn.Module):
         """``(output, counts per expert)`` from the one operator that computes the whole block
         (``mi355_moe::moe_block``), or None when a stage has to be visible or is not what it computes: a
         hook or an override anywhere below, an observer, another auxiliary loss, router, dispatcher,
-        activation or shared expert, a weight of a tensor subclass, fp64, no tokens, a tracing compiler, a
-        dispatch mode or a function transform.  Both ways give the same bits
+        activation or shared expert, a weight that is no parameter or of a tensor subclass, fp64, no tokens,
+        a tracing compiler, a dispatch mode or a function transform.  Both ways give the same bits
         (the load-balance loss: the same sums in another order).  In training the counts leave out the
         tokens of ``padding_mask``."""
         if (
@@ -273,9 +274,11 @@ class MoE(nn.Module):
         if not experts.fuses_activation() or not _is_own_dispatcher(dispatcher):
             return None
         dtype = tokens.dtype
+        # (a weight may also be an attribute that is no parameter: a sharding or replicating wrapper's view)
         p = experts._parameters
-        w1, w3, w2 = p["w1_EFD"], p["w3_EFD"], p["w2_EDF"]
-        gate_weight, gate_bias = gate._parameters["weight"], gate._parameters["bias"]
+        w1, w3, w2 = p.get("w1_EFD"), p.get("w3_EFD"), p.get("w2_EDF")
+        p = gate._parameters
+        gate_weight, gate_bias = p.get("weight"), p.get("bias", gate)
         for w in (w1, w3, w2, gate_weight):
             if type(w) not in _PLAIN_TENSORS:
                 return None
