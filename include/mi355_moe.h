@@ -12,6 +12,10 @@
  * PyTorch ops.  Each declaration therefore cites the reference lines whose
  * arithmetic it replaces (paths relative to the reference checkout).
  *
+ * Pointers are as aligned as an allocation of its own (16 bytes).  The grouped experts and linear maps off
+ * the bf16 MFMA path and the router gate also take operands aligned to their element only, on
+ * slower kernels.
+ *
  * Shape legend: T tokens, D model dim, E experts, K experts per token, N = T*K
  * assignment slots (flat index t*K + k), F expert hidden dim, R rows of the
  * expert-major buffer, El = number of local experts (hi - lo).
@@ -81,7 +85,7 @@ int mi355_router_gate_fwd(const void* x, int x_dtype, const void* w, int w_dtype
 /*
  * The same product left as `splits` (T,E) partial sums, for a consumer that adds them itself
  * (mi355_route_plan): mi355_router_gate_fwd_splits is their number, 0 where this form does not
- * exist.  logit_bias goes in here when splits is 1 and is the consumer's to add otherwise.
+ * exist.  x, w and partial start on 16-byte boundaries (MI355_EINVAL otherwise).  logit_bias goes in here when splits is 1 and is the consumer's to add otherwise.
  * pieces: scratch of mi355_router_gate_fwd_pieces_bytes (NULL if that is 0); it holds the
  * weight pieces afterwards and may be handed to mi355_router_gate_add_bwd.
  */

@@ -10,6 +10,7 @@
 
 #include <cstdarg>
 #include <cstdio>
+#include <initializer_list>
 
 #include "../../include/mi355_moe.h"
 
@@ -28,6 +29,11 @@ int check_launch(const char* what);
   } while (0)
 
 inline bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+inline bool aligned16(std::initializer_list<const void*> ps) {
+  for (const void* p : ps)
+    if (!aligned16(p)) return false;
+  return true;
+}
 inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 
 // One-time set-up per device (kernel attributes are per device): `needed()` is true until

@@ -191,7 +191,7 @@ extern "C" int mi355_grouped_swiglu_fwd(const void* rows, const int32_t* token_o
   if (token_of_row)
     return fail(MI355_EUNSUP, "grouped_swiglu_fwd: the token gather needs bf16 with D and F multiples of 64; "
                               "materialise the rows with mi355_permute_rows_fwd instead");
-  if (any_path_ok(dtype, D, F, row_capacity)) {
+  if (any_path_ok(dtype, D, F, row_capacity, {rows, w1, w3, w2, gate, up, h, y})) {
     const AnySeg g{seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity, El};
     if (int rc = any_gateup(g, dtype, rows, w1, w3, gate, up, h, D, F, row_capacity, s)) return rc;
     return any_linear(g, dtype, h, w2, y, F, D, row_capacity, s);
@@ -241,7 +241,7 @@ extern "C" int mi355_grouped_swiglu_bwd(const void* dy, const void* rows,
   // (with no rows at all nothing is gathered: only the zero weight gradients remain to be written)
   if (token_of_row && row_capacity > 0 && tile_capacity > 0)
     return fail(MI355_EUNSUP, "grouped_swiglu_bwd: the token gather needs bf16 with D and F multiples of 64");
-  if (any_path_ok(dtype, D, F, row_capacity)) {
+  if (any_path_ok(dtype, D, F, row_capacity, {dy, rows, w1, w3, w2, gate, up, h, dgate, dup, drows, dw1, dw3, dw2})) {
     const AnySeg g{seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity, El};
     const bool some = row_capacity > 0 && tile_capacity > 0;
     if (some)
@@ -321,7 +321,7 @@ extern "C" int mi355_grouped_linear_fwd(const void* x, const void* w, int dtype,
     return bf16_grouped_fwd(nullptr, nullptr, 0, nullptr, nullptr, w, seg_offsets, seg_counts, tile_expert, tile_row0,
                             num_tiles, tile_capacity, nullptr, nullptr, const_cast<void*>(x), y, El, O, I, row_capacity, 2,
                             s);
-  if (any_path_ok(dtype, I, O, row_capacity))
+  if (any_path_ok(dtype, I, O, row_capacity, {x, w, y}))
     return any_linear({seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity, El}, dtype, x, w, y, I, O,
                       row_capacity, s);
   const Seg sg{seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity};
@@ -352,7 +352,7 @@ extern "C" int mi355_grouped_linear_bwd(const void* dy, const void* x, const voi
                               nullptr, nullptr, nullptr, nullptr, dw, El, O, I, 16, s);
     return MI355_OK;
   }
-  if (any_path_ok(dtype, I, O, row_capacity)) {
+  if (any_path_ok(dtype, I, O, row_capacity, {dy, x, w, dx, dw})) {
     const AnySeg g{seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity, El};
     if (dx && rows)
       if (int rc = any_linear_dx(g, dtype, dy, w, dx, I, O, row_capacity, s)) return rc;

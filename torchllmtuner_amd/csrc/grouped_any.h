@@ -14,7 +14,7 @@ struct AnyGrad {  // c (El, M, N) = per segment a^T (rows, M) . b (rows, N)
   int64_t M, N;
 };
 
-bool any_path_ok(int dtype, int64_t D, int64_t F, int64_t R);
+bool any_path_ok(int dtype, int64_t D, int64_t F, int64_t R, std::initializer_list<const void*> matrices);
 int any_gateup(const AnySeg& g, int dtype, const void* rows, const void* w1, const void* w3, void* gate, void* up, void* h,
                int64_t D, int64_t F, int64_t R, hipStream_t s);
 // y (R, O) = x (R, I) . w (El, O, I)^T, and its input gradient

@@ -5,7 +5,8 @@
 // TM x TN output tile, each wave (TM/2) x (TN/2) in 32x32 accumulators (v_mfma_f32_32x32x16_bf16, or
 // v_mfma_f32_32x32x2_f32 for fp32), 128 bytes of the contraction per step, two LDS stages, the next
 // step's operands held in registers.  Operands are fetched 16 bytes at a time whatever the width
-// (buffer loads: dword alignment suffices, and what lies past a matrix reads as zero); the tail of
+// (buffer loads: dword alignment suffices for them, and what lies past a matrix reads as zero; the ends store
+// four elements at a time, so the matrices themselves start on 16-byte boundaries); the tail of
 // the contraction is zeroed as it is parked.  LDS holds an operand as it lies in memory -- contraction
 // contiguous [row][128 B + 16] or strided [k][cols + pad], the pads chosen so that fragment reads
 // are free of bank conflicts -- and the fragment reads (b128, b32, or the transposing b64 for bf16)
@@ -456,9 +457,10 @@ int64_t dw_tiles(AnyArgs& p, int64_t El, int tile) {
 
 }  // namespace
 
-// (a matrix of rows and an expert's weights within the 32-bit range of the operand offsets)
-bool any_path_ok(int dtype, int64_t D, int64_t F, int64_t R) {
-  return (dtype == MI355_F32 || dtype == MI355_BF16) && D % 4 == 0 && F % 4 == 0 &&
+// (a matrix of rows and an expert's weights within the 32-bit range of the operand offsets; matrices that
+// start anywhere else than an allocation would go to the strided kernels, which load element by element)
+bool any_path_ok(int dtype, int64_t D, int64_t F, int64_t R, std::initializer_list<const void*> matrices) {
+  return aligned16(matrices) && (dtype == MI355_F32 || dtype == MI355_BF16) && D % 4 == 0 && F % 4 == 0 &&
          std::max(R * std::max(D, F), D * F) * (dtype == MI355_F32 ? 4 : 2) < (int64_t{1} << 32) - 4;
 }
 

@@ -458,7 +458,7 @@ extern "C" int mi355_router_gate_fwd(const void* x, int x_dtype, const void* w, 
   MI355_REQUIRE(T < (1ll << 31) && D < (1ll << 31), "router_gate_fwd: shape exceeds int32");
   if (T == 0) return MI355_OK;
   MI355_REQUIRE(x && w && logits, "router_gate_fwd: null pointer");
-  const int splits = aligned16(x) && aligned16(w) ? router_fwd_splits(x_dtype, w_dtype, T, D, E) : 0;
+  const int splits = aligned16({x, w, logit_bias, logits, workspace}) ? router_fwd_splits(x_dtype, w_dtype, T, D, E) : 0;
   const int64_t pieces = splits ? router_fwd_pieces_bytes(x_dtype, w_dtype, T, D, E) : 0;
   if (splits > 0 && (workspace || (splits == 1 && pieces == 0))) {
     float* partial = splits > 1 ? reinterpret_cast<float*>(static_cast<char*>(workspace) + pieces) : logits;
@@ -501,12 +501,14 @@ extern "C" int mi355_router_gate_add_bwd(const float* dlogits, const void* x, in
   MI355_REQUIRE(T >= 0 && D >= 1 && E >= 1 && T < (1ll << 31) && D < (1ll << 31),
                 "router_gate_bwd: bad shape");
   hipStream_t s = as_stream(stream);
-  if (workspace && router_x3_ok(x_dtype, w_dtype, D, E)) {
+  // (both of these fetch and store 16 bytes at a time; the strided kernel looks for itself)
+  const bool vec = workspace && aligned16({dlogits, x, w, pieces, addend, dx, dw, workspace});
+  if (vec && router_x3_ok(x_dtype, w_dtype, D, E)) {
     MI355_REQUIRE(dlogits && w && (x || !dw), "router_gate_bwd: null pointer");
     return router_x3_bwd(dlogits, x, static_cast<const float*>(w), pieces, addend, dx, static_cast<float*>(dw),
                          workspace, T, D, E, s);
   }
-  if (workspace && T > 0 && router_few_ok(x_dtype, w_dtype, D, E) && (dx || dw)) {
+  if (vec && T > 0 && router_few_ok(x_dtype, w_dtype, D, E) && (dx || dw)) {
     MI355_REQUIRE(dlogits && w && (x || !dw), "router_gate_bwd: null pointer");
     return router_few_bwd(dlogits, x, x_dtype, static_cast<const float*>(w), addend, dx, static_cast<float*>(dw), workspace,
                           T, D, E, s);

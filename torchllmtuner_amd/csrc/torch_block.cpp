@@ -300,7 +300,7 @@ Grads block_backward(const Block& b, const Tensor& kept, const Tensor& dout_, co
   const auto opts = b.x.options();
   const int64_t item = b.dt == MI355_F32 ? 4 : 2;
   const hipStream_t main = static_cast<hipStream_t>(L.stream);
-  const Tensor dout = (dout_.scalar_type() == b.x.scalar_type() ? dout_ : dout_.to(b.x.scalar_type())).contiguous();
+  const Tensor dout = dense(dout_.scalar_type() == b.x.scalar_type() ? dout_ : dout_.to(b.x.scalar_type()));
   Kept k;
   Carver held{static_cast<char*>(kept.data_ptr())};
   k.layout(held, b, true);
@@ -515,8 +515,6 @@ struct MoeBlock : public torch::autograd::Function<MoeBlock> {
   }
 };
 
-Tensor contiguous(const OptTensor& t) { return t.has_value() && t->defined() ? t->contiguous() : Tensor(); }
-
 void check_weights(const Block& b) {
   const Tensor &x = b.x, &w1 = b.w1, &w2 = b.w2;
   TORCH_CHECK_VALUE(x.dim() == 2 && x.size(0) >= 1 && b.gate_w.dim() == 2 && b.gate_w.size(1) == x.size(1), "gate weight ",
@@ -567,8 +565,8 @@ void check_stats(const Block& b, const Stats& st) {
 // The block of a forward call, checked.
 std::pair<Block, Stats> block_of(BLOCK_PARAMS) {
   const Stats st{some(histogram), some(aux_acc), some(aux_denominator), aux_coeff};
-  Block b{x.contiguous(), gate_w.contiguous(), contiguous(gate_b), contiguous(expert_b), w1.contiguous(),
-          w3.contiguous(), w2.contiguous(), contiguous(sg), contiguous(su), contiguous(sd), contiguous(mask),
+  Block b{dense(x), dense(gate_w), dense(gate_b), dense(expert_b), dense(w1), dense(w3), dense(w2), dense(sg), dense(su),
+          dense(sd), dense(mask),
           Config{K, score_func, route_norm, num_groups, num_limited, lo, hi, align, round_terms, overlap_shared,
                  st.aux_denominator.defined(), route_scale}};
   check_weights(b);
@@ -608,8 +606,8 @@ std::tuple<Tensor, Tensor, Tensor> moe_block_fwd_meta(BLOCK_PARAMS) {
 
 // The block and what is asked of a backward call, checked.
 std::pair<Block, Needs> block_bwd_of(BLOCK_BWD_PARAMS) {
-  Block b{x.contiguous(), gate_w.contiguous(), contiguous(gate_b), Tensor(), w1.contiguous(), w3.contiguous(),
-          w2.contiguous(), contiguous(sg), contiguous(su), contiguous(sd), contiguous(mask),
+  Block b{dense(x), dense(gate_w), dense(gate_b), Tensor(), dense(w1), dense(w3), dense(w2), dense(sg), dense(su), dense(sd),
+          dense(mask),
           Config{K, score_func, route_norm, 0, 0, lo, hi, align, 0, overlap_shared, aux, route_scale}};
   check_weights(b);
   b.sizes();
@@ -625,7 +623,7 @@ std::pair<Block, Needs> block_bwd_of(BLOCK_BWD_PARAMS) {
 
 NineTensors moe_block_bwd(BLOCK_BWD_PARAMS) {
   const auto [b, need] = block_bwd_of(BLOCK_BWD_ARGS);
-  Grads g = block_backward(b, kept, dout, need);
+  Grads g = block_backward(b, dense(kept), dout, need);  // (a saved-tensor hook may hand back a view)
   return {g.x, g.gate_w, g.gate_b, g.w1, g.w3, g.w2, g.sg, g.su, g.sd};
 }
 

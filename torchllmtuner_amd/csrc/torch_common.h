@@ -101,7 +101,14 @@ inline void check(int rc, const char* what) {
   TORCH_CHECK(false, what, " failed (", rc, "): ", msg);
 }
 
-inline Tensor cf(const Tensor& t) { return t.scalar_type() == at::kFloat ? t.contiguous() : t.to(at::kFloat).contiguous(); }
+// The tensor as the kernels read it: contiguous, and starting on a 16-byte boundary as an allocation of its own
+// does.  A view into a flat buffer need not, and the kernels fetch 16 bytes at a time: such a one is copied.
+inline Tensor dense(const Tensor& t) {
+  Tensor c = t.contiguous();
+  return reinterpret_cast<uintptr_t>(ptr(c)) % 16 == 0 ? c : c.clone();
+}
+inline Tensor dense(const OptTensor& t) { return t.has_value() && t->defined() ? dense(*t) : Tensor(); }
+inline Tensor cf(const Tensor& t) { return dense(t.scalar_type() == at::kFloat ? t : t.to(at::kFloat)); }
 inline Tensor bytes(int64_t n, const Tensor& like) {
   return at::empty({n > 0 ? n : 1}, like.options().dtype(at::kByte));
 }

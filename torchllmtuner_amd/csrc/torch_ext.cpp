@@ -28,7 +28,7 @@ using namespace mi355_torch;
 // ------------------------------------------------------------------ router
 Tensor router_gate_fwd(const Tensor& x_, const Tensor& w_, const OptTensor& bias_) {
   Launch L(x_);
-  const Tensor x = x_.contiguous(), w = w_.contiguous();
+  const Tensor x = dense(x_), w = dense(w_);
   TORCH_CHECK_VALUE(x.dim() == 2 && w.dim() == 2 && w.size(1) == x.size(1), "gate weight ", w.sizes(),
                     " does not match input ", x.sizes());
   const int64_t T = x.size(0), D = x.size(1), E = w.size(0);
@@ -47,7 +47,7 @@ Tensor router_gate_fwd(const Tensor& x_, const Tensor& w_, const OptTensor& bias
 std::tuple<Tensor, Tensor> router_gate_bwd(const Tensor& dlogits_, const Tensor& x_, const Tensor& w_, bool need_dx,
                                            bool need_dw) {
   Launch L(x_);
-  const Tensor dl = cf(dlogits_), x = x_.contiguous(), w = w_.contiguous();
+  const Tensor dl = cf(dlogits_), x = dense(x_), w = dense(w_);
   const int64_t T = x.size(0), D = x.size(1), E = w.size(0);
   Tensor dx = need_dx ? at::empty_like(x) : none_like(x);
   Tensor dw = need_dw ? at::empty_like(w) : none_like(w);
@@ -67,7 +67,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> router_select_fwd(const Tensor& logit
                                                              bool want_map) {
   Launch L(logits_);
   TORCH_CHECK_TYPE(logits_.scalar_type() == at::kFloat, "router logits must be float32");
-  const Tensor logits = logits_.contiguous();
+  const Tensor logits = dense(logits_);
   const int64_t T = logits.size(0), E = logits.size(1);
   OptTensor bias;
   if (bias_.has_value()) bias = cf(*bias_);
@@ -89,7 +89,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> router_select_cutoff_fwd(const Tensor
                                                                     double route_scale) {
   Launch L(logits_);
   TORCH_CHECK_TYPE(logits_.scalar_type() == at::kFloat, "router logits must be float32");
-  const Tensor logits = logits_.contiguous();
+  const Tensor logits = dense(logits_);
   const int64_t T = logits.size(0), E = logits.size(1);
   OptTensor bias;
   if (bias_.has_value()) bias = cf(*bias_);
@@ -108,7 +108,7 @@ Tensor router_select_bwd(const Tensor& logits_, const Tensor& ids_, const OptTen
                          const OptTensor& dscores_, int64_t score_func, bool route_norm, double route_scale,
                          int64_t mode) {
   Launch L(logits_);
-  const Tensor logits = logits_.contiguous(), ids = ids_.contiguous();
+  const Tensor logits = dense(logits_), ids = dense(ids_);
   const int64_t T = logits.size(0), E = logits.size(1), K = ids.size(1);
   OptTensor dw, ds;
   if (dweights_.has_value()) dw = cf(*dweights_);
@@ -129,7 +129,7 @@ void quantile_observe(Tensor histogram, const Tensor& scores_, const Tensor& cut
   const Tensor scores = cf(scores_), cutoff = cf(cutoff_.reshape({-1})), bias = cf(bias_);
   const int64_t T = scores.size(0), E = scores.size(1);
   OptTensor pad;
-  if (pad_.has_value()) pad = pad_->contiguous();
+  if (pad_.has_value()) pad = dense(*pad_);
   check(mi355_quantile_observe(fptr(scores), fptr(cutoff), fptr(bias), static_cast<const uint8_t*>(ptr(pad)),
                                histogram.data_ptr<int64_t>(), T, E, histogram.size(1), L.stream),
         "quantile_observe");
@@ -138,7 +138,7 @@ void quantile_observe(Tensor histogram, const Tensor& scores_, const Tensor& cut
 Tensor quantile_estimate(const Tensor& histogram_, const Tensor& bias_, int64_t K) {
   Launch L(histogram_);
   TORCH_CHECK_TYPE(histogram_.scalar_type() == at::kLong, "histogram_EB must be int64");
-  const Tensor hist = histogram_.contiguous(), bias = cf(bias_);
+  const Tensor hist = dense(histogram_), bias = cf(bias_);
   const int64_t E = hist.size(0), B = hist.size(1);
   Tensor out = at::empty({E}, bias.options());
   Tensor ws = at::empty({2 * E}, bias.options());
@@ -152,7 +152,7 @@ std::tuple<Tensor, Tensor> rms_norm_fwd(const Tensor& x_, const Tensor& weight_,
   Launch L(x_);
   TORCH_CHECK_TYPE(x_.scalar_type() == weight_.scalar_type(), "rms_norm: input (", x_.scalar_type(), ") and weight (",
                    weight_.scalar_type(), ") must share a dtype");
-  const Tensor x = x_.contiguous(), weight = weight_.contiguous();
+  const Tensor x = dense(x_), weight = dense(weight_);
   const int64_t D = weight.numel(), rows = D > 0 ? x.numel() / D : 0;
   Tensor y = at::empty_like(x);
   Tensor rstd = at::empty({rows}, x.options().dtype(at::kFloat));
@@ -165,8 +165,8 @@ std::tuple<Tensor, Tensor> rms_norm_fwd(const Tensor& x_, const Tensor& weight_,
 std::tuple<Tensor, Tensor> rms_norm_bwd(const Tensor& dy_, const Tensor& x_, const Tensor& weight_,
                                         const Tensor& rstd, bool need_dx, bool need_dw) {
   Launch L(x_);
-  const Tensor x = x_.contiguous(), weight = weight_.contiguous();
-  const Tensor dy = (dy_.scalar_type() == x.scalar_type() ? dy_ : dy_.to(x.scalar_type())).contiguous();
+  const Tensor x = dense(x_), weight = dense(weight_);
+  const Tensor dy = dense(dy_.scalar_type() == x.scalar_type() ? dy_ : dy_.to(x.scalar_type()));
   const int64_t D = weight.numel(), rows = D > 0 ? x.numel() / D : 0;
   Tensor dx = need_dx ? at::empty_like(x) : none_like(x);
   Tensor dw = need_dw ? at::empty_like(weight) : none_like(weight);
@@ -181,10 +181,10 @@ std::tuple<Tensor, Tensor> rms_norm_bwd(const Tensor& dy_, const Tensor& x_, con
 Tensor balance_loss_fwd(const Tensor& scores_, const Tensor& map_, const OptTensor& pad_) {
   Launch L(scores_);
   TORCH_CHECK_TYPE(scores_.scalar_type() == at::kFloat, "router scores must be float32");
-  const Tensor scores = scores_.contiguous(), map = map_.contiguous();
+  const Tensor scores = dense(scores_), map = dense(map_);
   const int64_t T = scores.size(0), E = scores.size(1);
   OptTensor pad;
-  if (pad_.has_value()) pad = pad_->contiguous();
+  if (pad_.has_value()) pad = dense(*pad_);
   Tensor out = at::empty({1 + E}, scores.options());
   Tensor ws = bytes(mi355_balance_loss_workspace_bytes(T, E), scores);
   check(mi355_balance_loss_fwd(fptr(scores), static_cast<const uint8_t*>(ptr(map)),
@@ -196,10 +196,11 @@ Tensor balance_loss_fwd(const Tensor& scores_, const Tensor& map_, const OptTens
 
 Tensor balance_loss_bwd(const Tensor& scores_, const Tensor& f_, const OptTensor& pad_, const Tensor& grad_) {
   Launch L(scores_);
-  const Tensor scores = scores_.contiguous(), f = cf(f_), g = cf(grad_.reshape({1}));
+  // (f and g are read one by one, and f lies behind the loss in one tensor: as it is)
+  const Tensor scores = dense(scores_), f = f_.to(at::kFloat).contiguous(), g = grad_.reshape({1}).to(at::kFloat);
   const int64_t T = scores.size(0), E = scores.size(1);
   OptTensor pad;
-  if (pad_.has_value()) pad = pad_->contiguous();
+  if (pad_.has_value()) pad = dense(*pad_);
   Tensor out = at::empty_like(scores);
   check(mi355_balance_loss_bwd(fptr(scores), fptr(f), static_cast<const uint8_t*>(ptr(pad)), fptr(g),
                                out.data_ptr<float>(), T, E, L.stream),
@@ -212,7 +213,7 @@ int64_t tile_m() { return mi355_grouped_tile_m(MI355_BF16); }
 
 std::tuple<Tensor, Tensor, Tensor> permute_plan(const Tensor& ids_, int64_t E, int64_t lo, int64_t hi, int64_t align) {
   Launch L(ids_);
-  const Tensor ids = (ids_.scalar_type() == at::kLong ? ids_ : ids_.to(at::kLong)).contiguous();
+  const Tensor ids = dense(ids_.scalar_type() == at::kLong ? ids_ : ids_.to(at::kLong));
   TORCH_CHECK_VALUE(ids.dim() == 2, "expert ids must have shape (tokens, top_k)");
   const int64_t T = ids.size(0), K = ids.size(1), N = T * K, El = hi - lo, tm = tile_m();
   TORCH_CHECK_VALUE(El >= 1, "permute_plan: empty local expert range");
@@ -241,7 +242,7 @@ std::tuple<Tensor, Tensor, Tensor> permute_plan(const Tensor& ids_, int64_t E, i
 
 Tensor segments_from_counts(const Tensor& counts_, int64_t total_rows) {
   Launch L(counts_);
-  const Tensor counts = (counts_.scalar_type() == at::kInt ? counts_ : counts_.to(at::kInt)).contiguous();
+  const Tensor counts = dense(counts_.scalar_type() == at::kInt ? counts_ : counts_.to(at::kInt));
   const int64_t El = counts.size(0), tm = tile_m();
   const int64_t tile_cap = total_rows / tm + El + 1;
   Tensor small = at::empty({(El + 1) + 2 * El + 2 * tile_cap + 1}, counts.options());
@@ -261,7 +262,7 @@ Tensor segments_from_counts(const Tensor& counts_, int64_t total_rows) {
 Tensor permute_rows_fwd(const Tensor& x_, const Tensor& row_of_slot, const OptTensor& slot_of_row,
                         const Tensor& total_rows, int64_t K, int64_t row_capacity) {
   Launch L(x_);
-  const Tensor x = x_.contiguous();
+  const Tensor x = dense(x_);
   const int64_t T = x.size(0), D = x.size(1);
   Tensor rows = at::empty({row_capacity, D}, x.options());
   check(mi355_permute_rows_fwd(ptr(x), dtype_code(x), iptr(row_of_slot), iptr(slot_of_row), iptr(total_rows),
@@ -272,7 +273,7 @@ Tensor permute_rows_fwd(const Tensor& x_, const Tensor& row_of_slot, const OptTe
 
 Tensor permute_rows_bwd(const Tensor& drows_, const Tensor& row_of_slot, int64_t T, int64_t K) {
   Launch L(drows_);
-  const Tensor drows = drows_.contiguous();
+  const Tensor drows = dense(drows_);
   const int64_t D = drows.size(1);
   Tensor dx = at::empty({T, D}, drows.options());
   check(mi355_permute_rows_bwd(ptr(drows), dtype_code(drows), iptr(row_of_slot), ptr(dx), T, D, K, L.stream),
@@ -287,7 +288,7 @@ Tensor combine_fwd(const Tensor& y_, const Tensor& weights_, const Tensor& row_o
   (void)slot_of_row;
   (void)total_rows;
   Launch L(y_);
-  const Tensor y = y_.contiguous(), w = cf(weights_);
+  const Tensor y = dense(y_), w = cf(weights_);
   const int64_t D = y.size(1);
   Tensor out = at::empty({T, D}, y.options());
   check(mi355_combine_fwd(ptr(y), dtype_code(y), fptr(w), iptr(row_of_slot), ptr(out), T, D, K, (int)round_terms,
@@ -300,8 +301,8 @@ std::tuple<Tensor, Tensor> combine_bwd(const Tensor& dout_, const Tensor& y_, co
                                        const Tensor& row_of_slot, const OptTensor& slot_of_row,
                                        const OptTensor& total_rows, int64_t K) {
   Launch L(y_);
-  const Tensor y = y_.contiguous(), w = cf(weights_);
-  const Tensor dout = (dout_.scalar_type() == y.scalar_type() ? dout_ : dout_.to(y.scalar_type())).contiguous();
+  const Tensor y = dense(y_), w = cf(weights_);
+  const Tensor dout = dense(dout_.scalar_type() == y.scalar_type() ? dout_ : dout_.to(y.scalar_type()));
   const int64_t T = dout.size(0), D = y.size(1), R = y.size(0);
   Tensor dy = at::empty_like(y);
   Tensor dw = at::empty({T, K}, y.options().dtype(at::kFloat));
@@ -358,7 +359,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> grouped_swiglu_fwd(
     const Tensor& seg_offsets, const Tensor& seg_counts, const Tensor& tile_expert, const Tensor& tile_row0,
     const Tensor& num_tiles, int64_t row_capacity, bool zero_fill) {
   Launch L(rows_);
-  const Tensor rows = rows_.contiguous(), w1 = w1_.contiguous(), w3 = w3_.contiguous(), w2 = w2_.contiguous();
+  const Tensor rows = dense(rows_), w1 = dense(w1_), w3 = dense(w3_), w2 = dense(w2_);
   check_weights(rows, w1, w3, w2);
   const int64_t D = rows.size(1), El = w1.size(0), F = w1.size(1), R = row_capacity;
   const Plan p = plan_of(seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles);
@@ -374,12 +375,13 @@ std::tuple<Tensor, Tensor, Tensor, Tensor> grouped_swiglu_fwd(
 
 std::tuple<Tensor, Tensor, Tensor, Tensor> grouped_swiglu_bwd(
     const Tensor& dy_, const Tensor& rows_, const OptTensor& token_of_row, const Tensor& w1_, const Tensor& w3_,
-    const Tensor& w2_, const Tensor& gate, const Tensor& up, const Tensor& h, const Tensor& seg_offsets,
+    const Tensor& w2_, const Tensor& gate_, const Tensor& up_, const Tensor& h_, const Tensor& seg_offsets,
     const Tensor& seg_counts, const Tensor& tile_expert, const Tensor& tile_row0, const Tensor& num_tiles,
     bool need_drows, bool need_dw, bool zero_fill) {
   Launch L(rows_);
-  const Tensor rows = rows_.contiguous(), w1 = w1_.contiguous(), w3 = w3_.contiguous(), w2 = w2_.contiguous();
-  const Tensor dy = (dy_.scalar_type() == rows.scalar_type() ? dy_ : dy_.to(rows.scalar_type())).contiguous();
+  const Tensor rows = dense(rows_), w1 = dense(w1_), w3 = dense(w3_), w2 = dense(w2_);
+  const Tensor gate = dense(gate_), up = dense(up_), h = dense(h_);
+  const Tensor dy = dense(dy_.scalar_type() == rows.scalar_type() ? dy_ : dy_.to(rows.scalar_type()));
   const int64_t D = rows.size(1), El = w1.size(0), F = w1.size(1), R = dy.size(0);
   const Plan p = plan_of(seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles);
   Tensor dgate = at::empty_like(gate), dup = at::empty_like(up);
@@ -402,7 +404,7 @@ Tensor grouped_linear_fwd(const Tensor& x_, const Tensor& w_, const Tensor& seg_
                           const Tensor& tile_expert, const Tensor& tile_row0, const Tensor& num_tiles,
                           bool zero_fill) {
   Launch L(x_);
-  const Tensor x = x_.contiguous(), w = w_.contiguous();
+  const Tensor x = dense(x_), w = dense(w_);
   TORCH_CHECK_VALUE(x.dim() == 2 && w.dim() == 3 && w.size(2) == x.size(1), "grouped weight ", w.sizes(),
                     " does not match rows ", x.sizes());
   TORCH_CHECK_TYPE(w.scalar_type() == x.scalar_type(), "grouped weight and rows must share one dtype");
@@ -420,8 +422,8 @@ std::tuple<Tensor, Tensor> grouped_linear_bwd(const Tensor& dy_, const Tensor& x
                                               const Tensor& tile_expert, const Tensor& tile_row0,
                                               const Tensor& num_tiles, bool need_dx, bool need_dw, bool zero_fill) {
   Launch L(x_);
-  const Tensor x = x_.contiguous(), w = w_.contiguous();
-  const Tensor dy = (dy_.scalar_type() == x.scalar_type() ? dy_ : dy_.to(x.scalar_type())).contiguous();
+  const Tensor x = dense(x_), w = dense(w_);
+  const Tensor dy = dense(dy_.scalar_type() == x.scalar_type() ? dy_ : dy_.to(x.scalar_type()));
   const int64_t R = x.size(0), I = x.size(1), El = w.size(0), O = w.size(1);
   TORCH_CHECK_VALUE(dy.dim() == 2 && dy.size(0) == R && dy.size(1) == O, "grouped_linear_bwd: gradient ", dy.sizes(),
                     " does not match (", R, ", ", O, ")");
@@ -445,7 +447,7 @@ std::tuple<Tensor, Tensor, Tensor> gather_experts_combine_fwd(
     int64_t row_capacity, bool round_terms, bool save_gate_up) {
   (void)slot_of_row;  // for the backward only (the row -> slot index behind the row scales)
   Launch L(x_);
-  const Tensor x = x_.contiguous(), w1 = w1_.contiguous(), w3 = w3_.contiguous(), w2 = w2_.contiguous();
+  const Tensor x = dense(x_), w1 = dense(w1_), w3 = dense(w3_), w2 = dense(w2_);
   check_weights(x, w1, w3, w2);
   const Tensor w = cf(weights_);
   const int64_t T = x.size(0), D = x.size(1), El = w1.size(0), F = w1.size(1), R = row_capacity;
@@ -471,13 +473,13 @@ std::tuple<Tensor, Tensor, Tensor> gather_experts_combine_fwd(
 // Returns (dx, dw1, dw3, dw2, dweights).
 std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor> gather_experts_combine_bwd(
     const Tensor& dout_, const Tensor& x_, const Tensor& weights_, const Tensor& w1_, const Tensor& w3_,
-    const Tensor& w2_, const Tensor& gate, const Tensor& up, const Tensor& token_of_row, const Tensor& slot_of_row,
+    const Tensor& w2_, const Tensor& gate_, const Tensor& up_, const Tensor& token_of_row, const Tensor& slot_of_row,
     const Tensor& row_of_slot, const Tensor& seg_offsets, const Tensor& seg_counts, const Tensor& tile_expert,
     const Tensor& tile_row0, const Tensor& num_tiles, int64_t K, bool need_dx, bool need_dw) {
   Launch L(x_);
-  const Tensor x = x_.contiguous(), w1 = w1_.contiguous(), w3 = w3_.contiguous(), w2 = w2_.contiguous();
-  const Tensor dout = (dout_.scalar_type() == x.scalar_type() ? dout_ : dout_.to(x.scalar_type())).contiguous();
-  const Tensor w = cf(weights_);
+  const Tensor x = dense(x_), w1 = dense(w1_), w3 = dense(w3_), w2 = dense(w2_);
+  const Tensor dout = dense(dout_.scalar_type() == x.scalar_type() ? dout_ : dout_.to(x.scalar_type()));
+  const Tensor w = cf(weights_), gate = dense(gate_), up = dense(up_);
   const int64_t T = x.size(0), D = x.size(1), El = w1.size(0), F = w1.size(1), R = gate.size(0);
   const int64_t slots = mi355_grouped_combine_bwd_slots(dtype_code(x), D, F);
   TORCH_CHECK(slots > 0, "gather_experts_combine_bwd does not cover this dtype/shape");
