@@ -91,3 +91,17 @@ def test_the_backward_operator_refuses_what_the_forward_did_not_keep():
             op(*args(torch.empty_like(x), kept[:-256]))
         with pytest.raises(ValueError, match="gradient"):
             op(*args(torch.empty(T + 1, D, dtype=BF, device="meta"), kept))
+
+
+@pytest.mark.parametrize("shared", [False, True])
+def test_the_backward_has_no_derivative_and_says_so(shared):
+    gate_w, w1, w3, w2, three, gate_b = _weights(shared, True)
+    x = torch.empty(T, D, dtype=BF, device="meta", requires_grad=True)
+    wanted = [t for t in (x, gate_w, gate_b, w1, w3, w2, *three) if t is not None]
+    out, _ = _call(x, gate_w, w1, w3, w2, three, gate_b)
+    grads = torch.autograd.grad(out, wanted, torch.ones_like(out), create_graph=True)  # by itself no error
+    for g in grads:
+        with pytest.raises(RuntimeError, match="moe_block_bwd is not implemented"):
+            torch.autograd.grad(g, w1, torch.ones_like(g), retain_graph=True, allow_unused=True)
+    out, _ = _call(x, gate_w, w1, w3, w2, three, gate_b)
+    assert not any(g.requires_grad for g in torch.autograd.grad(out, wanted, torch.ones_like(out)))

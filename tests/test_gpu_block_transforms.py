@@ -69,10 +69,10 @@ def test_a_traced_block_computes_what_the_block_computes(dtype, D, F, shared):
     counted = block.tokens_per_expert_E.clone()
     got, want = graph(_x(2, dtype, D)), step(_x(2, dtype, D))
     # With a shared expert the stages add the three input gradients in another order than the one operator: two
-    # roundings of half an ulp on either side, of sums of about the total's size.
+    # roundings on either side (unit roundoff 2^-8 for bf16, 2^-24 for fp32), of sums of about the total's size.
     order = {1} if shared else set()
     _equal([t for i, t in enumerate(got) if i not in order], [t for i, t in enumerate(want) if i not in order])
-    bound = 4 * 2.0 ** (-9 if dtype == torch.bfloat16 else -24)
+    bound = 4 * 2.0 ** (-8 if dtype == torch.bfloat16 else -24)
     assert float((got[1] - want[1]).detach().float().norm()) <= bound * float(want[1].detach().float().norm())
     assert int((block.tokens_per_expert_E - counted).sum()) == 2 * T * K  # the graph counts, and so does the step
 
@@ -204,3 +204,14 @@ def test_weights_that_are_plain_attributes(which):
                 object.__setattr__(module, name, module._parameters.pop(name).detach().requires_grad_())
         assert block._forward_as_one(x) is None
         _equal([block(x)], [want])
+
+
+def test_a_gradient_penalty_raises():
+    for dtype, D, F, shared in SHAPES:
+        block, x = _block(dtype, D, F, shared), _x(1, dtype, D).requires_grad_()
+        gout = _x(2, dtype, D)
+        plain = torch.autograd.grad(block(x), x, gout)[0]
+        dx, = torch.autograd.grad(block(x), x, gout, create_graph=True)
+        _equal([dx], [plain])
+        with pytest.raises(RuntimeError, match="moe_block_bwd is not implemented"):
+            dx.float().square().sum().backward()

@@ -25,6 +25,7 @@
 // reads in one allocation, a pass's scratch in another.  Work on the
 // library's side streams is forked from the current stream and joined before the operator returns, so
 // buffers need no record_stream.
+#include <torch/csrc/autograd/autograd_not_implemented_fallback.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/library.h>
@@ -490,7 +491,10 @@ struct MoeBlock : public torch::autograd::Function<MoeBlock> {
     const int gb = 2, w = gb + (s[2].defined() ? 1 : 0) + (c.back() ? 1 : 0), sh = w + 3;
     auto wants = [&](int i) { return ctx->needs_input_grad(i); };
     const bool shared = s[6].defined();
-    at::AutoDispatchBelowADInplaceOrView below;
+    // A pass that is itself differentiated (create_graph) leaves the gradients with a node that raises: there
+    // is no derivative of the backward, and without one a gradient penalty would leave the block out unnoticed.
+    std::optional<at::AutoDispatchBelowADInplaceOrView> below;
+    if (!at::GradMode::is_enabled()) below.emplace();
     static auto op = typed_op<BlockBwdSig>("mi355_moe::moe_block_bwd");
     auto [dx, dgate_w, dgate_b, dw1, dw3, dw2, dsg, dsu, dsd] =
         op.call(grads[0], s[0], s[1], opt(s[2]), s[3], s[4], s[5], opt(s[6]), opt(s[7]), opt(s[8]), s[9], opt(s[10]), c[0],
@@ -673,4 +677,7 @@ TORCH_LIBRARY_IMPL(mi355_moe, Meta, m) {
   m.impl("moe_block_fwd", moe_block_fwd_meta);
   m.impl("moe_block_bwd", moe_block_bwd_meta);
 }
-TORCH_LIBRARY_IMPL(mi355_moe, Autograd, m) { m.impl("moe_block", moe_block_autograd); }
+TORCH_LIBRARY_IMPL(mi355_moe, Autograd, m) {
+  m.impl("moe_block", moe_block_autograd);
+  m.impl("moe_block_bwd", torch::autograd::autogradNotImplementedFallback());
+}
