@@ -291,3 +291,44 @@ def test_rms_norm_rows_in_registers_match_fp64(dtype, rows, D):
         assert err < tol, f"{name}: rel-L2 {err}"
     only_dw = ops.rms_norm_bwd(dy.to(DEV), x.to(DEV), w.to(DEV), rstd, need_dx=False)[1]
     assert torch.equal(only_dw, dw)
+
+
+def test_default_overlap_adds_the_input_gradients_in_another_order_than_the_stages():
+    """With a shared expert beside the routed path, as by default, the engine adds the stages' three bf16 input
+    gradients as (routed + gate) + shared; the operator as (routed + shared) + gate, whatever the overlap.  All
+    else is the same bits; the two sums differ by their roundings."""
+    dtype, T, D, E, K, F = torch.bfloat16, 1025, 512, 64, 4, 384
+    spec = R.RouterSpec(E, K, score_func="softmax", route_norm=True)
+    p = make_params(E, D, F, dtype, seed=3, std=0.05, shared_F=448)
+    g = torch.Generator().manual_seed(4)
+    x, gout = (torch.randn(T, D, generator=g).to(dtype).to(DEV) for _ in range(2))
+
+    def run(in_stages, overlap=True, shared=True, gate=True):
+        block = build_block(p, spec, D, F, dtype, DEV).train()
+        assert block.overlap_shared_experts
+        block.overlap_shared_experts = overlap
+        if not shared:
+            block.shared_experts = None
+        if in_stages:
+            block.router.register_forward_hook(lambda m, a, out: None if gate else (out[0].detach(), *out[1:]))
+        xin = x.clone().requires_grad_()
+        out = block(xin)
+        out.backward(gout)
+        return [xin.grad, out.detach(), block.tokens_per_expert_E] + [q.grad for q in block.parameters() if q.grad is not None]
+
+    one, stages = run(False), run(True)
+    for overlap in (True, False):
+        for a, b in zip(one, run(False, overlap), strict=True):
+            assert torch.equal(a, b)
+    for i, (a, b) in enumerate(zip(one[1:], stages[1:], strict=True)):
+        assert torch.equal(a, b), f"tensor {i}"
+    assert torch.equal(one[0], run(True, overlap=False)[0])  # (one stream: the operator's order)
+    # routed, gate and shared by themselves bound the two roundings of either sum (unit roundoff 2^-8)
+    block = build_block(p, spec, D, F, dtype, DEV)
+    xin = x.clone().requires_grad_()
+    block.shared_experts(xin).backward(gout)
+    shared, routed, routed_gate = (t.double() for t in (xin.grad, run(True, shared=False, gate=False)[0], run(True, shared=False)[0]))
+    total = routed_gate + shared
+    bound = 2.0 ** -8 * (routed_gate.abs() + (routed + shared).abs() + 2 * total.abs()) * (1 + 2.0 ** -5) + 1e-30
+    diff = (one[0].double() - stages[0].double()).abs()
+    assert bool((diff <= bound).all()), float((diff / bound).max())

@@ -19,7 +19,11 @@
 //     launches instead of four, the score gradient's pieces are summed by the selection's backward, and
 //     the additions of (T, D) tensors -- shared expert's output, the two or three input gradients -- ride
 //     in kernels that hold the other operand anyway.
-// Every kernel and every rounding is the stage operators' own: both ways give the same bits.
+// Every kernel and every rounding is the stage operators' own: both ways give the same bits, but for the order of
+// two sums.  The load-balance loss adds its tokens up in another order, and with a shared expert the input
+// gradient is (routed + shared) + gate here, while the autograd engine adds the stages' three as
+// (routed + gate) + shared when the shared expert runs on its own stream, as it does by default: as many
+// roundings, other bits.
 //
 // Memory.  From PyTorch's allocator on the current stream: the results one by one, what the backward
 // reads in one allocation, a pass's scratch in another.  Work on the

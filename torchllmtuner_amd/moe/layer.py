@@ -237,9 +237,9 @@ class MoE(nn.Module):
         (``mi355_moe::moe_block``), or None when a stage has to be visible or is not what it computes: a
         hook or an override anywhere below, an observer, another auxiliary loss, router, dispatcher,
         activation or shared expert, a weight that is no parameter or of a tensor subclass, fp64, no tokens,
-        a tracing compiler, a dispatch mode or a function transform.  Both ways give the same bits
-        (the load-balance loss: the same sums in another order).  In training the counts leave out the
-        tokens of ``padding_mask``."""
+        a tracing compiler, a dispatch mode or a function transform.  Both ways give the same bits, but for
+        the order of sums in the load-balance loss and, with a shared expert that runs beside the routed
+        ones, in the input gradient.  In training the counts leave out the tokens of ``padding_mask``."""
         if (
             torch.compiler.is_compiling()
             or _intercepted()
