@@ -412,8 +412,13 @@ __global__ __launch_bounds__(256) void any_dx_dw_kernel(AnyArgs dx, AnyArgs dw, 
 template <int MODE, int TM, int TN>
 int launch_any(const AnyArgs& p, int dtype, int64_t blocks, hipStream_t s, const char* what) {
   if (blocks <= 0) return MI355_OK;
-  if (TM == 32 || dtype == MI355_F32) hipLaunchKernelGGL((any_kernel<float, MODE, TM, TN>), dim3((unsigned)blocks), dim3(256), 0, s, p);
-  else if constexpr (TM != 32) hipLaunchKernelGGL((any_kernel<uint16_t, MODE, TM, TN>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+  if (dtype == MI355_F32) {
+    hipLaunchKernelGGL((any_kernel<float, MODE, TM, TN>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+  } else if constexpr (TM != 32) {
+    hipLaunchKernelGGL((any_kernel<uint16_t, MODE, TM, TN>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+  } else {
+    return fail(MI355_EUNSUP, "%s: 32-row tiles are for fp32", what);
+  }
   return check_launch(what);
 }
 
