@@ -293,6 +293,49 @@ def test_rms_norm_rows_in_registers_match_fp64(dtype, rows, D):
     assert torch.equal(only_dw, dw)
 
 
+@pytest.mark.parametrize("T,E,K,local,align,groups", [
+    (1, 1, 1, None, 1, None), (32, 60, 16, None, 1, None), (33, 128, 8, (32, 96), 1, None), (64, 256, 16, None, 128, (8, 4)),
+    (65, 17, 3, None, 1, None), (1000, 256, 8, (0, 32), 16, (8, 4)), (8191, 128, 8, None, 1, None), (8193, 128, 8, (5, 6), 1, None),
+    (16449, 64, 2, None, 16, None)])
+def test_route_plan_equals_selection_and_plan(T, E, K, local, align, groups):
+    """The C entry without statistics: ids, weights and every array of the plan, against the selection and the plan
+    as two calls; around the sizes at which its launches change."""
+    from torchllmtuner_amd import _lib, ops
+
+    print(f"route plan T={T} E={E} K={K} local={local} align={align} groups={groups}", flush=True)
+    lo, hi = local or (0, E)
+    El, splits = hi - lo, 3
+    g = torch.Generator().manual_seed(T)
+    partial = torch.randn(splits, T, E, generator=g).to(DEV)
+    bias, expert_b = torch.randn(E, generator=g).to(DEV), (0.1 * torch.randn(E, generator=g)).to(DEV)
+    logits = partial[0] + partial[1] + partial[2] + bias
+    G, L = groups or (0, 0)
+    w, ids, _ = ops.router_select_fwd(logits, expert_b, K, "sigmoid", True, 2.5, G, L)
+    plan = ops.permute_plan(ids, E, lo, hi, align)
+    i32 = lambda n: torch.full((n,), -7, dtype=torch.int32, device=DEV)
+    f32 = lambda *n: torch.full(n, float("nan"), device=DEV)
+    R_, cap = plan.row_capacity, plan.tile_capacity
+    got_logits, got_w, got_ids = f32(T, E), f32(T, K), torch.empty(T, K, dtype=torch.int64, device=DEV)
+    counts, offsets, seg_counts, ros, sor, tor = i32(E), i32(El + 1), i32(2 * El), i32(T * K), i32(R_), i32(R_)
+    scale, te, tr, nt = f32(R_), i32(cap), i32(cap), i32(1)
+    lib = _lib.load()
+    work = torch.empty(max(1, lib.mi355_route_plan_workspace_bytes(T, K, E)), dtype=torch.uint8, device=DEV)
+    rc = lib.mi355_route_plan(
+        partial.data_ptr(), splits, bias.data_ptr(), got_logits.data_ptr(), expert_b.data_ptr(), T, E, K, 0, 1, 2.5, G, L,
+        got_w.data_ptr(), got_ids.data_ptr(), lo, hi, align, ops.TILE_M, counts.data_ptr(), offsets.data_ptr(),
+        seg_counts.data_ptr(), ros.data_ptr(), sor.data_ptr(), tor.data_ptr(), scale.data_ptr(), R_, te.data_ptr(),
+        tr.data_ptr(), nt.data_ptr(), cap, work.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, "route_plan")
+    n = int(nt)
+    for name, a, b in (("logits", got_logits, logits), ("ids", got_ids, ids), ("weights", got_w, w), ("counts", counts, plan.counts_E),
+                       ("offsets", offsets, plan.seg_offsets), ("seg_counts", seg_counts[:El], plan.seg_counts),
+                       ("order", seg_counts[El:], plan.expert_order), ("row_of_slot", ros, plan.row_of_slot),
+                       ("slot_of_row", sor, plan.slot_of_row), ("token_of_row", tor, plan.token_of_row),
+                       ("row_scale", scale, ops.combine_row_scale(w, plan)), ("num_tiles", nt, plan.num_tiles),
+                       ("tile_expert", te[:n], plan.tile_expert[:n]), ("tile_row0", tr[:n], plan.tile_row0[:n])):
+        assert torch.equal(a, b), name
+
+
 def test_default_overlap_adds_the_input_gradients_in_another_order_than_the_stages():
     """With a shared expert beside the routed path, as by default, the engine adds the stages' three bf16 input
     gradients as (routed + gate) + shared; the operator as (routed + shared) + gate, whatever the overlap.  All
