@@ -235,8 +235,9 @@ def test_gate_gradients_of_few_experts_match_fp64(dtype, T, D, E):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("D,K,addend", [(2056, 8, True), (8, 1, False), (516, 11, True), (70, 3, True)])
 def test_combine_of_few_tokens_equals_that_of_many(dtype, D, K, addend):
-    """The combine deals a row's columns over waves below 4096 tokens: the tokens of a 4096-token call, bit for
-    bit, with absent slots, more than eight slots and rows that are not whole 16-byte pieces; and fp64 sums."""
+    """The combine deals a row's columns over workgroups: the tokens of a 4096-token call, bit for bit, whatever the
+    number of tokens, with absent slots, more than eight slots, rows that end inside a 1 KiB piece and rows that
+    are not whole 16-byte vectors; and fp64 sums."""
     from torchllmtuner_amd import _lib
 
     print(f"combine {dtype} D={D} K={K}", flush=True)

@@ -1,6 +1,6 @@
 // Weighted unpermute-combine and its backward (which also yields the router's
-// score gradient).  Both are bandwidth kernels: one wavefront per token, 16-byte
-// lanes along D, the K row indices and weights held in lanes 0..K-1 and broadcast
+// score gradient).  Both are bandwidth kernels: a wavefront per token (or per 1 KiB of a
+// token's row), 16-byte lanes along D, the K row indices and weights held in lanes 0..K-1 and broadcast
 // by shuffles.  No atomics: every output element has exactly one writer, so the
 // result is deterministic.
 #include <algorithm>
@@ -56,15 +56,23 @@ __device__ __forceinline__ void plus(float (&a)[Vec<T>::N], const uint4& v) {
   for (int q = 0; q < Vec<T>::N; ++q) a[q] = round_to<T>(a[q]) + f[q];
 }
 
-// SMALL_K: K <= 8, the eight-row chunk below is the only one.  Pieces of G vectors per lane are dealt over
-// gridDim.y.
-template <typename T, bool SMALL_K, int G>
+// SMALL_K: K <= 8, the eight-row chunk below is the only one.
+//   A token's row is cut into `pieces` of 1 KiB, one wave each, and the workgroups of a token's pieces follow one
+// another: few tokens fill the chip, and what runs at one time reads whole rows.  (All tokens' first
+// pieces, then all second ones, and so on reads the same KiB of rows that lie a power of two apart, few memory channels
+// at a time.)  Eight bf16 rows a token, us, one wave a row in passes of 4 KiB / pieces in that other order / here:
+//   8192 tokens of 1024 columns 37 / 29 / 29, of 2048 57 / 71 / 54 (5.6 TB/s), of 4096 112 / 134 / 107, of 7168
+//   197 / 193 / 186; 3000 of 2048 21 / 23 / 21; 1000 of 4096 18 / 13 / 13; 128 of 7168 21 / 5.1 / 5.1; 1 of 2048
+//   6.6 / 3.7 / 3.7.  Sixteen rows, 8192 of 2048 108 / 137 / 100.  One row in eight present (one rank's share of 8
+//   ranks), 4095 of 7168 44 / 33 / 33, 8192 of 2048 22 / 20 / 19.
+template <typename T, bool SMALL_K>
 __global__ __launch_bounds__(256) void combine_fwd_kernel(
     const T* __restrict__ y, const float* __restrict__ weights,
     const int32_t* __restrict__ row_of_slot, const T* __restrict__ addend, T* __restrict__ out, int T_, int D, int K,
-    int round_terms) {
+    int round_terms, int pieces) {
   const int lane = threadIdx.x & 63;
-  const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int tokens = blockIdx.x / pieces, piece = blockIdx.x % pieces;
+  const int t = tokens * 4 + (threadIdx.x >> 6);
   if (t >= T_) return;
   const int64_t s0 = static_cast<int64_t>(t) * K;
   const int row = lane < K ? row_of_slot[s0 + lane] : -1;
@@ -92,22 +100,17 @@ __global__ __launch_bounds__(256) void combine_fwd_kernel(
   // Loops are uniform across the wave (shuffles need every lane).
   if (D % V == 0) {
     const int nv = D / V;
-    // G vectors per lane and pass (4 KiB of every row per wave with G = 4) from eight rows at a time, all
-    // requested before the first is used: 32 KiB in flight per wave.  Rows and weights are
-    // wave-uniform; the terms are still added in visiting order.
+    // one vector per lane from eight rows at a time, all requested before the first is used.  Rows and weights
+    // are wave-uniform; the terms are added in visiting order.
     constexpr int B = 8;
-    auto request = [&](int base, int p0, uint4 (&v)[B][G], float (&ww)[B]) {
+    auto request = [&](int i, int p0, uint4 (&v)[B], float (&ww)[B]) {
 #pragma unroll
       for (int j = 0; j < B; ++j) {
         const int p = max(min(p0 + j, nvalid - 1), 0);  // past the end: not loaded, not used
         const int r = __builtin_amdgcn_readlane(o_row, p);  // p is wave-uniform
         ww[j] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(o_w), p));
         const uint4* src = reinterpret_cast<const uint4*>(y + static_cast<int64_t>(max(r, 0)) * D);
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-          const int i = base + g * kWave + lane;
-          v[j][g] = (p0 + j < nvalid && i < nv) ? load_stream(src + i) : make_uint4(0, 0, 0, 0);
-        }
+        v[j] = (p0 + j < nvalid && i < nv) ? load_stream(src + i) : make_uint4(0, 0, 0, 0);
       }
     };
     auto add_terms = [&](float (&a)[V], const uint4& v, float w) {
@@ -119,56 +122,26 @@ __global__ __launch_bounds__(256) void combine_fwd_kernel(
         a[q] += round_terms ? round_to<T>(term) : term;
       }
     };
-    for (int base = blockIdx.y * G * kWave; base < nv; base += gridDim.y * G * kWave) {
-      if constexpr (SMALL_K) {
-        // one chunk: each vector is summed and stored on its own (8 live accumulators, not 32,
-        // which is what lets three waves share a SIMD)
-        uint4 v[B][G];
+    for (int base = piece * kWave; base < nv; base += pieces * kWave) {
+      const int i = base + lane;
+      float a[V];
+#pragma unroll
+      for (int q = 0; q < V; ++q) a[q] = 0.0f;
+      for (int p0 = 0; p0 < (SMALL_K ? 1 : nvalid); p0 += B) {
+        uint4 v[B];
         float ww[B];
-        request(base, 0, v, ww);
+        request(i, p0, v, ww);
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-          float a[V];
-#pragma unroll
-          for (int q = 0; q < V; ++q) a[q] = 0.0f;
-#pragma unroll
-          for (int j = 0; j < B; ++j)
-            if (j < nvalid) add_terms(a, v[j][g], ww[j]);
-          const int i = base + g * kWave + lane;
-          if (i < nv) {
-            if (add) plus<T>(a, reinterpret_cast<const uint4*>(add)[i]);
-            reinterpret_cast<uint4*>(dst)[i] = Vec<T>::pack(a);
-          }
-        }
-      } else {
-        float a[G][V];
-#pragma unroll
-        for (int g = 0; g < G; ++g)
-#pragma unroll
-          for (int q = 0; q < V; ++q) a[g][q] = 0.0f;
-        for (int p0 = 0; p0 < nvalid; p0 += B) {
-          uint4 v[B][G];
-          float ww[B];
-          request(base, p0, v, ww);
-#pragma unroll
-          for (int j = 0; j < B; ++j)
-            if (p0 + j < nvalid) {
-#pragma unroll
-              for (int g = 0; g < G; ++g) add_terms(a[g], v[j][g], ww[j]);
-            }
-        }
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-          const int i = base + g * kWave + lane;
-          if (i < nv) {
-            if (add) plus<T>(a[g], reinterpret_cast<const uint4*>(add)[i]);
-            reinterpret_cast<uint4*>(dst)[i] = Vec<T>::pack(a[g]);
-          }
-        }
+        for (int j = 0; j < B; ++j)
+          if (p0 + j < nvalid) add_terms(a, v[j], ww[j]);
+      }
+      if (i < nv) {
+        if (add) plus<T>(a, reinterpret_cast<const uint4*>(add)[i]);
+        reinterpret_cast<uint4*>(dst)[i] = Vec<T>::pack(a);
       }
     }
   } else {
-    for (int base = blockIdx.y * kWave; base < D; base += gridDim.y * kWave) {
+    for (int base = piece * kWave; base < D; base += pieces * kWave) {
       const int i = base + lane;
       const bool on = i < D;
       float a = 0.0f;
@@ -357,28 +330,23 @@ extern "C" int mi355_combine_add_fwd(const void* y, int dtype, const float* weig
   if (T == 0) return MI355_OK;
   MI355_REQUIRE(weights && row_of_slot && out, "combine_fwd: null pointer");
   MI355_REQUIRE(!addend || dtype != MI355_F64, "combine_fwd: no fp64 form with an addend");
-  // Few tokens: one wave a token leaves most of the chip idle and a wide row to several passes of one wave, so
-  // a wave takes 1 KiB of the row instead of 4.  4 KiB / 1 KiB a wave, eight rows of 2048 columns a token: 1 token 6.0 /
-  // 3.9 us, 33 7.7 / 5.0, 1000 12.7 / 10.8, 8192 52.5 / 54.5; 3000 tokens of 6 x 1024 15.0 / 11.5; 128 of 7168 columns
-  // 22.4 / 5.0.
-  const bool spread = T < 4096;
-  const int64_t pieces = (D * (dtype == MI355_F32 ? 4 : 2) + 1023) / 1024;  // 64 lanes of 16 bytes
-  const dim3 grid((unsigned)((T + 3) / 4), spread ? (unsigned)std::min<int64_t>(pieces, 1024) : 1);
+  const int64_t tokens = (T + 3) / 4;  // groups of one workgroup's four
+  const int64_t kib = (D * (dtype == MI355_F32 ? 4 : 2) + 1023) / 1024;  // 64 lanes of 16 bytes
+  const int64_t pieces = std::max<int64_t>(1, std::min<int64_t>(kib, 0xffffff / tokens));  // a launch: below 2^32 lanes
   auto launch = [&](auto kernel, auto* yp, auto* op) {
-    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, as_stream(stream), yp, weights, row_of_slot,
-                       static_cast<decltype(yp)>(addend), op, (int)T, (int)D, (int)K, round_terms);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(tokens * pieces)), dim3(256), 0, as_stream(stream), yp, weights, row_of_slot,
+                       static_cast<decltype(yp)>(addend), op, (int)T, (int)D, (int)K, round_terms, (int)pieces);
   };
   auto run = [&](auto* yp, auto* op) {
     using E = std::remove_pointer_t<decltype(op)>;
-    if (K <= 8) launch(spread ? combine_fwd_kernel<E, true, 1> : combine_fwd_kernel<E, true, 4>, yp, op);
-    else launch(spread ? combine_fwd_kernel<E, false, 1> : combine_fwd_kernel<E, false, 4>, yp, op);
+    launch(K <= 8 ? combine_fwd_kernel<E, true> : combine_fwd_kernel<E, false>, yp, op);
   };
   if (dtype == MI355_F32) {
     run(static_cast<const float*>(y), static_cast<float*>(out));
   } else if (dtype == MI355_BF16) {
     run(static_cast<const uint16_t*>(y), static_cast<uint16_t*>(out));
   } else if (dtype == MI355_F64) {
-    hipLaunchKernelGGL(combine_fwd_f64_kernel, dim3(grid.x), dim3(256), 0, as_stream(stream), static_cast<const double*>(y),
+    hipLaunchKernelGGL(combine_fwd_f64_kernel, dim3((unsigned)tokens), dim3(256), 0, as_stream(stream), static_cast<const double*>(y),
                        weights, row_of_slot, static_cast<double*>(out), (int)T, (int)D, (int)K);
   } else
     return fail(MI355_EINVAL, "combine_fwd: unknown dtype %d", dtype);
