@@ -296,7 +296,8 @@ def test_rms_norm_rows_in_registers_match_fp64(dtype, rows, D):
 
 @pytest.mark.parametrize("T,E,K,local,align,groups", [
     (1, 1, 1, None, 1, None), (32, 60, 16, None, 1, None), (33, 128, 8, (32, 96), 1, None), (64, 256, 16, None, 128, (8, 4)),
-    (65, 17, 3, None, 1, None), (1000, 256, 8, (0, 32), 16, (8, 4)), (8191, 128, 8, None, 1, None), (8193, 128, 8, (5, 6), 1, None),
+    (65, 17, 3, None, 1, None), (1000, 256, 8, (0, 32), 16, (8, 4)), (7000, 132, 4, None, 1, None),
+    (7001, 132, 4, None, 1, None), (8192, 128, 8, None, 1, None), (8193, 128, 8, (5, 6), 1, None),
     (16449, 64, 2, None, 16, None)])
 def test_route_plan_equals_selection_and_plan(T, E, K, local, align, groups):
     """The C entry without statistics: ids, weights and every array of the plan, against the selection and the plan

@@ -12,7 +12,7 @@
 //                   both directions; the first workgroup writes the plan's lists.
 // A single workgroup does both at once.  Bound by launches, instruction issue and dependent latency throughout: at 33
 // tokens of 128 experts the four launches this replaces took 29 us of GPU time, at 8192 tokens
-// (8 each) 39 us; here 12 and 23.
+// (8 each) 39 us; here 12 and 19.
 #include <algorithm>
 #include <type_traits>
 
@@ -422,23 +422,27 @@ __global__ __launch_bounds__(kLanes) void route_rows_kernel(const float* __restr
 }
 
 // Lanes per workgroup.  Selection is bound by instruction issue, so its tokens want to be spread over the
-// CUs; but every workgroup of route_rows reads all histograms, so there should not be more than two hundred
-// or so.  Both kernels together at 128 experts, 1024 / 512 / 256 lanes: 21 / 15 / 16 us at 1000 tokens, 22 / 19 / 26 at
-// 4096, 23 / 22 / 30 at 8192.  Up to 64 tokens one workgroup does everything, up to 32 with 512 lanes: fewer
-// waves to clear counters for and to meet at barriers (8 tokens 9.9 us with 1024, 9.6 with 512; 32 tokens 11.5 / 10.9).
-int route_lanes(int64_t T) { return T <= 32 || (T > 64 && T < 8192) ? 512 : 1024; }
-int route_chunks(int64_t T) {
-  const int64_t rows = route_lanes(T) / 16, groups = (T + rows - 1) / rows;
+// CUs: 512 lanes, as long as each of at most kMaxBlocks workgroups has one chunk of tokens (8192).  Every workgroup of
+// route_rows reads all histograms, so with more than 128 experts the line lies lower.  Up to 64 tokens one
+// workgroup does everything, with 512 lanes where they hold the tokens (32): fewer waves to clear counters for and to
+// meet at barriers.  All launches together, us, 512 / 1024 lanes:
+//   experts, choices   8 tokens    32           33           64           1000         7000         8192         9000
+//    64, 6              7.5 / 8.1   8.2 / 8.7   11.3 / 9.6   11.3 / 10.5  11.9 / 14.7  14.2 / 15.5  14.2 / 15.7  17.6 / 15.9
+//   128, 8              9.5 / 10.3 10.9 / 11.6  13.8 / 12.2  13.9 / 13.7  14.9 / 18.0  18.8 / 19.9  19.4 / 20.1  24.1 / 21.3
+//   256, 8             14.1 / 14.4 16.9 / 17.4  20.3 / 18.7  20.9 / 21.5  21.5 / 26.3  29.0 / 29.8  31.3 / 29.2  37.1 / 31.6
+int route_lanes(int64_t T, int64_t E) { return T <= 32 || (T > 64 && T <= (E > 128 ? 7000 : 8192)) ? 512 : 1024; }
+int route_chunks(int64_t T, int64_t E) {
+  const int64_t rows = route_lanes(T, E) / 16, groups = (T + rows - 1) / rows;
   return static_cast<int>((groups + kMaxBlocks - 1) / kMaxBlocks);
 }
-int64_t route_blocks(int64_t T) {
-  const int64_t per = static_cast<int64_t>(route_chunks(T)) * (route_lanes(T) / 16);
+int64_t route_blocks(int64_t T, int64_t E) {
+  const int64_t per = static_cast<int64_t>(route_chunks(T, E)) * (route_lanes(T, E) / 16);
   return (T + per - 1) / per;
 }
 // calls f(integral_constant lanes)
 template <typename Fn>
-void with_lanes(int64_t T, Fn f) {
-  const int lanes = route_lanes(T);
+void with_lanes(int64_t T, int64_t E, Fn f) {
+  const int lanes = route_lanes(T, E);
   if (lanes == 512) f(std::integral_constant<int, 512>{});
   else f(std::integral_constant<int, 1024>{});
 }
@@ -453,11 +457,11 @@ extern "C" int mi355_route_plan_covers(int64_t E, int64_t K, int num_groups, int
 }
 
 extern "C" int64_t mi355_route_plan_workspace_bytes(int64_t T, int64_t K, int64_t E) {
-  if (K < 1 || E < 1 || T < 1 || route_blocks(T) == 1) return 0;
-  return (T * K + route_blocks(T) * E) * (int64_t)sizeof(int32_t);
+  if (K < 1 || E < 1 || T < 1 || route_blocks(T, E) == 1) return 0;
+  return (T * K + route_blocks(T, E) * E) * (int64_t)sizeof(int32_t);
 }
 extern "C" int64_t mi355_route_stats_workspace_bytes(int64_t T, int64_t E) {
-  return T < 1 || E < 1 ? 0 : 2 * route_blocks(T) * E * (int64_t)sizeof(int32_t);
+  return T < 1 || E < 1 ? 0 : 2 * route_blocks(T, E) * E * (int64_t)sizeof(int32_t);
 }
 
 static int route_plan(const float* partial, int splits, const float* logit_bias, float* logits,
@@ -485,23 +489,23 @@ static int route_plan(const float* partial, int splits, const float* logit_bias,
   MI355_REQUIRE(partial && splits >= 1 && aligned16(partial) && weights && ids && counts_E && seg_offsets &&
                     seg_counts && row_of_slot && slot_of_row && token_of_row && tile_expert && tile_row0 && num_tiles,
                 "route_plan: null or misaligned pointer");
-  MI355_REQUIRE(route_blocks(T) == 1 || workspace, "route_plan: workspace required");
+  MI355_REQUIRE(route_blocks(T, E) == 1 || workspace, "route_plan: workspace required");
   hipStream_t s = as_stream(stream);
   const SelectArgs sel{expert_bias, (int)E, (int)K, score_func, route_norm, route_scale, num_groups, num_limited};
   const PlanOut p{(int)lo, (int)hi, (int)align, (int)tile_m, (int)row_capacity, (int)tile_capacity, counts_E,
                   seg_offsets, seg_counts, row_of_slot, slot_of_row, token_of_row, row_scale, tile_expert, tile_row0,
                   num_tiles};
-  const int chunks = route_chunks(T);
-  const int blocks = (int)route_blocks(T);
+  const int chunks = route_chunks(T, E);
+  const int blocks = (int)route_blocks(T, E);
   uint32_t* rank = static_cast<uint32_t*>(workspace);
   int32_t* hist = reinterpret_cast<int32_t*>(rank + (blocks > 1 ? T * K : 0));
   // every row has a slot when all experts are local and nothing is padded
   const int fill = !(lo == 0 && hi == E && align == 1 && row_capacity == T * K);
   const bool stats = st.valid_counts || st.f;
-  const int waves = route_lanes(T) / kWave;
+  const int waves = route_lanes(T, E) / kWave;
   const size_t lds = ((1 + waves) * E * (stats ? 2 : 1) + (blocks == 1 ? layout_words((int)E) : 0)) * sizeof(int32_t);
   with_row_shape(E, [&](auto vpr, auto full) {
-    with_lanes(T, [&](auto lanes) {
+    with_lanes(T, E, [&](auto lanes) {
       hipLaunchKernelGGL((route_rank_kernel<decltype(vpr)::value, decltype(full)::value, decltype(lanes)::value>), dim3(blocks),
                          dim3(lanes), lds, s, partial, splits, logit_bias, logits, sel, weights, ids, rank, hist, (int)T,
                          chunks, fill, p, st);
@@ -509,7 +513,7 @@ static int route_plan(const float* partial, int splits, const float* logit_bias,
   });
   if (int rc = check_launch("route_rank")) return rc;
   if (blocks > 1) {
-    with_lanes(T, [&](auto lanes) {
+    with_lanes(T, E, [&](auto lanes) {
       hipLaunchKernelGGL(route_rows_kernel<decltype(lanes)::value>, dim3(blocks), dim3(lanes), layout_words((int)E) * sizeof(int32_t),
                          s, weights, ids, rank, hist, (int)T, (int)E, (int)K, chunks, p, st);
     });
@@ -547,7 +551,7 @@ extern "C" int mi355_route_plan_stats(
   MI355_REQUIRE(!aux_acc || aux_acc_dtype == MI355_F32 || aux_acc_dtype == MI355_BF16, "route_plan_stats: aux_acc is fp32 or bf16");
   MI355_REQUIRE((!aux_f_E && !valid_counts_E) || stats_workspace, "route_plan_stats: workspace required");
   int32_t* block_valid = static_cast<int32_t*>(stats_workspace);
-  float* block_share = block_valid ? reinterpret_cast<float*>(block_valid + (T >= 1 ? route_blocks(T) : 0) * E) : nullptr;
+  float* block_share = block_valid ? reinterpret_cast<float*>(block_valid + (T >= 1 ? route_blocks(T, E) : 0) * E) : nullptr;
   const StatsOut st{padding_mask_T, valid_counts_E, scores_TE, cutoff_T, aux_f_E, aux_scale, aux_acc, aux_acc_dtype, aux_denominator,
                     aux_coeff, block_valid, block_share};
   return route_plan(partial, splits, logit_bias, logits, expert_bias, T, E, K, score_func, route_norm, route_scale,
