@@ -7,8 +7,8 @@
 // split the contraction of 16 output columns (of gate and up, or 32 of the down projection) of one
 // expert; every wave loads its weights straight into MFMA fragments, 16 KiB requested ahead, up
 // to sixteen waves to a CU, and the four partial tiles are added in wave order through LDS.
-//   Bound by HBM: 709 MB of gate and up weights (33 tokens of 128 experts, 2048 x 768) in 117 us, 6.0 TB/s
-// where a plain read in this pattern reaches 6.15 (145 us before); one token, 50 MB, 14 us (31 before).
+//   Bound by HBM: 709 MB of gate and up weights (33 tokens of 128 experts, 2048 x 768) in 116 us, 6.1 TB/s
+// where a plain read in this pattern reaches 6.15 (145 us before); one token, 50 MB, 13 us (31 before).
 // Waves along the contraction rather than side by side: at one token 12-25 us less in all, at 33 the
 // same.  32 or 64 rows per wave instead of 16 need registers that the requests in flight want: slower.
 //   A contraction step is 64 wide: lane group g = lane / 16 holds k = 16 g .. 16 g + 15 of it (two

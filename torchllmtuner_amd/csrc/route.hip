@@ -12,7 +12,7 @@
 //                   both directions; the first workgroup writes the plan's lists.
 // A single workgroup does both at once.  Bound by launches, instruction issue and dependent latency throughout: at 33
 // tokens of 128 experts the four launches this replaces took 29 us of GPU time, at 8192 tokens
-// (8 each) 39 us; here 12 and 19.
+// (8 each) 39 us; here 13 and 21.
 #include <algorithm>
 #include <type_traits>
 

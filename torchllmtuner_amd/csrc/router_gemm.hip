@@ -70,8 +70,8 @@ __global__ __launch_bounds__(256) void split_kernel(const float* __restrict__ w,
 // of k inside a 32-wide step is a permutation (lane half h holds k = 16 h ..) that both operands
 // share, so that each lane reads whole 32- or 64-byte pieces of a row.
 // This replaces a kernel that walked the whole contraction in 128-expert tiles behind a separate
-// weight-splitting launch: 1 token of 2048 x 128 experts 34 -> 5 us, 1000 tokens 43 -> 14 us, 128
-// tokens of 7168 x 256 experts 131 -> 12 us.  From 1024 tokens on, with widths on its grid, the
+// weight-splitting launch: 1 token of 2048 x 128 experts 34 -> 8 us, 1000 tokens 43 -> 12 us, 128
+// tokens of 7168 x 256 experts 131 -> 12 us (profiled inside the block, the weights from memory).  From 1024 tokens on, with widths on its grid, the
 // 128-token kernel below reads the weights four times less often and is the faster one.
 constexpr int R_BM = 32, R_BN = 32, R_WAVES = 8, R_STEP = 32;
 
@@ -491,7 +491,7 @@ __global__ __launch_bounds__(W_NT, 2) void gate_dw_kernel(const float* __restric
 // keep up with memory.  A thread owns four columns.  dW workgroups (the first `dw_blocks`): eight experts,
 // 256 columns and a slice of the tokens, the four waves on every fourth token, joined through LDS in wave
 // order; the slices' sums are added by splitk_reduce.  dx workgroups: 32 tokens x 256 columns, dlogits in LDS.
-// 1531 tokens, 320 x 16, bf16: 9 us with the sum, 47 with the strided GEMMs it replaces.
+// 1531 tokens, 320 x 16, bf16: 12 us with the sum, 47 with the strided GEMMs it replaces.
 constexpr int S_EB = 8, S_COLS = 256, S_TOK = 32, S_MAX_E = 32;
 
 __device__ __forceinline__ f32x4 load_cols(const float* p) { return *reinterpret_cast<const f32x4*>(p); }

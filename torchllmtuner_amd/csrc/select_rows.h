@@ -161,8 +161,8 @@ struct RowChoice {
 // winner (lanes hold ascending experts, so ties go to the lower index), and its expert travels to
 // lane k by a permute nothing waits for.  Where the choice is by logit, the winner's logit is in
 // the key, so only the K winners' score functions are evaluated.  Per token of 128 experts and K = 8 about half
-// the instructions of the (value, index, score) triples compared and carried before: one wave alone
-// 5.1 -> 2.4 us, sixteen waves of a workgroup 10.0 -> 4.5.
+// the instructions of the (value, index, score) triples compared and carried before: the selection of 8192
+// tokens as a kernel of its own 8.7 -> 5.9 us.
 template <int VPR, bool FULL>
 __device__ __forceinline__ RowChoice select_row(const SelectArgs& p, const float (&x)[VPR], int l, bool want_scores,
                                                 bool want_cutoff, float (&s)[VPR], float& cutoff) {
