@@ -4,6 +4,7 @@ these see."""
 
 import pytest
 import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
 from torch.fx.experimental.proxy_tensor import make_fx
 from torch.utils._python_dispatch import TorchDispatchMode
 
@@ -27,8 +28,8 @@ def _call(x, gate_w, w1, w3, w2, shared=(None, None, None), gate_b=None):
     return ops.moe_block(x, gate_w, gate_b, None, w1, w3, w2, shared, K, "softmax", True, 1.0, 0, 0, 0, E, 1, True, True)
 
 
-def _weights(shared, bias, dtype=BF):
-    mk = lambda *s, dtype=dtype: torch.empty(s, dtype=dtype, device="meta", requires_grad=True)
+def _weights(shared, bias, dtype=BF, device="meta"):
+    mk = lambda *s, dtype=dtype: torch.empty(s, dtype=dtype, device=device, requires_grad=True)
     three = (mk(192, D), mk(192, D), mk(D, 192)) if shared else (None, None, None)
     return mk(E, D, dtype=torch.float32), mk(E, F, D), mk(E, F, D), mk(E, D, F), three, mk(E, dtype=torch.float32) if bias else None
 
@@ -50,6 +51,21 @@ def test_a_dispatch_mode_sees_the_block_operators_and_not_their_allocations(shar
     with torch.no_grad(), Names() as names:
         out, counts = _call(x, gate_w, w1, w3, w2, three, gate_b)
     assert names.seen == ["moe_block"] and out.shape == (T, D)
+
+
+@pytest.mark.parametrize("grad", [True, False])
+def test_fake_tensors_go_through_without_a_look_at_their_memory(grad):
+    with FakeTensorMode(), torch.set_grad_enabled(grad):
+        x = torch.empty(T, D, dtype=BF, device="cuda", requires_grad=True)
+        gate_w, w1, w3, w2, three, gate_b = _weights(True, True, device="cuda")
+        for t in (x, gate_w, w1, w3, w2, *three, gate_b):
+            torch._C._set_throw_on_mutable_data_ptr(t)
+        out, counts = _call(x, gate_w, w1, w3, w2, three, gate_b)
+        assert (out.shape, out.dtype, out.device.type, out.requires_grad) == ((T, D), BF, "cuda", grad)
+        assert (counts.shape, counts.dtype, counts.device.type) == ((E,), torch.int32, "cuda")
+        kept = torch.ops.mi355_moe.moe_block_fwd(x, gate_w, gate_b, None, w1, w3, w2, *three, K, 1, True, 1.0, 0, 0, 0, E, 1, True,
+                                                 True, None, None, None, 0.0, None)[2]
+        assert kept.dtype == torch.uint8 and kept.device.type == "cuda"
 
 
 def test_a_trace_records_the_block_operators():

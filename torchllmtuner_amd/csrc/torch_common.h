@@ -105,6 +105,7 @@ inline void check(int rc, const char* what) {
 // does.  A view into a flat buffer need not, and the kernels fetch 16 bytes at a time: such a one is copied.
 inline Tensor dense(const Tensor& t) {
   Tensor c = t.contiguous();
+  if (!c.is_cuda()) return c;  // (shapes only: no memory to look at)
   return reinterpret_cast<uintptr_t>(ptr(c)) % 16 == 0 ? c : c.clone();
 }
 inline Tensor dense(const OptTensor& t) { return t.has_value() && t->defined() ? dense(*t) : Tensor(); }
