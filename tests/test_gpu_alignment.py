@@ -2,6 +2,8 @@
 one to a boundary the kernels' 16-byte accesses want; the C entry points that have a form which loads
 element by element take that."""
 
+import contextlib
+
 import pytest
 import torch
 
@@ -54,6 +56,31 @@ def test_block_with_misaligned_operands_equals_the_aligned_one(dtype, T, D, E, F
 
     for i, (a, b) in enumerate(zip(run(shifted), run(lambda t: t))):
         assert torch.equal(a, b), f"tensor {i} differs by {float((a.float() - b.float()).abs().max())}"
+
+
+@pytest.mark.parametrize("dtype,D,F,shared", [(torch.bfloat16, 384, 448, 128), (torch.float32, 68, 36, 60)])
+def test_what_the_backward_reads_may_come_back_from_a_hook_anywhere(dtype, D, F, shared):
+    print(f"saved-tensor hooks {dtype} D={D}", flush=True)
+    p = make_params(16, D, F, dtype, seed=2, std=0.05, shared_F=shared)
+    g = torch.Generator().manual_seed(3)
+    x, gout = (torch.randn(70, D, generator=g).to(dtype).to(DEV) for _ in range(2))
+
+    def run(hooks):
+        block = build_block(p, R.RouterSpec(16, 2, score_func="softmax", route_norm=True), D, F, dtype, DEV).train()
+        xin = x.clone().requires_grad_()
+        with hooks:
+            out = block(xin)
+        out.backward(gout)
+        return [out.detach(), xin.grad] + [q.grad for q in block.parameters()]
+
+    away = torch.autograd.graph.saved_tensors_hooks(lambda t: t.cpu(), lambda t: shifted(t, 3))
+    want = run(contextlib.nullcontext())
+    for hooks in (away, torch.autograd.graph.save_on_cpu()):
+        for i, (a, b) in enumerate(zip(run(hooks), want, strict=True)):
+            assert torch.equal(a, b), f"tensor {i}"
+    block = build_block(p, R.RouterSpec(16, 2, score_func="softmax", route_norm=True), D, F, dtype, DEV).eval()
+    with torch.inference_mode():
+        assert torch.equal(block(x.clone()), want[0])
 
 
 def _call(name, *args):
