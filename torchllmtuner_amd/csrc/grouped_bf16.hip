@@ -114,6 +114,7 @@ struct RowArgs {
 
 struct TileMeta {
   int e, row0, valid, n0, nt;
+  int k_start;  // the contraction's first K step; it goes on from step 0 after the last
 };
 
 // sum over each group of 16 consecutive lanes, left in all 16 (DPP row operations)
@@ -127,7 +128,14 @@ __device__ __forceinline__ float row16_sum(float v) {
 
 // SAVE_GU (GATEUP only): also write gate and up, which the backward reads; a forward-only caller
 // leaves them out -- a third of the kernel's output bytes and of its epilogue's LDS traffic.
-template <int MODE, int NJ, bool GATHER, int WM, bool SAVE_GU = true>
+//
+// TURN (weights with the contraction contiguous): a tile's contraction starts at a K step of its own, by expert and
+// column tile, and goes on from step 0 after the last.  Workgroups run in step, and with the same start all of
+// them read the same 128 bytes of weight rows that lie a row length apart: rows of 2048 elements, 4 KiB, then meet few memory
+// channels at a time.  The column tile counts only where the output is a whole number of tiles: a last tile
+// that would overhang computes some of its neighbour's columns again and must give the same bits, so both add up in
+// the same order.  An expert's row tiles and, where there are several, its column tiles stay in step: they share operands in L2.
+template <int MODE, int NJ, bool GATHER, int WM, bool SAVE_GU = true, bool TURN = false>
 __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
   constexpr int WN = 8 / WM;               // waves along the columns (WM along the rows)
   constexpr int TBM = 64 * WM;             // rows of the tile
@@ -138,6 +146,7 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
   constexpr bool DH_LIKE = (MODE == RM_DH || MODE == RM_DLIN);  // same operands, different epilogue
   constexpr bool B_KS = (DH_LIKE || MODE == RM_DX);
   static_assert(!GATHER || MODE == RM_GATEUP || MODE == RM_DH, "only gate/up and dH gather their rows");
+  static_assert(!TURN || !B_KS, "only contractions that are contiguous in memory are turned");
   static_assert(!(GATHER && MODE == RM_DH) || NJ == 4, "the fused dH epilogue reduces over 16 lanes per row");
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
 
@@ -198,6 +207,7 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
     constexpr int W = (MODE == RM_GATEUP ? BNT / 2 : BNT);
     m.n0 = min(nt * W, Ncols - W);
     m.nt = nt;
+    m.k_start = TURN ? (5 * m.e + (nrt == 1 && Ncols % W == 0 ? 3 * nt : 0)) % ksteps : 0;
     return m;
   };
 
@@ -253,6 +263,7 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
   __amdgpu_buffer_rsrc_t rsA0, rsA1;  // A rows (k = 0); DX: second half of the contraction (dup)
   __amdgpu_buffer_rsrc_t rsB0, rsB1;  // B tile origin in the first / second weight stack
   uint32_t voffA[NA];
+  int k_start = 0;
   // source rows of the A tile: the tile's own rows, or token rows through the gather index
   auto load_asrc = [&](const TileMeta& m, int (&asrc)[NA]) {
 #pragma unroll
@@ -278,6 +289,7 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
     const int64_t borg = B_KS ? static_cast<int64_t>(m.n0) : static_cast<int64_t>(m.n0) * ldb;
     rsB0 = make_rsrc(B0 + borg);
     rsB1 = make_rsrc(B1 + borg);
+    k_start = m.k_start;
   };
   // chunk i of the A / B tile of the K step that starts at k0
   auto load_a = [&](int k0, int i) -> u32x4 {
@@ -303,7 +315,11 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
       return __builtin_amdgcn_raw_buffer_load_b128(second ? rsB1 : rsB0, voffB[B_REGULAR ? 0 : i], so, 0);
     }
   };
-  auto kofs = [&](int ks) { return ks * BK; };
+  auto kofs = [&](int ks) {
+    if constexpr (!TURN) return ks * BK;
+    ks += k_start;
+    return (ks < ksteps ? ks : ks - ksteps) * BK;
+  };
   // request every chunk of K step `step` of the fetch tile
   // (chunk after chunk in the order of a K step of the loop below, and kept in that order: the
   // loop's waits count the requests that follow the one they need along every way into the loop,
@@ -968,7 +984,7 @@ constexpr int W_LDS_BYTES = 8 * 64 * 136 * 2;  // 139264: the 8 epilogue regions
 // width: output columns; gate/up tiles hold both halves of their column range.  Tiles are always
 // 256 wide (a 192-wide KS tile would not hold the swizzle: 24 chunks per row are not a multiple
 // of the 16 the key permutes); an overhanging last tile shifts back.
-template <int MODE, bool GATHER = false, bool SAVE_GU = true>
+template <int MODE, bool GATHER = false, bool SAVE_GU = true, bool TURN = false>
 static int launch_row(RowArgs& a, int64_t width, int64_t tile_capacity, hipStream_t s, const char* what) {
   constexpr int div = MODE == RM_GATEUP ? 2 : 1;
   a.n_tiles = (int)((width + 256 / div - 1) / (256 / div));
@@ -992,11 +1008,11 @@ static int launch_row(RowArgs& a, int64_t width, int64_t tile_capacity, hipStrea
   }
   static PerDeviceOnce configured;  // one per kernel instantiation
   if (configured.needed()) {
-    if (int rc = set_lds(row_tiled_kernel<MODE, 4, GATHER, 4, SAVE_GU>, W_LDS_BYTES)) return rc;
+    if (int rc = set_lds(row_tiled_kernel<MODE, 4, GATHER, 4, SAVE_GU, TURN>, W_LDS_BYTES)) return rc;
     configured.done();
   }
   const unsigned blocks = std::min(round8(tile_capacity * a.n_tiles), resident_blocks());
-  hipLaunchKernelGGL((row_tiled_kernel<MODE, 4, GATHER, 4, SAVE_GU>), dim3(blocks), dim3(NT), W_LDS_BYTES, s, a);
+  hipLaunchKernelGGL((row_tiled_kernel<MODE, 4, GATHER, 4, SAVE_GU, TURN>), dim3(blocks), dim3(NT), W_LDS_BYTES, s, a);
   return check_launch(what);
 }
 
@@ -1015,6 +1031,13 @@ int few_rows_fwd(int stage, const void* a, const int32_t* a_src, int64_t a_rows,
 static bool few_rows(int64_t El, int64_t R, int64_t D, int64_t F) {
   return R <= std::max<int64_t>(8 * El, 64) && R * std::max(D, F) * 2 < (int64_t{1} << 32);
 }
+
+// Turned contractions: where weight rows lie a multiple of 4 KiB apart (2048 elements) and most experts have one row
+// tile, so that the product is a read of the weights.  Block forward, 128 experts of 2048 x 768, eight a token, us, as ever / turned:
+// 150 tokens 278 / 243, 300 269 / 248, 600 303 / 263, 1000 279-306 / 271, 2000 340 / 313, 3000 (187 rows) 378 / 365, 4000 (250) 474 / 476,
+// 8192 766 / 779; 64 experts of 2048 x 2048, 700 tokens of six 355 / 329, 4096 x 1024 366 / 336; rows of 1024, 1536 and 7168 elements
+// the same within 1 %.
+static bool turned(int64_t El, int64_t R, int64_t K) { return El > 1 && R <= 200 * El && K * 2 % 4096 == 0; }
 
 int bf16_grouped_fwd(const void* rows, const int32_t* token_of_row, int64_t num_tokens, const void* w1,
                      const void* w3, const void* w2, const int32_t* seg_offsets, const int32_t* seg_counts,
@@ -1042,7 +1065,10 @@ int bf16_grouped_fwd(const void* rows, const int32_t* token_of_row, int64_t num_
     // gate == up == null: a forward-only caller; the kernel then writes h alone
     const bool save = gate != nullptr;
     int rc;
-    if (token_of_row)
+    if (token_of_row && turned(El, row_capacity, D))
+      rc = save ? launch_row<RM_GATEUP, true, true, true>(a, F, tile_capacity, s, "grouped gate/up")
+                : launch_row<RM_GATEUP, true, false, true>(a, F, tile_capacity, s, "grouped gate/up (h only)");
+    else if (token_of_row)
       rc = save ? launch_row<RM_GATEUP, true>(a, F, tile_capacity, s, "grouped gate/up")
                 : launch_row<RM_GATEUP, true, false>(a, F, tile_capacity, s, "grouped gate/up (h only)");
     else
@@ -1054,7 +1080,9 @@ int bf16_grouped_fwd(const void* rows, const int32_t* token_of_row, int64_t num_
     RowArgs b = a;
     b.a_src = nullptr;
     b.a0 = (const uint16_t*)h; b.b0 = (const uint16_t*)w2; b.o0 = (uint16_t*)y;
-    if (int rc = launch_row<RM_DOWN>(b, D, tile_capacity, s, "grouped down")) return rc;
+    if (int rc = turned(El, row_capacity, F) ? launch_row<RM_DOWN, false, true, true>(b, D, tile_capacity, s, "grouped down")
+                      : launch_row<RM_DOWN>(b, D, tile_capacity, s, "grouped down"))
+      return rc;
   }
   return MI355_OK;
 }
