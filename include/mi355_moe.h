@@ -200,6 +200,13 @@ int mi355_router_select_dots_bwd(const float* logits_TE, const int64_t* ids_TK, 
                                  const float* aux_f_E, const float* aux_scale, const uint8_t* padding_mask_T,
                                  float* dlogits_TE, int64_t T, int64_t E, int64_t K, int score_func,
                                  int route_norm, float route_scale, void* stream);
+/* The same with the weights' gradient formed here: dweights[t][k] = <dout[t], y[row_of_slot[t*K+k]]>, the dot products of
+ * mi355_combine_bwd bit for bit.  dout (T,D) and y (row_capacity,D) fp32 or bf16 (dtype), on 16-byte boundaries. */
+int mi355_router_select_rows_bwd(const float* logits_TE, const int64_t* ids_TK, const void* dout, const void* y,
+                                 int dtype, const int32_t* row_of_slot, int64_t row_capacity, int64_t D,
+                                 const float* aux_f_E, const float* aux_scale, const uint8_t* padding_mask_T,
+                                 float* dlogits_TE, int64_t T, int64_t E, int64_t K, int score_func,
+                                 int route_norm, float route_scale, void* stream);
 
 
 /*
@@ -513,6 +520,27 @@ int mi355_grouped_swiglu_combine_bwd(const void* dout, const void* x, const int3
                                      void* dup, void* hs, float* dot_partial, void* drows,
                                      void* dw1, void* dw3, void* dw2, int64_t El, int64_t D,
                                      int64_t F, int64_t row_capacity, int stages, void* stream);
+/*
+ * mi355_permute_rows_fwd + mi355_grouped_swiglu_fwd, and the expert side of mi355_combine_bwd + mi355_grouped_swiglu_bwd, for
+ * fp32 and for bf16 widths off the grid above, with the tokens' rows read where they lie: x and dout are
+ * (num_tokens,D), row r stands for row token_of_row[r], of dout scaled by row_scale[r] and rounded.  The same bits as the
+ * two calls, without the copies in row order.  mi355_grouped_gather_covers: 1 where they serve a case (widths
+ * multiples of four, matrices below 4 GiB and on 16-byte boundaries).  gate, up and h are always written, drows, dw1, dw3, dw2
+ * may be NULL.  At least one row.
+ */
+int mi355_grouped_gather_covers(int dtype, int64_t D, int64_t F, int64_t row_capacity, int64_t num_tokens);
+int mi355_grouped_gather_fwd(const void* x, const int32_t* token_of_row, int64_t num_tokens, const void* w1,
+                             const void* w3, const void* w2, int dtype, const int32_t* seg_offsets,
+                             const int32_t* seg_counts, const int32_t* tile_expert, const int32_t* tile_row0,
+                             const int32_t* num_tiles, int64_t tile_capacity, void* gate, void* up, void* h, void* y,
+                             int64_t El, int64_t D, int64_t F, int64_t row_capacity, void* stream);
+int mi355_grouped_gather_bwd(const void* dout, const void* x, const int32_t* token_of_row, int64_t num_tokens,
+                             const float* row_scale, const void* w1, const void* w3, const void* w2, const void* gate,
+                             const void* up, const void* h, int dtype, const int32_t* seg_offsets,
+                             const int32_t* seg_counts, const int32_t* tile_expert, const int32_t* tile_row0,
+                             const int32_t* num_tiles, int64_t tile_capacity, void* dgate, void* dup, void* drows,
+                             void* dw1, void* dw3, void* dw2, int64_t El, int64_t D, int64_t F, int64_t row_capacity,
+                             void* stream);
 int mi355_combine_row_scale(const float* weights_TK, const int32_t* slot_of_row, float* row_scale,
                             int64_t T, int64_t K, int64_t row_capacity, void* stream);
 /* dweights[t][k] = sum_j dot_partial[row_of_slot[t*K+k]][j], summed in ascending j; 0 for

@@ -7,38 +7,10 @@
 #include <type_traits>
 
 #include "common.h"
+#include "row_vec.h"
 
 namespace mi355 {
 namespace {
-
-template <typename T>
-struct Vec {
-  static constexpr int N = 16 / sizeof(T);
-  __device__ static void unpack(const uint4& v, float (&f)[N]);
-  __device__ static uint4 pack(const float (&f)[N]);
-};
-template <>
-__device__ inline void Vec<float>::unpack(const uint4& v, float (&f)[4]) {
-  f[0] = __uint_as_float(v.x); f[1] = __uint_as_float(v.y);
-  f[2] = __uint_as_float(v.z); f[3] = __uint_as_float(v.w);
-}
-template <>
-__device__ inline uint4 Vec<float>::pack(const float (&f)[4]) {
-  return make_uint4(__float_as_uint(f[0]), __float_as_uint(f[1]), __float_as_uint(f[2]),
-                    __float_as_uint(f[3]));
-}
-template <>
-__device__ inline void Vec<uint16_t>::unpack(const uint4& v, float (&f)[8]) {
-  f[0] = __uint_as_float(v.x << 16); f[1] = __uint_as_float(v.x & 0xffff0000u);
-  f[2] = __uint_as_float(v.y << 16); f[3] = __uint_as_float(v.y & 0xffff0000u);
-  f[4] = __uint_as_float(v.z << 16); f[5] = __uint_as_float(v.z & 0xffff0000u);
-  f[6] = __uint_as_float(v.w << 16); f[7] = __uint_as_float(v.w & 0xffff0000u);
-}
-template <>
-__device__ inline uint4 Vec<uint16_t>::pack(const float (&f)[8]) {
-  return make_uint4(pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]), pack_bf16x2(f[4], f[5]),
-                    pack_bf16x2(f[6], f[7]));
-}
 
 template <typename T>
 __device__ __forceinline__ float round_to(float v);

@@ -193,7 +193,7 @@ extern "C" int mi355_grouped_swiglu_fwd(const void* rows, const int32_t* token_o
                               "materialise the rows with mi355_permute_rows_fwd instead");
   if (any_path_ok(dtype, D, F, row_capacity, {rows, w1, w3, w2, gate, up, h, y})) {
     const AnySeg g{seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity, El};
-    if (int rc = any_gateup(g, dtype, rows, w1, w3, gate, up, h, D, F, row_capacity, s)) return rc;
+    if (int rc = any_gateup(g, dtype, rows, w1, w3, gate, up, h, D, F, row_capacity, nullptr, s)) return rc;
     return any_linear(g, dtype, h, w2, y, F, D, row_capacity, s);
   }
   const Seg sg{seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity};
@@ -245,14 +245,14 @@ extern "C" int mi355_grouped_swiglu_bwd(const void* dy, const void* rows,
     const AnySeg g{seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity, El};
     const bool some = row_capacity > 0 && tile_capacity > 0;
     if (some)
-      if (int rc = any_dh(g, dtype, dy, w2, gate, up, dgate, dup, D, F, row_capacity, s)) return rc;
+      if (int rc = any_dh(g, dtype, dy, w2, gate, up, dgate, dup, D, F, row_capacity, nullptr, s)) return rc;
     // the weight gradients also cover the no-rows case: every expert's gradient is written (zeros)
     AnyGrad grads[3];
     int count = 0;
-    if (dw2) grads[count++] = {dy, h, dw2, D, F};
-    if (dw1) grads[count++] = {dgate, rows, dw1, F, D};
-    if (dw3) grads[count++] = {dup, rows, dw3, F, D};
-    return any_backward(g, dtype, dgate, dup, w1, w3, some ? drows : nullptr, D, F, grads, count, row_capacity, s);
+    if (dw2) grads[count++] = {dy, h, dw2, D, F, 0};
+    if (dw1) grads[count++] = {dgate, rows, dw1, F, D, 0};
+    if (dw3) grads[count++] = {dup, rows, dw3, F, D, 0};
+    return any_backward(g, dtype, dgate, dup, w1, w3, some ? drows : nullptr, D, F, grads, count, row_capacity, nullptr, s);
   }
   const Seg sg{seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity};
   if (row_capacity > 0 && tile_capacity > 0) {
@@ -356,8 +356,8 @@ extern "C" int mi355_grouped_linear_bwd(const void* dy, const void* x, const voi
     const AnySeg g{seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity, El};
     if (dx && rows)
       if (int rc = any_linear_dx(g, dtype, dy, w, dx, I, O, row_capacity, s)) return rc;
-    const AnyGrad grad{dy, x, dw, O, I};
-    return any_backward(g, dtype, nullptr, nullptr, nullptr, nullptr, nullptr, I, O, &grad, dw ? 1 : 0, row_capacity, s);
+    const AnyGrad grad{dy, x, dw, O, I, 0};
+    return any_backward(g, dtype, nullptr, nullptr, nullptr, nullptr, nullptr, I, O, &grad, dw ? 1 : 0, row_capacity, nullptr, s);
   }
   // dx = dy . w[e]: B(k=o, n=i) = w[e][o][i]
   if (dx && rows)
@@ -398,4 +398,55 @@ extern "C" int mi355_grouped_swiglu_combine_bwd(
   return bf16_grouped_bwd(dout, x, token_of_row, num_tokens, w1, w3, w2, gate, up, hs, row_scale, dot_partial,
                           seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity, dgate, dup,
                           drows, dw1, dw3, dw2, El, D, F, stages ? stages : 0x7c, as_stream(stream));
+}
+
+// ---- experts of any width, the tokens' rows read in place ------------------------------------------
+static bool gather_ok(int dtype, int64_t D, int64_t F, int64_t R, int64_t T, std::initializer_list<const void*> matrices) {
+  return !(dtype == MI355_BF16 && bf16_fast_path_ok(D, F)) && T >= 1 && T < (1ll << 31) &&
+         any_path_ok(dtype, D, F, std::max(R, T), matrices);
+}
+
+extern "C" int mi355_grouped_gather_covers(int dtype, int64_t D, int64_t F, int64_t row_capacity, int64_t num_tokens) {
+  return D >= 1 && F >= 1 && row_capacity >= 1 && gather_ok(dtype, D, F, row_capacity, num_tokens, {}) ? 1 : 0;
+}
+
+extern "C" int mi355_grouped_gather_fwd(const void* x, const int32_t* token_of_row, int64_t num_tokens, const void* w1,
+                                        const void* w3, const void* w2, int dtype, const int32_t* seg_offsets,
+                                        const int32_t* seg_counts, const int32_t* tile_expert, const int32_t* tile_row0,
+                                        const int32_t* num_tiles, int64_t tile_capacity, void* gate, void* up, void* h,
+                                        void* y, int64_t El, int64_t D, int64_t F, int64_t row_capacity, void* stream) {
+  if (int rc = check_common("grouped_gather_fwd", dtype, El, D, F, row_capacity, tile_capacity)) return rc;
+  MI355_REQUIRE(row_capacity >= 1 && tile_capacity >= 1 && x && token_of_row && w1 && w3 && w2 && seg_offsets && seg_counts &&
+                    tile_expert && tile_row0 && num_tiles && gate && up && h && y,
+                "grouped_gather_fwd: null pointer");
+  if (!gather_ok(dtype, D, F, row_capacity, num_tokens, {x, w1, w3, w2, gate, up, h, y}))
+    return fail(MI355_EUNSUP, "grouped_gather_fwd: not covered; use mi355_permute_rows_fwd and mi355_grouped_swiglu_fwd");
+  const AnySeg g{seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity, El};
+  const AnyFold fold{token_of_row, num_tokens, nullptr};
+  if (int rc = any_gateup(g, dtype, x, w1, w3, gate, up, h, D, F, row_capacity, &fold, as_stream(stream))) return rc;
+  return any_linear(g, dtype, h, w2, y, F, D, row_capacity, as_stream(stream));
+}
+
+extern "C" int mi355_grouped_gather_bwd(const void* dout, const void* x, const int32_t* token_of_row, int64_t num_tokens,
+                                        const float* row_scale, const void* w1, const void* w3, const void* w2,
+                                        const void* gate, const void* up, const void* h, int dtype,
+                                        const int32_t* seg_offsets, const int32_t* seg_counts, const int32_t* tile_expert,
+                                        const int32_t* tile_row0, const int32_t* num_tiles, int64_t tile_capacity,
+                                        void* dgate, void* dup, void* drows, void* dw1, void* dw3, void* dw2, int64_t El,
+                                        int64_t D, int64_t F, int64_t row_capacity, void* stream) {
+  if (int rc = check_common("grouped_gather_bwd", dtype, El, D, F, row_capacity, tile_capacity)) return rc;
+  MI355_REQUIRE(row_capacity >= 1 && tile_capacity >= 1 && dout && x && token_of_row && row_scale && w1 && w3 && w2 && gate &&
+                    up && h && seg_offsets && seg_counts && tile_expert && tile_row0 && num_tiles && dgate && dup,
+                "grouped_gather_bwd: null pointer");
+  if (!gather_ok(dtype, D, F, row_capacity, num_tokens, {dout, x, w1, w3, w2, gate, up, h, dgate, dup, drows, dw1, dw3, dw2}))
+    return fail(MI355_EUNSUP, "grouped_gather_bwd: not covered; use mi355_combine_bwd and mi355_grouped_swiglu_bwd");
+  const AnySeg g{seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity, El};
+  const AnyFold fold{token_of_row, num_tokens, row_scale};
+  if (int rc = any_dh(g, dtype, dout, w2, gate, up, dgate, dup, D, F, row_capacity, &fold, as_stream(stream))) return rc;
+  AnyGrad grads[3];
+  int count = 0;
+  if (dw2) grads[count++] = {dout, h, dw2, D, F, 1};
+  if (dw1) grads[count++] = {dgate, x, dw1, F, D, 2};
+  if (dw3) grads[count++] = {dup, x, dw3, F, D, 2};
+  return any_backward(g, dtype, dgate, dup, w1, w3, drows, D, F, grads, count, row_capacity, &fold, as_stream(stream));
 }

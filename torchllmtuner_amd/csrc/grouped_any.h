@@ -8,24 +8,32 @@ struct AnySeg {
   const int32_t *seg_offsets, *seg_counts, *tile_expert, *tile_row0, *num_tiles;
   int64_t tile_capacity, El;
 };
+// The tokens' rows in place of copies in row order: row r of x (rows) or, scaled by row_scale[r], of the output gradient (dy) is
+// row token_of_row[r] of a matrix of `tokens` rows.
+struct AnyFold {
+  const int32_t* token_of_row;
+  int64_t tokens;
+  const float* row_scale;  // (backward)
+};
 struct AnyGrad {  // c (El, M, N) = per segment a^T (rows, M) . b (rows, N)
   const void *a, *b;
   void* c;
   int64_t M, N;
+  int through;  // with a fold: 1 a is the output gradient's, 2 b is the tokens'
 };
 
 bool any_path_ok(int dtype, int64_t D, int64_t F, int64_t R, std::initializer_list<const void*> matrices);
 int any_gateup(const AnySeg& g, int dtype, const void* rows, const void* w1, const void* w3, void* gate, void* up, void* h,
-               int64_t D, int64_t F, int64_t R, hipStream_t s);
+               int64_t D, int64_t F, int64_t R, const AnyFold* fold, hipStream_t s);
 // y (R, O) = x (R, I) . w (El, O, I)^T, and its input gradient
 int any_linear(const AnySeg& g, int dtype, const void* x, const void* w, void* y, int64_t I, int64_t O, int64_t R,
                hipStream_t s);
 int any_linear_dx(const AnySeg& g, int dtype, const void* dy, const void* w, void* dx, int64_t I, int64_t O, int64_t R,
                   hipStream_t s);
 int any_dh(const AnySeg& g, int dtype, const void* dy, const void* w2, const void* gate, const void* up, void* dgate,
-           void* dup, int64_t D, int64_t F, int64_t R, hipStream_t s);
+           void* dup, int64_t D, int64_t F, int64_t R, const AnyFold* fold, hipStream_t s);
 // drows (null: not wanted) = dgate . w1 + dup . w3, and at most three weight gradients
 int any_backward(const AnySeg& g, int dtype, const void* dgate, const void* dup, const void* w1, const void* w3, void* drows,
-                 int64_t D, int64_t F, const AnyGrad* grads, int count, int64_t R, hipStream_t s);
+                 int64_t D, int64_t F, const AnyGrad* grads, int count, int64_t R, const AnyFold* fold, hipStream_t s);
 
 }  // namespace mi355

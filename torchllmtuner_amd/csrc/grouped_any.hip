@@ -36,6 +36,7 @@ struct AnyDw {  // c[e] (M, N) = a[segment e]^T (rows, M) . b[segment e] (rows, 
   const void *a, *b;
   void* c;
   int M, N, nt, first;  // column tiles; first block of the problem
+  int through;          // FOLD: 1 a's rows through the row index, scaled; 2 b's rows through it
 };
 
 struct AnyArgs {
@@ -48,6 +49,11 @@ struct AnyArgs {
   int col_tiles;
   AnyDw dw[3];
   int num_dw;
+  // FOLD: row r of the tokens' matrix (GATEUP a0, DH a0, a weight gradient's a or b) is its row src[r] of src_rows, of the
+  // output gradient scaled by scale[r] (and rounded, as a copy of it would be)
+  const int32_t* src;
+  int src_rows;
+  const float* scale;
 };
 
 template <typename T> struct El;
@@ -142,6 +148,20 @@ __device__ __forceinline__ f32x16 any_mfma(const f32x4& b, const f32x4& a, f32x1
   return acc;
 }
 
+// a chunk of a row, scaled and rounded
+__device__ __forceinline__ u32x4 any_scale(float, const u32x4& v, float f) {
+  u32x4 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = __float_as_uint(__uint_as_float(v[i]) * f);
+  return r;
+}
+__device__ __forceinline__ u32x4 any_scale(uint16_t, const u32x4& v, float f) {
+  u32x4 r;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) r[i] = pack2(__uint_as_float(v[i] << 16) * f, __uint_as_float(v[i] & 0xffff0000u) * f);
+  return r;
+}
+
 // LDS of one instantiation: two stages; on 32-row tiles also the four waves' partial tiles
 template <typename T, int MODE, int TM, int TN>
 constexpr int any_lds() {
@@ -151,7 +171,12 @@ constexpr int any_lds() {
   return stages > parts ? stages : parts;
 }
 
-template <typename T, int MODE, int TM, int TN>
+// FOLD: the tokens' rows are read through the plan's row index, and the output gradient's are scaled by the routing weight,
+// where they are fetched: no copy of either in row order exists.  A weight gradient's contraction runs over the rows, so
+// its indexes are requested as many steps before their rows as those are before their use.  What it saves is two launches and
+// two passes over row-ordered copies; a training step of the block, us, copied / in place: 512 fp32 tokens of 8 x 256 x 512 132 / 126, 1531
+// bf16 of 16 x 320 x 232 136 / 128, 4096 of 32 x 480 x 432 (four each) 358 / 324, 4096 fp32 of 16 x 640 x 1024 1999 / 1989.
+template <typename T, int MODE, int TM, int TN, bool FOLD>
 __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
   constexpr bool A_KS = MODE == ANY_DW, B_KS = MODE == ANY_DH || MODE == ANY_DX || MODE == ANY_KS || MODE == ANY_DW;
   using OA = Operand<T, A_KS, TM>;
@@ -173,6 +198,9 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
   T *C0 = static_cast<T*>(p.c0);
   int lda = p.K, ldb = p.ldb;
   int64_t a_bytes, b_bytes;
+  constexpr bool ROWS_FOLD = FOLD && (MODE == ANY_GATEUP || MODE == ANY_DH), K_FOLD = FOLD && MODE == ANY_DW;
+  bool through_a = false, through_b = false;  // K_FOLD
+  int64_t first_row = 0;
   if constexpr (MODE == ANY_DW) {
     int d = 0;
     while (d + 1 < p.num_dw && block >= p.dw[d + 1].first) ++d;
@@ -192,6 +220,19 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
     a_bytes = ((p.rows - first) * M - m0) * static_cast<int64_t>(sizeof(T));
     b_bytes = ((p.rows - first) * N - n0) * static_cast<int64_t>(sizeof(T));
     C0 = static_cast<T*>(w.c) + static_cast<int64_t>(e) * M * N;
+    if constexpr (K_FOLD) {
+      first_row = first;
+      through_a = w.through == 1;
+      through_b = w.through == 2;
+      if (through_a) {
+        A0 = static_cast<const T*>(w.a) + m0;
+        a_bytes = (static_cast<int64_t>(p.src_rows) * M - m0) * static_cast<int64_t>(sizeof(T));
+      }
+      if (through_b) {
+        B0 = static_cast<const T*>(w.b) + n0;
+        b_bytes = (static_cast<int64_t>(p.src_rows) * N - n0) * static_cast<int64_t>(sizeof(T));
+      }
+    }
   } else {
     constexpr int SUBS = 256 / TM;
     const int slot = block / p.col_tiles, tile = slot / SUBS;
@@ -203,8 +244,8 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
     if (m_valid <= 0) return;
     row0 = first;
     n0 = (block % p.col_tiles) * (MODE == ANY_GATEUP ? TN / 2 : TN);
-    A0 = static_cast<const T*>(p.a0) + row0 * lda;
-    a_bytes = (p.rows - row0) * lda * static_cast<int64_t>(sizeof(T));
+    A0 = static_cast<const T*>(p.a0) + (ROWS_FOLD ? 0 : row0 * lda);
+    a_bytes = (ROWS_FOLD ? p.src_rows : p.rows - row0) * lda * static_cast<int64_t>(sizeof(T));
     if (MODE == ANY_DX) A1 = static_cast<const T*>(p.a1) + row0 * lda;
     const int64_t w = e * p.w_elems + (B_KS ? n0 : static_cast<int64_t>(n0) * ldb);
     B0 = static_cast<const T*>(p.b0) + w;
@@ -213,10 +254,18 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
   }
   // ---- operand offsets (bytes): fixed per lane, plus the step's
   uint32_t offA[OA::N], offB[OB::N];
+  float row_scale[MODE == ANY_DH && FOLD ? OA::N : 1];
+  auto source = [&](int64_t row) { return static_cast<uint32_t>(min(max(p.src[row], 0), p.src_rows - 1)); };
 #pragma unroll
   for (int i = 0; i < OA::N; ++i) {
     const int q = tid + 256 * i, r = q / OA::CPR, c = (q % OA::CPR) * OA::E;
-    offA[i] = (A_KS ? static_cast<uint32_t>(r) * lda + c : static_cast<uint32_t>(min(r, m_valid - 1)) * lda + c) * sizeof(T);
+    if constexpr (ROWS_FOLD) {
+      const int64_t row = row0 + min(r, m_valid - 1);
+      offA[i] = (source(row) * lda + c) * sizeof(T);
+      if constexpr (MODE == ANY_DH) row_scale[i] = p.scale[row];
+    } else {
+      offA[i] = (A_KS ? static_cast<uint32_t>(r) * lda + c : static_cast<uint32_t>(min(r, m_valid - 1)) * lda + c) * sizeof(T);
+    }
   }
   const int b_rows = (MODE == ANY_GATEUP ? TN / 2 : TN);  // KC: weight rows of the tile (of each of the two)
 #pragma unroll
@@ -230,6 +279,22 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
   const auto rsA0 = any_rsrc(A0, a_bytes), rsB0 = any_rsrc(B0, b_bytes);
   const auto rsA1 = MODE == ANY_DX ? any_rsrc(A1, a_bytes) : rsA0;
   const auto rsB1 = (MODE == ANY_GATEUP || MODE == ANY_DX) ? any_rsrc(B1, b_bytes) : rsB0;
+  // K_FOLD: source rows of the steps ahead; scales of the steps held
+  uint32_t srcA[K_FOLD ? AHEAD : 1][K_FOLD ? OA::N : 1], srcB[K_FOLD ? AHEAD : 1][K_FOLD ? OB::N : 1];
+  float k_scale[K_FOLD ? AHEAD : 1][K_FOLD ? OA::N : 1];
+  auto row_of = [&](int s, int chunk_row) -> int64_t { return first_row + min(s * BKE + chunk_row, K - 1); };
+  auto request_sources = [&](int slot, int s) {
+    if constexpr (K_FOLD) {
+      if (through_a) {
+#pragma unroll
+        for (int i = 0; i < OA::N; ++i) srcA[slot][i] = p.src[row_of(s, (tid + 256 * i) / OA::CPR)];
+      }
+      if (through_b) {
+#pragma unroll
+        for (int i = 0; i < OB::N; ++i) srcB[slot][i] = p.src[row_of(s, (tid + 256 * i) / OB::CPR)];
+      }
+    }
+  };
   auto fetch = [&](int slot, int s) {
     const bool second = MODE == ANY_DX && s >= half_steps;
     const uint32_t k = static_cast<uint32_t>(second ? s - half_steps : s) * BKE;
@@ -243,16 +308,40 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
       rsB = any_rsrc(second ? B1 : B0, bn);
       rsU = MODE == ANY_GATEUP ? any_rsrc(B1, bn) : rsB;
     }
+    // (a source row is clamped where it is used, not where it is requested: that would wait for it)
+    auto within = [&](uint32_t row) { return static_cast<uint32_t>(min(max(static_cast<int>(row), 0), p.src_rows - 1)); };
 #pragma unroll
-    for (int i = 0; i < OA::N; ++i) ra[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(rsA, offA[i] + ka, 0, 0);
+    for (int i = 0; i < OA::N; ++i) {
+      uint32_t at = offA[i] + ka;
+      if constexpr (K_FOLD)
+        if (through_a) at = (within(srcA[slot][i]) * lda + ((tid + 256 * i) % OA::CPR) * OA::E) * sizeof(T);
+      ra[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(rsA, at, 0, 0);
+      if constexpr (K_FOLD)
+        if (through_a) k_scale[slot][i] = p.scale[row_of(s, (tid + 256 * i) / OA::CPR)];
+    }
 #pragma unroll
-    for (int i = 0; i < OB::N; ++i)
-      rb[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(i >= OB::N / 2 ? rsU : rsB, offB[i] + kb, 0, 0);
+    for (int i = 0; i < OB::N; ++i) {
+      uint32_t at = offB[i] + kb;
+      if constexpr (K_FOLD)
+        if (through_b) at = (within(srcB[slot][i]) * ldb + ((tid + 256 * i) % OB::CPR) * OB::E) * sizeof(T);
+      rb[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(i >= OB::N / 2 ? rsU : rsB, at, 0, 0);
+    }
+    request_sources(slot, s + AHEAD);
   };
   auto park = [&](int slot, int s) {
     T* As = smem + (s & 1) * STAGE;
     T* Bs = As + OA::ELEMS;
     const int kv = K - (MODE == ANY_DX && s >= half_steps ? s - half_steps : s) * BKE;
+    if constexpr (FOLD && MODE == ANY_DH) {
+#pragma unroll
+      for (int i = 0; i < OA::N; ++i) ra[slot][i] = any_scale(T{}, ra[slot][i], row_scale[i]);
+    }
+    if constexpr (K_FOLD) {
+      if (through_a) {
+#pragma unroll
+        for (int i = 0; i < OA::N; ++i) ra[slot][i] = any_scale(T{}, ra[slot][i], k_scale[slot][i]);
+      }
+    }
     if (kv < BKE) {  // the tail: whatever was read past the contraction must not meet anything
 #pragma unroll
       for (int i = 0; i < OA::N; ++i) ra[slot][i] = OA::clip(ra[slot][i], tid, i, kv);
@@ -291,6 +380,7 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
   };
   if constexpr (!KSPLIT) {
     if (steps > 0) {
+      request_sources(0, 0);
       fetch(0, 0);
       park(0, 0);
       if (steps > 1) fetch(0, 1);
@@ -306,6 +396,8 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
     }
   } else {
     if (steps > 0) {
+#pragma unroll
+      for (int i = 0; i < AHEAD; ++i) request_sources(i, i);
 #pragma unroll
       for (int i = 0; i < AHEAD; ++i) fetch(i, i);
       park(0, 0);
@@ -391,33 +483,39 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
   }
 }
 
-template <typename T, int MODE, int TM, int TN>
+template <typename T, int MODE, int TM, int TN, bool FOLD>
 __global__ __launch_bounds__(256) void any_kernel(AnyArgs p) {
   __shared__ __attribute__((aligned(16))) T smem[any_lds<T, MODE, TM, TN>()];
-  any_tile<T, MODE, TM, TN>(p, blockIdx.x, smem);
+  any_tile<T, MODE, TM, TN, FOLD>(p, blockIdx.x, smem);
 }
 
 // The input gradient and the weight gradients of a backward pass read the same buffers and write different
 // ones: with few tiles each they share a launch (at 512 fp32 tokens of 8 experts 26 + 16 us one after the
 // other).  The longer contraction starts first.
-template <typename T, int TX, int TW>
+template <typename T, int TX, int TW, bool FOLD>
 __global__ __launch_bounds__(256) void any_dx_dw_kernel(AnyArgs dx, AnyArgs dw, int dx_blocks, int dw_blocks, int dw_first) {
   constexpr int A = any_lds<T, ANY_DX, TX, TX>(), B = any_lds<T, ANY_DW, TW, TW>();
   __shared__ __attribute__((aligned(16))) T smem[A > B ? A : B];
   const int block = static_cast<int>(blockIdx.x) - (dw_first ? dw_blocks : 0);  // of dx
-  if (block >= 0 && block < dx_blocks) any_tile<T, ANY_DX, TX, TX>(dx, block, smem);
-  else any_tile<T, ANY_DW, TW, TW>(dw, dw_first ? blockIdx.x : block - dx_blocks, smem);
+  if (block >= 0 && block < dx_blocks) any_tile<T, ANY_DX, TX, TX, false>(dx, block, smem);
+  else any_tile<T, ANY_DW, TW, TW, FOLD>(dw, dw_first ? blockIdx.x : block - dx_blocks, smem);
 }
 
 template <int MODE, int TM, int TN>
 int launch_any(const AnyArgs& p, int dtype, int64_t blocks, hipStream_t s, const char* what) {
   if (blocks <= 0) return MI355_OK;
-  if (dtype == MI355_F32) {
-    hipLaunchKernelGGL((any_kernel<float, MODE, TM, TN>), dim3((unsigned)blocks), dim3(256), 0, s, p);
-  } else if constexpr (TM != 32) {
-    hipLaunchKernelGGL((any_kernel<uint16_t, MODE, TM, TN>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+  if (dtype != MI355_F32 && TM == 32) return fail(MI355_EUNSUP, "%s: 32-row tiles are for fp32", what);
+  auto run = [&](auto fold) {
+    constexpr bool FOLD = decltype(fold)::value;
+    const dim3 grid((unsigned)blocks), lanes(256);
+    if (dtype == MI355_F32) hipLaunchKernelGGL((any_kernel<float, MODE, TM, TN, FOLD>), grid, lanes, 0, s, p);
+    else if constexpr (TM != 32) hipLaunchKernelGGL((any_kernel<uint16_t, MODE, TM, TN, FOLD>), grid, lanes, 0, s, p);
+  };
+  if constexpr (MODE == ANY_GATEUP || MODE == ANY_DH || MODE == ANY_DW) {
+    if (p.src) run(std::true_type{});
+    else run(std::false_type{});
   } else {
-    return fail(MI355_EUNSUP, "%s: 32-row tiles are for fp32", what);
+    run(std::false_type{});
   }
   return check_launch(what);
 }
@@ -469,8 +567,11 @@ bool any_path_ok(int dtype, int64_t D, int64_t F, int64_t R, std::initializer_li
          std::max(R * std::max(D, F), D * F) * (dtype == MI355_F32 ? 4 : 2) < (int64_t{1} << 32) - 4;
 }
 
-static AnyArgs any_args(const AnySeg& g, int64_t rows) {
+static AnyArgs any_args(const AnySeg& g, int64_t rows, const AnyFold* f = nullptr) {
   AnyArgs p{};
+  if (f) {
+    p.src = f->token_of_row; p.src_rows = (int)f->tokens; p.scale = f->row_scale;
+  }
   p.rows = rows;
   p.seg_offsets = g.seg_offsets; p.seg_counts = g.seg_counts; p.tile_expert = g.tile_expert;
   p.tile_row0 = g.tile_row0; p.num_tiles = g.num_tiles;
@@ -478,8 +579,8 @@ static AnyArgs any_args(const AnySeg& g, int64_t rows) {
 }
 
 int any_gateup(const AnySeg& g, int dtype, const void* rows, const void* w1, const void* w3, void* gate, void* up, void* h,
-               int64_t D, int64_t F, int64_t R, hipStream_t s) {
-  AnyArgs p = any_args(g, R);
+               int64_t D, int64_t F, int64_t R, const AnyFold* f, hipStream_t s) {
+  AnyArgs p = any_args(g, R, f);
   p.a0 = rows; p.b0 = w1; p.b1 = w3; p.c0 = gate; p.c1 = up; p.c2 = h;
   p.K = (int)D; p.N = (int)F; p.ldb = (int)D; p.w_elems = D * F;
   return launch_rows<ANY_GATEUP>(p, dtype, g.tile_capacity, g.El, F, s, "grouped gate/up");
@@ -502,20 +603,21 @@ int any_linear_dx(const AnySeg& g, int dtype, const void* dy, const void* w, voi
 }
 
 int any_dh(const AnySeg& g, int dtype, const void* dy, const void* w2, const void* gate, const void* up, void* dgate,
-           void* dup, int64_t D, int64_t F, int64_t R, hipStream_t s) {
-  AnyArgs p = any_args(g, R);
+           void* dup, int64_t D, int64_t F, int64_t R, const AnyFold* f, hipStream_t s) {
+  AnyArgs p = any_args(g, R, f);
   p.a0 = dy; p.b0 = w2; p.c0 = dgate; p.c1 = dup; p.gate = gate; p.up = up;
   p.K = (int)D; p.N = (int)F; p.ldb = (int)F; p.w_elems = D * F;
   return launch_rows<ANY_DH>(p, dtype, g.tile_capacity, g.El, F, s, "grouped dh");
 }
 
 int any_backward(const AnySeg& g, int dtype, const void* dgate, const void* dup, const void* w1, const void* w3, void* drows,
-                 int64_t D, int64_t F, const AnyGrad* grads, int count, int64_t R, hipStream_t s) {
+                 int64_t D, int64_t F, const AnyGrad* grads, int count, int64_t R, const AnyFold* f, hipStream_t s) {
   AnyArgs p = any_args(g, R);
   p.a0 = dgate; p.a1 = dup; p.b0 = w1; p.b1 = w3; p.c0 = drows;
   p.K = (int)F; p.N = (int)D; p.ldb = (int)D; p.w_elems = D * F;
-  AnyArgs w = any_args(g, R);
-  for (int i = 0; i < count; ++i) w.dw[i] = {grads[i].a, grads[i].b, grads[i].c, (int)grads[i].M, (int)grads[i].N, 0, 0};
+  AnyArgs w = any_args(g, R, f);
+  for (int i = 0; i < count; ++i)
+    w.dw[i] = {grads[i].a, grads[i].b, grads[i].c, (int)grads[i].M, (int)grads[i].N, 0, 0, grads[i].through};
   w.num_dw = count;
   const bool dw_large = count && dw_tiles(w, g.El, 128) >= 512;
   int64_t tiles = count ? dw_tiles(w, g.El, dw_large ? 128 : 64) : 0;
@@ -532,9 +634,14 @@ int any_backward(const AnySeg& g, int dtype, const void* dgate, const void* dup,
     auto run = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, p, w, (int)dx_blocks, (int)tiles, dw_first);
     };
-    if (dtype == MI355_BF16) run(any_dx_dw_kernel<uint16_t, 64, 64>);
-    else if (dw_small) run(t == 64 ? any_dx_dw_kernel<float, 64, 32> : any_dx_dw_kernel<float, 32, 32>);
-    else run(t == 64 ? any_dx_dw_kernel<float, 64, 64> : any_dx_dw_kernel<float, 32, 64>);
+    auto choose = [&](auto fold) {
+      constexpr bool FOLD = decltype(fold)::value;
+      if (dtype == MI355_BF16) run(any_dx_dw_kernel<uint16_t, 64, 64, FOLD>);
+      else if (dw_small) run(t == 64 ? any_dx_dw_kernel<float, 64, 32, FOLD> : any_dx_dw_kernel<float, 32, 32, FOLD>);
+      else run(t == 64 ? any_dx_dw_kernel<float, 64, 64, FOLD> : any_dx_dw_kernel<float, 32, 64, FOLD>);
+    };
+    if (f) choose(std::true_type{});
+    else choose(std::false_type{});
     return check_launch("grouped drows and weight gradients");
   }
   if (drows)

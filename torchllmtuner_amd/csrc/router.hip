@@ -6,9 +6,11 @@
 // sum and every arg-max are DPP reductions, and the K winners are written by lanes 0..K-1.  No
 // LDS, no atomics; HBM traffic is the (T,E) logits once plus the (T,K) outputs.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "gemm_generic.h"
+#include "row_vec.h"
 #include "select_rows.h"
 
 namespace mi355 {
@@ -319,6 +321,14 @@ __device__ __forceinline__ float slot_dweight(const DotPieces& d, const float* d
   return sum;
 }
 
+// ... or as nothing has left it yet: the output gradient and the experts' rows, whose dot products the wave of the token
+// forms itself (T of the kernel below; void: no such rows).
+struct DotRows {
+  const void *dout, *y;
+  const int32_t* row_of_slot;
+  int D, rows;
+};
+
 // The load-balance loss's part of the score gradient (aux.hip's formula), for the tokens that are not padding.
 struct BalanceGrad {
   const float* f;  // (E) or null: no loss
@@ -326,17 +336,17 @@ struct BalanceGrad {
   const uint8_t* padding;
 };
 
-template <int VPL>
+template <int VPL, typename T = void>
 __global__ __launch_bounds__(256) void select_bwd_kernel(
     const float* __restrict__ logits, const int64_t* __restrict__ ids,
-    const float* __restrict__ dweights, const float* __restrict__ dscores, DotPieces dots, BalanceGrad bal,
-    float* __restrict__ dlogits, int T, int E, int K, int score_func, int route_norm,
+    const float* __restrict__ dweights, const float* __restrict__ dscores, DotPieces dots, DotRows rows, BalanceGrad bal,
+    float* __restrict__ dlogits, int T_, int E, int K, int score_func, int route_norm,
     float route_scale, int mode) {
   extern __shared__ float lds[];  // per wave: sc[E], ds[E]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int t_raw = blockIdx.x * 4 + wave;
-  const bool active = t_raw < T;
-  const int t = active ? t_raw : T - 1;  // inactive waves shadow the last token, store nothing
+  const bool active = t_raw < T_;
+  const int t = active ? t_raw : T_ - 1;  // inactive waves shadow the last token, store nothing
   float* sc = lds + static_cast<size_t>(wave) * 2 * E;
   float* ds = sc + E;
 
@@ -372,12 +382,20 @@ __global__ __launch_bounds__(256) void select_bwd_kernel(
   }
   __syncthreads();
 
-  if (mode != MI355_SELECT_FIXED && (dweights || dots.partial)) {
+  constexpr bool kRows = !std::is_void_v<T>;
+  if (mode != MI355_SELECT_FIXED && (kRows || dweights || dots.partial)) {
     // lanes 0..K-1 own one selected expert each (K <= 64)
     int id = lane < K ? static_cast<int>(ids[static_cast<int64_t>(t) * K + lane]) : 0;
     id = min(max(id, 0), E - 1);
     const float sk = lane < K ? sc[id] : 0.0f;
-    const float dw = lane < K ? slot_dweight(dots, dweights, static_cast<int64_t>(t) * K + lane) : 0.0f;
+    float dw;
+    if constexpr (kRows) {
+      const int row = lane < K ? rows.row_of_slot[static_cast<int64_t>(t) * K + lane] : -1;
+      dw = row_dots<T>(static_cast<const T*>(rows.dout) + static_cast<int64_t>(t) * rows.D, static_cast<const T*>(rows.y),
+                       row < rows.rows ? row : -1, K, rows.D);
+    } else {
+      dw = lane < K ? slot_dweight(dots, dweights, static_cast<int64_t>(t) * K + lane) : 0.0f;
+    }
     float g;
     if (route_norm) {
       const float denom = wave_sum_dpp(sk) + 1e-20f;
@@ -641,7 +659,7 @@ static int select_bwd(const float* logits, const int64_t* ids, const float* dwei
   const dim3 grid((unsigned)((T + 3) / 4));
   const size_t lds = (size_t)4 * 2 * E * sizeof(float);
   DISPATCH_VPL(E, hipLaunchKernelGGL(select_bwd_kernel<VPL>, grid, dim3(256), lds, as_stream(stream),
-                                     logits, ids, dweights, dscores_TE, dots, bal, dlogits, (int)T, (int)E,
+                                     logits, ids, dweights, dscores_TE, dots, DotRows{}, bal, dlogits, (int)T, (int)E,
                                      (int)K, score_func, route_norm, route_scale, select_mode));
   return check_launch("router_select_bwd");
 }
@@ -668,4 +686,31 @@ extern "C" int mi355_router_select_dots_bwd(const float* logits, const int64_t* 
                     pieces ? DotPieces{dots, row_of_slot, (int)pieces, (int)row_capacity} : DotPieces{},
                     BalanceGrad{aux_f_E, aux_scale, padding_mask_T}, dlogits, T, E, K, score_func, route_norm, route_scale,
                     MI355_SELECT_TOPK, stream);
+}
+
+extern "C" int mi355_router_select_rows_bwd(const float* logits, const int64_t* ids, const void* dout, const void* y, int dtype,
+                                            const int32_t* row_of_slot, int64_t row_capacity, int64_t D, const float* aux_f_E,
+                                            const float* aux_scale, const uint8_t* padding_mask_T, float* dlogits, int64_t T,
+                                            int64_t E, int64_t K, int score_func, int route_norm, float route_scale,
+                                            void* stream) {
+  if (int rc = check_router_args(T, E, K)) return rc;
+  MI355_REQUIRE(K <= 64, "router_select_rows_bwd: top_k > 64 unsupported");
+  MI355_REQUIRE(dtype == MI355_F32 || dtype == MI355_BF16, "router_select_rows_bwd: fp32 or bf16 rows");
+  MI355_REQUIRE(row_capacity >= 0 && row_capacity < (1ll << 31) && D >= 1 && D < (1ll << 31),
+                "router_select_rows_bwd: bad shape");
+  if (T == 0) return MI355_OK;
+  MI355_REQUIRE(logits && ids && dlogits && dout && y && row_of_slot && aligned16({dout, y}),
+                "router_select_rows_bwd: null or misaligned pointer");
+  MI355_REQUIRE(!aux_f_E || aux_scale, "router_select_rows_bwd: the loss needs its scale");
+  const DotRows rows{dout, y, row_of_slot, (int)D, (int)row_capacity};
+  const BalanceGrad bal{aux_f_E, aux_scale, padding_mask_T};
+  const dim3 grid((unsigned)((T + 3) / 4));
+  const size_t lds = (size_t)4 * 2 * E * sizeof(float);
+  auto launch = [&](auto* kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), lds, as_stream(stream), logits, ids, nullptr, nullptr, DotPieces{}, rows, bal,
+                       dlogits, (int)T, (int)E, (int)K, score_func, route_norm, route_scale, (int)MI355_SELECT_TOPK);
+  };
+  if (dtype == MI355_F32) { DISPATCH_VPL(E, launch(select_bwd_kernel<VPL, float>)); }
+  else { DISPATCH_VPL(E, launch(select_bwd_kernel<VPL, uint16_t>)); }
+  return check_launch("router_select_rows_bwd");
 }

@@ -68,6 +68,7 @@ struct Block {
   int dt, gate_dt;
   int splits;           // partial sums of the router's forward (0: the kernel without them)
   int64_t piece_bytes;  // its weight pieces
+  bool gather;         // the kernels of any width serve the routed part and read the tokens' rows in place
   bool folded;         // the folded kernels (token gather, combine's backward inside the experts') serve the routed part
   bool shared_folded;  // the bf16 MFMA kernels serve the shared expert
 
@@ -80,6 +81,7 @@ struct Block {
     dt = dtype_code(x);
     gate_dt = dtype_code(gate_w);
     folded = mi355_grouped_combine_bwd_slots(dt, D, F) > 0 && T * D * 2 < (int64_t{1} << 32);
+    gather = !folded && mi355_grouped_gather_covers(dt, D, F, R, T);
     Fs = sg.defined() ? sg.size(0) : 0;
     shared_cap = Fs > 0 ? (T + tile_m - 1) / tile_m : 0;
     splits = mi355_router_gate_fwd_splits(dt, gate_dt, T, D, E);
@@ -147,7 +149,7 @@ struct Kept {
       up = c.take(b.R * b.F, item);
     }
     if (!b.folded) {
-      rows = c.take(b.R * b.D, item);
+      if (!b.gather) rows = c.take(b.R * b.D, item);
       h = c.take(b.R * b.F, item);
       y = c.take(b.R * b.D, item);
     }
@@ -265,7 +267,7 @@ std::tuple<Tensor, Tensor, Tensor> block_forward(const Block& b, const Stats& st
             b.T, b.E, c.K, (int)c.score_func, (int)c.route_norm, (float)c.route_scale, (int)c.num_groups,
             (int)c.num_limited, k.weights, k.ids, c.lo, c.hi, c.align, b.tile_m,
             stats ? all_counts : counts.data_ptr<int32_t>(), k.seg_offsets, k.seg_counts, k.row_of_slot, k.slot_of_row,
-            k.token_of_row, save && b.folded ? k.row_scale : nullptr, b.R, k.tile_expert, k.tile_row0, k.num_tiles,
+            k.token_of_row, save && (b.folded || b.gather) ? k.row_scale : nullptr, b.R, k.tile_expert, k.tile_row0, k.num_tiles,
             b.tile_cap, plan_work, padding, stats ? counts.data_ptr<int32_t>() : nullptr, scores, cutoff, k.aux_f,
             k.aux_scale, ptr(st.aux_acc), st.aux_acc.defined() ? dtype_code(st.aux_acc) : MI355_F32, fptr(st.aux_denominator), (float)st.aux_coeff, stats_work,
             L.stream),
@@ -276,14 +278,20 @@ std::tuple<Tensor, Tensor, Tensor> block_forward(const Block& b, const Stats& st
           "quantile_observe");
 
   // routed experts
-  if (!b.folded)
+  if (!b.folded && !b.gather)
     check(mi355_permute_rows_fwd(ptr(b.x), b.dt, k.row_of_slot, c.align > 1 ? k.slot_of_row : nullptr,
                                  k.seg_offsets + b.El, k.rows, b.T, b.D, c.K, b.R, L.stream),
           "permute_rows_fwd");
-  check(mi355_grouped_swiglu_fwd(b.folded ? ptr(b.x) : k.rows, b.folded ? k.token_of_row : nullptr, b.folded ? b.T : b.R,
-                                 ptr(b.w1), ptr(b.w3), ptr(b.w2), b.dt, k.seg_offsets, k.seg_counts, k.tile_expert,
-                                 k.tile_row0, k.num_tiles, b.tile_cap, k.gate, k.up, h, y, b.El, b.D, b.F, b.R, L.stream),
-        "grouped_swiglu_fwd");
+  if (b.gather)
+    check(mi355_grouped_gather_fwd(ptr(b.x), k.token_of_row, b.T, ptr(b.w1), ptr(b.w3), ptr(b.w2), b.dt, k.seg_offsets,
+                                   k.seg_counts, k.tile_expert, k.tile_row0, k.num_tiles, b.tile_cap, k.gate, k.up, h, y, b.El,
+                                   b.D, b.F, b.R, L.stream),
+          "grouped_gather_fwd");
+  else
+    check(mi355_grouped_swiglu_fwd(b.folded ? ptr(b.x) : k.rows, b.folded ? k.token_of_row : nullptr, b.folded ? b.T : b.R,
+                                   ptr(b.w1), ptr(b.w3), ptr(b.w2), b.dt, k.seg_offsets, k.seg_counts, k.tile_expert,
+                                   k.tile_row0, k.num_tiles, b.tile_cap, k.gate, k.up, h, y, b.El, b.D, b.F, b.R, L.stream),
+          "grouped_swiglu_fwd");
   if (b.Fs > 0 && !aux) shared_forward(b, k, y_shared, L.stream);
   shared.join();
   check(mi355_combine_add_fwd(y, b.dt, k.weights, k.row_of_slot, y_shared, ptr(out), b.T, b.D, c.K, (int)c.round_terms,
@@ -350,7 +358,7 @@ Grads block_backward(const Block& b, const Tensor& kept, const Tensor& dout_, co
     if (b.folded) {
       hs = cv.take(b.R * b.F, item);
       dots = cv.take<float>(b.R * slots);
-    } else {
+    } else if (!b.gather) {
       dy = cv.take(b.R * b.D, item);
       dots = cv.take<float>(b.N);
     }
@@ -426,6 +434,19 @@ Grads block_backward(const Block& b, const Tensor& kept, const Tensor& dout_, co
     row_sum();
     if (logits) select();
     if (need.experts && !side) run(kWeights, L.stream);
+  } else if (b.gather) {
+    if (logits)
+      check(mi355_router_select_rows_bwd(k.logits, k.ids, ptr(dout), k.y, b.dt, k.row_of_slot, b.R, b.D, k.aux_f, k.aux_scale,
+                                         static_cast<const uint8_t*>(ptr(b.mask)), dlogits, b.T, b.E, c.K, (int)c.score_func,
+                                         (int)c.route_norm, (float)c.route_scale, L.stream),
+            "router_select_rows_bwd");
+    if (need.x || need.experts)
+      check(mi355_grouped_gather_bwd(ptr(dout), ptr(b.x), k.token_of_row, b.T, k.row_scale, ptr(b.w1), ptr(b.w3), ptr(b.w2),
+                                     k.gate, k.up, k.h, b.dt, k.seg_offsets, k.seg_counts, k.tile_expert, k.tile_row0,
+                                     k.num_tiles, b.tile_cap, dgate, dup, drows, ptr(g.w1), ptr(g.w3), ptr(g.w2), b.El, b.D,
+                                     b.F, b.R, L.stream),
+            "grouped_gather_bwd");
+    row_sum();
   } else {
     const int32_t* pad = c.align > 1 ? k.slot_of_row : nullptr;
     check(mi355_combine_bwd(ptr(dout), k.y, b.dt, k.weights, k.row_of_slot, pad, k.seg_offsets + b.El, dy, dots, b.T, b.D,
