@@ -521,12 +521,24 @@ int mi355_grouped_swiglu_combine_bwd(const void* dout, const void* x, const int3
                                      void* dw1, void* dw3, void* dw2, int64_t El, int64_t D,
                                      int64_t F, int64_t row_capacity, int stages, void* stream);
 /*
+ * The end of a block's backward with up to 32 experts and a fp32 gate weight (mi355_router_gate_rows_bwd_covers), in one launch:
+ * dx = dlogits . w + (the sum of drows over a token's K slots + addend), the bits of mi355_permute_rows_add_bwd and
+ * mi355_router_gate_add_bwd, and dw = the sum of the slices that mi355_grouped_gather_bwd left in dw_partial.  dx, dw, addend
+ * may be NULL.
+ */
+int mi355_router_gate_rows_bwd_covers(int x_dtype, int w_dtype, int64_t D, int64_t E);
+int mi355_router_gate_rows_bwd(const float* dlogits, int x_dtype, const float* w, const void* drows,
+                               const int32_t* row_of_slot, int64_t row_capacity, int64_t K, const void* addend, void* dx,
+                               const float* dw_partial, float* dw, int64_t T, int64_t D, int64_t E, void* stream);
+/*
  * mi355_permute_rows_fwd + mi355_grouped_swiglu_fwd, and the expert side of mi355_combine_bwd + mi355_grouped_swiglu_bwd, for
  * fp32 and for bf16 widths off the grid above, with the tokens' rows read where they lie: x and dout are
  * (num_tokens,D), row r stands for row token_of_row[r], of dout scaled by row_scale[r] and rounded.  The same bits as the
  * two calls, without the copies in row order.  mi355_grouped_gather_covers: 1 where they serve a case (widths
  * multiples of four, matrices below 4 GiB and on 16-byte boundaries).  gate, up and h are always written, drows, dw1, dw3, dw2
- * may be NULL.  At least one row.
+ * may be NULL.  At least one row.  dlogits (NULL: not wanted; where mi355_router_gate_rows_bwd_covers): the slices of the router
+ * gate's weight gradient are formed in the same launches, into gate_partial (the workspace of mi355_router_gate_bwd), for
+ * mi355_router_gate_rows_bwd to add up.
  */
 int mi355_grouped_gather_covers(int dtype, int64_t D, int64_t F, int64_t row_capacity, int64_t num_tokens);
 int mi355_grouped_gather_fwd(const void* x, const int32_t* token_of_row, int64_t num_tokens, const void* w1,
@@ -539,7 +551,8 @@ int mi355_grouped_gather_bwd(const void* dout, const void* x, const int32_t* tok
                              const void* up, const void* h, int dtype, const int32_t* seg_offsets,
                              const int32_t* seg_counts, const int32_t* tile_expert, const int32_t* tile_row0,
                              const int32_t* num_tiles, int64_t tile_capacity, void* dgate, void* dup, void* drows,
-                             void* dw1, void* dw3, void* dw2, int64_t El, int64_t D, int64_t F, int64_t row_capacity,
+                             void* dw1, void* dw3, void* dw2, const float* dlogits, float* gate_partial,
+                             int64_t gate_experts, int64_t El, int64_t D, int64_t F, int64_t row_capacity,
                              void* stream);
 int mi355_combine_row_scale(const float* weights_TK, const int32_t* slot_of_row, float* row_scale,
                             int64_t T, int64_t K, int64_t row_capacity, void* stream);

@@ -61,6 +61,10 @@ bool router_few_ok(int x_dtype, int w_dtype, int64_t D, int64_t E);
 int64_t router_few_bwd_workspace(int64_t T, int64_t D, int64_t E);
 int router_few_bwd(const float* dlogits, const void* x, int x_dtype, const float* w, const void* addend, void* dx, float* dw,
                    void* workspace, int64_t T, int64_t D, int64_t E, hipStream_t s);
+// The same where the dW parts have run (`partial`, a slice of the tokens each) and the addend is the sum of the experts' rows.
+int router_rows_bwd(const float* dlogits, int x_dtype, const float* w, const void* rows, const int32_t* row_of_slot,
+                    int64_t row_capacity, int64_t K, const void* addend, void* dx, const float* partial, float* dw, int64_t T,
+                    int64_t D, int64_t E, hipStream_t s);
 // Forward: `splits` (T, E) partial sums of the contraction, to be added in order (with the bias,
 // unless splits is 1: then it is added already and the one partial is the logits); 0 = no kernel
 // of that file serves the case.  `pieces` is scratch of router_fwd_pieces_bytes.

@@ -245,7 +245,7 @@ extern "C" int mi355_grouped_swiglu_bwd(const void* dy, const void* rows,
     const AnySeg g{seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity, El};
     const bool some = row_capacity > 0 && tile_capacity > 0;
     if (some)
-      if (int rc = any_dh(g, dtype, dy, w2, gate, up, dgate, dup, D, F, row_capacity, nullptr, s)) return rc;
+      if (int rc = any_dh(g, dtype, dy, w2, gate, up, dgate, dup, D, F, row_capacity, nullptr, nullptr, s)) return rc;
     // the weight gradients also cover the no-rows case: every expert's gradient is written (zeros)
     AnyGrad grads[3];
     int count = 0;
@@ -432,7 +432,8 @@ extern "C" int mi355_grouped_gather_bwd(const void* dout, const void* x, const i
                                         const void* gate, const void* up, const void* h, int dtype,
                                         const int32_t* seg_offsets, const int32_t* seg_counts, const int32_t* tile_expert,
                                         const int32_t* tile_row0, const int32_t* num_tiles, int64_t tile_capacity,
-                                        void* dgate, void* dup, void* drows, void* dw1, void* dw3, void* dw2, int64_t El,
+                                        void* dgate, void* dup, void* drows, void* dw1, void* dw3, void* dw2,
+                                        const float* dlogits, float* gate_partial, int64_t gate_experts, int64_t El,
                                         int64_t D, int64_t F, int64_t row_capacity, void* stream) {
   if (int rc = check_common("grouped_gather_bwd", dtype, El, D, F, row_capacity, tile_capacity)) return rc;
   MI355_REQUIRE(row_capacity >= 1 && tile_capacity >= 1 && dout && x && token_of_row && row_scale && w1 && w3 && w2 && gate &&
@@ -442,7 +443,14 @@ extern "C" int mi355_grouped_gather_bwd(const void* dout, const void* x, const i
     return fail(MI355_EUNSUP, "grouped_gather_bwd: not covered; use mi355_combine_bwd and mi355_grouped_swiglu_bwd");
   const AnySeg g{seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity, El};
   const AnyFold fold{token_of_row, num_tokens, row_scale};
-  if (int rc = any_dh(g, dtype, dout, w2, gate, up, dgate, dup, D, F, row_capacity, &fold, as_stream(stream))) return rc;
+  MI355_REQUIRE(!dlogits || (gate_partial && gate_experts >= 1 && aligned16({dlogits, gate_partial})),
+                "grouped_gather_bwd: null or misaligned pointer");
+  if (dlogits && !router_few_ok(dtype, MI355_F32, D, gate_experts))
+    return fail(MI355_EUNSUP, "grouped_gather_bwd: the gate's gradient is not covered; use mi355_router_gate_bwd");
+  const AnyGate job{dlogits, x, gate_partial, gate_experts};
+  if (int rc = any_dh(g, dtype, dout, w2, gate, up, dgate, dup, D, F, row_capacity, &fold, dlogits ? &job : nullptr,
+                      as_stream(stream)))
+    return rc;
   AnyGrad grads[3];
   int count = 0;
   if (dw2) grads[count++] = {dout, h, dw2, D, F, 1};

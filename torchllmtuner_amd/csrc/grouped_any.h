@@ -15,6 +15,13 @@ struct AnyFold {
   int64_t tokens;
   const float* row_scale;  // (backward)
 };
+// The router gate's weight gradient, to be formed beside dH (with a fold): dlogits (tokens, E) fp32, x the tokens, of the rows' dtype.
+struct AnyGate {
+  const float* dlogits;
+  const void* x;
+  float* partial;
+  int64_t E;
+};
 struct AnyGrad {  // c (El, M, N) = per segment a^T (rows, M) . b (rows, N)
   const void *a, *b;
   void* c;
@@ -31,7 +38,7 @@ int any_linear(const AnySeg& g, int dtype, const void* x, const void* w, void* y
 int any_linear_dx(const AnySeg& g, int dtype, const void* dy, const void* w, void* dx, int64_t I, int64_t O, int64_t R,
                   hipStream_t s);
 int any_dh(const AnySeg& g, int dtype, const void* dy, const void* w2, const void* gate, const void* up, void* dgate,
-           void* dup, int64_t D, int64_t F, int64_t R, const AnyFold* fold, hipStream_t s);
+           void* dup, int64_t D, int64_t F, int64_t R, const AnyFold* fold, const AnyGate* router, hipStream_t s);
 // drows (null: not wanted) = dgate . w1 + dup . w3, and at most three weight gradients
 int any_backward(const AnySeg& g, int dtype, const void* dgate, const void* dup, const void* w1, const void* w3, void* drows,
                  int64_t D, int64_t F, const AnyGrad* grads, int count, int64_t R, const AnyFold* fold, hipStream_t s);

@@ -26,6 +26,7 @@
 #include "bf16_tiles.h"
 #include "common.h"
 #include "grouped_any.h"
+#include "router_few.h"
 
 namespace mi355 {
 namespace {
@@ -489,6 +490,19 @@ __global__ __launch_bounds__(256) void any_kernel(AnyArgs p) {
   any_tile<T, MODE, TM, TN, FOLD>(p, blockIdx.x, smem);
 }
 
+// The experts' dH and, in the workgroups past its `blocks`, the router gate's weight gradient: both need what the
+// selection's backward left, neither the other, and neither fills the chip.  With the gate's input gradient taking the sum over a
+// token's rows along, and the slices' sum beside it, a backward has four launches instead of seven: a training step of 1531 bf16 tokens of
+// 16 x 320 x 232 128 -> 109 us, 512 fp32 of 8 x 256 x 512 126 -> 119, 100 bf16 of 4 x 200 x 104 139 -> 122.
+template <typename T, int TM, int TN>
+__global__ __launch_bounds__(256) void any_dh_gate_kernel(AnyArgs p, GateDw gate, int blocks) {
+  constexpr int A = any_lds<T, ANY_DH, TM, TN>(), B = kGateDwLds * 4 / sizeof(T);
+  __shared__ __attribute__((aligned(16))) T smem[A > B ? A : B];
+  const int block = blockIdx.x;
+  if (block < blocks) any_tile<T, ANY_DH, TM, TN, true>(p, block, smem);
+  else gate_dw_part<T>(gate, block - blocks, reinterpret_cast<float*>(smem));
+}
+
 // The input gradient and the weight gradients of a backward pass read the same buffers and write different
 // ones: with few tiles each they share a launch (at 512 fp32 tokens of 8 experts 26 + 16 us one after the
 // other).  The longer contraction starts first.
@@ -502,9 +516,20 @@ __global__ __launch_bounds__(256) void any_dx_dw_kernel(AnyArgs dx, AnyArgs dw, 
 }
 
 template <int MODE, int TM, int TN>
-int launch_any(const AnyArgs& p, int dtype, int64_t blocks, hipStream_t s, const char* what) {
+int launch_any(const AnyArgs& p, int dtype, int64_t blocks, hipStream_t s, const char* what, const GateDw* gate = nullptr) {
   if (blocks <= 0) return MI355_OK;
   if (dtype != MI355_F32 && TM == 32) return fail(MI355_EUNSUP, "%s: 32-row tiles are for fp32", what);
+  if constexpr (MODE == ANY_DH) {
+    if (gate) {
+      const dim3 grid((unsigned)(blocks + gate_dw_parts(*gate))), lanes(256);
+      if (dtype == MI355_F32) {
+        hipLaunchKernelGGL((any_dh_gate_kernel<float, TM, TN>), grid, lanes, 0, s, p, *gate, (int)blocks);
+      } else if constexpr (TM != 32) {
+        hipLaunchKernelGGL((any_dh_gate_kernel<uint16_t, TM, TN>), grid, lanes, 0, s, p, *gate, (int)blocks);
+      }
+      return check_launch(what);
+    }
+  }
   auto run = [&](auto fold) {
     constexpr bool FOLD = decltype(fold)::value;
     const dim3 grid((unsigned)blocks), lanes(256);
@@ -536,15 +561,16 @@ int row_tile(const AnyArgs& p, int dtype, int64_t El, int64_t cols) {
 }
 
 template <int MODE>
-int launch_rows(AnyArgs& p, int dtype, int64_t tile_capacity, int64_t El, int64_t cols, hipStream_t s, const char* what) {
+int launch_rows(AnyArgs& p, int dtype, int64_t tile_capacity, int64_t El, int64_t cols, hipStream_t s, const char* what,
+                const GateDw* gate = nullptr) {
   constexpr bool GU = MODE == ANY_GATEUP;
   const int t = row_tile(p, dtype, El, cols), width = GU && t == 128 ? 64 : t;
   p.col_tiles = (int)((cols + width - 1) / width);
   const int64_t blocks = tile_capacity * (256 / t) * p.col_tiles;
   MI355_REQUIRE(blocks < (1ll << 30), "%s: too many tiles", what);
-  if (t == 128) return launch_any<MODE, 128, 128>(p, dtype, blocks, s, what);
-  return t == 64 ? launch_any<MODE, 64, GU ? 128 : 64>(p, dtype, blocks, s, what)
-                 : launch_any<MODE, 32, GU ? 64 : 32>(p, dtype, blocks, s, what);
+  if (t == 128) return launch_any<MODE, 128, 128>(p, dtype, blocks, s, what, gate);
+  return t == 64 ? launch_any<MODE, 64, GU ? 128 : 64>(p, dtype, blocks, s, what, gate)
+                 : launch_any<MODE, 32, GU ? 64 : 32>(p, dtype, blocks, s, what, gate);
 }
 
 int64_t dw_tiles(AnyArgs& p, int64_t El, int tile) {
@@ -603,11 +629,13 @@ int any_linear_dx(const AnySeg& g, int dtype, const void* dy, const void* w, voi
 }
 
 int any_dh(const AnySeg& g, int dtype, const void* dy, const void* w2, const void* gate, const void* up, void* dgate,
-           void* dup, int64_t D, int64_t F, int64_t R, const AnyFold* f, hipStream_t s) {
+           void* dup, int64_t D, int64_t F, int64_t R, const AnyFold* f, const AnyGate* router, hipStream_t s) {
   AnyArgs p = any_args(g, R, f);
   p.a0 = dy; p.b0 = w2; p.c0 = dgate; p.c1 = dup; p.gate = gate; p.up = up;
   p.K = (int)D; p.N = (int)F; p.ldb = (int)F; p.w_elems = D * F;
-  return launch_rows<ANY_DH>(p, dtype, g.tile_capacity, g.El, F, s, "grouped dh");
+  GateDw job{};
+  if (router) job = gate_dw_job(router->dlogits, router->x, router->partial, f->tokens, D, router->E);
+  return launch_rows<ANY_DH>(p, dtype, g.tile_capacity, g.El, F, s, "grouped dh", router ? &job : nullptr);
 }
 
 int any_backward(const AnySeg& g, int dtype, const void* dgate, const void* dup, const void* w1, const void* w3, void* drows,

@@ -559,6 +559,26 @@ extern "C" int mi355_router_gate_add_bwd(const float* dlogits, const void* x, in
   return MI355_OK;
 }
 
+extern "C" int mi355_router_gate_rows_bwd_covers(int x_dtype, int w_dtype, int64_t D, int64_t E) {
+  return E >= 1 && router_few_ok(x_dtype, w_dtype, D, E) ? 1 : 0;
+}
+
+extern "C" int mi355_router_gate_rows_bwd(const float* dlogits, int x_dtype, const float* w, const void* drows,
+                                          const int32_t* row_of_slot, int64_t row_capacity, int64_t K, const void* addend,
+                                          void* dx, const float* dw_partial, float* dw, int64_t T, int64_t D, int64_t E,
+                                          void* stream) {
+  MI355_REQUIRE(T >= 1 && T < (1ll << 31) && D >= 1 && D < (1ll << 31) && E >= 1 && K >= 1 && K <= 64 && row_capacity >= 0 &&
+                    row_capacity < (1ll << 31),
+                "router_gate_rows_bwd: bad shape");
+  if (!router_few_ok(x_dtype, MI355_F32, D, E))
+    return fail(MI355_EUNSUP, "router_gate_rows_bwd: not covered; use mi355_permute_rows_add_bwd and mi355_router_gate_add_bwd");
+  MI355_REQUIRE(!dx || (dlogits && w && drows && row_of_slot), "router_gate_rows_bwd: null pointer");
+  MI355_REQUIRE(!dw || dw_partial, "router_gate_rows_bwd: null pointer");
+  MI355_REQUIRE(aligned16({dlogits, w, drows, addend, dx, dw_partial, dw}), "router_gate_rows_bwd: misaligned pointer");
+  return router_rows_bwd(dlogits, x_dtype, w, drows, row_of_slot, row_capacity, K, addend, dx, dw_partial, dw, T, D, E,
+                         as_stream(stream));
+}
+
 extern "C" int mi355_router_gate_bwd(const float* dlogits, const void* x, int x_dtype,
                                      const void* w, int w_dtype, void* dx, void* dw,
                                      void* workspace, int64_t T, int64_t D, int64_t E,

@@ -17,6 +17,7 @@
 #include "bf16_tiles.h"
 #include "common.h"
 #include "gemm_generic.h"
+#include "router_few.h"
 
 namespace mi355 {
 namespace {
@@ -485,76 +486,23 @@ __global__ __launch_bounds__(W_NT, 2) void gate_dw_kernel(const float* __restric
   }
 }
 
-// ---- both gradients for few experts -----------------------------------------------------
-// dW = dlogits^T . x and dx = dlogits . W (+ addend) in one launch, for up to 32 experts: both then read
-// or write a (T, D) matrix against a handful of rows, too thin for matrix tiles, and the vector units
-// keep up with memory.  A thread owns four columns.  dW workgroups (the first `dw_blocks`): eight experts,
-// 256 columns and a slice of the tokens, the four waves on every fourth token, joined through LDS in wave
-// order; the slices' sums are added by splitk_reduce.  dx workgroups: 32 tokens x 256 columns, dlogits in LDS.
-// 1531 tokens, 320 x 16, bf16: 12 us with the sum, 47 with the strided GEMMs it replaces.
-constexpr int S_EB = 8, S_COLS = 256, S_TOK = 32, S_MAX_E = 32;
-
-__device__ __forceinline__ f32x4 load_cols(const float* p) { return *reinterpret_cast<const f32x4*>(p); }
-__device__ __forceinline__ f32x4 load_cols(const uint16_t* p) {
-  const u32x2 v = *reinterpret_cast<const u32x2*>(p);
-  return {__uint_as_float(v[0] << 16), __uint_as_float(v[0] & 0xffff0000u), __uint_as_float(v[1] << 16),
-          __uint_as_float(v[1] & 0xffff0000u)};
-}
-__device__ __forceinline__ void store_cols(float* p, const f32x4& v) { *reinterpret_cast<f32x4*>(p) = v; }
-__device__ __forceinline__ void store_cols(uint16_t* p, const f32x4& v) {
-  *reinterpret_cast<u32x2*>(p) = u32x2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
-}
-
+// ---- both gradients for few experts (router_few.h) ---------------------------------------
+// What dx parts read besides dlogits and W.  rows: null, or the experts' input gradients, whose sum over the token's K
+// slots in ascending order, rounded, comes in front of the addend as permute_rows_bwd's does.
 template <typename TX>
-__global__ __launch_bounds__(256) void gate_bwd_few_kernel(const float* __restrict__ dlogits, const TX* __restrict__ x,
-                                                           const float* __restrict__ w, const TX* __restrict__ addend,
-                                                           TX* __restrict__ dx, float* __restrict__ partial, int T,
-                                                           int D, int E, int dw_blocks, int splits, int rows_per_split) {
-  __shared__ __attribute__((aligned(16))) float lds[4 * S_EB * S_COLS];
+struct GateDx {
+  const TX *addend, *rows;
+  const int32_t* row_of_slot;
+  int K, row_capacity;
+};
+
+template <typename TX, bool ROWS>
+__device__ __forceinline__ void gate_dx_part(const float* __restrict__ dlogits, const float* __restrict__ w,
+                                             const GateDx<TX>& g, TX* __restrict__ dx, int T, int D, int E, int part,
+                                             float* lds) {
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col_blocks = (D + S_COLS - 1) / S_COLS;
-  if (static_cast<int>(blockIdx.x) < dw_blocks) {
-    const int cb = blockIdx.x % col_blocks, rest = blockIdx.x / col_blocks, split = rest % splits, e0 = rest / splits * S_EB;
-    const int n = min(cb * S_COLS + lane * 4, D - 4);  // (D % 4 == 0; lanes past the end repeat the last columns)
-    const int t0 = split * rows_per_split, t1 = min(T, t0 + rows_per_split);
-    f32x4 acc[S_EB];
-#pragma unroll
-    for (int e = 0; e < S_EB; ++e) acc[e] = f32x4{0, 0, 0, 0};
-    constexpr int U = 4;  // tokens requested together
-    for (int t = t0 + wave; t < t1; t += 4 * U) {
-      f32x4 xv[U];
-      float dl[U][S_EB];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int tt = t + 4 * u;
-        const bool live = tt < t1;
-        xv[u] = load_cols(x + static_cast<int64_t>(live ? tt : t) * D + n);
-#pragma unroll
-        for (int e = 0; e < S_EB; ++e)
-          dl[u][e] = live && e0 + e < E ? dlogits[static_cast<int64_t>(tt) * E + e0 + e] : 0.0f;
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-#pragma unroll
-        for (int e = 0; e < S_EB; ++e)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) acc[e][i] = fmaf(dl[u][e], xv[u][i], acc[e][i]);
-    }
-#pragma unroll
-    for (int e = 0; e < S_EB; ++e) *reinterpret_cast<f32x4*>(lds + (wave * S_EB + e) * S_COLS + lane * 4) = acc[e];
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < S_EB / 4; ++i) {
-      const int e = wave * (S_EB / 4) + i;
-      f32x4 v = *reinterpret_cast<const f32x4*>(lds + e * S_COLS + lane * 4);
-#pragma unroll
-      for (int j = 1; j < 4; ++j) v += *reinterpret_cast<const f32x4*>(lds + (j * S_EB + e) * S_COLS + lane * 4);
-      if (e0 + e < E && cb * S_COLS + lane * 4 < D)
-        store_cols(partial + (static_cast<int64_t>(split) * E + e0 + e) * D + cb * S_COLS + lane * 4, v);
-    }
-    return;
-  }
-  const int b = blockIdx.x - dw_blocks, cb = b % col_blocks, t0 = b / col_blocks * S_TOK;
+  const int cb = part % col_blocks, t0 = part / col_blocks * S_TOK;
   const int tokens = min(S_TOK, T - t0), n = cb * S_COLS + lane * 4;
   constexpr int PITCH = S_MAX_E;
   for (int i = tid; i < S_TOK * PITCH; i += 256) {
@@ -563,6 +511,23 @@ __global__ __launch_bounds__(256) void gate_bwd_few_kernel(const float* __restri
   }
   __syncthreads();
   if (n >= D) return;
+  f32x4 sum[ROWS ? 8 : 1];
+  if constexpr (ROWS) {
+    // the rows go out first: the product below runs while they arrive.  One slot of eight tokens at a time.
+#pragma unroll
+    for (int t = 0; t < 8; ++t) sum[t] = f32x4{0, 0, 0, 0};
+    const int32_t* slots = g.row_of_slot + (static_cast<int64_t>(t0) + wave * 8) * g.K;
+    for (int k = 0; k < g.K; ++k) {
+      f32x4 v[8];
+#pragma unroll
+      for (int t = 0; t < 8; ++t) {
+        const int row = wave * 8 + t < tokens ? slots[t * g.K + k] : -1;  // wave-uniform
+        v[t] = row >= 0 && row < g.row_capacity ? load_cols(g.rows + static_cast<int64_t>(row) * D + n) : f32x4{0, 0, 0, 0};
+      }
+#pragma unroll
+      for (int t = 0; t < 8; ++t) sum[t] += v[t];
+    }
+  }
   f32x4 acc[8];  // tokens wave * 8 ..
 #pragma unroll
   for (int t = 0; t < 8; ++t) acc[t] = f32x4{0, 0, 0, 0};
@@ -579,18 +544,61 @@ __global__ __launch_bounds__(256) void gate_bwd_few_kernel(const float* __restri
         for (int i = 0; i < 4; ++i) acc[t][i] = fmaf(d[j], wv[j][i], acc[t][i]);
     }
   }
+  auto rounded = [](float v) { return sizeof(TX) == 2 ? round_bf16(v) : v; };
 #pragma unroll
   for (int t = 0; t < 8; ++t) {
     if (wave * 8 + t >= tokens) break;
     const int64_t at = static_cast<int64_t>(t0 + wave * 8 + t) * D + n;
     f32x4 v = acc[t];
-    if (addend) {  // added to the rounded sum and rounded again, like a separate addition
-      const f32x4 a = load_cols(addend + at);
+    // each sum is added to the rounded one before it and rounded again, as separate additions would be
+    if (ROWS || g.addend) {
+      f32x4 a = g.addend ? load_cols(g.addend + at) : f32x4{0, 0, 0, 0};
+      if constexpr (ROWS) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = (sizeof(TX) == 2 ? round_bf16(v[i]) : v[i]) + a[i];
+        for (int i = 0; i < 4; ++i) a[i] = g.addend ? rounded(rounded(sum[t][i]) + a[i]) : rounded(sum[t][i]);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = rounded(v[i]) + a[i];
     }
     store_cols(dx + at, v);
   }
+}
+
+template <typename TX>
+__global__ __launch_bounds__(256) void gate_bwd_few_kernel(GateDw dw, const float* __restrict__ dlogits,
+                                                           const float* __restrict__ w, GateDx<TX> g, TX* __restrict__ dx,
+                                                           int T, int D, int E, int dw_parts) {
+  __shared__ __attribute__((aligned(16))) float lds[kGateDwLds];
+  const int block = blockIdx.x;
+  if (block < dw_parts) gate_dw_part<TX>(dw, block, lds);
+  else gate_dx_part<TX, false>(dlogits, w, g, dx, T, D, E, block - dw_parts, lds);
+}
+
+// dx with the sum over the token's rows, and beside it the sum of dW's slices, in their order: the two ends of a backward
+// whose dW parts ran in an earlier launch.
+template <typename TX>
+__global__ __launch_bounds__(256) void gate_rows_bwd_kernel(const float* __restrict__ dlogits, const float* __restrict__ w,
+                                                            GateDx<TX> g, TX* __restrict__ dx,
+                                                            const float* __restrict__ partial, float* __restrict__ dw,
+                                                            int splits, int T, int D, int E, int dx_parts) {
+  __shared__ __attribute__((aligned(16))) float lds[S_TOK * S_MAX_E];
+  const int block = blockIdx.x;
+  if (block < dx_parts) {
+    gate_dx_part<TX, true>(dlogits, w, g, dx, T, D, E, block, lds);
+    return;
+  }
+  const int64_t n = static_cast<int64_t>(E) * D, i = static_cast<int64_t>(block - dx_parts) * 256 + threadIdx.x;
+  if (i >= n) return;
+  float sum = 0.0f;
+  constexpr int B = 8;  // in flight
+  for (int z0 = 0; z0 < splits; z0 += B) {
+    float v[B];
+#pragma unroll
+    for (int b = 0; b < B; ++b) v[b] = z0 + b < splits ? partial[(z0 + b) * n + i] : 0.0f;
+#pragma unroll
+    for (int b = 0; b < B; ++b) sum += v[b];
+  }
+  dw[i] = sum;
 }
 
 template <typename K>
@@ -631,36 +639,49 @@ int dw_splits(int64_t T, int64_t D, int64_t E) {
   return static_cast<int>(best);
 }
 
-// Slices of the tokens for gate_bwd_few_kernel's dW: about two workgroups per CU, at least 32 tokens each.
-int few_splits(int64_t T, int64_t D, int64_t E) {
-  const int64_t tiles = ((D + S_COLS - 1) / S_COLS) * ((E + S_EB - 1) / S_EB);
-  return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({512 / tiles, (T + 31) / 32, 64})));
-}
-
 }  // namespace
 
 bool router_few_ok(int x_dtype, int w_dtype, int64_t D, int64_t E) {
   return w_dtype == MI355_F32 && (x_dtype == MI355_BF16 || x_dtype == MI355_F32) && D % 4 == 0 && D >= 4 && E <= S_MAX_E;
 }
-int64_t router_few_bwd_workspace(int64_t T, int64_t D, int64_t E) { return few_splits(T, D, E) * E * D * 4; }
+int64_t router_few_bwd_workspace(int64_t T, int64_t D, int64_t E) { return gate_dw_splits(T, D, E) * E * D * 4; }
 
 int router_few_bwd(const float* dlogits, const void* x, int x_dtype, const float* w, const void* addend, void* dx, float* dw,
                    void* workspace, int64_t T, int64_t D, int64_t E, hipStream_t s) {
-  const int splits = few_splits(T, D, E), col_blocks = (int)((D + S_COLS - 1) / S_COLS);
-  const int rows = (int)((T + splits - 1) / splits);
-  const int64_t dw_blocks = dw ? (int64_t)col_blocks * splits * ((E + S_EB - 1) / S_EB) : 0;
-  const int64_t blocks = dw_blocks + (dx ? (T + S_TOK - 1) / S_TOK * col_blocks : 0);
+  const int splits = gate_dw_splits(T, D, E);
+  const GateDw job = gate_dw_job(dlogits, x, splits > 1 ? static_cast<float*>(workspace) : dw, T, D, E);
+  const int64_t dw_parts = dw ? gate_dw_parts(job) : 0;
+  const int64_t blocks = dw_parts + (dx ? (T + S_TOK - 1) / S_TOK * ((D + S_COLS - 1) / S_COLS) : 0);
   MI355_REQUIRE(blocks < (1ll << 31), "router_gate_bwd: too many tokens");
-  float* partial = splits > 1 ? static_cast<float*>(workspace) : dw;
-  auto launch = [&](auto* kernel, auto* xp) {
+  auto launch = [&](auto* xp) {
     using TX = std::remove_const_t<std::remove_pointer_t<decltype(xp)>>;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, s, dlogits, xp, w, static_cast<const TX*>(addend),
-                       static_cast<TX*>(dx), partial, (int)T, (int)D, (int)E, (int)dw_blocks, splits, rows);
+    hipLaunchKernelGGL(gate_bwd_few_kernel<TX>, dim3((unsigned)blocks), dim3(256), 0, s, job, dlogits, w,
+                       GateDx<TX>{static_cast<const TX*>(addend), nullptr, nullptr, 0, 0}, static_cast<TX*>(dx), (int)T, (int)D,
+                       (int)E, (int)dw_parts);
   };
-  if (x_dtype == MI355_BF16) launch(gate_bwd_few_kernel<uint16_t>, static_cast<const uint16_t*>(x));
-  else launch(gate_bwd_few_kernel<float>, static_cast<const float*>(x));
+  if (x_dtype == MI355_BF16) launch(static_cast<const uint16_t*>(x));
+  else launch(static_cast<const float*>(x));
   if (int rc = check_launch("router_gate_bwd")) return rc;
-  return dw && splits > 1 ? launch_splitk_reduce(partial, dw, MI355_F32, E * D, splits, s) : MI355_OK;
+  return dw && splits > 1 ? launch_splitk_reduce(job.partial, dw, MI355_F32, E * D, splits, s) : MI355_OK;
+}
+
+int router_rows_bwd(const float* dlogits, int x_dtype, const float* w, const void* rows, const int32_t* row_of_slot,
+                    int64_t row_capacity, int64_t K, const void* addend, void* dx, const float* partial, float* dw, int64_t T,
+                    int64_t D, int64_t E, hipStream_t s) {
+  const int splits = gate_dw_splits(T, D, E);
+  const int64_t dx_parts = dx ? (T + S_TOK - 1) / S_TOK * ((D + S_COLS - 1) / S_COLS) : 0;
+  const int64_t blocks = dx_parts + (dw ? (E * D + 255) / 256 : 0);
+  MI355_REQUIRE(blocks < (1ll << 31), "router_gate_rows_bwd: too many tokens");
+  if (blocks == 0) return MI355_OK;
+  auto launch = [&](auto* xp) {
+    using TX = std::remove_pointer_t<decltype(xp)>;
+    const GateDx<TX> g{static_cast<const TX*>(addend), static_cast<const TX*>(rows), row_of_slot, (int)K, (int)row_capacity};
+    hipLaunchKernelGGL(gate_rows_bwd_kernel<TX>, dim3((unsigned)blocks), dim3(256), 0, s, dlogits, w, g, xp, partial, dw,
+                       splits, (int)T, (int)D, (int)E, (int)dx_parts);
+  };
+  if (x_dtype == MI355_BF16) launch(static_cast<uint16_t*>(dx));
+  else launch(static_cast<float*>(dx));
+  return check_launch("router_gate_rows_bwd");
 }
 
 bool router_x3_ok(int x_dtype, int w_dtype, int64_t D, int64_t E) {

@@ -336,6 +336,9 @@ Grads block_backward(const Block& b, const Tensor& kept, const Tensor& dout_, co
     like(g.sd, b.sd);
   }
   const int64_t slots = b.folded ? mi355_grouped_combine_bwd_slots(b.dt, b.D, b.F) : 0;
+  // the gate's weight gradient in slices beside the experts' dH, its input gradient together with the row sum
+  const bool joined = b.gather && mi355_router_gate_rows_bwd_covers(b.dt, b.gate_dt, b.D, b.E);
+  const bool joined_dw = joined && need.gate_w && (need.x || need.experts);
   const int64_t gate_bytes = need.x || need.gate_w ? mi355_router_gate_bwd_workspace_bytes(b.T, b.D, b.E) : 0;
   void *s_dgate = nullptr, *s_dup = nullptr, *dx_shared = nullptr, *dx_routed = nullptr, *dgate = nullptr, *dup = nullptr,
        *drows = nullptr, *hs = nullptr, *dy = nullptr, *gate_work = nullptr;
@@ -350,7 +353,7 @@ Grads block_backward(const Block& b, const Tensor& kept, const Tensor& dout_, co
     }
     if (!routed) return;
     if (need.x) {
-      dx_routed = cv.take(b.T * b.D, item);
+      if (!joined) dx_routed = cv.take(b.T * b.D, item);
       drows = cv.take(b.R * b.D, item);
     }
     dgate = cv.take(b.R * b.F, item);
@@ -443,10 +446,11 @@ Grads block_backward(const Block& b, const Tensor& kept, const Tensor& dout_, co
     if (need.x || need.experts)
       check(mi355_grouped_gather_bwd(ptr(dout), ptr(b.x), k.token_of_row, b.T, k.row_scale, ptr(b.w1), ptr(b.w3), ptr(b.w2),
                                      k.gate, k.up, k.h, b.dt, k.seg_offsets, k.seg_counts, k.tile_expert, k.tile_row0,
-                                     k.num_tiles, b.tile_cap, dgate, dup, drows, ptr(g.w1), ptr(g.w3), ptr(g.w2), b.El, b.D,
-                                     b.F, b.R, L.stream),
+                                     k.num_tiles, b.tile_cap, dgate, dup, drows, ptr(g.w1), ptr(g.w3), ptr(g.w2),
+                                     joined_dw ? dlogits : nullptr, static_cast<float*>(gate_work), b.E, b.El, b.D, b.F, b.R,
+                                     L.stream),
             "grouped_gather_bwd");
-    row_sum();
+    if (!joined) row_sum();
   } else {
     const int32_t* pad = c.align > 1 ? k.slot_of_row : nullptr;
     check(mi355_combine_bwd(ptr(dout), k.y, b.dt, k.weights, k.row_of_slot, pad, k.seg_offsets + b.El, dy, dots, b.T, b.D,
@@ -462,10 +466,22 @@ Grads block_backward(const Block& b, const Tensor& kept, const Tensor& dout_, co
   }
 
   // ---- router gate; the input gradient is complete with its part
-  if (need.x || need.gate_w)
+  if (joined && need.x) {
+    shared.join();
+    check(mi355_router_gate_rows_bwd(dlogits, b.dt, fptr(b.gate_w), drows, k.row_of_slot, b.R, c.K, dx_shared, ptr(g.x),
+                                     static_cast<const float*>(gate_work), joined_dw ? g.gate_w.data_ptr<float>() : nullptr,
+                                     b.T, b.D, b.E, L.stream),
+          "router_gate_rows_bwd");
+  } else if (joined_dw) {
+    check(mi355_router_gate_rows_bwd(nullptr, b.dt, nullptr, nullptr, nullptr, b.R, c.K, nullptr, nullptr,
+                                     static_cast<const float*>(gate_work), g.gate_w.data_ptr<float>(), b.T, b.D, b.E,
+                                     L.stream),
+          "router_gate_rows_bwd");
+  } else if (need.x || need.gate_w) {
     check(mi355_router_gate_add_bwd(dlogits, ptr(b.x), b.dt, ptr(b.gate_w), b.gate_dt, k.pieces, dx_routed, ptr(g.x),
                                     ptr(g.gate_w), gate_work, b.T, b.D, b.E, L.stream),
           "router_gate_bwd");
+  }
   if (need.gate_b) g.gate_b = dlogits_t.sum(0).to(b.gate_b.scalar_type());
   weights.join();
   shared.join();
