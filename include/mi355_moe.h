@@ -363,6 +363,21 @@ int mi355_route_plan_stats(const float* partial, int splits, const float* logit_
                            const uint8_t* padding_mask_T, int32_t* valid_counts_E, float* scores_TE,
                            float* cutoff_T, float* aux_f_E, float* aux_scale, void* aux_acc,
                            int aux_acc_dtype, const float* aux_denominator, float aux_coeff, void* stats_workspace, void* stream);
+/* The gate's projection (mi355_router_gate_fwd_partial, its one slice) and mi355_route_plan_stats in one launch less, the same
+ * bits, for up to 32 experts: mi355_route_gate_plan_covers.  x (T,D) fp32 or bf16, w fp32, on 16-byte boundaries; logits_TE
+ * may be NULL. */
+int mi355_route_gate_plan_covers(int x_dtype, int w_dtype, int64_t T, int64_t D, int64_t E, int64_t K, int num_groups);
+int mi355_route_gate_plan_stats(const void* x, int x_dtype, const float* w, int64_t D, const float* logit_bias, float* logits_TE,
+                           const float* expert_bias, int64_t T, int64_t E, int64_t K, int score_func,
+                           int route_norm, float route_scale, int num_groups, int num_limited,
+                           float* weights_TK, int64_t* ids_TK, int64_t lo, int64_t hi, int64_t align,
+                           int64_t tile_m, int32_t* counts_E, int32_t* seg_offsets, int32_t* seg_counts,
+                           int32_t* row_of_slot, int32_t* slot_of_row, int32_t* token_of_row,
+                           float* row_scale, int64_t row_capacity, int32_t* tile_expert, int32_t* tile_row0,
+                           int32_t* num_tiles, int64_t tile_capacity, void* workspace,
+                           const uint8_t* padding_mask_T, int32_t* valid_counts_E, float* scores_TE,
+                           float* cutoff_T, float* aux_f_E, float* aux_scale, void* aux_acc,
+                           int aux_acc_dtype, const float* aux_denominator, float aux_coeff, void* stats_workspace, void* stream);
 
 
 /*

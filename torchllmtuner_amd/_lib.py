@@ -84,6 +84,12 @@ SIGNATURES = {
         [P, I, P, P, P, L, L, L, I, I, F, I, I, P, P, L, L, L, L, P, P, P, P, P, P, P, L, P, P, P, L, P,
          P, P, P, P, P, P, P, I, P, F, P, P],
     ),
+    "mi355_route_gate_plan_covers": (I, [I, I, L, L, L, L, I]),
+    "mi355_route_gate_plan_stats": (
+        I,
+        [P, I, P, L, P, P, P, L, L, L, I, I, F, I, I, P, P, L, L, L, L, P, P, P, P, P, P, P, L, P, P, P, L, P,
+         P, P, P, P, P, P, P, I, P, F, P, P],
+    ),
     "mi355_combine_add_fwd": (I, [P, I, P, P, P, P, L, L, L, I, P]),
     "mi355_permute_rows_add_bwd": (I, [P, I, P, P, P, L, L, L, P]),
     "mi355_segments_dense": (I, [L, L, P, P, P, P, P, L, P]),

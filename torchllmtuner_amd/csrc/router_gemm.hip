@@ -16,6 +16,7 @@
 
 #include "bf16_tiles.h"
 #include "common.h"
+#include "gate_rows.h"
 #include "gemm_generic.h"
 #include "router_few.h"
 
@@ -28,23 +29,6 @@ __device__ __forceinline__ int kc_off(int row, int chunk) {
 template <int COLS>
 __device__ __forceinline__ int ks_off(int k, int chunk) {
   return k * COLS + ((chunk ^ ks_key(k)) << 3);
-}
-
-// 8 consecutive fp32 -> three 16-byte chunks of bf16 pieces (hi, mid, lo)
-__device__ __forceinline__ void split8(const f32x4& a, const f32x4& b, u32x4& hi, u32x4& mid, u32x4& lo) {
-  float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-  float r1[8], r2[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    r1[i] = v[i] - round_bf16(v[i]);
-    r2[i] = r1[i] - round_bf16(r1[i]);
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    hi[i] = pack_bf16x2(v[2 * i], v[2 * i + 1]);
-    mid[i] = pack_bf16x2(r1[2 * i], r1[2 * i + 1]);
-    lo[i] = pack_bf16x2(r2[2 * i], r2[2 * i + 1]);
-  }
 }
 
 // W (n fp32) -> out[s][n] bf16, s < nsplit
@@ -74,83 +58,17 @@ __global__ __launch_bounds__(256) void split_kernel(const float* __restrict__ w,
 // weight-splitting launch: 1 token of 2048 x 128 experts 34 -> 8 us, 1000 tokens 43 -> 12 us, 128
 // tokens of 7168 x 256 experts 131 -> 12 us (profiled inside the block, the weights from memory).  From 1024 tokens on, with widths on its grid, the
 // 128-token kernel below reads the weights four times less often and is the faster one.
-constexpr int R_BM = 32, R_BN = 32, R_WAVES = 8, R_STEP = 32;
-
-template <typename TX>
-__device__ __forceinline__ void load16_masked(const TX* p, int k, int k_end, f32x4 (&v)[4]) {
-  // fp32: four pieces of four, each inside the row or zero (D % 4 == 0)
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-    v[j] = k + 4 * j < k_end ? *reinterpret_cast<const f32x4*>(p + k + 4 * j) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-}
-__device__ __forceinline__ void load16_masked(const uint16_t* p, int k, int k_end, u32x4 (&v)[2]) {
-#pragma unroll
-  for (int j = 0; j < 2; ++j)
-    v[j] = k + 8 * j < k_end ? *reinterpret_cast<const u32x4*>(p + k + 8 * j) : u32x4{0, 0, 0, 0};
-}
-
 template <typename TX>
 __global__ __launch_bounds__(64 * R_WAVES) void gate_rows_kernel(const TX* __restrict__ x,
                                                                  const float* __restrict__ w,
                                                                  const float* __restrict__ bias,
                                                                  float* __restrict__ out, int T, int D, int E,
                                                                  int k_per_wave) {
-  constexpr bool BF = sizeof(TX) == 2;
-  __shared__ __attribute__((aligned(16))) float red[R_WAVES][4][64][4];  // [wave][q][lane][i]
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  __shared__ __attribute__((aligned(16))) float red[R_WAVES][4][64][4];
+  const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, q = tid >> 6;
   const int t0 = blockIdx.x * R_BM, n0 = blockIdx.y * R_BN;
-  const int half = lane >> 5;
-  const TX* xp = x + static_cast<int64_t>(min(t0 + (lane & 31), T - 1)) * D;
-  const float* wp = w + static_cast<int64_t>(min(n0 + (lane & 31), E - 1)) * D;
-  const int k0 = (blockIdx.z * R_WAVES + wave) * k_per_wave;
-  const int k1 = min(k0 + k_per_wave, D);
-  f32x16 acc;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
-  constexpr int B = 4;  // steps requested together: 128 of the contraction, 24 KiB (bf16 x) per wave
-  for (int kb = k0; kb < k1; kb += B * R_STEP) {
-    f32x4 wv[B][4];
-    std::conditional_t<BF, u32x4[B][2], f32x4[B][4]> xv;
-#pragma unroll
-    for (int b = 0; b < B; ++b) {
-      const int k = kb + b * R_STEP + 16 * half;
-      load16_masked(wp, k, k1, wv[b]);
-      load16_masked(xp, k, k1, xv[b]);
-    }
-#pragma unroll
-    for (int b = 0; b < B; ++b) {
-      if (kb + b * R_STEP >= k1) break;  // wave-uniform
-      if constexpr (BF) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          u32x4 hi, mid, lo;
-          split8(wv[b][2 * j], wv[b][2 * j + 1], hi, mid, lo);
-          const bf16x8 a = __builtin_bit_cast(bf16x8, xv[b][j]);
-          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, hi), a, acc, 0, 0, 0);
-          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, mid), a, acc, 0, 0, 0);
-          acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, lo), a, acc, 0, 0, 0);
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(wv[b][j][i], xv[b][j][i], acc, 0, 0, 0);
-      }
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const f32x4 v = {acc[q * 4], acc[q * 4 + 1], acc[q * 4 + 2], acc[q * 4 + 3]};
-    *reinterpret_cast<f32x4*>(red[wave][q][lane]) = v;
-  }
-  __syncthreads();
+  f32x4 v = gate_rows_tile<TX>(x, w, T, D, E, t0, n0, blockIdx.z, k_per_wave, red);
   if (tid >= 256) return;
-  // lane = token row (lane & 31); piece q = expert columns q * 8 + (lane >> 5) * 4 + 0..3
-  const int q = tid >> 6;
-  f32x4 v = *reinterpret_cast<const f32x4*>(red[0][q][lane]);
-#pragma unroll
-  for (int i = 1; i < R_WAVES; ++i) v += *reinterpret_cast<const f32x4*>(red[i][q][lane]);
   const int t = t0 + (lane & 31), n = n0 + q * 8 + half * 4;
   if (t >= T || n >= E) return;
   float* dst = out + (static_cast<int64_t>(blockIdx.z) * T + t) * E + n;
@@ -727,8 +645,7 @@ int router_fwd_partial(const void* x, int x_dtype, const float* w, const float* 
                        in_kernel_bias, partial, (int)T, (int)D, (int)E, (int)(D / splits));
     return check_launch("router_gate_fwd");
   }
-  const int64_t per_wave = (D + splits * R_WAVES - 1) / (splits * R_WAVES);
-  const int k_per_wave = (int)((per_wave + R_STEP - 1) / R_STEP * R_STEP);
+  const int k_per_wave = gate_rows_k(D, splits);
   const dim3 grid((unsigned)((T + R_BM - 1) / R_BM), (unsigned)((E + R_BN - 1) / R_BN), (unsigned)splits);
   if (x_dtype == MI355_BF16)
     hipLaunchKernelGGL(gate_rows_kernel<uint16_t>, grid, dim3(64 * R_WAVES), 0, s, static_cast<const uint16_t*>(x), w,

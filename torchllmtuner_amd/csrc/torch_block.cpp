@@ -251,26 +251,35 @@ std::tuple<Tensor, Tensor, Tensor> block_forward(const Block& b, const Stats& st
     shared_forward(b, k, y_shared, aux->stream);
   }
 
-  // router: partial logits, then selection and plan
+  // router: partial logits, then selection and plan; few experts in one launch less
   float* partial = b.splits > 1 ? static_cast<float*>(gate_work) : k.logits;
-  if (b.splits > 0)
+  const bool one_launch = mi355_route_gate_plan_covers(b.dt, b.gate_dt, b.T, b.D, b.E, c.K, (int)c.num_groups);
+  if (one_launch) {
+    // (in front of the selection, below)
+  } else if (b.splits > 0) {
     check(mi355_router_gate_fwd_partial(ptr(b.x), b.dt, fptr(b.gate_w), fptr(gate_b), partial, k.pieces, b.T, b.D, b.E,
                                         L.stream),
           "router_gate_fwd");
-  else
+  } else {
     check(mi355_router_gate_fwd(ptr(b.x), b.dt, ptr(b.gate_w), b.gate_dt, fptr(gate_b), k.logits, gate_work, b.T, b.D,
                                 b.E, L.stream),
           "router_gate_fwd");
+  }
   const uint8_t* padding = static_cast<const uint8_t*>(ptr(b.mask));
-  check(mi355_route_plan_stats(
-            partial, b.splits > 1 ? b.splits : 1, fptr(gate_b), save && b.splits > 1 ? k.logits : nullptr, fptr(expert_b),
-            b.T, b.E, c.K, (int)c.score_func, (int)c.route_norm, (float)c.route_scale, (int)c.num_groups,
-            (int)c.num_limited, k.weights, k.ids, c.lo, c.hi, c.align, b.tile_m,
-            stats ? all_counts : counts.data_ptr<int32_t>(), k.seg_offsets, k.seg_counts, k.row_of_slot, k.slot_of_row,
-            k.token_of_row, save && (b.folded || b.gather) ? k.row_scale : nullptr, b.R, k.tile_expert, k.tile_row0, k.num_tiles,
-            b.tile_cap, plan_work, padding, stats ? counts.data_ptr<int32_t>() : nullptr, scores, cutoff, k.aux_f,
-            k.aux_scale, ptr(st.aux_acc), st.aux_acc.defined() ? dtype_code(st.aux_acc) : MI355_F32, fptr(st.aux_denominator), (float)st.aux_coeff, stats_work,
-            L.stream),
+  // what both forms take behind the logits
+  auto plan = [&](auto f, auto... logits) {
+    return f(logits..., fptr(expert_b), b.T, b.E, c.K, (int)c.score_func, (int)c.route_norm, (float)c.route_scale,
+             (int)c.num_groups, (int)c.num_limited, k.weights, k.ids, c.lo, c.hi, c.align, b.tile_m,
+             stats ? all_counts : counts.data_ptr<int32_t>(), k.seg_offsets, k.seg_counts, k.row_of_slot, k.slot_of_row,
+             k.token_of_row, save && (b.folded || b.gather) ? k.row_scale : nullptr, b.R, k.tile_expert, k.tile_row0,
+             k.num_tiles, b.tile_cap, plan_work, padding, stats ? counts.data_ptr<int32_t>() : nullptr, scores, cutoff, k.aux_f,
+             k.aux_scale, ptr(st.aux_acc), st.aux_acc.defined() ? dtype_code(st.aux_acc) : MI355_F32,
+             fptr(st.aux_denominator), (float)st.aux_coeff, stats_work, L.stream);
+  };
+  check(one_launch ? plan(mi355_route_gate_plan_stats, ptr(b.x), b.dt, fptr(b.gate_w), b.D, fptr(gate_b),
+                          save ? k.logits : nullptr)
+                   : plan(mi355_route_plan_stats, partial, b.splits > 1 ? b.splits : 1, fptr(gate_b),
+                          save && b.splits > 1 ? k.logits : nullptr),
         "route_plan");
   if (st.histogram.defined())
     check(mi355_quantile_observe(scores, cutoff, fptr(expert_b), padding, st.histogram.data_ptr<int64_t>(), b.T, b.E,
