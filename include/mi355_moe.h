@@ -363,6 +363,19 @@ int mi355_route_plan_stats(const float* partial, int splits, const float* logit_
                            const uint8_t* padding_mask_T, int32_t* valid_counts_E, float* scores_TE,
                            float* cutoff_T, float* aux_f_E, float* aux_scale, void* aux_acc,
                            int aux_acc_dtype, const float* aux_denominator, float aux_coeff, void* stats_workspace, void* stream);
+/* Forward of a handful of tokens without a plan, bf16 (mi355_choice_covers): row t*K + k is choice k of token t.
+ * mi355_choice_gateup_fwd selects (partial, splits, logit_bias as in mi355_route_plan) and writes h (T*K,F) of the choices in
+ * [lo,hi), weights_TK, ids_TK (local expert or -1) and counts_E; mi355_choice_down_fwd projects down and combines (addend (T,D)
+ * or NULL).  The bits of mi355_route_plan, mi355_grouped_swiglu_fwd and mi355_combine_add_fwd. */
+int mi355_choice_covers(int64_t T, int64_t D, int64_t F, int64_t E, int64_t K, int num_groups);
+int mi355_choice_gateup_fwd(const float* partial, int splits, const float* logit_bias, const float* expert_bias,
+                            int64_t T, int64_t E, int64_t K, int score_func, int route_norm, float route_scale,
+                            int num_groups, int num_limited, int64_t lo, int64_t hi, const void* x, const void* w1,
+                            const void* w3, void* h, float* weights_TK, int32_t* ids_TK, int32_t* counts_E,
+                            int64_t D, int64_t F, void* stream);
+int mi355_choice_down_fwd(const void* h, const void* w2, const float* weights_TK, const int32_t* ids_TK,
+                          const void* addend, void* out, int64_t T, int64_t K, int64_t El, int64_t D, int64_t F,
+                          int round_terms, void* stream);
 /* The gate's projection (mi355_router_gate_fwd_partial, its one slice) and mi355_route_plan_stats in one launch less, the same
  * bits, for up to 32 experts: mi355_route_gate_plan_covers.  x (T,D) fp32 or bf16, w fp32, on 16-byte boundaries; logits_TE
  * may be NULL. */

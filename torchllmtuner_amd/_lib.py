@@ -84,6 +84,12 @@ SIGNATURES = {
         [P, I, P, P, P, L, L, L, I, I, F, I, I, P, P, L, L, L, L, P, P, P, P, P, P, P, L, P, P, P, L, P,
          P, P, P, P, P, P, P, I, P, F, P, P],
     ),
+    "mi355_choice_covers": (I, [L, L, L, L, L, I]),
+    "mi355_choice_gateup_fwd": (
+        I,
+        [P, I, P, P, L, L, L, I, I, F, I, I, L, L, P, P, P, P, P, P, P, L, L, P],
+    ),
+    "mi355_choice_down_fwd": (I, [P, P, P, P, P, P, L, L, L, L, L, I, P]),
     "mi355_route_gate_plan_covers": (I, [I, I, L, L, L, L, I]),
     "mi355_route_gate_plan_stats": (
         I,

@@ -17,6 +17,7 @@
 
 #include "bf16_tiles.h"
 #include "common.h"
+#include "select_rows.h"
 
 namespace mi355 {
 namespace {
@@ -38,17 +39,13 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t few_rsrc(const void* base) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, -1, 0x00020000);
 }
 
-template <bool GATEUP>
-__global__ __launch_bounds__(256, 4) void few_rows_kernel(FewArgs p) {
+// Column group cg of the product of expert e with rows row0 .. row0 + rows - 1; a row is source(row) of a, or itself.
+template <bool GATEUP, typename Source>
+__device__ __forceinline__ void few_rows_tile(const FewArgs& p, int e, int row0, int rows, int cg, bool through,
+                                              Source source, f32x4 (&part)[4][2][64]) {
   constexpr int kPairs = 4;  // 64-wide contraction steps requested together
-  __shared__ f32x4 part[4][2][64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, g = lane >> 4;
-  const int t = blockIdx.x / p.col_groups, cg = blockIdx.x - t * p.col_groups;
-  if (t >= *p.num_tiles) return;
-  const int e = __builtin_amdgcn_readfirstlane(p.tile_expert[t]), row0 = __builtin_amdgcn_readfirstlane(p.tile_row0[t]);
-  const int cnt = p.seg_counts[e], seg0 = p.seg_offsets[e];
-  const int rows = min(even_tile_rows(cnt, 256), seg0 + cnt - row0);
   const int K = p.K, N = p.N;
   // this wave's share of the contraction
   const int steps = K >> 6, s0 = steps * wave >> 2, s1 = steps * (wave + 1) >> 2;
@@ -60,7 +57,7 @@ __global__ __launch_bounds__(256, 4) void few_rows_kernel(FewArgs p) {
   const uint32_t off1 = GATEUP ? off0 : off0 + static_cast<uint32_t>(32 * K);
   for (int sub = 0; sub < rows; sub += 16) {
     const int row = row0 + min(sub + r16, rows - 1);
-    const int index = p.a_src ? p.a_src[row] : row;
+    const int index = through ? source(row) : row;
     f32x4 acc0 = {0, 0, 0, 0}, acc1 = {0, 0, 0, 0};
     u32x4 b0[kPairs][2], b1[kPairs][2], a[kPairs][2];
     uint32_t offA;
@@ -88,7 +85,7 @@ __global__ __launch_bounds__(256, 4) void few_rows_kernel(FewArgs p) {
 #pragma unroll
     for (int i = 0; i < kPairs; ++i) request_w(i, min(s0 + i, s1 - 1));
     __builtin_amdgcn_sched_barrier(0);
-    const int src = p.a_src ? min(max(index, 0), p.a_rows - 1) : row;
+    const int src = through ? min(max(index, 0), p.a_rows - 1) : row;
     offA = (static_cast<uint32_t>(src) * static_cast<uint32_t>(K) + g * 16) * 2u;
 #pragma unroll
     for (int i = 0; i < kPairs; ++i) request_a(i, min(s0 + i, s1 - 1));
@@ -148,6 +145,178 @@ __global__ __launch_bounds__(256, 4) void few_rows_kernel(FewArgs p) {
   }
 }
 
+template <bool GATEUP>
+__global__ __launch_bounds__(256, 4) void few_rows_kernel(FewArgs p) {
+  __shared__ f32x4 part[4][2][64];
+  const int t = blockIdx.x / p.col_groups, cg = blockIdx.x - t * p.col_groups;
+  if (t >= *p.num_tiles) return;
+  const int e = __builtin_amdgcn_readfirstlane(p.tile_expert[t]), row0 = __builtin_amdgcn_readfirstlane(p.tile_row0[t]);
+  const int cnt = p.seg_counts[e], seg0 = p.seg_offsets[e];
+  const int rows = min(even_tile_rows(cnt, 256), seg0 + cnt - row0);
+  few_rows_tile<GATEUP>(p, e, row0, rows, cg, p.a_src != nullptr, [&](int row) { return p.a_src[row]; }, part);
+}
+
+// ---- a handful of tokens, forward only: no plan ---------------------------------------------------
+// One or a few tokens' choices are K rows each, nearly all of different experts, and grouping them saves nothing.  Row t K + k is
+// choice k of token t: the first launch selects in every workgroup that needs the choice (a row of 16 lanes, about a
+// microsecond, against a launch of its own) and forms gate and up of its row; the second takes the
+// down projection of all K choices of a token for 16 columns and combines them, waves along choices and halves of
+// the contraction.  With the gate's projection three launches instead of five; every sum in the order of the grouped kernels, the
+// same bits.  Up to four tokens (torch_block.cpp), all experts here: block forward of 128 experts of 2048 x 768, eight a token, us,
+// grouped / this: one token 39.7 / 28.7, 2 49 / 40, 3 60 / 55, 4 72 / 68, 6 96 / 99, 8 111 / 125 -- the experts that tokens share are read
+// once per token here.  On one rank's share (32 of 256 experts) seven in eight workgroups select for nothing: four tokens 118 / 165.
+struct ChoiceIn {
+  const float *partial, *logit_bias;  // (splits, T, E)
+  int splits, T, lo, hi;
+  SelectArgs sel;
+  float* weights;  // (T, K)
+  int32_t* ids;    // (T, K): local expert, -1 elsewhere
+  int32_t* counts; // (E)
+};
+
+// token t's choices, by a row of 16 lanes each (lane l < K: choice l)
+template <int VPR, bool FULL>
+__device__ __forceinline__ RowChoice choose(const ChoiceIn& c, int t, int l) {
+  const int E = c.sel.E;
+  float x[VPR], s[VPR], cutoff;
+  load_row<VPR, FULL>(c.partial + static_cast<int64_t>(t) * E, l, E, x);
+  for (int z = 1; z < c.splits; ++z) {
+    float y[VPR];
+    load_row<VPR, FULL>(c.partial + (static_cast<int64_t>(z) * c.T + t) * E, l, E, y);
+#pragma unroll
+    for (int j = 0; j < VPR; ++j) x[j] += y[j];
+  }
+  if (c.splits > 1 && c.logit_bias) {
+#pragma unroll
+    for (int j = 0; j < VPR; ++j)
+      if (FULL || l * VPR + j < E) x[j] += c.logit_bias[l * VPR + j];
+  }
+  return select_row<VPR, FULL>(c.sel, x, l, false, false, s, cutoff);
+}
+
+constexpr int kChoiceTokens = 16;  // a row of 16 lanes each in one workgroup of four waves
+
+template <int VPR, bool FULL>
+__global__ __launch_bounds__(256, 4) void choice_gateup_kernel(FewArgs p, ChoiceIn c) {
+  __shared__ f32x4 part[4][2][64];
+  const int lane = threadIdx.x & 63, K = c.sel.K;
+  const int row = blockIdx.x / p.col_groups, cg = blockIdx.x - row * p.col_groups;
+  if (row == c.T * K) {
+    // the last workgroup: everyone's choices for the second launch, and the experts' loads
+    int* count = reinterpret_cast<int*>(part);
+    for (int e = threadIdx.x; e < c.sel.E; e += 256) count[e] = 0;
+    __syncthreads();
+    const int t = threadIdx.x >> 4, l = lane & 15;
+    const RowChoice ch = choose<VPR, FULL>(c, min(t, c.T - 1), l);
+    if (t < c.T && l < K) {
+      c.weights[t * K + l] = ch.weight;
+      c.ids[t * K + l] = ch.id >= c.lo && ch.id < c.hi ? ch.id - c.lo : -1;
+      if (ch.id >= 0 && ch.id < c.sel.E) atomicAdd(&count[ch.id], 1);
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < c.sel.E; e += 256) c.counts[e] = count[e];
+    return;
+  }
+  const int t = row / K;
+  const RowChoice ch = choose<VPR, FULL>(c, t, lane & 15);
+  const int id = __builtin_amdgcn_readlane(ch.id, row - t * K);
+  if (id < c.lo || id >= c.hi) return;  // (the same for the whole workgroup)
+  few_rows_tile<true>(p, id - c.lo, row, 1, cg, true, [&](int) { return t; }, part);
+}
+
+struct ChoiceOut {
+  const uint16_t *h, *w2, *addend;  // (T K, F), (El, D, F), (T, D) or null
+  uint16_t* out;
+  const float* weights;
+  const int32_t* ids;
+  int K, D, F, El, round_terms;
+};
+
+// A workgroup is eight columns of one token; a wave takes one choice and two quarters of the contraction at a time, in one
+// MFMA: operand rows 0-7 are the columns (and the choice's row) over quarter `pair`, rows 8-15 the same over quarter pair + 2, and of the
+// result the two diagonal blocks are what is wanted.  One token, eight choices of 2048 x 768 (25 MB): 7.7 us, where 16 columns
+// a workgroup, half the chip, took 12.9 and the grouped product with the combine behind it 11.4.
+constexpr int kChoiceCols = 8, kChoiceWaves = 16;
+
+__global__ __launch_bounds__(64 * kChoiceWaves) void choice_down_kernel(ChoiceOut p) {
+  constexpr int kAhead = 4;  // 64-wide steps requested together
+  __shared__ float part[16][4][kChoiceCols];  // choice, quarter of the contraction, column
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+  const int groups = p.D / kChoiceCols, t = blockIdx.x / groups, n0 = (blockIdx.x - t * groups) * kChoiceCols;
+  const int r8 = lane & 7, second = lane >> 3 & 1, g = lane >> 4;
+  const int K = p.K, F = p.F, steps = F >> 6;
+  const int my_e = lane < K ? p.ids[t * K + lane] : -1;
+  const float my_w = lane < K ? p.weights[t * K + lane] : 0.0f;
+  for (int u = wave; u < 2 * K; u += waves) {
+    const int k = u >> 1, pair = u & 1;
+    const int e = __builtin_amdgcn_readlane(my_e, k);
+    if (e < 0 || e >= p.El) continue;
+    const auto rsB = few_rsrc(p.w2 + (static_cast<int64_t>(e) * p.D + n0) * F), rsA = few_rsrc(p.h + (static_cast<int64_t>(t) * K + k) * F);
+    // this lane's quarter
+    const int q = pair + 2 * second, s0 = steps * q >> 2, s1 = steps * (q + 1) >> 2;
+    const int n = max((steps * (pair + 1) >> 2) - (steps * pair >> 2), (steps * (pair + 3) >> 2) - (steps * (pair + 2) >> 2));
+    const uint32_t offB = static_cast<uint32_t>(r8 * F + g * 16) * 2u, offA = static_cast<uint32_t>(g * 16) * 2u;
+    f32x4 acc = {0, 0, 0, 0};
+    u32x4 b[kAhead][2], a[kAhead][2];
+    auto request = [&](int i, int s) {
+      const uint32_t at = static_cast<uint32_t>(min(s0 + s, s1 - 1)) * 128u;  // (the shorter quarter's last step again: zeroed below)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        b[i][h] = __builtin_amdgcn_raw_buffer_load_b128(rsB, offB + at + 16 * h, 0, 0);
+        a[i][h] = __builtin_amdgcn_raw_buffer_load_b128(rsA, offA + at + 16 * h, 0, 0);
+      }
+    };
+    auto multiply = [&](int i, int s) {
+      const bool live = s0 + s < s1;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const u32x4 zero = {0, 0, 0, 0};
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, live ? b[i][h] : zero),
+                                                      __builtin_bit_cast(bf16x8, live ? a[i][h] : zero), acc, 0, 0, 0);
+      }
+    };
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) request(i, min(i, n - 1));
+    for (int s = 0; s < n; s += kAhead) {
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) {
+        if (s + i < n) multiply(i, s + i);
+        if (s + i + kAhead < n) request(i, s + i + kAhead);
+      }
+    }
+    // lane = activation row lane & 15, its four values = weight rows 4 g ..: rows 0 (columns 0-7) and 8 (columns 8-15)
+    if (r8 == 0 && (g >> 1) == second) *reinterpret_cast<f32x4*>(&part[k][q][4 * (g & 1)]) = acc;
+  }
+  if (wave != 0) {
+    __syncthreads();
+    return;
+  }
+  // the token's terms in ascending order of their experts, as the combine visits their rows
+  const bool here = my_e >= 0 && my_e < p.El;
+  int pos = 0;
+  for (int k = 0; k < K; ++k) {
+    const int e = __builtin_amdgcn_readlane(my_e, k);
+    pos += e >= 0 && e < my_e ? 1 : 0;
+  }
+  const int terms = __popcll(__ballot(here));
+  const int to = (here ? pos : 63) << 2;
+  const int o_k = __builtin_amdgcn_ds_permute(to, lane);
+  const float o_w = __int_as_float(__builtin_amdgcn_ds_permute(to, __float_as_int(my_w)));
+  __syncthreads();
+  float sum = 0.0f;
+  for (int n = 0; n < terms; ++n) {
+    const int k = __builtin_amdgcn_readlane(o_k, n);
+    const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(o_w), n));
+    const float y = round_bf16(((part[k][0][r8] + part[k][1][r8]) + part[k][2][r8]) + part[k][3][r8]);
+    const float term = y * w;
+    sum += p.round_terms ? round_bf16(term) : term;
+  }
+  if (lane >= kChoiceCols) return;
+  const int64_t o = static_cast<int64_t>(t) * p.D + n0 + r8;
+  if (p.addend) sum = round_bf16(sum) + bf16_to_f32(p.addend[o]);
+  p.out[o] = f32_to_bf16(sum);
+}
+
 }  // namespace
 
 // gate/up (stage 1) or down (stage 2) of the forward; the arguments of bf16_grouped_fwd.
@@ -169,3 +338,57 @@ int few_rows_fwd(int stage, const void* a, const int32_t* a_src, int64_t a_rows,
 }
 
 }  // namespace mi355
+
+using namespace mi355;
+
+namespace mi355 {
+bool bf16_fast_path_ok(int64_t D, int64_t F);
+}
+
+extern "C" int mi355_choice_covers(int64_t T, int64_t D, int64_t F, int64_t E, int64_t K, int num_groups) {
+  return T >= 1 && T <= kChoiceTokens && E >= 1 && K >= 1 && K <= E && bf16_fast_path_ok(D, F) &&
+                 T * K * std::max(D, F) * 2 < (1ll << 31) && select_row_covers(E, K, num_groups, MI355_SELECT_TOPK)
+             ? 1 : 0;
+}
+
+extern "C" int mi355_choice_gateup_fwd(const float* partial, int splits, const float* logit_bias, const float* expert_bias,
+                                       int64_t T, int64_t E, int64_t K, int score_func, int route_norm, float route_scale,
+                                       int num_groups, int num_limited, int64_t lo, int64_t hi, const void* x, const void* w1,
+                                       const void* w3, void* h, float* weights_TK, int32_t* ids_TK, int32_t* counts_E,
+                                       int64_t D, int64_t F, void* stream) {
+  if (!mi355_choice_covers(T, D, F, E, K, num_groups))
+    return fail(MI355_EUNSUP, "choice_gateup_fwd: not covered; use mi355_route_plan and mi355_grouped_swiglu_fwd");
+  MI355_REQUIRE(score_func >= 0 && score_func <= 2, "choice_gateup_fwd: unknown score_func %d", score_func);
+  if (num_groups > 0)
+    MI355_REQUIRE(E % num_groups == 0 && E / num_groups >= 2 && num_limited >= 1 && num_limited <= num_groups &&
+                      K <= (int64_t)num_limited * (E / num_groups),
+                  "choice_gateup_fwd: bad group config G=%d L=%d", num_groups, num_limited);
+  MI355_REQUIRE(0 <= lo && lo < hi && hi <= E, "choice_gateup_fwd: bad local range [%lld,%lld)", (long long)lo, (long long)hi);
+  MI355_REQUIRE(partial && splits >= 1 && x && w1 && w3 && h && weights_TK && ids_TK && counts_E &&
+                    aligned16({partial, x, w1, w3, h}),
+                "choice_gateup_fwd: null or misaligned pointer");
+  FewArgs p{};
+  p.a = (const uint16_t*)x; p.a_rows = (int)T;
+  p.b0 = (const uint16_t*)w1; p.b1 = (const uint16_t*)w3; p.out = (uint16_t*)h;
+  p.K = (int)D; p.N = (int)F; p.col_groups = (int)(F / 16);
+  const ChoiceIn c{partial, logit_bias, splits, (int)T, (int)lo, (int)hi,
+                   SelectArgs{expert_bias, (int)E, (int)K, score_func, route_norm, route_scale, num_groups, num_limited},
+                   weights_TK, ids_TK, counts_E};
+  with_row_shape(E, [&](auto vpr, auto full) {
+    hipLaunchKernelGGL((choice_gateup_kernel<decltype(vpr)::value, decltype(full)::value>),
+                       dim3((unsigned)(T * K * p.col_groups + 1)), dim3(256), 0, as_stream(stream), p, c);
+  });
+  return check_launch("choice_gateup");
+}
+
+extern "C" int mi355_choice_down_fwd(const void* h, const void* w2, const float* weights_TK, const int32_t* ids_TK,
+                                     const void* addend, void* out, int64_t T, int64_t K, int64_t El, int64_t D, int64_t F,
+                                     int round_terms, void* stream) {
+  MI355_REQUIRE(T >= 1 && T <= kChoiceTokens && K >= 1 && K <= 16 && El >= 1 && bf16_fast_path_ok(D, F), "choice_down_fwd: bad shape");
+  MI355_REQUIRE(h && w2 && weights_TK && ids_TK && out && aligned16({h, w2}), "choice_down_fwd: null or misaligned pointer");
+  const ChoiceOut p{(const uint16_t*)h, (const uint16_t*)w2, (const uint16_t*)addend, (uint16_t*)out, weights_TK, ids_TK,
+                    (int)K, (int)D, (int)F, (int)El, round_terms};
+  const int waves = (int)std::min<int64_t>(kChoiceWaves, 2 * K);
+  hipLaunchKernelGGL(choice_down_kernel, dim3((unsigned)(T * (D / kChoiceCols))), dim3(64 * waves), 0, as_stream(stream), p);
+  return check_launch("choice_down");
+}

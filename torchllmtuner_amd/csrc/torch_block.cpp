@@ -153,17 +153,19 @@ struct Kept {
       h = c.take(b.R * b.F, item);
       y = c.take(b.R * b.D, item);
     }
-    if (b.Fs > 0) {
-      s_offsets = c.take<int32_t>(2);
-      s_counts = c.take<int32_t>(2);
-      s_expert = c.take<int32_t>(b.shared_cap);
-      s_row0 = c.take<int32_t>(b.shared_cap);
-      s_num = c.take<int32_t>(1);
-      s_h = c.take(b.T * b.Fs, item);
-      if (save || !b.shared_folded) {
-        s_gate = c.take(b.T * b.Fs, item);
-        s_up = c.take(b.T * b.Fs, item);
-      }
+    if (b.Fs > 0) layout_shared(c, b, save);
+  }
+  void layout_shared(Carver& c, const Block& b, bool save) {
+    const int64_t item = b.dt == MI355_F32 ? 4 : 2;
+    s_offsets = c.take<int32_t>(2);
+    s_counts = c.take<int32_t>(2);
+    s_expert = c.take<int32_t>(b.shared_cap);
+    s_row0 = c.take<int32_t>(b.shared_cap);
+    s_num = c.take<int32_t>(1);
+    s_h = c.take(b.T * b.Fs, item);
+    if (save || !b.shared_folded) {
+      s_gate = c.take(b.T * b.Fs, item);
+      s_up = c.take(b.T * b.Fs, item);
     }
   }
 };
@@ -200,6 +202,57 @@ void shared_forward(const Block& b, const Kept& k, void* y, void* stream) {
                                  k.s_expert, k.s_row0, k.s_num, b.shared_cap, k.s_gate, k.s_up, k.s_h, y, 1, b.D, b.Fs,
                                  b.T, stream),
         "shared expert");
+}
+
+// The forward of a handful of tokens that nobody differentiates and no statistics hang on, without a plan: (output, counts per
+// expert).  Four tokens, all experts here: grouped_few.hip has both sides measured.
+bool few_choices(const Block& b, const Stats& st) {
+  return b.dt == MI355_BF16 && b.folded && b.splits > 0 && b.piece_bytes == 0 && b.c.align == 1 && !b.mask.defined() && !b.c.aux &&
+         !st.histogram.defined() && b.T <= 4 && b.c.lo == 0 && b.c.hi == b.E && mi355_choice_covers(b.T, b.D, b.F, b.E, b.c.K, (int)b.c.num_groups);
+}
+
+std::tuple<Tensor, Tensor> choices_forward(const Block& b) {
+  Launch L(b.x);
+  const Config& c = b.c;
+  const auto opts = b.x.options();
+  const hipStream_t main = static_cast<hipStream_t>(L.stream);
+  Tensor counts = at::empty({b.E}, opts.dtype(at::kInt));
+  Tensor out = at::empty({b.T, b.D}, opts);
+  Kept k;  // (the shared expert's part)
+  float *partial = nullptr, *weights = nullptr;
+  int32_t* ids = nullptr;
+  void *h = nullptr, *y_shared = nullptr;
+  Tensor scratch = carve(b.x, [&](Carver& cv) {
+    partial = cv.take<float>(b.splits * b.T * b.E);
+    weights = cv.take<float>(b.N);
+    ids = cv.take<int32_t>(b.N);
+    h = cv.take(b.N * b.F, 2);
+    if (b.Fs > 0) {
+      y_shared = cv.take(b.T * b.D, 2);
+      k.layout_shared(cv, b, false);
+    }
+  });
+  Tensor gate_b, expert_b;
+  if (b.gate_b.defined()) gate_b = cf(b.gate_b);
+  if (b.expert_b.defined()) expert_b = cf(b.expert_b);
+  SideStream* aux = b.Fs > 0 && c.overlap ? side_stream(b.x.device().index(), main, 1) : nullptr;
+  Fork shared(aux, main);
+  if (aux) {
+    shared.start();
+    shared_forward(b, k, y_shared, aux->stream);
+  }
+  check(mi355_router_gate_fwd_partial(ptr(b.x), b.dt, fptr(b.gate_w), fptr(gate_b), partial, nullptr, b.T, b.D, b.E, L.stream),
+        "router_gate_fwd");
+  check(mi355_choice_gateup_fwd(partial, b.splits, fptr(gate_b), fptr(expert_b), b.T, b.E, c.K, (int)c.score_func,
+                                (int)c.route_norm, (float)c.route_scale, (int)c.num_groups, (int)c.num_limited, c.lo, c.hi,
+                                ptr(b.x), ptr(b.w1), ptr(b.w3), h, weights, ids, counts.data_ptr<int32_t>(), b.D, b.F, L.stream),
+        "choice_gateup_fwd");
+  if (b.Fs > 0 && !aux) shared_forward(b, k, y_shared, L.stream);
+  shared.join();
+  check(mi355_choice_down_fwd(h, ptr(b.w2), weights, ids, y_shared, ptr(out), b.T, c.K, b.El, b.D, b.F, (int)c.round_terms,
+                              L.stream),
+        "choice_down_fwd");
+  return {out, counts};
 }
 
 // (output, counts per expert, what the backward reads)
@@ -631,6 +684,7 @@ std::pair<Block, Stats> block_of(BLOCK_PARAMS) {
 
 std::tuple<Tensor, Tensor> moe_block(BLOCK_PARAMS) {
   const auto [b, st] = block_of(BLOCK_ARGS);
+  if (few_choices(b, st)) return choices_forward(b);
   auto [out, counts, kept] = block_forward(b, st, false);
   return {out, counts};
 }
