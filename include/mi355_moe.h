@@ -549,6 +549,16 @@ int mi355_grouped_swiglu_combine_bwd(const void* dout, const void* x, const int3
                                      void* dw1, void* dw3, void* dw2, int64_t El, int64_t D,
                                      int64_t F, int64_t row_capacity, int stages, void* stream);
 /*
+ * mi355_permute_rows_add_bwd and mi355_router_gate_add_bwd in one launch (and the sum of dw's slices), the same bits: dx =
+ * dlogits . w + (the sum of drows over a token's K <= 16 slots + addend).  dw, addend, pieces may be NULL; w fp32.
+ * mi355_router_gate_sum_bwd_covers: bf16 tokens, D and E multiples of 64.
+ */
+int mi355_router_gate_sum_bwd_covers(int x_dtype, int w_dtype, int64_t D, int64_t E, int64_t K);
+int mi355_router_gate_sum_bwd(const float* dlogits, const void* x, int x_dtype, const float* w, const void* pieces,
+                              const void* drows, const int32_t* row_of_slot, int64_t row_capacity, int64_t K,
+                              const void* addend, void* dx, float* dw, void* workspace, int64_t T, int64_t D,
+                              int64_t E, void* stream);
+/*
  * The end of a block's backward with up to 32 experts and a fp32 gate weight (mi355_router_gate_rows_bwd_covers), in one launch:
  * dx = dlogits . w + (the sum of drows over a token's K slots + addend), the bits of mi355_permute_rows_add_bwd and
  * mi355_router_gate_add_bwd, and dw = the sum of the slices that mi355_grouped_gather_bwd left in dw_partial.  dx, dw, addend

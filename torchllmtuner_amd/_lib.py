@@ -70,6 +70,8 @@ SIGNATURES = {
     "mi355_router_gate_add_bwd": (I, [P, P, I, P, I, P, P, P, P, P, L, L, L, P]),
     "mi355_router_select_dots_bwd": (I, [P, P, P, L, P, L, P, P, P, P, L, L, L, I, I, F, P]),
     "mi355_router_select_rows_bwd": (I, [P, P, P, P, I, P, L, L, P, P, P, P, L, L, L, I, I, F, P]),
+    "mi355_router_gate_sum_bwd_covers": (I, [I, I, L, L, L]),
+    "mi355_router_gate_sum_bwd": (I, [P, P, I, P, P, P, P, L, L, P, P, P, P, L, L, L, P]),
     "mi355_router_gate_rows_bwd_covers": (I, [I, I, L, L]),
     "mi355_router_gate_rows_bwd": (I, [P, I, P, P, P, L, L, P, P, P, P, L, L, L, P]),
     "mi355_grouped_gather_covers": (I, [I, L, L, L, L]),

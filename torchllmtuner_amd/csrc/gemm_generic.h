@@ -52,6 +52,14 @@ dim3 gemm_grid_kseg(int M, int N, int El);
 int launch_splitk_reduce(const float* partial, void* out, int out_dtype, int64_t MN,
                          int ksplit, hipStream_t stream);
 
+// What a router's input gradient is added to (all null: nothing): `rows`, the experts' input gradients, summed over a token's K <= 16
+// slots, and `addend`, each sum rounded.
+struct RowSum {
+  const void* addend = nullptr;
+  const void* rows = nullptr;
+  const int32_t* row_of_slot = nullptr;
+  int64_t K = 0, row_capacity = 0;
+};
 // Router projections (router_gemm.hip).  Backward: three bf16 MFMAs per fp32 product, for bf16
 // tokens, fp32 weights, D and E multiples of 64.
 bool router_x3_ok(int x_dtype, int w_dtype, int64_t D, int64_t E);
@@ -74,7 +82,7 @@ int router_fwd_partial(const void* x, int x_dtype, const float* w, const float* 
                        int64_t T, int64_t D, int64_t E, hipStream_t s);
 int router_logits_reduce(const float* partial, const float* bias, float* logits, int64_t T, int64_t E, int splits,
                          hipStream_t s);
-int router_x3_bwd(const float* dlogits, const void* x, const float* w, const void* pieces, const void* addend,
+int router_x3_bwd(const float* dlogits, const void* x, const float* w, const void* pieces, const RowSum& sum,
                   void* dx, float* dw, void* workspace, int64_t T, int64_t D, int64_t E, hipStream_t s);
 
 }  // namespace mi355

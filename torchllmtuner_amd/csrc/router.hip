@@ -523,7 +523,7 @@ extern "C" int mi355_router_gate_add_bwd(const float* dlogits, const void* x, in
   const bool vec = workspace && aligned16({dlogits, x, w, pieces, addend, dx, dw, workspace});
   if (vec && router_x3_ok(x_dtype, w_dtype, D, E)) {
     MI355_REQUIRE(dlogits && w && (x || !dw), "router_gate_bwd: null pointer");
-    return router_x3_bwd(dlogits, x, static_cast<const float*>(w), pieces, addend, dx, static_cast<float*>(dw),
+    return router_x3_bwd(dlogits, x, static_cast<const float*>(w), pieces, RowSum{addend}, dx, static_cast<float*>(dw),
                          workspace, T, D, E, s);
   }
   if (vec && T > 0 && router_few_ok(x_dtype, w_dtype, D, E) && (dx || dw)) {
@@ -557,6 +557,25 @@ extern "C" int mi355_router_gate_add_bwd(const float* dlogits, const void* x, in
       return launch_splitk_reduce(static_cast<const float*>(workspace), dw, w_dtype, E * D, split, s);
   }
   return MI355_OK;
+}
+
+extern "C" int mi355_router_gate_sum_bwd_covers(int x_dtype, int w_dtype, int64_t D, int64_t E, int64_t K) {
+  return E >= 1 && K >= 1 && K <= 16 && router_x3_ok(x_dtype, w_dtype, D, E) ? 1 : 0;
+}
+
+extern "C" int mi355_router_gate_sum_bwd(const float* dlogits, const void* x, int x_dtype, const float* w, const void* pieces,
+                                         const void* drows, const int32_t* row_of_slot, int64_t row_capacity, int64_t K,
+                                         const void* addend, void* dx, float* dw, void* workspace, int64_t T, int64_t D,
+                                         int64_t E, void* stream) {
+  MI355_REQUIRE(T >= 1 && T < (1ll << 31) && D >= 1 && D < (1ll << 31) && row_capacity >= 0 && row_capacity < (1ll << 31),
+                "router_gate_sum_bwd: bad shape");
+  if (!mi355_router_gate_sum_bwd_covers(x_dtype, MI355_F32, D, E, K))
+    return fail(MI355_EUNSUP, "router_gate_sum_bwd: not covered; use mi355_permute_rows_add_bwd and mi355_router_gate_add_bwd");
+  MI355_REQUIRE(dlogits && x && w && drows && row_of_slot && dx && workspace &&
+                    aligned16({dlogits, x, w, pieces, drows, addend, dx, dw, workspace}),
+                "router_gate_sum_bwd: null or misaligned pointer");
+  const RowSum sum{addend, drows, row_of_slot, K, row_capacity};
+  return router_x3_bwd(dlogits, x, w, pieces, sum, dx, dw, workspace, T, D, E, as_stream(stream));
 }
 
 extern "C" int mi355_router_gate_rows_bwd_covers(int x_dtype, int w_dtype, int64_t D, int64_t E) {

@@ -224,20 +224,38 @@ __global__ __launch_bounds__(256) void logits_reduce_kernel(const float* __restr
 // Tile 128 tokens x 128 columns, 8 waves as 2 x 4, each 64 x 32.  Per K step of 64
 // experts: dlogits tile split on the fly into hi / mid (KC), W hi / mid tiles KS.
 constexpr int X_BM = 128, X_BN = 128, X_NT = 512;
+constexpr int X_ELEMS = 2 * X_BM * BK + 2 * BK * X_BN;  // LDS of a tile: 64 KiB
 
-__global__ __launch_bounds__(X_NT, 2) void gate_dx_kernel(const float* __restrict__ dlogits,
-                                                         const uint16_t* __restrict__ ws,
-                                                         const uint16_t* __restrict__ addend,
-                                                         uint16_t* __restrict__ dx, int T, int D, int E) {
-  extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
+// the sums of two bf16 pairs, rounded
+__device__ __forceinline__ uint32_t add_bf16x2(uint32_t a, uint32_t b) {
+  return pack_bf16x2(__uint_as_float(a << 16) + __uint_as_float(b << 16),
+                     __uint_as_float(a & 0xffff0000u) + __uint_as_float(b & 0xffff0000u));
+}
+
+// What comes in front of the product: an addend, and (ROWS) the sum of the experts' input gradients over a token's K slots in
+// ascending order, as permute_rows_bwd forms it.
+struct GateSum {
+  const uint16_t *addend, *rows;
+  const int32_t* row_of_slot;
+  int K, row_capacity;
+};
+constexpr int kMaxSumK = 16;
+
+// Tile `part` of dx, column tiles of a row tile one after the other: together they read whole rows, where all row tiles of one
+// column tile would read pieces a power of two apart, few memory channels at a time.
+template <bool ROWS>
+__device__ __forceinline__ void gate_dx_tile(const float* __restrict__ dlogits, const uint16_t* __restrict__ ws,
+                                             const GateSum& g, uint16_t* __restrict__ dx, int T, int D, int E, int part,
+                                             uint16_t* smem) {
   uint16_t* A_hi = smem;                    // [128][64] KC
   uint16_t* A_mid = A_hi + X_BM * BK;
   uint16_t* B_hi = A_mid + X_BM * BK;       // [64][128] KS
   uint16_t* B_mid = B_hi + BK * X_BN;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = (wave >> 2) * 64, wn = (wave & 3) * 32;
-  const int t0 = blockIdx.x * X_BM;
-  const int n0 = min(static_cast<int>(blockIdx.y) * X_BN, D - X_BN);  // D >= 128: a last tile starts early
+  const int col_tiles = (D + X_BN - 1) / X_BN;
+  const int t0 = part / col_tiles * X_BM;
+  const int n0 = min(part % col_tiles * X_BN, D - X_BN);  // D >= 128: a last tile starts early
   const int64_t ED = static_cast<int64_t>(E) * D;
   f32x16 acc[2];
 #pragma unroll
@@ -263,6 +281,46 @@ __global__ __launch_bounds__(X_NT, 2) void gate_dx_kernel(const float* __restric
     }
   };
   fetch(0);
+  // this thread's pieces of the output: row (tid >> 4) + 32 i, columns 8 (tid & 15) ..
+  const int o_row = tid >> 4, o_col = n0 + (tid & 15) * 8;
+  constexpr int kOut = X_BM * X_BN / 8 / X_NT;  // 4
+  u32x4 front[ROWS ? kOut : 1];
+  if constexpr (ROWS) {
+    int32_t* slots = reinterpret_cast<int32_t*>(smem + X_ELEMS);  // [128][K]
+    for (int i = tid; i < X_BM * g.K; i += X_NT) slots[i] = t0 + i / g.K < T ? g.row_of_slot[static_cast<int64_t>(t0) * g.K + i] : -1;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kOut; ++i) {
+      const int r = o_row + 32 * i;
+      float sum[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) sum[j] = 0.0f;
+      constexpr int B = 8;  // rows requested together
+      for (int k0 = 0; k0 < g.K; k0 += B) {
+        uint4 v[B];
+#pragma unroll
+        for (int k = 0; k < B; ++k) {
+          const int row = k0 + k < g.K ? slots[r * g.K + min(k0 + k, g.K - 1)] : -1;
+          v[k] = row >= 0 && row < g.row_capacity
+                     ? load_stream(reinterpret_cast<const uint4*>(g.rows + static_cast<int64_t>(row) * D + o_col))
+                     : make_uint4(0, 0, 0, 0);
+        }
+#pragma unroll
+        for (int k = 0; k < B; ++k) {
+          const uint32_t w[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
+#pragma unroll
+          for (int j = 0; j < 8; ++j) sum[j] += __uint_as_float(j & 1 ? w[j >> 1] & 0xffff0000u : w[j >> 1] << 16);
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) front[i][j] = pack_bf16x2(sum[2 * j], sum[2 * j + 1]);
+      if (g.addend && t0 + r < T) {
+        const u32x4 a = *reinterpret_cast<const u32x4*>(g.addend + static_cast<int64_t>(t0 + r) * D + o_col);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) front[i][j] = add_bf16x2(front[i][j], a[j]);
+      }
+    }
+  }
   for (int k0 = 0; k0 < E; k0 += BK) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -291,35 +349,32 @@ __global__ __launch_bounds__(X_NT, 2) void gate_dx_kernel(const float* __restric
     }
     __syncthreads();
   }
-  // through the wave's private LDS region (64 x 32 bf16), then 16-byte row pieces
-  using S = WaveStage<32>;
-  uint16_t* st = smem + wave * S::ELEMS;
+  // through LDS, then whole 256-byte pieces of rows
+  constexpr int PITCH = X_BN + 8;
 #pragma unroll
   for (int m = 0; m < 2; ++m)
 #pragma unroll
     for (int q = 0; q < 4; ++q)
-      S::put4(st, m, 0, lane, q, acc[m][q * 4], acc[m][q * 4 + 1], acc[m][q * 4 + 2], acc[m][q * 4 + 3]);
-  __builtin_amdgcn_s_waitcnt(0xc07f);
-  __builtin_amdgcn_wave_barrier();
+      *reinterpret_cast<u32x2*>(smem + (wm + m * 32 + (lane & 31)) * PITCH + wn + q * 8 + (lane >> 5) * 4) =
+          u32x2{pack2(acc[m][q * 4], acc[m][q * 4 + 1]), pack2(acc[m][q * 4 + 2], acc[m][q * 4 + 3])};
+  __syncthreads();
 #pragma unroll
-  for (int it = 0; it < 4; ++it) {
-    const int idx = it * 64 + lane;
-    const int m = idx >> 2, c = idx & 3;
-    const int t = t0 + wm + m;
-    if (t < T) {
-      const int64_t at = static_cast<int64_t>(t) * D + n0 + wn + c * 8;
-      u32x4 v = *reinterpret_cast<const u32x4*>(st + m * S::PITCH + c * 8);
-      if (addend) {
-        // the gradient that came back along the tokens' other uses: added here instead of by a pass of
-        // its own over three (T, D) tensors (17 us at 8192 x 2048), with that pass's rounding
-        const u32x4 a = *reinterpret_cast<const u32x4*>(addend + at);
+  for (int i = 0; i < kOut; ++i) {
+    const int r = o_row + 32 * i;
+    if (t0 + r >= T) continue;
+    const int64_t at = static_cast<int64_t>(t0 + r) * D + o_col;
+    u32x4 v = *reinterpret_cast<const u32x4*>(smem + r * PITCH + (tid & 15) * 8);
+    // the gradient that came back along the tokens' other uses: added here instead of by a pass of
+    // its own over three (T, D) tensors (17 us at 8192 x 2048), with that pass's rounding
+    if constexpr (ROWS) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          v[i] = pack_bf16x2(__uint_as_float(v[i] << 16) + __uint_as_float(a[i] << 16),
-                             __uint_as_float(v[i] & 0xffff0000u) + __uint_as_float(a[i] & 0xffff0000u));
-      }
-      *reinterpret_cast<u32x4*>(dx + at) = v;
+      for (int j = 0; j < 4; ++j) v[j] = add_bf16x2(v[j], front[i][j]);
+    } else if (g.addend) {
+      const u32x4 a = *reinterpret_cast<const u32x4*>(g.addend + at);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = add_bf16x2(v[j], a[j]);
     }
+    *reinterpret_cast<u32x4*>(dx + at) = v;
   }
 }
 
@@ -328,18 +383,17 @@ __global__ __launch_bounds__(X_NT, 2) void gate_dx_kernel(const float* __restric
 // tokens: dlogits tile split into three pieces (KS), x tile (KS).
 constexpr int W_BM = 128, W_BN = 128, W_NT = 512;
 
-__global__ __launch_bounds__(W_NT, 2) void gate_dw_kernel(const float* __restrict__ dlogits,
-                                                         const uint16_t* __restrict__ x,
-                                                         float* __restrict__ partial, int T, int D, int E,
-                                                         int rows_per_split) {
-  extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
+__device__ __forceinline__ void gate_dw_tile(const float* __restrict__ dlogits, const uint16_t* __restrict__ x,
+                                             float* __restrict__ partial, int T, int D, int E, int rows_per_split, int part,
+                                             uint16_t* smem) {
   uint16_t* A_p = smem;                 // 3 x [64][128] KS
   uint16_t* B_s = smem + 3 * BK * W_BM;  // [64][128] KS
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = (wave >> 1) * 32, wn = (wave & 1) * 64;
-  const int n0 = min(static_cast<int>(blockIdx.x) * W_BN, D - W_BN);
-  const int m0 = blockIdx.y * W_BM;  // E % 64 == 0; a last tile of 64 experts clamps its rows
-  const int split = blockIdx.z;
+  const int col_tiles = (D + W_BN - 1) / W_BN, row_tiles = (E + W_BM - 1) / W_BM;
+  const int n0 = min(part % col_tiles * W_BN, D - W_BN);
+  const int m0 = part / col_tiles % row_tiles * W_BM;  // E % 64 == 0; a last tile of 64 experts clamps its rows
+  const int split = part / (col_tiles * row_tiles);
   const int t_begin = split * rows_per_split, t_end = min(T, t_begin + rows_per_split);
   f32x16 acc[2];
 #pragma unroll
@@ -406,6 +460,29 @@ __global__ __launch_bounds__(W_NT, 2) void gate_dw_kernel(const float* __restric
         *reinterpret_cast<f32x4*>(dst + n * 32 + q * 8 + (lane >> 5) * 4) = v;
       }
   }
+}
+
+// Both in one launch, the dW tiles first.  In a training step they run beside the experts' weight gradients, whose workgroups hold a
+// CU each until the product ends: every launch of this chain waits for one of them to finish, so there are few.  With the row sum
+// in front (ROWS) the launch reads 2 T D elements less; alone, us, row sum + dx + dW / this: 3000 tokens of 6 x 1024, 64 experts 30 / 19,
+// 8192 of 8 x 2048, 128 experts 102 / 86, 16384 194 / 169.  Inside a training step only the short ones gain: 64 experts of 1024 x 512, six a
+// token, 300 tokens 233 / 223, 700 263 / 256, 3000 417 / 414, four of 64, 2000 tokens 273 / 264; 128 of 2048 x 768, 2500 tokens 1160 / 1153, 4000
+// 1520 / 1529, 16384 skewed 4655 / 4708.
+struct GateBwd {
+  const float* dlogits;
+  const uint16_t *x, *ws;  // ws: the weight's hi and mid pieces
+  GateSum sum;
+  uint16_t* dx;
+  float* partial;
+  int T, D, E, rows_per_split, dw_tiles;
+};
+template <bool ROWS>
+__global__ __launch_bounds__(X_NT, 4) void gate_bwd_kernel(GateBwd p) {
+  static_assert(X_NT == W_NT, "both tiles on the same workgroup");
+  extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
+  const int block = blockIdx.x;
+  if (block < p.dw_tiles) gate_dw_tile(p.dlogits, p.x, p.partial, p.T, p.D, p.E, p.rows_per_split, block, smem);
+  else gate_dx_tile<ROWS>(p.dlogits, p.ws, p.sum, p.dx, p.T, p.D, p.E, block - p.dw_tiles, smem);
 }
 
 // ---- both gradients for few experts (router_few.h) ---------------------------------------
@@ -540,7 +617,7 @@ int fwd_splits(int64_t T, int64_t D, int64_t E) {
   while (s < 8 && tiles * s < 256 && D % (2 * s * BK) == 0 && D / (2 * s) >= 4 * BK) s *= 2;
   return static_cast<int>(s);
 }
-constexpr int X_LDS = (2 * X_BM * BK + 2 * BK * X_BN) * 2;     // 65536
+constexpr int X_LDS = X_ELEMS * 2;                              // 65536
 constexpr int W_LDS = (3 * BK * W_BM + BK * W_BN) * 2;         // 65536
 
 // Splits of the token contraction for dW.  Two workgroups fit a CU, so the launch runs in
@@ -668,37 +745,36 @@ int router_logits_reduce(const float* partial, const float* bias, float* logits,
   return check_launch("router_gate_fwd");
 }
 
-int router_x3_bwd(const float* dlogits, const void* x, const float* w, const void* pieces, const void* addend,
+int router_x3_bwd(const float* dlogits, const void* x, const float* w, const void* pieces, const RowSum& sum,
                   void* dx, float* dw, void* workspace, int64_t T, int64_t D, int64_t E, hipStream_t s) {
   static PerDeviceOnce configured;
   if (configured.needed()) {
-    if (int rc = set_dyn_lds(gate_dx_kernel, X_LDS)) return rc;
-    if (int rc = set_dyn_lds(gate_dw_kernel, W_LDS)) return rc;
+    for (auto* kernel : {gate_bwd_kernel<false>, gate_bwd_kernel<true>})
+      if (int rc = set_dyn_lds(kernel, std::max(X_LDS + X_BM * kMaxSumK * 4, W_LDS))) return rc;
     configured.done();
   }
   uint16_t* ws = static_cast<uint16_t*>(workspace);
-  const int64_t n = E * D;
-  if (dx && T > 0) {
-    // (the forward's pieces, when its caller kept them: hi and mid come first there too)
-    if (!pieces)
-      hipLaunchKernelGGL(split_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, s, w, ws, n, 2);
-    hipLaunchKernelGGL(gate_dx_kernel, dim3((unsigned)((T + X_BM - 1) / X_BM), (unsigned)((D + X_BN - 1) / X_BN)),
-                       dim3(X_NT), X_LDS, s, dlogits, pieces ? static_cast<const uint16_t*>(pieces) : ws,
-                       static_cast<const uint16_t*>(addend), static_cast<uint16_t*>(dx), (int)T, (int)D, (int)E);
-    if (int rc = check_launch("router_gate_bwd dx")) return rc;
-  }
-  if (dw) {
-    const int splits = dw_splits(T, D, E);
-    const int rows_per_split = (int)(((T + splits - 1) / splits + BK - 1) / BK * BK);
-    float* partial = reinterpret_cast<float*>(ws + 2 * n);
-    hipLaunchKernelGGL(gate_dw_kernel,
-                       dim3((unsigned)((D + W_BN - 1) / W_BN), (unsigned)((E + W_BM - 1) / W_BM), (unsigned)splits),
-                       dim3(W_NT), W_LDS, s, dlogits, static_cast<const uint16_t*>(x), partial, (int)T, (int)D,
-                       (int)E, rows_per_split);
-    if (int rc = check_launch("router_gate_bwd dw")) return rc;
-    return launch_splitk_reduce(partial, dw, MI355_F32, n, splits, s);
-  }
-  return MI355_OK;
+  const int64_t n = E * D, cols = (D + X_BN - 1) / X_BN;
+  const bool want_dx = dx && T > 0;
+  // (the forward's pieces, when its caller kept them: hi and mid come first there too)
+  if (want_dx && !pieces)
+    hipLaunchKernelGGL(split_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, s, w, ws, n, 2);
+  const int splits = dw ? dw_splits(T, D, E) : 0;
+  const int64_t dw_tiles = cols * ((E + W_BM - 1) / W_BM) * splits;
+  const int64_t blocks = dw_tiles + (want_dx ? (T + X_BM - 1) / X_BM * cols : 0);
+  MI355_REQUIRE(blocks < (1ll << 31), "router_gate_bwd: too many tokens");
+  if (blocks == 0) return MI355_OK;
+  const GateBwd p{dlogits, static_cast<const uint16_t*>(x), pieces ? static_cast<const uint16_t*>(pieces) : ws,
+                  GateSum{static_cast<const uint16_t*>(sum.addend), static_cast<const uint16_t*>(sum.rows), sum.row_of_slot,
+                          (int)sum.K, (int)sum.row_capacity},
+                  static_cast<uint16_t*>(dx), reinterpret_cast<float*>(ws + 2 * n), (int)T, (int)D, (int)E,
+                  splits ? (int)(((T + splits - 1) / splits + BK - 1) / BK * BK) : 0, (int)dw_tiles};
+  if (sum.rows)
+    hipLaunchKernelGGL(gate_bwd_kernel<true>, dim3((unsigned)blocks), dim3(X_NT), std::max(X_LDS + X_BM * (int)sum.K * 4, W_LDS), s, p);
+  else
+    hipLaunchKernelGGL(gate_bwd_kernel<false>, dim3((unsigned)blocks), dim3(X_NT), std::max(X_LDS, W_LDS), s, p);
+  if (int rc = check_launch("router_gate_bwd")) return rc;
+  return dw ? launch_splitk_reduce(p.partial, dw, MI355_F32, n, splits, s) : MI355_OK;
 }
 
 }  // namespace mi355

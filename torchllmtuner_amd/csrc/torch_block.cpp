@@ -114,6 +114,8 @@ Tensor carve(const Tensor& like, Layout layout) {
   return t;
 }
 
+constexpr int64_t kShortRowSum = 6 << 20;  // elements of the tokens
+
 // What the backward reads besides the inputs, in one allocation: the plan's and the router's arrays, the
 // activations, the shared expert's plan and activations.
 struct Kept {
@@ -400,6 +402,10 @@ Grads block_backward(const Block& b, const Tensor& kept, const Tensor& dout_, co
   const int64_t slots = b.folded ? mi355_grouped_combine_bwd_slots(b.dt, b.D, b.F) : 0;
   // the gate's weight gradient in slices beside the experts' dH, its input gradient together with the row sum
   const bool joined = b.gather && mi355_router_gate_rows_bwd_covers(b.dt, b.gate_dt, b.D, b.E);
+  // ... or, behind the matrix-core kernels, both gradients and the row sum together, where they are short: beside the experts'
+  // weight gradients, whose workgroups keep to their tiles and their CUs, a long launch holds back whichever of those its own CUs
+  // were due to (router_gemm.hip has both sides)
+  const bool summed = b.folded && need.x && b.T * b.D <= kShortRowSum && mi355_router_gate_sum_bwd_covers(b.dt, b.gate_dt, b.D, b.E, c.K);
   const bool joined_dw = joined && need.gate_w && (need.x || need.experts);
   const int64_t gate_bytes = need.x || need.gate_w ? mi355_router_gate_bwd_workspace_bytes(b.T, b.D, b.E) : 0;
   void *s_dgate = nullptr, *s_dup = nullptr, *dx_shared = nullptr, *dx_routed = nullptr, *dgate = nullptr, *dup = nullptr,
@@ -415,7 +421,7 @@ Grads block_backward(const Block& b, const Tensor& kept, const Tensor& dout_, co
     }
     if (!routed) return;
     if (need.x) {
-      if (!joined) dx_routed = cv.take(b.T * b.D, item);
+      if (!joined && !summed) dx_routed = cv.take(b.T * b.D, item);
       drows = cv.take(b.R * b.D, item);
     }
     dgate = cv.take(b.R * b.F, item);
@@ -496,7 +502,7 @@ Grads block_backward(const Block& b, const Tensor& kept, const Tensor& dout_, co
       run(kWeights, side->stream);
     }
     if (need.x) run(MI355_STAGE_DX, L.stream);
-    row_sum();
+    if (!summed) row_sum();
     if (logits) select();
     if (need.experts && !side) run(kWeights, L.stream);
   } else if (b.gather) {
@@ -528,7 +534,13 @@ Grads block_backward(const Block& b, const Tensor& kept, const Tensor& dout_, co
   }
 
   // ---- router gate; the input gradient is complete with its part
-  if (joined && need.x) {
+  if (summed) {
+    shared.join();
+    check(mi355_router_gate_sum_bwd(dlogits, ptr(b.x), b.dt, fptr(b.gate_w), k.pieces, drows, k.row_of_slot, b.R, c.K, dx_shared,
+                                    ptr(g.x), need.gate_w ? g.gate_w.data_ptr<float>() : nullptr, gate_work, b.T, b.D, b.E,
+                                    L.stream),
+          "router_gate_sum_bwd");
+  } else if (joined && need.x) {
     shared.join();
     check(mi355_router_gate_rows_bwd(dlogits, b.dt, fptr(b.gate_w), drows, k.row_of_slot, b.R, c.K, dx_shared, ptr(g.x),
                                      static_cast<const float*>(gate_work), joined_dw ? g.gate_w.data_ptr<float>() : nullptr,
