@@ -495,59 +495,70 @@ struct GateDx {
   int K, row_capacity;
 };
 
-template <typename TX, bool ROWS>
+// TW tokens a wave.  With the rows in front (ROWS) two: the launch is the last of a backward, bound by the latency of its row
+// reads, and wants many waves (1531 tokens of 4 x 320, 16 experts: 18.0 us with eight a wave, 6.6 with two; 512 fp32 of 2 x 256 7.6, 4.0).
+template <typename TX, bool ROWS, int TW>
 __device__ __forceinline__ void gate_dx_part(const float* __restrict__ dlogits, const float* __restrict__ w,
                                              const GateDx<TX>& g, TX* __restrict__ dx, int T, int D, int E, int part,
                                              float* lds) {
+  constexpr int TOK = 4 * TW;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col_blocks = (D + S_COLS - 1) / S_COLS;
-  const int cb = part % col_blocks, t0 = part / col_blocks * S_TOK;
-  const int tokens = min(S_TOK, T - t0), n = cb * S_COLS + lane * 4;
+  const int cb = part % col_blocks, t0 = part / col_blocks * TOK;
+  const int tokens = min(TOK, T - t0), n = cb * S_COLS + lane * 4;
   constexpr int PITCH = S_MAX_E;
-  for (int i = tid; i < S_TOK * PITCH; i += 256) {
+  for (int i = tid; i < TOK * PITCH; i += 256) {
     const int t = i / PITCH, e = i % PITCH;
     lds[i] = t < tokens && e < E ? dlogits[static_cast<int64_t>(t0 + t) * E + e] : 0.0f;
   }
   __syncthreads();
   if (n >= D) return;
-  f32x4 sum[ROWS ? 8 : 1];
+  f32x4 sum[ROWS ? TW : 1];
   if constexpr (ROWS) {
-    // the rows go out first: the product below runs while they arrive.  One slot of eight tokens at a time.
+    // the rows go out first: the product below runs while they arrive
+    constexpr int B = 8 / TW;  // slots requested together
 #pragma unroll
-    for (int t = 0; t < 8; ++t) sum[t] = f32x4{0, 0, 0, 0};
-    const int32_t* slots = g.row_of_slot + (static_cast<int64_t>(t0) + wave * 8) * g.K;
-    for (int k = 0; k < g.K; ++k) {
-      f32x4 v[8];
+    for (int t = 0; t < TW; ++t) sum[t] = f32x4{0, 0, 0, 0};
+    const int32_t* slots = g.row_of_slot + (static_cast<int64_t>(t0) + wave * TW) * g.K;
+    for (int k0 = 0; k0 < g.K; k0 += B) {
+      f32x4 v[B][TW];
 #pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        const int row = wave * 8 + t < tokens ? slots[t * g.K + k] : -1;  // wave-uniform
-        v[t] = row >= 0 && row < g.row_capacity ? load_cols(g.rows + static_cast<int64_t>(row) * D + n) : f32x4{0, 0, 0, 0};
-      }
+      for (int k = 0; k < B; ++k)
 #pragma unroll
-      for (int t = 0; t < 8; ++t) sum[t] += v[t];
+        for (int t = 0; t < TW; ++t) {
+          const int row = k0 + k < g.K && wave * TW + t < tokens ? slots[t * g.K + k0 + k] : -1;  // wave-uniform
+          v[k][t] = row >= 0 && row < g.row_capacity ? load_cols(g.rows + static_cast<int64_t>(row) * D + n) : f32x4{0, 0, 0, 0};
+        }
+#pragma unroll
+      for (int k = 0; k < B; ++k)
+#pragma unroll
+        for (int t = 0; t < TW; ++t) sum[t] += v[k][t];
     }
   }
-  f32x4 acc[8];  // tokens wave * 8 ..
+  f32x4 acc[TW];
 #pragma unroll
-  for (int t = 0; t < 8; ++t) acc[t] = f32x4{0, 0, 0, 0};
-  for (int e = 0; e < E; e += 4) {
-    f32x4 wv[4];
+  for (int t = 0; t < TW; ++t) acc[t] = f32x4{0, 0, 0, 0};
+  constexpr int EB = TW >= 8 ? 4 : 8;  // experts requested together
+  for (int e = 0; e < E; e += EB) {
+    f32x4 wv[EB];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) wv[j] = load_cols(w + static_cast<int64_t>(min(e + j, E - 1)) * D + n);
+    for (int j = 0; j < EB; ++j) wv[j] = load_cols(w + static_cast<int64_t>(min(e + j, E - 1)) * D + n);
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      const f32x4 d = *reinterpret_cast<const f32x4*>(lds + (wave * 8 + t) * PITCH + e);  // zero past E
+    for (int t = 0; t < TW; ++t)
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
+      for (int q = 0; q < EB / 4; ++q) {
+        const f32x4 d = *reinterpret_cast<const f32x4*>(lds + (wave * TW + t) * PITCH + e + 4 * q);  // zero past E
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc[t][i] = fmaf(d[j], wv[j][i], acc[t][i]);
-    }
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[t][i] = fmaf(d[j], wv[4 * q + j][i], acc[t][i]);
+      }
   }
   auto rounded = [](float v) { return sizeof(TX) == 2 ? round_bf16(v) : v; };
 #pragma unroll
-  for (int t = 0; t < 8; ++t) {
-    if (wave * 8 + t >= tokens) break;
-    const int64_t at = static_cast<int64_t>(t0 + wave * 8 + t) * D + n;
+  for (int t = 0; t < TW; ++t) {
+    if (wave * TW + t >= tokens) break;
+    const int64_t at = static_cast<int64_t>(t0 + wave * TW + t) * D + n;
     f32x4 v = acc[t];
     // each sum is added to the rounded one before it and rounded again, as separate additions would be
     if (ROWS || g.addend) {
@@ -570,8 +581,10 @@ __global__ __launch_bounds__(256) void gate_bwd_few_kernel(GateDw dw, const floa
   __shared__ __attribute__((aligned(16))) float lds[kGateDwLds];
   const int block = blockIdx.x;
   if (block < dw_parts) gate_dw_part<TX>(dw, block, lds);
-  else gate_dx_part<TX, false>(dlogits, w, g, dx, T, D, E, block - dw_parts, lds);
+  else gate_dx_part<TX, false, S_TOK / 4>(dlogits, w, g, dx, T, D, E, block - dw_parts, lds);
 }
+
+constexpr int kRowsTok = 8;  // tokens of a dx part with the rows in front
 
 // dx with the sum over the token's rows, and beside it the sum of dW's slices, in their order: the two ends of a backward
 // whose dW parts ran in an earlier launch.
@@ -580,10 +593,10 @@ __global__ __launch_bounds__(256) void gate_rows_bwd_kernel(const float* __restr
                                                             GateDx<TX> g, TX* __restrict__ dx,
                                                             const float* __restrict__ partial, float* __restrict__ dw,
                                                             int splits, int T, int D, int E, int dx_parts) {
-  __shared__ __attribute__((aligned(16))) float lds[S_TOK * S_MAX_E];
+  __shared__ __attribute__((aligned(16))) float lds[kRowsTok * S_MAX_E];
   const int block = blockIdx.x;
   if (block < dx_parts) {
-    gate_dx_part<TX, true>(dlogits, w, g, dx, T, D, E, block, lds);
+    gate_dx_part<TX, true, kRowsTok / 4>(dlogits, w, g, dx, T, D, E, block, lds);
     return;
   }
   const int64_t n = static_cast<int64_t>(E) * D, i = static_cast<int64_t>(block - dx_parts) * 256 + threadIdx.x;
@@ -668,7 +681,7 @@ int router_rows_bwd(const float* dlogits, int x_dtype, const float* w, const voi
                     int64_t row_capacity, int64_t K, const void* addend, void* dx, const float* partial, float* dw, int64_t T,
                     int64_t D, int64_t E, hipStream_t s) {
   const int splits = gate_dw_splits(T, D, E);
-  const int64_t dx_parts = dx ? (T + S_TOK - 1) / S_TOK * ((D + S_COLS - 1) / S_COLS) : 0;
+  const int64_t dx_parts = dx ? (T + kRowsTok - 1) / kRowsTok * ((D + S_COLS - 1) / S_COLS) : 0;
   const int64_t blocks = dx_parts + (dw ? (E * D + 255) / 256 : 0);
   MI355_REQUIRE(blocks < (1ll << 31), "router_gate_rows_bwd: too many tokens");
   if (blocks == 0) return MI355_OK;
