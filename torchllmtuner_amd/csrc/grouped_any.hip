@@ -8,7 +8,7 @@
 // (buffer loads: dword alignment suffices for them, and what lies past a matrix reads as zero; the ends store
 // four elements at a time, so the matrices themselves start on 16-byte boundaries); the tail of
 // the contraction is zeroed as it is parked.  LDS holds an operand as it lies in memory -- contraction
-// contiguous [row][128 B + 16] or strided [k][cols + pad], the pads chosen so that fragment reads
+// contiguous [row][128 B + 16] or strided [k][cols], padded (fp32) or its chunks swizzled (bf16) so that fragment reads
 // are free of bank conflicts -- and the fragment reads (b128, b32, or the transposing b64 for bf16)
 // make up for the difference.
 //   Products and their fused ends: gate and up in one pass with SwiGLU; down; dh with the SwiGLU
@@ -63,7 +63,7 @@ template <> struct El<float> {
   using V4 = f32x4;
 };
 template <> struct El<uint16_t> {
-  static constexpr int KS_PAD = 32;  // four consecutive k rows a quarter of the banks apart
+  static constexpr int KS_PAD = 0;   // (swizzled, below)
   using V4 = u32x2;
 };
 
@@ -98,9 +98,16 @@ struct Operand {
   static constexpr int CPR = KS ? ROWS / E : 8;  // chunks per stored row
   static constexpr int N = ROWS * 8 / 256;       // chunks per lane and step
 
+  // bf16, strided: a transposing read touches 64 bytes of four consecutive k rows per 32 lanes, and each row gets a quarter of the
+  // banks -- rows of 128 bytes lie on alternate halves already.  (Padding for it took half as much LDS again, and with it
+  // two of five workgroups a CU.  A training step of 4096 tokens of 32 x 480 x 432, four each, 323 -> 315 us, of 4 x 440 x 432 273 -> 264.)
+  static __device__ __forceinline__ int swizzle(int k) {
+    if constexpr (KS && sizeof(T) == 2) return CPR >= 16 ? (k & 3) << 2 : (k >> 1 & 1) << 2;
+    else return 0;
+  }
   static __device__ __forceinline__ int at(int tid, int i) {
     const int q = tid + 256 * i;
-    return (q / CPR) * PITCH + (q % CPR) * E;
+    return (q / CPR) * PITCH + ((q % CPR) ^ swizzle(q / CPR)) * E;
   }
   // keep what lies inside the contraction (kv of BKE elements); a multiple of four
   static __device__ __forceinline__ u32x4 clip(const u32x4& v, int tid, int i, int kv) {
@@ -123,7 +130,8 @@ __device__ __forceinline__ bf16x8 any_frag(const uint16_t* tile, int row, int kk
     return *reinterpret_cast<const bf16x8*>(tile + (row + (lane & 31)) * O::PITCH + kk * 16 + 8 * (lane >> 5));
   } else {
     const int g = lane >> 4, i = lane & 15;
-    const uint16_t* p = tile + (kk * 16 + 8 * (g >> 1) + (i >> 2)) * O::PITCH + row + 16 * (g & 1) + 4 * (i & 3);
+    const int k = kk * 16 + 8 * (g >> 1) + (i >> 2), c = row + 16 * (g & 1) + 4 * (i & 3);  // (row k + 4 has row k's key)
+    const uint16_t* p = tile + k * O::PITCH + (((c >> 3) ^ O::swizzle(k)) << 3) + (c & 7);
     const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(p));
     const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(p + 4 * O::PITCH));
     return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
@@ -281,7 +289,10 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
   const auto rsA1 = MODE == ANY_DX ? any_rsrc(A1, a_bytes) : rsA0;
   const auto rsB1 = (MODE == ANY_GATEUP || MODE == ANY_DX) ? any_rsrc(B1, b_bytes) : rsB0;
   // K_FOLD: source rows of the steps ahead; scales of the steps held
-  uint32_t srcA[K_FOLD ? AHEAD : 1][K_FOLD ? OA::N : 1], srcB[K_FOLD ? AHEAD : 1][K_FOLD ? OB::N : 1];
+  // (bf16, one step requested ahead: the indexes go two, so that a step's are older than the rows of the step before it
+  // and waiting for them does not wait for those; fp32 steps are long enough without)
+  constexpr int SRC = K_FOLD && sizeof(T) == 2 ? 2 : AHEAD;
+  uint32_t srcA[K_FOLD ? SRC : 1][K_FOLD ? OA::N : 1], srcB[K_FOLD ? SRC : 1][K_FOLD ? OB::N : 1];
   float k_scale[K_FOLD ? AHEAD : 1][K_FOLD ? OA::N : 1];
   auto row_of = [&](int s, int chunk_row) -> int64_t { return first_row + min(s * BKE + chunk_row, K - 1); };
   auto request_sources = [&](int slot, int s) {
@@ -296,7 +307,7 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
       }
     }
   };
-  auto fetch = [&](int slot, int s) {
+  auto fetch = [&](int slot, int s, int src) {  // src: the slot of its sources
     const bool second = MODE == ANY_DX && s >= half_steps;
     const uint32_t k = static_cast<uint32_t>(second ? s - half_steps : s) * BKE;
     const uint32_t ka = (A_KS ? k * lda : k) * sizeof(T), kb = (B_KS ? k * ldb : k) * sizeof(T);
@@ -315,7 +326,7 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
     for (int i = 0; i < OA::N; ++i) {
       uint32_t at = offA[i] + ka;
       if constexpr (K_FOLD)
-        if (through_a) at = (within(srcA[slot][i]) * lda + ((tid + 256 * i) % OA::CPR) * OA::E) * sizeof(T);
+        if (through_a) at = (within(srcA[src][i]) * lda + ((tid + 256 * i) % OA::CPR) * OA::E) * sizeof(T);
       ra[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(rsA, at, 0, 0);
       if constexpr (K_FOLD)
         if (through_a) k_scale[slot][i] = p.scale[row_of(s, (tid + 256 * i) / OA::CPR)];
@@ -324,10 +335,10 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
     for (int i = 0; i < OB::N; ++i) {
       uint32_t at = offB[i] + kb;
       if constexpr (K_FOLD)
-        if (through_b) at = (within(srcB[slot][i]) * ldb + ((tid + 256 * i) % OB::CPR) * OB::E) * sizeof(T);
+        if (through_b) at = (within(srcB[src][i]) * ldb + ((tid + 256 * i) % OB::CPR) * OB::E) * sizeof(T);
       rb[slot][i] = __builtin_amdgcn_raw_buffer_load_b128(i >= OB::N / 2 ? rsU : rsB, at, 0, 0);
     }
-    request_sources(slot, s + AHEAD);
+    request_sources(src, s + SRC);
   };
   auto park = [&](int slot, int s) {
     T* As = smem + (s & 1) * STAGE;
@@ -381,28 +392,37 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
   };
   if constexpr (!KSPLIT) {
     if (steps > 0) {
-      request_sources(0, 0);
-      fetch(0, 0);
+#pragma unroll
+      for (int i = 0; i < SRC; ++i) request_sources(i, i);
+      fetch(0, 0, 0);
       park(0, 0);
-      if (steps > 1) fetch(0, 1);
+      if (steps > 1) fetch(0, 1, SRC - 1);
     }
     __syncthreads();
-    for (int s = 0; s < steps; ++s) {
+    auto step = [&](int s, int src) {
       if (s + 1 < steps) park(0, s + 1);
-      if (s + 2 < steps) fetch(0, s + 2);
+      if (s + 2 < steps) fetch(0, s + 2, src);
       const T* As = smem + (s & 1) * STAGE;
 #pragma unroll
       for (int kk = 0; kk < KK; ++kk) multiply(As, As + OA::ELEMS, kk);
       __syncthreads();
+    };
+    if constexpr (SRC == 1) {
+      for (int s = 0; s < steps; ++s) step(s, 0);
+    } else {
+      for (int s = 0; s < steps; s += 2) {
+        step(s, 0);
+        if (s + 1 < steps) step(s + 1, 1);
+      }
     }
   } else {
     if (steps > 0) {
 #pragma unroll
       for (int i = 0; i < AHEAD; ++i) request_sources(i, i);
 #pragma unroll
-      for (int i = 0; i < AHEAD; ++i) fetch(i, i);
+      for (int i = 0; i < AHEAD; ++i) fetch(i, i, i);
       park(0, 0);
-      fetch(0, AHEAD);
+      fetch(0, AHEAD, 0);
       phase_barrier();
     }
     for (int s0 = 0; s0 < steps; s0 += AHEAD) {
@@ -411,7 +431,7 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
         const int s = s0 + i;
         if (s >= steps) goto done;
         if (s + 1 < steps) park((i + 1) % AHEAD, s + 1);
-        fetch((i + 1) % AHEAD, s + 1 + AHEAD);
+        fetch((i + 1) % AHEAD, s + 1 + AHEAD, (i + 1) % AHEAD);
         const T* As = smem + (s & 1) * STAGE;
         multiply(As, As + OA::ELEMS, wave);
         phase_barrier();
