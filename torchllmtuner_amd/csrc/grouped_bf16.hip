@@ -1025,9 +1025,9 @@ int few_rows_fwd(int stage, const void* a, const int32_t* a_src, int64_t a_rows,
 // Up to eight rows per expert on average (rows and experts are what the host knows; one expert's share of
 // a wider router counts rows it does not get, which only errs towards the large tiles), or 64 rows in all.
 // A 16-row pass over an expert's weights costs the same for one row as for sixteen and a second pass
-// reads them again, from L2 at best: measured at 128 experts of 2048 x 768 the block takes 217 us against
-// 248 at 33 tokens (2 rows on average), 264 against 268 at 128 (8), 307 against 271 at 200 (12); one dense
-// segment of 7168 x 2048, 4 us of difference at 60 rows and -55 at 128.
+// reads them again, from L2 at best: measured at 128 experts of 2048 x 768 the block takes 201 us against
+// 221 at 33 tokens (2 rows on average), 224 against 234 at 64, 238 against 240 at 128 (8), 251 against 241 at 160 (10), 275 against 242 at
+// 200; one dense segment of 7168 x 2048, 4 us of difference at 60 rows and -55 at 128.
 static bool few_rows(int64_t El, int64_t R, int64_t D, int64_t F) {
   return R <= std::max<int64_t>(8 * El, 64) && R * std::max(D, F) * 2 < (int64_t{1} << 32);
 }

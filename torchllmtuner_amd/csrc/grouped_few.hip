@@ -8,7 +8,9 @@
 // expert; every wave loads its weights straight into MFMA fragments, 16 KiB requested ahead, up
 // to sixteen waves to a CU, and the four partial tiles are added in wave order through LDS.
 //   Bound by HBM: 709 MB of gate and up weights (33 tokens of 128 experts, 2048 x 768) in 116 us, 6.1 TB/s
-// where a plain read in this pattern reaches 6.15 (145 us before); one token, 50 MB, 13 us (31 before).
+// where a plain read in this pattern reaches 6.15 (145 us before); one token, 50 MB, 13 us (31 before).  The 354 MB of the down
+// projection, three contraction steps a wave, in 57 us: with four requested, the last twice, and the row counts looked up in front of
+// the weights it was 69.
 // Waves along the contraction rather than side by side: at one token 12-25 us less in all, at 33 the
 // same.  32 or 64 rows per wave instead of 16 need registers that the requests in flight want: slower.
 //   A contraction step is 64 wide: lane group g = lane / 16 holds k = 16 g .. 16 g + 15 of it (two
@@ -39,11 +41,14 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t few_rsrc(const void* base) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, -1, 0x00020000);
 }
 
-// Column group cg of the product of expert e with rows row0 .. row0 + rows - 1; a row is source(row) of a, or itself.
-template <bool GATEUP, typename Source>
-__device__ __forceinline__ void few_rows_tile(const FewArgs& p, int e, int row0, int rows, int cg, bool through,
-                                              Source source, f32x4 (&part)[4][2][64]) {
-  constexpr int kPairs = 4;  // 64-wide contraction steps requested together
+// Column group cg of the product of expert e with the rows that where() names (the first and how many, at least one: looked up once
+// the first weights are on their way); a row is source(row) of a, or itself.  kPairs: 64-wide contraction steps requested together.
+struct FewRows {
+  int row0, rows;
+};
+template <bool GATEUP, int kPairs, typename Source, typename Where>
+__device__ __forceinline__ void few_rows_tile(const FewArgs& p, int e, int cg, bool through, Source source, Where where,
+                                              f32x4 (&part)[4][2][64]) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, g = lane >> 4;
   const int K = p.K, N = p.N;
@@ -55,20 +60,30 @@ __device__ __forceinline__ void few_rows_tile(const FewArgs& p, int e, int row0,
   const auto rs0 = few_rsrc(p.b0 + we), rs1 = few_rsrc(p.b1 + we), rsA = few_rsrc(p.a);
   const uint32_t off0 = static_cast<uint32_t>((n0 + r16) * K + g * 16) * 2u;
   const uint32_t off1 = GATEUP ? off0 : off0 + static_cast<uint32_t>(32 * K);
+  u32x4 b0[kPairs][2], b1[kPairs][2], a[kPairs][2];
+  auto request_w = [&](int i, int step) {
+    const int k = step * 128;  // bytes
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      b0[i][h] = __builtin_amdgcn_raw_buffer_load_b128(rs0, off0 + 16 * h, k, 0);
+      b1[i][h] = __builtin_amdgcn_raw_buffer_load_b128(rs1, off1 + 16 * h, k, 0);
+    }
+  };
+  // the first weights go out before the rows are known (past the end: the last step again, not used)
+  auto request_first = [&]() {
+#pragma unroll
+    for (int i = 0; i < kPairs; ++i) request_w(i, min(s0 + i, s1 - 1));
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  request_first();
+  const FewRows at_rows = where();
+  const int row0 = at_rows.row0, rows = at_rows.rows;
   for (int sub = 0; sub < rows; sub += 16) {
+    if (sub) request_first();
     const int row = row0 + min(sub + r16, rows - 1);
     const int index = through ? source(row) : row;
     f32x4 acc0 = {0, 0, 0, 0}, acc1 = {0, 0, 0, 0};
-    u32x4 b0[kPairs][2], b1[kPairs][2], a[kPairs][2];
     uint32_t offA;
-    auto request_w = [&](int i, int step) {
-      const int k = step * 128;  // bytes
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        b0[i][h] = __builtin_amdgcn_raw_buffer_load_b128(rs0, off0 + 16 * h, k, 0);
-        b1[i][h] = __builtin_amdgcn_raw_buffer_load_b128(rs1, off1 + 16 * h, k, 0);
-      }
-    };
     auto request_a = [&](int i, int step) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) a[i][h] = __builtin_amdgcn_raw_buffer_load_b128(rsA, offA + 16 * h, step * 128, 0);
@@ -81,10 +96,6 @@ __device__ __forceinline__ void few_rows_tile(const FewArgs& p, int e, int row0,
         acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, b1[i][h]), af, acc1, 0, 0, 0);
       }
     };
-    // the first weights go out before the row's index is back (past the end: the last step again, not used)
-#pragma unroll
-    for (int i = 0; i < kPairs; ++i) request_w(i, min(s0 + i, s1 - 1));
-    __builtin_amdgcn_sched_barrier(0);
     const int src = through ? min(max(index, 0), p.a_rows - 1) : row;
     offA = (static_cast<uint32_t>(src) * static_cast<uint32_t>(K) + g * 16) * 2u;
 #pragma unroll
@@ -145,15 +156,21 @@ __device__ __forceinline__ void few_rows_tile(const FewArgs& p, int e, int row0,
   }
 }
 
-template <bool GATEUP>
+template <bool GATEUP, int kPairs>
 __global__ __launch_bounds__(256, 4) void few_rows_kernel(FewArgs p) {
   __shared__ f32x4 part[4][2][64];
   const int t = blockIdx.x / p.col_groups, cg = blockIdx.x - t * p.col_groups;
-  if (t >= *p.num_tiles) return;
-  const int e = __builtin_amdgcn_readfirstlane(p.tile_expert[t]), row0 = __builtin_amdgcn_readfirstlane(p.tile_row0[t]);
-  const int cnt = p.seg_counts[e], seg0 = p.seg_offsets[e];
-  const int rows = min(even_tile_rows(cnt, 256), seg0 + cnt - row0);
-  few_rows_tile<GATEUP>(p, e, row0, rows, cg, p.a_src != nullptr, [&](int row) { return p.a_src[row]; }, part);
+  // looked up together (an entry past the last tile is not used): every lookup in a row is a round trip in front of the weights
+  const int tiles = *p.num_tiles, e = __builtin_amdgcn_readfirstlane(p.tile_expert[t]),
+            row0 = __builtin_amdgcn_readfirstlane(p.tile_row0[t]);
+  if (t >= tiles) return;
+  few_rows_tile<GATEUP, kPairs>(
+      p, e, cg, p.a_src != nullptr, [&](int row) { return p.a_src[row]; },
+      [&]() -> FewRows {
+        const int cnt = p.seg_counts[e], seg0 = p.seg_offsets[e];
+        return {row0, min(even_tile_rows(cnt, 256), seg0 + cnt - row0)};
+      },
+      part);
 }
 
 // ---- a handful of tokens, forward only: no plan ---------------------------------------------------
@@ -221,7 +238,8 @@ __global__ __launch_bounds__(256, 4) void choice_gateup_kernel(FewArgs p, Choice
   const RowChoice ch = choose<VPR, FULL>(c, t, lane & 15);
   const int id = __builtin_amdgcn_readlane(ch.id, row - t * K);
   if (id < c.lo || id >= c.hi) return;  // (the same for the whole workgroup)
-  few_rows_tile<true>(p, id - c.lo, row, 1, cg, true, [&](int) { return t; }, part);
+  few_rows_tile<true, 4>(
+      p, id - c.lo, cg, true, [&](int) { return t; }, [&]() -> FewRows { return {row, 1}; }, part);
 }
 
 struct ChoiceOut {
@@ -332,8 +350,10 @@ int few_rows_fwd(int stage, const void* a, const int32_t* a_src, int64_t a_rows,
   p.num_tiles = num_tiles; p.K = (int)K; p.N = (int)N;
   p.col_groups = (int)(N / (stage == 1 ? 16 : 32));
   const dim3 grid((unsigned)(tiles * p.col_groups));
-  if (stage == 1) hipLaunchKernelGGL(few_rows_kernel<true>, grid, dim3(256), 0, s, p);
-  else hipLaunchKernelGGL(few_rows_kernel<false>, grid, dim3(256), 0, s, p);
+  // (up to 768: three steps a wave)
+  if (stage == 1) hipLaunchKernelGGL((few_rows_kernel<true, 4>), grid, dim3(256), 0, s, p);
+  else if (K <= 12 * 64) hipLaunchKernelGGL((few_rows_kernel<false, 3>), grid, dim3(256), 0, s, p);
+  else hipLaunchKernelGGL((few_rows_kernel<false, 4>), grid, dim3(256), 0, s, p);
   return check_launch("grouped forward, few rows");
 }
 
