@@ -1,0 +1,84 @@
+"""fp32 expert products on tiles of 64 rows and more, whose operands are multiplied as three bf16 pieces each, against fp64."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from tests.helpers import rel_l2
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from torchllmtuner_amd import ops as o
+
+    return o
+
+
+def problem(ops, counts, D, Fd):
+    g = torch.Generator().manual_seed(11)
+    El, R = len(counts), sum(counts)
+    ids = torch.repeat_interleave(torch.arange(El), torch.tensor(counts))[:, None]
+    x, dy = (torch.randn(R, D, generator=g).to(DEV) for _ in "xy")
+    w1, w3, w2 = ((torch.randn(*s, generator=g) * 0.03).to(DEV) for s in ((El, Fd, D), (El, Fd, D), (El, D, Fd)))
+    rows = list(torch.arange(R).split(list(counts)))  # the plan keeps an expert's rows in token order
+    return ops.permute_plan(ids.to(DEV), El), x, dy, w1, w3, w2, [r.to(DEV) for r in rows]
+
+
+def per_expert(rows, fn, like):
+    out = torch.empty(like.shape, dtype=torch.float64, device=DEV)
+    for e, r in enumerate(rows):
+        out[r] = fn(e, r)
+    return out
+
+
+# every product on 64-row tiles; some of them on 32-row ones; all on 128-row ones.  Segments that end inside a tile, widths
+# that end inside one and inside a step of 32
+@pytest.mark.parametrize("counts,D,Fd", [((520, 1000, 65), 772, 580), ((300, 70, 0, 401), 516, 900),
+                                         ((3100, 2900, 3001), 900, 908)])
+def test_products_against_fp64(ops, counts, D, Fd):
+    print(f"fp32 pieces {counts} D={D} F={Fd}", flush=True)
+    plan, x, dy, w1, w3, w2, rows = problem(ops, counts, D, Fd)
+    y, gate, up, h = ops.grouped_swiglu_fwd(x, w1, w3, w2, plan)
+    dx, dw1, dw3, dw2 = ops.grouped_swiglu_bwd(dy, x, w1, w3, w2, gate, up, h, plan)
+    # a sum of n products, rounded to 24 bits as it grows: a walk of at most n roundings of half an ulp each
+    def bound(n):
+        return n ** 0.5 * 2.0 ** -24
+
+    d = [t.double() for t in (x, dy, w1, w3, w2, gate, up, h)]
+    xd, dyd, w1d, w3d, w2d, gd, ud, hd = d
+    assert rel_l2(gate, per_expert(rows, lambda e, r: xd[r] @ w1d[e].T, gate)) < bound(D)
+    assert rel_l2(up, per_expert(rows, lambda e, r: xd[r] @ w3d[e].T, up)) < bound(D)
+    assert rel_l2(y, per_expert(rows, lambda e, r: hd[r] @ w2d[e].T, y)) < bound(Fd)
+    # (the element-wise ends: a few roundings each, below the sums' own)
+    sig = torch.sigmoid(gd)
+    dh = per_expert(rows, lambda e, r: dyd[r] @ w2d[e], h)
+    dg, du = dh * ud * sig * (1 + gd * (1 - sig)), dh * F.silu(gd)
+    want = per_expert(rows, lambda e, r: dg[r] @ w1d[e] + du[r] @ w3d[e], dx)
+    assert rel_l2(dx, want) < bound(D) + bound(2 * Fd)
+    for got, a, b, chain in ((dw1, dg, xd, bound(D)), (dw3, du, xd, bound(D)), (dw2, dyd, hd, 0.0)):
+        want = torch.stack([a[r].T @ b[r] for r in rows])
+        assert rel_l2(got, want) < chain + bound(max(counts))
+
+
+def test_infinities_overflow_and_nan(ops):
+    """A value beyond bf16's range and one that is none: what an fp32 product of the row gives, and nothing elsewhere."""
+    plan, x, _, w1, w3, w2, rows = problem(ops, (520, 1000, 65), 772, 580)
+    clean = ops.grouped_swiglu_fwd(x, w1, w3, w2, plan)[1]
+    x[3, 700], x[600, 1], x[601, 5] = float("inf"), float("nan"), 3.4e38  # (rounds to infinity in bf16)
+    w1[1, 9, 5] = 0.0
+    w1[1, 8, 5] = 0.5
+    gate = ops.grouped_swiglu_fwd(x, w1, w3, w2, plan)[1]
+    torch.cuda.synchronize()
+    assert torch.equal(gate[3], torch.sign(w1[0, :, 700]) * float("inf"))
+    assert gate[600].isnan().all()
+    assert gate[601].isfinite().all() and gate[601, 8].item() == pytest.approx(1.7e38, rel=1e-6)
+    same = torch.ones(len(x), dtype=torch.bool, device=DEV)
+    same[[3, 600, 601]] = False
+    cols = torch.tensor([c for c in range(580) if c not in (8, 9)], device=DEV)
+    # rows that share a tile with one of the three are formed in the other way: the same up to rounding
+    assert rel_l2(gate[same][:, cols], clean[same][:, cols]) < 2 * 772 ** 0.5 * 2.0 ** -24

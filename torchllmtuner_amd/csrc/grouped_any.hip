@@ -2,9 +2,9 @@
 // are below the 384 columns) of the kernels in grouped_bf16.hip.  Widths are multiples of four.
 //
 // One kernel template over the element type, the product and the tile: 256 lanes as 2 x 2 waves on a
-// TM x TN output tile, each wave (TM/2) x (TN/2) in 32x32 accumulators (v_mfma_f32_32x32x16_bf16, or
-// v_mfma_f32_32x32x2_f32 for fp32), 128 bytes of the contraction per step, two LDS stages, the next
-// step's operands held in registers.  Operands are fetched 16 bytes at a time whatever the width
+// TM x TN output tile, each wave (TM/2) x (TN/2) in 32x32 accumulators (v_mfma_f32_32x32x16_bf16; fp32 on 32-row
+// tiles v_mfma_f32_32x32x2_f32, on larger ones products of bf16 pieces, below), 128 bytes of the contraction per step,
+// two LDS stages (of pieces one), the next step's operands held in registers.  Operands are fetched 16 bytes at a time whatever the width
 // (buffer loads: dword alignment suffices for them, and what lies past a matrix reads as zero; the ends store
 // four elements at a time, so the matrices themselves start on 16-byte boundaries); the tail of
 // the contraction is zeroed as it is parked.  LDS holds an operand as it lies in memory -- contraction
@@ -17,9 +17,8 @@
 // contractions.  Small tiles are used until the large ones fill the chip: 64 rows, and for fp32 32 x 32, where
 // the four waves hold the same tile and split each step's contraction (their shares are added through LDS in
 // wave order) and four steps are requested ahead.
-//   512 tokens of 8 fp32 experts of 256 x 512, gate/up + down and the backward experts: 30 + 46 us on 64-row
-// tiles, 25 + 33 us now; 200 tokens of 16 of 640 x 1024, two each, 88 + 171 us, 49 + 97 now;
-// 1531 tokens of 16 bf16 experts of 320 x 232, 23 + 41 us.
+//   512 tokens of 8 fp32 experts of 256 x 512, two each, gate/up + down and the backward experts 26 + 33 us; 200 tokens of 16 of
+// 640 x 1024, two each, 51 + 83; 4096 of them, four each, 450 + 930; 1531 tokens of 16 bf16 experts of 320 x 232, 23 + 44 us.
 #include <algorithm>
 #include <type_traits>
 
@@ -148,6 +147,50 @@ __device__ __forceinline__ f32x4 any_frag(const float* tile, int row, int kk, in
   for (int j = 0; j < 4; ++j) v[j] = tile[(k + j) * O::PITCH + row + (lane & 31)];
   return v;
 }
+
+// fp32 on tiles of 64 rows and more, where the matrix cores were the bound (137 TFLOP/s a large product, these 100): an operand
+// is parked as three bf16 pieces, each the nearest to what the ones before leave, 24 bits and their signs together, and a product is
+// the six products of pieces whose weights are within 2^-16 of the first; what is left out is 2^-26 of it.  bf16 products are
+// 16 times as fast.  The six of 16 k are added up, the smallest first, before they meet the sum, which so is rounded once for every
+// 16 products: over steps of 64-4096 tokens of 64-640 x 96-1020 the rms error against fp64 is 0.30-0.95 of what fp32 products
+// gave (2409 tokens of 8 x 360 x 648: dx 8.2e-7 -> 2.7e-7, dw2 6.7e-7 -> 2.3e-7; added to the sum one by one, 4-10 % faster, 0.8-1.4).
+//   Split where it is parked, once a workgroup, not where each of the waves reads it (5.5 vector instructions an element); one
+// stage, so that LDS (61 KB on 128-row tiles) holds two workgroups a CU and one splits while the other multiplies.  A training step,
+// us, fp32 products / pieces: 4096 tokens of 16 x 640 x 1020 (four each) 2009 / 1573, 4096 of 4 (two each) 1033 / 845, 1000 of 16 x
+// 512 x 800 (three each) 353 / 262, 1500 of 8 x 320 x 400 (three each) 196 / 169.  Two, three and four steps requested ahead: large
+// products 3-9 % slower, small ones the same.
+//   A value that is not finite, or rounds to infinity, has NaN for its second piece: a tile with a NaN is formed again by
+// fp32 products, which say what it is.  (Values below 2^-110 lose bits: bf16 ends at 2^-133.)
+template <bool KS, int ROWS>
+struct Pieces {
+  using O = Operand<float, KS, ROWS>;       // (the chunks of four that a lane fetches)
+  static constexpr int PITCH = KS ? ROWS : 40;  // 80 bytes: 16 rows' b128 reads fall on 64 different banks
+  static constexpr int ELEMS = (KS ? O::BKE : ROWS) * PITCH;
+  static __device__ __forceinline__ int at(int tid, int i) {
+    const int q = tid + 256 * i, r = q / O::CPR, c = q % O::CPR;
+    if constexpr (!KS) return r * PITCH + c * 4;
+    else return r * PITCH + (((c >> 1) ^ Operand<uint16_t, true, ROWS>::swizzle(r)) << 3) + (c & 1) * 4;
+  }
+  static __device__ __forceinline__ void park(uint16_t* tile, int tid, int i, const u32x4& v) {
+    u32x2 hi, mid, lo;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const float a = __uint_as_float(v[2 * j]), b = __uint_as_float(v[2 * j + 1]);
+      hi[j] = pack_bf16x2(a, b);
+      const float a1 = a - __uint_as_float(hi[j] << 16), b1 = b - __uint_as_float(hi[j] & 0xffff0000u);
+      mid[j] = pack_bf16x2(a1, b1);
+      lo[j] = pack_bf16x2(a1 - __uint_as_float(mid[j] << 16), b1 - __uint_as_float(mid[j] & 0xffff0000u));
+    }
+    uint16_t* p = tile + at(tid, i);
+    *reinterpret_cast<u32x2*>(p) = hi;
+    *reinterpret_cast<u32x2*>(p + ELEMS) = mid;
+    *reinterpret_cast<u32x2*>(p + 2 * ELEMS) = lo;
+  }
+  static __device__ __forceinline__ bf16x8 frag(const uint16_t* tile, int row, int kk, int lane) {
+    if constexpr (!KS) return *reinterpret_cast<const bf16x8*>(tile + (row + (lane & 31)) * PITCH + kk * 16 + 8 * (lane >> 5));
+    else return any_frag<true, ROWS>(tile, row, kk, lane);
+  }
+};
 __device__ __forceinline__ f32x16 any_mfma(const bf16x8& b, const bf16x8& a, const f32x16& acc) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, a, acc, 0, 0, 0);
 }
@@ -171,12 +214,18 @@ __device__ __forceinline__ u32x4 any_scale(uint16_t, const u32x4& v, float f) {
   return r;
 }
 
+template <typename T, int TM> constexpr bool any_split() { return sizeof(T) == 4 && TM >= 64; }
+
 // LDS of one instantiation: two stages; on 32-row tiles also the four waves' partial tiles
 template <typename T, int MODE, int TM, int TN>
 constexpr int any_lds() {
   constexpr bool B_KS = MODE == ANY_DH || MODE == ANY_DX || MODE == ANY_KS || MODE == ANY_DW;
   constexpr int stages = 2 * (Operand<T, MODE == ANY_DW, TM>::ELEMS + Operand<T, B_KS, TN>::ELEMS);
   constexpr int parts = TM == 32 ? 4 * 32 * TN * 4 / (int)sizeof(T) : 0;
+  if (any_split<T, TM>()) {
+    constexpr int pieces = 3 * (Pieces<MODE == ANY_DW, TM>::ELEMS + Pieces<B_KS, TN>::ELEMS) / 2;
+    return stages / 2 > pieces ? stages / 2 : pieces;
+  }
   return stages > parts ? stages : parts;
 }
 
@@ -197,6 +246,7 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
   static_assert(KK == 4, "a step's fragments are dealt to four waves");
   constexpr int AHEAD = TM == 32 ? 4 : 1;  // steps requested ahead
   constexpr int STAGE = OA::ELEMS + OB::ELEMS;
+  constexpr bool SPLIT = any_split<T, TM>();
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = KSPLIT ? 0 : (wave >> 1) * (TM / 2), wn = KSPLIT ? 0 : (wave & 1) * (TN / 2);
 
@@ -340,9 +390,7 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
     }
     request_sources(src, s + SRC);
   };
-  auto park = [&](int slot, int s) {
-    T* As = smem + (s & 1) * STAGE;
-    T* Bs = As + OA::ELEMS;
+  auto prepare = [&](int slot, int s) {  // what was requested, scaled and clipped
     const int kv = K - (MODE == ANY_DX && s >= half_steps ? s - half_steps : s) * BKE;
     if constexpr (FOLD && MODE == ANY_DH) {
 #pragma unroll
@@ -360,6 +408,11 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
 #pragma unroll
       for (int i = 0; i < OB::N; ++i) rb[slot][i] = OB::clip(rb[slot][i], tid, i, kv);
     }
+  };
+  auto park = [&](int slot, int s, int stage) {
+    T* As = smem + stage * STAGE;
+    T* Bs = As + OA::ELEMS;
+    prepare(slot, s);
 #pragma unroll
     for (int i = 0; i < OA::N; ++i) *reinterpret_cast<u32x4*>(As + OA::at(tid, i)) = ra[slot][i];
 #pragma unroll
@@ -390,17 +443,86 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
       for (int i = 0; i < MI; ++i) acc[i][j] = any_mfma(bf, af[i], acc[i][j]);
     }
   };
-  if constexpr (!KSPLIT) {
+  if constexpr (SPLIT) {
+    using PA = Pieces<A_KS, TM>;
+    using PB = Pieces<B_KS, TN>;
+    uint16_t* As = reinterpret_cast<uint16_t*>(smem);
+    uint16_t* Bs = As + 3 * PA::ELEMS;
+    if (steps > 0) {
+      request_sources(0, 0);
+      fetch(0, 0, 0);
+    }
+    for (int s = 0; s < steps; ++s) {
+      prepare(0, s);
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < OA::N; ++i) PA::park(As, tid, i, ra[0][i]);
+#pragma unroll
+      for (int i = 0; i < OB::N; ++i) PB::park(Bs, tid, i, rb[0][i]);
+      if (s + 1 < steps) fetch(0, s + 1, 0);
+      __syncthreads();
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk) {
+        bf16x8 af[3][MI];
+#pragma unroll
+        for (int piece = 0; piece < 3; ++piece)
+#pragma unroll
+          for (int i = 0; i < MI; ++i) af[piece][i] = PA::frag(As + piece * PA::ELEMS, wm + i * 32, kk, lane);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+          bf16x8 bf[3];
+#pragma unroll
+          for (int piece = 0; piece < 3; ++piece) bf[piece] = PB::frag(Bs + piece * PB::ELEMS, bcol(j), kk, lane);
+          f32x16 part[MI];
+#pragma unroll
+          for (int i = 0; i < MI; ++i) part[i] = f32x16{};
+#pragma unroll
+          for (int sum = 2; sum >= 0; --sum)
+#pragma unroll
+            for (int pb = 0; pb <= sum; ++pb)
+#pragma unroll
+              for (int i = 0; i < MI; ++i) part[i] = any_mfma(bf[pb], af[sum - pb][i], part[i]);
+#pragma unroll
+          for (int i = 0; i < MI; ++i) acc[i][j] += part[i];
+        }
+      }
+    }
+    bool nan = false;
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) nan |= acc[i][j][v] != acc[i][j][v];
+    if (__syncthreads_or(nan)) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+      for (int s = 0; s < steps; ++s) {
+        request_sources(0, s);
+        fetch(0, s, 0);
+        __syncthreads();
+        park(0, s, 0);
+        __syncthreads();
+        const T* Af = smem;
+#pragma unroll 1
+        for (int kk = 0; kk < KK; ++kk) multiply(Af, Af + OA::ELEMS, kk);
+      }
+    }
+  } else if constexpr (!KSPLIT) {
     if (steps > 0) {
 #pragma unroll
       for (int i = 0; i < SRC; ++i) request_sources(i, i);
       fetch(0, 0, 0);
-      park(0, 0);
+      park(0, 0, 0);
       if (steps > 1) fetch(0, 1, SRC - 1);
     }
     __syncthreads();
     auto step = [&](int s, int src) {
-      if (s + 1 < steps) park(0, s + 1);
+      if (s + 1 < steps) park(0, s + 1, (s + 1) & 1);
       if (s + 2 < steps) fetch(0, s + 2, src);
       const T* As = smem + (s & 1) * STAGE;
 #pragma unroll
@@ -421,7 +543,7 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
       for (int i = 0; i < AHEAD; ++i) request_sources(i, i);
 #pragma unroll
       for (int i = 0; i < AHEAD; ++i) fetch(i, i, i);
-      park(0, 0);
+      park(0, 0, 0);
       fetch(0, AHEAD, 0);
       phase_barrier();
     }
@@ -430,7 +552,7 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
       for (int i = 0; i < AHEAD; ++i) {
         const int s = s0 + i;
         if (s >= steps) goto done;
-        if (s + 1 < steps) park((i + 1) % AHEAD, s + 1);
+        if (s + 1 < steps) park((i + 1) % AHEAD, s + 1, (s + 1) & 1);
         fetch((i + 1) % AHEAD, s + 1 + AHEAD, (i + 1) % AHEAD);
         const T* As = smem + (s & 1) * STAGE;
         multiply(As, As + OA::ELEMS, wave);
@@ -504,8 +626,10 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
   }
 }
 
+// (two workgroups a CU said to the compiler: at most 256 registers, and products then go to ordinary ones -- from the others every
+// partial sum had to be copied before it could be added)
 template <typename T, int MODE, int TM, int TN, bool FOLD>
-__global__ __launch_bounds__(256) void any_kernel(AnyArgs p) {
+__global__ __launch_bounds__(256, 2) void any_kernel(AnyArgs p) {
   __shared__ __attribute__((aligned(16))) T smem[any_lds<T, MODE, TM, TN>()];
   any_tile<T, MODE, TM, TN, FOLD>(p, blockIdx.x, smem);
 }
@@ -515,7 +639,7 @@ __global__ __launch_bounds__(256) void any_kernel(AnyArgs p) {
 // token's rows along, and the slices' sum beside it, a backward has four launches instead of seven: a training step of 1531 bf16 tokens of
 // 16 x 320 x 232 128 -> 109 us, 512 fp32 of 8 x 256 x 512 126 -> 119, 100 bf16 of 4 x 200 x 104 139 -> 122.
 template <typename T, int TM, int TN>
-__global__ __launch_bounds__(256) void any_dh_gate_kernel(AnyArgs p, GateDw gate, int blocks) {
+__global__ __launch_bounds__(256, 2) void any_dh_gate_kernel(AnyArgs p, GateDw gate, int blocks) {
   constexpr int A = any_lds<T, ANY_DH, TM, TN>(), B = kGateDwLds * 4 / sizeof(T);
   __shared__ __attribute__((aligned(16))) T smem[A > B ? A : B];
   const int block = blockIdx.x;
@@ -527,7 +651,7 @@ __global__ __launch_bounds__(256) void any_dh_gate_kernel(AnyArgs p, GateDw gate
 // ones: with few tiles each they share a launch (at 512 fp32 tokens of 8 experts 26 + 16 us one after the
 // other).  The longer contraction starts first.
 template <typename T, int TX, int TW, bool FOLD>
-__global__ __launch_bounds__(256) void any_dx_dw_kernel(AnyArgs dx, AnyArgs dw, int dx_blocks, int dw_blocks, int dw_first) {
+__global__ __launch_bounds__(256, 2) void any_dx_dw_kernel(AnyArgs dx, AnyArgs dw, int dx_blocks, int dw_blocks, int dw_first) {
   constexpr int A = any_lds<T, ANY_DX, TX, TX>(), B = any_lds<T, ANY_DW, TW, TW>();
   __shared__ __attribute__((aligned(16))) T smem[A > B ? A : B];
   const int block = static_cast<int>(blockIdx.x) - (dw_first ? dw_blocks : 0);  // of dx
@@ -566,17 +690,16 @@ int launch_any(const AnyArgs& p, int dtype, int64_t blocks, hipStream_t s, const
 }
 
 // Large tiles (128 x 128) once they give two workgroups for every CU; before that 64-row ones.  fp32 products
-// run on 32 x 32 tiles where 64-row ones leave CUs without work or, with few rows per expert, are mostly
-// padding: an fp32 step of a 64-row tile is 0.9 us of MFMA time on four waves, full or not.  Experts' forward
+// run on 32 x 32 tiles where 64-row ones leave CUs without work or, with few rows per expert, are mostly padding.  Experts' forward
 // / backward in us, 64 against 32:
-//   few tiles: 40-80 (64 tokens of 8 experts, 256 x 512) 27 / 38 against 18 / 25, 96-192 29 / 44 against
-//     25 / 33, 216-432 (375 rows per expert) 40 / 61 against 48 / 74;
-//   16 experts of 640 x 1024: 25 rows each 88 / 171 against 49 / 97, 64 rows 90 / 201 against 74 / 153, 160 rows
-//     152 / 287 against 134 / 269, 225 rows 152 / 319 against 165 / 332.
-// bf16 steps are 16 times shorter and gain nothing (14 / 17 against 14 / 18, slower with more tiles).
+//   few tiles: 119 (75 rows per expert, 320 x 400) 29 / 40 against 21 / 27, 135 (375, 256 x 300) 26 / 35 against 23 / 31, 152 (250,
+//     512 x 512) 40 / 49 against 34 / 45, 250 (750, 256 x 300) 30 / 42 against 37 / 46, 312 (250, 256 x 512) 34 / 48 against 35 / 47;
+//   16 experts of 640 x 1024: 25 rows each 73 / 124 against 50 / 84, 50 rows 75 / 128 against 67 / 118, 75 rows 77 / 138 against
+//     81 / 138, 250 rows 145 / 279 against 189 / 338.
+// bf16 steps are shorter and gain nothing (14 / 17 against 14 / 18, slower with more tiles).
 int row_tile(const AnyArgs& p, int dtype, int64_t El, int64_t cols) {
   auto tiles = [&](int64_t t) { return (p.rows / t + std::min(El, p.rows)) * ((cols + t - 1) / t); };
-  if (dtype == MI355_F32 && (p.rows <= 160 * El || tiles(64) < 200)) return 32;
+  if (dtype == MI355_F32 && (p.rows <= 64 * El || tiles(64) < 200)) return 32;
   return tiles(128) >= 512 ? 128 : 64;
 }
 
@@ -667,9 +790,13 @@ int any_backward(const AnySeg& g, int dtype, const void* dgate, const void* dup,
   for (int i = 0; i < count; ++i)
     w.dw[i] = {grads[i].a, grads[i].b, grads[i].c, (int)grads[i].M, (int)grads[i].N, 0, 0, grads[i].through};
   w.num_dw = count;
-  const bool dw_large = count && dw_tiles(w, g.El, 128) >= 512;
+  // Weight gradients on 128 x 128 tiles once these fill the chip; fp32 ones where their contraction is long enough to be what
+  // takes the time (us, the backward, 64 / 128: 250 rows an expert 279 / 290, 500 497 / 482, 1000 950 / 895).  fp32 on 32 x 32 tiles while
+  // there are few (us, 64 / 32: 48 tiles 32 / 24, 96 28 / 22, 240 35 / 38).
+  const bool f32 = dtype == MI355_F32;
+  const bool dw_large = count && dw_tiles(w, g.El, 128) >= (f32 ? 448 : 512) && !(f32 && R < 400 * g.El);
   int64_t tiles = count ? dw_tiles(w, g.El, dw_large ? 128 : 64) : 0;
-  const bool dw_small = dtype == MI355_F32 && tiles < 256;  // as in row_tile
+  const bool dw_small = f32 && tiles < 160;
   if (dw_small) tiles = dw_tiles(w, g.El, 32);
   MI355_REQUIRE(tiles < (1ll << 30), "grouped weight gradients: too many tiles");
   const int t = row_tile(p, dtype, g.El, D);
