@@ -689,7 +689,11 @@ int launch_any(const AnyArgs& p, int dtype, int64_t blocks, hipStream_t s, const
   return check_launch(what);
 }
 
-// Large tiles (128 x 128) once they give two workgroups for every CU; before that 64-row ones.  fp32 products
+// Large tiles (128 x 128) once they give two workgroups for every CU, for bf16 already where they give every second CU one: its
+// steps are mostly loads and LDS, which a large tile has half as many of (the forward, us, 64 / 128: 141 tiles, 2000 rows of 32 x
+// 300 x 300, 18.3 / 19.0; 156, 4000 of 8 x 480 x 432, 30.7 / 26.4; 186, 6000 of 16 x 440 x 360, 41.7 / 34.6; 252, 4000 of 32 x
+// 480 x 432, 40.0 / 33.5).  Not so dH, whose end has as much to do (4000 of 8 x 480 x 432: the backward 52 / 56), and not the input
+// gradient where the weight gradients share its launch, which is worth more (8000 of 4 x 480 x 432: 86 / 94): two a CU.  fp32 products
 // run on 32 x 32 tiles where 64-row ones leave CUs without work or, with few rows per expert, are mostly padding.  Experts' forward
 // / backward in us, 64 against 32:
 //   few tiles: 119 (75 rows per expert, 320 x 400) 29 / 40 against 21 / 27, 135 (375, 256 x 300) 26 / 35 against 23 / 31, 152 (250,
@@ -697,17 +701,17 @@ int launch_any(const AnyArgs& p, int dtype, int64_t blocks, hipStream_t s, const
 //   16 experts of 640 x 1024: 25 rows each 73 / 124 against 50 / 84, 50 rows 75 / 128 against 67 / 118, 75 rows 77 / 138 against
 //     81 / 138, 250 rows 145 / 279 against 189 / 338.
 // bf16 steps are shorter and gain nothing (14 / 17 against 14 / 18, slower with more tiles).
-int row_tile(const AnyArgs& p, int dtype, int64_t El, int64_t cols) {
+int row_tile(const AnyArgs& p, int dtype, int64_t El, int64_t cols, int bf16_large) {
   auto tiles = [&](int64_t t) { return (p.rows / t + std::min(El, p.rows)) * ((cols + t - 1) / t); };
   if (dtype == MI355_F32 && (p.rows <= 64 * El || tiles(64) < 200)) return 32;
-  return tiles(128) >= 512 ? 128 : 64;
+  return tiles(128) >= (dtype == MI355_F32 ? 512 : bf16_large) ? 128 : 64;
 }
 
 template <int MODE>
 int launch_rows(AnyArgs& p, int dtype, int64_t tile_capacity, int64_t El, int64_t cols, hipStream_t s, const char* what,
                 const GateDw* gate = nullptr) {
   constexpr bool GU = MODE == ANY_GATEUP;
-  const int t = row_tile(p, dtype, El, cols), width = GU && t == 128 ? 64 : t;
+  const int t = row_tile(p, dtype, El, cols, MODE == ANY_DH ? 512 : 150), width = GU && t == 128 ? 64 : t;
   p.col_tiles = (int)((cols + width - 1) / width);
   const int64_t blocks = tile_capacity * (256 / t) * p.col_tiles;
   MI355_REQUIRE(blocks < (1ll << 30), "%s: too many tiles", what);
@@ -794,12 +798,15 @@ int any_backward(const AnySeg& g, int dtype, const void* dgate, const void* dup,
   // takes the time (us, the backward, 64 / 128: 250 rows an expert 279 / 290, 500 497 / 482, 1000 950 / 895).  fp32 on 32 x 32 tiles while
   // there are few (us, 64 / 32: 48 tiles 32 / 24, 96 28 / 22, 240 35 / 38).
   const bool f32 = dtype == MI355_F32;
-  const bool dw_large = count && dw_tiles(w, g.El, 128) >= (f32 ? 448 : 512) && !(f32 && R < 400 * g.El);
+  // bf16 ones also where the input gradient is large enough for a launch of its own (16000 rows of 8 x 480 x 432, 384 tiles: 183 / 162;
+  // a step of 4000 tokens of 4 x 480 x 428, four each, 192 tiles: 264 / 277).
+  const bool alone = !f32 && drows && row_tile(p, dtype, g.El, D, 512) == 128;
+  const bool dw_large = count && dw_tiles(w, g.El, 128) >= (f32 ? 448 : alone ? 300 : 512) && !(f32 && R < 400 * g.El);
   int64_t tiles = count ? dw_tiles(w, g.El, dw_large ? 128 : 64) : 0;
   const bool dw_small = f32 && tiles < 160;
   if (dw_small) tiles = dw_tiles(w, g.El, 32);
   MI355_REQUIRE(tiles < (1ll << 30), "grouped weight gradients: too many tiles");
-  const int t = row_tile(p, dtype, g.El, D);
+  const int t = row_tile(p, dtype, g.El, D, count && !dw_large ? 512 : 150);
   if (drows && count && !dw_large && t < 128) {
     p.col_tiles = (int)((D + t - 1) / t);
     const int64_t dx_blocks = g.tile_capacity * (256 / t) * p.col_tiles;
