@@ -25,7 +25,7 @@ int bf16_grouped_fwd(const void* rows, const int32_t* token_of_row, int64_t num_
 int bf16_fused_dot_slots(int64_t F);
 int bf16_grouped_linear_dx(const void* dy, const void* w, const int32_t* seg_offsets, const int32_t* seg_counts,
                            const int32_t* tile_expert, const int32_t* tile_row0, const int32_t* num_tiles,
-                           int64_t tile_capacity, void* dx, int64_t O, int64_t I, hipStream_t s);
+                           int64_t tile_capacity, void* dx, int64_t El, int64_t O, int64_t I, hipStream_t s);
 int bf16_grouped_bwd(const void* dy, const void* rows, const int32_t* token_of_row, int64_t num_tokens,
                      const void* w1, const void* w3, const void* w2, const void* gate, const void* up,
                      const void* h, const float* row_scale, float* dot_partial,
@@ -343,7 +343,7 @@ extern "C" int mi355_grouped_linear_bwd(const void* dy, const void* x, const voi
   if (dtype == MI355_BF16 && bf16_fast_path_ok(O, I) && rows) {
     if (dx)
       if (int rc = bf16_grouped_linear_dx(dy, w, seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles,
-                                          tile_capacity, dx, O, I, s))
+                                          tile_capacity, dx, El, O, I, s))
         return rc;
     // dw[e] (O, I) = dy[segment]^T . x[segment]: the dW2 product of the SwiGLU backward
     if (dw)

@@ -117,12 +117,14 @@ struct TileMeta {
   int k_start;  // the contraction's first K step; it goes on from step 0 after the last
 };
 
-// sum over each group of 16 consecutive lanes, left in all 16 (DPP row operations)
+// sum over each group of 16 (8) consecutive lanes, left in all of them (DPP row operations)
+template <int LANES = 16>
 __device__ __forceinline__ float row16_sum(float v) {
   v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xf, 0xf, false));   // quad_perm [1,0,3,2]
   v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xf, 0xf, false));   // quad_perm [2,3,0,1]
   v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xf, 0xf, false));  // row_half_mirror
-  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xf, 0xf, false));  // row_mirror
+  if constexpr (LANES == 16)
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x140, 0xf, 0xf, false));  // row_mirror
   return v;
 }
 
@@ -147,7 +149,7 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
   constexpr bool B_KS = (DH_LIKE || MODE == RM_DX);
   static_assert(!GATHER || MODE == RM_GATEUP || MODE == RM_DH, "only gate/up and dH gather their rows");
   static_assert(!TURN || !B_KS, "only contractions that are contiguous in memory are turned");
-  static_assert(!(GATHER && MODE == RM_DH) || NJ == 4, "the fused dH epilogue reduces over 16 lanes per row");
+  static_assert(!(GATHER && MODE == RM_DH) || NJ == 4 || NJ == 2, "the fused dH epilogue reduces over 16 lanes per row, or 8 and a second wave");
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -448,12 +450,13 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
   // 16-column tile = 4*(lane>>4) + i.
   uint16_t* st = smem + wave * (64 * 136);  // 8 waves x 17 KiB < 160 KiB; the barrier ending the K loop freed the tiles
   if constexpr (MODE == RM_GATEUP) {
-    // per 32-row half: three 32 x 64 tiles gate | up | h at columns 0, 64, 128 of a
-    // [32][192+8] region (12.5 KiB per wave); without gate and up, h alone in a [32][64+8] region
+    // per 32-row half: three 32 x 16 NJ tiles gate | up | h side by side, a [32][48 NJ + 8] region (12.5 KiB
+    // per wave with NJ = 4); without gate and up, h alone in a [32][16 NJ + 8] region
     constexpr int NT3 = SAVE_GU ? 3 : 1;       // output tiles per row
-    using S = WaveStage<64 * NT3>;
+    constexpr int WC = 16 * NJ, CPT = WC / 8;  // columns and chunks of one of them
+    using S = WaveStage<WC * NT3>;
     uint16_t* sg = smem + wave * (32 * S::PITCH);
-    const int f0 = n0 + wn * 64;
+    const int f0 = n0 + wn * WC;
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
       if (wave_m + half * 32 >= valid) continue;  // no real rows in this half (uniform per wave)
@@ -472,21 +475,21 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
           }
           if constexpr (SAVE_GU) {
             S::put16(sg, ml, j * 16, lane, g[0], g[1], g[2], g[3]);
-            S::put16(sg, ml, 64 + j * 16, lane, u[0], u[1], u[2], u[3]);
+            S::put16(sg, ml, WC + j * 16, lane, u[0], u[1], u[2], u[3]);
           }
-          S::put16(sg, ml, (SAVE_GU ? 128 : 0) + j * 16, lane, h[0], h[1], h[2], h[3]);
+          S::put16(sg, ml, (SAVE_GU ? 2 * WC : 0) + j * 16, lane, h[0], h[1], h[2], h[3]);
         }
       __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the wave's own LDS writes have landed
       __builtin_amdgcn_wave_barrier();
-      // 32 rows x NT3 tiles x 8 chunks, 4 NT3 per lane
+      // 32 rows x NT3 tiles x CPT chunks, CPT / 2 NT3 per lane
 #pragma unroll 4
-      for (int it = 0; it < 4 * NT3; ++it) {
+      for (int it = 0; it < CPT / 2 * NT3; ++it) {
         const int idx = it * 64 + lane;
-        const int m = idx / (8 * NT3), rem = idx % (8 * NT3), t = rem >> 3, c = rem & 7;
+        const int m = idx / (CPT * NT3), rem = idx % (CPT * NT3), t = rem / CPT, c = rem % CPT;
         const int f = f0 + c * 8;  // < F: tiles never overhang in the columns
         const int mr = wm + half * 32 + m;
         if (mr < valid) {
-          const u32x4 v = *reinterpret_cast<const u32x4*>(sg + m * S::PITCH + t * 64 + c * 8);
+          const u32x4 v = *reinterpret_cast<const u32x4*>(sg + m * S::PITCH + t * WC + c * 8);
           uint16_t* dst = (!SAVE_GU ? p.o2 : (t == 0 ? p.o0 : (t == 1 ? p.o1 : p.o2))) + static_cast<int64_t>(row0 + mr) * F + f;
           *reinterpret_cast<u32x4*>(dst) = v;
         }
@@ -539,6 +542,8 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
         chunk_at(it, m, c);
         return row0 + wm + m;
       };
+      [[maybe_unused]] float* dots = reinterpret_cast<float*>(st + 64 * S::PITCH);
+      static_assert(64 * S::PITCH + 128 <= 64 * 136 || NJ == 4, "the rows' sums lie behind the wave's tile");
       u32x4 gq[G], uq[G];
       float sq[G];
 #pragma unroll
@@ -602,10 +607,11 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
             // columns below the tile's nominal start belong to its neighbour (a last tile
             // that would overhang starts early): they must not be counted twice
             if (c0 + c * 8 < ntile * BNT) dot = 0.0f;
-            const float total = row16_sum(dot);
+            const float total = row16_sum<CH>(dot);
             // all 16 lanes of the row store the same value to the same address (unconditional,
-            // like every other access of this epilogue)
-            p.dot_partial[static_cast<int64_t>(row0 + wm + m) * p.dot_slots + ntile * WN + wn] = total;
+            // like every other access of this epilogue); of a narrow tile, whose 128 columns are two waves', to LDS
+            if constexpr (NJ == 4) p.dot_partial[static_cast<int64_t>(row0 + wm + m) * p.dot_slots + ntile * WN + wn] = total;
+            else dots[m] = total;
           }
         }
         if (g0 + G < CH) {
@@ -634,6 +640,18 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
   // every wave is done with its staging region before the next tile's operands are parked;
   // only LDS traffic is waited for, the tile's stores keep draining
   phase_barrier();
+  if constexpr (MODE == RM_DH && GATHER && NJ == 2) {
+    // a narrow tile's slot: both waves' sums; the slots past the last tile's, which a wide tile would have filled, are zero
+    if (wn == 0 && lane < valid - wave_m) {
+      const float* dots = reinterpret_cast<const float*>(st + 64 * WaveStage<32 * NJ>::PITCH);
+      const float* other = reinterpret_cast<const float*>(st + 64 * 136 + 64 * WaveStage<32 * NJ>::PITCH);
+      float* slot = p.dot_partial + static_cast<int64_t>(row0 + wm + lane) * p.dot_slots;
+      slot[ntile] = dots[lane] + other[lane];
+      if (ntile == p.n_tiles - 1)
+        for (int i = p.n_tiles; i < p.dot_slots; ++i) slot[i] = 0.0f;
+    }
+    phase_barrier();
+  }
   if (!more) break;
   within += stride;
   cur = nxt;
@@ -981,30 +999,39 @@ static unsigned resident_blocks() {
 
 constexpr int W_LDS_BYTES = 8 * 64 * 136 * 2;  // 139264: the 8 epilogue regions (> 2 stages = 131072)
 
-// width: output columns; gate/up tiles hold both halves of their column range.  Tiles are always
-// 256 wide (a 192-wide KS tile would not hold the swizzle: 24 chunks per row are not a multiple
+// Whether a product of El experts and n 256-column tiles runs on 128-column ones instead: twice the work items, each with the
+// whole contraction.  Where experts of equal load would occupy at most half the CUs (three eighths where the tiles are
+// mostly full, and a narrow one so has as many rows to stage for half the products).  us, wide / narrow: the block forward, 1000 tokens of
+// 16 experts of 1024 x 512, four each, 69 / 55, of 32 63 / 53, 300 tokens 55 / 47 and 56 / 49; a training step of 2000 of 16 226 / 212
+// (with dH narrow; gate/up and down too, 128 tiles of 250 rows, 215), of 32 230 / 217, of 60 267 / 257, 1000 of 64, six each, 249 / 235,
+// 1000 of 16 of 1984 x 1024 338 / 315; 128 tiles of 250 rows (4000 of 16) 326 / 334, 4000 of 60 394 / 418.
+// One dense segment: the input gradient alone (the dH of 4096 rows x 2048 columns is 16 x 8 tiles).  It runs beside other products, and
+// narrow gate/up and down tiles take CUs those would have had (one rank's share, 1000 tokens: 595 / 638).
+static bool narrow(int mode, int64_t El, int64_t n, int64_t tile_capacity) {
+  const int64_t cus = resident_blocks();
+  if (El == 1) return (mode == RM_DH || mode == RM_DLIN) && tile_capacity * n * 4 <= cus * 3;
+  const int64_t spare = std::max<int64_t>(tile_capacity - El - 1, 0);  // 256 rows each
+  const int64_t tiles = El * std::max<int64_t>((spare + El - 1) / El, 1);
+  return tiles * n <= (spare * 10 > tiles * 7 ? cus * 3 / 8 : cus / 2);
+}
+
+// width: output columns; gate/up tiles hold both halves of their column range.  Tiles are
+// 256 or 128 wide (a 192-wide KS tile would not hold the swizzle: 24 chunks per row are not a multiple
 // of the 16 the key permutes); an overhanging last tile shifts back.
 template <int MODE, bool GATHER = false, bool SAVE_GU = true, bool TURN = false>
-static int launch_row(RowArgs& a, int64_t width, int64_t tile_capacity, hipStream_t s, const char* what) {
+static int launch_row(RowArgs& a, int64_t width, int64_t El, int64_t tile_capacity, hipStream_t s, const char* what) {
   constexpr int div = MODE == RM_GATEUP ? 2 : 1;
   a.n_tiles = (int)((width + 256 / div - 1) / (256 / div));
-  // A product with so few row tiles that 256-column tiles would leave a quarter of the CUs or more without work
-  // (the dH of one dense segment: 4096 rows x 2048 columns are 16 x 8 tiles) runs on 128-column
-  // tiles instead: twice the work items, each with the whole contraction.  Only where the
-  // epilogue does not depend on the tile width (the folded dH writes one partial per 128
-  // columns of a 256-column tile).
-  if constexpr ((MODE == RM_DH || MODE == RM_DLIN) && !GATHER) {
-    if (tile_capacity * a.n_tiles * 4 <= resident_blocks() * 3 && width >= 128) {  // (the capacity is an upper bound)
-      a.n_tiles = (int)((width + 127) / 128);
-      static PerDeviceOnce narrow_configured;
-      if (narrow_configured.needed()) {
-        if (int rc = set_lds(row_tiled_kernel<MODE, 2, GATHER, 4, SAVE_GU>, W_LDS_BYTES)) return rc;
-        narrow_configured.done();
-      }
-      const unsigned blocks = std::min(round8(tile_capacity * a.n_tiles), resident_blocks());
-      hipLaunchKernelGGL((row_tiled_kernel<MODE, 2, GATHER, 4, SAVE_GU>), dim3(blocks), dim3(NT), W_LDS_BYTES, s, a);
-      return check_launch(what);
+  if (narrow(MODE, El, a.n_tiles, tile_capacity)) {
+    a.n_tiles = (int)((width + 128 / div - 1) / (128 / div));
+    static PerDeviceOnce narrow_configured;
+    if (narrow_configured.needed()) {
+      if (int rc = set_lds(row_tiled_kernel<MODE, 2, GATHER, 4, SAVE_GU, TURN>, W_LDS_BYTES)) return rc;
+      narrow_configured.done();
     }
+    const unsigned blocks = std::min(round8(tile_capacity * a.n_tiles), resident_blocks());
+    hipLaunchKernelGGL((row_tiled_kernel<MODE, 2, GATHER, 4, SAVE_GU, TURN>), dim3(blocks), dim3(NT), W_LDS_BYTES, s, a);
+    return check_launch(what);
   }
   static PerDeviceOnce configured;  // one per kernel instantiation
   if (configured.needed()) {
@@ -1066,22 +1093,22 @@ int bf16_grouped_fwd(const void* rows, const int32_t* token_of_row, int64_t num_
     const bool save = gate != nullptr;
     int rc;
     if (token_of_row && turned(El, row_capacity, D))
-      rc = save ? launch_row<RM_GATEUP, true, true, true>(a, F, tile_capacity, s, "grouped gate/up")
-                : launch_row<RM_GATEUP, true, false, true>(a, F, tile_capacity, s, "grouped gate/up (h only)");
+      rc = save ? launch_row<RM_GATEUP, true, true, true>(a, F, El, tile_capacity, s, "grouped gate/up")
+                : launch_row<RM_GATEUP, true, false, true>(a, F, El, tile_capacity, s, "grouped gate/up (h only)");
     else if (token_of_row)
-      rc = save ? launch_row<RM_GATEUP, true>(a, F, tile_capacity, s, "grouped gate/up")
-                : launch_row<RM_GATEUP, true, false>(a, F, tile_capacity, s, "grouped gate/up (h only)");
+      rc = save ? launch_row<RM_GATEUP, true>(a, F, El, tile_capacity, s, "grouped gate/up")
+                : launch_row<RM_GATEUP, true, false>(a, F, El, tile_capacity, s, "grouped gate/up (h only)");
     else
-      rc = save ? launch_row<RM_GATEUP>(a, F, tile_capacity, s, "grouped gate/up")
-                : launch_row<RM_GATEUP, false, false>(a, F, tile_capacity, s, "grouped gate/up (h only)");
+      rc = save ? launch_row<RM_GATEUP>(a, F, El, tile_capacity, s, "grouped gate/up")
+                : launch_row<RM_GATEUP, false, false>(a, F, El, tile_capacity, s, "grouped gate/up (h only)");
     if (rc) return rc;
   }
   if (stages & STAGE_DOWN) {
     RowArgs b = a;
     b.a_src = nullptr;
     b.a0 = (const uint16_t*)h; b.b0 = (const uint16_t*)w2; b.o0 = (uint16_t*)y;
-    if (int rc = turned(El, row_capacity, F) ? launch_row<RM_DOWN, false, true, true>(b, D, tile_capacity, s, "grouped down")
-                      : launch_row<RM_DOWN>(b, D, tile_capacity, s, "grouped down"))
+    if (int rc = turned(El, row_capacity, F) ? launch_row<RM_DOWN, false, true, true>(b, D, El, tile_capacity, s, "grouped down")
+                      : launch_row<RM_DOWN>(b, D, El, tile_capacity, s, "grouped down"))
       return rc;
   }
   return MI355_OK;
@@ -1090,12 +1117,12 @@ int bf16_grouped_fwd(const void* rows, const int32_t* token_of_row, int64_t num_
 // dx = dy . w[e] over the listed segments: dy (rows, O), w (El, O, I), dx (rows, I)
 int bf16_grouped_linear_dx(const void* dy, const void* w, const int32_t* seg_offsets, const int32_t* seg_counts,
                            const int32_t* tile_expert, const int32_t* tile_row0, const int32_t* num_tiles,
-                           int64_t tile_capacity, void* dx, int64_t O, int64_t I, hipStream_t s) {
+                           int64_t tile_capacity, void* dx, int64_t El, int64_t O, int64_t I, hipStream_t s) {
   RowArgs a{};
   a.seg_offsets = seg_offsets; a.seg_counts = seg_counts; a.tile_expert = tile_expert;
   a.tile_row0 = tile_row0; a.num_tiles = num_tiles; a.D = (int)O; a.F = (int)I;
   a.a0 = (const uint16_t*)dy; a.b0 = (const uint16_t*)w; a.o0 = (uint16_t*)dx;
-  return launch_row<RM_DLIN>(a, I, tile_capacity, s, "grouped linear dx");
+  return launch_row<RM_DLIN>(a, I, El, tile_capacity, s, "grouped linear dx");
 }
 
 int bf16_fused_dot_slots(int64_t F) {
@@ -1125,17 +1152,17 @@ int bf16_grouped_bwd(const void* dy, const void* rows, const int32_t* token_of_r
       a.a_src = token_of_row; a.a_rows = (int)num_tokens; a.row_scale = row_scale; a.dot_partial = dot_partial;
       a.o2 = (uint16_t*)const_cast<void*>(h);
       a.dot_slots = bf16_fused_dot_slots(F);
-      if (int rc = launch_row<RM_DH, true>(a, F, tile_capacity, s, "grouped dh + combine")) return rc;
+      if (int rc = launch_row<RM_DH, true>(a, F, El, tile_capacity, s, "grouped dh + combine")) return rc;
       a.a_src = nullptr;
     } else {
-      if (int rc = launch_row<RM_DH>(a, F, tile_capacity, s, "grouped dh")) return rc;
+      if (int rc = launch_row<RM_DH>(a, F, El, tile_capacity, s, "grouped dh")) return rc;
     }
   }
   if (drows && (stages & STAGE_DX)) {
     RowArgs b = a;
     b.a0 = (const uint16_t*)dgate; b.a1 = (const uint16_t*)dup;
     b.b0 = (const uint16_t*)w1; b.b1 = (const uint16_t*)w3; b.o0 = (uint16_t*)drows;
-    if (int rc = launch_row<RM_DX>(b, D, tile_capacity, s, "grouped drows")) return rc;
+    if (int rc = launch_row<RM_DX>(b, D, El, tile_capacity, s, "grouped drows")) return rc;
   }
   static PerDeviceOnce wconfigured;
   if (wconfigured.needed()) {
