@@ -116,6 +116,14 @@ Tensor carve(const Tensor& like, Layout layout) {
 
 constexpr int64_t kShortRowSum = 6 << 20;  // elements of the tokens
 
+// A folded backward so small that the host is what takes the time: a second stream's fork and join cost it more than the weight
+// gradients gain beside the input gradient.  A training step, us, beside / behind it: 200, 600, 1000 tokens of 16 experts of 1024 x 512,
+// four each, 166 / 129, 161 / 146, 176 / 160, 2000 of them 217 / 227; 200, 1000 of 32 171 / 151, 176 / 176, 2000 218 / 225; 300 of 60 of 512 x
+// 448, two each, 183 / 140; 1500 of 32 of 640 x 640, three each, 288 tiles, 176 / 196; 200 of 60 of 1024 x 512, 480 tiles, 177 / 190.
+bool short_backward(int64_t El, int64_t D, int64_t F, int64_t R) {
+  return El * ((D + 255) / 256) * ((F + 255) / 256) <= 256 && R * D * F <= (int64_t{1} << 31);
+}
+
 // What the backward reads besides the inputs, in one allocation: the plan's and the router's arrays, the
 // activations, the shared expert's plan and activations.
 struct Kept {
@@ -440,8 +448,8 @@ Grads block_backward(const Block& b, const Tensor& kept, const Tensor& dout_, co
   // ---- shared expert: dH and dX beside the routed part where they may be, its weight gradients in front
   // of the routed ones on the stream those use
   SideStream* aux = run_shared && c.overlap && routed ? side_stream(device, main, 1) : nullptr;
-  SideStream* side = routed && need.x && ((b.folded && need.experts) || (b.shared_folded && aux && need.shared))
-                         ? side_stream(device, main, 0) : nullptr;
+  const bool beside = b.folded && need.experts && (aux || !short_backward(b.El, b.D, b.F, b.R));
+  SideStream* side = routed && need.x && (beside || (b.shared_folded && aux && need.shared)) ? side_stream(device, main, 0) : nullptr;
   Fork shared(aux, main), weights(side, main);
   if (run_shared) {
     if (aux) shared.start();
