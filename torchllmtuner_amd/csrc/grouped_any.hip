@@ -5,8 +5,8 @@
 // TM x TN output tile, each wave (TM/2) x (TN/2) in 32x32 accumulators (v_mfma_f32_32x32x16_bf16; fp32 on 32-row
 // tiles v_mfma_f32_32x32x2_f32, on larger ones products of bf16 pieces, below), 128 bytes of the contraction per step,
 // two LDS stages (of pieces one), the next step's operands held in registers.  Operands are fetched 16 bytes at a time whatever the width
-// (buffer loads: dword alignment suffices for them, and what lies past a matrix reads as zero; the ends store
-// four elements at a time, so the matrices themselves start on 16-byte boundaries); the tail of
+// (buffer loads: dword alignment suffices for them, and what lies past a matrix reads as zero; the ends
+// access whole fours of elements, so the matrices themselves start on 16-byte boundaries); the tail of
 // the contraction is zeroed as it is parked.  LDS holds an operand as it lies in memory -- contraction
 // contiguous [row][128 B + 16] or strided [k][cols], padded (fp32) or its chunks swizzled (bf16) so that fragment reads
 // are free of bank conflicts -- and the fragment reads (b128, b32, or the transposing b64 for bf16)
@@ -68,14 +68,32 @@ template <> struct El<uint16_t> {
 
 __device__ __forceinline__ f32x4 any_pack(float, float a, float b, float c, float d) { return {a, b, c, d}; }
 __device__ __forceinline__ u32x2 any_pack(uint16_t, float a, float b, float c, float d) { return {pack2(a, b), pack2(c, d)}; }
-__device__ __forceinline__ void any_unpack(const f32x4& v, float (&f)[4]) {
+// COUNT values of a row, on 8 bytes (bf16) or 16
+template <typename T, int COUNT> struct Row;
+template <> struct Row<float, 4> {
+  static __device__ __forceinline__ void load(const float* p, float (&f)[4]) {
+    const f32x4 v = *reinterpret_cast<const f32x4*>(p);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) f[i] = v[i];
-}
-__device__ __forceinline__ void any_unpack(const u32x2& v, float (&f)[4]) {
+    for (int i = 0; i < 4; ++i) f[i] = v[i];
+  }
+  template <typename V> static __device__ __forceinline__ void store(float* p, const V& v) {
+    *reinterpret_cast<f32x4*>(p) = f32x4{v[0], v[1], v[2], v[3]};
+  }
+};
+template <int COUNT> struct Row<uint16_t, COUNT> {
+  typedef uint32_t Words __attribute__((ext_vector_type(COUNT / 2), aligned(8)));
+  static __device__ __forceinline__ void load(const uint16_t* p, float (&f)[COUNT]) {
+    const Words v = *reinterpret_cast<const Words*>(p);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) f[i] = __uint_as_float(i & 1 ? v[i >> 1] & 0xffff0000u : v[i >> 1] << 16);
-}
+    for (int i = 0; i < COUNT; ++i) f[i] = __uint_as_float(i & 1 ? v[i >> 1] & 0xffff0000u : v[i >> 1] << 16);
+  }
+  template <typename V> static __device__ __forceinline__ void store(uint16_t* p, const V& v) {
+    Words w;
+#pragma unroll
+    for (int i = 0; i < COUNT / 2; ++i) w[i] = pack2(v[2 * i], v[2 * i + 1]);
+    *reinterpret_cast<Words*>(p) = w;
+  }
+};
 template <typename T>
 __device__ __forceinline__ float any_round(float v) {
   if constexpr (sizeof(T) == 2) return round_bf16(v);
@@ -511,6 +529,7 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
 #pragma unroll 1
         for (int kk = 0; kk < KK; ++kk) multiply(Af, Af + OA::ELEMS, kk);
       }
+      __syncthreads();
     }
   } else if constexpr (!KSPLIT) {
     if (steps > 0) {
@@ -579,50 +598,83 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
     }
   }
 
-  // ---- epilogue: lane = output row lane & 31 of the block, four consecutive columns per q
-  using V4 = typename El<T>::V4;
+  // ---- the fused ends, on N values of one output row from column n on
+  auto finish = [&](int64_t at, auto count, const auto& v, const auto& u) {
+    constexpr int COUNT = decltype(count)::value;
+    using C = Row<T, COUNT>;
+    if constexpr (MODE == ANY_GATEUP) {
+      float h[COUNT];
 #pragma unroll
-  for (int i = 0; i < MI; ++i) {
-    const int m = wm + i * 32 + (lane & 31);
-    if (m >= m_valid) continue;
+      for (int r = 0; r < COUNT; ++r) h[r] = any_round<T>(v[r] / (1.0f + expf(-v[r]))) * u[r];
+      C::store(C0 + at, v);
+      C::store(static_cast<T*>(p.c1) + at, u);
+      C::store(static_cast<T*>(p.c2) + at, h);
+    } else if constexpr (MODE == ANY_DH) {
+      float g[COUNT], up[COUNT], dg[COUNT], du[COUNT];
+      C::load(static_cast<const T*>(p.gate) + at, g);
+      C::load(static_cast<const T*>(p.up) + at, up);
 #pragma unroll
-    for (int j = 0; j < (MODE == ANY_GATEUP ? NJ / 2 : NJ); ++j)
+      for (int r = 0; r < COUNT; ++r) {
+        const float sig = 1.0f / (1.0f + expf(-g[r]));
+        du[r] = v[r] * any_round<T>(g[r] * sig);
+        dg[r] = any_round<T>(v[r] * up[r]) * (sig * (1.0f + g[r] * (1.0f - sig)));
+      }
+      C::store(C0 + at, dg);
+      C::store(static_cast<T*>(p.c1) + at, du);
+    } else {
+      C::store(C0 + at, v);
+    }
+  };
+  const int64_t c_row0 = MODE == ANY_DW ? m0 : row0;
+  // the accumulators hold, per lane, output row lane & 31 of a block and four consecutive columns per q
+  if constexpr (KSPLIT) {
+    const int m = lane & 31;
 #pragma unroll
-      for (int q = 0; q < (KSPLIT ? 1 : 4); ++q) {
-        const int n = n0 + (KSPLIT ? wave * 8 : MODE == ANY_GATEUP ? (wave & 1) * (TN / 4) : wn) + j * 32 + q * 8 + 4 * (lane >> 5);
-        if (n >= N) continue;  // N is a multiple of four
-        const int64_t at = (MODE == ANY_DW ? static_cast<int64_t>(m0 + m) : row0 + m) * N + n;
-        const f32x16& c = acc[i][j];
-        float v[4] = {c[q * 4], c[q * 4 + 1], c[q * 4 + 2], c[q * 4 + 3]};
-        if constexpr (MODE == ANY_GATEUP) {
-          const f32x16& cu = acc[i][j + NJ / 2];
-          float h[4], u[4];
+    for (int j = 0; j < (MODE == ANY_GATEUP ? NJ / 2 : NJ); ++j) {
+      const int n = n0 + wave * 8 + j * 32 + 4 * (lane >> 5);
+      if (m >= m_valid || n >= N) continue;  // N is a multiple of four
+      const f32x16 &c = acc[0][j], &cu = acc[0][MODE == ANY_GATEUP ? j + NJ / 2 : j];
+      finish((c_row0 + m) * N + n, std::integral_constant<int, 4>{}, f32x4{c[0], c[1], c[2], c[3]}, f32x4{cu[0], cu[1], cu[2], cu[3]});
+    }
+  } else {
+    // Through LDS, 32 rows at a time, so that a row's columns are read and written together, 16 bytes a lane: four columns of 32
+    // rows an instruction were 32 lines for 256 bytes (bf16).  Experts' forward / backward, us, before and now: 16000 rows of 8 x 480 x
+    // 432 70 / 163, 66 / 135; of 32 x 472 x 364 79 / 167, 75 / 148; 6000 of 16 x 440 x 360 34 / 69, 33 / 63; fp32, 16000 of 16 x
+    // 640 x 1024 472 / 976, 463 / 958.
+    constexpr int E = OA::E, NB = MODE == ANY_GATEUP ? NJ / 2 : NJ, W = 32 * NB, CH = W / E, P = W + E;
+    constexpr int TILES = MODE == ANY_GATEUP ? 2 : 1;
+    static_assert(4 * TILES * 32 * P <= any_lds<T, MODE, TM, TN>(), "the waves' tiles fit");
+    T* st = smem + wave * (TILES * 32 * P);
+    const int c0 = n0 + (MODE == ANY_GATEUP ? (wave & 1) * (TN / 4) : wn);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            v[r] = any_round<T>(v[r]);
-            u[r] = any_round<T>(cu[q * 4 + r]);
-            h[r] = any_round<T>(v[r] / (1.0f + expf(-v[r]))) * u[r];
-          }
-          *reinterpret_cast<V4*>(C0 + at) = any_pack(T{}, v[0], v[1], v[2], v[3]);
-          *reinterpret_cast<V4*>(static_cast<T*>(p.c1) + at) = any_pack(T{}, u[0], u[1], u[2], u[3]);
-          *reinterpret_cast<V4*>(static_cast<T*>(p.c2) + at) = any_pack(T{}, h[0], h[1], h[2], h[3]);
-        } else if constexpr (MODE == ANY_DH) {
-          float g[4], u[4], dg[4], du[4];
-          any_unpack(*reinterpret_cast<const V4*>(static_cast<const T*>(p.gate) + at), g);
-          any_unpack(*reinterpret_cast<const V4*>(static_cast<const T*>(p.up) + at), u);
+    for (int i = 0; i < MI; ++i) {
+      if (wm + i * 32 >= m_valid) break;
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float dh = any_round<T>(v[r]);
-            const float sig = 1.0f / (1.0f + expf(-g[r]));
-            du[r] = dh * any_round<T>(g[r] * sig);
-            dg[r] = any_round<T>(dh * u[r]) * (sig * (1.0f + g[r] * (1.0f - sig)));
-          }
-          *reinterpret_cast<V4*>(C0 + at) = any_pack(T{}, dg[0], dg[1], dg[2], dg[3]);
-          *reinterpret_cast<V4*>(static_cast<T*>(p.c1) + at) = any_pack(T{}, du[0], du[1], du[2], du[3]);
-        } else {
-          *reinterpret_cast<V4*>(C0 + at) = any_pack(T{}, v[0], v[1], v[2], v[3]);
+      for (int j = 0; j < NJ; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f32x16& c = acc[i][j];
+          *reinterpret_cast<typename El<T>::V4*>(st + ((j / NB) * 32 + (lane & 31)) * P + (j % NB) * 32 + q * 8 + 4 * (lane >> 5)) =
+              any_pack(T{}, c[q * 4], c[q * 4 + 1], c[q * 4 + 2], c[q * 4 + 3]);
+        }
+      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the wave's own writes have landed
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int it = 0; it < CH / 2; ++it) {
+        const int idx = it * 64 + lane, m = idx / CH, c = (idx % CH) * E;
+        const int row = wm + i * 32 + m, n = c0 + c;
+        if (row < m_valid && n < N) {
+          float v[E], u[E];
+          Row<T, E>::load(st + m * P + c, v);
+          if constexpr (MODE == ANY_GATEUP) Row<T, E>::load(st + (32 + m) * P + c, u);
+          const int64_t at = (c_row0 + row) * N + n;
+          if (E == 4 || n + E <= N) finish(at, std::integral_constant<int, E>{}, v, u);
+          else finish(at, std::integral_constant<int, 4>{}, v, u);  // (N is a multiple of four)
         }
       }
+      __builtin_amdgcn_s_waitcnt(0xc07f);
+      __builtin_amdgcn_wave_barrier();
+    }
   }
 }
 
