@@ -1011,6 +1011,10 @@ constexpr int W_LDS_BYTES = 8 * 64 * 136 * 2;  // 139264: the 8 epilogue regions
 // 16 experts of 1024 x 512, four each, 69 / 55, of 32 63 / 53, 300 tokens 55 / 47 and 56 / 49; a training step of 2000 of 16 226 / 212
 // (with dH narrow; gate/up and down too, 128 tiles of 250 rows, 215), of 32 230 / 217, of 60 267 / 257, 1000 of 64, six each, 249 / 235,
 // 1000 of 16 of 1984 x 1024 338 / 315; 128 tiles of 250 rows (4000 of 16) 326 / 334, 4000 of 60 394 / 418.
+// Forward products also where wide tiles are one round of workgroups and a mostly empty second one (three rounds of half the work; the
+// forward: 4000 tokens of 60 of 1280 x 640, two each, 142 / 138, 800 of 64 of 1280 x 640, six each, 119 / 117, 2500 of 16 of 1792 x
+// 1024, four each, 172 / 169; one and a half rounds, 1200 of 128 of 640 x 640, four each, 115 / 117; the input gradient so, beside the
+// weight gradients: a step of 5000 of 32 of 1024 x 704, four each, 507 / 524).
 // One dense segment: the input gradient alone (the dH of 4096 rows x 2048 columns is 16 x 8 tiles).  It runs beside other products, and
 // narrow gate/up and down tiles take CUs those would have had (one rank's share, 1000 tokens: 595 / 638).
 static bool narrow(int mode, int64_t El, int64_t n, int64_t tile_capacity) {
@@ -1018,6 +1022,7 @@ static bool narrow(int mode, int64_t El, int64_t n, int64_t tile_capacity) {
   if (El == 1) return (mode == RM_DH || mode == RM_DLIN) && tile_capacity * n * 4 <= cus * 3;
   const int64_t spare = std::max<int64_t>(tile_capacity - El - 1, 0);  // 256 rows each
   const int64_t tiles = El * std::max<int64_t>((spare + El - 1) / El, 1);
+  if ((mode == RM_GATEUP || mode == RM_DOWN) && tiles * n > cus && tiles * n * 8 <= cus * 11) return true;
   return tiles * n <= (spare * 10 > tiles * 7 ? cus * 3 / 8 : cus / 2);
 }
 
