@@ -18,7 +18,7 @@
 // the four waves hold the same tile and split each step's contraction (their shares are added through LDS in
 // wave order) and four steps are requested ahead.
 //   512 tokens of 8 fp32 experts of 256 x 512, two each, gate/up + down and the backward experts 26 + 33 us; 200 tokens of 16 of
-// 640 x 1024, two each, 51 + 83; 4096 of them, four each, 450 + 930; 1531 tokens of 16 bf16 experts of 320 x 232, 23 + 44 us.
+// 640 x 1024, two each, 51 + 83; 4096 of them, four each, 450 + 930; 1531 tokens of 16 bf16 experts of 320 x 232, 21 + 40 us.
 #include <algorithm>
 #include <type_traits>
 

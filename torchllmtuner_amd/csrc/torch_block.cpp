@@ -13,8 +13,8 @@
 // look between the stages (hooks, other dispatchers, other routers, tracing, dispatch modes); MoE.forward
 // comes here when nothing hangs on the stages.  What the single operator saves:
 //   * host time: a forward pass is one trip through the dispatcher and about ten C calls instead of four
-//     operators, a plan object and its views (83 -> 35 us at one token), a training step has one autograd
-//     node instead of three to five;
+//     operators, a plan object and its views (83 -> 28 us at one token, launches included), a training step has one
+//     autograd node instead of three to five;
 //   * launches: the router's partial logits are summed by the selection, selection and plan are one or two
 //     launches instead of four, the score gradient's pieces are summed by the selection's backward, and
 //     the additions of (T, D) tensors -- shared expert's output, the two or three input gradients -- ride
