@@ -20,9 +20,11 @@ def ops():
 
 
 # widths that end inside a narrow tile, inside a wide one and at one; 576: five narrow tiles where wide ones leave six pieces a row.
-# The last two: too many tiles for narrow ones, and row tiles that are mostly full, of which only the small products are
+# Then many experts: all products on wide tiles (with 70, gate/up on narrow ones for a second round that is mostly empty), also with rows
+# of 4 KiB; and row tiles that are mostly full, of which only the small products are narrow
 @pytest.mark.parametrize("counts,D,Fd", [((60, 0, 100, 257, 3), 448, 576), ((300, 9, 1, 17), 640, 384), ((40, 30), 2048, 448),
-                                         ((16,) * 70, 384, 448), ((250, 251, 240), 1024, 512)])
+                                         ((16,) * 70, 384, 448), ((12,) * 100, 2048, 448), ((12,) * 100, 448, 2048),
+                                         ((250, 251, 240), 1024, 512)])
 def test_products(ops, counts, D, Fd):
     print(f"narrow tiles {counts[:5]} D={D} F={Fd}", flush=True)
     g = torch.Generator().manual_seed(7)
