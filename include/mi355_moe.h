@@ -551,7 +551,7 @@ int mi355_grouped_swiglu_combine_bwd(const void* dout, const void* x, const int3
 /*
  * mi355_permute_rows_add_bwd and mi355_router_gate_add_bwd in one launch (and the sum of dw's slices), the same bits: dx =
  * dlogits . w + (the sum of drows over a token's K <= 16 slots + addend).  dw, addend, pieces may be NULL; w fp32.
- * mi355_router_gate_sum_bwd_covers: bf16 tokens, D and E multiples of 64.
+ * mi355_router_gate_sum_bwd_covers: bf16 tokens, D and E multiples of 64, or up to 32 experts and D a multiple of four.
  */
 int mi355_router_gate_sum_bwd_covers(int x_dtype, int w_dtype, int64_t D, int64_t E, int64_t K);
 int mi355_router_gate_sum_bwd(const float* dlogits, const void* x, int x_dtype, const float* w, const void* pieces,

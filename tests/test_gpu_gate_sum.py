@@ -10,7 +10,8 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
-@pytest.mark.parametrize("T,D,E,K", [(1, 128, 64, 1), (127, 192, 64, 3), (128, 384, 128, 8), (129, 448, 192, 9), (700, 1024, 256, 16)])
+@pytest.mark.parametrize("T,D,E,K", [(1, 128, 64, 1), (127, 192, 64, 3), (128, 384, 128, 8), (129, 448, 192, 9), (700, 1024, 256, 16),
+                                     (1, 64, 4, 1), (9, 260, 16, 4), (700, 448, 32, 9)])  # the last three: up to 32 experts, tiles of 8 tokens
 @pytest.mark.parametrize("extra", [(), ("addend",), ("addend", "no dw")])
 def test_gate_backward_with_the_row_sum(T, D, E, K, extra):
     from torchllmtuner_amd import _lib

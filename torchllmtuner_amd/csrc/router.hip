@@ -528,7 +528,7 @@ extern "C" int mi355_router_gate_add_bwd(const float* dlogits, const void* x, in
   }
   if (vec && T > 0 && router_few_ok(x_dtype, w_dtype, D, E) && (dx || dw)) {
     MI355_REQUIRE(dlogits && w && (x || !dw), "router_gate_bwd: null pointer");
-    return router_few_bwd(dlogits, x, x_dtype, static_cast<const float*>(w), addend, dx, static_cast<float*>(dw), workspace,
+    return router_few_bwd(dlogits, x, x_dtype, static_cast<const float*>(w), RowSum{addend}, dx, static_cast<float*>(dw), workspace,
                           T, D, E, s);
   }
   if (dx && T > 0) {
@@ -560,7 +560,10 @@ extern "C" int mi355_router_gate_add_bwd(const float* dlogits, const void* x, in
 }
 
 extern "C" int mi355_router_gate_sum_bwd_covers(int x_dtype, int w_dtype, int64_t D, int64_t E, int64_t K) {
-  return E >= 1 && K >= 1 && K <= 16 && router_x3_ok(x_dtype, w_dtype, D, E) ? 1 : 0;
+  return E >= 1 && K >= 1 && K <= 16 && x_dtype == MI355_BF16 &&
+                 (router_x3_ok(x_dtype, w_dtype, D, E) || router_few_ok(x_dtype, w_dtype, D, E))
+             ? 1
+             : 0;
 }
 
 extern "C" int mi355_router_gate_sum_bwd(const float* dlogits, const void* x, int x_dtype, const float* w, const void* pieces,
@@ -575,6 +578,8 @@ extern "C" int mi355_router_gate_sum_bwd(const float* dlogits, const void* x, in
                     aligned16({dlogits, x, w, pieces, drows, addend, dx, dw, workspace}),
                 "router_gate_sum_bwd: null or misaligned pointer");
   const RowSum sum{addend, drows, row_of_slot, K, row_capacity};
+  if (router_few_ok(x_dtype, MI355_F32, D, E))
+    return router_few_bwd(dlogits, x, x_dtype, w, sum, dx, dw, workspace, T, D, E, as_stream(stream));
   return router_x3_bwd(dlogits, x, w, pieces, sum, dx, dw, workspace, T, D, E, as_stream(stream));
 }
 

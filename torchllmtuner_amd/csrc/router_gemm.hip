@@ -574,17 +574,17 @@ __device__ __forceinline__ void gate_dx_part(const float* __restrict__ dlogits, 
   }
 }
 
-template <typename TX>
+constexpr int kRowsTok = 8;  // tokens of a dx part with the rows in front
+
+template <typename TX, bool ROWS>
 __global__ __launch_bounds__(256) void gate_bwd_few_kernel(GateDw dw, const float* __restrict__ dlogits,
                                                            const float* __restrict__ w, GateDx<TX> g, TX* __restrict__ dx,
                                                            int T, int D, int E, int dw_parts) {
   __shared__ __attribute__((aligned(16))) float lds[kGateDwLds];
   const int block = blockIdx.x;
   if (block < dw_parts) gate_dw_part<TX>(dw, block, lds);
-  else gate_dx_part<TX, false, S_TOK / 4>(dlogits, w, g, dx, T, D, E, block - dw_parts, lds);
+  else gate_dx_part<TX, ROWS, (ROWS ? kRowsTok : S_TOK) / 4>(dlogits, w, g, dx, T, D, E, block - dw_parts, lds);
 }
-
-constexpr int kRowsTok = 8;  // tokens of a dx part with the rows in front
 
 // dx with the sum over the token's rows, and beside it the sum of dW's slices, in their order: the two ends of a backward
 // whose dW parts ran in an earlier launch.
@@ -658,18 +658,24 @@ bool router_few_ok(int x_dtype, int w_dtype, int64_t D, int64_t E) {
 }
 int64_t router_few_bwd_workspace(int64_t T, int64_t D, int64_t E) { return gate_dw_splits(T, D, E) * E * D * 4; }
 
-int router_few_bwd(const float* dlogits, const void* x, int x_dtype, const float* w, const void* addend, void* dx, float* dw,
+int router_few_bwd(const float* dlogits, const void* x, int x_dtype, const float* w, const RowSum& sum, void* dx, float* dw,
                    void* workspace, int64_t T, int64_t D, int64_t E, hipStream_t s) {
   const int splits = gate_dw_splits(T, D, E);
   const GateDw job = gate_dw_job(dlogits, x, splits > 1 ? static_cast<float*>(workspace) : dw, T, D, E);
   const int64_t dw_parts = dw ? gate_dw_parts(job) : 0;
-  const int64_t blocks = dw_parts + (dx ? (T + S_TOK - 1) / S_TOK * ((D + S_COLS - 1) / S_COLS) : 0);
+  const int tok = sum.rows ? kRowsTok : S_TOK;
+  const int64_t blocks = dw_parts + (dx ? (T + tok - 1) / tok * ((D + S_COLS - 1) / S_COLS) : 0);
   MI355_REQUIRE(blocks < (1ll << 31), "router_gate_bwd: too many tokens");
   auto launch = [&](auto* xp) {
     using TX = std::remove_const_t<std::remove_pointer_t<decltype(xp)>>;
-    hipLaunchKernelGGL(gate_bwd_few_kernel<TX>, dim3((unsigned)blocks), dim3(256), 0, s, job, dlogits, w,
-                       GateDx<TX>{static_cast<const TX*>(addend), nullptr, nullptr, 0, 0}, static_cast<TX*>(dx), (int)T, (int)D,
-                       (int)E, (int)dw_parts);
+    const GateDx<TX> g{static_cast<const TX*>(sum.addend), static_cast<const TX*>(sum.rows), sum.row_of_slot, (int)sum.K,
+                       (int)sum.row_capacity};
+    auto run = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, s, job, dlogits, w, g, static_cast<TX*>(dx), (int)T, (int)D,
+                         (int)E, (int)dw_parts);
+    };
+    if constexpr (sizeof(TX) == 2) run(sum.rows ? gate_bwd_few_kernel<TX, true> : gate_bwd_few_kernel<TX, false>);
+    else run(gate_bwd_few_kernel<TX, false>);  // (fp32 tokens: the experts' launches take the parts along)
   };
   if (x_dtype == MI355_BF16) launch(static_cast<const uint16_t*>(x));
   else launch(static_cast<const float*>(x));

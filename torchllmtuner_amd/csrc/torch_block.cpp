@@ -412,8 +412,10 @@ Grads block_backward(const Block& b, const Tensor& kept, const Tensor& dout_, co
   const bool joined = b.gather && mi355_router_gate_rows_bwd_covers(b.dt, b.gate_dt, b.D, b.E);
   // ... or, behind the matrix-core kernels, both gradients and the row sum together, where they are short: beside the experts'
   // weight gradients, whose workgroups keep to their tiles and their CUs, a long launch holds back whichever of those its own CUs
-  // were due to (router_gemm.hip has both sides)
-  const bool summed = b.folded && need.x && b.T * b.D <= kShortRowSum && mi355_router_gate_sum_bwd_covers(b.dt, b.gate_dt, b.D, b.E, c.K);
+  // were due to (router_gemm.hip has both sides).  Up to 32 experts that is where nothing runs beside (a step, us, apart / together: 1000
+  // tokens of 16, 32 experts of 1024 x 512, four each, 159 / 154, 178 / 170; 2500 of 32 of 1536 x 768, four each, 438 / 447).
+  const bool short_sum = b.E > 32 ? b.T * b.D <= kShortRowSum : short_backward(b.El, b.D, b.F, b.R);
+  const bool summed = b.folded && need.x && short_sum && mi355_router_gate_sum_bwd_covers(b.dt, b.gate_dt, b.D, b.E, c.K);
   const bool joined_dw = joined && need.gate_w && (need.x || need.experts);
   const int64_t gate_bytes = need.x || need.gate_w ? mi355_router_gate_bwd_workspace_bytes(b.T, b.D, b.E) : 0;
   void *s_dgate = nullptr, *s_dup = nullptr, *dx_shared = nullptr, *dx_routed = nullptr, *dgate = nullptr, *dup = nullptr,
