@@ -48,9 +48,10 @@ __device__ __forceinline__ void load16_masked(const uint16_t* p, int k, int k_en
     v[j] = k + 8 * j < k_end ? *reinterpret_cast<const u32x4*>(p + k + 8 * j) : u32x4{0, 0, 0, 0};
 }
 
-// One slice of the contraction, by the 64 R_WAVES lanes of a workgroup (ends behind a barrier).  Lanes below 256: the sum of
-// token lane & 31 and the experts q * 8 + (lane >> 5) * 4 + 0..3 of the tile, q their wave.
-template <typename TX>
+// One slice of the contraction, by the 64 R_WAVES lanes of a workgroup (ends behind a barrier).  Lanes below 8 BN: the sum of
+// token lane & 31 and the experts q * 8 + (lane >> 5) * 4 + 0..3 of the tile, q their wave.  BN below 32: the tile's first BN experts
+// alone, the same sums in the same order (an element of the matrix instruction's result depends on its own row and column).
+template <typename TX, int BN = R_BN>
 __device__ __forceinline__ f32x4 gate_rows_tile(const TX* __restrict__ x, const float* __restrict__ w, int T, int D, int E,
                                                 int t0, int n0, int split, int k_per_wave, float (&red)[R_WAVES][4][64][4] /* wave, q, lane, i */) {
   constexpr bool BF = sizeof(TX) == 2;
@@ -63,14 +64,15 @@ __device__ __forceinline__ f32x4 gate_rows_tile(const TX* __restrict__ x, const 
   f32x16 acc;
 #pragma unroll
   for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
-  constexpr int B = 4;  // steps requested together: 128 of the contraction, 24 KiB (bf16 x) per wave
+  const int w_end = (lane & 31) < BN ? k1 : 0;  // (what the other lanes hold is not read)
+  constexpr int B = 4;  // steps requested together: 128 of the contraction, 24 KiB (bf16 x, 32 experts) per wave
   for (int kb = k0; kb < k1; kb += B * R_STEP) {
     f32x4 wv[B][4];
     std::conditional_t<BF, u32x4[B][2], f32x4[B][4]> xv;
 #pragma unroll
     for (int b = 0; b < B; ++b) {
       const int k = kb + b * R_STEP + 16 * half;
-      load16_masked(wp, k, k1, wv[b]);
+      load16_masked(wp, k, w_end, wv[b]);
       load16_masked(xp, k, k1, xv[b]);
     }
 #pragma unroll
@@ -96,12 +98,12 @@ __device__ __forceinline__ f32x4 gate_rows_tile(const TX* __restrict__ x, const 
     }
   }
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
+  for (int q = 0; q < BN / 8; ++q) {
     const f32x4 v = {acc[q * 4], acc[q * 4 + 1], acc[q * 4 + 2], acc[q * 4 + 3]};
     *reinterpret_cast<f32x4*>(red[wave][q][lane]) = v;
   }
   __syncthreads();
-  const int q = (tid >> 6) & 3;
+  const int q = (tid >> 6) & (BN / 8 - 1);
   f32x4 v = *reinterpret_cast<const f32x4*>(red[0][q][lane]);
 #pragma unroll
   for (int i = 1; i < R_WAVES; ++i) v += *reinterpret_cast<const f32x4*>(red[i][q][lane]);

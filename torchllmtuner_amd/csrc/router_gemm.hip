@@ -47,7 +47,7 @@ __global__ __launch_bounds__(256) void split_kernel(const float* __restrict__ w,
 
 // ---- logits(T,E) = x(T,D) . W(E,D)^T + bias, few tokens or any widths --------------------
 // Bound by latency: at one token the product is one read of W (1 MB at 128 x 2048), which wants to
-// be in flight all at once and in as few launches as possible.  A workgroup takes 32 tokens x 32
+// be in flight all at once and in as few launches as possible.  A workgroup takes 32 tokens x up to 32
 // experts and a slice of the contraction; its eight waves split that slice, and every wave reads
 // its operands straight into MFMA fragments (no LDS, no barrier in the loop; a weight is used by
 // one wave of one workgroup per 32 tokens), the fp32 weights becoming their three bf16 pieces in
@@ -58,7 +58,7 @@ __global__ __launch_bounds__(256) void split_kernel(const float* __restrict__ w,
 // weight-splitting launch: 1 token of 2048 x 128 experts 34 -> 8 us, 1000 tokens 43 -> 12 us, 128
 // tokens of 7168 x 256 experts 131 -> 12 us (profiled inside the block, the weights from memory).  From 1024 tokens on, with widths on its grid, the
 // 128-token kernel below reads the weights four times less often and is the faster one.
-template <typename TX>
+template <typename TX, int BN>
 __global__ __launch_bounds__(64 * R_WAVES) void gate_rows_kernel(const TX* __restrict__ x,
                                                                  const float* __restrict__ w,
                                                                  const float* __restrict__ bias,
@@ -66,9 +66,9 @@ __global__ __launch_bounds__(64 * R_WAVES) void gate_rows_kernel(const TX* __res
                                                                  int k_per_wave) {
   __shared__ __attribute__((aligned(16))) float red[R_WAVES][4][64][4];
   const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, q = tid >> 6;
-  const int t0 = blockIdx.x * R_BM, n0 = blockIdx.y * R_BN;
-  f32x4 v = gate_rows_tile<TX>(x, w, T, D, E, t0, n0, blockIdx.z, k_per_wave, red);
-  if (tid >= 256) return;
+  const int t0 = blockIdx.x * R_BM, n0 = blockIdx.y * BN;
+  f32x4 v = gate_rows_tile<TX, BN>(x, w, T, D, E, t0, n0, blockIdx.z, k_per_wave, red);
+  if (tid >= 8 * BN) return;
   const int t = t0 + (lane & 31), n = n0 + q * 8 + half * 4;
   if (t >= T || n >= E) return;
   float* dst = out + (static_cast<int64_t>(blockIdx.z) * T + t) * E + n;
@@ -88,15 +88,22 @@ __global__ __launch_bounds__(64 * R_WAVES) void gate_rows_kernel(const TX* __res
 
 // Splits of the contraction over workgroups: about 128 of it per wave (one batch of requests)
 // while that leaves the launch below four workgroups a CU; each split costs its consumer one
-// more read of the (T, E) partial sums.  Where a contraction is split anyway and there is a CU for each part, half of that per
-// wave: block forward of 128 experts of 2048 x 768, us, 128 / 64 / 32 per wave: one token 28.7 / 27.1 / 27.2, 33 tokens 210 / 207 / 206,
-// 200 244 / 241 / 240, 1000 (256 parts at 128) 273 / 274 / 277; one rank's share of 256 of 7168 x 2048 the same throughout.
+// more read of the (T, E) partial sums.  The number decides the order in which a logit is summed, and so which of two experts whose logits
+// are equal to the last bits a token takes: it is not a setting to be moved with the number of tokens.
 int rows_splits(int64_t T, int64_t D, int64_t E) {
   const int64_t tiles = ((T + R_BM - 1) / R_BM) * ((E + R_BN - 1) / R_BN);
-  auto parts = [&](int64_t per_wave) { return (D + per_wave * R_WAVES - 1) / (per_wave * R_WAVES); };
-  int64_t want = parts(128);
-  if (want > 1) want = std::max(want, std::min(parts(64), 256 / tiles));
+  const int64_t want = (D + 128 * R_WAVES - 1) / (128 * R_WAVES);
   return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>({want, 8, 1024 / tiles})));
+}
+
+// Experts a workgroup takes: as few of 32, 16 and 8 as leave it a CU of its own.  Fewer of them are less for a wave to wait for, at
+// the same sums.  Block forward of 128 experts of 2048 x 768, eight a token, us, 32 / 16 / 8: one token (8 workgroups of 32) 28.5 / 27.2 /
+// 26.5, four 67.6 / 66.2 / 65.4, 33 tokens (16) 210.0 / 207.6 / 206.8, 200 (56) 243.9 / 242.0 / 241.3, 500 (128) 255.9 / 254.0 / 258.1, 1000
+// (256) 271.8 / 275.7 / 283.7; 300 of 64 of 1536 x 640, four each (40), 117.2 / 115.5 / 114.5; 128 of one rank's share of 256 of
+// 7168 x 2048 (224) 454 / 458 / 465.
+int rows_experts(int64_t t_tiles, int64_t E, int splits) {
+  const int64_t parts = t_tiles * ((E + R_BN - 1) / R_BN) * splits;
+  return parts <= 64 ? 8 : parts <= 128 ? 16 : R_BN;
 }
 
 // The same product for many tokens: 128 tokens x 128 experts per workgroup, 8 waves as 2 x 4
@@ -746,13 +753,22 @@ int router_fwd_partial(const void* x, int x_dtype, const float* w, const float* 
     return check_launch("router_gate_fwd");
   }
   const int k_per_wave = gate_rows_k(D, splits);
-  const dim3 grid((unsigned)((T + R_BM - 1) / R_BM), (unsigned)((E + R_BN - 1) / R_BN), (unsigned)splits);
-  if (x_dtype == MI355_BF16)
-    hipLaunchKernelGGL(gate_rows_kernel<uint16_t>, grid, dim3(64 * R_WAVES), 0, s, static_cast<const uint16_t*>(x), w,
-                       in_kernel_bias, partial, (int)T, (int)D, (int)E, k_per_wave);
-  else
-    hipLaunchKernelGGL(gate_rows_kernel<float>, grid, dim3(64 * R_WAVES), 0, s, static_cast<const float*>(x), w,
-                       in_kernel_bias, partial, (int)T, (int)D, (int)E, k_per_wave);
+  const int64_t t_tiles = (T + R_BM - 1) / R_BM;
+  auto launch = [&](auto* xp, auto bn) {
+    constexpr int BN = decltype(bn)::value;
+    using TX = std::remove_const_t<std::remove_pointer_t<decltype(xp)>>;
+    const dim3 grid((unsigned)t_tiles, (unsigned)((E + BN - 1) / BN), (unsigned)splits);
+    hipLaunchKernelGGL((gate_rows_kernel<TX, BN>), grid, dim3(64 * R_WAVES), 0, s, xp, w, in_kernel_bias, partial, (int)T, (int)D,
+                       (int)E, k_per_wave);
+  };
+  auto choose = [&](auto* xp) {
+    const int bn = rows_experts(t_tiles, E, splits);
+    if (bn == 8) launch(xp, std::integral_constant<int, 8>{});
+    else if (bn == 16) launch(xp, std::integral_constant<int, 16>{});
+    else launch(xp, std::integral_constant<int, 32>{});
+  };
+  if (x_dtype == MI355_BF16) choose(static_cast<const uint16_t*>(x));
+  else choose(static_cast<const float*>(x));
   return check_launch("router_gate_fwd");
 }
 
