@@ -82,3 +82,46 @@ def test_infinities_overflow_and_nan(ops):
     cols = torch.tensor([c for c in range(580) if c not in (8, 9)], device=DEV)
     # rows that share a tile with one of the three are formed in the other way: the same up to rounding
     assert rel_l2(gate[same][:, cols], clean[same][:, cols]) < 2 * 772 ** 0.5 * 2.0 ** -24
+
+
+def reference(x, dy, w1, w3, w2, gate, up, h, rows):
+    """fp64 products of what each launch is given; what it rounds in between (dgate, dup) is not."""
+    x, dy, w1, w3, w2, gate, up, h = (t.double() for t in (x, dy, w1, w3, w2, gate, up, h))
+    sig = torch.sigmoid(gate)
+    dh = per_expert(rows, lambda e, r: dy[r] @ w2[e], h)
+    dg, du = dh * up * (sig * (1 + gate * (1 - sig))), dh * (gate * sig)
+    dw = lambda a, b: torch.stack([a[r].T @ b[r] for r in rows])
+    return dict(gate=per_expert(rows, lambda e, r: x[r] @ w1[e].T, gate), up=per_expert(rows, lambda e, r: x[r] @ w3[e].T, up),
+                y=per_expert(rows, lambda e, r: h[r] @ w2[e].T, x), dx=per_expert(rows, lambda e, r: dg[r] @ w1[e] + du[r] @ w3[e], x),
+                dw1=dw(dg, x), dw3=dw(du, x), dw2=dw(dy, h))
+
+
+# 64-row and 128-row tiles
+@pytest.mark.parametrize("counts,D,Fd", [((520, 1000, 65), 772, 580), ((3100, 2900, 3001), 900, 908)])
+def test_values_whose_pieces_end_below_bf16(ops, counts, D, Fd):
+    """From 2^-110 down to fp32's own end a third piece would lose bits; rows and experts of such values are as exact as others."""
+    print(f"fp32 pieces, small values {counts}", flush=True)
+    plan, x, dy, w1, w3, w2, rows = problem(ops, counts, D, Fd)
+    small = 2.0 ** -118
+    x[3] *= small        # gate, up
+    x[600] *= 2.0 ** -58  # h is about 2^-118: down
+    dy[700] *= small     # dh, then the input gradient
+    dy[rows[2]] *= small  # the weight gradients of an expert
+    y, gate, up, h = ops.grouped_swiglu_fwd(x, w1, w3, w2, plan)
+    dx, dw1, dw3, dw2 = ops.grouped_swiglu_bwd(dy, x, w1, w3, w2, gate, up, h, plan)
+    want = reference(x, dy, w1, w3, w2, gate, up, h, rows)
+
+    def bound(n):  # as above
+        return n ** 0.5 * 2.0 ** -24
+
+    def err(got, ref):  # scaled: the norms of such values are below what rel_l2 divides by
+        return rel_l2(got.double() / small, ref / small)
+
+    assert err(gate[3], want["gate"][3]) < bound(D) and err(up[3], want["up"][3]) < bound(D)
+    assert 0 < float(h[600].abs().max()) < 2.0 ** -110
+    assert err(y[600], want["y"][600]) < bound(Fd)
+    few = torch.cat([torch.tensor([700], device=DEV), rows[2]])
+    assert err(dx[few], want["dx"][few]) < bound(D) + bound(2 * Fd)
+    assert err(dw2[2], want["dw2"][2]) < bound(max(counts))
+    for got, name in ((dw1, "dw1"), (dw3, "dw3")):
+        assert err(got[2], want[name][2]) < bound(D) + bound(max(counts))
