@@ -125,3 +125,86 @@ def test_values_whose_pieces_end_below_bf16(ops, counts, D, Fd):
     assert err(dw2[2], want["dw2"][2]) < bound(max(counts))
     for got, name in ((dw1, "dw1"), (dw3, "dw3")):
         assert err(got[2], want[name][2]) < bound(D) + bound(max(counts))
+
+
+def test_products_that_only_their_first_pieces_overflow(ops):
+    """(2 - 2^-13) 2^63 rounds up to 2^64 in bf16, and the square of that is no fp32 value, while its own is."""
+    plan, x, _, w1, w3, w2, _ = problem(ops, (520, 1000, 65), 772, 580)
+    big = (2 - 2.0 ** -13) * 2.0 ** 63
+    x[10] = 0
+    x[10, 5] = w1[0, 7, 5] = big
+    gate = ops.grouped_swiglu_fwd(x, w1, w3, w2, plan)[1]
+    assert gate[10, 7].item() == pytest.approx(big * big, rel=1e-6) and gate[10].isfinite().all()
+
+
+def same(a, b):
+    return bool(((a == b) | (a.isnan() & b.isnan())).all())
+
+
+def alike(got, ref, tol):
+    """Infinities of one sign and NaN in the same places, the rest within tol."""
+    ref = ref.to(got.device)
+    assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got.isinf(), ref.isinf())
+    assert torch.equal(got[got.isinf()] > 0, ref[ref.isinf()] > 0)
+    finite = ref.isfinite()
+    assert rel_l2(got[finite], ref[finite]) < tol
+
+
+# 64-row tiles throughout, 128-row ones throughout (the weight gradients' too)
+@pytest.mark.parametrize("T,D,Fd,E", [(900, 772, 580, 3), (4500, 900, 908, 3)])
+def test_not_finite_and_small_values_in_every_product_copied_and_read_in_place(ops, T, D, Fd, E):
+    from torchllmtuner_amd import _lib
+
+    print(f"fp32 pieces, not finite T={T}", flush=True)
+    lib, g = _lib.load(), torch.Generator().manual_seed(T)
+    ids = torch.stack([torch.randperm(E, generator=g)[:2] for _ in range(T)])
+    plan = ops.permute_plan(ids.to(DEV), E)
+    x, dout = (torch.randn(T, D, generator=g).to(DEV) for _ in "xd")
+    w1, w3, w2 = ((torch.randn(*s, generator=g) * 0.03).to(DEV) for s in ((E, Fd, D), (E, Fd, D), (E, D, Fd)))
+    weights = torch.rand(T, 2, generator=g).to(DEV)
+    x[3, 700], x[200, 1], x[201] = float("inf"), float("nan"), x[201] * 2.0 ** -118
+    dout[5, 71], dout[320, 8], dout[321] = float("-inf"), float("nan"), dout[321] * 2.0 ** -118
+    tok, R = plan.token_of_row.long(), plan.row_capacity
+    scale = ops.combine_row_scale(weights, plan)
+    rows_x, dy = x[tok], dout[tok] * scale[:, None]
+    rows = [r for r in torch.arange(R, device=DEV).split(plan.seg_counts.tolist())]
+    copied = ops.grouped_swiglu_fwd(rows_x, w1, w3, w2, plan)
+    y, gate, up, h = copied
+    p = lambda t: t.data_ptr()
+    stream = torch.cuda.current_stream().cuda_stream
+    plan_args = [p(t) for t in plan.segments()] + [plan.tile_capacity]
+    assert lib.mi355_grouped_gather_covers(0, D, Fd, R, T) == 1
+    gathered = [torch.empty_like(t) for t in copied]
+    rc = lib.mi355_grouped_gather_fwd(p(x), p(plan.token_of_row), T, p(w1), p(w3), p(w2), 0, *plan_args, p(gathered[1]),
+                                      p(gathered[2]), p(gathered[3]), p(gathered[0]), E, D, Fd, R, stream)
+    assert rc == 0
+    for name, a, b in zip(("y", "gate", "up", "h"), gathered, copied):
+        assert same(a, b), name
+    want = reference(rows_x, dy, w1, w3, w2, gate, up, h, rows)
+
+    def bound(n):
+        return n ** 0.5 * 2.0 ** -24
+
+    alike(gate, want["gate"], bound(D))
+    alike(up, want["up"], bound(D))
+    alike(y, want["y"], bound(Fd))
+    # backward on a clean forward (every gradient of an expert with a NaN activation would be NaN), then on this one
+    for fx, clean in ((torch.where(x.isfinite(), x, 1.0), True), (x, False)):
+        rows_f = fx[tok]
+        _, gate, up, h = ops.grouped_swiglu_fwd(rows_f, w1, w3, w2, plan)
+        grads = ops.grouped_swiglu_bwd(dy, rows_f, w1, w3, w2, gate, up, h, plan)
+        dgate, dup = torch.empty_like(gate), torch.empty_like(gate)
+        got = [torch.empty_like(t) for t in grads]
+        rc = lib.mi355_grouped_gather_bwd(p(dout), p(fx), p(plan.token_of_row), T, p(scale), p(w1), p(w3), p(w2), p(gate), p(up),
+                                          p(h), 0, *plan_args, p(dgate), p(dup), *(p(t) for t in got), None, None, 0, E, D,
+                                          Fd, R, stream)
+        assert rc == 0
+        for name, a, b in zip(("dx", "dw1", "dw3", "dw2"), got, grads):
+            assert same(a, b), name
+        if not clean:
+            continue
+        want = reference(rows_f, dy, w1, w3, w2, gate, up, h, rows)
+        alike(grads[0], want["dx"], bound(D) + bound(2 * Fd))
+        alike(grads[3], want["dw2"], bound(max(len(r) for r in rows)))
+        for i, name in ((1, "dw1"), (2, "dw3")):
+            alike(grads[i], want[name], bound(D) + bound(max(len(r) for r in rows)))

@@ -177,9 +177,9 @@ __device__ __forceinline__ f32x4 any_frag(const float* tile, int row, int kk, in
 // us, fp32 products / pieces: 4096 tokens of 16 x 640 x 1020 (four each) 2009 / 1573, 4096 of 4 (two each) 1033 / 845, 1000 of 16 x
 // 512 x 800 (three each) 353 / 262, 1500 of 8 x 320 x 400 (three each) 196 / 169.  Two, three and four steps requested ahead: large
 // products 3-9 % slower, small ones the same.
-//   Three pieces hold what fp32 does from 2^-110 on (bf16 ends at 2^-133); a value that is not finite, or rounds to infinity, has NaN
-// for its second piece.  A tile one of whose operands' values has lost bits, or with a NaN, is formed again by fp32 products, which
-// say what it is.  Looking costs 0.7-1.5 % of
+//   Three pieces hold what fp32 does from 2^-110 on (bf16 ends at 2^-133) and as long as the first of them and their products stay
+// finite: a value that is not finite, or rounds to infinity, has NaN for its second piece.  A tile one of whose operands' values has lost bits,
+// or with a result that is not finite, is formed again by fp32 products, which say what it is.  Looking costs 0.7-1.5 % of
 // those steps (us, without / with: 1550 / 1561, 870 / 879, 261 / 265, 173 / 175; by comparing every value with 2^-110 8 %).
 template <bool KS, int ROWS>
 struct Pieces {
@@ -520,7 +520,13 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
 #pragma unroll
       for (int j = 0; j < NJ; ++j)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) again |= acc[i][j][v] != acc[i][j][v];
+        for (int q = 0; q < 4; ++q) {
+          const int n = n0 + bcol(j) - (MODE == ANY_GATEUP && j >= NJ / 2 ? TN / 2 : 0) + q * 8 + 4 * (lane >> 5);
+          bool finite = true;
+#pragma unroll
+          for (int v = 0; v < 4; ++v) finite &= fabsf(acc[i][j][q * 4 + v]) < INFINITY;
+          again |= !finite && wm + i * 32 + (lane & 31) < m_valid && n < N;
+        }
     if (__syncthreads_or(again)) {
 #pragma unroll
       for (int i = 0; i < MI; ++i)
