@@ -174,8 +174,8 @@ __device__ __forceinline__ f32x4 any_frag(const float* tile, int row, int kk, in
 // gave (2409 tokens of 8 x 360 x 648: dx 8.2e-7 -> 2.7e-7, dw2 6.7e-7 -> 2.3e-7; added to the sum one by one, 4-10 % faster, 0.8-1.4).
 //   Split where it is parked, once a workgroup, not where each of the waves reads it (5.5 vector instructions an element); one
 // stage, so that LDS (61 KB on 128-row tiles) holds two workgroups a CU and one splits while the other multiplies.  A training step,
-// us, fp32 products / pieces: 4096 tokens of 16 x 640 x 1020 (four each) 2009 / 1573, 4096 of 4 (two each) 1033 / 845, 1000 of 16 x
-// 512 x 800 (three each) 353 / 262, 1500 of 8 x 320 x 400 (three each) 196 / 169.  Two, three and four steps requested ahead: large
+// us, fp32 products / pieces on the same tiles: 4096 tokens of 16 x 640 x 1020 (four each) 2012 / 1538, 4096 of 4 (two each) 1053 / 864, 1000
+// of 16 x 512 x 800 (three each) 322 / 262, 1500 of 8 x 320 x 400 (three each) 198 / 172.  Two, three and four steps requested ahead: large
 // products 3-9 % slower, small ones the same.
 //   Three pieces hold what fp32 does from 2^-110 on (bf16 ends at 2^-133) and as long as the first of them and their products stay
 // finite: a value that is not finite, or rounds to infinity, has NaN for its second piece.  A tile one of whose operands' values has lost bits,
@@ -767,6 +767,9 @@ int launch_any(const AnyArgs& p, int dtype, int64_t blocks, hipStream_t s, const
 //     512 x 512) 40 / 49 against 34 / 45, 250 (750, 256 x 300) 30 / 42 against 37 / 46, 312 (250, 256 x 512) 34 / 48 against 35 / 47;
 //   16 experts of 640 x 1024: 25 rows each 73 / 124 against 50 / 84, 50 rows 75 / 128 against 67 / 118, 75 rows 77 / 138 against
 //     81 / 138, 250 rows 145 / 279 against 189 / 338.
+// The lines for pieces (64 rows per expert; the weight gradients' 160 and 448 tiles and 400 rows, below) against those fp32 products had
+// (160; 256 and 512 tiles, no rows), a training step, us, theirs / these: 200 tokens of 16 x 640 x 1020, two each, 185 / 162, 400, four each, 310 / 282,
+// 600 of 16 x 512 x 800, four each, 283 / 243, 1000 of 8 x 640 x 640, two each, 229 / 205; from 2000 tokens of 16 x 640 x 1020 on the same.
 // bf16 steps are shorter and gain nothing (14 / 17 against 14 / 18, slower with more tiles).
 int row_tile(const AnyArgs& p, int dtype, int64_t El, int64_t cols, int bf16_large) {
   auto tiles = [&](int64_t t) { return (p.rows / t + std::min(El, p.rows)) * ((cols + t - 1) / t); };

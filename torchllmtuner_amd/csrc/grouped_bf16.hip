@@ -1015,6 +1015,10 @@ constexpr int W_LDS_BYTES = 8 * 64 * 136 * 2;  // 139264: the 8 epilogue regions
 // forward: 4000 tokens of 60 of 1280 x 640, two each, 142 / 138, 800 of 64 of 1280 x 640, six each, 119 / 117, 2500 of 16 of 1792 x
 // 1024, four each, 172 / 169; one and a half rounds, 1200 of 128 of 640 x 640, four each, 115 / 117; the input gradient so, beside the
 // weight gradients: a step of 5000 of 32 of 1024 x 704, four each, 507 / 524).
+// Alone, 1500 products of 4 to 128 experts of 512-2048 x 448-1024, 20-500 rows each, time on narrow tiles / on wide ones: partly full, up to half the CUs
+// 0.66-0.82 (328 of 328 faster), above that up to one round 1.01-1.34 but for 20 whose width a wide tile overhangs by half; mostly full, up to
+// three eighths 0.63-1.21 (149 of 154 faster), from there to half 0.65-1.24 (46 of 88); forward, one to one and three eighths rounds 0.69-0.99 (42
+// of 42) and, mostly full, 0.66-1.15 (21 of 30), up to one and a half 0.87-1.16 (72 of 93).
 // One dense segment: the input gradient alone (the dH of 4096 rows x 2048 columns is 16 x 8 tiles).  It runs beside other products, and
 // narrow gate/up and down tiles take CUs those would have had (one rank's share, 1000 tokens: 595 / 638).
 static bool narrow(int mode, int64_t El, int64_t n, int64_t tile_capacity) {
@@ -1074,7 +1078,8 @@ static bool few_rows(int64_t El, int64_t R, int64_t D, int64_t F) {
 // tile, so that the product is a read of the weights.  Block forward, 128 experts of 2048 x 768, eight a token, us, as ever / turned:
 // 150 tokens 278 / 243, 300 269 / 248, 600 303 / 263, 1000 279-306 / 271, 2000 340 / 313, 3000 (187 rows) 378 / 365, 4000 (250) 474 / 476,
 // 8192 766 / 779; 64 experts of 2048 x 2048, 700 tokens of six 355 / 329, 4096 x 1024 366 / 336; rows of 1024, 1536 and 7168 elements
-// the same within 1 %.
+// the same within 1 %.  The fp32 sums are the same products in another order, so a bf16 result may round the other way: across 200 rows
+// an expert (and 8, grouped_few.hip) a token's bits depend on how many come with it (1000 tokens of that block: 3e-4 of the output, at most a bf16 step).
 static bool turned(int64_t El, int64_t R, int64_t K) { return El > 1 && R <= 200 * El && K * 2 % 4096 == 0; }
 
 int bf16_grouped_fwd(const void* rows, const int32_t* token_of_row, int64_t num_tokens, const void* w1,
