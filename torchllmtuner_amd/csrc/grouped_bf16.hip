@@ -10,36 +10,42 @@
 // Shape of the kernels.  256x256 output tiles for the row-tiled products and the weight
 // gradients alike, eight waves per workgroup as 4 (rows) x 2 (columns), two per SIMD, each
 // wave a 64x128 accumulator tile; one workgroup per CU, two 64 KiB LDS stages of operand
-// tiles (overlaid by the eight 17 KiB epilogue regions).  Row tiles come from the
-// permutation plan's tile list (up to 256 rows of one expert each).
+// tiles.  Row tiles come from the permutation plan's tile list (up to 256 rows of one expert each).
 //
-// What bounds them, measured on MI355X.  With operands of random bits the card's power
-// management holds the core clock near 1.5-1.9 GHz (2.4 GHz with constant operands): a
-// register-resident MFMA loop sustains 1.45-1.95 PFLOP/s instead of the 2.5 PFLOP/s of the
-// data sheet, the same loop fed from LDS and staging its operands from L2 about 1.0-1.1.
-// The K loops here run at that rate; operand traffic is not the limit (L2 delivers
-// 50 B/clk/CU to a tile-shaped read pattern, HBM 10 B/clk/CU, and making every operand
-// cache-resident changes nothing).  What is left is everything around the K loop, hence:
+// K loop of the row-tiled products.  Operands go from memory straight into LDS (1 KiB a wave and instruction,
+// the swizzle applied to the address each lane asks for), so no register holds them on the way: 64
+// of a wave's 256 registers hold two sets of fragments instead, and the next quarter's fragments are
+// read under this quarter's MFMAs.  A K step of 64 is four quarters of 16 MFMAs and two barriers: behind the first, where the rows and half of the
+// weights have been read, their part of the stage is requested for the K step after the next; behind the second, the other half.  Every request has
+// one and a half K steps to arrive.  Requests and reads go out between the 16-row blocks of MFMAs: in bursts
+// behind the barriers they cost 7 % (all eight waves issue them at once while the matrix cores run dry).  The requests
+// run on into the next tile, whose first two K steps land while this one's results are written through 4 KiB a wave of LDS of their own.
+// A tile's 16-row blocks are dealt to the wave rows in turn and the loop exists for 0 to 4 blocks a wave, so
+// that a tile that is not full costs what its rows cost and no branch stands between MFMAs (a branch per block: 3-5 % of a full tile).
+//
+// What that measured, us, operands parked in LDS through registers / straight into LDS: 128 experts of 2048 x 768, 8192 tokens of eight each: gate/up
+// 487 / 433, down 250 / 226, dH 309 / 289, dRows 443 / 392; one dense segment of 4096 rows of 7168 x 2048 198 / 172, 109 / 98, 130 / 107, 209 / 185 (gate
+// and up not kept: 1.38 PFLOP/s), 300 rows of it 129 / 90, 41 / 31, 92 / 64, 80 / 60; 32 experts of 7168 x 2048, 128 rows each 385 / 366,
+// 217 / 204, 203 / 195, 399 / 387 (there the weights' way from memory counts), nine rows each 317 / 314, 169 / 168, 164 / 159, 317 / 334: the one
+// that lost, a read of the weights at 5.6 TB/s.  The same bits.
+//
+// What is left.  With operands of random bits the card's power management holds the core clock near 1.5-1.9 GHz
+// (a register-resident MFMA loop sustains 1.45-2.2 PFLOP/s by operand values instead of the 2.5 of the data sheet); with constant operands the same
+// launches take 10-20 % less.  Without requests the loop takes 20-35 % less, without barriers 1-3 %.  Around the loop:
 //   * persistent workgroups: block b serves XCD b % 8 and walks that XCD's contiguous
 //     run of tiles with stride gridDim/8, so the tiles in flight on an XCD are
 //     neighbours that share an expert's weights in its L2, and no workgroup launch sits
 //     between two tiles;
-//   * tile metadata looked up two tiles ahead, the first K step of the next tile
-//     requested before the epilogue of the current one; the barrier between tiles waits
-//     for LDS traffic only, so a tile's stores drain under the next tile's work;
+//   * tile metadata looked up two tiles ahead;
 //   * hardware bf16 conversion and transcendental-unit sigmoid in the epilogues (they
-//     were VALU bound);
-//   * a wave skips the MFMAs of 16-row blocks that hold no real rows (last tile of an
-//     expert).
+//     were VALU bound).
 //
-// K loop: one barrier per K step of 64.  Per quarter step a wave reads its fragments,
+// K loop of the weight gradients: one barrier per K step of 64.  Per quarter step a wave reads its fragments,
 // parks a quarter of the next step's operands (held in registers) in the other LDS
 // stage, refills those registers with the step after, and issues its MFMAs.  The
 // pipeline tail is peeled at compile time: every load of the steady state is
 // unconditional, so the compiler counts outstanding loads exactly instead of draining
-// the queue once per K step.  Operands are fetched with buffer loads: a wave-uniform
-// resource (the tile's origin), a fixed 32-bit per-thread offset and a scalar K offset,
-// so no per-thread 64-bit address arithmetic or address registers sit in the loop.
+// the queue once per K step.
 //
 // MFMA of the row-tiled kernels: v_mfma_f32_16x16x32_bf16.  Per lane 8 bf16 of each operand (row lane%16,
 // k = 8*(lane/16)..+7), 4 fp32 of the result (column lane%16, rows 4*(lane/16) + i).
@@ -68,14 +74,64 @@ __device__ __forceinline__ float fast_sigmoid(float x) {
   return __builtin_amdgcn_rcpf(1.0f + __expf(-x));
 }
 
-// Raw buffer resource over `base` (wave-uniform): byte offsets up to 4 GiB, no stride, no
-// swizzle; loads through it take a 32-bit per-thread offset and a scalar offset.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, -1, 0x00020000);
-}
-
 // int32 data that no kernel of this file writes (the plan's arrays), for uniform lookups
 typedef const int32_t __attribute__((address_space(4))) * const_i32;
+
+typedef const __attribute__((address_space(3))) char* lds_cptr;
+
+// LDS of the row-tiled kernels, in bytes: two stages of operands (A tile, B tile), 4 KiB a wave for its results
+constexpr uint32_t A_BYTES = 32768, STAGE_BYTES = 65536;
+constexpr int R_LDS_BYTES = 2 * STAGE_BYTES + 8 * 4096;
+
+// Requests 16 (4) bytes a lane from base + voff + soff, straight into LDS: lane l's land at byte lds + 16 l (4 l).  Written
+// out because the compiler drains the whole load counter in front of every LDS read once it knows of such a request; waited for by lds_wait.
+// (base, soff and lds are wave-uniform; byte offsets up to 4 GiB; the wait states are for scalar registers that a vector instruction wrote just before)
+__device__ __forceinline__ u32x4 lds_rsrc(uint64_t base) {
+  return u32x4{static_cast<uint32_t>(base), static_cast<uint32_t>(base >> 32), 0xffffffffu, 0x00020000u};
+}
+__device__ __forceinline__ void lds_load16(uint64_t base, uint32_t voff, uint32_t soff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               ::"s"(lds), "v"(voff), "s"(lds_rsrc(base)), "s"(soff) : "memory");
+}
+__device__ __forceinline__ void lds_load4(uint64_t base, uint32_t voff, uint32_t soff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dword %1, %2, %3 offen lds"
+               ::"s"(lds), "v"(voff), "s"(lds_rsrc(base)), "s"(soff) : "memory");
+}
+// at most N of the wave's requests and stores are still under way
+template <int N>
+__device__ __forceinline__ void lds_wait() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// the wave's LDS reads and writes are done, and at most N of its requests under way; then the workgroup's barrier
+template <int N>
+__device__ __forceinline__ void lds_sync() {
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (N < 63) lds_wait<N>();
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+// the same value, of which the compiler knows nothing: what is formed from it is formed there, not held in registers over a K loop
+__device__ __forceinline__ int opaque(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+// orders a wave's LDS writes and reads of its own region
+__device__ __forceinline__ void wave_lds_sync() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_wave_barrier();
+}
+__device__ __forceinline__ bf16x8 lds_read16(uint32_t at) {
+  return *(const __attribute__((address_space(3))) bf16x8*)(at);
+}
+__device__ __forceinline__ int lds_read_i32(uint32_t at) { return *(const __attribute__((address_space(3))) int*)(at); }
+// eight k of 16 columns from rows of PITCH bytes, k as the 16x16x32 MFMA wants them (frag16_ks)
+template <uint32_t PITCH>
+__device__ __forceinline__ bf16x8 lds_read_tr(uint32_t at) {
+  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(at));
+  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(at + 4 * PITCH));
+  const s16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  return __builtin_bit_cast(bf16x8, v);
+}
 
 // RM_DLIN: the product of RM_DH (rows . w[e], the weight's contraction axis strided) with a plain epilogue:
 // the input gradient of one grouped linear map
@@ -108,8 +164,8 @@ struct RowArgs {
   int n_tiles;
 };
 
-// Row-tiled kernel: 64 WM rows of one expert x 32 NJ (8 / WM) output columns, 8 waves as WM
-// (rows) x 8 / WM (columns), each wave 64 x 32 NJ.  GATEUP's columns are half gate and half
+// Row-tiled kernel: 256 rows of one expert x 64 NJ output columns, 8 waves as 4 (rows) x 2 (columns), each wave
+// 64 rows -- the 16-row blocks w, w + 4, w + 8, w + 12 for wave row w -- x 32 NJ.  GATEUP's columns are half gate and half
 // up columns of the same f range, so a wave holds gate and up of the same 16 NJ f.
 
 struct TileMeta {
@@ -137,24 +193,30 @@ __device__ __forceinline__ float row16_sum(float v) {
 // channels at a time.  The column tile counts only where the output is a whole number of tiles: a last tile
 // that would overhang computes some of its neighbour's columns again and must give the same bits, so both add up in
 // the same order.  An expert's row tiles and, where there are several, its column tiles stay in step: they share operands in L2.
-template <int MODE, int NJ, bool GATHER, int WM, bool SAVE_GU = true, bool TURN = false>
+template <int MODE, int NJ, bool GATHER, bool SAVE_GU = true, bool TURN = false>
 __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
-  constexpr int WN = 8 / WM;               // waves along the columns (WM along the rows)
+  constexpr int WM = 4, WN = 2;            // waves along the rows and along the columns
   constexpr int TBM = 64 * WM;             // rows of the tile
   constexpr int BNT = 32 * NJ * WN;        // output columns of the tile (WN waves x NJ x 32)
-  constexpr int NA = TBM / 64;             // 16-byte A chunks staged per thread and K step
+  constexpr int NA = TBM / 64;             // 1 KiB pieces of the A tile a wave requests per K step
   constexpr int NB = BNT / 64;             // the same for B
-  constexpr int STAGE = (TBM + BNT) * BK;  // elements per LDS stage
   constexpr bool DH_LIKE = (MODE == RM_DH || MODE == RM_DLIN);  // same operands, different epilogue
   constexpr bool B_KS = (DH_LIKE || MODE == RM_DX);
+  // Pieces of B requested behind barrier X and behind barrier Y: the columns that a wave's first half of MFMAs reads and the others; with the
+  // contraction strided its first and its last 32 k (whole rows of the tile, 512 bytes: 256-byte halves of all 64 k, requested apart, cost 4-8 % where the product
+  // is a read of the weights).  Narrow down tiles: a piece holds both halves of a wave's columns.
+  constexpr int NBX = MODE == RM_DOWN && NJ == 2 ? 0 : NB / 2, NBY = NB - NBX;
+  constexpr int VM = NBX ? NA + NB : NA;   // requests younger than those a barrier of the loop waits for
+  constexpr int VM_EPI = NBX ? NBY : 0;    // ... than those that the next tile's first K step needs
   static_assert(!GATHER || MODE == RM_GATEUP || MODE == RM_DH, "only gate/up and dH gather their rows");
   static_assert(!TURN || !B_KS, "only contractions that are contiguous in memory are turned");
   static_assert(!(GATHER && MODE == RM_DH) || NJ == 4 || NJ == 2, "the fused dH epilogue reduces over 16 lanes per row, or 8 and a second wave");
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_cptr)smem));
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave / WN) * 64, wn = wave % WN;
-  const int wave_m = __builtin_amdgcn_readfirstlane(wm);  // the same value, known to be wave-uniform
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = wave / WN, wn = wave % WN;
   const int D = p.D, F = p.F;
   const int Kdim = (MODE == RM_GATEUP || DH_LIKE) ? D : (MODE == RM_DOWN ? F : 2 * F);
   const int lda = (MODE == RM_GATEUP || DH_LIKE) ? D : F;
@@ -164,10 +226,7 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
 
   // Persistent workgroups: block b serves XCD b % 8 and walks that XCD's contiguous run
   // of the tile list with stride gridDim/8, the order in which the hardware dispatcher
-  // would have started one-tile blocks.  Tile metadata is looked up two tiles ahead and
-  // the first operands of the next tile are requested before the epilogue of the current
-  // one, so neither lookup nor first fetch sits between two K loops; a tile's stores
-  // drain under the next tile's work.
+  // would have started one-tile blocks.  Tile metadata is looked up two tiles ahead.
   const int num_tiles = *p.num_tiles;
   const int total = num_tiles * p.n_tiles;
   const int chunk = (total + 7) >> 3;
@@ -213,149 +272,141 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
     return m;
   };
 
-  // ---- global -> register staging: 16-byte chunks q = tid + 512*i ---------------------
-  // KC tiles (8 chunks per row): row (tid>>3) + 64*i, chunk tid&7.
-  // KS tile (BNT/8 chunks per k row): chunk q -> k = q / (BNT/8), chunk q % (BNT/8).
-  u32x4 ra[NA], rb[NB];
-  const int kc_row = tid >> 3, kc_chunk = tid & 7;
-  const int kc_lds = kc_row * BK + ((kc_chunk ^ ((kc_row >> 1) & 7)) << 3);  // + i*64*BK (64 % 16 == 0)
-  int b_lds[NB];
-#pragma unroll
-  for (int i = 0; i < NB; ++i) {
-    if constexpr (!B_KS) {
-      b_lds[i] = kc_lds + i * 64 * BK;
-    } else {
-      constexpr int CPR = BNT / 8;  // chunks per k row
-      const int q = tid + NT * i;
-      const int k = q / CPR, cc = q % CPR;
-      b_lds[i] = k * BNT + ((cc ^ ks_key16(k)) << 3);
-    }
-  }
-  // a wave's 64 x (32 NJ) accumulator tile is 4 x NJ2 MFMA tiles of 16 x 16; with
-  // gate/up the first NJ column tiles are gate columns, the last NJ the same f of up
-  constexpr int NJ2 = 2 * NJ;
-  int bcol[NJ2];
-#pragma unroll
-  for (int nj = 0; nj < NJ2; ++nj) {
-    if constexpr (MODE == RM_GATEUP)
-      bcol[nj] = (nj < NJ ? 0 : BNT / 2) + wn * (16 * NJ) + (nj % NJ) * 16;
-    else
-      bcol[nj] = wn * (32 * NJ) + nj * 16;
-  }
-
-  // Operand addresses are a wave-uniform buffer resource (the tile's origin) plus a fixed 32-bit
-  // per-thread byte offset plus a scalar offset (K step, chunk round): the form buffer loads take
-  // without any per-thread 64-bit arithmetic or address registers.  The B offsets never change;
-  // the A offsets follow the tile's rows.
-  constexpr bool B_REGULAR = !B_KS || (NT % (BNT / 8) == 0);  // chunk index -> fixed row stride
-  constexpr int NBV = B_REGULAR ? 1 : NB;
+  // ---- operand requests: 1 KiB a wave and instruction, straight into LDS --------------------
   const int ldb = B_KS ? Ncols : (MODE == RM_GATEUP ? D : F);
-  uint32_t voffB[NBV];
+  const int kc_row = 8 * wave + (lane >> 3);
+  const int kc_chunk = (lane & 7) ^ ((kc_row >> 1) & 7);
+  uint32_t voffB;
   if constexpr (!B_KS) {
-    voffB[0] = static_cast<uint32_t>(kc_row * ldb + kc_chunk * 8) * 2u;
+    voffB = static_cast<uint32_t>(kc_row * ldb + kc_chunk * 8) * 2u;
   } else {
-    constexpr int CPR = BNT / 8;
-#pragma unroll
-    for (int i = 0; i < NBV; ++i) {
-      const int q = tid + NT * i;
-      voffB[i] = static_cast<uint32_t>((q / CPR) * ldb + (q % CPR) * 8) * 2u;
-    }
+    constexpr int CPR = BNT / 8;  // 16-byte chunks per k row
+    const int k = (64 / CPR) * wave + lane / CPR, cc = (lane % CPR) ^ ks_key16(k);
+    voffB = static_cast<uint32_t>(k * ldb + cc * 8) * 2u;
   }
-  // state of the tile whose operands are being fetched
-  __amdgpu_buffer_rsrc_t rsA0, rsA1;  // A rows (k = 0); DX: second half of the contraction (dup)
-  __amdgpu_buffer_rsrc_t rsB0, rsB1;  // B tile origin in the first / second weight stack
+  // state of the tile whose operands are being requested
+  uint64_t gA0, gA1, gB0, gB1;  // A rows (k = 0), DX: second half of the contraction (dup); the B tile's origin in both weight stacks
   uint32_t voffA[NA];
-  int k_start = 0;
-  // source rows of the A tile: the tile's own rows, or token rows through the gather index
-  auto load_asrc = [&](const TileMeta& m, int (&asrc)[NA]) {
-#pragma unroll
-    for (int i = 0; i < NA; ++i) {
-      const int r = max(min(kc_row + 64 * i, m.valid - 1), 0);
-      // (the index as loaded: it is clamped to [0, a_rows) where it is used, in setup(), a whole K
-      // loop later, so that nothing waits for this load here)
-      asrc[i] = GATHER ? p.a_src[m.row0 + r] : r;
-    }
-  };
+  int k_start = 0, fk = 0;
   auto setup = [&](const TileMeta& m, const int (&asrc)[NA]) {
     const int64_t arow = GATHER ? 0 : static_cast<int64_t>(m.row0) * lda;
-    rsA0 = make_rsrc(p.a0 + arow);
-    rsA1 = (MODE == RM_DX) ? make_rsrc(p.a1 + arow) : rsA0;
+    gA0 = reinterpret_cast<uint64_t>(p.a0 + arow);
+    gA1 = (MODE == RM_DX) ? reinterpret_cast<uint64_t>(p.a1 + arow) : gA0;
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
       const int src = GATHER ? min(max(asrc[i], 0), p.a_rows - 1) : asrc[i];
       voffA[i] = (static_cast<uint32_t>(src) * static_cast<uint32_t>(lda) + static_cast<uint32_t>(kc_chunk * 8)) * 2u;
     }
-    const uint16_t* B0 = p.b0 + m.e * wsz;
-    const uint16_t* B1 = (MODE == RM_GATEUP || MODE == RM_DX) ? p.b1 + m.e * wsz : B0;
     // KC: the tile's first weight row is n0; KS: its first column is n0
-    const int64_t borg = B_KS ? static_cast<int64_t>(m.n0) : static_cast<int64_t>(m.n0) * ldb;
-    rsB0 = make_rsrc(B0 + borg);
-    rsB1 = make_rsrc(B1 + borg);
+    const int64_t borg = m.e * wsz + (B_KS ? static_cast<int64_t>(m.n0) : static_cast<int64_t>(m.n0) * ldb);
+    gB0 = reinterpret_cast<uint64_t>(p.b0 + borg);
+    gB1 = (MODE == RM_GATEUP || MODE == RM_DX) ? reinterpret_cast<uint64_t>(p.b1 + borg) : gB0;
     k_start = m.k_start;
+    fk = 0;
   };
-  // chunk i of the A / B tile of the K step that starts at k0
-  auto load_a = [&](int k0, int i) -> u32x4 {
-    if constexpr (MODE == RM_DX) {
-      if (k0 >= F) return __builtin_amdgcn_raw_buffer_load_b128(rsA1, voffA[i], (k0 - F) * 2, 0);
-    }
-    return __builtin_amdgcn_raw_buffer_load_b128(rsA0, voffA[i], k0 * 2, 0);
-  };
-  auto load_b = [&](int k0, int i) -> u32x4 {
-    if constexpr (MODE == RM_GATEUP) {
-      // rows 0..BNT/2 of the tile come from w1, the rest from w3, same f range
-      const int so = (64 * (i % (NB / 2)) * ldb + k0) * 2;
-      return __builtin_amdgcn_raw_buffer_load_b128(i >= NB / 2 ? rsB1 : rsB0, voffB[0], so, 0);
-    } else if constexpr (MODE == RM_DOWN) {
-      return __builtin_amdgcn_raw_buffer_load_b128(rsB0, voffB[0], (64 * i * ldb + k0) * 2, 0);
-    } else {
-      int kk0 = k0;
-      bool second = false;
-      if constexpr (MODE == RM_DX) {
-        if (k0 >= F) { kk0 = k0 - F; second = true; }
-      }
-      const int so = (kk0 + (B_REGULAR ? i * (NT / (BNT / 8)) : 0)) * ldb * 2;
-      return __builtin_amdgcn_raw_buffer_load_b128(second ? rsB1 : rsB0, voffB[B_REGULAR ? 0 : i], so, 0);
-    }
-  };
-  auto kofs = [&](int ks) {
-    if constexpr (!TURN) return ks * BK;
-    ks += k_start;
+  auto tile_row = [&](const TileMeta& m, int i) { return max(min(kc_row + 64 * i, m.valid - 1), 0); };
+  auto kofs = [&]() {
+    if constexpr (!TURN) return fk * BK;
+    const int ks = fk + k_start;
     return (ks < ksteps ? ks : ks - ksteps) * BK;
   };
-  // request every chunk of K step `step` of the fetch tile
-  // (chunk after chunk in the order of a K step of the loop below, and kept in that order: the
-  // loop's waits count the requests that follow the one they need along every way into the loop,
-  // so every way must issue them alike -- with all A chunks first the park of the first B chunk
-  // waited for five requests more than it needed)
-  auto issue = [&](int step) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      __builtin_amdgcn_sched_barrier(0);
-      if (q < NA) ra[q] = load_a(kofs(step), q);
-#pragma unroll
-      for (int i = (q * NB) / 4; i < ((q + 1) * NB) / 4; ++i) rb[i] = load_b(kofs(step), i);
+  uint32_t fst = 0;  // LDS stage (byte offset) the requests go to
+  const uint32_t wdst = lds0 + wave * 1024u;
+  auto req_a = [&](int i) {
+    int k0 = kofs();
+    uint64_t g = gA0;
+    if constexpr (MODE == RM_DX) {
+      if (k0 >= F) { k0 -= F; g = gA1; }
     }
-    __builtin_amdgcn_sched_barrier(0);
+    lds_load16(g, voffA[i], k0 * 2, fst + wdst + i * 8192u);
   };
+  auto req_b = [&](int i) {
+    int k0 = kofs();
+    const uint32_t dst = fst + wdst + A_BYTES + i * 8192u;
+    if constexpr (MODE == RM_GATEUP) {
+      // rows 0..BNT/2 of the tile come from w1, the rest from w3, same f range
+      lds_load16(i >= NB / 2 ? gB1 : gB0, voffB, (64 * (i % (NB / 2)) * ldb + k0) * 2, dst);
+    } else if constexpr (MODE == RM_DOWN) {
+      lds_load16(gB0, voffB, (64 * i * ldb + k0) * 2, dst);
+    } else {
+      uint64_t g = gB0;
+      if constexpr (MODE == RM_DX) {
+        if (k0 >= F) { k0 -= F; g = gB1; }
+      }
+      lds_load16(g, voffB, (k0 + i * (BK / NB)) * ldb * 2, dst);
+    }
+  };
+  // the pieces of B in the order of the halves
+  auto b_piece = [](int h, int j) { return MODE == RM_DOWN && NBX ? h + 2 * j : h * NBX + j; };
+  auto req_x = [&](int i) {
+    if (i < NA) req_a(i);
+    else req_b(b_piece(0, i - NA));
+  };
+  auto req_y = [&](int j) { req_b(b_piece(1, j)); };
+  auto issue = [&]() {
+#pragma unroll
+    for (int i = 0; i < NA + NBX; ++i) req_x(i);
+#pragma unroll
+    for (int j = 0; j < NBY; ++j) req_y(j);
+    fst ^= STAGE_BYTES;
+    ++fk;
+  };
+
+  // ---- fragment reads ------------------------------------------------------------------------
+  const int l15 = lane & 15, l4 = lane >> 4;
+  const uint32_t cpos = static_cast<uint32_t>((l4 ^ (l15 >> 1)) * 16);  // k 0..31; k 32..63: ^ 64
+  uint32_t ra = lds0 + (16 * wr + l15) * 128u + cpos;
+  uint32_t rb[B_KS ? 4 : 1];
+  if constexpr (!B_KS) {
+    rb[0] = lds0 + A_BYTES + (wn * (MODE == RM_GATEUP ? 16 * NJ : 32 * NJ) + l15) * 128u + cpos;
+  } else {
+    const int k = 8 * l4 + (l15 >> 2);
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const int c = wn * 4 * NJ + b * 2 + ((l15 & 3) >> 1);
+      rb[b] = lds0 + A_BYTES + k * (BNT * 2u) + (c ^ ks_key16(k)) * 16u + (l15 & 1) * 8u;
+    }
+  }
+  auto rd_a = [&](bf16x8 (&f)[4], int kk, int mi) { f[mi] = lds_read16((kk ? ra ^ 64u : ra) + mi * 8192u); };
+  auto rd_b = [&](bf16x8 (&f)[NJ], int kk, int hb, int b) {
+    if constexpr (!B_KS) {
+      const uint32_t base = kk ? rb[0] ^ 64u : rb[0];
+      f[b] = lds_read16(base + (MODE == RM_GATEUP ? hb * (BNT / 2) * 128u + b * 2048u : (hb * NJ + b) * 2048u));
+    } else {
+      f[b] = lds_read_tr<BNT * 2>((NJ == 4 ? rb[b] ^ (hb * 128u) : rb[(hb * NJ + b) & 3]) + kk * 32u * (BNT * 2u));
+    }
+  };
+
+  constexpr int NJ2 = 2 * NJ;
+  f32x4 acc[4][NJ2];
 
   TileMeta cur = load_meta(within);
   TileMeta nxt = load_meta(exists(within + stride) ? within + stride : within);
+  const uint32_t epi = 2 * STAGE_BYTES + wave * 4096u;  // the wave's own 4 KiB
   {
     int asrc[NA];
-    load_asrc(cur, asrc);
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+      const int r = tile_row(cur, i);
+      asrc[i] = GATHER ? p.a_src[cur.row0 + r] : r;
+    }
     setup(cur, asrc);
-    issue(0);
+    issue();
+    issue();
+    lds_sync<VM_EPI>();
   }
 
   for (;;) {
   const bool more = exists(within + stride);
   // the tile after the next: looked up now, used one tile later
   const TileMeta nxt2 = load_meta(exists(within + 2 * stride) ? within + 2 * stride : within);
-  int nsrc[NA];
-  load_asrc(nxt, nsrc);
   const int row0 = cur.row0, valid = cur.valid, n0 = cur.n0, ntile = cur.nt;
+  if constexpr (GATHER) {
+    // the next tile's row indices into the wave's own LDS: lane 8 i + r has that of row r of its i-th piece
+    const int ol = opaque(lane), r = max(min(8 * wave + (ol & 7) + 64 * ((ol >> 3) & 3), nxt.valid - 1), 0);
+    lds_load4(reinterpret_cast<uint64_t>(p.a_src + nxt.row0), r * 4u, 0, lds0 + epi);
+  }
 
-  f32x4 acc[4][NJ2];
 #pragma unroll
   for (int mi = 0; mi < 4; ++mi)
 #pragma unroll
@@ -363,108 +414,115 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) acc[mi][nj][i] = 0.0f;
 
-  // K step 0 (requested before the previous epilogue) -> LDS stage 0, K step 1 -> registers
+  // The tile's 16-row blocks are dealt to the four wave rows in turn, so that a tile that is not full keeps all waves
+  // equally busy; the K loop is instantiated for the number of blocks a wave has.
+  const int act = min(max(((valid + 15) >> 4) - wr + 3, 0) >> 2, 4);
+  auto next_tile = [&]() {
+    if (more) {
+      int asrc[NA];
 #pragma unroll
-  for (int i = 0; i < NA; ++i) *reinterpret_cast<u32x4*>(smem + kc_lds + i * 64 * BK) = ra[i];
+      for (int i = 0; i < NA; ++i)
+        asrc[i] = GATHER ? lds_read_i32(lds0 + epi + (8 * i + (opaque(lane) >> 3)) * 4) : tile_row(nxt, i);
+      setup(nxt, asrc);
+    } else {
+      fk = 0;
+    }
+  };
+  auto k_loop = [&](auto act_t) {
+    constexpr int ACT = decltype(act_t)::value;
+    // A quarter of a K step's MFMAs; what else the quarter holds -- requests of the K step after the next, fragment reads of the
+    // next quarter -- goes out between its 16-row blocks, where the matrix core is busy with the block before.
+    auto mm = [&](const bf16x8 (&af)[4], const bf16x8 (&bf)[NJ], int hb, auto between) {
 #pragma unroll
-  for (int i = 0; i < NB; ++i) *reinterpret_cast<u32x4*>(smem + TBM * BK + b_lds[i]) = rb[i];
-  if (ksteps > 1) issue(1);
-  __syncthreads();
-
-  // One K step.  HAS_NEXT: the registers hold tile ks+1 and are parked in the other LDS
-  // stage.  HAS_NEXT2: tile ks+2 is fetched into the registers.  Both are compile-time
-  // so that every load of the steady-state loop is unconditional: the compiler can then
-  // count outstanding loads exactly and wait only for the three oldest before each park,
-  // instead of draining the queue (vmcnt(0)) once per K step.
-  // The last tile of an expert is partly empty: a wave skips the MFMAs of its 16-row
-  // blocks that hold no real rows (a wave-uniform branch; operands are still staged and
-  // every barrier met).
-  const int act = min(max((valid - wave_m + 15) >> 4, 0), 4);
-  auto kstep = [&](int ks, auto has_next_t, auto has_next2_t) {
-    constexpr bool has_next = decltype(has_next_t)::value;
-    constexpr bool has_next2 = decltype(has_next2_t)::value;
-    const uint16_t* As = smem + (ks & 1) * STAGE;
-    const uint16_t* Bs = As + TBM * BK;
-    uint16_t* An = smem + ((ks + 1) & 1) * STAGE;
-    uint16_t* Bn = An + TBM * BK;
+      for (int mi = 0; mi < 4; ++mi) {
+        __builtin_amdgcn_sched_barrier(0);
+        between(mi);
+        __builtin_amdgcn_sched_barrier(0);
+        if (mi < ACT) {
 #pragma unroll
-    for (int kk = 0; kk < BK / 32; ++kk) {
-      bf16x8 af[4];
-#pragma unroll
-      for (int mi = 0; mi < 4; ++mi) af[mi] = frag16_kc(As, wm + mi * 16, kk, lane);
-#pragma unroll
-      for (int hb = 0; hb < 2; ++hb) {
-        bf16x8 bf[NJ];
-#pragma unroll
-        for (int b = 0; b < NJ; ++b) {
-          if constexpr (B_KS)
-            bf[b] = frag16_ks<BNT>(Bs, bcol[hb * NJ + b], kk, lane);
-          else
-            bf[b] = frag16_kc(Bs, bcol[hb * NJ + b], kk, lane);
-        }
-        // a quarter of the staging traffic rides along with each quarter of the MFMAs:
-        // park the held chunks of tile ks+1 in the other LDS stage, then refill the
-        // same registers with the same chunks of tile ks+2.
-        const int q = kk * 2 + hb;
-        if constexpr (has_next) {
-          // A: two chunks ride with the first two quarters, or one with each of the four
-          if (q < NA) *reinterpret_cast<u32x4*>(An + kc_lds + q * 64 * BK) = ra[q];
-#pragma unroll
-          for (int i = (q * NB) / 4; i < ((q + 1) * NB) / 4; ++i)
-            *reinterpret_cast<u32x4*>(Bn + b_lds[i]) = rb[i];
-        }
-        if constexpr (has_next2) {
-          if (q < NA) ra[q] = load_a(kofs(ks + 2), q);
-#pragma unroll
-          for (int i = (q * NB) / 4; i < ((q + 1) * NB) / 4; ++i) rb[i] = load_b(kofs(ks + 2), i);
-        }
-#pragma unroll
-        for (int mi = 0; mi < 4; ++mi) {
-          if (mi < act) {
-#pragma unroll
-            for (int b = 0; b < NJ; ++b)
-              acc[mi][hb * NJ + b] =
-                  __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[b], af[mi], acc[mi][hb * NJ + b], 0, 0, 0);
-          }
+          for (int b = 0; b < NJ; ++b)
+            acc[mi][hb * NJ + b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[b], af[mi], acc[mi][hb * NJ + b], 0, 0, 0);
         }
       }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    bf16x8 a0[4], a1[4], b0[NJ], b1[NJ];
+#pragma unroll
+    for (int i = 0; i < ACT; ++i) rd_a(a0, 0, i);
+#pragma unroll
+    for (int b = 0; b < NJ; ++b) rd_b(b0, 0, 0, b);
+    for (int ks = 0; ks < ksteps; ++ks) {
+      if (ks == ksteps - 2) next_tile();
+      // contraction contiguous: first columns k 0-31, k 32-63, last columns likewise; strided: k 0-31 first and last columns, k 32-63 likewise
+      mm(a0, b0, 0, [&](int q) {
+        if (q < ACT) rd_a(a1, 1, q);
+        if (q < NJ) rd_b(b1, B_KS ? 0 : 1, B_KS ? 1 : 0, q);
+      });
+      if (NBX > 0 && ks > 0) lds_wait<VM>();
+      lds_sync<63>();
+      mm(B_KS ? a0 : a1, b1, B_KS ? 1 : 0, [&](int q) {
+        if (q == 0) return;
+        req_x(q - 1);
+#pragma unroll
+        for (int b = (q - 1) * 2; b < q * 2 && b < NJ; ++b) rd_b(b0, B_KS ? 1 : 0, B_KS ? 0 : 1, b);
+      });
+      mm(B_KS ? a1 : a0, b0, B_KS ? 0 : 1, [&](int q) {
+        if (q + 3 < NA + NBX) req_x(q + 3);
+#pragma unroll
+        for (int b = q * 2; b < q * 2 + 2 && b < NJ; ++b) rd_b(b1, 1, 1, b);
+      });
+      if (ks > 0) lds_wait<VM>();
+      lds_sync<63>();
+      ra ^= STAGE_BYTES;
+#pragma unroll
+      for (int b = 0; b < (B_KS ? 4 : 1); ++b) rb[b] ^= STAGE_BYTES;
+      mm(a1, b1, 1, [&](int q) {
+        if (q == 0) return;
+        if (q - 1 < NBY) req_y(q - 1);
+#pragma unroll
+        for (int i = (q - 1) * 2; i < q * 2 && i < 4; ++i) {
+          if (i < ACT) rd_a(a0, 0, i);
+          if (i < NJ) rd_b(b0, 0, 0, i);
+        }
+      });
+      fst ^= STAGE_BYTES;
+      ++fk;
     }
-    __syncthreads();
   };
-  using T_ = std::true_type;
-  using F_ = std::false_type;
-  int ks = 0;
-  for (; ks + 2 < ksteps; ++ks) kstep(ks, T_{}, T_{});
-  if (ks + 1 < ksteps) { kstep(ks, T_{}, F_{}); ++ks; }
-  if (ks < ksteps) kstep(ks, F_{}, F_{});
-
-  // switch the fetch state to the next tile and request its first K step: the loads
-  // are in flight while the epilogue below runs
-  if (more) {
-    setup(nxt, nsrc);
-    issue(0);
+  switch (act) {
+    case 0: k_loop(std::integral_constant<int, 0>{}); break;
+    case 1: k_loop(std::integral_constant<int, 1>{}); break;
+    case 2: k_loop(std::integral_constant<int, 2>{}); break;
+    case 3: k_loop(std::integral_constant<int, 3>{}); break;
+    default: k_loop(std::integral_constant<int, 4>{});
   }
 
-  // ---- epilogue: through the wave's private LDS region, 16-byte coalesced rows ---------
+  // ---- epilogue: 16 rows at a time through the wave's own LDS, 16-byte coalesced rows ----
   // acc[mi][nj][i]: output row = wm + mi*16 + (lane&15); output column within the nj-th
   // 16-column tile = 4*(lane>>4) + i.
-  uint16_t* st = smem + wave * (64 * 136);  // 8 waves x 17 KiB < 160 KiB; the barrier ending the K loop freed the tiles
+  const int el = opaque(lane);
+  constexpr int CH = 4 * NJ;  // 16-byte chunks per row of the wave's sub-tile
+  auto key = [](int m) { return CH == 16 ? m : m >> 1; };
+  auto put = [&](int m0, int nj, float v0, float v1, float v2, float v3) {
+    const u32x2 pk = {pack2(v0, v1), pack2(v2, v3)};
+    const int c = nj * 2 + ((el >> 4) >> 1);
+    *reinterpret_cast<u32x2*>(reinterpret_cast<char*>(smem) + epi + (el & 15) * (CH * 16) + ((c ^ key((el & 15))) * 16) + ((el >> 4) & 1) * 8) = pk;
+  };
+  auto get = [&](int m, int c) {
+    return *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(smem) + epi + m * (CH * 16) + ((c ^ key(m)) * 16));
+  };
   if constexpr (MODE == RM_GATEUP) {
-    // per 32-row half: three 32 x 16 NJ tiles gate | up | h side by side, a [32][48 NJ + 8] region (12.5 KiB
-    // per wave with NJ = 4); without gate and up, h alone in a [32][16 NJ + 8] region
-    constexpr int NT3 = SAVE_GU ? 3 : 1;       // output tiles per row
+    // 16 rows of gate and up side by side (16 NJ columns each), then of h in the same place
     constexpr int WC = 16 * NJ, CPT = WC / 8;  // columns and chunks of one of them
-    using S = WaveStage<WC * NT3>;
-    uint16_t* sg = smem + wave * (32 * S::PITCH);
     const int f0 = n0 + wn * WC;
+    lds_wait<VM_EPI>();
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      if (wave_m + half * 32 >= valid) continue;  // no real rows in this half (uniform per wave)
+    for (int mi = 0; mi < 4; ++mi) {
+      if (mi >= act) continue;
 #pragma unroll
-      for (int ml = 0; ml < 2; ++ml)
+      for (int part = SAVE_GU ? 0 : 1; part < 2; ++part) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-          const int mi = half * 2 + ml;
           float g[4], u[4], h[4];
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
@@ -473,61 +531,59 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
             const float s = round_bf16(g[r] * fast_sigmoid(g[r]));
             h[r] = s * u[r];
           }
-          if constexpr (SAVE_GU) {
-            S::put16(sg, ml, j * 16, lane, g[0], g[1], g[2], g[3]);
-            S::put16(sg, ml, WC + j * 16, lane, u[0], u[1], u[2], u[3]);
+          if (part == 0) {
+            put(mi, j, g[0], g[1], g[2], g[3]);
+            put(mi, NJ + j, u[0], u[1], u[2], u[3]);
+          } else {
+            put(mi, j, h[0], h[1], h[2], h[3]);
           }
-          S::put16(sg, ml, (SAVE_GU ? 2 * WC : 0) + j * 16, lane, h[0], h[1], h[2], h[3]);
         }
-      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the wave's own LDS writes have landed
-      __builtin_amdgcn_wave_barrier();
-      // 32 rows x NT3 tiles x CPT chunks, CPT / 2 NT3 per lane
-#pragma unroll 4
-      for (int it = 0; it < CPT / 2 * NT3; ++it) {
-        const int idx = it * 64 + lane;
-        const int m = idx / (CPT * NT3), rem = idx % (CPT * NT3), t = rem / CPT, c = rem % CPT;
-        const int f = f0 + c * 8;  // < F: tiles never overhang in the columns
-        const int mr = wm + half * 32 + m;
-        if (mr < valid) {
-          const u32x4 v = *reinterpret_cast<const u32x4*>(sg + m * S::PITCH + t * WC + c * 8);
-          uint16_t* dst = (!SAVE_GU ? p.o2 : (t == 0 ? p.o0 : (t == 1 ? p.o1 : p.o2))) + static_cast<int64_t>(row0 + mr) * F + f;
-          *reinterpret_cast<u32x4*>(dst) = v;
+        wave_lds_sync();
+        const int chunks = part == 0 ? CH : CPT;  // per row
+#pragma unroll
+        for (int it = 0; it < chunks / 4; ++it) {
+          const int idx = it * 64 + el;
+          const int m = idx / chunks, rem = idx % chunks, t = rem / CPT, c = rem % CPT;
+          const int mr = mi * 64 + wr * 16 + m;
+          if (mr < valid) {
+            const u32x4 v = get(m, rem);
+            uint16_t* dst = (part == 1 ? p.o2 : (t == 0 ? p.o0 : p.o1)) + static_cast<int64_t>(row0 + mr) * F + f0 + c * 8;
+            *reinterpret_cast<u32x4*>(dst) = v;
+          }
         }
+        wave_lds_sync();
       }
-      __builtin_amdgcn_s_waitcnt(0xc07f);
-      __builtin_amdgcn_wave_barrier();
     }
-  } else if (wave_m < valid) {
-    using S = WaveStage<32 * NJ>;
-    constexpr int CH = 4 * NJ;  // 16-byte chunks per row of the wave's sub-tile
-#pragma unroll
-    for (int mi = 0; mi < 4; ++mi)
-#pragma unroll
-      for (int nj = 0; nj < NJ2; ++nj)
-        S::put16(st, mi, nj * 16, lane, acc[mi][nj][0], acc[mi][nj][1], acc[mi][nj][2], acc[mi][nj][3]);
-    __builtin_amdgcn_s_waitcnt(0xc07f);
-    __builtin_amdgcn_wave_barrier();
+  } else if (act > 0) {
     const int c0 = n0 + wn * (32 * NJ);
-    // 64 rows x CH chunks, CH per lane; a row's bytes go out contiguously; tiles never
+    // 64 rows x CH chunks, CH per el; a row's bytes go out contiguously; tiles never
     // overhang in the columns.  Where the epilogue also LOADS (dH), lanes whose row lies past
     // the tile's real rows redo the last real row instead (the same bytes to the same
     // address), so that every load and store is unconditional: the compiler then knows how
     // many are in flight and waits for exactly the ones it needs -- with predicated accesses
     // every wait drains the whole queue, stores included (one counter serves both here).
-    const int last = valid - 1 - wm;  // >= 0 in this branch
-    auto chunk_at = [&](int it, int& m, int& c) {
-      const int idx = it * 64 + lane;
-      m = min(idx / CH, last);
+    constexpr int IPB = CH / 4;  // 16-byte pieces a el has of a block of 16 rows
+    // the u-th of them in the mi-th block: row of the block and chunk; row of the tile
+    auto chunk_at = [&](int mi, int u, int& m, int& c) {
+      const int idx = u * 64 + el;
+      m = min(idx / CH, valid - 1 - (mi * 64 + wr * 16));
       c = idx % CH;
     };
-    auto offset_at = [&](int it) -> int64_t {
+    auto row_at = [&](int mi, int m) { return row0 + mi * 64 + wr * 16 + m; };
+    auto offset_at = [&](int mi, int u) -> int64_t {
       int m, c;
-      chunk_at(it, m, c);
-      return static_cast<int64_t>(row0 + wm + m) * Ncols + c0 + c * 8;
+      chunk_at(mi, u, m, c);
+      return static_cast<int64_t>(row_at(mi, m)) * Ncols + c0 + c * 8;
+    };
+    auto stage = [&](int mi) {
+#pragma unroll
+      for (int nj = 0; nj < NJ2; ++nj)
+        put(mi, nj, acc[mi][nj][0], acc[mi][nj][1], acc[mi][nj][2], acc[mi][nj][3]);
+      wave_lds_sync();
     };
     if constexpr (MODE == RM_DH) {
       // SwiGLU backward on 8 consecutive f: dgate = dh*up*silu'(gate), dup = dh*silu(gate).
-      // gate and up of the next four chunks are requested before the current four are stored:
+      // gate and up of the next 16 rows are requested before the current ones are stored:
       // a load issued behind a store cannot complete before it.
       // With the combine's backward folded in (FUSE), the staged value is the unscaled dh row:
       // its product with the row's h (recomputed from gate and up) summed over f is the
@@ -535,44 +591,38 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
       // and written once per row and 128-column slot; dh itself is then scaled by the score,
       // and score * h goes out as the operand of the dW2 product.
       constexpr bool FUSE = GATHER;
-      constexpr int G = 4;
-      static_assert(CH % G == 0, "chunks per row come in groups of four");
-      auto row_at = [&](int it) -> int {
-        int m, c;
-        chunk_at(it, m, c);
-        return row0 + wm + m;
-      };
-      [[maybe_unused]] float* dots = reinterpret_cast<float*>(st + 64 * S::PITCH);
-      static_assert(64 * S::PITCH + 128 <= 64 * 136 || NJ == 4, "the rows' sums lie behind the wave's tile");
+      constexpr int G = IPB;
+      [[maybe_unused]] float* dots = reinterpret_cast<float*>(reinterpret_cast<char*>(smem) + epi + 2048);
       u32x4 gq[G], uq[G];
-      float sq[G];
+      float sq = 1.0f;  // lane l: the score of the block's row l % 16
+      auto request = [&](int mi, u32x4 (&g)[G], u32x4 (&u)[G], float& sc) {
 #pragma unroll
-      for (int u = 0; u < G; ++u) {
-        const int64_t o = offset_at(u);
-        gq[u] = *reinterpret_cast<const u32x4*>(p.gate + o);
-        uq[u] = *reinterpret_cast<const u32x4*>(p.up + o);
-        if constexpr (FUSE) sq[u] = p.row_scale[row_at(u)];
-      }
-#pragma unroll
-      for (int g0 = 0; g0 < CH; g0 += G) {
-        u32x4 gn[G], un[G];
-        float sn[G];
-        if (g0 + G < CH) {
-#pragma unroll
-          for (int u = 0; u < G; ++u) {
-            const int64_t o = offset_at(g0 + G + u);
-            gn[u] = *reinterpret_cast<const u32x4*>(p.gate + o);
-            un[u] = *reinterpret_cast<const u32x4*>(p.up + o);
-            if constexpr (FUSE) sn[u] = p.row_scale[row_at(g0 + G + u)];
-          }
+        for (int i = 0; i < G; ++i) {
+          int m, c;
+          chunk_at(mi, i, m, c);
+          const int64_t o = offset_at(mi, i);
+          g[i] = *reinterpret_cast<const u32x4*>(p.gate + o);
+          u[i] = *reinterpret_cast<const u32x4*>(p.up + o);
         }
+        if constexpr (FUSE) sc = p.row_scale[row_at(mi, min(el & 15, valid - 1 - (mi * 64 + wr * 16)))];
+      };
+      request(0, gq, uq, sq);
+      lds_wait<2 * G>();  // (2 G requests and more are younger than the next tile's operands)
+#pragma unroll
+      for (int mi = 0; mi < 4; ++mi) {
+        if (mi >= act) break;
+        u32x4 gn[G], un[G];
+        float sn;
+        // (the last block again past it: every load is unconditional)
+        if (mi < 3) request(min(mi + 1, act - 1), gn, un, sn);
+        stage(mi);
 #pragma unroll
         for (int u = 0; u < G; ++u) {
           int m, c;
-          chunk_at(g0 + u, m, c);
-          const u32x4 v = *reinterpret_cast<const u32x4*>(st + m * S::PITCH + c * 8);
+          chunk_at(mi, u, m, c);
+          const u32x4 v = get(m, c);
           const u32x4 gv = gq[u], uv = uq[u];
-          const float sc = FUSE ? sq[u] : 1.0f;
+          const float sc = FUSE ? __shfl(sq, m) : 1.0f;
           float dot = 0.0f;
           u32x4 dg, du, hs;
 #pragma unroll
@@ -599,7 +649,7 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
             du[w] = pack2(r_du[0], r_du[1]);
             if constexpr (FUSE) hs[w] = pack2(r_hs[0], r_hs[1]);
           }
-          const int64_t o = offset_at(g0 + u);
+          const int64_t o = offset_at(mi, u);
           *reinterpret_cast<u32x4*>(p.o0 + o) = dg;
           *reinterpret_cast<u32x4*>(p.o1 + o) = du;
           if constexpr (FUSE) {
@@ -610,53 +660,58 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
             const float total = row16_sum<CH>(dot);
             // all 16 lanes of the row store the same value to the same address (unconditional,
             // like every other access of this epilogue); of a narrow tile, whose 128 columns are two waves', to LDS
-            if constexpr (NJ == 4) p.dot_partial[static_cast<int64_t>(row0 + wm + m) * p.dot_slots + ntile * WN + wn] = total;
-            else dots[m] = total;
+            if constexpr (NJ == 4) p.dot_partial[static_cast<int64_t>(row_at(mi, m)) * p.dot_slots + ntile * WN + wn] = total;
+            else dots[mi * 16 + m] = total;
           }
         }
-        if (g0 + G < CH) {
+        wave_lds_sync();
+        if (mi < 3) {
 #pragma unroll
           for (int u = 0; u < G; ++u) {
             gq[u] = gn[u];
             uq[u] = un[u];
-            if constexpr (FUSE) sq[u] = sn[u];
           }
+          if constexpr (FUSE) sq = sn;
         }
       }
     } else {
-      // plain copies, unconditional as well: lanes past the last real row store that row again
-      // (same bytes, same address; the line is still in L2), so the stores are countable and
-      // the next tile's first operands are not held up behind them (0.3 % per step; with an
-      // expert's tiles equally tall a tile is rarely less than half full)
-#pragma unroll 4
-      for (int it = 0; it < CH; ++it) {
-        const int idx = it * 64 + lane;
-        const int m = min(idx / CH, last), c = idx % CH;
-        *reinterpret_cast<u32x4*>(p.o0 + static_cast<int64_t>(row0 + wm + m) * Ncols + c0 + c * 8) =
-            *reinterpret_cast<const u32x4*>(st + m * S::PITCH + c * 8);
+      lds_wait<VM_EPI>();
+#pragma unroll
+      for (int mi = 0; mi < 4; ++mi) {
+        if (mi < act) {
+          stage(mi);
+#pragma unroll
+          for (int u = 0; u < IPB; ++u) {
+            int m, c;
+            chunk_at(mi, u, m, c);
+            *reinterpret_cast<u32x4*>(p.o0 + offset_at(mi, u)) = get(m, c);
+          }
+        }
+        wave_lds_sync();
       }
     }
+  } else {
+    lds_wait<VM_EPI>();
   }
-  // every wave is done with its staging region before the next tile's operands are parked;
-  // only LDS traffic is waited for, the tile's stores keep draining
-  phase_barrier();
   if constexpr (MODE == RM_DH && GATHER && NJ == 2) {
     // a narrow tile's slot: both waves' sums; the slots past the last tile's, which a wide tile would have filled, are zero
-    if (wn == 0 && lane < valid - wave_m) {
-      const float* dots = reinterpret_cast<const float*>(st + 64 * WaveStage<32 * NJ>::PITCH);
-      const float* other = reinterpret_cast<const float*>(st + 64 * 136 + 64 * WaveStage<32 * NJ>::PITCH);
-      float* slot = p.dot_partial + static_cast<int64_t>(row0 + wm + lane) * p.dot_slots;
-      slot[ntile] = dots[lane] + other[lane];
+    lds_sync<63>();
+    const int m = (el >> 4) * 64 + wr * 16 + (el & 15);  // of the tile
+    if (wn == 0 && m < valid) {
+      const float* dots = reinterpret_cast<const float*>(reinterpret_cast<const char*>(smem) + epi + 2048);
+      const float* other = dots + 1024;
+      float* slot = p.dot_partial + static_cast<int64_t>(row0 + m) * p.dot_slots;
+      slot[ntile] = dots[el] + other[el];
       if (ntile == p.n_tiles - 1)
         for (int i = p.n_tiles; i < p.dot_slots; ++i) slot[i] = 0.0f;
     }
-    phase_barrier();
   }
   if (!more) break;
   within += stride;
   cur = nxt;
   nxt = nxt2;
   }
+  lds_wait<0>();
 }
 
 // ---- weight gradients: C[e](M,N) = sum_{r in segment e} A[r][m] * B[r][n] ----------
@@ -1041,20 +1096,20 @@ static int launch_row(RowArgs& a, int64_t width, int64_t El, int64_t tile_capaci
     a.n_tiles = (int)((width + 128 / div - 1) / (128 / div));
     static PerDeviceOnce narrow_configured;
     if (narrow_configured.needed()) {
-      if (int rc = set_lds(row_tiled_kernel<MODE, 2, GATHER, 4, SAVE_GU, TURN>, W_LDS_BYTES)) return rc;
+      if (int rc = set_lds(row_tiled_kernel<MODE, 2, GATHER, SAVE_GU, TURN>, R_LDS_BYTES)) return rc;
       narrow_configured.done();
     }
     const unsigned blocks = std::min(round8(tile_capacity * a.n_tiles), resident_blocks());
-    hipLaunchKernelGGL((row_tiled_kernel<MODE, 2, GATHER, 4, SAVE_GU, TURN>), dim3(blocks), dim3(NT), W_LDS_BYTES, s, a);
+    hipLaunchKernelGGL((row_tiled_kernel<MODE, 2, GATHER, SAVE_GU, TURN>), dim3(blocks), dim3(NT), R_LDS_BYTES, s, a);
     return check_launch(what);
   }
   static PerDeviceOnce configured;  // one per kernel instantiation
   if (configured.needed()) {
-    if (int rc = set_lds(row_tiled_kernel<MODE, 4, GATHER, 4, SAVE_GU, TURN>, W_LDS_BYTES)) return rc;
+    if (int rc = set_lds(row_tiled_kernel<MODE, 4, GATHER, SAVE_GU, TURN>, R_LDS_BYTES)) return rc;
     configured.done();
   }
   const unsigned blocks = std::min(round8(tile_capacity * a.n_tiles), resident_blocks());
-  hipLaunchKernelGGL((row_tiled_kernel<MODE, 4, GATHER, 4, SAVE_GU, TURN>), dim3(blocks), dim3(NT), W_LDS_BYTES, s, a);
+  hipLaunchKernelGGL((row_tiled_kernel<MODE, 4, GATHER, SAVE_GU, TURN>), dim3(blocks), dim3(NT), R_LDS_BYTES, s, a);
   return check_launch(what);
 }
 
