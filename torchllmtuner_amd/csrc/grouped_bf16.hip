@@ -89,9 +89,14 @@ constexpr int R_LDS_BYTES = 2 * STAGE_BYTES + 8 * 4096;
 __device__ __forceinline__ u32x4 lds_rsrc(uint64_t base) {
   return u32x4{static_cast<uint32_t>(base), static_cast<uint32_t>(base >> 32), 0xffffffffu, 0x00020000u};
 }
+template <bool STREAM = false>  // with the non-temporal hint
 __device__ __forceinline__ void lds_load16(uint64_t base, uint32_t voff, uint32_t soff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               ::"s"(lds), "v"(voff), "s"(lds_rsrc(base)), "s"(soff) : "memory");
+  if constexpr (STREAM)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
+                 ::"s"(lds), "v"(voff), "s"(lds_rsrc(base)), "s"(soff) : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 ::"s"(lds), "v"(voff), "s"(lds_rsrc(base)), "s"(soff) : "memory");
 }
 __device__ __forceinline__ void lds_load4(uint64_t base, uint32_t voff, uint32_t soff, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dword %1, %2, %3 offen lds"
@@ -162,6 +167,7 @@ struct RowArgs {
   const int32_t* num_tiles;
   int D, F;
   int n_tiles;
+  int stream;  // weights of experts with one row tile are read with the non-temporal hint
 };
 
 // Row-tiled kernel: 256 rows of one expert x 64 NJ output columns, 8 waves as 4 (rows) x 2 (columns), each wave
@@ -171,6 +177,7 @@ struct RowArgs {
 struct TileMeta {
   int e, row0, valid, n0, nt;
   int k_start;  // the contraction's first K step; it goes on from step 0 after the last
+  bool stream;  // no other tile reads the weights
 };
 
 // sum over each group of 16 (8) consecutive lanes, left in all of them (DPP row operations)
@@ -268,6 +275,7 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
     constexpr int W = (MODE == RM_GATEUP ? BNT / 2 : BNT);
     m.n0 = min(nt * W, Ncols - W);
     m.nt = nt;
+    m.stream = p.stream && nrt == 1;
     m.k_start = TURN ? (5 * m.e + (nrt == 1 && Ncols % W == 0 ? 3 * nt : 0)) % ksteps : 0;
     return m;
   };
@@ -288,6 +296,7 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
   uint64_t gA0, gA1, gB0, gB1;  // A rows (k = 0), DX: second half of the contraction (dup); the B tile's origin in both weight stacks
   uint32_t voffA[NA];
   int k_start = 0, fk = 0;
+  bool stream = false;
   auto setup = [&](const TileMeta& m, const int (&asrc)[NA]) {
     const int64_t arow = GATHER ? 0 : static_cast<int64_t>(m.row0) * lda;
     gA0 = reinterpret_cast<uint64_t>(p.a0 + arow);
@@ -302,6 +311,7 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
     gB0 = reinterpret_cast<uint64_t>(p.b0 + borg);
     gB1 = (MODE == RM_GATEUP || MODE == RM_DX) ? reinterpret_cast<uint64_t>(p.b1 + borg) : gB0;
     k_start = m.k_start;
+    stream = m.stream;
     fk = 0;
   };
   auto tile_row = [&](const TileMeta& m, int i) { return max(min(kc_row + 64 * i, m.valid - 1), 0); };
@@ -322,19 +332,23 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
   };
   auto req_b = [&](int i) {
     int k0 = kofs();
-    const uint32_t dst = fst + wdst + A_BYTES + i * 8192u;
+    uint64_t g = gB0;
+    uint32_t so;
     if constexpr (MODE == RM_GATEUP) {
       // rows 0..BNT/2 of the tile come from w1, the rest from w3, same f range
-      lds_load16(i >= NB / 2 ? gB1 : gB0, voffB, (64 * (i % (NB / 2)) * ldb + k0) * 2, dst);
+      if (i >= NB / 2) g = gB1;
+      so = (64 * (i % (NB / 2)) * ldb + k0) * 2;
     } else if constexpr (MODE == RM_DOWN) {
-      lds_load16(gB0, voffB, (64 * i * ldb + k0) * 2, dst);
+      so = (64 * i * ldb + k0) * 2;
     } else {
-      uint64_t g = gB0;
       if constexpr (MODE == RM_DX) {
         if (k0 >= F) { k0 -= F; g = gB1; }
       }
-      lds_load16(g, voffB, (k0 + i * (BK / NB)) * ldb * 2, dst);
+      so = (k0 + i * (BK / NB)) * ldb * 2;
     }
+    const uint32_t dst = fst + wdst + A_BYTES + i * 8192u;
+    if (stream) lds_load16<true>(g, voffB, so, dst);
+    else lds_load16(g, voffB, so, dst);
   };
   // the pieces of B in the order of the halves
   auto b_piece = [](int h, int j) { return MODE == RM_DOWN && NBX ? h + 2 * j : h * NBX + j; };
@@ -1085,12 +1099,24 @@ static bool narrow(int mode, int64_t El, int64_t n, int64_t tile_capacity) {
   return tiles * n <= (spare * 10 > tiles * 7 ? cus * 3 / 8 : cus / 2);
 }
 
+// Whether experts with one row tile -- whose weights no other tile reads -- have them read with the non-temporal hint: where the three weight stacks do
+// not stay in the 256 MB of memory-side cache from one product to the next, putting them there costs more than it can give back.  us, as ever / with the hint:
+//   one product, 128 experts of 2048 x 768, 1000 tokens of eight: gate/up 165 / 150 (5.4 TB/s), down 93 / 86, dH 107 / 95, dRows 153 / 147; 32 of 7168 x
+//   2048, nine rows each: 312 / 276 (6.8 TB/s), 170 / 149, 161 / 141, 336 / 299, 128 rows each 363 / 337, 203 / 184, 194 / 169, 387 / 369
+//   block forward, then a training step, 24 / 80 / 180 rows an expert, time with the hint over without, by the stacks' size: 16 experts of 1024 x 512 (48 MiB) 1.08
+//   1.07 1.08, 1.0-1.03; 16 of 2048 x 1024 (192) 1.11 1.12 1.12, 1.10 1.08 1.05; 60 of 1280 x 640 (281) 1.01 1.06 1.03, 1.04 1.01 0.99; 32 of 1792 x
+//   1024 (336) 0.91 0.95 1.02, 1.0 1.01 1.01; 60 of 2048 x 512 (360) 0.92 0.95 0.99, 0.92 0.94 0.97; 128 of 1024 x 512 (384) 0.90 0.98 1.01, 0.96 0.92 0.92;
+//   128 of 1024 x 1024 (768) 0.90 0.97 0.96, 0.94 0.84 0.93
+// With two row tiles or more an expert, which share the weights in L2, the hint costs 2-8 % (8192 tokens of the first block, 16384 of a skewed router).
+static bool streamed(int64_t El, int64_t D, int64_t F) { return El * D * F * 6 > (int64_t{320} << 20); }
+
 // width: output columns; gate/up tiles hold both halves of their column range.  Tiles are
 // 256 or 128 wide (a 192-wide KS tile would not hold the swizzle: 24 chunks per row are not a multiple
 // of the 16 the key permutes); an overhanging last tile shifts back.
 template <int MODE, bool GATHER = false, bool SAVE_GU = true, bool TURN = false>
 static int launch_row(RowArgs& a, int64_t width, int64_t El, int64_t tile_capacity, hipStream_t s, const char* what) {
   constexpr int div = MODE == RM_GATEUP ? 2 : 1;
+  a.stream = streamed(El, a.D, a.F);
   a.n_tiles = (int)((width + 256 / div - 1) / (256 / div));
   if (narrow(MODE, El, a.n_tiles, tile_capacity)) {
     a.n_tiles = (int)((width + 128 / div - 1) / (128 / div));
