@@ -1,5 +1,6 @@
-"""The wide row tiles' ring of operand stages and dealt 16-row blocks, row by row against fp32 products: row counts on either
-side of a block, of a round of the four wave rows and of a tile; contractions of six K steps (the fewest) and of odd numbers of
+"""The rings of operand stages of the wide row tiles, whose 16-row blocks are dealt to the waves, and of the weight gradients, row by
+row and expert by expert against fp32 products: row counts on either side of a block, of a round of the four wave rows, of a tile and of one and two
+K steps of a weight gradient; contractions of six K steps (the fewest) and of odd numbers of
 them; more tiles than workgroups, so that one tile's operands arrive while another's results leave."""
 
 from __future__ import annotations
@@ -29,11 +30,11 @@ def test_rows(counts, D, Fd):
     plan = wide(ops.permute_plan(ids.to(DEV), El))
     weights = torch.rand(R, 1, generator=g).to(DEV)
     y, gate, up, h = ops.grouped_swiglu_fwd(x, w1, w3, w2, plan, gather=True)
-    dx, _, _, _, dweights = ops.grouped_swiglu_combine_bwd(dout, x, weights, w1, w3, w2, gate, up, plan)
+    dx, dw1, dw3, dw2, dweights = ops.grouped_swiglu_combine_bwd(dout, x, weights, w1, w3, w2, gate, up, plan)
     tok = plan.token_of_row.long()
     rows = ops.permute_rows_fwd(x, plan)
     linear = ops.grouped_linear(rows, w1, plan)
-    dlinear = ops.grouped_linear_bwd(linear, rows, w1, plan)[0]
+    dlinear, dwlinear = ops.grouped_linear_bwd(linear, rows, w1, plan)
     gather = ops.grouped_swiglu_fwd(rows, w1, w3, w2, plan)
     assert all(torch.equal(a, b) for a, b in zip((y, gate, up, h), gather))
     slot, start = plan.row_of_slot.flatten().long(), 0
@@ -43,6 +44,7 @@ def test_rows(counts, D, Fd):
     dots[slot] = dweights.flatten()
     for e, n in enumerate(counts):
         if n == 0:
+            assert not any(t[e].any() for t in (dw1, dw3, dw2, dwlinear))
             continue
         r = slice(start, start + n)
         start += n
@@ -61,3 +63,41 @@ def test_rows(counts, D, Fd):
         dg, du = dh * uf * sig * (1 + gf * (1 - sig)), dh * gf * sig
         # dh, its products with up and with the activation's derivative and the row itself: four roundings of at most 2^-9 each
         assert row_errors(drows[r], dg @ w1[e].float() + du @ w3[e].float()) < 2.0 ** -7
+        # one rounding; and those of dh, hs or the operands above before it
+        assert row_errors(dwlinear[e].flatten()[None], (linear[r].float().T @ xe).flatten()[None]) < 2.0 ** -8
+        for got, want in ((dw1[e], dg.T @ xe), (dw3[e], du.T @ xe), (dw2[e], de.T @ (s * h[r].float()))):
+            assert row_errors(got.flatten()[None], want.flatten()[None]) < 2.0 ** -7
+
+
+@pytest.mark.parametrize("counts", [(63, 1, 70, 129, 5), (128, 200, 64, 0, 3, 65), (1,) * 20])
+def test_rows_of_other_experts_stay_out_of_a_weight_gradient(counts):
+    """The last K step of an expert's contraction reads past its rows: what lies there must not count, whatever it is."""
+    from torchllmtuner_amd import ops
+
+    print(f"weight gradients beside rows that are not finite {counts[:6]}", flush=True)
+    g = torch.Generator().manual_seed(3)
+    El, R, D, Fd = len(counts), sum(counts), 448, 384
+    ids = torch.repeat_interleave(torch.arange(El), torch.tensor(counts))[:, None]
+    plan = ops.permute_plan(ids.to(DEV), El)
+    assert torch.equal(plan.token_of_row.cpu().long(), torch.arange(R))
+    x, dy = torch.randn(R, D, generator=g).bfloat16(), torch.randn(R, Fd, generator=g).bfloat16()
+    w = (torch.randn(El, Fd, D, generator=g) * 0.03).bfloat16().to(DEV)
+    gate, up = (torch.randn(R, Fd, generator=g).bfloat16().to(DEV) for _ in "gu")
+    w2 = (torch.randn(El, D, Fd, generator=g) * 0.03).bfloat16().to(DEV)
+    weights = torch.rand(R, 1, generator=g).to(DEV)
+
+    def grads(x, dy):
+        x, dy = x.to(DEV), dy.to(DEV)
+        dout = x.flip(1).contiguous()
+        return [ops.grouped_linear_bwd(dy, x, w, plan)[1], *ops.grouped_swiglu_combine_bwd(dout, x, weights, w, w, w2, gate, up, plan)[1:4]]
+
+    clean = grads(x, dy)
+    start = 0
+    for bad, n in enumerate(counts):
+        if n:
+            xb, dyb = x.clone(), dy.clone()
+            xb[start:start + n], dyb[start:start + n] = float("nan"), float("inf")
+            for a, b in zip(clean, grads(xb, dyb)):
+                for e in range(El):
+                    assert torch.equal(a[e], b[e]) if e != bad else not bool(b[e].isfinite().any())
+        start += n

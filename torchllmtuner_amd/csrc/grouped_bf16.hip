@@ -40,14 +40,17 @@
 //   * hardware bf16 conversion and transcendental-unit sigmoid in the epilogues (they
 //     were VALU bound).
 //
-// K loop of the weight gradients: one barrier per K step of 64.  Per quarter step a wave reads its fragments,
-// parks a quarter of the next step's operands (held in registers) in the other LDS
-// stage, refills those registers with the step after, and issues its MFMAs.  The
-// pipeline tail is peeled at compile time: every load of the steady state is
-// unconditional, so the compiler counts outstanding loads exactly instead of draining
-// the queue once per K step.
+// The weight gradients' loop is the same, with both operands' contraction strided: what a barrier frees is the first or the last 32 k of both.
+// Rows past the segment lie past the end of the buffer that a request names, which makes them zeros.  A gathered operand's row indices are requested a K step before
+// its rows, into the wave's own LDS.  The contraction is the rows, two to eight K steps of an expert where the load is balanced, so requests run over tile ends into
+// as many as two tiles, and a tile's stores may still be under way in the next one's first step: their number is known, and waits count them.
+// What bounds them: 128 experts of 2048 x 768, 512 rows each: 248 / 222 us, 241 / 218, 241 / 217 (0.93 PFLOP/s; operands parked through registers / straight into
+// LDS), a tile 18 us, 13 of them K steps; 16384 tokens of a skewed router 477 / 437, 468 / 425; 32 of 7168 x 2048, 128 rows each 231 / 209, 228 / 206 (the
+// results, written at 4.6 TB/s); one dense segment of 4096 rows 116 / 102, 120 / 105; 12 or fewer rows an expert of 2048 x 768 75 / 77 (written at 5.2 TB/s).
+// Beside the MFMAs the loop has 48 reads and 140 other instructions a wave and K step, and they count: with addresses formed from scratch at each request (100
+// more) it took 8-10 % longer, with the row indices in scalar registers 3 %.
 //
-// MFMA of the row-tiled kernels: v_mfma_f32_16x16x32_bf16.  Per lane 8 bf16 of each operand (row lane%16,
+// MFMA of both: v_mfma_f32_16x16x32_bf16.  Per lane 8 bf16 of each operand (row lane%16,
 // k = 8*(lane/16)..+7), 4 fp32 of the result (column lane%16, rows 4*(lane/16) + i).
 // With random operand bits this shape sustains about 14 % more than 32x32x16 on this
 // card (2.17 against 1.90 PFLOP/s register-resident, +7 % in a whole K loop).  The weight tile is passed as the FIRST operand
@@ -97,6 +100,17 @@ __device__ __forceinline__ void lds_load16(uint64_t base, uint32_t voff, uint32_
   else
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                  ::"s"(lds), "v"(voff), "s"(lds_rsrc(base)), "s"(soff) : "memory");
+}
+// the same from a buffer of `bytes` bytes; zeros for what lies past its end
+__device__ __forceinline__ void lds_load16_within(uint64_t base, uint32_t bytes, uint32_t voff, uint32_t lds) {
+  const u32x4 rsrc = {static_cast<uint32_t>(base), static_cast<uint32_t>(base >> 32), bytes, 0x00020000u};
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+               ::"s"(lds), "v"(voff), "s"(rsrc) : "memory");
+}
+__device__ __forceinline__ void lds_load4_within(uint64_t base, uint32_t bytes, uint32_t voff, uint32_t lds) {
+  const u32x4 rsrc = {static_cast<uint32_t>(base), static_cast<uint32_t>(base >> 32), bytes, 0x00020000u};
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dword %1, %2, 0 offen lds"
+               ::"s"(lds), "v"(voff), "s"(rsrc) : "memory");
 }
 __device__ __forceinline__ void lds_load4(uint64_t base, uint32_t voff, uint32_t soff, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dword %1, %2, %3 offen lds"
@@ -731,7 +745,6 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
 // ---- weight gradients: C[e](M,N) = sum_{r in segment e} A[r][m] * B[r][n] ----------
 // 256 x 256 output tile, 8 waves as 4 (m) x 2 (n), each wave 64 x 128; both operands KS.
 constexpr int WBM = 256, WBN = 256;
-constexpr int W_STAGE = (WBM + WBN) * BK;  // 64 KiB
 
 struct WgradArgs {
   const uint16_t* a;  // (rows, M) row-major
@@ -752,9 +765,16 @@ struct WgradArgs {
 
 template <bool GATHER, bool GATHER_A = false>
 __global__ __launch_bounds__(NT, 2) void wgrad_kernel(WgradArgs p) {
+  constexpr int PITCH = 512;  // bytes of an operand's k row in LDS
+  constexpr bool INDEXED = GATHER || GATHER_A;
+  constexpr int VM = 8;       // requests younger than those a barrier of the loop waits for: two groups of four
+  constexpr int VMY = VM + INDEXED;  // ... and, at the second barrier, the row indices
+  constexpr int STORES = 16;  // of a tile's results, a lane
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 128;
+  const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_cptr)smem));
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = wave >> 1, wn = wave & 1;
   const int M = p.M, N = p.N;
   const int per_e = p.m_tiles * p.n_tiles;
   if (blockIdx.y) {
@@ -762,28 +782,12 @@ __global__ __launch_bounds__(NT, 2) void wgrad_kernel(WgradArgs p) {
     p.c = p.c1;
   }
 
-  // KS tiles of 256 columns = 32 chunks per k row: k = (tid>>5) + 16*i, chunk tid&31
-  u32x4 ra[4], rb[4];
-  const int ks_k = tid >> 5, ks_chunk = tid & 31;
-  int lds_off[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int k = ks_k + 16 * i;
-    lds_off[i] = k * 256 + ((ks_chunk ^ ks_key(k)) << 3);
-  }
-  const u32x4 zero = {0, 0, 0, 0};
-
   // Persistent workgroups.  A tile's cost is its expert's row count (the contraction
   // length), which a skewed router spreads over two orders of magnitude, so tiles are not
   // walked in expert order: experts are taken by descending row count (the plan's order,
   // second half of seg_counts) and dealt to the eight XCDs a round at a time, and the CUs of an
   // XCD deal that XCD's tiles round-robin among themselves -- the longest contractions
-  // start first and in parallel, and an expert's tiles still share one L2.  The K extent
-  // is short for a balanced router (a handful of 64-row steps), so what surrounds the K
-  // loop matters too: the first operands of the next tile are requested before the
-  // epilogue of the current one and land while it runs, segment bounds are looked up
-  // ahead, and with a gathered B operand the row indices of a K step are fetched one step
-  // before its data.
+  // start first and in parallel, and an expert's tiles still share one L2.
   const int El = p.El;
   const int xcd = blockIdx.x & 7;
   // The plan arrays are read-only here and every lookup is workgroup-uniform: read through
@@ -805,236 +809,307 @@ __global__ __launch_bounds__(NT, 2) void wgrad_kernel(WgradArgs p) {
   int within = blockIdx.x >> 3;
   if (within >= n_x) return;
   auto exists = [&](int w) { return w < n_x; };
-  // this XCD's w-th tile (w clamped to an existing tile) as rank * per_e + tile in expert
-  auto flat_of = [&](int w) -> int {
+  struct Tile {
+    int e, seg0, cnt, m0, n0;
+  };
+  // this XCD's w-th tile (w clamped to an existing tile): the rank of its expert, and its tile in the expert
+  auto place = [&](int w, int& rank) -> int {
     w = exists(w) ? w : within;
-    if (w >= n_full) return 8 * n_full + p0 + (w - n_full);
-    const int round = w / per_e;
-    return (round * 8 + ((round & 1) ? 7 - xcd : xcd)) * per_e + (w - round * per_e);
+    const bool full = w < n_full;
+    const int u = full ? w : p0 + (w - n_full), r = u / per_e;
+    rank = full ? r * 8 + ((r & 1) ? 7 - xcd : xcd) : (El & ~7) + r;
+    return u - r * per_e;
   };
   // (clamped: an order array the caller never filled must not turn into a wild address)
-  auto expert_at = [&](int flat) -> int { return min(max(order[flat / per_e], 0), El - 1); };
-  auto expert_of = [&](int w) -> int { return expert_at(flat_of(w)); };
-  auto tile_in_expert = [&](int w) -> int { return flat_of(w) % per_e; };
-
-  // state of the tile whose operands are being fetched
-  int e = expert_of(within);
+  auto expert_at = [&](int w) -> int {
+    int rank;
+    place(w, rank);
+    return min(max(order[rank], 0), El - 1);
+  };
   // a last tile that would overhang starts early instead (M, N >= 256) and recomputes a few
   // rows or columns of its neighbour -- the same values -- so every tile is whole
-  int m0 = min((tile_in_expert(within) / p.n_tiles) * WBM, M - WBM);
-  int n0 = min((tile_in_expert(within) % p.n_tiles) * WBN, N - WBN);
-  int seg0 = seg_offsets[e], cnt = seg_counts[e];
-  const uint16_t* a_base;
-  const uint16_t* b_base;
-  auto set_bases = [&]() {
-    a_base = p.a + (GATHER_A ? 0 : static_cast<int64_t>(seg0) * M) + min(m0 + ks_chunk * 8, M - 8);
-    b_base = p.b + (GATHER ? 0 : static_cast<int64_t>(seg0) * N) + min(n0 + ks_chunk * 8, N - 8);
+  auto tile_at = [&](int w, int e) -> Tile {
+    int rank;
+    const int t = place(w, rank), m = t / p.n_tiles;
+    return {e, seg_offsets[e], seg_counts[e], min(m * WBM, M - WBM), min((t - m * p.n_tiles) * WBN, N - WBN)};
   };
-  // B row of this thread's chunk i in K step `step` of segment (s0, c): its own row, or
-  // (gather) the source row from the index array.  Needs c > 0.
-  // (a gathered index is returned as loaded and clamped to [0, src_rows) only where it is used,
-  // a K step later: clamping here would make the wave wait for the index right away, and with it
-  // -- the load counter retires in order -- for every operand load requested before it)
-  auto row_index = [&](int s0, int c, int step, int i) -> int {
-    const int k = min(step * BK + ks_k + 16 * i, c - 1);
-    return GATHER ? p.b_src[s0 + k] : k;
+  // (field by field: a choice between the structures would leave them in memory)
+  auto either = [](bool c, Tile a, Tile b) -> Tile {
+    return {c ? a.e : b.e, c ? a.seg0 : b.seg0, c ? a.cnt : b.cnt, c ? a.m0 : b.m0, c ? a.n0 : b.n0};
   };
-  // the same for the A row (its own row unless A is gathered too)
-  auto a_row_index = [&](int s0, int c, int step, int i) -> int {
-    const int k = min(step * BK + ks_k + 16 * i, c - 1);
-    return GATHER_A ? p.a_src[s0 + k] : k;
-  };
-  auto clamp_src = [&](int r) -> int { return min(max(r, 0), p.src_rows - 1); };
-  // Loads of one K step, unconditional: rows past the segment re-read its last row and
-  // the A side is zeroed when it is parked, so the products vanish.  Needs cnt > 0.
-  auto load_ab = [&](int step, int i, int brow, int arow_g) {
-    const int k = GATHER_A ? clamp_src(arow_g) : min(step * BK + ks_k + 16 * i, cnt - 1);
-    const int kb = GATHER ? clamp_src(brow) : brow;
-    ra[i] = *reinterpret_cast<const u32x4*>(a_base + static_cast<int64_t>(k) * M);
-    rb[i] = *reinterpret_cast<const u32x4*>(b_base + static_cast<int64_t>(kb) * N);
-  };
-  auto park = [&](int step, int i, uint16_t* An, uint16_t* Bn, int count) {
-    const bool live = step * BK + ks_k + 16 * i < count;
-    *reinterpret_cast<u32x4*>(An + lds_off[i]) = live ? ra[i] : zero;
-    *reinterpret_cast<u32x4*>(Bn + lds_off[i]) = rb[i];
-  };
-  int bidx[4];  // B rows of the K step that is requested next
-  int aidx[4];  // A rows likewise (used when A is gathered)
-  set_bases();
-  if (cnt > 0) {
-    // (requests always go out as operands, then the next index, chunk after chunk: the K loop's
-    // waits count the requests that follow the one they need along every way into the loop)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      __builtin_amdgcn_sched_barrier(0);
-      load_ab(0, i, row_index(seg0, cnt, 0, i), a_row_index(seg0, cnt, 0, i));
-      bidx[i] = row_index(seg0, cnt, 1, i);
-      aidx[i] = a_row_index(seg0, cnt, 1, i);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  // expert and segment of the next tile, expert of the one after it (its segment is
-  // looked up inside the loop, the expert after that too)
-  int ne = expert_of(within + stride);
-  int nseg0 = seg_offsets[ne], ncnt = seg_counts[ne];
-  int e2 = expert_of(within + 2 * stride);
+  Tile t0 = tile_at(within, expert_at(within));
 
+  // ---- operand requests: two k rows of 256 columns a wave and instruction, straight into LDS ----
+  const int krow = 2 * wave + (lane >> 5);
+  const uint32_t cc16 = static_cast<uint32_t>((lane & 31) ^ ks_key16(krow)) * 16u;
+  const uint32_t voffA = GATHER_A ? cc16 : static_cast<uint32_t>(krow * M) * 2u + cc16;
+  const uint32_t voffB = GATHER ? cc16 : static_cast<uint32_t>(krow * N) * 2u + cc16;
+  const uint32_t wdst = lds0 + wave * 1024u;
+  uint32_t fst = 0;  // LDS stage (byte offset) the requests go to
+  // State of the K step whose operands are being requested, kept up by additions (scalar arithmetic between the MFMAs is what this loop has least room
+  // for): how many tiles ahead, rows of the segment from this step on, operand addresses and bytes to the segment's end
+  int ahead = 0, left;
+  uint64_t gA, gB;
+  uint32_t bytesA, bytesB;
+  [[maybe_unused]] uint32_t voffG[4];  // where the lane's pieces of the gathered operand lie
+  // The same for its row indices, which are requested a K step earlier still: all 64 of a step into one of four 256-byte places of the wave's own LDS, which its results
+  // go through too: what has been requested is in registers by then
+  [[maybe_unused]] int i_ahead = 0, i_left = 0;
+  [[maybe_unused]] uint64_t ix = 0;
+  [[maybe_unused]] uint32_t i_to = 0, i_from = 0;
+  const uint32_t epi = 2 * STAGE_BYTES + wave * 4096u;
+  const uint32_t ldA = static_cast<uint32_t>(M) * 2u, ldB = static_cast<uint32_t>(N) * 2u;  // bytes
+  // bytes of the gathered operand; an offset past them for rows past the segment (which a matrix of almost 4 GiB does not leave: its first row then)
+  const uint64_t src_bytes = static_cast<uint64_t>(p.src_rows) * (GATHER ? ldB : ldA);
+  const uint32_t nowhere = src_bytes > 0xfffffe00u ? 0u : 0xfffffe00u;
+  int fm0, fn0;
+  auto set_bytes = [&]() {
+    // (a step of 64 rows ends before the next row's first column)
+    const uint32_t rows = static_cast<uint32_t>(min(max(left, 0), BK));
+    if constexpr (!GATHER_A) bytesA = rows ? rows * ldA - fm0 * 2u : 0u;
+    if constexpr (!GATHER) bytesB = rows ? rows * ldB - fn0 * 2u : 0u;
+  };
+  auto request_indices = [&]() {
+    if constexpr (INDEXED) {
+      lds_load4_within(ix, static_cast<uint32_t>(max(i_left, 0)) * 4u, opaque(lane) * 4u, lds0 + epi + i_to);
+      i_to = (i_to + 256) & 1023;
+    }
+  };
+  auto indices_of = [&](Tile t) {
+    if constexpr (INDEXED) {
+      i_left = t.cnt;
+      ix = reinterpret_cast<uint64_t>((GATHER ? p.b_src : p.a_src) + t.seg0);
+    }
+  };
+  auto to_tile = [&](Tile t) {
+    left = t.cnt;
+    fm0 = t.m0;
+    fn0 = t.n0;
+    gA = reinterpret_cast<uint64_t>(p.a + (GATHER_A ? 0 : static_cast<int64_t>(t.seg0) * M) + t.m0);
+    gB = reinterpret_cast<uint64_t>(p.b + (GATHER ? 0 : static_cast<int64_t>(t.seg0) * N) + t.n0);
+    if constexpr (GATHER_A) bytesA = static_cast<uint32_t>(src_bytes - t.m0 * 2u);
+    if constexpr (GATHER) bytesB = static_cast<uint32_t>(src_bytes - t.n0 * 2u);
+  };
+  auto read_indices = [&]() {
+    if constexpr (INDEXED) {
+      const uint32_t at = lds0 + epi + i_from + (2 * wave + (opaque(lane) >> 5)) * 4u;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) voffG[i] = lds_read_i32(at + 64 * i);
+      i_from = (i_from + 256) & 1023;
+    }
+  };
+  auto take_row = [&](int i) {
+    if constexpr (INDEXED) {
+      const int r = min(max(static_cast<int>(voffG[i]), 0), p.src_rows - 1);
+      voffG[i] = static_cast<uint32_t>(r) * (GATHER ? ldB : ldA) + cc16;
+      if (left < BK && 2 * wave + (opaque(lane) >> 5) + 16 * i >= left) voffG[i] = nowhere + cc16;
+    }
+  };
+  auto req = [&](bool is_a, int i) {
+    const uint32_t dst = fst + wdst + (is_a ? 0u : A_BYTES) + i * 8192u;
+    const uint32_t voff = (is_a ? GATHER_A : GATHER) ? voffG[i] : opaque(is_a ? voffA : voffB) + 16u * i * (is_a ? ldA : ldB);
+    lds_load16_within(is_a ? gA : gB, is_a ? bytesA : bytesB, voff, dst);
+  };
+  // pieces 0 and 1 of both operands hold a K step's first 32 k, 2 and 3 the others
+  auto req_q = [&](int half, int j) { req(j < 2, 2 * half + (j & 1)); };
+  // The tiles after the first, the expert of the one after those.  Requests run two K steps ahead, their row indices three: of as many tiles
+  // where each has one K step.  (Looked up once the first tile's operands are on their way, where it has enough steps.)
+  Tile t1 = t0, t2 = t0, t3 = t0;
+  auto next_step = [&]() {
+    fst ^= STAGE_BYTES;
+    left -= BK;
+    if (left > 0) {
+      if constexpr (!GATHER_A) gA += BK * static_cast<uint64_t>(ldA);
+      if constexpr (!GATHER) gB += BK * static_cast<uint64_t>(ldB);
+    } else {
+      ++ahead;
+      to_tile(either(ahead == 1, t1, either(ahead == 2, t2, t3)));
+    }
+    set_bytes();
+  };
+  auto next_indices = [&]() {
+    if constexpr (INDEXED) {
+      i_left -= BK;
+      if (i_left > 0) {
+        ix += BK * 4;
+      } else {
+        ++i_ahead;
+        indices_of(either(i_ahead == 1, t1, either(i_ahead == 2, t2, t3)));
+      }
+      request_indices();
+    }
+  };
+  auto req_all = [&]() {
+    if constexpr (INDEXED) {
+      read_indices();
+#pragma unroll
+      for (int i = 0; i < 4; ++i) take_row(i);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) req_q(j >> 2, j & 3);
+    next_step();
+  };
+  to_tile(t0);
+  indices_of(t0);
+  set_bytes();
+  request_indices();
+  const bool early = t0.cnt > 2 * BK;
+  if (early) {
+    next_indices();
+    if constexpr (INDEXED) lds_wait<0>();
+    req_all();
+    req_all();
+  }
+  t1 = tile_at(within + stride, expert_at(within + stride));
+  t2 = tile_at(within + 2 * stride, expert_at(within + 2 * stride));
+  t3 = tile_at(within + 3 * stride, expert_at(within + 3 * stride));
+  int e4 = expert_at(within + 4 * stride);
+  if (!early) {
+    next_indices();
+    if constexpr (INDEXED) lds_wait<0>();
+    req_all();
+    req_all();
+  }
+  next_indices();
+
+  // ---- fragment reads ------------------------------------------------------------------------
+  const int l15 = lane & 15, l4 = lane >> 4;
+  uint32_t ra[4], rb[4];
+  {
+    const int k = 8 * l4 + (l15 >> 2);
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      const int x = b * 2 + ((l15 & 3) >> 1);
+      ra[b] = lds0 + k * PITCH + ((wr * 8 + x) ^ ks_key16(k)) * 16u + (l15 & 1) * 8u;
+      rb[b] = lds0 + A_BYTES + k * PITCH + ((wn * 16 + x) ^ ks_key16(k)) * 16u + (l15 & 1) * 8u;
+    }
+  }
+  auto rd_a = [&](bf16x8 (&fr)[4], int kk, int mi) { fr[mi] = lds_read_tr<PITCH>(ra[mi] + kk * 32u * PITCH); };
+  auto rd_b = [&](bf16x8 (&fr)[4], int kk, int hb, int b) { fr[b] = lds_read_tr<PITCH>((rb[b] ^ (hb * 128u)) + kk * 32u * PITCH); };
+
+  lds_sync<INDEXED ? 0 : 4>();
+  read_indices();
+  bool first = true;
   for (;;) {
     const bool more = exists(within + stride);
-    const int nw = within + stride;
-    // two tiles ahead: segment bounds, used one tile later; three ahead: the expert
-    const int n2seg0 = seg_offsets[e2], n2cnt = seg_counts[e2];
-    const int e3 = expert_of(within + 3 * stride);
-    // next tile: B rows of its first K step (its bounds were looked up a tile ago)
-    int nidx[4], nidx_a[4];
-    if (ncnt > 0) {
+    f32x4 acc[4][8];
+    // a quarter of a K step's MFMAs, requests and fragment reads between its blocks, as in the row-tiled kernel
+    // (ZERO: to nothing, not to the sum so far -- 128 registers set to zero are half a microsecond a tile)
+    auto mm = [&](auto zero_t, const bf16x8 (&af)[4], const bf16x8 (&bf)[4], int hb, auto between) {
+      constexpr bool ZERO = decltype(zero_t)::value;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        nidx[i] = row_index(nseg0, ncnt, 0, i);
-        nidx_a[i] = a_row_index(nseg0, ncnt, 0, i);
-      }
-    }
-    const int c_e = e, c_m0 = m0, c_n0 = n0, c_cnt = cnt, c_seg0 = seg0;
-    const int ksteps = (cnt + BK - 1) / BK;
-
-    // 64 x 128 per wave as 2 x 4 tiles of v_mfma_f32_32x32x16_bf16: with both operands read
-    // through LDS transposes the 16x16x32 shape of the row-tiled kernels measured slower here
-    f32x16 acc[2][4];
-#pragma unroll
-    for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-      for (int nj = 0; nj < 4; ++nj)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[mi][nj][i] = 0.0f;
-
-    if (ksteps > 0) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) park(0, i, smem, smem + WBM * BK, c_cnt);
-      if (ksteps > 1) {
-        // in the order of a K step of the loop below (operands, then the next index, chunk after
-        // chunk, and kept in that order): the loop's waits count the requests that follow the one
-        // they need, on both ways into the loop, so both ways must issue them alike
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          __builtin_amdgcn_sched_barrier(0);
-          load_ab(1, i, bidx[i], aidx[i]);
-          bidx[i] = row_index(c_seg0, c_cnt, 2, i);
-          aidx[i] = a_row_index(c_seg0, c_cnt, 2, i);
-        }
+      for (int mi = 0; mi < 4; ++mi) {
         __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    __syncthreads();
-
-    // One K step: a quarter of the staging rides along with each quarter of the MFMAs.
-    // The flags are compile-time so that the loads of the steady state are unconditional
-    // and the compiler counts outstanding loads exactly.
-    auto kstep = [&](int ks, auto has_next_t, auto has_next2_t) {
-      constexpr bool has_next = decltype(has_next_t)::value;
-      constexpr bool has_next2 = decltype(has_next2_t)::value;
-      const uint16_t* As = smem + (ks & 1) * W_STAGE;
-      const uint16_t* Bs = As + WBM * BK;
-      uint16_t* An = smem + ((ks + 1) & 1) * W_STAGE;
-      uint16_t* Bn = An + WBM * BK;
-#pragma unroll
-      for (int kk = 0; kk < BK / 16; ++kk) {
-        // the last K step of a segment is usually ragged: its 16-row slices past the last real
-        // row hold zeros and are skipped (workgroup-uniform; only this instantiation branches)
-        if constexpr (!has_next) {
-          if (ks * BK + kk * 16 >= c_cnt) continue;
-        }
-        bf16x8 af[2], bf[4];
-#pragma unroll
-        for (int mi = 0; mi < 2; ++mi) af[mi] = frag_ks<256>(As, wm + mi * 32, kk, lane);
-#pragma unroll
-        for (int nj = 0; nj < 4; ++nj) bf[nj] = frag_ks<256>(Bs, wn + nj * 32, kk, lane);
-        if constexpr (has_next) park(ks + 1, kk, An, Bn, c_cnt);
-        // Nothing is moved across this point: the requests below stay in their quarter of the K
-        // step (left alone, the compiler gathers all of a step's global loads at its end, where
-        // the data they fetch is parked a moment later instead of a whole step later, and the
-        // wave waits out the memory latency once per K step), and an index is clamped a whole
-        // step after it was requested.  What lies between two such points -- this quarter's
-        // requests and MFMAs, the next quarter's fragment reads and its park -- is still
-        // interleaved freely.
+        between(mi);
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (has_next2) {
-          load_ab(ks + 2, kk, bidx[kk], aidx[kk]);
-          bidx[kk] = row_index(c_seg0, c_cnt, ks + 3, kk);
-          aidx[kk] = a_row_index(c_seg0, c_cnt, ks + 3, kk);
-        }
 #pragma unroll
-        for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-          for (int nj = 0; nj < 4; ++nj)
-            acc[mi][nj] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf[nj], af[mi], acc[mi][nj], 0, 0, 0);
+        for (int b = 0; b < 4; ++b)
+          acc[mi][hb * 4 + b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[b], af[mi], ZERO ? f32x4{0, 0, 0, 0} : acc[mi][hb * 4 + b], 0, 0, 0);
       }
-      __syncthreads();
+      __builtin_amdgcn_sched_barrier(0);
     };
-    using T_ = std::true_type;
-    using F_ = std::false_type;
-    int ks = 0;
-    for (; ks + 2 < ksteps; ++ks) kstep(ks, T_{}, T_{});
-    if (ks + 1 < ksteps) { kstep(ks, T_{}, F_{}); ++ks; }
-    if (ks < ksteps) kstep(ks, F_{}, F_{});
-
-    // switch the fetch state to the next tile and request its first K step
-    if (more) {
-      e = ne;
-      const int nt = tile_in_expert(nw);
-      m0 = min((nt / p.n_tiles) * WBM, M - WBM);
-      n0 = min((nt % p.n_tiles) * WBN, N - WBN);
-      seg0 = nseg0;
-      cnt = ncnt;
-      set_bases();
-      if (cnt > 0) {
+    bf16x8 a0[4], a1[4], b0[4], b1[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          __builtin_amdgcn_sched_barrier(0);
-          load_ab(0, i, nidx[i], nidx_a[i]);
-          bidx[i] = row_index(seg0, cnt, 1, i);
-          aidx[i] = a_row_index(seg0, cnt, 1, i);
+    for (int i = 0; i < 4; ++i) {
+      rd_a(a0, 0, i);
+      rd_b(b0, 0, 0, i);
+    }
+    const int ksteps = max((t0.cnt + BK - 1) / BK, 1);  // (no rows: one step of zeros)
+    auto kstep = [&](int ks, auto first_t) {
+      constexpr bool FIRST = decltype(first_t)::value;
+      using F_ = std::false_type;
+      mm(first_t, a0, b0, 0, [&](int q) {
+        rd_b(b1, 0, 1, q);
+        if (q == 3 && INDEXED && !FIRST) {
+          lds_wait<VM>();
+          read_indices();
         }
-        __builtin_amdgcn_sched_barrier(0);
+      });
+      // (the last tile's stores may still be under way in the first step and, up to its first barrier, the second)
+      if constexpr (FIRST) {
+        if (!first) lds_wait<VM + STORES>();
+      } else {
+        if (INDEXED || ks > 1 || first) lds_wait<VM>();
+        else lds_wait<VM + STORES>();
       }
-    }
+      lds_sync<63>();
+      mm(first_t, a0, b1, 1, [&](int q) {
+        rd_a(a1, 1, q);
+        rd_b(b0, 1, 0, q);
+        if (q == 0) return;
+        take_row(q - 1);
+        if (q == 1) next_indices();
+        if (q == 3) take_row(3);
+        req_q(0, q - 1);
+      });
+      mm(F_{}, a1, b0, 0, [&](int q) {
+        rd_b(b1, 1, 1, q);
+        if (q == 0) req_q(0, 3);
+      });
+      if constexpr (!FIRST) lds_wait<VMY>();
+      else if (!first) lds_wait<VM + STORES>();
+      lds_sync<63>();
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        ra[b] ^= STAGE_BYTES;
+        rb[b] ^= STAGE_BYTES;
+      }
+      mm(F_{}, a1, b1, 1, [&](int q) {
+        if (q == 0) return;
+        rd_a(a0, 0, q - 1);
+        rd_b(b0, 0, 0, q - 1);
+        req_q(1, q - 1);
+        if (q < 3) return;
+        rd_a(a0, 0, 3);
+        rd_b(b0, 0, 0, 3);
+        req_q(1, 3);
+        next_step();
+      });
+    };
+    kstep(0, std::true_type{});
+    for (int ks = 1; ks < ksteps; ++ks) kstep(ks, std::false_type{});
 
-    using S = WaveStage<128>;
-    uint16_t* st = smem + wave * S::ELEMS;
-#pragma unroll
-    for (int mi = 0; mi < 2; ++mi)
-#pragma unroll
-      for (int nj = 0; nj < 4; ++nj)
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          S::put4(st, mi, nj * 32, lane, q, acc[mi][nj][q * 4], acc[mi][nj][q * 4 + 1],
-                  acc[mi][nj][q * 4 + 2], acc[mi][nj][q * 4 + 3]);
-    __builtin_amdgcn_s_waitcnt(0xc07f);
-    __builtin_amdgcn_wave_barrier();
-    uint16_t* C = p.c + static_cast<int64_t>(c_e) * M * N;
-#pragma unroll 4
-    for (int it = 0; it < 16; ++it) {
-      const int idx = it * 64 + lane;
-      const int m = c_m0 + wm + (idx >> 4), n = c_n0 + wn + (idx & 15) * 8;
-      // whole tiles only: the stores are unconditional, so the compiler knows how many follow
-      // the operand loads requested above and the next tile's wait for those loads does not
-      // also wait for these stores (one counter serves both)
-      // (non-temporal: a weight gradient is several times the size of L2 and is read next by the
-      // optimizer; written through the cache as ordinary stores, an expert's 30-60 MB of results push
-      // its own operands out of L2 between two of its tiles -- with few rows per expert, where the
-      // product is bound by these writes, the gathered rows were fetched from memory several times over)
-      __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(st + (idx >> 4) * S::PITCH + (idx & 15) * 8),
-                                  reinterpret_cast<u32x4*>(C + static_cast<int64_t>(m) * N + n));
+    // the tile's results, 16 rows at a time through the wave's own LDS
+    const int el = opaque(lane);
+    char* own = reinterpret_cast<char*>(smem) + epi;
+    uint16_t* C = p.c + static_cast<int64_t>(t0.e) * M * N + static_cast<int64_t>(t0.m0 + wr * 64) * N + t0.n0 + wn * 128;
+    if constexpr (INDEXED) {
+      lds_wait<VM>();
+      read_indices();
     }
-    // staging regions are free again before the next tile's operands are parked; only
-    // the LDS traffic is waited for, the tile's stores keep draining
-    phase_barrier();
+#pragma unroll
+    for (int mi = 0; mi < 4; ++mi) {
+#pragma unroll
+      for (int nj = 0; nj < 8; ++nj) {
+        const int m = el & 15, c = nj * 2 + (el >> 5);
+        const u32x2 pk = {pack2(acc[mi][nj][0], acc[mi][nj][1]), pack2(acc[mi][nj][2], acc[mi][nj][3])};
+        *reinterpret_cast<u32x2*>(own + m * 256 + ((c ^ m) * 16) + ((el >> 4) & 1) * 8) = pk;
+      }
+      wave_lds_sync();
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int m = u * 4 + (el >> 4), c = el & 15;
+        // (non-temporal: a weight gradient is several times the size of L2 and is read next by the
+        // optimizer; written through the cache as ordinary stores, an expert's 30-60 MB of results push
+        // its own operands out of L2 between two of its tiles -- with few rows per expert, where the
+        // product is bound by these writes, the gathered rows were fetched from memory several times over)
+        __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(own + m * 256 + ((c ^ m) * 16)),
+                                    reinterpret_cast<u32x4*>(C + static_cast<int64_t>(mi * 16 + m) * N + c * 8));
+      }
+      wave_lds_sync();
+    }
     if (!more) break;
+    first = false;
     within += stride;
-    ne = e2;
-    e2 = e3;
-    nseg0 = n2seg0;
-    ncnt = n2cnt;
+    t0 = t1;
+    t1 = t2;
+    t2 = t3;
+    t3 = tile_at(within + 3 * stride, e4);
+    e4 = expert_at(within + 4 * stride);
+    --ahead;
+    --i_ahead;
   }
+  lds_wait<0>();
 }
 
 template <typename K>
@@ -1072,7 +1147,6 @@ static unsigned resident_blocks() {
   return n;
 }
 
-constexpr int W_LDS_BYTES = 8 * 64 * 136 * 2;  // 139264: the 8 epilogue regions (> 2 stages = 131072)
 
 // Whether a product of El experts and n 256-column tiles runs on 128-column ones instead: twice the work items, each with the
 // whole contraction.  Where experts of equal load would occupy at most half the CUs (three eighths where the tiles are
@@ -1263,9 +1337,9 @@ int bf16_grouped_bwd(const void* dy, const void* rows, const int32_t* token_of_r
   }
   static PerDeviceOnce wconfigured;
   if (wconfigured.needed()) {
-    if (int rc = set_lds(wgrad_kernel<false>, W_LDS_BYTES)) return rc;
-    if (int rc = set_lds(wgrad_kernel<true>, W_LDS_BYTES)) return rc;
-    if (int rc = set_lds(wgrad_kernel<false, true>, W_LDS_BYTES)) return rc;
+    if (int rc = set_lds(wgrad_kernel<false>, R_LDS_BYTES)) return rc;
+    if (int rc = set_lds(wgrad_kernel<true>, R_LDS_BYTES)) return rc;
+    if (int rc = set_lds(wgrad_kernel<false, true>, R_LDS_BYTES)) return rc;
     wconfigured.done();
   }
   auto wgrad = [&](const void* A, const void* B, const int32_t* b_src, void* C, int64_t M, int64_t N, const char* what,
@@ -1279,11 +1353,11 @@ int bf16_grouped_bwd(const void* dy, const void* rows, const int32_t* token_of_r
     w.a1 = (const uint16_t*)A1; w.c1 = (uint16_t*)C1;
     const dim3 grid(std::min(round8(w.total), resident_blocks()), C1 ? 2 : 1);
     if (a_src)
-      hipLaunchKernelGGL((wgrad_kernel<false, true>), grid, dim3(NT), W_LDS_BYTES, s, w);
+      hipLaunchKernelGGL((wgrad_kernel<false, true>), grid, dim3(NT), R_LDS_BYTES, s, w);
     else if (b_src)
-      hipLaunchKernelGGL(wgrad_kernel<true>, grid, dim3(NT), W_LDS_BYTES, s, w);
+      hipLaunchKernelGGL(wgrad_kernel<true>, grid, dim3(NT), R_LDS_BYTES, s, w);
     else
-      hipLaunchKernelGGL(wgrad_kernel<false>, grid, dim3(NT), W_LDS_BYTES, s, w);
+      hipLaunchKernelGGL(wgrad_kernel<false>, grid, dim3(NT), R_LDS_BYTES, s, w);
     return check_launch(what);
   };
   // folded combine: dW2 = (gathered output gradient)^T . (row_scale * h)
