@@ -101,3 +101,31 @@ def test_rows_of_other_experts_stay_out_of_a_weight_gradient(counts):
                 for e in range(El):
                     assert torch.equal(a[e], b[e]) if e != bad else not bool(b[e].isfinite().any())
         start += n
+
+
+# rows an expert on either side of the 16 a pass takes; contractions of six steps (one or two a wave) and seven; weights past the
+# memory-side cache, read with the non-temporal hint, of experts with a few rows (El = 40) and with one row tile (the last)
+@pytest.mark.parametrize("counts,D,Fd", [((16, 0, 17, 1, 33, 5, 15, 2), 384, 448), ((40, 3, 1, 0, 0, 9), 448, 384), ((1,), 384, 640), ((60,), 1024, 512),
+                                         ((3, 1, 20, 0) * 10, 2048, 768), ((200, 9, 40, 256) * 10, 2048, 768)])
+def test_few_rows_and_streamed_weights(counts, D, Fd):
+    from torchllmtuner_amd import ops
+
+    print(f"few rows {counts[:8]} D={D} F={Fd}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(D)
+    El, R = len(counts), sum(counts)
+    ids = torch.repeat_interleave(torch.arange(El), torch.tensor(counts))[torch.randperm(R, generator=torch.Generator().manual_seed(1))][:, None]
+    normal = lambda *s, std=1.0: (torch.randn(*s, generator=g, device=DEV) * std).bfloat16()
+    x, w1, w3, w2 = normal(R, D), normal(El, Fd, D, std=0.03), normal(El, Fd, D, std=0.03), normal(El, D, Fd, std=0.03)
+    plan = ops.permute_plan(ids.to(DEV), El)
+    y, gate, up, h = ops.grouped_swiglu_fwd(x, w1, w3, w2, plan, gather=True)
+    if R <= 8 * El or D % 2048:  # (beyond, rows of 4 KiB are summed in turned order where they are gathered)
+        copied = ops.grouped_swiglu_fwd(ops.permute_rows_fwd(x, plan), w1, w3, w2, plan)
+        assert all(torch.equal(a, b) for a, b in zip((y, gate, up, h), copied))
+    tok, start = plan.token_of_row.long(), 0
+    for e, n in enumerate(counts):
+        r = slice(start, start + n)
+        start += n
+        if n:
+            xe = x[tok[r]].float()
+            for got, want in ((gate[r], xe @ w1[e].float().T), (up[r], xe @ w3[e].float().T), (y[r], h[r].float() @ w2[e].float().T)):
+                assert row_errors(got, want) < 2.0 ** -8

@@ -83,6 +83,75 @@ __device__ __forceinline__ bf16x8 frag16_ks(const uint16_t* tile, int col, int k
   return __builtin_bit_cast(bf16x8, v);
 }
 
+// ---- requests straight into LDS ----------------------------------------------------------
+typedef const __attribute__((address_space(3))) char* lds_cptr;
+
+// Requests 16 (4) bytes a lane from base + voff + soff, straight into LDS: lane l's land at byte lds + 16 l (4 l).  Written
+// out because the compiler drains the whole load counter in front of every LDS read once it knows of such a request; waited for by lds_wait.
+// (base, soff and lds are wave-uniform; byte offsets up to 4 GiB; the wait states are for scalar registers that a vector instruction wrote just before)
+__device__ __forceinline__ u32x4 lds_rsrc(uint64_t base) {
+  return u32x4{static_cast<uint32_t>(base), static_cast<uint32_t>(base >> 32), 0xffffffffu, 0x00020000u};
+}
+template <bool STREAM = false>  // with the non-temporal hint
+__device__ __forceinline__ void lds_load16(uint64_t base, uint32_t voff, uint32_t soff, uint32_t lds) {
+  if constexpr (STREAM)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
+                 ::"s"(lds), "v"(voff), "s"(lds_rsrc(base)), "s"(soff) : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 ::"s"(lds), "v"(voff), "s"(lds_rsrc(base)), "s"(soff) : "memory");
+}
+// the same from a buffer of `bytes` bytes; zeros for what lies past its end
+__device__ __forceinline__ void lds_load16_within(uint64_t base, uint32_t bytes, uint32_t voff, uint32_t lds) {
+  const u32x4 rsrc = {static_cast<uint32_t>(base), static_cast<uint32_t>(base >> 32), bytes, 0x00020000u};
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+               ::"s"(lds), "v"(voff), "s"(rsrc) : "memory");
+}
+__device__ __forceinline__ void lds_load4_within(uint64_t base, uint32_t bytes, uint32_t voff, uint32_t lds) {
+  const u32x4 rsrc = {static_cast<uint32_t>(base), static_cast<uint32_t>(base >> 32), bytes, 0x00020000u};
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dword %1, %2, 0 offen lds"
+               ::"s"(lds), "v"(voff), "s"(rsrc) : "memory");
+}
+__device__ __forceinline__ void lds_load4(uint64_t base, uint32_t voff, uint32_t soff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dword %1, %2, %3 offen lds"
+               ::"s"(lds), "v"(voff), "s"(lds_rsrc(base)), "s"(soff) : "memory");
+}
+// at most N of the wave's requests and stores are still under way
+template <int N>
+__device__ __forceinline__ void lds_wait() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// the wave's LDS reads and writes are done, and at most N of its requests under way; then the workgroup's barrier
+template <int N>
+__device__ __forceinline__ void lds_sync() {
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (N < 63) lds_wait<N>();
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+// the same value, of which the compiler knows nothing: what is formed from it is formed there, not held in registers over a K loop
+__device__ __forceinline__ int opaque(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+// orders a wave's LDS writes and reads of its own region
+__device__ __forceinline__ void wave_lds_sync() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_wave_barrier();
+}
+__device__ __forceinline__ bf16x8 lds_read16(uint32_t at) {
+  return *(const __attribute__((address_space(3))) bf16x8*)(at);
+}
+__device__ __forceinline__ int lds_read_i32(uint32_t at) { return *(const __attribute__((address_space(3))) int*)(at); }
+// eight k of 16 columns from rows of PITCH bytes, k as the 16x16x32 MFMA wants them (frag16_ks)
+template <uint32_t PITCH>
+__device__ __forceinline__ bf16x8 lds_read_tr(uint32_t at) {
+  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(at));
+  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(at + 4 * PITCH));
+  const s16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  return __builtin_bit_cast(bf16x8, v);
+}
+
 // Workgroup barrier that waits for this wave's own LDS operations only: global loads and
 // stores stay in flight across it.
 __device__ __forceinline__ void phase_barrier() {

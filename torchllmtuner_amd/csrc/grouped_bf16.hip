@@ -80,77 +80,9 @@ __device__ __forceinline__ float fast_sigmoid(float x) {
 // int32 data that no kernel of this file writes (the plan's arrays), for uniform lookups
 typedef const int32_t __attribute__((address_space(4))) * const_i32;
 
-typedef const __attribute__((address_space(3))) char* lds_cptr;
-
 // LDS of the row-tiled kernels, in bytes: two stages of operands (A tile, B tile), 4 KiB a wave for its results
 constexpr uint32_t A_BYTES = 32768, STAGE_BYTES = 65536;
 constexpr int R_LDS_BYTES = 2 * STAGE_BYTES + 8 * 4096;
-
-// Requests 16 (4) bytes a lane from base + voff + soff, straight into LDS: lane l's land at byte lds + 16 l (4 l).  Written
-// out because the compiler drains the whole load counter in front of every LDS read once it knows of such a request; waited for by lds_wait.
-// (base, soff and lds are wave-uniform; byte offsets up to 4 GiB; the wait states are for scalar registers that a vector instruction wrote just before)
-__device__ __forceinline__ u32x4 lds_rsrc(uint64_t base) {
-  return u32x4{static_cast<uint32_t>(base), static_cast<uint32_t>(base >> 32), 0xffffffffu, 0x00020000u};
-}
-template <bool STREAM = false>  // with the non-temporal hint
-__device__ __forceinline__ void lds_load16(uint64_t base, uint32_t voff, uint32_t soff, uint32_t lds) {
-  if constexpr (STREAM)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
-                 ::"s"(lds), "v"(voff), "s"(lds_rsrc(base)), "s"(soff) : "memory");
-  else
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                 ::"s"(lds), "v"(voff), "s"(lds_rsrc(base)), "s"(soff) : "memory");
-}
-// the same from a buffer of `bytes` bytes; zeros for what lies past its end
-__device__ __forceinline__ void lds_load16_within(uint64_t base, uint32_t bytes, uint32_t voff, uint32_t lds) {
-  const u32x4 rsrc = {static_cast<uint32_t>(base), static_cast<uint32_t>(base >> 32), bytes, 0x00020000u};
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-               ::"s"(lds), "v"(voff), "s"(rsrc) : "memory");
-}
-__device__ __forceinline__ void lds_load4_within(uint64_t base, uint32_t bytes, uint32_t voff, uint32_t lds) {
-  const u32x4 rsrc = {static_cast<uint32_t>(base), static_cast<uint32_t>(base >> 32), bytes, 0x00020000u};
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dword %1, %2, 0 offen lds"
-               ::"s"(lds), "v"(voff), "s"(rsrc) : "memory");
-}
-__device__ __forceinline__ void lds_load4(uint64_t base, uint32_t voff, uint32_t soff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dword %1, %2, %3 offen lds"
-               ::"s"(lds), "v"(voff), "s"(lds_rsrc(base)), "s"(soff) : "memory");
-}
-// at most N of the wave's requests and stores are still under way
-template <int N>
-__device__ __forceinline__ void lds_wait() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-// the wave's LDS reads and writes are done, and at most N of its requests under way; then the workgroup's barrier
-template <int N>
-__device__ __forceinline__ void lds_sync() {
-  __builtin_amdgcn_sched_barrier(0);
-  if constexpr (N < 63) lds_wait<N>();
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
-// the same value, of which the compiler knows nothing: what is formed from it is formed there, not held in registers over a K loop
-__device__ __forceinline__ int opaque(int v) {
-  asm volatile("" : "+v"(v));
-  return v;
-}
-// orders a wave's LDS writes and reads of its own region
-__device__ __forceinline__ void wave_lds_sync() {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_wave_barrier();
-}
-__device__ __forceinline__ bf16x8 lds_read16(uint32_t at) {
-  return *(const __attribute__((address_space(3))) bf16x8*)(at);
-}
-__device__ __forceinline__ int lds_read_i32(uint32_t at) { return *(const __attribute__((address_space(3))) int*)(at); }
-// eight k of 16 columns from rows of PITCH bytes, k as the 16x16x32 MFMA wants them (frag16_ks)
-template <uint32_t PITCH>
-__device__ __forceinline__ bf16x8 lds_read_tr(uint32_t at) {
-  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(at));
-  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(at + 4 * PITCH));
-  const s16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-  return __builtin_bit_cast(bf16x8, v);
-}
 
 // RM_DLIN: the product of RM_DH (rows . w[e], the weight's contraction axis strided) with a plain epilogue:
 // the input gradient of one grouped linear map
@@ -1217,14 +1149,15 @@ static int launch_row(RowArgs& a, int64_t width, int64_t El, int64_t tile_capaci
 int few_rows_fwd(int stage, const void* a, const int32_t* a_src, int64_t a_rows, const void* b0, const void* b1,
                  void* gate, void* up, void* out, const int32_t* seg_offsets, const int32_t* seg_counts,
                  const int32_t* tile_expert, const int32_t* tile_row0, const int32_t* num_tiles, int64_t tiles, int64_t K,
-                 int64_t N, hipStream_t s);
+                 int64_t N, bool stream, hipStream_t s);
 
 // Up to eight rows per expert on average (rows and experts are what the host knows; one expert's share of
 // a wider router counts rows it does not get, which only errs towards the large tiles), or 64 rows in all.
 // A 16-row pass over an expert's weights costs the same for one row as for sixteen and a second pass
-// reads them again, from L2 at best: measured at 128 experts of 2048 x 768 the block takes 201 us against
-// 221 at 33 tokens (2 rows on average), 224 against 234 at 64, 238 against 240 at 128 (8), 251 against 241 at 160 (10), 275 against 242 at
-// 200; one dense segment of 7168 x 2048, 4 us of difference at 60 rows and -55 at 128.
+// reads them again, from L2 at best.  Block forward of 128 experts of 2048 x 768, these kernels / the row tiles, us: 16 tokens (1 row on average) 133 / 147, 33 183 /
+// 200, 64 202 / 210, 100 (6) 205 / 216, 128 (8) 216 / 215; 32 of 256 experts of 7168 x 2048, 16 tokens 186 / 230, 32 (counted as 8 rows, one of them here) 245 / 254.  One dense
+// segment of 7168 x 2048 alone, gate/up and down, 60 rows 41 + 16 / 79 + 26, 128 rows 79 + 25 / 93 + 30; but beside the routed experts of that share, whose CUs it takes
+// then, 128 rows 422 / 401.
 static bool few_rows(int64_t El, int64_t R, int64_t D, int64_t F) {
   return R <= std::max<int64_t>(8 * El, 64) && R * std::max(D, F) * 2 < (int64_t{1} << 32);
 }
@@ -1244,13 +1177,14 @@ int bf16_grouped_fwd(const void* rows, const int32_t* token_of_row, int64_t num_
                      int64_t F, int64_t row_capacity, int stages, hipStream_t s) {
   if (few_rows(El, row_capacity, D, F)) {
     const int64_t tiles = std::min(tile_capacity, std::min(El, row_capacity) + row_capacity / 256);
+    const bool stream = streamed(std::min(El, row_capacity), D, F);  // (of the experts that can have rows)
     if (stages & STAGE_GATEUP)
       if (int rc = few_rows_fwd(1, rows, token_of_row, num_tokens, w1, w3, gate, up, h, seg_offsets, seg_counts,
-                                tile_expert, tile_row0, num_tiles, tiles, D, F, s))
+                                tile_expert, tile_row0, num_tiles, tiles, D, F, stream, s))
         return rc;
     if (stages & STAGE_DOWN)
       return few_rows_fwd(2, h, nullptr, 0, w2, w2, nullptr, nullptr, y, seg_offsets, seg_counts, tile_expert, tile_row0,
-                          num_tiles, tiles, F, D, s);
+                          num_tiles, tiles, F, D, stream, s);
     return MI355_OK;
   }
   RowArgs a{};

@@ -5,16 +5,18 @@
 // stream the same weights through LDS in 1 MB work items, one workgroup per CU in lockstep: at one
 // token 48 items for 256 CUs, at 33 tokens 2.6 rounds of them.  Here a workgroup is four waves that
 // split the contraction of 16 output columns (of gate and up, or 32 of the down projection) of one
-// expert; every wave loads its weights straight into MFMA fragments, 16 KiB requested ahead, up
-// to sixteen waves to a CU, and the four partial tiles are added in wave order through LDS.
-//   Bound by HBM: 709 MB of gate and up weights (33 tokens of 128 experts, 2048 x 768) in 116 us, 6.1 TB/s
-// where a plain read in this pattern reaches 6.15 (145 us before); one token, 50 MB, 13 us (31 before).  The 354 MB of the down
-// projection, three contraction steps a wave, in 57 us: with four requested, the last twice, and the row counts looked up in front of
-// the weights it was 69.
+// expert, and the four partial tiles are added in wave order through LDS.
+//   A wave's weights go straight into LDS of its own, two contraction steps of 64 ahead (8 KiB, 128 KiB a CU), in whole 128-byte lines, eight rows an
+// instruction, and are read from there as MFMA fragments: no barrier stands in the loop.  Asked for as
+// fragments, 64 bytes of 16 rows an instruction with 16 KiB in registers ahead, a line is two requests, and the non-temporal hint makes the
+// second one go to memory again (5-11 % slower).  In lines the hint gains what it gains in the 256-row kernels (`streamed` there).
+//   Bound by HBM, us, fragments / lines / lines with the hint: gate and up of 33 tokens of 128 experts of 2048 x 768 (709 MB) 120 / 121 / 105 (6.8 TB/s), down
+// 57 / 60 / 54; 100 tokens 148 / 145 / 130, 68 / 70 / 65; 32 experts of 7168 x 2048, three rows each 330 / 304 / 271, 150 / 152 / 133; one
+// dense segment of it, where half the chip has to do, 16 rows 21 / 13, 8 / 7, 60 rows 77 / 41, 25 / 14; five tokens of the first, 36 / 35, 19 / 19.  One step ahead and twice the workgroups a
+// CU: the same within 3 %, but the dense segment 23 and 10; three ahead: 4-6 % slower.
 // Waves along the contraction rather than side by side: at one token 12-25 us less in all, at 33 the
 // same.  32 or 64 rows per wave instead of 16 need registers that the requests in flight want: slower.
-//   A contraction step is 64 wide: lane group g = lane / 16 holds k = 16 g .. 16 g + 15 of it (two
-// 16-byte loads, so that a row's 128 bytes are one request) for both operands alike.
+//   A contraction step is 64 wide: lane group g = lane / 16 holds k = 16 g .. 16 g + 15 of it for both operands alike.
 #include <algorithm>
 
 #include "bf16_tiles.h"
@@ -41,98 +43,115 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t few_rsrc(const void* base) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, -1, 0x00020000);
 }
 
+constexpr int kFewSteps = 2;                          // contraction steps of a wave in LDS
+constexpr uint32_t kFewStep = 6144;                   // bytes of one: 16 weight rows, 16 more, 16 activation rows, 128 each
+constexpr int kFewLds = 4 * kFewSteps * kFewStep;     // of a workgroup; the partial tiles (8 KiB) take their place
+
 // Column group cg of the product of expert e with the rows that where() names (the first and how many, at least one: looked up once
-// the first weights are on their way); a row is source(row) of a, or itself.  kPairs: 64-wide contraction steps requested together.
+// the first weights are on their way); a row is source(row) of a, or itself.
 struct FewRows {
   int row0, rows;
 };
-template <bool GATEUP, int kPairs, typename Source, typename Where>
-__device__ __forceinline__ void few_rows_tile(const FewArgs& p, int e, int cg, bool through, Source source, Where where,
-                                              f32x4 (&part)[4][2][64]) {
+template <bool GATEUP, bool STREAM, typename Source, typename Where>
+__device__ __forceinline__ void few_rows_tile(const FewArgs& p, int e, int cg, bool through, Source source, Where where, char* ring) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, g = lane >> 4;
   const int K = p.K, N = p.N;
   // this wave's share of the contraction
-  const int steps = K >> 6, s0 = steps * wave >> 2, s1 = steps * (wave + 1) >> 2;
+  const int steps = K >> 6, s0 = steps * wave >> 2, n = (steps * (wave + 1) >> 2) - s0;
   // weight rows: 16 columns of gate and the same of up, or 32 columns of the one matrix (N % 32 == 0)
   const int n0 = cg * (GATEUP ? 16 : 32);
-  const int64_t we = static_cast<int64_t>(e) * N * K;
-  const auto rs0 = few_rsrc(p.b0 + we), rs1 = few_rsrc(p.b1 + we), rsA = few_rsrc(p.a);
-  const uint32_t off0 = static_cast<uint32_t>((n0 + r16) * K + g * 16) * 2u;
-  const uint32_t off1 = GATEUP ? off0 : off0 + static_cast<uint32_t>(32 * K);
-  u32x4 b0[kPairs][2], b1[kPairs][2], a[kPairs][2];
-  auto request_w = [&](int i, int step) {
-    const int k = step * 128;  // bytes
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      b0[i][h] = __builtin_amdgcn_raw_buffer_load_b128(rs0, off0 + 16 * h, k, 0);
-      b1[i][h] = __builtin_amdgcn_raw_buffer_load_b128(rs1, off1 + 16 * h, k, 0);
-    }
+  const int64_t we = static_cast<int64_t>(e) * N * K + static_cast<int64_t>(n0) * K + s0 * 64;
+  const uint64_t w0 = reinterpret_cast<uint64_t>(p.b0 + we);
+  const uint64_t w1 = reinterpret_cast<uint64_t>(GATEUP ? p.b1 + we : p.b0 + we + static_cast<int64_t>(16) * K);
+  const uint64_t act = reinterpret_cast<uint64_t>(p.a + s0 * 64);
+  const uint32_t own = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_cptr)ring)) + wave * (kFewSteps * kFewStep);
+  // an instruction's eight rows: this lane's, and its 16 bytes -- chunk c of row r of 16 lies at c ^ (r >> 1)
+  const int r8 = lane >> 3, c_lo = (lane & 7) ^ (r8 >> 1), c_hi = c_lo ^ 4;
+  const uint32_t off_lo = static_cast<uint32_t>(r8 * K + c_lo * 8) * 2u, off_hi = static_cast<uint32_t>((r8 + 8) * K + c_hi * 8) * 2u;
+  auto request_w = [&](int s) {
+    const uint32_t k = s * 128u, to = own + (s % kFewSteps) * kFewStep;
+    lds_load16<STREAM>(w0, off_lo, k, to);
+    lds_load16<STREAM>(w0, off_hi, k, to + 1024);
+    lds_load16<STREAM>(w1, off_lo, k, to + 2048);
+    lds_load16<STREAM>(w1, off_hi, k, to + 3072);
   };
-  // the first weights go out before the rows are known (past the end: the last step again, not used)
   auto request_first = [&]() {
 #pragma unroll
-    for (int i = 0; i < kPairs; ++i) request_w(i, min(s0 + i, s1 - 1));
-    __builtin_amdgcn_sched_barrier(0);
+    for (int i = 0; i < kFewSteps; ++i)
+      if (i < n) request_w(i);
   };
+  // the first weights go out before the rows are known
   request_first();
   const FewRows at_rows = where();
   const int row0 = at_rows.row0, rows = at_rows.rows;
   for (int sub = 0; sub < rows; sub += 16) {
     if (sub) request_first();
-    const int row = row0 + min(sub + r16, rows - 1);
-    const int index = through ? source(row) : row;
-    f32x4 acc0 = {0, 0, 0, 0}, acc1 = {0, 0, 0, 0};
-    uint32_t offA;
-    auto request_a = [&](int i, int step) {
+    uint32_t off_a[2];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) a[i][h] = __builtin_amdgcn_raw_buffer_load_b128(rsA, offA + 16 * h, step * 128, 0);
+    for (int h = 0; h < 2; ++h) {
+      const int row = row0 + min(sub + r8 + 8 * h, rows - 1);
+      const int src = through ? min(max(source(row), 0), p.a_rows - 1) : row;
+      off_a[h] = (static_cast<uint32_t>(src) * static_cast<uint32_t>(K) + (h ? c_hi : c_lo) * 8u) * 2u;
+    }
+    auto request_a = [&](int s) {
+      const uint32_t k = s * 128u, to = own + (s % kFewSteps) * kFewStep + 4096;
+      lds_load16(act, off_a[0], k, to);
+      lds_load16(act, off_a[1], k, to + 1024);
     };
-    auto multiply = [&](int i) {
+#pragma unroll
+    for (int i = 0; i < kFewSteps; ++i)
+      if (i < n) request_a(i);
+    f32x4 acc0 = {0, 0, 0, 0}, acc1 = {0, 0, 0, 0};
+    auto multiply = [&](int s) {
+      const uint32_t at = own + (s % kFewSteps) * kFewStep + r16 * 128u;
+      bf16x8 b0[2], b1[2], a[2];
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const bf16x8 af = __builtin_bit_cast(bf16x8, a[i][h]);
-        acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, b0[i][h]), af, acc0, 0, 0, 0);
-        acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, b1[i][h]), af, acc1, 0, 0, 0);
+        const uint32_t piece = ((2 * g + h) ^ (r16 >> 1)) * 16u;  // k 16 g + 8 h ..
+        b0[h] = lds_read16(at + piece);
+        b1[h] = lds_read16(at + piece + 2048);
+        a[h] = lds_read16(at + piece + 4096);
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the step's place is free for requests then)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b0[h], a[h], acc0, 0, 0, 0);
+        acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b1[h], a[h], acc1, 0, 0, 0);
       }
     };
-    const int src = through ? min(max(index, 0), p.a_rows - 1) : row;
-    offA = (static_cast<uint32_t>(src) * static_cast<uint32_t>(K) + g * 16) * 2u;
-#pragma unroll
-    for (int i = 0; i < kPairs; ++i) request_a(i, min(s0 + i, s1 - 1));
-    int s = s0;
-    for (; s + 2 * kPairs <= s1; s += kPairs) {
-#pragma unroll
-      for (int i = 0; i < kPairs; ++i) {
-        multiply(i);
-        request_w(i, s + kPairs + i);
-        request_a(i, s + kPairs + i);
-      }
+    // the first steps are waited for together (their weights were requested in front of all their rows), the others in turn
+    static_assert(kFewSteps == 2, "the waits below are written out");
+    lds_wait<0>();
+    int s = 0;
+    for (; s + kFewSteps < n; ++s) {
+      if (s >= kFewSteps) lds_wait<6>();
+      multiply(s);
+      request_w(s + kFewSteps);
+      request_a(s + kFewSteps);
     }
-    // at most 2 kPairs - 1 steps are left, kPairs of them requested
-#pragma unroll
-    for (int i = 0; i < kPairs; ++i) {
-      if (s + i < s1) multiply(i);
-      if (s + kPairs + i < s1) {
-        request_w(i, s + kPairs + i);
-        request_a(i, s + kPairs + i);
-      }
+    if (s < n) {
+      lds_wait<6>();
+      multiply(s++);
     }
-#pragma unroll
-    for (int i = 0; i < kPairs; ++i)
-      if (s + kPairs + i < s1) multiply(i);
-    part[wave][0][lane] = acc0;
-    part[wave][1][lane] = acc1;
+    if (s < n) {
+      lds_wait<0>();
+      multiply(s);
+    }
+    f32x4* part = reinterpret_cast<f32x4*>(ring);  // [4][2][64]
+    __syncthreads();
+    part[(wave * 2 + 0) * 64 + lane] = acc0;
+    part[(wave * 2 + 1) * 64 + lane] = acc1;
     __syncthreads();
     // lane = activation row lane & 15, its four values = columns 4 g .. 4 g + 3 of a 16-column tile
     auto sum = [&](int tile) {
-      f32x4 v = part[0][tile][lane];
+      f32x4 v = part[tile * 64 + lane];
 #pragma unroll
-      for (int w = 1; w < 4; ++w) v += part[w][tile][lane];
+      for (int w = 1; w < 4; ++w) v += part[(w * 2 + tile) * 64 + lane];
       return v;
     };
     if (wave < (GATEUP ? 1 : 2) && sub + r16 < rows) {
-      const int64_t at = static_cast<int64_t>(row) * N + n0 + 16 * wave + 4 * g;
+      const int64_t at = static_cast<int64_t>(row0 + sub + r16) * N + n0 + 16 * wave + 4 * g;
       if constexpr (GATEUP) {
         const f32x4 v = sum(0), u = sum(1);
         float gv[4], uv[4], hv[4];
@@ -156,21 +175,21 @@ __device__ __forceinline__ void few_rows_tile(const FewArgs& p, int e, int cg, b
   }
 }
 
-template <bool GATEUP, int kPairs>
-__global__ __launch_bounds__(256, 4) void few_rows_kernel(FewArgs p) {
-  __shared__ f32x4 part[4][2][64];
+template <bool GATEUP, bool STREAM>
+__global__ __launch_bounds__(256) void few_rows_kernel(FewArgs p) {
+  extern __shared__ __attribute__((aligned(16))) char ring[];
   const int t = blockIdx.x / p.col_groups, cg = blockIdx.x - t * p.col_groups;
   // looked up together (an entry past the last tile is not used): every lookup in a row is a round trip in front of the weights
   const int tiles = *p.num_tiles, e = __builtin_amdgcn_readfirstlane(p.tile_expert[t]),
             row0 = __builtin_amdgcn_readfirstlane(p.tile_row0[t]);
   if (t >= tiles) return;
-  few_rows_tile<GATEUP, kPairs>(
+  few_rows_tile<GATEUP, STREAM>(
       p, e, cg, p.a_src != nullptr, [&](int row) { return p.a_src[row]; },
       [&]() -> FewRows {
         const int cnt = p.seg_counts[e], seg0 = p.seg_offsets[e];
         return {row0, min(even_tile_rows(cnt, 256), seg0 + cnt - row0)};
       },
-      part);
+      ring);
 }
 
 // ---- a handful of tokens, forward only: no plan ---------------------------------------------------
@@ -214,13 +233,13 @@ __device__ __forceinline__ RowChoice choose(const ChoiceIn& c, int t, int l) {
 constexpr int kChoiceTokens = 16;  // a row of 16 lanes each in one workgroup of four waves
 
 template <int VPR, bool FULL>
-__global__ __launch_bounds__(256, 4) void choice_gateup_kernel(FewArgs p, ChoiceIn c) {
-  __shared__ f32x4 part[4][2][64];
+__global__ __launch_bounds__(256) void choice_gateup_kernel(FewArgs p, ChoiceIn c) {
+  extern __shared__ __attribute__((aligned(16))) char ring[];
   const int lane = threadIdx.x & 63, K = c.sel.K;
   const int row = blockIdx.x / p.col_groups, cg = blockIdx.x - row * p.col_groups;
   if (row == c.T * K) {
     // the last workgroup: everyone's choices for the second launch, and the experts' loads
-    int* count = reinterpret_cast<int*>(part);
+    int* count = reinterpret_cast<int*>(ring);
     for (int e = threadIdx.x; e < c.sel.E; e += 256) count[e] = 0;
     __syncthreads();
     const int t = threadIdx.x >> 4, l = lane & 15;
@@ -238,8 +257,8 @@ __global__ __launch_bounds__(256, 4) void choice_gateup_kernel(FewArgs p, Choice
   const RowChoice ch = choose<VPR, FULL>(c, t, lane & 15);
   const int id = __builtin_amdgcn_readlane(ch.id, row - t * K);
   if (id < c.lo || id >= c.hi) return;  // (the same for the whole workgroup)
-  few_rows_tile<true, 4>(
-      p, id - c.lo, cg, true, [&](int) { return t; }, [&]() -> FewRows { return {row, 1}; }, part);
+  few_rows_tile<true, false>(
+      p, id - c.lo, cg, true, [&](int) { return t; }, [&]() -> FewRows { return {row, 1}; }, ring);
 }
 
 struct ChoiceOut {
@@ -337,11 +356,11 @@ __global__ __launch_bounds__(64 * kChoiceWaves) void choice_down_kernel(ChoiceOu
 
 }  // namespace
 
-// gate/up (stage 1) or down (stage 2) of the forward; the arguments of bf16_grouped_fwd.
+// gate/up (stage 1) or down (stage 2) of the forward; the arguments of bf16_grouped_fwd.  stream: weights with the non-temporal hint.
 int few_rows_fwd(int stage, const void* a, const int32_t* a_src, int64_t a_rows, const void* b0, const void* b1,
                  void* gate, void* up, void* out, const int32_t* seg_offsets, const int32_t* seg_counts,
                  const int32_t* tile_expert, const int32_t* tile_row0, const int32_t* num_tiles, int64_t tiles, int64_t K,
-                 int64_t N, hipStream_t s) {
+                 int64_t N, bool stream, hipStream_t s) {
   FewArgs p{};
   p.a = (const uint16_t*)a; p.a_src = a_src; p.a_rows = (int)a_rows;
   p.b0 = (const uint16_t*)b0; p.b1 = (const uint16_t*)b1;
@@ -350,10 +369,9 @@ int few_rows_fwd(int stage, const void* a, const int32_t* a_src, int64_t a_rows,
   p.num_tiles = num_tiles; p.K = (int)K; p.N = (int)N;
   p.col_groups = (int)(N / (stage == 1 ? 16 : 32));
   const dim3 grid((unsigned)(tiles * p.col_groups));
-  // (up to 768: three steps a wave)
-  if (stage == 1) hipLaunchKernelGGL((few_rows_kernel<true, 4>), grid, dim3(256), 0, s, p);
-  else if (K <= 12 * 64) hipLaunchKernelGGL((few_rows_kernel<false, 3>), grid, dim3(256), 0, s, p);
-  else hipLaunchKernelGGL((few_rows_kernel<false, 4>), grid, dim3(256), 0, s, p);
+  const auto kernel = stage == 1 ? (stream ? few_rows_kernel<true, true> : few_rows_kernel<true, false>)
+                                 : (stream ? few_rows_kernel<false, true> : few_rows_kernel<false, false>);
+  hipLaunchKernelGGL(kernel, grid, dim3(256), kFewLds, s, p);
   return check_launch("grouped forward, few rows");
 }
 
@@ -396,7 +414,7 @@ extern "C" int mi355_choice_gateup_fwd(const float* partial, int splits, const f
                    weights_TK, ids_TK, counts_E};
   with_row_shape(E, [&](auto vpr, auto full) {
     hipLaunchKernelGGL((choice_gateup_kernel<decltype(vpr)::value, decltype(full)::value>),
-                       dim3((unsigned)(T * K * p.col_groups + 1)), dim3(256), 0, as_stream(stream), p, c);
+                       dim3((unsigned)(T * K * p.col_groups + 1)), dim3(256), kFewLds, as_stream(stream), p, c);
   });
   return check_launch("choice_gateup");
 }
