@@ -60,6 +60,7 @@
 //
 // The LDS layouts (KC / KS) and fragment reads are in bf16_tiles.h.
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <type_traits>
 
@@ -1080,29 +1081,25 @@ static unsigned resident_blocks() {
 }
 
 
-// Whether a product of El experts and n 256-column tiles runs on 128-column ones instead: twice the work items, each with the
-// whole contraction.  Where experts of equal load would occupy at most half the CUs (three eighths where the tiles are
-// mostly full, and a narrow one so has as many rows to stage for half the products).  us, wide / narrow: the block forward, 1000 tokens of
-// 16 experts of 1024 x 512, four each, 69 / 55, of 32 63 / 53, 300 tokens 55 / 47 and 56 / 49; a training step of 2000 of 16 226 / 212
-// (with dH narrow; gate/up and down too, 128 tiles of 250 rows, 215), of 32 230 / 217, of 60 267 / 257, 1000 of 64, six each, 249 / 235,
-// 1000 of 16 of 1984 x 1024 338 / 315; 128 tiles of 250 rows (4000 of 16) 326 / 334, 4000 of 60 394 / 418.
-// Forward products also where wide tiles are one round of workgroups and a mostly empty second one (three rounds of half the work; the
-// forward: 4000 tokens of 60 of 1280 x 640, two each, 142 / 138, 800 of 64 of 1280 x 640, six each, 119 / 117, 2500 of 16 of 1792 x
-// 1024, four each, 172 / 169; one and a half rounds, 1200 of 128 of 640 x 640, four each, 115 / 117; the input gradient so, beside the
-// weight gradients: a step of 5000 of 32 of 1024 x 704, four each, 507 / 524).
-// Alone, 1500 products of 4 to 128 experts of 512-2048 x 448-1024, 20-500 rows each, time on narrow tiles / on wide ones: partly full, up to half the CUs
-// 0.66-0.82 (328 of 328 faster), above that up to one round 1.01-1.34 but for 20 whose width a wide tile overhangs by half; mostly full, up to
-// three eighths 0.63-1.21 (149 of 154 faster), from there to half 0.65-1.24 (46 of 88); forward, one to one and three eighths rounds 0.69-0.99 (42
-// of 42) and, mostly full, 0.66-1.15 (21 of 30), up to one and a half 0.87-1.16 (72 of 93).
+// Whether a product of El experts runs on 128-column tiles (`narrow_n` of them across) instead of 256-column ones (`wide_n`): where their rounds of
+// workgroups, seven tenths as long, take less time.  The number of row tiles is that of loads spread like independent draws around the mean
+// (experts of 256 rows on average have one tile and a half each); one expert's share of a wider router counts rows it does not get, which errs
+// towards wide tiles.  A narrow tile's time over a wide one's, launch included, where both are one round: 0.60-0.73 mostly full, 0.68-0.83 partly; three rounds over two
+// 0.85-0.92, four over two 1.02-1.3.  Of 450 products (gate/up, down, dH, dRows of 4 to 48 experts of 640 x 448 to 2048 x 768, 40 to 500 rows each) 269
+// run on narrow tiles, two of them up to 17 % slower than on wide ones, the others up to 40 % faster, and 29 of the rest would gain.  (A rule of halves and three eighths of
+// one round of evenly filled tiles had chosen 14 that lose and left 60.)
 // One dense segment: the input gradient alone (the dH of 4096 rows x 2048 columns is 16 x 8 tiles).  It runs beside other products, and
 // narrow gate/up and down tiles take CUs those would have had (one rank's share, 1000 tokens: 595 / 638).
-static bool narrow(int mode, int64_t El, int64_t n, int64_t tile_capacity) {
+static bool narrow(int mode, int64_t El, int64_t wide_n, int64_t narrow_n, int64_t tile_capacity) {
   const int64_t cus = resident_blocks();
-  if (El == 1) return (mode == RM_DH || mode == RM_DLIN) && tile_capacity * n * 4 <= cus * 3;
+  if (El == 1) return (mode == RM_DH || mode == RM_DLIN) && tile_capacity * wide_n * 4 <= cus * 3;
   const int64_t spare = std::max<int64_t>(tile_capacity - El - 1, 0);  // 256 rows each
-  const int64_t tiles = El * std::max<int64_t>((spare + El - 1) / El, 1);
-  if ((mode == RM_GATEUP || mode == RM_DOWN) && tiles * n > cus && tiles * n * 8 <= cus * 11) return true;
-  return tiles * n <= (spare * 10 > tiles * 7 ? cus * 3 / 8 : cus / 2);
+  if (spare * wide_n > 4 * cus) return false;
+  const double mean = (static_cast<double>(spare) + 0.5) * 256.0 / static_cast<double>(El), sd = std::sqrt(mean);
+  double tiles = 1.0;
+  for (int j = 256; j < mean + 5.0 * sd; j += 256) tiles += 0.5 * std::erfc((j + 0.5 - mean) / (sd * std::sqrt(2.0)));
+  auto rounds = [&](int64_t n) { return std::ceil((tiles * static_cast<double>(El * n) - 0.5) / static_cast<double>(cus)); };
+  return rounds(narrow_n) * 0.7 < rounds(wide_n);
 }
 
 // Whether experts with one row tile -- whose weights no other tile reads -- have them read with the non-temporal hint: where the three weight stacks do
@@ -1124,8 +1121,9 @@ static int launch_row(RowArgs& a, int64_t width, int64_t El, int64_t tile_capaci
   constexpr int div = MODE == RM_GATEUP ? 2 : 1;
   a.stream = streamed(El, a.D, a.F);
   a.n_tiles = (int)((width + 256 / div - 1) / (256 / div));
-  if (narrow(MODE, El, a.n_tiles, tile_capacity)) {
-    a.n_tiles = (int)((width + 128 / div - 1) / (128 / div));
+  const int64_t narrow_n = (width + 128 / div - 1) / (128 / div);
+  if (narrow(MODE, El, a.n_tiles, narrow_n, tile_capacity)) {
+    a.n_tiles = (int)narrow_n;
     static PerDeviceOnce narrow_configured;
     if (narrow_configured.needed()) {
       if (int rc = set_lds(row_tiled_kernel<MODE, 2, GATHER, SAVE_GU, TURN>, R_LDS_BYTES)) return rc;
