@@ -118,13 +118,15 @@ Tensor carve(const Tensor& like, Layout layout) {
 constexpr int64_t kShortRowSum = 6 << 20;
 
 // A folded backward so small that the host is what takes the time: a second stream's fork and join cost it more than the weight
-// gradients gain beside the input gradient.  A training step, us, beside / behind it: 200, 600, 1000 tokens of 16 experts of 1024 x 512,
-// four each, 166 / 129, 161 / 146, 176 / 160, 2000 of them 217 / 227; 200, 1000 of 32 171 / 151, 176 / 176, 2000 218 / 225; 300 of 60 of 512 x
-// 448, two each, 183 / 140; 1500 of 32 of 640 x 640, three each, 288 tiles, 176 / 196; 200 of 60 of 1024 x 512, 480 tiles, 177 / 190.
-// Of 111 steps of 8 to 64 experts of 512-2048 x 448-768, 128 to 4000 tokens of four each, the 43 within both lines take 0.64-0.98 of their
-// time beside it; the others 0.75-1.13, the least of them below 700 tokens and 400 tiles.
+// gradients gain beside the input gradient.  A training step, us, beside / behind it: 64 experts of 768 x 448 (384 tiles), two each, 100 to 1500 tokens 208 / 149,
+// 204 / 155, 208 / 156, 198 / 157, 200 / 160, 204 / 168; 32 of 640 x 640 (288), four each, 300 to 1500 tokens 197 / 140, 199 / 145, 200 / 159, 203 / 166, 204 / 187;
+// 48 of 1024 x 512 (384), four each, 208 / 177, 212 / 201, 211 / 192, 215 / 205, 214 / 218; 60 of it (480), three each, 212 / 191, 212 / 215, 214 / 203, 213 / 205, 224 / 224; 64 of it
+// (512), six each, 300 to 1500 tokens 211 / 188, 213 / 193, 213 / 202, 219 / 222, 249 / 248; 24 of 1536 x 768 (432), four each, 209 / 174, 209 / 189, 210 / 202, 225 / 225, 269 /
+// 282; 128 of 768 x 512 (768) 249 / 257, 254 / 259, 266 / 272.  32 of 1024 x 704 (384), four each, 300 to 2500 tokens 203 / 158,
+// 203 / 164, 203 / 180, 208 / 188, 216 / 216, 288 / 292.  The second line lies where the products take as long as the host: 1500 tokens of the 48, 1000 of the 64
+// or of the last, 700 of the 24.
 bool short_backward(int64_t El, int64_t D, int64_t F, int64_t R) {
-  return El * ((D + 255) / 256) * ((F + 255) / 256) <= 256 && R * D * F <= (int64_t{1} << 31);
+  return El * ((D + 255) / 256) * ((F + 255) / 256) <= 512 && R * D * F <= (int64_t{3} << 30);
 }
 
 // What the backward reads besides the inputs, in one allocation: the plan's and the router's arrays, the
