@@ -488,6 +488,16 @@ int mi355_grouped_swiglu_fwd(const void* rows, const int32_t* token_of_row, int6
                              int64_t tile_capacity, void* gate, void* up, void* h,
                              void* y, int64_t El, int64_t D, int64_t F,
                              int64_t row_capacity, void* stream);
+/* The same results where other launches run beside it on another stream (a shared expert beside the router and the routed
+ * experts): the matrix-core kernels may leave some CUs to those. */
+int mi355_grouped_swiglu_fwd_beside(const void* rows, const int32_t* token_of_row, int64_t num_tokens,
+                                    const void* w1, const void* w3, const void* w2, int dtype,
+                                    const int32_t* seg_offsets,
+                                    const int32_t* seg_counts, const int32_t* tile_expert,
+                                    const int32_t* tile_row0, const int32_t* num_tiles,
+                                    int64_t tile_capacity, void* gate, void* up, void* h,
+                                    void* y, int64_t El, int64_t D, int64_t F,
+                                    int64_t row_capacity, void* stream);
 
 /*
  * Backward of the above (autograd-derived in the reference):

@@ -129,3 +129,25 @@ def test_few_rows_and_streamed_weights(counts, D, Fd):
             xe = x[tok[r]].float()
             for got, want in ((gate[r], xe @ w1[e].float().T), (up[r], xe @ w3[e].float().T), (y[r], h[r].float() @ w2[e].float().T)):
                 assert row_errors(got, want) < 2.0 ** -8
+
+
+# the shared expert's gate/up tiles, four to 256 tokens, on either side of seven eighths of the CUs, one and one and a half rounds of them
+@pytest.mark.parametrize("tokens", [56 * 256, 57 * 256 - 3, 64 * 256, 65 * 256, 96 * 256, 96 * 256 + 1])
+def test_shared_expert_beside_the_router(tokens):
+    """Beside the router on fewer workgroups, or in place on all: the same bits, forward and in the shared expert's gradients."""
+    from tests.helpers import build_block, make_params
+    from oracle import moe_ref as R
+
+    print(f"shared expert beside the router, {tokens} tokens", flush=True)
+    D, E, Fd = 384, 8, 384
+    block = build_block(make_params(E, D, Fd, torch.bfloat16, seed=1, std=0.05, shared_F=448), R.RouterSpec(E, 1), D, Fd, torch.bfloat16, DEV)
+    x, gout = (torch.randn(tokens, D, generator=torch.Generator(device=DEV).manual_seed(i), device=DEV).bfloat16() for i in (1, 2))
+    results = []
+    for overlap in (True, False, True):
+        block.overlap_shared_experts = overlap
+        block.zero_grad()
+        out = block(x)
+        out.backward(gout)
+        results.append([out.detach().clone(), *(p.grad.clone() for p in block.shared_experts.parameters())])
+    for other in results[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(results[0], other))

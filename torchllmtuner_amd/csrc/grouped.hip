@@ -165,13 +165,15 @@ extern "C" int64_t mi355_grouped_tile_m(int dtype) {
   return tile_m_for(dtype);
 }
 
-extern "C" int mi355_grouped_swiglu_fwd(const void* rows, const int32_t* token_of_row, int64_t num_tokens,
-                                        const void* w1, const void* w3, const void* w2, int dtype, const int32_t* seg_offsets,
-                                        const int32_t* seg_counts, const int32_t* tile_expert,
-                                        const int32_t* tile_row0, const int32_t* num_tiles,
-                                        int64_t tile_capacity, void* gate, void* up, void* h, void* y,
-                                        int64_t El, int64_t D, int64_t F, int64_t row_capacity,
-                                        void* stream) {
+namespace {
+// mi355_grouped_swiglu_fwd; stages: of the matrix-core path (3, with or without that it runs beside others)
+int swiglu_fwd(const void* rows, const int32_t* token_of_row, int64_t num_tokens,
+               const void* w1, const void* w3, const void* w2, int dtype, const int32_t* seg_offsets,
+               const int32_t* seg_counts, const int32_t* tile_expert,
+               const int32_t* tile_row0, const int32_t* num_tiles,
+               int64_t tile_capacity, void* gate, void* up, void* h, void* y,
+               int64_t El, int64_t D, int64_t F, int64_t row_capacity,
+               int stages, void* stream) {
   if (int rc = check_common("grouped_swiglu_fwd", dtype, El, D, F, row_capacity, tile_capacity)) return rc;
   if (int rc = check_gather("grouped_swiglu_fwd", row_capacity > 0 ? token_of_row : nullptr, num_tokens, D, dtype)) return rc;
   if (row_capacity == 0 || tile_capacity == 0) return MI355_OK;
@@ -187,7 +189,7 @@ extern "C" int mi355_grouped_swiglu_fwd(const void* rows, const int32_t* token_o
   hipStream_t s = as_stream(stream);
   if (fast)
     return bf16_grouped_fwd(rows, token_of_row, num_tokens, w1, w3, w2, seg_offsets, seg_counts, tile_expert,
-                            tile_row0, num_tiles, tile_capacity, gate, up, h, y, El, D, F, row_capacity, 3, s);
+                            tile_row0, num_tiles, tile_capacity, gate, up, h, y, El, D, F, row_capacity, stages, s);
   if (token_of_row)
     return fail(MI355_EUNSUP, "grouped_swiglu_fwd: the token gather needs bf16 with D and F multiples of 64; "
                               "materialise the rows with mi355_permute_rows_fwd instead");
@@ -213,6 +215,29 @@ extern "C" int mi355_grouped_swiglu_fwd(const void* rows, const int32_t* token_o
   if (int rc = check_launch("swiglu_fwd")) return rc;
   // down: B(k=f, n=d) = w2[e][d][f]
   return rowseg(sg, h, F, w2, 1, F, D * F, y, D, F, dtype, 0, s);
+}
+}  // namespace
+
+extern "C" int mi355_grouped_swiglu_fwd(const void* rows, const int32_t* token_of_row, int64_t num_tokens,
+                                        const void* w1, const void* w3, const void* w2, int dtype, const int32_t* seg_offsets,
+                                        const int32_t* seg_counts, const int32_t* tile_expert,
+                                        const int32_t* tile_row0, const int32_t* num_tiles,
+                                        int64_t tile_capacity, void* gate, void* up, void* h, void* y,
+                                        int64_t El, int64_t D, int64_t F, int64_t row_capacity,
+                                        void* stream) {
+  return swiglu_fwd(rows, token_of_row, num_tokens, w1, w3, w2, dtype, seg_offsets, seg_counts, tile_expert, tile_row0,
+                    num_tiles, tile_capacity, gate, up, h, y, El, D, F, row_capacity, 3, stream);
+}
+
+extern "C" int mi355_grouped_swiglu_fwd_beside(const void* rows, const int32_t* token_of_row, int64_t num_tokens,
+                                               const void* w1, const void* w3, const void* w2, int dtype, const int32_t* seg_offsets,
+                                               const int32_t* seg_counts, const int32_t* tile_expert,
+                                               const int32_t* tile_row0, const int32_t* num_tiles,
+                                               int64_t tile_capacity, void* gate, void* up, void* h, void* y,
+                                               int64_t El, int64_t D, int64_t F, int64_t row_capacity,
+                                               void* stream) {
+  return swiglu_fwd(rows, token_of_row, num_tokens, w1, w3, w2, dtype, seg_offsets, seg_counts, tile_expert, tile_row0,
+                    num_tiles, tile_capacity, gate, up, h, y, El, D, F, row_capacity, 3 | 128, stream);
 }
 
 extern "C" int mi355_grouped_swiglu_bwd(const void* dy, const void* rows,

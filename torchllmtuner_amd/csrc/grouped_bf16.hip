@@ -1063,7 +1063,7 @@ bool bf16_fast_path_ok(int64_t D, int64_t F) {
   return D % 64 == 0 && F % 64 == 0 && D >= 384 && F >= 384 && D * F < (1ll << 30);
 }
 
-enum { STAGE_GATEUP = 1, STAGE_DOWN = 2, STAGE_DH = 4, STAGE_DX = 8, STAGE_DW2 = 16, STAGE_DW1 = 32, STAGE_DW3 = 64 };
+enum { STAGE_GATEUP = 1, STAGE_DOWN = 2, STAGE_DH = 4, STAGE_DX = 8, STAGE_DW2 = 16, STAGE_DW1 = 32, STAGE_DW3 = 64, STAGE_BESIDE = 128 };
 
 static unsigned round8(int64_t v) { return static_cast<unsigned>((v + 7) / 8 * 8); }
 
@@ -1113,11 +1113,24 @@ static bool narrow(int mode, int64_t El, int64_t wide_n, int64_t narrow_n, int64
 // With two row tiles or more an expert, which share the weights in L2, the hint costs 2-8 % (8192 tokens of the first block, 16384 of a skewed router).
 static bool streamed(int64_t El, int64_t D, int64_t F) { return El * D * F * 6 > (int64_t{320} << 20); }
 
+// Workgroups of a gate/up product that runs beside the launches of a router (a shared expert's): a workgroup takes a CU whole until its list of tiles
+// ends, so a product that holds every CU makes each of them wait (rank and plan, 12 and 11 us alone, took 195 and 63), and the routed experts, often a
+// read of their weights, start when it has ended instead of running beside it.  An eighth of the CUs is enough to prevent that.  Block forward, us, all CUs / seven eighths /
+// three quarters: one rank's share of 7168 x 256 experts x 2048 at 3600 tokens (240 tiles) 847 / 840 / 842, 4096 996 / 893 / 886, 4500 1044 / 1021 / 1030,
+// 5500 (352) 1022 / 994 / 992; 64 experts of 2048 x 1408 and a shared one of twice that at 2600 tokens (242) 463 / 433 / 447; 32 of 1024 x 512, 8192 tokens
+// 218 / 211 / 209.  Past one and a half rounds of workgroups, where the product is long beside the router: 7000 tokens of the share 1416 / 1439 on
+// one box, 1401 / 1406 on another, 8192 1504 / 1529, 1482 / 1490, 5600 and 16384 of the second block 795 / 781 and 2000 / 2033.  The down projection starts behind the router: on fewer CUs nothing more, at some sizes 1-2 % slower.
+static unsigned beside_router_blocks(int64_t tiles) {
+  const unsigned n = resident_blocks();
+  return n >= 64 && tiles * 2 <= 3 * static_cast<int64_t>(n) ? n / 64 * 56 : n;
+}
+
 // width: output columns; gate/up tiles hold both halves of their column range.  Tiles are
 // 256 or 128 wide (a 192-wide KS tile would not hold the swizzle: 24 chunks per row are not a multiple
 // of the 16 the key permutes); an overhanging last tile shifts back.
 template <int MODE, bool GATHER = false, bool SAVE_GU = true, bool TURN = false>
-static int launch_row(RowArgs& a, int64_t width, int64_t El, int64_t tile_capacity, hipStream_t s, const char* what) {
+static int launch_row(RowArgs& a, int64_t width, int64_t El, int64_t tile_capacity, hipStream_t s, const char* what,
+                      bool beside = false) {
   constexpr int div = MODE == RM_GATEUP ? 2 : 1;
   a.stream = streamed(El, a.D, a.F);
   a.n_tiles = (int)((width + 256 / div - 1) / (256 / div));
@@ -1138,7 +1151,7 @@ static int launch_row(RowArgs& a, int64_t width, int64_t El, int64_t tile_capaci
     if (int rc = set_lds(row_tiled_kernel<MODE, 4, GATHER, SAVE_GU, TURN>, R_LDS_BYTES)) return rc;
     configured.done();
   }
-  const unsigned blocks = std::min(round8(tile_capacity * a.n_tiles), resident_blocks());
+  const unsigned blocks = std::min(round8(tile_capacity * a.n_tiles), beside ? beside_router_blocks(tile_capacity * a.n_tiles) : resident_blocks());
   hipLaunchKernelGGL((row_tiled_kernel<MODE, 4, GATHER, SAVE_GU, TURN>), dim3(blocks), dim3(NT), R_LDS_BYTES, s, a);
   return check_launch(what);
 }
@@ -1185,6 +1198,7 @@ int bf16_grouped_fwd(const void* rows, const int32_t* token_of_row, int64_t num_
                           num_tiles, tiles, F, D, stream, s);
     return MI355_OK;
   }
+  const bool beside = stages & STAGE_BESIDE;
   RowArgs a{};
   a.seg_offsets = seg_offsets; a.seg_counts = seg_counts; a.tile_expert = tile_expert;
   a.tile_row0 = tile_row0; a.num_tiles = num_tiles; a.D = (int)D; a.F = (int)F;
@@ -1196,14 +1210,14 @@ int bf16_grouped_fwd(const void* rows, const int32_t* token_of_row, int64_t num_
     const bool save = gate != nullptr;
     int rc;
     if (token_of_row && turned(El, row_capacity, D))
-      rc = save ? launch_row<RM_GATEUP, true, true, true>(a, F, El, tile_capacity, s, "grouped gate/up")
-                : launch_row<RM_GATEUP, true, false, true>(a, F, El, tile_capacity, s, "grouped gate/up (h only)");
+      rc = save ? launch_row<RM_GATEUP, true, true, true>(a, F, El, tile_capacity, s, "grouped gate/up", beside)
+                : launch_row<RM_GATEUP, true, false, true>(a, F, El, tile_capacity, s, "grouped gate/up (h only)", beside);
     else if (token_of_row)
-      rc = save ? launch_row<RM_GATEUP, true>(a, F, El, tile_capacity, s, "grouped gate/up")
-                : launch_row<RM_GATEUP, true, false>(a, F, El, tile_capacity, s, "grouped gate/up (h only)");
+      rc = save ? launch_row<RM_GATEUP, true>(a, F, El, tile_capacity, s, "grouped gate/up", beside)
+                : launch_row<RM_GATEUP, true, false>(a, F, El, tile_capacity, s, "grouped gate/up (h only)", beside);
     else
-      rc = save ? launch_row<RM_GATEUP>(a, F, El, tile_capacity, s, "grouped gate/up")
-                : launch_row<RM_GATEUP, false, false>(a, F, El, tile_capacity, s, "grouped gate/up (h only)");
+      rc = save ? launch_row<RM_GATEUP>(a, F, El, tile_capacity, s, "grouped gate/up", beside)
+                : launch_row<RM_GATEUP, false, false>(a, F, El, tile_capacity, s, "grouped gate/up (h only)", beside);
     if (rc) return rc;
   }
   if (stages & STAGE_DOWN) {

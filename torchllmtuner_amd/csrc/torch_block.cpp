@@ -210,12 +210,13 @@ struct Fork {
   }
 };
 
-void shared_forward(const Block& b, const Kept& k, void* y, void* stream) {
+// beside: on a stream of its own, beside the router and the routed experts
+void shared_forward(const Block& b, const Kept& k, void* y, void* stream, bool beside) {
   check(mi355_segments_dense(b.T, b.tile_m, k.s_offsets, k.s_counts, k.s_expert, k.s_row0, k.s_num, b.shared_cap, stream),
         "segments_dense");
-  check(mi355_grouped_swiglu_fwd(ptr(b.x), nullptr, b.T, ptr(b.sg), ptr(b.su), ptr(b.sd), b.dt, k.s_offsets, k.s_counts,
-                                 k.s_expert, k.s_row0, k.s_num, b.shared_cap, k.s_gate, k.s_up, k.s_h, y, 1, b.D, b.Fs,
-                                 b.T, stream),
+  const auto forward = beside ? mi355_grouped_swiglu_fwd_beside : mi355_grouped_swiglu_fwd;
+  check(forward(ptr(b.x), nullptr, b.T, ptr(b.sg), ptr(b.su), ptr(b.sd), b.dt, k.s_offsets, k.s_counts, k.s_expert, k.s_row0, k.s_num,
+                b.shared_cap, k.s_gate, k.s_up, k.s_h, y, 1, b.D, b.Fs, b.T, stream),
         "shared expert");
 }
 
@@ -254,7 +255,7 @@ std::tuple<Tensor, Tensor> choices_forward(const Block& b) {
   Fork shared(aux, main);
   if (aux) {
     shared.start();
-    shared_forward(b, k, y_shared, aux->stream);
+    shared_forward(b, k, y_shared, aux->stream, true);
   }
   check(mi355_router_gate_fwd_partial(ptr(b.x), b.dt, fptr(b.gate_w), fptr(gate_b), partial, nullptr, b.T, b.D, b.E, L.stream),
         "router_gate_fwd");
@@ -262,7 +263,7 @@ std::tuple<Tensor, Tensor> choices_forward(const Block& b) {
                                 (int)c.route_norm, (float)c.route_scale, (int)c.num_groups, (int)c.num_limited, c.lo, c.hi,
                                 ptr(b.x), ptr(b.w1), ptr(b.w3), h, weights, ids, counts.data_ptr<int32_t>(), b.D, b.F, L.stream),
         "choice_gateup_fwd");
-  if (b.Fs > 0 && !aux) shared_forward(b, k, y_shared, L.stream);
+  if (b.Fs > 0 && !aux) shared_forward(b, k, y_shared, L.stream, false);
   shared.join();
   check(mi355_choice_down_fwd(h, ptr(b.w2), weights, ids, y_shared, ptr(out), b.T, c.K, b.El, b.D, b.F, (int)c.round_terms,
                               L.stream),
@@ -316,7 +317,7 @@ std::tuple<Tensor, Tensor, Tensor> block_forward(const Block& b, const Stats& st
   Fork shared(aux, main);
   if (aux) {
     shared.start();
-    shared_forward(b, k, y_shared, aux->stream);
+    shared_forward(b, k, y_shared, aux->stream, true);
   }
 
   // router: partial logits, then selection and plan; few experts in one launch less
@@ -369,7 +370,7 @@ std::tuple<Tensor, Tensor, Tensor> block_forward(const Block& b, const Stats& st
                                    ptr(b.w1), ptr(b.w3), ptr(b.w2), b.dt, k.seg_offsets, k.seg_counts, k.tile_expert,
                                    k.tile_row0, k.num_tiles, b.tile_cap, k.gate, k.up, h, y, b.El, b.D, b.F, b.R, L.stream),
           "grouped_swiglu_fwd");
-  if (b.Fs > 0 && !aux) shared_forward(b, k, y_shared, L.stream);
+  if (b.Fs > 0 && !aux) shared_forward(b, k, y_shared, L.stream, false);
   shared.join();
   check(mi355_combine_add_fwd(y, b.dt, k.weights, k.row_of_slot, y_shared, ptr(out), b.T, b.D, c.K, (int)c.round_terms,
                               L.stream),
