@@ -363,6 +363,20 @@ int mi355_route_plan_stats(const float* partial, int splits, const float* logit_
                            const uint8_t* padding_mask_T, int32_t* valid_counts_E, float* scores_TE,
                            float* cutoff_T, float* aux_f_E, float* aux_scale, void* aux_acc,
                            int aux_acc_dtype, const float* aux_denominator, float aux_coeff, void* stats_workspace, void* stream);
+/* The same, and then mi355_quantile_observe(scores_TE, cutoff_T, expert_bias, padding_mask_T, histogram_EB, T, E, B) (NULL: not), in one
+ * launch less. */
+int mi355_route_plan_observe(const float* partial, int splits, const float* logit_bias, float* logits_TE,
+                             const float* expert_bias, int64_t T, int64_t E, int64_t K, int score_func,
+                             int route_norm, float route_scale, int num_groups, int num_limited,
+                             float* weights_TK, int64_t* ids_TK, int64_t lo, int64_t hi, int64_t align,
+                             int64_t tile_m, int32_t* counts_E, int32_t* seg_offsets, int32_t* seg_counts,
+                             int32_t* row_of_slot, int32_t* slot_of_row, int32_t* token_of_row,
+                             float* row_scale, int64_t row_capacity, int32_t* tile_expert, int32_t* tile_row0,
+                             int32_t* num_tiles, int64_t tile_capacity, void* workspace,
+                             const uint8_t* padding_mask_T, int32_t* valid_counts_E, float* scores_TE,
+                             float* cutoff_T, float* aux_f_E, float* aux_scale, void* aux_acc,
+                             int aux_acc_dtype, const float* aux_denominator, float aux_coeff, void* stats_workspace,
+                             int64_t* histogram_EB, int64_t B, void* stream);
 /* Forward of a handful of tokens without a plan, bf16 (mi355_choice_covers): row t*K + k is choice k of token t.
  * mi355_choice_gateup_fwd selects (partial, splits, logit_bias as in mi355_route_plan) and writes h (T*K,F) of the choices in
  * [lo,hi), weights_TK, ids_TK (local expert or -1) and counts_E; mi355_choice_down_fwd projects down and combines (addend (T,D)

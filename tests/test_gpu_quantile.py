@@ -272,3 +272,45 @@ def test_the_update_pushes_load_toward_balance():
     before = int(router(x, bias)[2][:, 0].sum())
     after = int(router(x, nxt)[2][:, 0].sum())
     assert after <= before
+
+
+# too few tokens for the plan's second launch or for LDS bins; the smallest that has them; more tokens than a chunk a workgroup (1024 lanes); fewer experts a
+# workgroup (B = 3000: two, 8192: one) with a last group that is not full, and bins that LDS does not hold
+@pytest.mark.parametrize("T,E,K,B", [(64, 64, 6, 500), (255, 60, 4, 500), (256, 63, 4, 500), (300, 61, 3, 3000), (777, 128, 2, 8192), (777, 40, 2, 8193),
+                                     (8193, 64, 4, 1000), (300, 24, 3, 500)])
+@pytest.mark.parametrize("masked,aux", [(False, False), (True, False), (False, True), (True, True)])
+def test_histogram_of_the_plans_second_launch(T, E, K, B, masked, aux):
+    """Counted behind the plan, with and without the workgroup of the statistics' sums: what the stages' own kernel counts, twice."""
+    from tests.helpers import make_params
+    from torchllmtuner_amd import moe
+
+    print(f"histogram behind the plan T={T} E={E} B={B} masked={masked} aux={aux}", flush=True)
+    D, F = 384, 384
+    p = make_params(E, D, F, torch.bfloat16, seed=T, std=0.05)
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T, D, generator=g).bfloat16().to(DEV)
+    mask = (torch.rand(T, generator=g) < 0.2).to(DEV) if masked else None
+    results = []
+    for in_stages in (False, True):
+        loss = moe.MicrobatchWiseLoadBalanceLoss(coeff=2.0) if aux else None
+        router = moe.QuantileBalancedTopKRouter(E, D, K, num_bins=B, route_norm=True, aux_loss=loss)
+        block = moe.MoE(E, moe.RoutedExperts(moe.GroupedExperts(D, F, E), moe.LocalTokenDispatcher(E, K)), router,
+                        load_balance_coeff=None).to(torch.bfloat16)
+        router.gate.float()
+        with torch.no_grad():
+            router.gate.weight.copy_(p.router_w_ED)
+            for q, w in zip(block.routed_experts.inner_experts.parameters(), (p.w1_EFD, p.w3_EFD, p.w2_EDF)):
+                q.copy_(w)
+            block.expert_bias_E.copy_(torch.linspace(-0.05, 0.05, E))
+        block = block.to(DEV).train()
+        if aux:
+            moe.AuxLoss.set_step_denominator(torch.tensor(float(T * K), device=DEV), model_parts=[block])
+        if in_stages:
+            router.register_forward_hook(lambda *a: None)
+        for _ in range(2):
+            block(x, padding_mask=mask)
+        results.append((router.quantile_balancer.required_bias_histogram_EB, block.tokens_per_expert_E))
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
+    valid = T - (int(mask.sum()) if masked else 0)
+    assert int(results[0][0].sum()) == 2 * valid * E

@@ -87,6 +87,11 @@ SIGNATURES = {
         [P, I, P, P, P, L, L, L, I, I, F, I, I, P, P, L, L, L, L, P, P, P, P, P, P, P, L, P, P, P, L, P,
          P, P, P, P, P, P, P, I, P, F, P, P],
     ),
+    "mi355_route_plan_observe": (
+        I,
+        [P, I, P, P, P, L, L, L, I, I, F, I, I, P, P, L, L, L, L, P, P, P, P, P, P, P, L, P, P, P, L, P,
+         P, P, P, P, P, P, P, I, P, F, P, P, L, P],
+    ),
     "mi355_choice_covers": (I, [L, L, L, L, L, I]),
     "mi355_choice_gateup_fwd": (
         I,

@@ -16,39 +16,18 @@
 #include <algorithm>
 
 #include "common.h"
+#include "quantile_observe.h"
 
 namespace mi355 {
 namespace {
-
-// min and max of bias[0..E) in every thread of a 256-thread workgroup
-__device__ __forceinline__ void bias_range(const float* __restrict__ bias, int E, float* red, float& mn,
-                                           float& mx) {
-  float lo = INFINITY, hi = -INFINITY;
-  for (int e = threadIdx.x; e < E; e += 256) {
-    lo = fminf(lo, bias[e]);
-    hi = fmaxf(hi, bias[e]);
-  }
-  red[threadIdx.x] = lo;
-  red[256 + threadIdx.x] = hi;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) {
-      red[threadIdx.x] = fminf(red[threadIdx.x], red[threadIdx.x + o]);
-      red[256 + threadIdx.x] = fmaxf(red[256 + threadIdx.x], red[256 + threadIdx.x + o]);
-    }
-    __syncthreads();
-  }
-  mn = red[0];
-  mx = red[256];
-}
 
 __global__ __launch_bounds__(256) void quantile_observe_kernel(
     const float* __restrict__ scores, const float* __restrict__ cutoff, const float* __restrict__ bias,
     const uint8_t* __restrict__ padding, unsigned long long* __restrict__ hist, int T, int E, int B) {
 #pragma clang fp contract(off)
-  __shared__ float red[512];
+  __shared__ float red[8];
   float mn, mx;
-  bias_range(bias, E, red, mn, mx);
+  bias_range<256>(bias, E, red, mn, mx);
   const float lower = mn - 1.0f;
   const float width = ((mx - mn) + 2.0f) / static_cast<float>(B);
   const float top = static_cast<float>(B - 1);
@@ -65,42 +44,11 @@ __global__ __launch_bounds__(256) void quantile_observe_kernel(
   }
 }
 
-// The same histogram through LDS: a workgroup owns `eg` neighbouring experts and a run of
-// tokens, counts their pairs in 32-bit LDS bins (a call adds fewer than 2^31 pairs to a
-// bin) and then adds its non-empty bins to the 64-bit histogram.  The required biases of
-// one expert cluster in a few dozen bins, so this replaces most of the global atomics,
-// which queue up on those few addresses, by LDS ones.
-__global__ __launch_bounds__(256) void quantile_observe_lds_kernel(
-    const float* __restrict__ scores, const float* __restrict__ cutoff, const float* __restrict__ bias,
-    const uint8_t* __restrict__ padding, unsigned long long* __restrict__ hist, int T, int E, int B,
-    int eg, int tokens_per_block) {
-#pragma clang fp contract(off)
+// The same histogram through LDS (quantile_observe.h)
+__global__ __launch_bounds__(256) void quantile_observe_lds_kernel(Observe o) {
   extern __shared__ unsigned bins[];  // [eg][B]
-  __shared__ float red[512];
-  float mn, mx;
-  bias_range(bias, E, red, mn, mx);
-  const float lower = mn - 1.0f;
-  const float width = ((mx - mn) + 2.0f) / static_cast<float>(B);
-  const float top = static_cast<float>(B - 1);
-  const int e0 = blockIdx.x * eg;
-  const int ne = min(eg, E - e0);
-  const int t0 = blockIdx.y * tokens_per_block;
-  const int nt = min(tokens_per_block, T - t0);
-  for (int i = threadIdx.x; i < eg * B; i += 256) bins[i] = 0u;
-  __syncthreads();
-  for (int i = threadIdx.x; i < nt * eg; i += 256) {
-    const int t = t0 + i / eg, j = i % eg;
-    if (j >= ne || (padding && padding[t])) continue;
-    const float required = cutoff[t] - scores[static_cast<int64_t>(t) * E + e0 + j];
-    float q = floorf((required - lower) / width);
-    q = fminf(fmaxf(q, 0.0f), top);
-    atomicAdd(bins + j * B + static_cast<int>(q), 1u);
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < ne * B; i += 256) {
-    const unsigned c = bins[i];
-    if (c) atomicAdd(hist + static_cast<int64_t>(e0) * B + i, static_cast<unsigned long long>(c));
-  }
+  __shared__ float red[8];
+  observe_part<256>(o, blockIdx.x, blockIdx.y, bins, red);
 }
 
 __device__ __forceinline__ long long wave_sum_i64(long long v) {
@@ -116,10 +64,10 @@ __global__ __launch_bounds__(256) void quantile_position_kernel(const long long*
                                                                 float* __restrict__ pos, int* __restrict__ observed_E,
                                                                 int E, int K, int B) {
 #pragma clang fp contract(off)
-  __shared__ float red[512];
+  __shared__ float red[8];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   float mn, mx;
-  bias_range(bias, E, red, mn, mx);
+  bias_range<256>(bias, E, red, mn, mx);
   const float width = ((mx - mn) + 2.0f) / static_cast<float>(B);
   const float lower = mn - 1.0f;
 
@@ -180,7 +128,7 @@ __global__ __launch_bounds__(256) void quantile_centre_kernel(const float* __res
   __shared__ int observed;  // some expert has a non-empty histogram
   if (threadIdx.x == 0) observed = 0;
   float mn, mx;
-  bias_range(bias, E, red, mn, mx);  // its barriers also publish `observed = 0`
+  bias_range<256>(bias, E, red, mn, mx);  // its barriers also publish `observed = 0`
   const float width = ((mx - mn) + 2.0f) / static_cast<float>(B);
   int any = 0;
   for (int e = threadIdx.x; e < E; e += 256) any |= observed_E[e];
@@ -216,16 +164,11 @@ extern "C" int mi355_quantile_observe(const float* scores_TE, const float* cutof
   if (T == 0) return MI355_OK;
   MI355_REQUIRE(scores_TE && cutoff_T && expert_bias_E && histogram_EB, "quantile_observe: null pointer");
   unsigned long long* hist = reinterpret_cast<unsigned long long*>(histogram_EB);
-  // experts per workgroup: what 32 KiB of LDS bins hold, at most 4 (more workgroups)
-  const int64_t eg = std::min<int64_t>(std::min<int64_t>(4, E), (32 * 1024) / (B * 4));
-  if (eg >= 1 && T >= 256) {
-    const int64_t groups = (E + eg - 1) / eg;
-    // about 256 workgroups, each with at least 256 tokens so that the LDS bins pay off
-    const int64_t chunks = std::max<int64_t>(1, std::min<int64_t>(T / 256, (256 + groups - 1) / groups));
-    const int64_t per = (T + chunks - 1) / chunks;
-    hipLaunchKernelGGL(quantile_observe_lds_kernel, dim3((unsigned)groups, (unsigned)((T + per - 1) / per)),
-                       dim3(256), (size_t)(eg * B * 4), as_stream(stream), scores_TE, cutoff_T, expert_bias_E,
-                       padding_mask_T, hist, (int)T, (int)E, (int)B, (int)eg, (int)per);
+  Observe o{scores_TE, cutoff_T, expert_bias_E, padding_mask_T, hist, (int)T, (int)E, (int)B, 0, 0};
+  unsigned groups, chunks;
+  observe_shape(T, E, B, o.eg, o.tokens, groups, chunks);
+  if (o.eg >= 1) {
+    hipLaunchKernelGGL(quantile_observe_lds_kernel, dim3(groups, chunks), dim3(256), (size_t)(o.eg * B * 4), as_stream(stream), o);
     return check_launch("quantile_observe");
   }
   const int64_t total = T * E;

@@ -9,7 +9,8 @@
 //   2. route_rows   the same partition: every workgroup sums the histograms below its own for its
 //                   slots' offsets (all of them, for the segments), which costs it a read of a few
 //                   dozen KiB from L2 and saves the launch of a scan, and writes its slots' rows in
-//                   both directions; the first workgroup writes the plan's lists.
+//                   both directions; the first workgroup writes the plan's lists.  What statistics a router keeps are summed,
+//                   and its required-bias histogram is counted, by workgroups of their own behind those.
 // A single workgroup does both at once.  Bound by launches, instruction issue and dependent latency throughout: at 33
 // tokens of 128 experts the four launches this replaces took 29 us of GPU time, at 8192 tokens
 // (8 each) 39 us; here 13 and 21.
@@ -19,6 +20,7 @@
 #include "common.h"
 #include "gate_rows.h"
 #include "gemm_generic.h"
+#include "quantile_observe.h"
 #include "select_rows.h"
 
 namespace mi355 {
@@ -161,10 +163,10 @@ __device__ __forceinline__ void place_slot(const LayoutLds& s, const PlanOut& p,
 }
 
 // Sums the workgroups' valid counts and score shares (in order), and the loss from them; one workgroup.
+template <int kBatch>  // loads of either kind in flight
 __device__ void finish_stats(const StatsOut& st, int E, int nb, float* red) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   constexpr float kEps = 1e-12f;  // F.normalize's clamp
-  constexpr int kBatch = 8;
   int valid = 0;
   float share = 0.0f;
   if (tid < E) {
@@ -397,7 +399,7 @@ __global__ __launch_bounds__(kLanes) void route_rank_kernel(
     for (int e = tid; e < E; e += kLanes) block_hist[static_cast<int64_t>(blockIdx.x) * E + e] = run[e];
     return;
   }
-  if (stats) finish_stats(st, E, 1, red_sh);  // (each lane reads back the counts it wrote)
+  if (stats) finish_stats<1>(st, E, 1, red_sh);  // (each lane reads back the counts it wrote)
   const LayoutLds s(extra, E);
   for (int e = tid; e < E; e += kLanes) {
     s.count[e] = run[e];
@@ -414,16 +416,31 @@ __global__ __launch_bounds__(kLanes) void route_rows_kernel(const float* __restr
                                                             const int64_t* __restrict__ ids,
                                                             const uint32_t* __restrict__ rank_in_block,
                                                             const int32_t* __restrict__ block_hist, int T, int E, int K,
-                                                            int chunks, PlanOut p, StatsOut st) {
+                                                            int chunks, PlanOut p, StatsOut st, int nb, Observe observe, int groups) {
   extern __shared__ int32_t lds[];
-  __shared__ float red_sh[4];
+  __shared__ float red_sh[2 * kLanes / kWave];
   const LayoutLds s(lds, E);
   const int tid = threadIdx.x;
+  // Behind the plan's workgroups: one for the statistics' sums, the histogram's.  Both are chains of latency that nothing here waits for: at 3000 tokens
+  // of 64 experts the sums made the first workgroup the last to end (16 us for 7), and a launch of its own for the histogram took 10 more; together
+  // 395 -> 381 us of a training step of 1024 x 64 x 512.
+  int extra = static_cast<int>(blockIdx.x) - nb;
+  if (extra >= 0 && (st.valid_counts || st.f)) {
+    if (extra == 0) {
+      finish_stats<32>(st, E, nb, red_sh);
+      return;
+    }
+    --extra;
+  }
+  if (extra >= 0) {
+    observe_part<kLanes>(observe, extra % groups, extra / groups, reinterpret_cast<unsigned*>(lds), red_sh);
+    return;
+  }
   for (int e = tid; e < E; e += kLanes) s.count[e] = s.before[e] = 0;
   __syncthreads();
   // every expert's slots in all workgroups and in those before this one, a slice of the histograms
   // per lane, sixteen loads in flight
-  const int parts = max(1, kLanes / E), nb = gridDim.x, per = (nb + parts - 1) / parts;
+  const int parts = max(1, kLanes / E), per = (nb + parts - 1) / parts;
   constexpr int kBatch = 16;
   for (int idx = tid; idx < E * parts; idx += kLanes) {
     const int e = idx % E, b0 = (idx / E) * per, b1 = min(nb, b0 + per);
@@ -443,10 +460,7 @@ __global__ __launch_bounds__(kLanes) void route_rows_kernel(const float* __restr
   }
   __syncthreads();
   plan_layout(s, p, blockIdx.x == 0);
-  if (blockIdx.x == 0) {
-    write_lists(s, p, E);
-    if (st.valid_counts || st.f) finish_stats(st, E, gridDim.x, red_sh);
-  }
+  if (blockIdx.x == 0) write_lists(s, p, E);
   const int per_block = chunks * (kLanes / 16) * K;
   const int first = blockIdx.x * per_block, last = min(T * K, first + per_block);
   for (int slot = first + tid; slot < last; slot += kLanes) {
@@ -507,7 +521,7 @@ static int route_plan(const float* partial, int splits, const float* logit_bias,
                                 int32_t* slot_of_row, int32_t* token_of_row, float* row_scale, int64_t row_capacity,
                                 int32_t* tile_expert, int32_t* tile_row0, int32_t* num_tiles, int64_t tile_capacity,
                                 void* workspace, const StatsOut& st, void* stream, const GateIn& gate = {},
-                                int x_dtype = MI355_F32) {
+                                int x_dtype = MI355_F32, int64_t* histogram = nullptr, int64_t B = 1) {
   MI355_REQUIRE(T >= 1 && T < (1ll << 26) && E >= 1 && K >= 1 && K <= E && T * K < (1ll << 30),
                 "route_plan: bad shape T=%lld E=%lld K=%lld", (long long)T, (long long)E, (long long)K);
   if (!select_row_covers(E, K, num_groups, MI355_SELECT_TOPK))
@@ -558,13 +572,19 @@ static int route_plan(const float* partial, int splits, const float* logit_bias,
     });
   });
   if (int rc = check_launch("route_rank")) return rc;
+  Observe o{st.scores, st.cutoff, expert_bias, st.padding, reinterpret_cast<unsigned long long*>(histogram), (int)T, (int)E, (int)B, 0, 0};
+  unsigned groups = 0, token_chunks = 0;
+  if (histogram && blocks > 1) observe_shape(T, E, B, o.eg, o.tokens, groups, token_chunks);
   if (blocks > 1) {
+    const size_t bytes = std::max<size_t>(layout_words((int)E), (size_t)o.eg * o.B) * sizeof(int32_t);
     with_lanes(T, E, [&](auto lanes) {
-      hipLaunchKernelGGL(route_rows_kernel<decltype(lanes)::value>, dim3(blocks), dim3(lanes), layout_words((int)E) * sizeof(int32_t),
-                         s, weights, ids, rank, hist, (int)T, (int)E, (int)K, chunks, p, st);
+      hipLaunchKernelGGL(route_rows_kernel<decltype(lanes)::value>, dim3(blocks + (stats ? 1 : 0) + groups * token_chunks), dim3(lanes), bytes,
+                         s, weights, ids, rank, hist, (int)T, (int)E, (int)K, chunks, p, st, blocks, o, (int)groups);
     });
-    return check_launch("route_rows");
+    if (int rc = check_launch("route_rows")) return rc;
   }
+  if (histogram && groups == 0)
+    return mi355_quantile_observe(st.scores, st.cutoff, expert_bias, st.padding, histogram, T, E, B, stream);
   return MI355_OK;
 }
 
@@ -582,6 +602,32 @@ extern "C" int mi355_route_plan(const float* partial, int splits, const float* l
                     tile_capacity, workspace, StatsOut{}, stream);
 }
 
+extern "C" int mi355_route_plan_observe(
+    const float* partial, int splits, const float* logit_bias, float* logits, const float* expert_bias, int64_t T,
+    int64_t E, int64_t K, int score_func, int route_norm, float route_scale, int num_groups, int num_limited,
+    float* weights, int64_t* ids, int64_t lo, int64_t hi, int64_t align, int64_t tile_m, int32_t* counts_E,
+    int32_t* seg_offsets, int32_t* seg_counts, int32_t* row_of_slot, int32_t* slot_of_row, int32_t* token_of_row,
+    float* row_scale, int64_t row_capacity, int32_t* tile_expert, int32_t* tile_row0, int32_t* num_tiles,
+    int64_t tile_capacity, void* workspace, const uint8_t* padding_mask_T, int32_t* valid_counts_E, float* scores_TE,
+    float* cutoff_T, float* aux_f_E, float* aux_scale, void* aux_acc, int aux_acc_dtype, const float* aux_denominator, float aux_coeff,
+    void* stats_workspace, int64_t* histogram_EB, int64_t B, void* stream) {
+  MI355_REQUIRE(!histogram_EB || (scores_TE && cutoff_T && expert_bias && B >= 1 && B < (1 << 24)),
+                "route_plan_observe: the histogram needs scores, cutoff, the expert bias and 1 <= B < 2^24 (%lld)", (long long)B);
+  MI355_REQUIRE(!cutoff_T || K < E, "route_plan_observe: top_k (%lld) must leave a (K+1)-th expert of %lld", (long long)K,
+                (long long)E);
+  MI355_REQUIRE(!aux_f_E || (aux_scale && aux_denominator), "route_plan_observe: the loss needs scale and denominator");
+  MI355_REQUIRE(!aux_acc || aux_acc_dtype == MI355_F32 || aux_acc_dtype == MI355_BF16, "route_plan_observe: aux_acc is fp32 or bf16");
+  MI355_REQUIRE((!aux_f_E && !valid_counts_E) || stats_workspace, "route_plan_observe: workspace required");
+  int32_t* block_valid = static_cast<int32_t*>(stats_workspace);
+  float* block_share = block_valid ? reinterpret_cast<float*>(block_valid + (T >= 1 ? route_blocks(T, E) : 0) * E) : nullptr;
+  const StatsOut st{padding_mask_T, valid_counts_E, scores_TE, cutoff_T, aux_f_E, aux_scale, aux_acc, aux_acc_dtype, aux_denominator,
+                    aux_coeff, block_valid, block_share};
+  return route_plan(partial, splits, logit_bias, logits, expert_bias, T, E, K, score_func, route_norm, route_scale,
+                    num_groups, num_limited, weights, ids, lo, hi, align, tile_m, counts_E, seg_offsets, seg_counts,
+                    row_of_slot, slot_of_row, token_of_row, row_scale, row_capacity, tile_expert, tile_row0, num_tiles,
+                    tile_capacity, workspace, st, stream, {}, MI355_F32, histogram_EB, B);
+}
+
 extern "C" int mi355_route_plan_stats(
     const float* partial, int splits, const float* logit_bias, float* logits, const float* expert_bias, int64_t T,
     int64_t E, int64_t K, int score_func, int route_norm, float route_scale, int num_groups, int num_limited,
@@ -591,19 +637,11 @@ extern "C" int mi355_route_plan_stats(
     int64_t tile_capacity, void* workspace, const uint8_t* padding_mask_T, int32_t* valid_counts_E, float* scores_TE,
     float* cutoff_T, float* aux_f_E, float* aux_scale, void* aux_acc, int aux_acc_dtype, const float* aux_denominator, float aux_coeff,
     void* stats_workspace, void* stream) {
-  MI355_REQUIRE(!cutoff_T || K < E, "route_plan_stats: top_k (%lld) must leave a (K+1)-th expert of %lld", (long long)K,
-                (long long)E);
-  MI355_REQUIRE(!aux_f_E || (aux_scale && aux_denominator), "route_plan_stats: the loss needs scale and denominator");
-  MI355_REQUIRE(!aux_acc || aux_acc_dtype == MI355_F32 || aux_acc_dtype == MI355_BF16, "route_plan_stats: aux_acc is fp32 or bf16");
-  MI355_REQUIRE((!aux_f_E && !valid_counts_E) || stats_workspace, "route_plan_stats: workspace required");
-  int32_t* block_valid = static_cast<int32_t*>(stats_workspace);
-  float* block_share = block_valid ? reinterpret_cast<float*>(block_valid + (T >= 1 ? route_blocks(T, E) : 0) * E) : nullptr;
-  const StatsOut st{padding_mask_T, valid_counts_E, scores_TE, cutoff_T, aux_f_E, aux_scale, aux_acc, aux_acc_dtype, aux_denominator,
-                    aux_coeff, block_valid, block_share};
-  return route_plan(partial, splits, logit_bias, logits, expert_bias, T, E, K, score_func, route_norm, route_scale,
-                    num_groups, num_limited, weights, ids, lo, hi, align, tile_m, counts_E, seg_offsets, seg_counts,
-                    row_of_slot, slot_of_row, token_of_row, row_scale, row_capacity, tile_expert, tile_row0, num_tiles,
-                    tile_capacity, workspace, st, stream);
+  return mi355_route_plan_observe(partial, splits, logit_bias, logits, expert_bias, T, E, K, score_func, route_norm, route_scale, num_groups,
+                                  num_limited, weights, ids, lo, hi, align, tile_m, counts_E, seg_offsets, seg_counts, row_of_slot,
+                                  slot_of_row, token_of_row, row_scale, row_capacity, tile_expert, tile_row0, num_tiles, tile_capacity,
+                                  workspace, padding_mask_T, valid_counts_E, scores_TE, cutoff_T, aux_f_E, aux_scale, aux_acc,
+                                  aux_acc_dtype, aux_denominator, aux_coeff, stats_workspace, nullptr, 1, stream);
 }
 
 // whole chunks of 32 tokens, one to a workgroup, and one slice of the contraction: the bits of the two calls

@@ -343,17 +343,19 @@ std::tuple<Tensor, Tensor, Tensor> block_forward(const Block& b, const Stats& st
              k.token_of_row, save && (b.folded || b.gather) ? k.row_scale : nullptr, b.R, k.tile_expert, k.tile_row0,
              k.num_tiles, b.tile_cap, plan_work, padding, stats ? counts.data_ptr<int32_t>() : nullptr, scores, cutoff, k.aux_f,
              k.aux_scale, ptr(st.aux_acc), st.aux_acc.defined() ? dtype_code(st.aux_acc) : MI355_F32,
-             fptr(st.aux_denominator), (float)st.aux_coeff, stats_work, L.stream);
+             fptr(st.aux_denominator), (float)st.aux_coeff);
   };
-  check(one_launch ? plan(mi355_route_gate_plan_stats, ptr(b.x), b.dt, fptr(b.gate_w), b.D, fptr(gate_b),
+  int64_t* histogram = st.histogram.defined() ? st.histogram.data_ptr<int64_t>() : nullptr;
+  const int64_t bins = histogram ? st.histogram.size(1) : 1;
+  auto with_gate = [&](auto... a) { return mi355_route_gate_plan_stats(a..., stats_work, L.stream); };
+  auto of_logits = [&](auto... a) { return mi355_route_plan_observe(a..., stats_work, histogram, bins, L.stream); };
+  check(one_launch ? plan(with_gate, ptr(b.x), b.dt, fptr(b.gate_w), b.D, fptr(gate_b),
                           save ? k.logits : nullptr)
-                   : plan(mi355_route_plan_stats, partial, b.splits > 1 ? b.splits : 1, fptr(gate_b),
+                   : plan(of_logits, partial, b.splits > 1 ? b.splits : 1, fptr(gate_b),
                           save && b.splits > 1 ? k.logits : nullptr),
         "route_plan");
-  if (st.histogram.defined())
-    check(mi355_quantile_observe(scores, cutoff, fptr(expert_b), padding, st.histogram.data_ptr<int64_t>(), b.T, b.E,
-                                 st.histogram.size(1), L.stream),
-          "quantile_observe");
+  if (histogram && one_launch)
+    check(mi355_quantile_observe(scores, cutoff, fptr(expert_b), padding, histogram, b.T, b.E, bins, L.stream), "quantile_observe");
 
   // routed experts
   if (!b.folded && !b.gather)
