@@ -48,3 +48,37 @@ def test_gate_backward_with_the_row_sum(T, D, E, K, extra):
         assert torch.equal(a, b)
     assert lib.mi355_router_gate_sum_bwd_covers(1, 0, D, E, 17) == 0 and lib.mi355_router_gate_sum_bwd_covers(1, 0, D, 60, K) == 0
     assert lib.mi355_router_gate_sum_bwd_covers(0, 0, D, E, K) == 0
+
+
+# more than 32 experts of no matrix tile: the fewest and the most, one part of 32 tokens and 256 columns and a little more, rows that are not whole
+# 16-byte pieces apart, on either side of 6 Mi elements, where strided products go on; 64 experts in fp32
+@pytest.mark.parametrize("T,D,E,dtype", [(1, 4, 36, "bf16"), (33, 260, 60, "bf16"), (300, 512, 60, "fp32"), (257, 516, 44, "bf16"), (6144, 1024, 60, "bf16"),
+                                         (6145, 1024, 60, "bf16"), (700, 448, 64, "fp32"), (64, 256, 62, "bf16")])
+@pytest.mark.parametrize("addend", [False, True])
+def test_gate_backward_between_the_tiles(T, D, E, dtype, addend):
+    from torchllmtuner_amd import _lib
+
+    print(f"gate backward T={T} D={D} E={E} {dtype} addend={addend}", flush=True)
+    lib, g = _lib.load(), torch.Generator(device=DEV).manual_seed(T + E)
+    dt = torch.bfloat16 if dtype == "bf16" else torch.float32
+    x, add = (torch.randn(T, D, generator=g, device=DEV).to(dt) for _ in "xa")
+    dl, w = torch.randn(T, E, generator=g, device=DEV) * 0.01, torch.randn(E, D, generator=g, device=DEV) * 0.02
+    dl[T // 2, E - 1] = float("inf")  # reaches one row of dx and one of dW, and nothing else
+    work = torch.empty(max(16, lib.mi355_router_gate_bwd_workspace_bytes(T, D, E)), dtype=torch.uint8, device=DEV)
+    dx, dw = torch.empty_like(x), torch.empty_like(w)
+    assert lib.mi355_router_gate_add_bwd(dl.data_ptr(), x.data_ptr(), int(dtype == "bf16"), w.data_ptr(), 0, None,
+                                         add.data_ptr() if addend else None, dx.data_ptr(), dw.data_ptr(), work.data_ptr(), T, D, E,
+                                         torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    want_x, want_w = dl.double() @ w.double(), dl.double().T @ x.double()
+    # fp32 products and sums (n + 1 roundings of at most 2^-24 of the terms' sizes), then, of bf16 tokens, one rounding, and another behind the addend
+    size_x, size_w = (dl.abs().double() @ w.abs().double()), dl.abs().double().T @ x.abs().double()
+    unit = 2.0 ** -8 if dtype == "bf16" else 2.0 ** -24
+    bound = (E + 1) * 2.0 ** -24 * size_x + unit * want_x.abs() * (1 + unit)
+    if addend:
+        want_x = want_x + add.double()
+        bound = bound * (1 + unit) + unit * want_x.abs()
+    for got, want, limit in ((dx, want_x, bound), (dw, want_w, (T + 1) * 2.0 ** -24 * size_w)):
+        finite = want.isfinite()
+        assert torch.equal(got.isfinite(), finite)
+        assert bool(((got.double() - want).abs() <= limit)[finite].all())

@@ -66,6 +66,7 @@ bool router_x3_ok(int x_dtype, int w_dtype, int64_t D, int64_t E);
 int64_t router_x3_bwd_workspace(int64_t T, int64_t D, int64_t E);
 // Backward for few experts, fp32 weights, D a multiple of four: both gradients in one launch (dx, dw: null = skip).
 bool router_few_ok(int x_dtype, int w_dtype, int64_t D, int64_t E);
+bool router_few_bwd_ok(int x_dtype, int w_dtype, int64_t T, int64_t D, int64_t E);
 int64_t router_few_bwd_workspace(int64_t T, int64_t D, int64_t E);
 int router_few_bwd(const float* dlogits, const void* x, int x_dtype, const float* w, const RowSum& sum, void* dx, float* dw,
                    void* workspace, int64_t T, int64_t D, int64_t E, hipStream_t s);

@@ -509,7 +509,7 @@ extern "C" int64_t mi355_router_gate_bwd_workspace_bytes(int64_t T, int64_t D, i
   const int s = gate_bwd_ksplit(T, D, E);
   const int64_t strided = s > 1 ? (int64_t)s * E * D * 4 : 0;
   const int64_t x3 = router_x3_ok(MI355_BF16, MI355_F32, D, E) ? router_x3_bwd_workspace(T, D, E) : 0;
-  const int64_t few = router_few_ok(MI355_F32, MI355_F32, D, E) ? router_few_bwd_workspace(T, D, E) : 0;
+  const int64_t few = router_few_bwd_ok(MI355_F32, MI355_F32, T, D, E) ? router_few_bwd_workspace(T, D, E) : 0;
   return std::max({strided, x3, few});
 }
 
@@ -526,7 +526,7 @@ extern "C" int mi355_router_gate_add_bwd(const float* dlogits, const void* x, in
     return router_x3_bwd(dlogits, x, static_cast<const float*>(w), pieces, RowSum{addend}, dx, static_cast<float*>(dw),
                          workspace, T, D, E, s);
   }
-  if (vec && T > 0 && router_few_ok(x_dtype, w_dtype, D, E) && (dx || dw)) {
+  if (vec && T > 0 && router_few_bwd_ok(x_dtype, w_dtype, T, D, E) && (dx || dw)) {
     MI355_REQUIRE(dlogits && w && (x || !dw), "router_gate_bwd: null pointer");
     return router_few_bwd(dlogits, x, x_dtype, static_cast<const float*>(w), RowSum{addend}, dx, static_cast<float*>(dw), workspace,
                           T, D, E, s);

@@ -1,4 +1,4 @@
-// Both gradients of a router gate of up to 32 experts, as parts of launches: by themselves (router_gemm.hip), or the weight's beside
+// Both gradients of a router gate of up to 32 experts (by themselves 64), as parts of launches: by themselves (router_gemm.hip), or the weight's beside
 // the experts' products (grouped_any.hip) and the input's together with the sum over a token's rows.
 //   dW = dlogits^T . x and dx = dlogits . W read or write a (T, D) matrix against a handful of rows, too thin for
 // matrix tiles, and the vector units keep up with memory.  A thread owns four columns.  dW parts: eight experts,

@@ -504,7 +504,7 @@ struct GateDx {
 
 // TW tokens a wave.  With the rows in front (ROWS) two: the launch is the last of a backward, bound by the latency of its row
 // reads, and wants many waves (1531 tokens of 4 x 320, 16 experts: 18.0 us with eight a wave, 6.6 with two; 512 fp32 of 2 x 256 7.6, 4.0).
-template <typename TX, bool ROWS, int TW>
+template <typename TX, bool ROWS, int TW, int PITCH = S_MAX_E>  // PITCH: experts at most
 __device__ __forceinline__ void gate_dx_part(const float* __restrict__ dlogits, const float* __restrict__ w,
                                              const GateDx<TX>& g, TX* __restrict__ dx, int T, int D, int E, int part,
                                              float* lds) {
@@ -513,7 +513,6 @@ __device__ __forceinline__ void gate_dx_part(const float* __restrict__ dlogits, 
   const int col_blocks = (D + S_COLS - 1) / S_COLS;
   const int cb = part % col_blocks, t0 = part / col_blocks * TOK;
   const int tokens = min(TOK, T - t0), n = cb * S_COLS + lane * 4;
-  constexpr int PITCH = S_MAX_E;
   for (int i = tid; i < TOK * PITCH; i += 256) {
     const int t = i / PITCH, e = i % PITCH;
     lds[i] = t < tokens && e < E ? dlogits[static_cast<int64_t>(t0 + t) * E + e] : 0.0f;
@@ -583,14 +582,15 @@ __device__ __forceinline__ void gate_dx_part(const float* __restrict__ dlogits, 
 
 constexpr int kRowsTok = 8;  // tokens of a dx part with the rows in front
 
-template <typename TX, bool ROWS>
+template <typename TX, bool ROWS, int MAX_E = S_MAX_E>
 __global__ __launch_bounds__(256) void gate_bwd_few_kernel(GateDw dw, const float* __restrict__ dlogits,
                                                            const float* __restrict__ w, GateDx<TX> g, TX* __restrict__ dx,
                                                            int T, int D, int E, int dw_parts) {
   __shared__ __attribute__((aligned(16))) float lds[kGateDwLds];
+  static_assert(S_TOK * MAX_E <= kGateDwLds, "a dx part's gradients");
   const int block = blockIdx.x;
   if (block < dw_parts) gate_dw_part<TX>(dw, block, lds);
-  else gate_dx_part<TX, ROWS, (ROWS ? kRowsTok : S_TOK) / 4>(dlogits, w, g, dx, T, D, E, block - dw_parts, lds);
+  else gate_dx_part<TX, ROWS, (ROWS ? kRowsTok : S_TOK) / 4, MAX_E>(dlogits, w, g, dx, T, D, E, block - dw_parts, lds);
 }
 
 // dx with the sum over the token's rows, and beside it the sum of dW's slices, in their order: the two ends of a backward
@@ -663,6 +663,15 @@ int dw_splits(int64_t T, int64_t D, int64_t E) {
 bool router_few_ok(int x_dtype, int w_dtype, int64_t D, int64_t E) {
   return w_dtype == MI355_F32 && (x_dtype == MI355_BF16 || x_dtype == MI355_F32) && D % 4 == 0 && D >= 4 && E <= S_MAX_E;
 }
+// ... without the rows in front, up to twice as many experts (60, which no matrix tile divides), while the tokens are few: strided products took three launches,
+// and beside the experts' weight gradients each waits for a CU.  Alone, us, those / these: 300 x 512, 60 experts 17.3 / 13.7, 1000 x 1024 21.9 / 15.6,
+// 2229 x 768 33.8 / 22.3, 3000 x 512, 36 experts 22.9 / 16.0, fp32 tokens, 64 experts 25.3 / 19.5; but 12000 x 1024 66 / 66, 8000 x 2048 79 / 86 (W is read once for
+// 32 tokens, x once for eight experts).  A training step: 2229 tokens of 60 experts of 768 x 384, eight each, 288 / 271, 3000 of 1024 x 512 377 / 369,
+// 5000 of 1280 x 640 (past the line) 596 / 597.  dx is the same sum in the same order, dW's error against fp64 is 0.3-0.95 times theirs.
+bool router_few_bwd_ok(int x_dtype, int w_dtype, int64_t T, int64_t D, int64_t E) {
+  return router_few_ok(x_dtype, w_dtype, D, E) ||
+         (router_few_ok(x_dtype, w_dtype, D, S_MAX_E) && E <= 2 * S_MAX_E && E % 4 == 0 && T * D <= (int64_t{6} << 20));
+}
 int64_t router_few_bwd_workspace(int64_t T, int64_t D, int64_t E) { return gate_dw_splits(T, D, E) * E * D * 4; }
 
 int router_few_bwd(const float* dlogits, const void* x, int x_dtype, const float* w, const RowSum& sum, void* dx, float* dw,
@@ -681,7 +690,8 @@ int router_few_bwd(const float* dlogits, const void* x, int x_dtype, const float
       hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, s, job, dlogits, w, g, static_cast<TX*>(dx), (int)T, (int)D,
                          (int)E, (int)dw_parts);
     };
-    if constexpr (sizeof(TX) == 2) run(sum.rows ? gate_bwd_few_kernel<TX, true> : gate_bwd_few_kernel<TX, false>);
+    if (E > S_MAX_E) run(gate_bwd_few_kernel<TX, false, 2 * S_MAX_E>);
+    else if constexpr (sizeof(TX) == 2) run(sum.rows ? gate_bwd_few_kernel<TX, true> : gate_bwd_few_kernel<TX, false>);
     else run(gate_bwd_few_kernel<TX, false>);  // (fp32 tokens: the experts' launches take the parts along)
   };
   if (x_dtype == MI355_BF16) launch(static_cast<const uint16_t*>(x));
