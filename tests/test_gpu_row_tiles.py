@@ -103,6 +103,45 @@ def test_rows_of_other_experts_stay_out_of_a_weight_gradient(counts):
         start += n
 
 
+# token matrices of 4 GiB less 256 and less 128 bytes, the largest that 32-bit byte offsets reach (rows are whole 128-byte lines)
+@pytest.mark.parametrize("T,D", [(5592405, 384), (1082401, 1984)])
+def test_rows_past_a_segment_of_the_largest_gathered_matrix(T, D):
+    """No token's row stands in for the rows past an expert's last one, not even the matrix's first, which is not finite here."""
+    from torchllmtuner_amd import _lib, ops
+
+    assert T * D * 2 in (2 ** 32 - 256, 2 ** 32 - 128)
+    print(f"gathered matrix {T} x {D}", flush=True)
+    lib, Fd, counts = _lib.load(), 384, (1, 63, 64, 65, 130)
+    g = torch.Generator(device=DEV).manual_seed(D)
+    El, R = len(counts), sum(counts)
+    plan = ops.permute_plan(torch.repeat_interleave(torch.arange(El), torch.tensor(counts))[:, None].to(DEV), El)
+    tok = torch.randint(1, T, (R,), generator=g, device=DEV, dtype=torch.int32)
+    tok[:1], tok[-1:] = T - 1, T - 1
+    normal = lambda *s: torch.randn(*s, generator=g, device=DEV).bfloat16()
+    x = torch.zeros(T, D, dtype=torch.bfloat16, device=DEV)  # the tokens, and the output gradient of dW2
+    x[tok.long()] = normal(R, D)
+    x[0] = float("nan")
+    dgate, dup, hs = (normal(R, Fd) for _ in "gus")
+    dw1, dw3, dw2 = (torch.empty(El, *s, dtype=torch.bfloat16, device=DEV) for s in ((Fd, D), (Fd, D), (D, Fd)))
+    w, gate, dots = normal(El, Fd, D), normal(R, Fd), torch.empty(R, 4, device=DEV)
+    scale = torch.ones(R, device=DEV)
+    at = lambda t: t.data_ptr()
+    for stage in (16, 32, 64):  # dW2, dW1, dW3
+        assert lib.mi355_grouped_swiglu_combine_bwd(
+            at(x), at(x), at(tok), T, at(scale), at(w), at(w), at(w), at(gate), at(gate), 1, at(plan.seg_offsets), at(plan.seg_counts),
+            at(plan.tile_expert), at(plan.tile_row0), at(plan.num_tiles), plan.tile_capacity, at(dgate), at(dup), at(hs), at(dots), None,
+            at(dw1), at(dw3), at(dw2), El, D, Fd, R, stage, torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    start = 0
+    for e, n in enumerate(counts):
+        r = slice(start, start + n)
+        start += n
+        xe = x[tok[r].long()].float()
+        for got, want in ((dw1[e], dgate[r].float().T @ xe), (dw3[e], dup[r].float().T @ xe), (dw2[e], xe.T @ hs[r].float())):
+            # one bf16 rounding of an fp32 sum
+            assert bool(got.isfinite().all()) and row_errors(got.flatten()[None], want.flatten()[None]) < 2.0 ** -8
+
+
 # rows an expert on either side of the 16 a pass takes; contractions of six steps (one or two a wave) and seven; weights past the
 # memory-side cache, read with the non-temporal hint, of experts with a few rows (El = 40) and with one row tile (the last)
 @pytest.mark.parametrize("counts,D,Fd", [((16, 0, 17, 1, 33, 5, 15, 2), 384, 448), ((40, 3, 1, 0, 0, 9), 448, 384), ((1,), 384, 640), ((60,), 1024, 512),

@@ -792,9 +792,9 @@ __global__ __launch_bounds__(NT, 2) void wgrad_kernel(WgradArgs p) {
   [[maybe_unused]] uint32_t i_to = 0, i_from = 0;
   const uint32_t epi = 2 * STAGE_BYTES + wave * 4096u;
   const uint32_t ldA = static_cast<uint32_t>(M) * 2u, ldB = static_cast<uint32_t>(N) * 2u;  // bytes
-  // bytes of the gathered operand; an offset past them for rows past the segment (which a matrix of almost 4 GiB does not leave: its first row then)
+  // bytes of the gathered operand; an offset past them for rows past the segment (whole 128-byte lines below 4 GiB: no operand has it, nor has one from a later column on)
   const uint64_t src_bytes = static_cast<uint64_t>(p.src_rows) * (GATHER ? ldB : ldA);
-  const uint32_t nowhere = src_bytes > 0xfffffe00u ? 0u : 0xfffffe00u;
+  constexpr uint32_t kNowhere = 0xffffff80u;
   int fm0, fn0;
   auto set_bytes = [&]() {
     // (a step of 64 rows ends before the next row's first column)
@@ -835,7 +835,7 @@ __global__ __launch_bounds__(NT, 2) void wgrad_kernel(WgradArgs p) {
     if constexpr (INDEXED) {
       const int r = min(max(static_cast<int>(voffG[i]), 0), p.src_rows - 1);
       voffG[i] = static_cast<uint32_t>(r) * (GATHER ? ldB : ldA) + cc16;
-      if (left < BK && 2 * wave + (opaque(lane) >> 5) + 16 * i >= left) voffG[i] = nowhere + cc16;
+      if (left < BK && 2 * wave + (opaque(lane) >> 5) + 16 * i >= left) voffG[i] = kNowhere;
     }
   };
   auto req = [&](bool is_a, int i) {
