@@ -338,6 +338,52 @@ def test_route_plan_equals_selection_and_plan(T, E, K, local, align, groups):
         assert torch.equal(a, b), name
 
 
+# the statistics' sums take 8 * (512 // E) workgroups of 32 tokens at a time, or 8 * (1024 // E) of 64 above 8192 tokens (7000 past 128 experts): whole rounds of
+# them and one workgroup more, the fewest workgroups, experts that do not divide the lanes, workgroups of several chunks of tokens
+@pytest.mark.parametrize("T,E,K", [(512, 256, 2), (513, 256, 2), (2048, 60, 4), (2049, 60, 4), (65, 1, 1), (8192, 128, 8), (8193, 128, 8), (7001, 256, 3), (16449, 5, 2),
+                                   (20000, 100, 16)])
+@pytest.mark.parametrize("counts,loss", [(True, True), (True, False), (False, True)])
+def test_statistics_of_many_workgroups(T, E, K, counts, loss):
+    """Valid counts, and the balance loss of them and of the tokens' score shares in fp64."""
+    from torchllmtuner_amd import _lib, ops
+
+    print(f"route plan statistics T={T} E={E} K={K} counts={counts} loss={loss}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(T + E)
+    logits = torch.randn(T, E, generator=g, device=DEV)
+    padding = torch.rand(T, generator=g, device=DEV) < 0.2
+    denominator = torch.tensor([float(T)], device=DEV)
+    i32 = lambda n: torch.full((n,), -7, dtype=torch.int32, device=DEV)
+    cap = T * K // ops.TILE_M + E + 1
+    w, ids = torch.empty(T, K, device=DEV), torch.empty(T, K, dtype=torch.int64, device=DEV)
+    total, offsets, seg_counts, ros, sor, tor, te, tr, nt, valid = (i32(n) for n in (E, E + 1, 2 * E, T * K, T * K, T * K, cap, cap, 1, E))
+    f, scale, acc = (torch.full((n,), v, device=DEV) for n, v in ((E, float("nan")), (1, float("nan")), (1, 0.5)))
+    lib = _lib.load()
+    work, stats = (torch.empty(max(1, n), dtype=torch.uint8, device=DEV)
+                   for n in (lib.mi355_route_plan_workspace_bytes(T, K, E), lib.mi355_route_stats_workspace_bytes(T, E)))
+    at = lambda t, wanted=True: t.data_ptr() if wanted else None
+    _lib.check(lib.mi355_route_plan_stats(
+        at(logits), 1, None, None, None, T, E, K, 1, 0, 1.0, 0, 0, at(w), at(ids), 0, E, 1, ops.TILE_M, at(total), at(offsets),
+        at(seg_counts), at(ros), at(sor), at(tor), None, T * K, at(te), at(tr), at(nt), cap, at(work), at(padding), at(valid, counts), None, None,
+        at(f, loss), at(scale, loss), at(acc, loss), 0, at(denominator), 2.0, at(stats), torch.cuda.current_stream().cuda_stream),
+        "route_plan_stats")
+    assert torch.equal(total.long(), torch.bincount(ids.flatten(), minlength=E))
+    want = torch.bincount(ids[~padding].flatten(), minlength=E)
+    assert torch.equal(valid.long(), want) if counts else bool((valid == -7).all())
+    if not loss:
+        assert bool(f.isnan().all()) and float(acc) == 0.5
+        return
+    scores = logits.double().softmax(1)
+    p = (scores / scores.sum(1, keepdim=True))[~padding].sum(0)
+    want_f = want.double() * (E / want.sum().clamp(min=1e-12))
+    want_loss = float((want_f * p).sum()) / T
+    assert abs(float(scale) * T / 2.0 - 1.0) <= 2.0 ** -23
+    # (one rounding; of f two.  Of the loss: each share an exponential, sums of up to 256 terms by fours and their quotients, 2^-20; then sums of at most T / 4096 + 2
+    # tokens of a wave, 16 waves, 256 workgroups and 8 steps of a tree over the experts, products, and the sum with what was there)
+    assert float((f.double() - want_f).abs().max()) <= 2.0 ** -22 * float(want_f.max())
+    bound = (2.0 ** -20 + (T / 4096 + 2 + 16 + 256 + 8 + 4) * 2.0 ** -24) * want_loss + 2.0 ** -24 * (0.5 + want_loss)
+    assert abs(float(acc) - 0.5 - want_loss) <= bound
+
+
 def test_default_overlap_adds_the_input_gradients_in_another_order_than_the_stages():
     """With a shared expert beside the routed path, as by default, the engine adds the stages' three bf16 input
     gradients as (routed + gate) + shared; the operator as (routed + shared) + gate, whatever the overlap.  All

@@ -162,31 +162,50 @@ __device__ __forceinline__ void place_slot(const LayoutLds& s, const PlanOut& p,
   p.row_of_slot[slot] = row;
 }
 
-// Sums the workgroups' valid counts and score shares (in order), and the loss from them; one workgroup.
-template <int kBatch>  // loads of either kind in flight
-__device__ void finish_stats(const StatsOut& st, int E, int nb, float* red) {
+// Every expert's valid slots and score shares of all workgroups, the shares in the workgroups' order; lane e < E has expert e's.  One workgroup of kLanes;
+// stage: kStatsWords words of LDS.  All lanes request what they find, a run of workgroups at a time, and hand the shares on through LDS to the
+// lane that adds them.  With 32 of either kind in flight in that lane's own registers the kernel had 198 of them at 512 lanes and spilled 70 at 1024 (50 and none
+// here), and all its workgroups were one to a CU: the launch at 3000 and 12000 tokens of 64 experts 10.0 / 7.9 us, 59.6 / 13.2.
+constexpr int kStatsBatch = 8;
+template <int kLanes>
+constexpr int kStatsWords = kLanes * kStatsBatch;
+template <int kLanes>
+__device__ __forceinline__ void sum_blocks(const StatsOut& st, int E, int nb, int32_t* stage, int& valid, float& share) {
+  const int tid = threadIdx.x, parts = kLanes / E, run = parts * E;  // E <= 256; lanes at work
+  float* shares = reinterpret_cast<float*>(stage);
+  int mine = 0;  // of expert tid % E
+  for (int b0 = 0; b0 < nb; b0 += parts * kStatsBatch) {
+    int v[kStatsBatch];
+    float p[kStatsBatch];
+#pragma unroll
+    for (int i = 0; i < kStatsBatch; ++i) {
+      const int at = (b0 + i * parts) * E + tid;
+      const bool in = tid < run && at < nb * E;
+      v[i] = in ? st.block_valid[at] : 0;
+      p[i] = in && st.f ? st.block_share[at] : 0.0f;
+    }
+#pragma unroll
+    for (int i = 0; i < kStatsBatch; ++i) {
+      mine += v[i];
+      if (tid < run) shares[i * run + tid] = p[i];
+    }
+    __syncthreads();
+    if (st.f && tid < E)
+#pragma unroll 8
+      for (int j = 0; j < min(parts * kStatsBatch, nb - b0); ++j) share += shares[j * E + tid];
+    __syncthreads();
+  }
+  if (tid < run) stage[tid] = mine;
+  __syncthreads();
+  if (tid < E)
+    for (int q = 0; q < parts; ++q) valid += stage[q * E + tid];
+}
+
+// Valid counts, and the loss from them and the score shares; one workgroup whose lane e < E has expert e's.
+__device__ void finish_stats(const StatsOut& st, int E, int valid, float share, float* red) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   constexpr float kEps = 1e-12f;  // F.normalize's clamp
-  int valid = 0;
-  float share = 0.0f;
-  if (tid < E) {
-    for (int b0 = 0; b0 < nb; b0 += kBatch) {
-      int v[kBatch];
-      float p[kBatch];
-#pragma unroll
-      for (int i = 0; i < kBatch; ++i) {
-        const int64_t at = static_cast<int64_t>(b0 + i) * E + tid;
-        v[i] = b0 + i < nb ? st.block_valid[at] : 0;
-        p[i] = st.f && b0 + i < nb ? st.block_share[at] : 0.0f;
-      }
-#pragma unroll
-      for (int i = 0; i < kBatch; ++i) {
-        valid += v[i];
-        share += p[i];
-      }
-    }
-    if (st.valid_counts) st.valid_counts[tid] = valid;
-  }
+  if (st.valid_counts && tid < E) st.valid_counts[tid] = valid;
   if (!st.f) return;
   // E <= 256: four waves hold everything
   auto total = [&](float v) {
@@ -399,7 +418,8 @@ __global__ __launch_bounds__(kLanes) void route_rank_kernel(
     for (int e = tid; e < E; e += kLanes) block_hist[static_cast<int64_t>(blockIdx.x) * E + e] = run[e];
     return;
   }
-  if (stats) finish_stats<1>(st, E, 1, red_sh);  // (each lane reads back the counts it wrote)
+  // (each lane reads back the counts it wrote)
+  if (stats) finish_stats(st, E, tid < E ? st.block_valid[tid] : 0, st.f && tid < E ? st.block_share[tid] : 0.0f, red_sh);
   const LayoutLds s(extra, E);
   for (int e = tid; e < E; e += kLanes) {
     s.count[e] = run[e];
@@ -411,30 +431,47 @@ __global__ __launch_bounds__(kLanes) void route_rank_kernel(
   if (tid < T * K && tid < kRows * K) place_slot(s, p, tid, my_e, my_rank, K, w_sh[tid]);
 }
 
-template <int kLanes>
+// What a router that keeps statistics has done behind the plan's nb workgroups, by workgroups of their own: one for the sums (counts or loss wanted), the
+// histogram's (groups > 0).  Both are chains of latency that nothing here waits for: at 3000 tokens of 64 experts the sums made the first workgroup the
+// last to end (16 us for 7), and a launch of its own for the histogram took 10 more; together 395 -> 381 us of a training step of 1024 x 64 x 512.
+struct Behind {
+  int nb;
+  StatsOut st;
+  Observe observe;
+  int groups;
+};
+// (a router without statistics, with those arguments and branches / without: 512 tokens of 8 experts 5.5 / 4.4 us, 1531 of 16 5.7 / 4.8, 8192 of 128 12.0 / 10.7)
+struct NothingBehind {};
+
+template <int kLanes, typename Extra>
 __global__ __launch_bounds__(kLanes) void route_rows_kernel(const float* __restrict__ weights,
                                                             const int64_t* __restrict__ ids,
                                                             const uint32_t* __restrict__ rank_in_block,
                                                             const int32_t* __restrict__ block_hist, int T, int E, int K,
-                                                            int chunks, PlanOut p, StatsOut st, int nb, Observe observe, int groups) {
+                                                            int chunks, PlanOut p, Extra behind) {
   extern __shared__ int32_t lds[];
-  __shared__ float red_sh[2 * kLanes / kWave];
   const LayoutLds s(lds, E);
   const int tid = threadIdx.x;
-  // Behind the plan's workgroups: one for the statistics' sums, the histogram's.  Both are chains of latency that nothing here waits for: at 3000 tokens
-  // of 64 experts the sums made the first workgroup the last to end (16 us for 7), and a launch of its own for the histogram took 10 more; together
-  // 395 -> 381 us of a training step of 1024 x 64 x 512.
-  int extra = static_cast<int>(blockIdx.x) - nb;
-  if (extra >= 0 && (st.valid_counts || st.f)) {
-    if (extra == 0) {
-      finish_stats<32>(st, E, nb, red_sh);
+  int nb = gridDim.x;
+  if constexpr (std::is_same_v<Extra, Behind>) {
+    __shared__ float red_sh[2 * kLanes / kWave];
+    nb = behind.nb;
+    const StatsOut& st = behind.st;
+    int extra = static_cast<int>(blockIdx.x) - nb;
+    if (extra >= 0 && (st.valid_counts || st.f)) {
+      if (extra == 0) {
+        int valid = 0;
+        float share = 0.0f;
+        sum_blocks<kLanes>(st, E, nb, lds, valid, share);
+        finish_stats(st, E, valid, share, red_sh);
+        return;
+      }
+      --extra;
+    }
+    if (extra >= 0) {
+      observe_part<kLanes>(behind.observe, extra % behind.groups, extra / behind.groups, reinterpret_cast<unsigned*>(lds), red_sh);
       return;
     }
-    --extra;
-  }
-  if (extra >= 0) {
-    observe_part<kLanes>(observe, extra % groups, extra / groups, reinterpret_cast<unsigned*>(lds), red_sh);
-    return;
   }
   for (int e = tid; e < E; e += kLanes) s.count[e] = s.before[e] = 0;
   __syncthreads();
@@ -576,10 +613,18 @@ static int route_plan(const float* partial, int splits, const float* logit_bias,
   unsigned groups = 0, token_chunks = 0;
   if (histogram && blocks > 1) observe_shape(T, E, B, o.eg, o.tokens, groups, token_chunks);
   if (blocks > 1) {
-    const size_t bytes = std::max<size_t>(layout_words((int)E), (size_t)o.eg * o.B) * sizeof(int32_t);
     with_lanes(T, E, [&](auto lanes) {
-      hipLaunchKernelGGL(route_rows_kernel<decltype(lanes)::value>, dim3(blocks + (stats ? 1 : 0) + groups * token_chunks), dim3(lanes), bytes,
-                         s, weights, ids, rank, hist, (int)T, (int)E, (int)K, chunks, p, st, blocks, o, (int)groups);
+      constexpr int kLanes = decltype(lanes)::value;
+      auto rows = [&](auto kernel, unsigned grid, size_t words, auto behind) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(kLanes), words * sizeof(int32_t), s, weights, ids, rank, hist, (int)T, (int)E, (int)K, chunks, p,
+                           behind);
+      };
+      const size_t words = layout_words((int)E);
+      if (stats || groups > 0)
+        rows(route_rows_kernel<kLanes, Behind>, blocks + (stats ? 1 : 0) + groups * token_chunks,
+             std::max<size_t>({words, (size_t)o.eg * o.B, stats ? (size_t)kStatsWords<kLanes> : 0}), Behind{blocks, st, o, (int)groups});
+      else
+        rows(route_rows_kernel<kLanes, NothingBehind>, blocks, words, NothingBehind{});
     });
     if (int rc = check_launch("route_rows")) return rc;
   }
