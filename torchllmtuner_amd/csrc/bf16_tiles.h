@@ -60,28 +60,9 @@ __device__ __forceinline__ bf16x8 frag_ks(const uint16_t* tile, int col, int kk,
 // 4 fp32 of the result: column lane%16, rows 4*(lane/16) + i.  With random operand bits
 // this shape sustains about 14 % more than 32x32x16 on MI355X (a quarter of the
 // accumulator bytes per instruction for half the flops, and power is what limits both).
-__device__ __forceinline__ bf16x8 frag16_kc(const uint16_t* tile, int row, int kk32, int lane) {
-  const int r = row + (lane & 15);
-  const int c = kk32 * 4 + (lane >> 4);
-  return *reinterpret_cast<const bf16x8*>(tile + r * BK + ((c ^ ((r >> 1) & 7)) << 3));
-}
-
 // KS key for the 16x16x32 reader: 32 lanes of a transpose read touch rows k..k+3 and
 // k+8..k+11, 32 bytes of each, so the eight rows get an eighth of the banks each.
 __device__ __forceinline__ int ks_key16(int k) { return ((k & 3) << 2) | (((k >> 3) & 1) << 1); }
-
-template <int COLS>
-__device__ __forceinline__ bf16x8 frag16_ks(const uint16_t* tile, int col, int kk32, int lane) {
-  const int g = lane >> 4, i = lane & 15;
-  const int k = kk32 * 32 + 8 * g + (i >> 2);  // key of row k + 4 equals that of row k
-  const int c = col + 4 * (i & 3);
-  const int off = (((c >> 3) ^ ks_key16(k)) << 3) + (c & 7);
-  const uint16_t* p = tile + k * COLS + off;
-  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(p));
-  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(LDS_PTR(p + 4 * COLS));
-  const s16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-  return __builtin_bit_cast(bf16x8, v);
-}
 
 // ---- requests straight into LDS ----------------------------------------------------------
 typedef const __attribute__((address_space(3))) char* lds_cptr;
@@ -139,15 +120,19 @@ __device__ __forceinline__ void wave_lds_sync() {
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_wave_barrier();
 }
-__device__ __forceinline__ bf16x8 lds_read16(uint32_t at) {
-  return *(const __attribute__((address_space(3))) bf16x8*)(at);
+// LDS at a byte address (by way of the pointers' width on the host, where this is only compiled)
+template <typename T>
+__device__ __forceinline__ __attribute__((address_space(3))) T* lds_at(uint32_t at) {
+  return (__attribute__((address_space(3))) T*)(static_cast<uintptr_t>(at));
 }
-__device__ __forceinline__ int lds_read_i32(uint32_t at) { return *(const __attribute__((address_space(3))) int*)(at); }
-// eight k of 16 columns from rows of PITCH bytes, k as the 16x16x32 MFMA wants them (frag16_ks)
+__device__ __forceinline__ bf16x8 lds_read16(uint32_t at) { return *lds_at<const bf16x8>(at); }
+__device__ __forceinline__ int lds_read_i32(uint32_t at) { return *lds_at<const int>(at); }
+// Eight k of 16 columns from rows of PITCH bytes, as the 16x16x32 MFMA wants them.  Lane i of group g = lane / 16 asks for the 8-byte piece i % 4 of the
+// 16 columns in row k = 8 g + i / 4 (chunk swizzled by ks_key16(k), the key of row k + 4 too) and receives column i of rows 8 g .. 8 g + 7.
 template <uint32_t PITCH>
 __device__ __forceinline__ bf16x8 lds_read_tr(uint32_t at) {
-  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(at));
-  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(at + 4 * PITCH));
+  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(lds_at<s16x4>(at));
+  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(lds_at<s16x4>(at + 4 * PITCH));
   const s16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
   return __builtin_bit_cast(bf16x8, v);
 }
@@ -162,32 +147,5 @@ __device__ __forceinline__ void phase_barrier() {
 }
 
 __device__ __forceinline__ uint32_t pack2(float a, float b) { return pack_bf16x2(a, b); }
-
-// ---- epilogue staging -----------------------------------------------------------------
-// A wave parks its 64 x W sub-tile (bf16) in its private LDS region, [64][W + 8], then
-// streams it out as 16-byte row pieces.  acc was produced with the weight fragment as
-// the first MFMA operand: lane = output row (lane & 31), registers = output columns.
-template <int W>
-struct WaveStage {
-  static constexpr int PITCH = W + 8;
-  static constexpr int ELEMS = 64 * PITCH;
-  // element (row m of 64, col n of W) for register i of the accumulator tile (mi, nj-th 32 columns)
-  __device__ static __forceinline__ void put4(uint16_t* st, int mi, int col0, int lane, int q,
-                                              float v0, float v1, float v2, float v3) {
-    const int m = mi * 32 + (lane & 31);
-    const int n = col0 + q * 8 + (lane >> 5) * 4;
-    u32x2 pk = {pack2(v0, v1), pack2(v2, v3)};
-    *reinterpret_cast<u32x2*>(st + m * PITCH + n) = pk;
-  }
-  // the same for a 16 x 16 accumulator tile (mi-th 16 rows): lane = row lane & 15,
-  // registers = columns col0 + 4 * (lane >> 4) .. + 3
-  __device__ static __forceinline__ void put16(uint16_t* st, int mi, int col0, int lane, float v0, float v1,
-                                               float v2, float v3) {
-    const int m = mi * 16 + (lane & 15);
-    const int n = col0 + 4 * (lane >> 4);
-    u32x2 pk = {pack2(v0, v1), pack2(v2, v3)};
-    *reinterpret_cast<u32x2*>(st + m * PITCH + n) = pk;
-  }
-};
 
 }  // namespace mi355

@@ -6,7 +6,7 @@
 // token 48 items for 256 CUs, at 33 tokens 2.6 rounds of them.  Here a workgroup is four waves that
 // split the contraction of 16 output columns (of gate and up, or 32 of the down projection) of one
 // expert, and the four partial tiles are added in wave order through LDS.
-//   A wave's weights go straight into LDS of its own, two contraction steps of 64 ahead (8 KiB, 128 KiB a CU), in whole 128-byte lines, eight rows an
+//   A wave's weights go straight into LDS of its own, two contraction steps of 64 ahead (8 KiB; three workgroups fit a CU's LDS: 96 KiB), in whole 128-byte lines, eight rows an
 // instruction, and are read from there as MFMA fragments: no barrier stands in the loop.  Asked for as
 // fragments, 64 bytes of 16 rows an instruction with 16 KiB in registers ahead, a line is two requests, and the non-temporal hint makes the
 // second one go to memory again (5-11 % slower).  In lines the hint gains what it gains in the 256-row kernels (`streamed` there).
