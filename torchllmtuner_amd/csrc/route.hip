@@ -201,11 +201,10 @@ __device__ __forceinline__ void sum_blocks(const StatsOut& st, int E, int nb, in
     for (int q = 0; q < parts; ++q) valid += stage[q * E + tid];
 }
 
-// Valid counts, and the loss from them and the score shares; one workgroup whose lane e < E has expert e's.
-__device__ void finish_stats(const StatsOut& st, int E, int valid, float share, float* red) {
+// The loss from the valid slots and score shares of lane e < E's expert; one workgroup.
+__device__ void finish_loss(const StatsOut& st, int E, int valid, float share, float* red) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   constexpr float kEps = 1e-12f;  // F.normalize's clamp
-  if (st.valid_counts && tid < E) st.valid_counts[tid] = valid;
   if (!st.f) return;
   // E <= 256: four waves hold everything
   auto total = [&](float v) {
@@ -418,8 +417,16 @@ __global__ __launch_bounds__(kLanes) void route_rank_kernel(
     for (int e = tid; e < E; e += kLanes) block_hist[static_cast<int64_t>(blockIdx.x) * E + e] = run[e];
     return;
   }
-  // (each lane reads back the counts it wrote)
-  if (stats) finish_stats(st, E, tid < E ? st.block_valid[tid] : 0, st.f && tid < E ? st.block_share[tid] : 0.0f, red_sh);
+  if (stats) {
+    int valid = 0;
+    float share = 0.0f;
+    if (tid < E) {  // (each lane reads back the counts it wrote)
+      valid = st.block_valid[tid];
+      share += st.f ? st.block_share[tid] : 0.0f;
+      if (st.valid_counts) st.valid_counts[tid] = valid;
+    }
+    finish_loss(st, E, valid, share, red_sh);
+  }
   const LayoutLds s(extra, E);
   for (int e = tid; e < E; e += kLanes) {
     s.count[e] = run[e];
@@ -463,7 +470,8 @@ __global__ __launch_bounds__(kLanes) void route_rows_kernel(const float* __restr
         int valid = 0;
         float share = 0.0f;
         sum_blocks<kLanes>(st, E, nb, lds, valid, share);
-        finish_stats(st, E, valid, share, red_sh);
+        if (st.valid_counts && tid < E) st.valid_counts[tid] = valid;
+        finish_loss(st, E, valid, share, red_sh);
         return;
       }
       --extra;
