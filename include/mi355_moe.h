@@ -512,6 +512,16 @@ int mi355_grouped_swiglu_fwd_beside(const void* rows, const int32_t* token_of_ro
                                     int64_t tile_capacity, void* gate, void* up, void* h,
                                     void* y, int64_t El, int64_t D, int64_t F,
                                     int64_t row_capacity, void* stream);
+/* The same results for a caller that knows how many of the row_capacity rows to expect (padded segments, one rank's share of the
+ * experts): that number, and not the capacity, chooses the kernels.  Any number up to the capacity is right. */
+int mi355_grouped_swiglu_fwd_expecting(const void* rows, const int32_t* token_of_row, int64_t num_tokens,
+                                       const void* w1, const void* w3, const void* w2, int dtype,
+                                       const int32_t* seg_offsets,
+                                       const int32_t* seg_counts, const int32_t* tile_expert,
+                                       const int32_t* tile_row0, const int32_t* num_tiles,
+                                       int64_t tile_capacity, void* gate, void* up, void* h,
+                                       void* y, int64_t El, int64_t D, int64_t F,
+                                       int64_t row_capacity, int64_t rows_expected, void* stream);
 
 /*
  * Backward of the above (autograd-derived in the reference):

@@ -21,7 +21,7 @@ int bf16_grouped_fwd(const void* rows, const int32_t* token_of_row, int64_t num_
                      const void* w3, const void* w2, const int32_t* seg_offsets, const int32_t* seg_counts,
                      const int32_t* tile_expert, const int32_t* tile_row0, const int32_t* num_tiles,
                      int64_t tile_capacity, void* gate, void* up, void* h, void* y, int64_t El, int64_t D,
-                     int64_t F, int64_t row_capacity, int stages, hipStream_t s);
+                     int64_t F, int64_t row_capacity, int64_t rows_expected, int stages, hipStream_t s);
 int bf16_fused_dot_slots(int64_t F);
 int bf16_grouped_linear_dx(const void* dy, const void* w, const int32_t* seg_offsets, const int32_t* seg_counts,
                            const int32_t* tile_expert, const int32_t* tile_row0, const int32_t* num_tiles,
@@ -172,7 +172,7 @@ int swiglu_fwd(const void* rows, const int32_t* token_of_row, int64_t num_tokens
                const int32_t* seg_counts, const int32_t* tile_expert,
                const int32_t* tile_row0, const int32_t* num_tiles,
                int64_t tile_capacity, void* gate, void* up, void* h, void* y,
-               int64_t El, int64_t D, int64_t F, int64_t row_capacity,
+               int64_t El, int64_t D, int64_t F, int64_t row_capacity, int64_t rows_expected,
                int stages, void* stream) {
   if (int rc = check_common("grouped_swiglu_fwd", dtype, El, D, F, row_capacity, tile_capacity)) return rc;
   if (int rc = check_gather("grouped_swiglu_fwd", row_capacity > 0 ? token_of_row : nullptr, num_tokens, D, dtype)) return rc;
@@ -189,7 +189,7 @@ int swiglu_fwd(const void* rows, const int32_t* token_of_row, int64_t num_tokens
   hipStream_t s = as_stream(stream);
   if (fast)
     return bf16_grouped_fwd(rows, token_of_row, num_tokens, w1, w3, w2, seg_offsets, seg_counts, tile_expert,
-                            tile_row0, num_tiles, tile_capacity, gate, up, h, y, El, D, F, row_capacity, stages, s);
+                            tile_row0, num_tiles, tile_capacity, gate, up, h, y, El, D, F, row_capacity, rows_expected, stages, s);
   if (token_of_row)
     return fail(MI355_EUNSUP, "grouped_swiglu_fwd: the token gather needs bf16 with D and F multiples of 64; "
                               "materialise the rows with mi355_permute_rows_fwd instead");
@@ -226,7 +226,7 @@ extern "C" int mi355_grouped_swiglu_fwd(const void* rows, const int32_t* token_o
                                         int64_t El, int64_t D, int64_t F, int64_t row_capacity,
                                         void* stream) {
   return swiglu_fwd(rows, token_of_row, num_tokens, w1, w3, w2, dtype, seg_offsets, seg_counts, tile_expert, tile_row0,
-                    num_tiles, tile_capacity, gate, up, h, y, El, D, F, row_capacity, 3, stream);
+                    num_tiles, tile_capacity, gate, up, h, y, El, D, F, row_capacity, row_capacity, 3, stream);
 }
 
 extern "C" int mi355_grouped_swiglu_fwd_beside(const void* rows, const int32_t* token_of_row, int64_t num_tokens,
@@ -237,7 +237,20 @@ extern "C" int mi355_grouped_swiglu_fwd_beside(const void* rows, const int32_t* 
                                                int64_t El, int64_t D, int64_t F, int64_t row_capacity,
                                                void* stream) {
   return swiglu_fwd(rows, token_of_row, num_tokens, w1, w3, w2, dtype, seg_offsets, seg_counts, tile_expert, tile_row0,
-                    num_tiles, tile_capacity, gate, up, h, y, El, D, F, row_capacity, 3 | 128, stream);
+                    num_tiles, tile_capacity, gate, up, h, y, El, D, F, row_capacity, row_capacity, 3 | 128, stream);
+}
+
+extern "C" int mi355_grouped_swiglu_fwd_expecting(const void* rows, const int32_t* token_of_row, int64_t num_tokens,
+                                                  const void* w1, const void* w3, const void* w2, int dtype, const int32_t* seg_offsets,
+                                                  const int32_t* seg_counts, const int32_t* tile_expert,
+                                                  const int32_t* tile_row0, const int32_t* num_tiles,
+                                                  int64_t tile_capacity, void* gate, void* up, void* h, void* y,
+                                                  int64_t El, int64_t D, int64_t F, int64_t row_capacity,
+                                                  int64_t rows_expected, void* stream) {
+  MI355_REQUIRE(rows_expected >= 0 && rows_expected <= row_capacity, "grouped_swiglu_fwd_expecting: %lld rows of %lld",
+                (long long)rows_expected, (long long)row_capacity);
+  return swiglu_fwd(rows, token_of_row, num_tokens, w1, w3, w2, dtype, seg_offsets, seg_counts, tile_expert, tile_row0,
+                    num_tiles, tile_capacity, gate, up, h, y, El, D, F, row_capacity, rows_expected, 3, stream);
 }
 
 extern "C" int mi355_grouped_swiglu_bwd(const void* dy, const void* rows,
@@ -324,7 +337,7 @@ extern "C" int mi355_grouped_swiglu_stage(int stage, const void* dy, const void*
   hipStream_t s = as_stream(stream);
   if (stage <= 2)
     return bf16_grouped_fwd(rows, token_of_row, num_tokens, w1, w3, w2, seg_offsets, seg_counts, tile_expert,
-                            tile_row0, num_tiles, tile_capacity, gate, up, h, y, El, D, F, row_capacity, stage, s);
+                            tile_row0, num_tiles, tile_capacity, gate, up, h, y, El, D, F, row_capacity, row_capacity, stage, s);
   return bf16_grouped_bwd(
       dy, rows, token_of_row, num_tokens, w1, w3, w2, gate, up, h, nullptr, nullptr, seg_offsets, seg_counts,
       tile_expert, tile_row0, num_tiles, tile_capacity, dgate, dup, drows, dw1, dw3, dw2, El, D, F, stage, s);
@@ -344,8 +357,8 @@ extern "C" int mi355_grouped_linear_fwd(const void* x, const void* w, int dtype,
   if (dtype == MI355_BF16 && bf16_fast_path_ok(O, I))
     // the down projection's kernel is this product: rows (R, I) . w[e] (O, I)^T
     return bf16_grouped_fwd(nullptr, nullptr, 0, nullptr, nullptr, w, seg_offsets, seg_counts, tile_expert, tile_row0,
-                            num_tiles, tile_capacity, nullptr, nullptr, const_cast<void*>(x), y, El, O, I, row_capacity, 2,
-                            s);
+                            num_tiles, tile_capacity, nullptr, nullptr, const_cast<void*>(x), y, El, O, I, row_capacity,
+                            row_capacity, 2, s);
   if (any_path_ok(dtype, I, O, row_capacity, {x, w, y}))
     return any_linear({seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity, El}, dtype, x, w, y, I, O,
                       row_capacity, s);

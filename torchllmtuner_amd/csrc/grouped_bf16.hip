@@ -1081,6 +1081,14 @@ static unsigned resident_blocks() {
 }
 
 
+// Pieces of `height` rows that a segment has, of a number of rows around the mean like the sum of independent draws.
+static double pieces(double mean, double sd, int height) {
+  if (sd == 0.0) return std::ceil(mean / height);
+  double n = 1.0;
+  for (int j = height; j < mean + 5.0 * sd; j += height) n += 0.5 * std::erfc((j + 0.5 - mean) / (sd * std::sqrt(2.0)));
+  return n;
+}
+
 // Whether a product of El experts runs on 128-column tiles (`narrow_n` of them across) instead of 256-column ones (`wide_n`): where their rounds of
 // workgroups, seven tenths as long, take less time.  The number of row tiles is that of loads spread like independent draws around the mean
 // (experts of 256 rows on average have one tile and a half each); one expert's share of a wider router counts rows it does not get, which errs
@@ -1095,9 +1103,7 @@ static bool narrow(int mode, int64_t El, int64_t wide_n, int64_t narrow_n, int64
   if (El == 1) return (mode == RM_DH || mode == RM_DLIN) && tile_capacity * wide_n * 4 <= cus * 3;
   const int64_t spare = std::max<int64_t>(tile_capacity - El - 1, 0);  // 256 rows each
   if (spare * wide_n > 4 * cus) return false;
-  const double mean = (static_cast<double>(spare) + 0.5) * 256.0 / static_cast<double>(El), sd = std::sqrt(mean);
-  double tiles = 1.0;
-  for (int j = 256; j < mean + 5.0 * sd; j += 256) tiles += 0.5 * std::erfc((j + 0.5 - mean) / (sd * std::sqrt(2.0)));
+  const double mean = (static_cast<double>(spare) + 0.5) * 256.0 / static_cast<double>(El), tiles = pieces(mean, std::sqrt(mean), 256);
   auto rounds = [&](int64_t n) { return std::ceil((tiles * static_cast<double>(El * n) - 0.5) / static_cast<double>(cus)); };
   return rounds(narrow_n) * 0.7 < rounds(wide_n);
 }
@@ -1162,15 +1168,40 @@ int few_rows_fwd(int stage, const void* a, const int32_t* a_src, int64_t a_rows,
                  const int32_t* tile_expert, const int32_t* tile_row0, const int32_t* num_tiles, int64_t tiles, int64_t K,
                  int64_t N, bool stream, hipStream_t s);
 
-// Up to eight rows per expert on average (rows and experts are what the host knows; one expert's share of
-// a wider router counts rows it does not get, which only errs towards the large tiles), or 64 rows in all.
+// grouped_short.hip
+int short_rows_fwd(int stage, bool tall, const void* a, const int32_t* a_src, int64_t a_rows, const void* b0, const void* b1,
+                   void* gate, void* up, void* out, const int32_t* seg_offsets, const int32_t* seg_counts, int64_t El, int64_t K,
+                   int64_t N, int64_t row_capacity, bool stream, bool turn, hipStream_t s);
+
+// Up to eight rows per expert (`rows` of all: what the host expects), or 64 rows in all.
 // A 16-row pass over an expert's weights costs the same for one row as for sixteen and a second pass
 // reads them again, from L2 at best.  Block forward of 128 experts of 2048 x 768, these kernels / the row tiles, us: 16 tokens (1 row on average) 133 / 147, 33 183 /
-// 200, 64 202 / 210, 100 (6) 205 / 216, 128 (8) 216 / 215; 32 of 256 experts of 7168 x 2048, 16 tokens 186 / 230, 32 (counted as 8 rows, one of them here) 245 / 254.  One dense
+// 200, 64 202 / 210, 100 (6) 205 / 216, 128 (8) 216 / 215; 32 of 256 experts of 7168 x 2048, 16 tokens 186 / 230, 32 245 / 254.  One dense
 // segment of 7168 x 2048 alone, gate/up and down, 60 rows 41 + 16 / 79 + 26, 128 rows 79 + 25 / 93 + 30; but beside the routed experts of that share, whose CUs it takes
-// then, 128 rows 422 / 401.
-static bool few_rows(int64_t El, int64_t R, int64_t D, int64_t F) {
-  return R <= std::max<int64_t>(8 * El, 64) && R * std::max(D, F) * 2 < (int64_t{1} << 32);
+// then, 128 rows 422 / 401.  Beyond, 64-row passes (grouped_short.hip).
+static bool few_rows(int64_t El, int64_t rows, int64_t R, int64_t D, int64_t F) {
+  return rows <= std::max<int64_t>(8 * El, 64) && R * std::max(D, F) * 2 < (int64_t{1} << 32);
+}
+
+// Rows of a pass of grouped_short.hip, 0 for the row tiles (block forward, us, row tiles / 64 / 128 rows a pass).
+//   Up to 45 rows an expert, where hardly one needs a second pass, 64: the figures there.
+//   As many where all passes are at most two workgroups a CU, and 256-row tiles would leave most CUs without one: 16 experts of 512 x 384, four each, 90 to 300
+// rows an expert 35-41 / 31-36 / 35-39; 16 of 1024 x 512, 90 to 220 rows 44-50 / 39-44 / 45-48, 300 51 / 53 / 54, 400 56 / 64 / 56; 32 of it, 90 rows 55 / 53 /
+// 52, 130 58 / 64 / 67; one dense segment of 7168 x 2048, 129 rows 132 / 78 / 118, 512 177 / 83 / 119, 1000 179 / 115 / 126, 1400 182 / 164 / 164, 2000
+// 187 / 238 / 185; of 2048 x 1408, 129 to 1400 rows 60-83 / 41-46 / 53-57.
+//   128 up to 90 rows where the weights stay in the memory-side cache: 16 of 2048 x 1024, 60 / 75 / 90 rows 74 / 78 / 66, 75 / 77 / 68, 76 / 77 / 70; 64 of 1024 x 512
+// 75 / 76 / 71, 77 / 81 / 74 (80 rows), 79 / 85 / 79; 64 of 640 x 704, 90 rows 80 / 79 / 75; 32 of 1280 x 640 71 / 68 / 72, 73 / 75 / 74, 75 / 77 / 78.  Weights from memory
+// arrive as fast through row tiles then (60 of 1728 x 960, 60 rows 150 / 162 / 151; 128 of 2048 x 768 261 / 300 / 267).
+//   A dense segment beside other products leaves them more CUs in passes of 128 (one rank's share of 7168 x 2048 with a shared expert of 2048, 128 tokens
+// 365 / 347 / 348, 200 390 / 398 / 391, 300 417 / 418 / 404, 512 460 / 484 / 464).
+static int short_rows(int64_t El, int64_t rows, int64_t D, int64_t F, bool beside) {
+  if (El > 256 || rows < 1) return 0;  // (what a wave there adds up)
+  if (El == 1 && beside) return rows <= 400 ? 128 : 0;
+  const double mean = static_cast<double>(rows) / static_cast<double>(El), sd = El == 1 ? 0.0 : std::sqrt(mean);
+  if (El > 1 && mean <= 45.0) return 64;
+  const int64_t groups = std::max((F + 63) / 64, (D + 127) / 128);
+  if (pieces(mean, sd, 64) * static_cast<double>(El * groups) <= 2.0 * resident_blocks()) return 64;
+  return El > 1 && mean <= 90.0 && !streamed(El, D, F) ? 128 : 0;
 }
 
 // Turned contractions: where weight rows lie a multiple of 4 KiB apart (2048 elements) and most experts have one row
@@ -1185,10 +1216,10 @@ int bf16_grouped_fwd(const void* rows, const int32_t* token_of_row, int64_t num_
                      const void* w3, const void* w2, const int32_t* seg_offsets, const int32_t* seg_counts,
                      const int32_t* tile_expert, const int32_t* tile_row0, const int32_t* num_tiles,
                      int64_t tile_capacity, void* gate, void* up, void* h, void* y, int64_t El, int64_t D,
-                     int64_t F, int64_t row_capacity, int stages, hipStream_t s) {
-  if (few_rows(El, row_capacity, D, F)) {
+                     int64_t F, int64_t row_capacity, int64_t rows_expected, int stages, hipStream_t s) {
+  const bool stream = streamed(std::min(El, row_capacity), D, F);  // (of the experts that can have rows)
+  if (few_rows(El, rows_expected, row_capacity, D, F)) {
     const int64_t tiles = std::min(tile_capacity, std::min(El, row_capacity) + row_capacity / 256);
-    const bool stream = streamed(std::min(El, row_capacity), D, F);  // (of the experts that can have rows)
     if (stages & STAGE_GATEUP)
       if (int rc = few_rows_fwd(1, rows, token_of_row, num_tokens, w1, w3, gate, up, h, seg_offsets, seg_counts,
                                 tile_expert, tile_row0, num_tiles, tiles, D, F, stream, s))
@@ -1196,6 +1227,15 @@ int bf16_grouped_fwd(const void* rows, const int32_t* token_of_row, int64_t num_
     if (stages & STAGE_DOWN)
       return few_rows_fwd(2, h, nullptr, 0, w2, w2, nullptr, nullptr, y, seg_offsets, seg_counts, tile_expert, tile_row0,
                           num_tiles, tiles, F, D, stream, s);
+    return MI355_OK;
+  }
+  if (const int pass = short_rows(El, rows_expected, D, F, stages & STAGE_BESIDE)) {
+    if (stages & STAGE_GATEUP)
+      if (int rc = short_rows_fwd(1, pass > 64, rows, token_of_row, num_tokens, w1, w3, gate, up, h, seg_offsets, seg_counts, El,
+                                  D, F, row_capacity, stream, turned(El, row_capacity, D), s))
+        return rc;
+    if (stages & STAGE_DOWN)
+      return short_rows_fwd(2, pass > 64, h, nullptr, 0, w2, w2, nullptr, nullptr, y, seg_offsets, seg_counts, El, F, D, row_capacity, stream, turned(El, row_capacity, F), s);
     return MI355_OK;
   }
   const bool beside = stages & STAGE_BESIDE;

@@ -64,18 +64,6 @@ struct LayoutLds {
 };
 constexpr int layout_words(int E) { return 5 * E + 2 + 8; }
 
-// inclusive sum over the wave: within the rows of 16 lanes, then lane 15 of each odd row's
-// predecessor, then lane 31 for the upper half
-__device__ __forceinline__ int wave_scan(int v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
-  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
-  return v;
-}
-
 // counts -> padded segment offsets, tiles before each local expert, rank by descending count; left in
 // LDS for all lanes (ends on a barrier).  One lane per local expert (at most 256: four waves) scans
 // rows and tiles; the ranks, one comparison per pair of experts, are shared by all lanes.
