@@ -163,6 +163,40 @@ def test_rms_norm_is_registered_for_the_gpu_only_and_validates_metadata():
         rms_norm_mi355(torch.ones(2, 4), torch.ones(4), 1e-6)
 
 
+def bf16_bases(*tensors, offset):
+    """Copies that start `offset` elements behind a 16-byte boundary."""
+    return [torch.empty(t.numel() + 8, dtype=t.dtype, device=DEV)[offset:offset + t.numel()].view(t.shape).copy_(t) for t in tensors]
+
+
+# rows of whole 8-byte pieces: one wave's one, two and four pieces a lane, four waves' two, four and eight, and rows past those; rows of
+# 16-byte pieces on bases that are only 8-byte aligned
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,D,offset", [(3, 4, 0), (700, 252, 0), (5, 260, 0), (700, 516, 0), (5, 1020, 0), (2100, 1028, 0),
+                                           (5, 2044, 0), (5, 2052, 0), (600, 4092, 0), (5, 4100, 0), (600, 8188, 0), (3, 8196, 0),
+                                           (33, 2048, 4), (33, 512, 4)])
+def test_rms_norm_of_rows_in_8_byte_pieces(rows, D, offset):
+    from torchllmtuner_amd import _lib
+
+    print(f"rms_norm 8-byte pieces rows={rows} D={D} offset={offset}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(rows + D)
+    x, dy = (torch.randn(rows, D, device=DEV, generator=g).bfloat16() for _ in "xd")
+    w = (1 + 0.3 * torch.randn(D, device=DEV, generator=g)).bfloat16()
+    x, dy, w, y, dx = bf16_bases(x, dy, w, torch.zeros_like(x), torch.zeros_like(x), offset=offset)
+    rstd, dw = torch.empty(rows, device=DEV), torch.empty_like(w)
+    lib, p, s = _lib.load(), lambda t: t.data_ptr(), torch.cuda.current_stream().cuda_stream
+    work = torch.empty(lib.mi355_rms_norm_bwd_workspace_bytes(rows, D), dtype=torch.uint8, device=DEV)
+    _lib.check(lib.mi355_rms_norm_fwd(p(x), p(w), 1, p(y), p(rstd), rows, D, 1e-6, s), "rms_norm_fwd")
+    _lib.check(lib.mi355_rms_norm_bwd(p(dy), p(x), p(w), p(rstd), 1, p(dx), p(dw), p(work), rows, D, s), "rms_norm_bwd")
+    xd, wd, gd = x.double(), w.double(), dy.double()
+    r = 1 / torch.sqrt((xd * xd).mean(1, keepdim=True) + 1e-6)
+    t = gd * wd
+    want = xd * r * wd, r * (t - xd * r * (t * xd * r).mean(1, keepdim=True)), (gd * xd * r).sum(0)
+    # one rounding to bf16 each, 2^-9 at most; rms of a row or of all columns below 2e-3 (dx of four columns: a difference of near-equal terms)
+    for name, a, b in zip(("y", "dx", "dw"), (y, dx, dw[None]), (want[0], want[1], want[2][None])):
+        err = (a.double() - b).norm(dim=1) / b.norm(dim=1).clamp_min(1e-3 * b.norm() / b.shape[0] ** 0.5)
+        assert float(err.max()) < 3e-3, name
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("shape", [(2, 3, 8), (300, 2048), (5, 100), (7, 1), (7, 2), (0, 64), (4, 2, 7168), (33, 4100)])

@@ -10,7 +10,7 @@
 //   dw[d]    = sum_t dy[t][d] * xh[t][d]
 // HBM-bound: a row is held in registers by one wave or by four, read once, and reduced there; dw as
 // per-workgroup column sums over a run of rows, combined by a second kernel in a fixed order (no
-// atomics, deterministic).  Rows too wide for that, or not in whole 16-byte pieces, are read again.
+// atomics, deterministic).  Rows too wide for that, or not in whole 8-byte pieces, are read again.
 #include <algorithm>
 #include <initializer_list>
 #include <type_traits>
@@ -64,29 +64,32 @@ struct Pack<uint16_t, 8> {
 template <typename T>
 constexpr int kVec = 16 / sizeof(T);
 
-// 16 bytes of T as N floats and back
+// N consecutive elements in registers as they lie in memory: 16 bytes, or 8 where rows are no whole number of 16
 template <typename T, int N>
-__device__ __forceinline__ void unpack16(const u32x4& q, float (&v)[N]) {
+using Piece = uint32_t __attribute__((ext_vector_type(N * sizeof(T) / 4)));
+// ... as N floats and back
+template <typename T, int N>
+__device__ __forceinline__ void unpack(const Piece<T, N>& q, float (&v)[N]) {
   if constexpr (std::is_same<T, float>::value) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = __uint_as_float(q[j]);
+    for (int j = 0; j < N; ++j) v[j] = __uint_as_float(q[j]);
   } else {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < N / 2; ++j) {
       v[2 * j] = __uint_as_float(q[j] << 16);
       v[2 * j + 1] = __uint_as_float(q[j] & 0xffff0000u);
     }
   }
 }
 template <typename T, int N>
-__device__ __forceinline__ u32x4 pack16(const float (&v)[N]) {
-  u32x4 q;
+__device__ __forceinline__ Piece<T, N> pack(const float (&v)[N]) {
+  Piece<T, N> q;
   if constexpr (std::is_same<T, float>::value) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) q[j] = __float_as_uint(v[j]);
+    for (int j = 0; j < N; ++j) q[j] = __float_as_uint(v[j]);
   } else {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) q[j] = pack_bf16x2(v[2 * j], v[2 * j + 1]);
+    for (int j = 0; j < N / 2; ++j) q[j] = pack_bf16x2(v[2 * j], v[2 * j + 1]);
   }
   return q;
 }
@@ -142,36 +145,36 @@ __device__ __forceinline__ float group_sum(float v, float (*red)[4], int slot) {
 }
 
 // The same with the row in registers between the sum and the scaling, requested at once: WAVES (1 or 4) to a
-// row, ITER sixteen-byte groups per lane.  Reading the row again for the scaling kept the kernel at 4.2-4.5 TB/s
+// row, ITER pieces per lane.  Reading the row again for the scaling kept the kernel at 4.2-4.5 TB/s
 // (8192 / 32768 rows of 2048 bf16: 15.9 / 60 us, 12.6 / 41 now); four waves to a row once one would hold more than
-// four groups a lane.
-template <typename T, int WAVES, int ITER>
+// four pieces a lane.
+template <typename T, int N, int WAVES, int ITER>
 __global__ __launch_bounds__(256) void rms_fwd_row_in_registers_kernel(const T* __restrict__ x, const T* __restrict__ w,
                                                                        T* __restrict__ y, float* __restrict__ rstd,
                                                                        int rows, int D, float eps) {
-  constexpr int N = kVec<T>, LANES = WAVES * kWave;
+  constexpr int LANES = WAVES * kWave;
   __shared__ float red[1][4];
   const int lane = threadIdx.x % LANES;
   const int row = blockIdx.x * (4 / WAVES) + threadIdx.x / LANES;
   if (row >= rows) return;  // (four waves to a row: the grid has no such workgroup)
   const int64_t o = static_cast<int64_t>(row) * D;
-  const u32x4 zero = {0, 0, 0, 0};
-  u32x4 q[ITER], g[ITER];
+  const Piece<T, N> zero = {};
+  Piece<T, N> q[ITER], g[ITER];
 #pragma unroll
   for (int k = 0; k < ITER; ++k) {
     const int i = (k * LANES + lane) * N;
-    q[k] = i < D ? *reinterpret_cast<const u32x4*>(x + o + i) : zero;
+    q[k] = i < D ? *reinterpret_cast<const Piece<T, N>*>(x + o + i) : zero;
   }
 #pragma unroll
   for (int k = 0; k < ITER; ++k) {
     const int i = (k * LANES + lane) * N;
-    g[k] = i < D ? *reinterpret_cast<const u32x4*>(w + i) : zero;
+    g[k] = i < D ? *reinterpret_cast<const Piece<T, N>*>(w + i) : zero;
   }
   float ss = 0.0f;
 #pragma unroll
   for (int k = 0; k < ITER; ++k) {
     float v[N];
-    unpack16<T, N>(q[k], v);
+    unpack<T, N>(q[k], v);
 #pragma unroll
     for (int j = 0; j < N; ++j) ss += v[j] * v[j];
   }
@@ -182,11 +185,11 @@ __global__ __launch_bounds__(256) void rms_fwd_row_in_registers_kernel(const T* 
     const int i = (k * LANES + lane) * N;
     if (i >= D) break;
     float v[N], gv[N], out[N];
-    unpack16<T, N>(q[k], v);
-    unpack16<T, N>(g[k], gv);
+    unpack<T, N>(q[k], v);
+    unpack<T, N>(g[k], gv);
 #pragma unroll
     for (int j = 0; j < N; ++j) out[j] = (v[j] * r) * gv[j];
-    *reinterpret_cast<u32x4*>(y + o + i) = pack16<T, N>(out);
+    *reinterpret_cast<Piece<T, N>*>(y + o + i) = pack<T, N>(out);
   }
   if (lane == 0 && rstd) rstd[row] = r;
 }
@@ -238,41 +241,40 @@ __global__ __launch_bounds__(256) void rms_dx_kernel(const T* __restrict__ dy, c
 // rows and writes one row of partial sums.
 constexpr int kFusedBlocks = 2048;  // at most; 512 until a workgroup would get more than 32 rows
 
-// Four waves to a row, ITER sixteen-byte groups per lane: the row of dy and x is held in registers and the next
+// Four waves to a row, ITER pieces per lane: the row of dy and x is held in registers and the next
 // one requested before it is reduced (one barrier a row); a lane keeps the dweight sums of the columns it owns.
 // One wave to a row read the row twice and had too few in flight: 32768 rows of 4096 / 8192 bf16
 // 283 / 520 us, 144 / 334 now; fp32 rows beyond 4096 columns took two passes (16384 of 5000: 418, 204 now).
-template <typename T, int ITER>
+template <typename T, int N, int ITER>
 __global__ __launch_bounds__(256) void rms_bwd_row_per_group_kernel(
     const T* __restrict__ dy, const T* __restrict__ x, const T* __restrict__ w, const float* __restrict__ rstd,
     T* __restrict__ dx, float* __restrict__ partial, int rows, int D, int rows_per_block) {
-  constexpr int N = kVec<T>;
   __shared__ float red[2][4];
-  const u32x4 zero = {0, 0, 0, 0};
+  const Piece<T, N> zero = {};
   float acc[ITER][N];
-  u32x4 g[ITER], cdy[ITER], cx[ITER];
+  Piece<T, N> g[ITER], cdy[ITER], cx[ITER];
   auto at = [&](int k) { return (k * 256 + static_cast<int>(threadIdx.x)) * N; };
 #pragma unroll
   for (int k = 0; k < ITER; ++k) {
-    g[k] = at(k) < D ? *reinterpret_cast<const u32x4*>(w + at(k)) : zero;
+    g[k] = at(k) < D ? *reinterpret_cast<const Piece<T, N>*>(w + at(k)) : zero;
 #pragma unroll
     for (int j = 0; j < N; ++j) acc[k][j] = 0.0f;
   }
-  auto fetch = [&](int row, u32x4 (&a)[ITER], u32x4 (&b)[ITER]) {
+  auto fetch = [&](int row, Piece<T, N> (&a)[ITER], Piece<T, N> (&b)[ITER]) {
     const int64_t o = static_cast<int64_t>(row) * D;
 #pragma unroll
     for (int k = 0; k < ITER; ++k) {
       a[k] = b[k] = zero;
       if (at(k) < D) {
-        a[k] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(dy + o + at(k)));
-        b[k] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(x + o + at(k)));
+        a[k] = __builtin_nontemporal_load(reinterpret_cast<const Piece<T, N>*>(dy + o + at(k)));
+        b[k] = __builtin_nontemporal_load(reinterpret_cast<const Piece<T, N>*>(x + o + at(k)));
       }
     }
   };
   const int r0 = blockIdx.x * rows_per_block, r1 = min(r0 + rows_per_block, rows);
   if (r0 < r1) fetch(r0, cdy, cx);
   for (int row = r0; row < r1; ++row) {
-    u32x4 ndy[ITER], nx[ITER];
+    Piece<T, N> ndy[ITER], nx[ITER];
     const bool more = row + 1 < r1;
     if (more) fetch(row + 1, ndy, nx);
     const float r = rstd[row];
@@ -280,9 +282,9 @@ __global__ __launch_bounds__(256) void rms_bwd_row_per_group_kernel(
 #pragma unroll
     for (int k = 0; k < ITER; ++k) {
       float a[N], b[N], gv[N];
-      unpack16<T, N>(cdy[k], a);
-      unpack16<T, N>(cx[k], b);
-      unpack16<T, N>(g[k], gv);
+      unpack<T, N>(cdy[k], a);
+      unpack<T, N>(cx[k], b);
+      unpack<T, N>(g[k], gv);
 #pragma unroll
       for (int j = 0; j < N; ++j) dot += (a[j] * gv[j]) * (b[j] * r);
     }
@@ -291,16 +293,16 @@ __global__ __launch_bounds__(256) void rms_bwd_row_per_group_kernel(
 #pragma unroll
     for (int k = 0; k < ITER; ++k) {
       float a[N], b[N], gv[N], out[N];
-      unpack16<T, N>(cdy[k], a);
-      unpack16<T, N>(cx[k], b);
-      unpack16<T, N>(g[k], gv);
+      unpack<T, N>(cdy[k], a);
+      unpack<T, N>(cx[k], b);
+      unpack<T, N>(g[k], gv);
 #pragma unroll
       for (int j = 0; j < N; ++j) {
         const float xh = b[j] * r;
         out[j] = r * (a[j] * gv[j] - xh * c);
         acc[k][j] += a[j] * xh;
       }
-      if (dx && at(k) < D) *reinterpret_cast<u32x4*>(dx + o + at(k)) = pack16<T, N>(out);
+      if (dx && at(k) < D) *reinterpret_cast<Piece<T, N>*>(dx + o + at(k)) = pack<T, N>(out);
     }
     if (more) {
 #pragma unroll
@@ -319,32 +321,31 @@ __global__ __launch_bounds__(256) void rms_bwd_row_per_group_kernel(
             make_float4(acc[k][j], acc[k][j + 1], acc[k][j + 2], acc[k][j + 3]);
 }
 
-// The same with one wave to a row, for rows of at most 4 x 64 sixteen-byte groups (2048 bf16 or 1024 fp32
+// The same with one wave to a row, for rows of at most 4 x 64 pieces (2048 bf16 or 1024 fp32
 // columns): a workgroup's four waves add their column sums up through LDS at the end, the weights stay in
 // registers across the rows, and the next row of the wave is requested before the current one is
 // reduced -- with one row in flight per wave the kernel waited out a memory round trip per row.
-template <typename T, int ITER>
+template <typename T, int N, int ITER>
 __global__ __launch_bounds__(256) void rms_bwd_rows_in_registers_kernel(
     const T* __restrict__ dy, const T* __restrict__ x, const T* __restrict__ w, const float* __restrict__ rstd,
     T* __restrict__ dx, float* __restrict__ partial, int rows, int D, int rows_per_block) {
-  constexpr int N = kVec<T>;
   extern __shared__ float colsum[];  // [D]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   float acc[ITER][N], g[ITER][N];
-  const u32x4 zero = {0, 0, 0, 0};
+  const Piece<T, N> zero = {};
 #pragma unroll
   for (int k = 0; k < ITER; ++k) {
     const int i = (k * kWave + lane) * N;
-    u32x4 q = zero;
-    if (i < D) q = *reinterpret_cast<const u32x4*>(w + i);
-    unpack16<T, N>(q, g[k]);
+    Piece<T, N> q = zero;
+    if (i < D) q = *reinterpret_cast<const Piece<T, N>*>(w + i);
+    unpack<T, N>(q, g[k]);
 #pragma unroll
     for (int j = 0; j < N; ++j) acc[k][j] = 0.0f;
   }
   const int r0 = blockIdx.x * rows_per_block;
   const int r1 = min(r0 + rows_per_block, rows);
-  u32x4 cdy[ITER], cx[ITER];
-  auto fetch = [&](int row, u32x4 (&a)[ITER], u32x4 (&b)[ITER]) {
+  Piece<T, N> cdy[ITER], cx[ITER];
+  auto fetch = [&](int row, Piece<T, N> (&a)[ITER], Piece<T, N> (&b)[ITER]) {
     const int64_t o = static_cast<int64_t>(row) * D;
 #pragma unroll
     for (int k = 0; k < ITER; ++k) {
@@ -352,15 +353,15 @@ __global__ __launch_bounds__(256) void rms_bwd_rows_in_registers_kernel(
       a[k] = zero;
       b[k] = zero;
       if (i < D) {
-        a[k] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(dy + o + i));
-        b[k] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(x + o + i));
+        a[k] = __builtin_nontemporal_load(reinterpret_cast<const Piece<T, N>*>(dy + o + i));
+        b[k] = __builtin_nontemporal_load(reinterpret_cast<const Piece<T, N>*>(x + o + i));
       }
     }
   };
   int row = r0 + wave;
   if (row < r1) fetch(row, cdy, cx);
   for (; row < r1; row += 4) {
-    u32x4 ndy[ITER], nx[ITER];
+    Piece<T, N> ndy[ITER], nx[ITER];
     const bool more = row + 4 < r1;
     if (more) fetch(row + 4, ndy, nx);
     const float r = rstd[row];
@@ -368,8 +369,8 @@ __global__ __launch_bounds__(256) void rms_bwd_rows_in_registers_kernel(
 #pragma unroll
     for (int k = 0; k < ITER; ++k) {
       float a[N], b[N];
-      unpack16<T, N>(cdy[k], a);
-      unpack16<T, N>(cx[k], b);
+      unpack<T, N>(cdy[k], a);
+      unpack<T, N>(cx[k], b);
 #pragma unroll
       for (int j = 0; j < N; ++j) dot += (a[j] * g[k][j]) * (b[j] * r);
     }
@@ -379,15 +380,15 @@ __global__ __launch_bounds__(256) void rms_bwd_rows_in_registers_kernel(
     for (int k = 0; k < ITER; ++k) {
       const int i = (k * kWave + lane) * N;
       float a[N], b[N], out[N];
-      unpack16<T, N>(cdy[k], a);
-      unpack16<T, N>(cx[k], b);
+      unpack<T, N>(cdy[k], a);
+      unpack<T, N>(cx[k], b);
 #pragma unroll
       for (int j = 0; j < N; ++j) {
         const float xh = b[j] * r;
         out[j] = r * (a[j] * g[k][j] - xh * c);
         acc[k][j] += a[j] * xh;
       }
-      if (dx && i < D) *reinterpret_cast<u32x4*>(dx + o + i) = pack16<T, N>(out);
+      if (dx && i < D) *reinterpret_cast<Piece<T, N>*>(dx + o + i) = pack<T, N>(out);
     }
     if (more) {
 #pragma unroll
@@ -465,12 +466,22 @@ __global__ __launch_bounds__(256) void rms_dw_final_kernel(const float* __restri
   }
 }
 
-int rows_are_16_byte_aligned(int64_t D, int dtype, std::initializer_list<const void*> ptrs) {
-  const int64_t per16 = dtype == MI355_F32 ? 4 : 8;
-  if (D % per16 != 0) return 0;
-  for (const void* p : ptrs)
-    if (reinterpret_cast<uintptr_t>(p) % 16 != 0) return 0;
-  return 1;
+// Elements of the largest piece, 16 or 8 bytes, that rows are whole numbers of and start on; 0 where they are neither.  Rows of an odd number of 8-byte
+// pieces (every other width a multiple of four) went through the kernels that read them again, an element a lane; in pieces, forward and backward of bf16, us:
+// 2984 x 6652 141 -> 50 (4.0 TB/s), 8192 x 2052 78 -> 44, 32768 x 1020 166 -> 66 (5.1), 32768 x 8188 1469 -> 543, 512 x 8188 134 -> 24.
+int row_piece(int64_t D, int dtype, std::initializer_list<const void*> ptrs) {
+  uintptr_t bits = 0;
+  for (const void* p : ptrs) bits |= reinterpret_cast<uintptr_t>(p);
+  const int item = dtype == MI355_F32 ? 4 : 2;
+  for (int bytes = 16; bytes >= 4 * item; bytes /= 2)
+    if (D % (bytes / item) == 0 && bits % bytes == 0) return bytes / item;
+  return 0;
+}
+// calls f(integral_constant piece) for what row_piece gives for T
+template <typename T, typename Fn>
+void with_piece(int piece, Fn f) {
+  if (piece == kVec<T>) f(std::integral_constant<int, kVec<T>>{});
+  else if constexpr (kVec<T> > 4) f(std::integral_constant<int, 4>{});
 }
 
 int check_shape(const char* what, int64_t rows, int64_t D, int dtype) {
@@ -492,30 +503,35 @@ extern "C" int mi355_rms_norm_fwd(const void* x, const void* weight, int dtype, 
   if (rows == 0) return MI355_OK;
   MI355_REQUIRE(x && weight && y, "rms_norm_fwd: null pointer");
   const dim3 grid((unsigned)((rows + 3) / 4));
-  const int vec = rows_are_16_byte_aligned(D, dtype, {x, weight, y});
+  const int piece = row_piece(D, dtype, {x, weight, y});
   auto run = [&](auto tag) {
     using T = decltype(tag);
-    const int64_t groups = (D / kVec<T> + kWave - 1) / kWave;  // 16-byte groups per lane
     const T *xp = static_cast<const T*>(x), *wp = static_cast<const T*>(weight);
     T* yp = static_cast<T*>(y);
-    auto launch = [&](auto waves, auto iter) {
-      constexpr int W = decltype(waves)::value;
-      hipLaunchKernelGGL((rms_fwd_row_in_registers_kernel<T, W, decltype(iter)::value>), W == 1 ? grid : dim3((unsigned)rows),
-                         dim3(256), 0, as_stream(stream), xp, wp, yp, rstd, (int)rows, (int)D, epsilon);
-    };
-    const std::integral_constant<int, 1> i1;
-    const std::integral_constant<int, 2> i2;
-    const std::integral_constant<int, 4> i4;
-    const std::integral_constant<int, 8> i8;
-    if (vec && groups <= 1) launch(i1, i1);
-    else if (vec && groups <= 2) launch(i1, i2);
-    else if (vec && groups <= 4) launch(i1, i4);
-    else if (vec && groups <= 8) launch(i4, i2);
-    else if (vec && groups <= 16) launch(i4, i4);
-    else if (vec && groups <= 32) launch(i4, i8);
-    else
-      hipLaunchKernelGGL(rms_fwd_kernel<T>, grid, dim3(256), 0, as_stream(stream), xp, wp, yp, rstd, (int)rows, (int)D,
-                         epsilon, vec);
+    const int64_t groups = piece ? (D / piece + kWave - 1) / kWave : INT64_MAX;  // pieces per lane of a wave
+    if (groups > 32) {
+      hipLaunchKernelGGL(rms_fwd_kernel<T>, grid, dim3(256), 0, as_stream(stream), xp, wp, yp, rstd, (int)rows, (int)D, epsilon,
+                         piece == kVec<T>);
+      return;
+    }
+    with_piece<T>(piece, [&](auto n) {
+      auto launch = [&](auto waves, auto iter) {
+        constexpr int W = decltype(waves)::value;
+        hipLaunchKernelGGL((rms_fwd_row_in_registers_kernel<T, decltype(n)::value, W, decltype(iter)::value>),
+                           W == 1 ? grid : dim3((unsigned)rows), dim3(256), 0, as_stream(stream), xp, wp, yp, rstd, (int)rows, (int)D,
+                           epsilon);
+      };
+      const std::integral_constant<int, 1> i1;
+      const std::integral_constant<int, 2> i2;
+      const std::integral_constant<int, 4> i4;
+      const std::integral_constant<int, 8> i8;
+      if (groups <= 1) launch(i1, i1);
+      else if (groups <= 2) launch(i1, i2);
+      else if (groups <= 4) launch(i1, i4);
+      else if (groups <= 8) launch(i4, i2);
+      else if (groups <= 16) launch(i4, i4);
+      else launch(i4, i8);
+    });
   };
   if (dtype == MI355_F32) run(float{}); else run(uint16_t{});
   return check_launch("rms_norm_fwd");
@@ -541,14 +557,12 @@ extern "C" int mi355_rms_norm_bwd(const void* dy, const void* x, const void* wei
   const dim3 fgrid((unsigned)((D + 15) / 16));
   auto run = [&](auto tag) {
     using T = decltype(tag);
-    // one pass for both when rows are 16-byte aligned and a lane's columns fit in registers
-    constexpr int N = 16 / sizeof(T);
-    const int64_t groups = (D / N + kWave - 1) / kWave;  // 16-byte groups per lane
-    const bool one_wave = groups <= 4;
-    if (dweight && rows > 0 && (groups <= 16 || (groups <= 32 && dtype == MI355_F32)) &&
-        rows_are_16_byte_aligned(D, dtype, {dy, x, weight, dx, workspace})) {
+    // one pass for both where a lane's columns fit in registers
+    const int piece = row_piece(D, dtype, {dy, x, weight, dx});
+    const int64_t groups = piece ? (D / piece + kWave - 1) / kWave : INT64_MAX;  // pieces per lane of a wave
+    if (dweight && rows > 0 && aligned16(workspace) && groups <= (piece == 4 ? 32 : 16)) {
       const int blocks = (int)std::min<int64_t>(std::min<int64_t>(kFusedBlocks, std::max<int64_t>(512, rows / 32)),
-                                                one_wave ? (rows + 3) / 4 : rows);
+                                                groups <= 4 ? (rows + 3) / 4 : rows);
       const int rpb = (int)((rows + blocks - 1) / blocks);
       const int used = (int)((rows + rpb - 1) / rpb);
       auto launch = [&](auto kernel, size_t lds) {
@@ -556,12 +570,15 @@ extern "C" int mi355_rms_norm_bwd(const void* dy, const void* x, const void* wei
                            static_cast<const T*>(weight), rstd, static_cast<T*>(dx), static_cast<float*>(workspace),
                            (int)rows, (int)D, rpb);
       };
-      if (groups <= 1) launch(rms_bwd_rows_in_registers_kernel<T, 1>, (size_t)D * 4);
-      else if (groups <= 2) launch(rms_bwd_rows_in_registers_kernel<T, 2>, (size_t)D * 4);
-      else if (groups <= 4) launch(rms_bwd_rows_in_registers_kernel<T, 4>, (size_t)D * 4);
-      else if (groups <= 8) launch(rms_bwd_row_per_group_kernel<T, 2>, 0);
-      else if (groups <= 16) launch(rms_bwd_row_per_group_kernel<T, 4>, 0);
-      else if constexpr (sizeof(T) == 4) launch(rms_bwd_row_per_group_kernel<T, 8>, 0);
+      with_piece<T>(piece, [&](auto n) {
+        constexpr int N = decltype(n)::value;
+        if (groups <= 1) launch(rms_bwd_rows_in_registers_kernel<T, N, 1>, (size_t)D * 4);
+        else if (groups <= 2) launch(rms_bwd_rows_in_registers_kernel<T, N, 2>, (size_t)D * 4);
+        else if (groups <= 4) launch(rms_bwd_rows_in_registers_kernel<T, N, 4>, (size_t)D * 4);
+        else if (groups <= 8) launch(rms_bwd_row_per_group_kernel<T, N, 2>, 0);
+        else if (groups <= 16) launch(rms_bwd_row_per_group_kernel<T, N, 4>, 0);
+        else if constexpr (N == 4) launch(rms_bwd_row_per_group_kernel<T, N, 8>, 0);
+      });
       hipLaunchKernelGGL(rms_dw_final_kernel<T>, fgrid, dim3(256), 0, s, static_cast<const float*>(workspace),
                          static_cast<T*>(dweight), used, (int)D);
       return;
@@ -569,7 +586,7 @@ extern "C" int mi355_rms_norm_bwd(const void* dy, const void* x, const void* wei
     if (dx && rows > 0)
       hipLaunchKernelGGL(rms_dx_kernel<T>, rgrid, dim3(256), 0, s, static_cast<const T*>(dy),
                          static_cast<const T*>(x), static_cast<const T*>(weight), rstd, static_cast<T*>(dx),
-                         (int)rows, (int)D, rows_are_16_byte_aligned(D, dtype, {dy, x, weight, dx}));
+                         (int)rows, (int)D, piece == kVec<T>);
     if (dweight) {
       if (rows > 0)
         hipLaunchKernelGGL(rms_dw_partial_kernel<T>, cgrid, dim3(256), 0, s, static_cast<const T*>(dy),
