@@ -190,3 +190,22 @@ def test_shared_expert_beside_the_router(tokens):
         results.append([out.detach().clone(), *(p.grad.clone() for p in block.shared_experts.parameters())])
     for other in results[1:]:
         assert all(torch.equal(a, b) for a, b in zip(results[0], other))
+
+
+def test_two_weight_gradients_in_one_launch_and_in_two():
+    """Many experts of one K step each: two launches; the same segments with room for more rows: one."""
+    from torchllmtuner_amd import ops
+
+    print("weight gradients in one launch and in two", flush=True)
+    El, D, Fd = 256, 448, 1088  # 2560 tiles
+    gen = torch.Generator(device=DEV).manual_seed(5)
+    normal = lambda *s: torch.empty(*s, dtype=torch.bfloat16, device=DEV).normal_(generator=gen)
+    counts = torch.arange(El, device=DEV) % 7
+    ids = torch.repeat_interleave(torch.arange(El, device=DEV), counts)[:, None]
+    x, dout, w1, w3, w2 = normal(ids.shape[0], D), normal(ids.shape[0], D), normal(El, Fd, D), normal(El, Fd, D), normal(El, D, Fd)
+    plan, weights = ops.permute_plan(ids, El), torch.rand(ids.shape[0], 1, device=DEV, generator=gen)
+    _, gate, up, _ = ops.grouped_swiglu_fwd(x, w1, w3, w2, plan, gather=True)
+    apart, together = (ops.grouped_swiglu_combine_bwd(dout, x, weights, w1, w3, w2, gate, up, q) for q in (plan, wide(plan)))
+    for name, a, b in zip(("dx", "dw1", "dw3", "dw2", "dweights"), apart, together):
+        assert torch.equal(a, b), name
+    assert not torch.equal(apart[1], apart[2])

@@ -692,7 +692,7 @@ struct WgradArgs {
   int M, N;
   int m_tiles, n_tiles;
   int total;  // El * m_tiles * n_tiles
-  const uint16_t* a1;  // second plane of the grid: another product with the same b
+  const uint16_t* a1;  // null, or the first operand of another product with the same b, and its result
   uint16_t* c1;
 };
 
@@ -710,10 +710,7 @@ __global__ __launch_bounds__(NT, 2) void wgrad_kernel(WgradArgs p) {
   const int wr = wave >> 1, wn = wave & 1;
   const int M = p.M, N = p.N;
   const int per_e = p.m_tiles * p.n_tiles;
-  if (blockIdx.y) {
-    p.a = p.a1;
-    p.c = p.c1;
-  }
+  const int pair = p.c1 != nullptr ? 1 : 0;  // two products of the same b: their tiles in turn
 
   // Persistent workgroups.  A tile's cost is its expert's row count (the contraction
   // length), which a skewed router spreads over two orders of magnitude, so tiles are not
@@ -737,17 +734,17 @@ __global__ __launch_bounds__(NT, 2) void wgrad_kernel(WgradArgs p) {
   const int pool = (El & 7) * per_e;
   const int p0 = static_cast<int>(static_cast<int64_t>(pool) * xcd >> 3);
   const int p1 = static_cast<int>(static_cast<int64_t>(pool) * (xcd + 1) >> 3);
-  const int n_x = n_full + (p1 - p0);  // tiles of this XCD
+  const int n_x = (n_full + (p1 - p0)) << pair;  // tiles of this XCD
   const int stride = gridDim.x >> 3;
   int within = blockIdx.x >> 3;
   if (within >= n_x) return;
   auto exists = [&](int w) { return w < n_x; };
   struct Tile {
-    int e, seg0, cnt, m0, n0;
+    int e, seg0, cnt, m0, n0, second;
   };
   // this XCD's w-th tile (w clamped to an existing tile): the rank of its expert, and its tile in the expert
   auto place = [&](int w, int& rank) -> int {
-    w = exists(w) ? w : within;
+    w = (exists(w) ? w : within) >> pair;
     const bool full = w < n_full;
     const int u = full ? w : p0 + (w - n_full), r = u / per_e;
     rank = full ? r * 8 + ((r & 1) ? 7 - xcd : xcd) : (El & ~7) + r;
@@ -764,11 +761,11 @@ __global__ __launch_bounds__(NT, 2) void wgrad_kernel(WgradArgs p) {
   auto tile_at = [&](int w, int e) -> Tile {
     int rank;
     const int t = place(w, rank), m = t / p.n_tiles;
-    return {e, seg_offsets[e], seg_counts[e], min(m * WBM, M - WBM), min((t - m * p.n_tiles) * WBN, N - WBN)};
+    return {e, seg_offsets[e], seg_counts[e], min(m * WBM, M - WBM), min((t - m * p.n_tiles) * WBN, N - WBN), (exists(w) ? w : within) & pair};
   };
   // (field by field: a choice between the structures would leave them in memory)
   auto either = [](bool c, Tile a, Tile b) -> Tile {
-    return {c ? a.e : b.e, c ? a.seg0 : b.seg0, c ? a.cnt : b.cnt, c ? a.m0 : b.m0, c ? a.n0 : b.n0};
+    return {c ? a.e : b.e, c ? a.seg0 : b.seg0, c ? a.cnt : b.cnt, c ? a.m0 : b.m0, c ? a.n0 : b.n0, c ? a.second : b.second};
   };
   Tile t0 = tile_at(within, expert_at(within));
 
@@ -818,7 +815,7 @@ __global__ __launch_bounds__(NT, 2) void wgrad_kernel(WgradArgs p) {
     left = t.cnt;
     fm0 = t.m0;
     fn0 = t.n0;
-    gA = reinterpret_cast<uint64_t>(p.a + (GATHER_A ? 0 : static_cast<int64_t>(t.seg0) * M) + t.m0);
+    gA = reinterpret_cast<uint64_t>((t.second ? p.a1 : p.a) + (GATHER_A ? 0 : static_cast<int64_t>(t.seg0) * M) + t.m0);
     gB = reinterpret_cast<uint64_t>(p.b + (GATHER ? 0 : static_cast<int64_t>(t.seg0) * N) + t.n0);
     if constexpr (GATHER_A) bytesA = static_cast<uint32_t>(src_bytes - t.m0 * 2u);
     if constexpr (GATHER) bytesB = static_cast<uint32_t>(src_bytes - t.n0 * 2u);
@@ -1005,7 +1002,7 @@ __global__ __launch_bounds__(NT, 2) void wgrad_kernel(WgradArgs p) {
     // the tile's results, 16 rows at a time through the wave's own LDS
     const int el = opaque(lane);
     char* own = reinterpret_cast<char*>(smem) + epi;
-    uint16_t* C = p.c + static_cast<int64_t>(t0.e) * M * N + static_cast<int64_t>(t0.m0 + wr * 64) * N + t0.n0 + wn * 128;
+    uint16_t* C = (t0.second ? p.c1 : p.c) + static_cast<int64_t>(t0.e) * M * N + static_cast<int64_t>(t0.m0 + wr * 64) * N + t0.n0 + wn * 128;
     if constexpr (INDEXED) {
       lds_wait<VM>();
       read_indices();
@@ -1337,7 +1334,7 @@ int bf16_grouped_bwd(const void* dy, const void* rows, const int32_t* token_of_r
     w.m_tiles = (int)((M + WBM - 1) / WBM); w.n_tiles = (int)((N + WBN - 1) / WBN);
     w.total = (int)(El * w.m_tiles * w.n_tiles);
     w.a1 = (const uint16_t*)A1; w.c1 = (uint16_t*)C1;
-    const dim3 grid(std::min(round8(w.total), resident_blocks()), C1 ? 2 : 1);
+    const dim3 grid(std::min(round8((int64_t)w.total * (C1 ? 2 : 1)), resident_blocks()));
     if (a_src)
       hipLaunchKernelGGL((wgrad_kernel<false, true>), grid, dim3(NT), R_LDS_BYTES, s, w);
     else if (b_src)
@@ -1349,10 +1346,14 @@ int bf16_grouped_bwd(const void* dy, const void* rows, const int32_t* token_of_r
   // folded combine: dW2 = (gathered output gradient)^T . (row_scale * h)
   if (dw2 && (stages & STAGE_DW2))
     if (int rc = wgrad(dy, h, nullptr, dw2, D, F, "grouped dw2", row_scale ? token_of_row : nullptr)) return rc;
-  // dW1 and dW3 share their second operand: where one's tiles occupy at most half the CUs, one launch has both side by side (training steps
-  // of 500, 2000, 4000 tokens of 16 experts of 1024 x 512, four each, 196 / 183, 213 / 205, 327 / 316 us).
+  // dW1 and dW3 share their second operand: one launch has both, a tile of one beside the same tile of the other, and ends once.  A training step, us, apart /
+  // together: 64 experts of 1024 x 512, six each, 300, 700, 1500, 3000, 5686 tokens 205 / 200, 242 / 236, 309 / 304, 382 / 367, 594 / 564; 64 of 768 x 448, two each, 489
+  // tokens 155 / 148; 32 of 832 x 640, five each, 6991 603 / 588; 16 of 2048 x 1024, four each, 3000 566 / 557; 128 of 2048 x 768, eight each, 1600 816 / 809, 4000 1370 / 1373,
+  // 8192 2213 / 2205, 16384 of a skewed router 4142 / 4120.  (As two planes of the grid, whose workgroups follow each other, 2645 tokens of it and 7222 of 32
+  // of 1600 x 960 lost 2-3 %.)  Not where many tiles of one K step each do nothing but write: 200 to 450 tokens of the 128 experts 698 / 701.
   const int64_t tiles = El * ((F + WBM - 1) / WBM) * ((D + WBN - 1) / WBN);
-  if (dw1 && dw3 && (stages & STAGE_DW1) && (stages & STAGE_DW3) && tiles * 2 <= resident_blocks())
+  const bool one_step = 4 * (tile_capacity - El - 1) <= El;  // 64 rows an expert
+  if (dw1 && dw3 && (stages & STAGE_DW1) && (stages & STAGE_DW3) && !(one_step && tiles > 8 * (int64_t)resident_blocks()))
     return wgrad(dgate, rows, token_of_row, dw1, F, D, "grouped dw1 and dw3", nullptr, dup, dw3);
   if (dw1 && (stages & STAGE_DW1)) if (int rc = wgrad(dgate, rows, token_of_row, dw1, F, D, "grouped dw1")) return rc;
   if (dw3 && (stages & STAGE_DW3)) if (int rc = wgrad(dup, rows, token_of_row, dw3, F, D, "grouped dw3")) return rc;
