@@ -626,6 +626,18 @@ int mi355_grouped_gather_bwd(const void* dout, const void* x, const int32_t* tok
                              void* dw1, void* dw3, void* dw2, const float* dlogits, float* gate_partial,
                              int64_t gate_experts, int64_t El, int64_t D, int64_t F, int64_t row_capacity,
                              void* stream);
+/* mi355_router_select_rows_bwd and, behind it, mi355_grouped_gather_bwd with its dlogits, for up to 64 experts: the same bits, where the experts'
+ * products are few tiles in a launch less.  gate_partial may be NULL (the gate's weight gradient is not wanted); E experts, K choices a token. */
+int mi355_grouped_gather_route_bwd(const void* dout, const void* x, const int32_t* token_of_row, int64_t num_tokens,
+                                   const float* row_scale, const void* w1, const void* w3, const void* w2, const void* gate,
+                                   const void* up, const void* h, int dtype, const int32_t* seg_offsets,
+                                   const int32_t* seg_counts, const int32_t* tile_expert, const int32_t* tile_row0,
+                                   const int32_t* num_tiles, int64_t tile_capacity, void* dgate, void* dup, void* drows,
+                                   void* dw1, void* dw3, void* dw2, const float* logits, const int64_t* ids, const void* y,
+                                   const int32_t* row_of_slot, const float* aux_f_E, const float* aux_scale,
+                                   const uint8_t* padding_mask_T, float* dlogits, float* gate_partial, int64_t E, int64_t K,
+                                   int score_func, int route_norm, float route_scale, int64_t El, int64_t D, int64_t F,
+                                   int64_t row_capacity, void* stream);
 int mi355_combine_row_scale(const float* weights_TK, const int32_t* slot_of_row, float* row_scale,
                             int64_t T, int64_t K, int64_t row_capacity, void* stream);
 /* dweights[t][k] = sum_j dot_partial[row_of_slot[t*K+k]][j], summed in ascending j; 0 for

@@ -82,6 +82,10 @@ SIGNATURES = {
         I,
         [P, P, P, L, P, P, P, P, P, P, P, I, P, P, P, P, P, L, P, P, P, P, P, P, P, P, L, L, L, L, L, P],
     ),
+    "mi355_grouped_gather_route_bwd": (
+        I,
+        [P, P, P, L, P, P, P, P, P, P, P, I, P, P, P, P, P, L, P, P, P, P, P, P, P, P, P, P, P, P, P, P, P, L, L, I, I, F, L, L, L, L, P],
+    ),
     "mi355_route_stats_workspace_bytes": (L, [L, L]),
     "mi355_route_plan_stats": (
         I,

@@ -283,14 +283,14 @@ extern "C" int mi355_grouped_swiglu_bwd(const void* dy, const void* rows,
     const AnySeg g{seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity, El};
     const bool some = row_capacity > 0 && tile_capacity > 0;
     if (some)
-      if (int rc = any_dh(g, dtype, dy, w2, gate, up, dgate, dup, D, F, row_capacity, nullptr, nullptr, s)) return rc;
+      if (int rc = any_dh(g, dtype, dy, w2, gate, up, dgate, dup, D, F, row_capacity, nullptr, nullptr, nullptr, s)) return rc;
     // the weight gradients also cover the no-rows case: every expert's gradient is written (zeros)
     AnyGrad grads[3];
     int count = 0;
     if (dw2) grads[count++] = {dy, h, dw2, D, F, 0};
     if (dw1) grads[count++] = {dgate, rows, dw1, F, D, 0};
     if (dw3) grads[count++] = {dup, rows, dw3, F, D, 0};
-    return any_backward(g, dtype, dgate, dup, w1, w3, some ? drows : nullptr, D, F, grads, count, row_capacity, nullptr, s);
+    return any_backward(g, dtype, dgate, dup, w1, w3, some ? drows : nullptr, D, F, grads, count, row_capacity, nullptr, nullptr, s);
   }
   const Seg sg{seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity};
   if (row_capacity > 0 && tile_capacity > 0) {
@@ -395,7 +395,7 @@ extern "C" int mi355_grouped_linear_bwd(const void* dy, const void* x, const voi
     if (dx && rows)
       if (int rc = any_linear_dx(g, dtype, dy, w, dx, I, O, row_capacity, s)) return rc;
     const AnyGrad grad{dy, x, dw, O, I, 0};
-    return any_backward(g, dtype, nullptr, nullptr, nullptr, nullptr, nullptr, I, O, &grad, dw ? 1 : 0, row_capacity, nullptr, s);
+    return any_backward(g, dtype, nullptr, nullptr, nullptr, nullptr, nullptr, I, O, &grad, dw ? 1 : 0, row_capacity, nullptr, nullptr, s);
   }
   // dx = dy . w[e]: B(k=o, n=i) = w[e][o][i]
   if (dx && rows)
@@ -465,6 +465,44 @@ extern "C" int mi355_grouped_gather_fwd(const void* x, const int32_t* token_of_r
   return any_linear(g, dtype, h, w2, y, F, D, row_capacity, as_stream(stream));
 }
 
+namespace {
+// select: the selection's backward is formed here too (it gives router's dlogits): beside dH, and the gate's weight gradient beside the products behind
+// it, where those are one launch; else in front.
+int gather_bwd(const void* dout, const void* x, const int32_t* token_of_row, int64_t num_tokens, const float* row_scale, const void* w1,
+               const void* w3, const void* w2, const void* gate, const void* up, const void* h, int dtype, const AnySeg& g, void* dgate,
+               void* dup, void* drows, void* dw1, void* dw3, void* dw2, const AnyGate* router, const AnySelect* select, int64_t D,
+               int64_t F, int64_t row_capacity, void* stream) {
+  if (int rc = check_common("grouped_gather_bwd", dtype, g.El, D, F, row_capacity, g.tile_capacity)) return rc;
+  MI355_REQUIRE(row_capacity >= 1 && g.tile_capacity >= 1 && dout && x && token_of_row && row_scale && w1 && w3 && w2 && gate &&
+                    up && h && g.seg_offsets && g.seg_counts && g.tile_expert && g.tile_row0 && g.num_tiles && dgate && dup,
+                "grouped_gather_bwd: null pointer");
+  if (!gather_ok(dtype, D, F, row_capacity, num_tokens, {dout, x, w1, w3, w2, gate, up, h, dgate, dup, drows, dw1, dw3, dw2}))
+    return fail(MI355_EUNSUP, "grouped_gather_bwd: not covered; use mi355_combine_bwd and mi355_grouped_swiglu_bwd");
+  const AnyFold fold{token_of_row, num_tokens, row_scale};
+  MI355_REQUIRE(!router || (router->dlogits && router->partial && router->E >= 1 && aligned16({router->dlogits, router->partial})),
+                "grouped_gather_bwd: null or misaligned pointer");
+  if (router && !router_few_ok(dtype, MI355_F32, D, router->E))
+    return fail(MI355_EUNSUP, "grouped_gather_bwd: the gate's gradient is not covered; use mi355_router_gate_bwd");
+  AnyGrad grads[3];
+  int count = 0;
+  if (dw2) grads[count++] = {dout, h, dw2, D, F, 1};
+  if (dw1) grads[count++] = {dgate, x, dw1, F, D, 2};
+  if (dw3) grads[count++] = {dup, x, dw3, F, D, 2};
+  const bool beside = select && any_backward_is_one_launch(g, dtype, drows, D, grads, count, row_capacity);
+  if (select && !beside)
+    if (int rc = mi355_router_select_rows_bwd(select->logits, select->ids, dout, select->y, dtype, select->row_of_slot, row_capacity, D,
+                                              select->aux_f, select->aux_scale, select->padding, select->dlogits, num_tokens,
+                                              select->E, select->K, select->score_func, select->route_norm, select->route_scale,
+                                              stream))
+      return rc;
+  if (int rc = any_dh(g, dtype, dout, w2, gate, up, dgate, dup, D, F, row_capacity, &fold, beside ? nullptr : router,
+                      beside ? select : nullptr, as_stream(stream)))
+    return rc;
+  return any_backward(g, dtype, dgate, dup, w1, w3, drows, D, F, grads, count, row_capacity, &fold, beside ? router : nullptr,
+                      as_stream(stream));
+}
+}  // namespace
+
 extern "C" int mi355_grouped_gather_bwd(const void* dout, const void* x, const int32_t* token_of_row, int64_t num_tokens,
                                         const float* row_scale, const void* w1, const void* w3, const void* w2,
                                         const void* gate, const void* up, const void* h, int dtype,
@@ -473,26 +511,30 @@ extern "C" int mi355_grouped_gather_bwd(const void* dout, const void* x, const i
                                         void* dgate, void* dup, void* drows, void* dw1, void* dw3, void* dw2,
                                         const float* dlogits, float* gate_partial, int64_t gate_experts, int64_t El,
                                         int64_t D, int64_t F, int64_t row_capacity, void* stream) {
-  if (int rc = check_common("grouped_gather_bwd", dtype, El, D, F, row_capacity, tile_capacity)) return rc;
-  MI355_REQUIRE(row_capacity >= 1 && tile_capacity >= 1 && dout && x && token_of_row && row_scale && w1 && w3 && w2 && gate &&
-                    up && h && seg_offsets && seg_counts && tile_expert && tile_row0 && num_tiles && dgate && dup,
-                "grouped_gather_bwd: null pointer");
-  if (!gather_ok(dtype, D, F, row_capacity, num_tokens, {dout, x, w1, w3, w2, gate, up, h, dgate, dup, drows, dw1, dw3, dw2}))
-    return fail(MI355_EUNSUP, "grouped_gather_bwd: not covered; use mi355_combine_bwd and mi355_grouped_swiglu_bwd");
-  const AnySeg g{seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity, El};
-  const AnyFold fold{token_of_row, num_tokens, row_scale};
-  MI355_REQUIRE(!dlogits || (gate_partial && gate_experts >= 1 && aligned16({dlogits, gate_partial})),
-                "grouped_gather_bwd: null or misaligned pointer");
-  if (dlogits && !router_few_ok(dtype, MI355_F32, D, gate_experts))
-    return fail(MI355_EUNSUP, "grouped_gather_bwd: the gate's gradient is not covered; use mi355_router_gate_bwd");
   const AnyGate job{dlogits, x, gate_partial, gate_experts};
-  if (int rc = any_dh(g, dtype, dout, w2, gate, up, dgate, dup, D, F, row_capacity, &fold, dlogits ? &job : nullptr,
-                      as_stream(stream)))
-    return rc;
-  AnyGrad grads[3];
-  int count = 0;
-  if (dw2) grads[count++] = {dout, h, dw2, D, F, 1};
-  if (dw1) grads[count++] = {dgate, x, dw1, F, D, 2};
-  if (dw3) grads[count++] = {dup, x, dw3, F, D, 2};
-  return any_backward(g, dtype, dgate, dup, w1, w3, drows, D, F, grads, count, row_capacity, &fold, as_stream(stream));
+  return gather_bwd(dout, x, token_of_row, num_tokens, row_scale, w1, w3, w2, gate, up, h, dtype,
+                    {seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity, El}, dgate, dup, drows, dw1, dw3, dw2,
+                    dlogits ? &job : nullptr, nullptr, D, F, row_capacity, stream);
+}
+
+extern "C" int mi355_grouped_gather_route_bwd(
+    const void* dout, const void* x, const int32_t* token_of_row, int64_t num_tokens, const float* row_scale, const void* w1,
+    const void* w3, const void* w2, const void* gate, const void* up, const void* h, int dtype, const int32_t* seg_offsets,
+    const int32_t* seg_counts, const int32_t* tile_expert, const int32_t* tile_row0, const int32_t* num_tiles, int64_t tile_capacity,
+    void* dgate, void* dup, void* drows, void* dw1, void* dw3, void* dw2, const float* logits, const int64_t* ids, const void* y,
+    const int32_t* row_of_slot, const float* aux_f_E, const float* aux_scale, const uint8_t* padding_mask_T, float* dlogits,
+    float* gate_partial, int64_t E, int64_t K, int score_func, int route_norm, float route_scale, int64_t El, int64_t D, int64_t F,
+    int64_t row_capacity, void* stream) {
+  if (E < 1 || E > kSelectBesideE || K < 1 || K > E)
+    return fail(MI355_EUNSUP, "grouped_gather_route_bwd: E=%lld K=%lld is not covered; use mi355_router_select_rows_bwd and "
+                              "mi355_grouped_gather_bwd", (long long)E, (long long)K);
+  MI355_REQUIRE(num_tokens >= 1 && num_tokens < (1ll << 31) && logits && ids && y && row_of_slot && dlogits && aligned16({dout, y}),
+                "grouped_gather_route_bwd: null or misaligned pointer");
+  MI355_REQUIRE(!aux_f_E || aux_scale, "grouped_gather_route_bwd: the loss needs its scale");
+  const AnyGate job{dlogits, x, gate_partial, E};
+  const AnySelect select{logits, ids, dout, y, row_of_slot, aux_f_E, aux_scale, padding_mask_T, dlogits, E, K, score_func, route_norm,
+                         route_scale};
+  return gather_bwd(dout, x, token_of_row, num_tokens, row_scale, w1, w3, w2, gate, up, h, dtype,
+                    {seg_offsets, seg_counts, tile_expert, tile_row0, num_tiles, tile_capacity, El}, dgate, dup, drows, dw1, dw3, dw2,
+                    gate_partial ? &job : nullptr, &select, D, F, row_capacity, stream);
 }

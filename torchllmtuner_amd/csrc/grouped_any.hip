@@ -26,6 +26,7 @@
 #include "common.h"
 #include "grouped_any.h"
 #include "router_few.h"
+#include "select_bwd.h"
 
 namespace mi355 {
 namespace {
@@ -701,45 +702,66 @@ __global__ __launch_bounds__(256, 2) void any_kernel(AnyArgs p) {
   any_tile<T, MODE, TM, TN, FOLD>(p, blockIdx.x, smem);
 }
 
-// The experts' dH and, in the workgroups past its `blocks`, the router gate's weight gradient: both need what the
-// selection's backward left, neither the other, and neither fills the chip.  With the gate's input gradient taking the sum over a
-// token's rows along, and the slices' sum beside it, a backward has four launches instead of seven: a training step of 1531 bf16 tokens of
-// 16 x 320 x 232 128 -> 109 us, 512 fp32 of 8 x 256 x 512 126 -> 119, 100 bf16 of 4 x 200 x 104 139 -> 122.
-template <typename T, int TM, int TN>
-__global__ __launch_bounds__(256, 2) void any_dh_gate_kernel(AnyArgs p, GateDw gate, int blocks) {
+// What runs beside the experts' products in workgroups past theirs: the router gate's weight gradient, or the selection's backward.
+template <typename T>
+__device__ __forceinline__ void beside_part(const GateDw& job, int part, float* lds) { gate_dw_part<T>(job, part, lds); }
+template <typename T>
+__device__ __forceinline__ void beside_part(const SelectBwd& job, int part, float* lds) { select_bwd_part<1, T>(job, part, lds); }
+int64_t beside_parts(const GateDw& job) { return gate_dw_parts(job); }
+int64_t beside_parts(const SelectBwd& job) { return select_bwd_parts(job); }
+
+// The experts' dH and one of those.  The selection's backward and dH read the output gradient and what the forward left, neither the other's result, and
+// neither fills the chip; the gate's weight gradient, which reads what the selection's left, then runs beside the input and weight gradients of the experts
+// (any_dx_dw_kernel), or, where those are launches of their own, here behind it.  With the gate's input gradient taking the sum over a
+// token's rows along, and the slices' sum beside it, a backward has three launches, or four, instead of seven.  The selection's backward as a launch of its own in
+// front / beside dH, a training step's GPU time and a whole step on a box where the host is what it waits for, us: 512 fp32 tokens of two of 8 x 256 x 512 84 / 80, 130 / 125; 1531 bf16 of
+// four of 16 x 320 x 232 92 / 86, 130 / 125; 105 of two of 16 x 464 x 168 63 / 59, 132 / 126; 3310 of two of 8 x 352 x 360 118 / 114, 130 / 125.
+template <typename T, int TM, int TN, typename Job>
+__global__ __launch_bounds__(256, 2) void any_dh_beside_kernel(AnyArgs p, Job job, int blocks) {
   constexpr int A = any_lds<T, ANY_DH, TM, TN>(), B = kGateDwLds * 4 / sizeof(T);
+  static_assert(kGateDwLds >= 4 * 2 * kSelectBesideE, "either job's LDS");
   __shared__ __attribute__((aligned(16))) T smem[A > B ? A : B];
   const int block = blockIdx.x;
   if (block < blocks) any_tile<T, ANY_DH, TM, TN, true>(p, block, smem);
-  else gate_dw_part<T>(gate, block - blocks, reinterpret_cast<float*>(smem));
+  else beside_part<T>(job, block - blocks, reinterpret_cast<float*>(smem));
 }
 
 // The input gradient and the weight gradients of a backward pass read the same buffers and write different
 // ones: with few tiles each they share a launch (at 512 fp32 tokens of 8 experts 26 + 16 us one after the
-// other).  The longer contraction starts first.
+// other).  The longer contraction starts first.  With a fold the gate's weight gradient may come last.
 template <typename T, int TX, int TW, bool FOLD>
-__global__ __launch_bounds__(256, 2) void any_dx_dw_kernel(AnyArgs dx, AnyArgs dw, int dx_blocks, int dw_blocks, int dw_first) {
-  constexpr int A = any_lds<T, ANY_DX, TX, TX>(), B = any_lds<T, ANY_DW, TW, TW>();
-  __shared__ __attribute__((aligned(16))) T smem[A > B ? A : B];
+__global__ __launch_bounds__(256, 2) void any_dx_dw_kernel(AnyArgs dx, AnyArgs dw, int dx_blocks, int dw_blocks, int dw_first, GateDw gate) {
+  constexpr int A = any_lds<T, ANY_DX, TX, TX>(), B = any_lds<T, ANY_DW, TW, TW>(), C = FOLD ? kGateDwLds * 4 / sizeof(T) : 0;
+  __shared__ __attribute__((aligned(16))) T smem[A > B ? (A > C ? A : C) : (B > C ? B : C)];
+  if constexpr (FOLD) {
+    if (static_cast<int>(blockIdx.x) >= dx_blocks + dw_blocks) {
+      gate_dw_part<T>(gate, blockIdx.x - dx_blocks - dw_blocks, reinterpret_cast<float*>(smem));
+      return;
+    }
+  }
   const int block = static_cast<int>(blockIdx.x) - (dw_first ? dw_blocks : 0);  // of dx
   if (block >= 0 && block < dx_blocks) any_tile<T, ANY_DX, TX, TX, false>(dx, block, smem);
   else any_tile<T, ANY_DW, TW, TW, FOLD>(dw, dw_first ? blockIdx.x : block - dx_blocks, smem);
 }
 
 template <int MODE, int TM, int TN>
-int launch_any(const AnyArgs& p, int dtype, int64_t blocks, hipStream_t s, const char* what, const GateDw* gate = nullptr) {
+int launch_any(const AnyArgs& p, int dtype, int64_t blocks, hipStream_t s, const char* what, const GateDw* gate = nullptr,
+               const SelectBwd* select = nullptr) {
   if (blocks <= 0) return MI355_OK;
   if (dtype != MI355_F32 && TM == 32) return fail(MI355_EUNSUP, "%s: 32-row tiles are for fp32", what);
   if constexpr (MODE == ANY_DH) {
-    if (gate) {
-      const dim3 grid((unsigned)(blocks + gate_dw_parts(*gate))), lanes(256);
+    auto beside = [&](const auto& job) {
+      using Job = std::decay_t<decltype(job)>;
+      const dim3 grid((unsigned)(blocks + beside_parts(job))), lanes(256);
       if (dtype == MI355_F32) {
-        hipLaunchKernelGGL((any_dh_gate_kernel<float, TM, TN>), grid, lanes, 0, s, p, *gate, (int)blocks);
+        hipLaunchKernelGGL((any_dh_beside_kernel<float, TM, TN, Job>), grid, lanes, 0, s, p, job, (int)blocks);
       } else if constexpr (TM != 32) {
-        hipLaunchKernelGGL((any_dh_gate_kernel<uint16_t, TM, TN>), grid, lanes, 0, s, p, *gate, (int)blocks);
+        hipLaunchKernelGGL((any_dh_beside_kernel<uint16_t, TM, TN, Job>), grid, lanes, 0, s, p, job, (int)blocks);
       }
       return check_launch(what);
-    }
+    };
+    if (select) return beside(*select);
+    if (gate) return beside(*gate);
   }
   auto run = [&](auto fold) {
     constexpr bool FOLD = decltype(fold)::value;
@@ -779,15 +801,15 @@ int row_tile(const AnyArgs& p, int dtype, int64_t El, int64_t cols, int bf16_lar
 
 template <int MODE>
 int launch_rows(AnyArgs& p, int dtype, int64_t tile_capacity, int64_t El, int64_t cols, hipStream_t s, const char* what,
-                const GateDw* gate = nullptr) {
+                const GateDw* gate = nullptr, const SelectBwd* select = nullptr) {
   constexpr bool GU = MODE == ANY_GATEUP;
   const int t = row_tile(p, dtype, El, cols, MODE == ANY_DH ? 512 : 150), width = GU && t == 128 ? 64 : t;
   p.col_tiles = (int)((cols + width - 1) / width);
   const int64_t blocks = tile_capacity * (256 / t) * p.col_tiles;
   MI355_REQUIRE(blocks < (1ll << 30), "%s: too many tiles", what);
-  if (t == 128) return launch_any<MODE, 128, 128>(p, dtype, blocks, s, what, gate);
-  return t == 64 ? launch_any<MODE, 64, GU ? 128 : 64>(p, dtype, blocks, s, what, gate)
-                 : launch_any<MODE, 32, GU ? 64 : 32>(p, dtype, blocks, s, what, gate);
+  if (t == 128) return launch_any<MODE, 128, 128>(p, dtype, blocks, s, what, gate, select);
+  return t == 64 ? launch_any<MODE, 64, GU ? 128 : 64>(p, dtype, blocks, s, what, gate, select)
+                 : launch_any<MODE, 32, GU ? 64 : 32>(p, dtype, blocks, s, what, gate, select);
 }
 
 int64_t dw_tiles(AnyArgs& p, int64_t El, int tile) {
@@ -846,45 +868,82 @@ int any_linear_dx(const AnySeg& g, int dtype, const void* dy, const void* w, voi
 }
 
 int any_dh(const AnySeg& g, int dtype, const void* dy, const void* w2, const void* gate, const void* up, void* dgate,
-           void* dup, int64_t D, int64_t F, int64_t R, const AnyFold* f, const AnyGate* router, hipStream_t s) {
+           void* dup, int64_t D, int64_t F, int64_t R, const AnyFold* f, const AnyGate* router, const AnySelect* select,
+           hipStream_t s) {
   AnyArgs p = any_args(g, R, f);
   p.a0 = dy; p.b0 = w2; p.c0 = dgate; p.c1 = dup; p.gate = gate; p.up = up;
   p.K = (int)D; p.N = (int)F; p.ldb = (int)F; p.w_elems = D * F;
   GateDw job{};
+  SelectBwd sel{};
   if (router) job = gate_dw_job(router->dlogits, router->x, router->partial, f->tokens, D, router->E);
-  return launch_rows<ANY_DH>(p, dtype, g.tile_capacity, g.El, F, s, "grouped dh", router ? &job : nullptr);
+  if (select)
+    sel = {select->logits, select->ids, nullptr, nullptr, DotPieces{}, DotRows{select->dout, select->y, select->row_of_slot, (int)D, (int)R},
+           BalanceGrad{select->aux_f, select->aux_scale, select->padding}, select->dlogits, (int)f->tokens, (int)select->E,
+           (int)select->K, select->score_func, select->route_norm, select->route_scale, MI355_SELECT_TOPK};
+  return launch_rows<ANY_DH>(p, dtype, g.tile_capacity, g.El, F, s, "grouped dh", router ? &job : nullptr, select ? &sel : nullptr);
 }
 
-int any_backward(const AnySeg& g, int dtype, const void* dgate, const void* dup, const void* w1, const void* w3, void* drows,
-                 int64_t D, int64_t F, const AnyGrad* grads, int count, int64_t R, const AnyFold* f, hipStream_t s) {
-  AnyArgs p = any_args(g, R);
-  p.a0 = dgate; p.a1 = dup; p.b0 = w1; p.b1 = w3; p.c0 = drows;
-  p.K = (int)F; p.N = (int)D; p.ldb = (int)D; p.w_elems = D * F;
-  AnyArgs w = any_args(g, R, f);
-  for (int i = 0; i < count; ++i)
-    w.dw[i] = {grads[i].a, grads[i].b, grads[i].c, (int)grads[i].M, (int)grads[i].N, 0, 0, grads[i].through};
-  w.num_dw = count;
+namespace {
+// How a backward pass is launched: the weight gradients' tile, the input gradient's, and whether they share a launch.
+struct BackwardPlan {
+  int64_t tiles;
+  bool dw_large, dw_small, one;
+  int t;
+};
+BackwardPlan backward_plan(const AnyArgs& p, AnyArgs& w, int dtype, int64_t El, int64_t D, const void* drows, int count, int64_t R) {
   // Weight gradients on 128 x 128 tiles once these fill the chip; fp32 ones where their contraction is long enough to be what
   // takes the time (us, the backward, 64 / 128: 250 rows an expert 279 / 290, 500 497 / 482, 1000 950 / 895).  fp32 on 32 x 32 tiles while
   // there are few (us, 64 / 32: 48 tiles 32 / 24, 96 28 / 22, 240 35 / 38).
   const bool f32 = dtype == MI355_F32;
   // bf16 ones also where the input gradient is large enough for a launch of its own (16000 rows of 8 x 480 x 432, 384 tiles: 183 / 162;
   // a step of 4000 tokens of 4 x 480 x 428, four each, 192 tiles: 264 / 277).
-  const bool alone = !f32 && drows && row_tile(p, dtype, g.El, D, 512) == 128;
-  const bool dw_large = count && dw_tiles(w, g.El, 128) >= (f32 ? 448 : alone ? 300 : 512) && !(f32 && R < 400 * g.El);
-  int64_t tiles = count ? dw_tiles(w, g.El, dw_large ? 128 : 64) : 0;
+  const bool alone = !f32 && drows && row_tile(p, dtype, El, D, 512) == 128;
+  const bool dw_large = count && dw_tiles(w, El, 128) >= (f32 ? 448 : alone ? 300 : 512) && !(f32 && R < 400 * El);
+  int64_t tiles = count ? dw_tiles(w, El, dw_large ? 128 : 64) : 0;
   const bool dw_small = f32 && tiles < 160;
-  if (dw_small) tiles = dw_tiles(w, g.El, 32);
+  if (dw_small) tiles = dw_tiles(w, El, 32);
+  const int t = row_tile(p, dtype, El, D, count && !dw_large ? 512 : 150);
+  return {tiles, dw_large, dw_small, drows && count && !dw_large && t < 128, t};
+}
+
+void set_grads(AnyArgs& w, const AnyGrad* grads, int count) {
+  for (int i = 0; i < count; ++i)
+    w.dw[i] = {grads[i].a, grads[i].b, grads[i].c, (int)grads[i].M, (int)grads[i].N, 0, 0, grads[i].through};
+  w.num_dw = count;
+}
+}  // namespace
+
+bool any_backward_is_one_launch(const AnySeg& g, int dtype, const void* drows, int64_t D, const AnyGrad* grads, int count, int64_t R) {
+  const AnyArgs p = any_args(g, R);
+  AnyArgs w = any_args(g, R);
+  set_grads(w, grads, count);
+  return backward_plan(p, w, dtype, g.El, D, drows, count, R).one;
+}
+
+int any_backward(const AnySeg& g, int dtype, const void* dgate, const void* dup, const void* w1, const void* w3, void* drows,
+                 int64_t D, int64_t F, const AnyGrad* grads, int count, int64_t R, const AnyFold* f, const AnyGate* router,
+                 hipStream_t s) {
+  AnyArgs p = any_args(g, R);
+  p.a0 = dgate; p.a1 = dup; p.b0 = w1; p.b1 = w3; p.c0 = drows;
+  p.K = (int)F; p.N = (int)D; p.ldb = (int)D; p.w_elems = D * F;
+  AnyArgs w = any_args(g, R, f);
+  set_grads(w, grads, count);
+  const BackwardPlan plan = backward_plan(p, w, dtype, g.El, D, drows, count, R);
+  const int64_t tiles = plan.tiles;
+  const bool dw_large = plan.dw_large, dw_small = plan.dw_small, one = plan.one;
+  const int t = plan.t;
   MI355_REQUIRE(tiles < (1ll << 30), "grouped weight gradients: too many tiles");
-  const int t = row_tile(p, dtype, g.El, D, count && !dw_large ? 512 : 150);
-  if (drows && count && !dw_large && t < 128) {
+  MI355_REQUIRE(!router || (one && f), "grouped backward: nothing to form the gate's gradient beside");
+  if (one) {
     p.col_tiles = (int)((D + t - 1) / t);
     const int64_t dx_blocks = g.tile_capacity * (256 / t) * p.col_tiles;
     MI355_REQUIRE(dx_blocks < (1ll << 30), "grouped drows: too many tiles");
-    const dim3 grid((unsigned)(dx_blocks + tiles));
+    GateDw gate{};
+    if (router) gate = gate_dw_job(router->dlogits, router->x, router->partial, f->tokens, D, router->E);
+    const dim3 grid((unsigned)(dx_blocks + tiles + (router ? gate_dw_parts(gate) : 0)));
     const int dw_first = R / g.El > 2 * F;
     auto run = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, p, w, (int)dx_blocks, (int)tiles, dw_first);
+      hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, p, w, (int)dx_blocks, (int)tiles, dw_first, gate);
     };
     auto choose = [&](auto fold) {
       constexpr bool FOLD = decltype(fold)::value;

@@ -10,8 +10,7 @@
 
 #include "common.h"
 #include "gemm_generic.h"
-#include "row_vec.h"
-#include "select_rows.h"
+#include "select_bwd.h"
 
 namespace mi355 {
 namespace {
@@ -24,37 +23,6 @@ __device__ __forceinline__ float pick(const float (&a)[VPL], int j) {
 #pragma unroll
   for (int q = 1; q < VPL; ++q) r = (j == q) ? a[q] : r;
   return r;
-}
-
-template <int VPL>
-__device__ __forceinline__ void compute_scores(const float* __restrict__ row, int E, int lane,
-                                               int score_func, float (&s)[VPL], float (&x)[VPL]) {
-#pragma unroll
-  for (int j = 0; j < VPL; ++j) {
-    const int e = lane + j * kWave;
-    x[j] = e < E ? row[e] : -INFINITY;
-  }
-  if (score_func == MI355_SCORE_SOFTMAX) {
-    float m = x[0];
-#pragma unroll
-    for (int j = 1; j < VPL; ++j) m = fmaxf(m, x[j]);
-    m = wave_max_dpp(m);
-    float sum = 0.0f;
-#pragma unroll
-    for (int j = 0; j < VPL; ++j) {
-      s[j] = (lane + j * kWave < E) ? expf(x[j] - m) : 0.0f;
-      sum += s[j];
-    }
-    sum = wave_sum_dpp(sum);
-#pragma unroll
-    for (int j = 0; j < VPL; ++j) s[j] = s[j] / sum;
-  } else if (score_func == MI355_SCORE_SIGMOID) {
-#pragma unroll
-    for (int j = 0; j < VPL; ++j) s[j] = 1.0f / (1.0f + expf(-x[j]));
-  } else {
-#pragma unroll
-    for (int j = 0; j < VPL; ++j) s[j] = sqrtf(softplus_f32(x[j]));
-  }
 }
 
 template <int VPL>
@@ -304,146 +272,10 @@ int launch_select_rows(const SelectArgs& p, const float* logits, float* weights,
   return check_launch(what);
 }
 
-// The weights' gradient as the folded expert backward leaves it: the sum, in order, of `pieces`
-// partial dot products of the slot's row (zero for a slot without one).  Added up here, by the one
-// reader, instead of by a launch of its own.
-struct DotPieces {
-  const float* partial;  // (rows, pieces) or null: dweights holds the sums
-  const int32_t* row_of_slot;
-  int pieces, rows;
-};
-__device__ __forceinline__ float slot_dweight(const DotPieces& d, const float* dweights, int64_t slot) {
-  if (!d.partial) return dweights[slot];
-  const int row = d.row_of_slot[slot];
-  float sum = 0.0f;
-  if (row >= 0 && row < d.rows)
-    for (int i = 0; i < d.pieces; ++i) sum += d.partial[static_cast<int64_t>(row) * d.pieces + i];
-  return sum;
-}
-
-// ... or as nothing has left it yet: the output gradient and the experts' rows, whose dot products the wave of the token
-// forms itself (T of the kernel below; void: no such rows).
-struct DotRows {
-  const void *dout, *y;
-  const int32_t* row_of_slot;
-  int D, rows;
-};
-
-// The load-balance loss's part of the score gradient (aux.hip's formula), for the tokens that are not padding.
-struct BalanceGrad {
-  const float* f;  // (E) or null: no loss
-  const float* scale;
-  const uint8_t* padding;
-};
-
 template <int VPL, typename T = void>
-__global__ __launch_bounds__(256) void select_bwd_kernel(
-    const float* __restrict__ logits, const int64_t* __restrict__ ids,
-    const float* __restrict__ dweights, const float* __restrict__ dscores, DotPieces dots, DotRows rows, BalanceGrad bal,
-    float* __restrict__ dlogits, int T_, int E, int K, int score_func, int route_norm,
-    float route_scale, int mode) {
-  extern __shared__ float lds[];  // per wave: sc[E], ds[E]
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int t_raw = blockIdx.x * 4 + wave;
-  const bool active = t_raw < T_;
-  const int t = active ? t_raw : T_ - 1;  // inactive waves shadow the last token, store nothing
-  float* sc = lds + static_cast<size_t>(wave) * 2 * E;
-  float* ds = sc + E;
-
-  const float* row = logits + static_cast<int64_t>(t) * E;
-  float s[VPL];
-  float xs[VPL];
-  compute_scores<VPL>(row, E, lane, score_func, s, xs);
-  float bal_mean = 0.0f, bal_inv = 0.0f;
-  if (bal.f && !(bal.padding && bal.padding[t])) {
-    float sum = 0.0f, dot = 0.0f;
-#pragma unroll
-    for (int j = 0; j < VPL; ++j) {
-      const int e = lane + j * kWave;
-      sum += e < E ? s[j] : 0.0f;
-      dot += e < E ? s[j] * bal.f[e] : 0.0f;
-    }
-    sum = wave_sum_dpp(sum);
-    dot = wave_sum_dpp(dot);
-    // below the clamp the normalised score is s / eps and the sum no longer enters
-    const float inv = 1.0f / fmaxf(sum, 1e-12f);
-    bal_mean = sum < 1e-12f ? 0.0f : dot * inv;
-    bal_inv = *bal.scale * inv;
-  }
-#pragma unroll
-  for (int j = 0; j < VPL; ++j) {
-    const int e = lane + j * kWave;
-    if (e < E) {
-      sc[e] = s[j];
-      float d = dscores ? dscores[static_cast<int64_t>(t) * E + e] : 0.0f;
-      if (bal.f) d += (bal.f[e] - bal_mean) * bal_inv;
-      ds[e] = d;
-    }
-  }
-  __syncthreads();
-
-  constexpr bool kRows = !std::is_void_v<T>;
-  if (mode != MI355_SELECT_FIXED && (kRows || dweights || dots.partial)) {
-    // lanes 0..K-1 own one selected expert each (K <= 64)
-    int id = lane < K ? static_cast<int>(ids[static_cast<int64_t>(t) * K + lane]) : 0;
-    id = min(max(id, 0), E - 1);
-    const float sk = lane < K ? sc[id] : 0.0f;
-    float dw;
-    if constexpr (kRows) {
-      const int row = lane < K ? rows.row_of_slot[static_cast<int64_t>(t) * K + lane] : -1;
-      dw = row_dots<T>(static_cast<const T*>(rows.dout) + static_cast<int64_t>(t) * rows.D, static_cast<const T*>(rows.y),
-                       row < rows.rows ? row : -1, K, rows.D);
-    } else {
-      dw = lane < K ? slot_dweight(dots, dweights, static_cast<int64_t>(t) * K + lane) : 0.0f;
-    }
-    float g;
-    if (route_norm) {
-      const float denom = wave_sum_dpp(sk) + 1e-20f;
-      const float dot = wave_sum_dpp(dw * sk);
-      g = route_scale * (dw / denom - dot / (denom * denom));
-    } else {
-      g = route_scale * dw;
-    }
-    // scatter-add into the dense score gradient, serially so a repeated id adds up
-    for (int k = 0; k < K; ++k) {
-      const int idk = __builtin_amdgcn_readlane(id, k);
-      const float gk = lane_f32(g, k);
-      if (lane == 0) ds[idk] += gk;
-    }
-  }
-  __syncthreads();
-
-  float d[VPL];
-#pragma unroll
-  for (int j = 0; j < VPL; ++j) {
-    const int e = lane + j * kWave;
-    d[j] = e < E ? ds[e] : 0.0f;
-  }
-  if (score_func == MI355_SCORE_SOFTMAX) {
-    float dot = 0.0f;
-#pragma unroll
-    for (int j = 0; j < VPL; ++j) dot += (lane + j * kWave < E) ? s[j] * d[j] : 0.0f;
-    dot = wave_sum_dpp(dot);
-#pragma unroll
-    for (int j = 0; j < VPL; ++j) d[j] = s[j] * (d[j] - dot);
-  } else if (score_func == MI355_SCORE_SIGMOID) {
-#pragma unroll
-    for (int j = 0; j < VPL; ++j) d[j] = d[j] * s[j] * (1.0f - s[j]);
-  } else {
-#pragma unroll
-    for (int j = 0; j < VPL; ++j) {
-      const int e = lane + j * kWave;
-      const float x = e < E ? row[e] : 0.0f;
-      const float sig = 1.0f / (1.0f + expf(-x));
-      const float dsp = x > 20.0f ? 1.0f : sig;  // d softplus / dx
-      d[j] = s[j] > 0.0f ? d[j] * dsp / (2.0f * s[j]) : 0.0f;
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < VPL; ++j) {
-    const int e = lane + j * kWave;
-    if (e < E && active) dlogits[static_cast<int64_t>(t) * E + e] = d[j];
-  }
+__global__ __launch_bounds__(256) void select_bwd_kernel(SelectBwd p) {
+  extern __shared__ float lds[];
+  select_bwd_part<VPL, T>(p, blockIdx.x, lds);
 }
 
 int check_router_args(int64_t T, int64_t E, int64_t K) {
@@ -700,11 +532,10 @@ static int select_bwd(const float* logits, const int64_t* ids, const float* dwei
   MI355_REQUIRE(K <= 64, "router_select_bwd: top_k > 64 unsupported");
   if (T == 0) return MI355_OK;
   MI355_REQUIRE(logits && ids && dlogits, "router_select_bwd: null pointer");
-  const dim3 grid((unsigned)((T + 3) / 4));
-  const size_t lds = (size_t)4 * 2 * E * sizeof(float);
-  DISPATCH_VPL(E, hipLaunchKernelGGL(select_bwd_kernel<VPL>, grid, dim3(256), lds, as_stream(stream),
-                                     logits, ids, dweights, dscores_TE, dots, DotRows{}, bal, dlogits, (int)T, (int)E,
-                                     (int)K, score_func, route_norm, route_scale, select_mode));
+  const SelectBwd p{logits, ids, dweights, dscores_TE, dots, DotRows{}, bal, dlogits, (int)T, (int)E,
+                    (int)K, score_func, route_norm, route_scale, select_mode};
+  DISPATCH_VPL(E, hipLaunchKernelGGL(select_bwd_kernel<VPL>, dim3((unsigned)select_bwd_parts(p)), dim3(256), select_bwd_lds(E),
+                                     as_stream(stream), p));
   return check_launch("router_select_bwd");
 }
 
@@ -746,13 +577,11 @@ extern "C" int mi355_router_select_rows_bwd(const float* logits, const int64_t* 
   MI355_REQUIRE(logits && ids && dlogits && dout && y && row_of_slot && aligned16({dout, y}),
                 "router_select_rows_bwd: null or misaligned pointer");
   MI355_REQUIRE(!aux_f_E || aux_scale, "router_select_rows_bwd: the loss needs its scale");
-  const DotRows rows{dout, y, row_of_slot, (int)D, (int)row_capacity};
-  const BalanceGrad bal{aux_f_E, aux_scale, padding_mask_T};
-  const dim3 grid((unsigned)((T + 3) / 4));
-  const size_t lds = (size_t)4 * 2 * E * sizeof(float);
+  const SelectBwd p{logits, ids, nullptr, nullptr, DotPieces{}, DotRows{dout, y, row_of_slot, (int)D, (int)row_capacity},
+                    BalanceGrad{aux_f_E, aux_scale, padding_mask_T}, dlogits, (int)T, (int)E, (int)K, score_func, route_norm,
+                    route_scale, MI355_SELECT_TOPK};
   auto launch = [&](auto* kernel) {
-    hipLaunchKernelGGL(kernel, grid, dim3(256), lds, as_stream(stream), logits, ids, nullptr, nullptr, DotPieces{}, rows, bal,
-                       dlogits, (int)T, (int)E, (int)K, score_func, route_norm, route_scale, (int)MI355_SELECT_TOPK);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)select_bwd_parts(p)), dim3(256), select_bwd_lds(E), as_stream(stream), p);
   };
   if (dtype == MI355_F32) { DISPATCH_VPL(E, launch(select_bwd_kernel<VPL, float>)); }
   else { DISPATCH_VPL(E, launch(select_bwd_kernel<VPL, uint16_t>)); }

@@ -525,18 +525,26 @@ Grads block_backward(const Block& b, const Tensor& kept, const Tensor& dout_, co
     if (logits) select();
     if (need.experts && !side) run(kWeights, L.stream);
   } else if (b.gather) {
-    if (logits)
-      check(mi355_router_select_rows_bwd(k.logits, k.ids, ptr(dout), k.y, b.dt, k.row_of_slot, b.R, b.D, k.aux_f, k.aux_scale,
-                                         static_cast<const uint8_t*>(ptr(b.mask)), dlogits, b.T, b.E, c.K, (int)c.score_func,
-                                         (int)c.route_norm, (float)c.route_scale, L.stream),
-            "router_select_rows_bwd");
-    if (need.x || need.experts)
-      check(mi355_grouped_gather_bwd(ptr(dout), ptr(b.x), k.token_of_row, b.T, k.row_scale, ptr(b.w1), ptr(b.w3), ptr(b.w2),
-                                     k.gate, k.up, k.h, b.dt, k.seg_offsets, k.seg_counts, k.tile_expert, k.tile_row0,
-                                     k.num_tiles, b.tile_cap, dgate, dup, drows, ptr(g.w1), ptr(g.w3), ptr(g.w2),
-                                     joined_dw ? dlogits : nullptr, static_cast<float*>(gate_work), b.E, b.El, b.D, b.F, b.R,
-                                     L.stream),
+    const bool experts = need.x || need.experts;
+    auto rows = [&](auto f, auto... route) {
+      check(f(ptr(dout), ptr(b.x), k.token_of_row, b.T, k.row_scale, ptr(b.w1), ptr(b.w3), ptr(b.w2), k.gate, k.up, k.h, b.dt,
+              k.seg_offsets, k.seg_counts, k.tile_expert, k.tile_row0, k.num_tiles, b.tile_cap, dgate, dup, drows, ptr(g.w1),
+              ptr(g.w3), ptr(g.w2), route..., b.El, b.D, b.F, b.R, L.stream),
             "grouped_gather_bwd");
+    };
+    const uint8_t* padding = static_cast<const uint8_t*>(ptr(b.mask));
+    float* gate_partial = joined_dw ? static_cast<float*>(gate_work) : nullptr;
+    if (logits && experts && b.E <= 64) {
+      rows(mi355_grouped_gather_route_bwd, k.logits, k.ids, k.y, k.row_of_slot, k.aux_f, k.aux_scale, padding, dlogits, gate_partial,
+           b.E, c.K, (int)c.score_func, (int)c.route_norm, (float)c.route_scale);
+    } else {
+      if (logits)
+        check(mi355_router_select_rows_bwd(k.logits, k.ids, ptr(dout), k.y, b.dt, k.row_of_slot, b.R, b.D, k.aux_f, k.aux_scale,
+                                           padding, dlogits, b.T, b.E, c.K, (int)c.score_func, (int)c.route_norm,
+                                           (float)c.route_scale, L.stream),
+              "router_select_rows_bwd");
+      if (experts) rows(mi355_grouped_gather_bwd, joined_dw ? dlogits : nullptr, gate_partial, b.E);
+    }
     if (!joined) row_sum();
   } else {
     const int32_t* pad = c.align > 1 ? k.slot_of_row : nullptr;
