@@ -68,3 +68,40 @@ def test_experts_of_a_skewed_router_are_a_chunks_too():
         whole = ops.router_select_fwd(gate(lib, x, w, bias), None, 8, "softmax", True, 1.0)[1]
         for n in (33, 500, 513):
             assert torch.equal(ops.router_select_fwd(gate(lib, x[:n], w, bias), None, 8, "softmax", True, 1.0)[1], whole[:n]), n
+
+
+# where the launches' widths change (33 and 65 tokens, 513 of more than 32 experts), by slices of a whole batch of requests, one more and one less
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,E,K,lo,hi,splits", [
+    (20, 256, 8, 0, 32, 7), (32, 256, 8, 224, 256, 8), (33, 256, 8, 0, 32, 4), (64, 256, 16, 0, 256, 5), (65, 256, 8, 0, 32, 7), (66, 33, 16, 1, 33, 8),
+    (300, 128, 8, 0, 128, 6), (512, 64, 6, 0, 64, 1), (513, 64, 6, 0, 8, 2), (512, 200, 3, 0, 200, 8)])
+def test_slices_in_order_and_plan_at_the_widths_of_its_launches(T, E, K, lo, hi, splits):
+    """Logits are the slices' sums in their order, and ids, weights and the plan are those of the selection and the plan as two calls, with every row
+    that has no slot empty."""
+    from torchllmtuner_amd import ops
+
+    print(f"route plan T={T} E={E} K={K} [{lo},{hi}) splits={splits}", flush=True)
+    g = torch.Generator().manual_seed(T + E)
+    partial = torch.randn(splits, T, E, generator=g).cuda()
+    logits = partial[0].clone()
+    for z in range(1, splits):
+        logits += partial[z]
+    w, ids, _ = ops.router_select_fwd(logits, None, K, "softmax", True, 1.0, 0, 0)
+    plan = ops.permute_plan(ids, E, lo, hi, 1)
+    i32 = lambda n: torch.full((n,), -7, dtype=torch.int32, device="cuda")
+    cap, R_ = plan.tile_capacity, plan.row_capacity
+    got_logits, got_w, got_ids = torch.empty(T, E, device="cuda"), torch.empty(T, K, device="cuda"), torch.empty(T, K, dtype=torch.int64, device="cuda")
+    counts, offsets, seg_counts, ros, sor, tor = (i32(n) for n in (E, hi - lo + 1, 2 * (hi - lo), T * K, R_, R_))
+    scale, te, tr, nt = torch.full((R_,), float("nan"), device="cuda"), i32(cap), i32(cap), i32(1)
+    lib = _lib.load()
+    work = torch.empty(max(1, lib.mi355_route_plan_workspace_bytes(T, K, E)), dtype=torch.uint8, device="cuda")
+    _lib.check(lib.mi355_route_plan(
+        partial.data_ptr(), splits, None, got_logits.data_ptr(), None, T, E, K, 1, 1, 1.0, 0, 0, got_w.data_ptr(), got_ids.data_ptr(), lo, hi, 1,
+        ops.TILE_M, counts.data_ptr(), offsets.data_ptr(), seg_counts.data_ptr(), ros.data_ptr(), sor.data_ptr(), tor.data_ptr(), scale.data_ptr(), R_,
+        te.data_ptr(), tr.data_ptr(), nt.data_ptr(), cap, work.data_ptr(), torch.cuda.current_stream().cuda_stream), "route_plan")
+    n = int(nt)
+    for name, a, b in (("logits", got_logits, logits), ("ids", got_ids, ids), ("weights", got_w, w), ("counts", counts, plan.counts_E),
+                       ("offsets", offsets, plan.seg_offsets), ("row_of_slot", ros, plan.row_of_slot), ("slot_of_row", sor, plan.slot_of_row),
+                       ("token_of_row", tor, plan.token_of_row), ("row_scale", scale, ops.combine_row_scale(w, plan)),
+                       ("num_tiles", nt, plan.num_tiles), ("tile_expert", te[:n], plan.tile_expert[:n])):
+        assert torch.equal(a, b), name

@@ -259,7 +259,8 @@ __global__ __launch_bounds__(kLanes) void route_rank_kernel(
       p.token_of_row[i] = -1;
       if (p.row_scale) p.row_scale[i] = 0.0f;
     }
-    if (single) __threadfence();  // before this workgroup's own rows, written below
+    // (A single workgroup writes its own rows below, behind barriers, which order a workgroup's stores.  A fence for the whole device here, which
+    // writes L2 back, held the first wave up for 4.6 us at 20 tokens of a share of 256 experts.)
   }
   for (int e = tid; e < E; e += kLanes) run[e] = 0;
   if (stats)
@@ -298,7 +299,9 @@ __global__ __launch_bounds__(kLanes) void route_rank_kernel(
       } else {
         load_row<VPR, FULL>(partial + static_cast<int64_t>(t) * E, l, E, x);
       }
-      constexpr int kAhead = VPR >= 16 ? 2 : 4;  // partial sums requested together
+      // Partial sums requested together, as many as registers hold: seven slices of 256 experts were four waits for loads and are two.  That and
+      // the fence above, one rank's share, forward of 12, 20 and 32 tokens, us: 180 / 177.7, 199.3 / 197.2, 251.4 / 248.8.
+      constexpr int kAhead = VPR < 16 ? 4 : kLanes <= 512 ? 6 : 3;
       for (int z0 = 1; z0 < splits; z0 += kAhead) {
         float y[kAhead][VPR];
 #pragma unroll
@@ -443,7 +446,7 @@ __global__ __launch_bounds__(kLanes) void route_rows_kernel(const float* __restr
                                                             const int64_t* __restrict__ ids,
                                                             const uint32_t* __restrict__ rank_in_block,
                                                             const int32_t* __restrict__ block_hist, int T, int E, int K,
-                                                            int chunks, PlanOut p, Extra behind) {
+                                                            int tokens /* of a workgroup */, PlanOut p, Extra behind) {
   extern __shared__ int32_t lds[];
   const LayoutLds s(lds, E);
   const int tid = threadIdx.x;
@@ -494,7 +497,7 @@ __global__ __launch_bounds__(kLanes) void route_rows_kernel(const float* __restr
   __syncthreads();
   plan_layout(s, p, blockIdx.x == 0);
   if (blockIdx.x == 0) write_lists(s, p, E);
-  const int per_block = chunks * (kLanes / 16) * K;
+  const int per_block = tokens * K;
   const int first = blockIdx.x * per_block, last = min(T * K, first + per_block);
   for (int slot = first + tid; slot < last; slot += kLanes) {
     const int64_t e = ids[slot];
@@ -512,20 +515,29 @@ __global__ __launch_bounds__(kLanes) void route_rows_kernel(const float* __restr
 //    64, 6              7.5 / 8.1   8.2 / 8.7   11.3 / 9.6   11.3 / 10.5  11.9 / 14.7  14.2 / 15.5  14.2 / 15.7  17.6 / 15.9
 //   128, 8              9.5 / 10.3 10.9 / 11.6  13.8 / 12.2  13.9 / 13.7  14.9 / 18.0  18.8 / 19.9  19.4 / 20.1  24.1 / 21.3
 //   256, 8             14.1 / 14.4 16.9 / 17.4  20.3 / 18.7  20.9 / 21.5  21.5 / 26.3  29.0 / 29.8  31.3 / 29.2  37.1 / 31.6
-int route_lanes(int64_t T, int64_t E) { return T <= 32 || (T > 64 && T <= (E > 128 ? 7000 : 8192)) ? 512 : 1024; }
+//   Of 65 to 512 tokens four waves, one to a SIMD: two that share one take turns, and there are CUs enough.  (Not with up to 32 experts, whose selection is
+// short and has the gate's projection in front, eight waves' work.)  The second launch keeps to 512 lanes.  Block forward, us, eight waves / four: one rank's share of 256 experts of
+// 7168 x 2048, 80 tokens 317.3 / 313.6, 128 352.4 / 350.3, 256 419.6 / 413.3, 512 433.1 / 434.1; 64 of 1024 x 512, six each, 100 54.2 / 53.4, 300 56.8 / 56.1, 1000
+// 70.2 / 69.9; 128 of 2048 x 768, 256 221.1 / 220.4, 512 to 3000 the same within the spread.
+int route_lanes(int64_t T, int64_t E) {
+  if (E > 32 && T > 64 && T <= 512) return 256;
+  return T <= 32 || (T > 64 && T <= (E > 128 ? 7000 : 8192)) ? 512 : 1024;
+}
 int route_chunks(int64_t T, int64_t E) {
   const int64_t rows = route_lanes(T, E) / 16, groups = (T + rows - 1) / rows;
   return static_cast<int>((groups + kMaxBlocks - 1) / kMaxBlocks);
 }
+int64_t route_tokens(int64_t T, int64_t E) { return static_cast<int64_t>(route_chunks(T, E)) * (route_lanes(T, E) / 16); }  // of a workgroup
 int64_t route_blocks(int64_t T, int64_t E) {
-  const int64_t per = static_cast<int64_t>(route_chunks(T, E)) * (route_lanes(T, E) / 16);
+  const int64_t per = route_tokens(T, E);
   return (T + per - 1) / per;
 }
 // calls f(integral_constant lanes)
 template <typename Fn>
 void with_lanes(int64_t T, int64_t E, Fn f) {
   const int lanes = route_lanes(T, E);
-  if (lanes == 512) f(std::integral_constant<int, 512>{});
+  if (lanes == 256) f(std::integral_constant<int, 256>{});
+  else if (lanes == 512) f(std::integral_constant<int, 512>{});
   else f(std::integral_constant<int, 1024>{});
 }
 
@@ -610,10 +622,10 @@ static int route_plan(const float* partial, int splits, const float* logit_bias,
   if (histogram && blocks > 1) observe_shape(T, E, B, o.eg, o.tokens, groups, token_chunks);
   if (blocks > 1) {
     with_lanes(T, E, [&](auto lanes) {
-      constexpr int kLanes = decltype(lanes)::value;
+      constexpr int kLanes = std::max(512, decltype(lanes)::value);
       auto rows = [&](auto kernel, unsigned grid, size_t words, auto behind) {
-        hipLaunchKernelGGL(kernel, dim3(grid), dim3(kLanes), words * sizeof(int32_t), s, weights, ids, rank, hist, (int)T, (int)E, (int)K, chunks, p,
-                           behind);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(kLanes), words * sizeof(int32_t), s, weights, ids, rank, hist, (int)T, (int)E, (int)K,
+                           (int)route_tokens(T, E), p, behind);
       };
       const size_t words = layout_words((int)E);
       if (stats || groups > 0)
