@@ -36,8 +36,8 @@ enum AnyMode { ANY_GATEUP, ANY_KC, ANY_DH, ANY_DX, ANY_KS, ANY_DW };
 struct AnyDw {  // c[e] (M, N) = a[segment e]^T (rows, M) . b[segment e] (rows, N)
   const void *a, *b;
   void* c;
-  int M, N, nt, first;  // column tiles; first block of the problem
-  int through;          // FOLD: 1 a's rows through the row index, scaled; 2 b's rows through it
+  int M, N, nt;  // nt: column tiles
+  int through;   // FOLD: 1 a's rows through the row index, scaled; 2 b's rows through it
 };
 
 struct AnyArgs {
@@ -46,8 +46,8 @@ struct AnyArgs {
   const void *gate, *up;          // DH
   int K, N, ldb;                  // contraction (of one half), output columns, row length of the weights
   int64_t rows, w_elems;          // rows of the buffers, elements of one expert's weights
-  const int32_t *seg_offsets, *seg_counts, *tile_expert, *tile_row0, *num_tiles;
-  int col_tiles;
+  const int32_t *seg_offsets, *seg_counts;
+  int El, col_tiles;
   AnyDw dw[3];
   int num_dw;
   // FOLD: row r of the tokens' matrix (GATEUP a0, DH a0, a weight gradient's a or b) is its row src[r] of src_rows, of the
@@ -56,6 +56,23 @@ struct AnyArgs {
   int src_rows;
   const float* scale;
 };
+
+// Which work a workgroup has.  Consecutive workgroups go to the eight XCDs in turn, each with an L2 of its own, and tiles that share rows or weights
+// should share one.  So an XCD has a run of the row products' tiles (expert, pass of TM rows, columns), without the passes that a plan's 256-row tiles
+// leave empty, and whole rows of a weight gradient's tiles, dealt in turn: those of an expert read the same strip of the first operand, and one that has most of
+// the rows, whose contraction is the longest, is still spread over all of them (a run of whole experts per XCD: 4096 tokens of a skewed router of 16 x 640 x 1020 1564
+// -> 1770 us, and nothing more elsewhere).  A training step, us, workgroups as they come / the row products' in runs / both: fp32, 225 tokens of 16 x 628 x 832, three each,
+// 195 / 157 / 155; 400 of 16 x 640 x 1020, four each, 271 / 238 / 238; 4096 of them 1478 / 1414 / 1410; 2723 of 8 x 176 x 276, four each, 170 / 165 / 163; 1500 of 8 x 320 x
+// 400, three each, 166 / 156 / 155; bf16, four each, 4096 of 32 x 472 x 364 252 / 211 / 202, of 8 x 400 x 300 211 / 190 / 178; 4000 of 4 x 480 x 428 231 / 215 / 203;
+// 1000 of 32 x 480 x 432 142 / 131 / 128; of skewed routers 185 / 160 / 158, 1564 / 1526 / 1525, 274 / 242 / 230.
+
+// the block-th tile of `total`; false: there is none
+__device__ __forceinline__ bool any_run(int& block, int total) {
+  const int xcd = block & 7, within = block >> 3, each = total >> 3, more = total & 7;
+  if (within >= each + (xcd < more ? 1 : 0)) return false;
+  block = xcd * each + min(xcd, more) + within;
+  return true;
+}
 
 template <typename T> struct El;
 template <> struct El<float> {
@@ -285,15 +302,24 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
   bool through_a = false, through_b = false;  // K_FOLD
   int64_t first_row = 0;
   if constexpr (MODE == ANY_DW) {
-    int d = 0;
-    while (d + 1 < p.num_dw && block >= p.dw[d + 1].first) ++d;
+    const int xcd = block & 7;
+    int d = 0, at = block >> 3, strip = 0, strips, before = 0;  // at: among the XCD's tiles; before: rows of tiles of the products before
+    for (;; ++d) {
+      if (d == p.num_dw) return;
+      strips = (p.dw[d].M + TM - 1) / TM;
+      const int first = (xcd - before) & 7, all = p.El * strips, mine = all > first ? (all - first + 7) >> 3 : 0, tiles = mine * p.dw[d].nt;
+      if (at < tiles) {
+        strip = first + 8 * (at / p.dw[d].nt);
+        break;
+      }
+      at -= tiles;
+      before += all;
+    }
     const AnyDw& w = p.dw[d];
-    const int local = block - w.first;
-    const int mt = (w.M + TM - 1) / TM, per = mt * w.nt;
-    const int e = local / per, t = local - e * per;
+    const int e = strip / strips;
     M = w.M; N = w.N;
-    m0 = (t / w.nt) * TM;
-    n0 = (t % w.nt) * TN;
+    m0 = (strip - e * strips) * TM;
+    n0 = (at % w.nt) * TN;
     m_valid = min(TM, M - m0);
     k_rows = p.seg_counts[e];
     const int64_t first = p.seg_offsets[e];
@@ -317,16 +343,32 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
       }
     }
   } else {
-    constexpr int SUBS = 256 / TM;
-    const int slot = block / p.col_tiles, tile = slot / SUBS;
-    if (tile >= *p.num_tiles) return;
-    const int e = p.tile_expert[tile], cnt = p.seg_counts[e], seg0 = p.seg_offsets[e], top = p.tile_row0[tile];
-    const int end = min(top + even_tile_rows(cnt, 256), seg0 + cnt);
-    const int first = top + (slot % SUBS) * TM;
-    m_valid = min(TM, end - first);
-    if (m_valid <= 0) return;
-    row0 = first;
-    n0 = (block % p.col_tiles) * (MODE == ANY_GATEUP ? TN / 2 : TN);
+    // Which expert, pass of TM rows and columns: every wave adds up the experts' passes itself.
+    auto passes_of = [&](int count) { return (count + TM - 1) / TM; };
+    auto count_of = [&](int b) { return b + lane < p.El ? p.seg_counts[b + lane] : 0; };
+    const int count0 = count_of(0);
+    int total = 0;
+    for (int b = 0; b < p.El; b += 64) total += __builtin_amdgcn_readlane(wave_scan(passes_of(b ? count_of(b) : count0)), 63);
+    if (!any_run(block, total * p.col_tiles)) return;
+    const int pass_of_all = block / p.col_tiles;
+    int e = 0, cnt = 0, before = 0, run = 0;
+    for (int b = 0; b < p.El; b += 64) {
+      const int c = b ? count_of(b) : count0, to = run + wave_scan(passes_of(c));
+      const unsigned long long past = __ballot(to > pass_of_all);
+      if (past) {
+        const int l = __ffsll(past) - 1;
+        e = b + l;
+        cnt = __builtin_amdgcn_readlane(c, l);
+        before = __builtin_amdgcn_readlane(to, l) - passes_of(cnt);
+        break;
+      }
+      run = __builtin_amdgcn_readlane(to, 63);
+    }
+    const int q = block - before * p.col_tiles;
+    const int pass = q / p.col_tiles;
+    row0 = p.seg_offsets[e] + pass * TM;
+    m_valid = min(TM, cnt - pass * TM);
+    n0 = (q - pass * p.col_tiles) * (MODE == ANY_GATEUP ? TN / 2 : TN);
     A0 = static_cast<const T*>(p.a0) + (ROWS_FOLD ? 0 : row0 * lda);
     a_bytes = (ROWS_FOLD ? p.src_rows : p.rows - row0) * lda * static_cast<int64_t>(sizeof(T));
     if (MODE == ANY_DX) A1 = static_cast<const T*>(p.a1) + row0 * lda;
@@ -778,6 +820,9 @@ int launch_any(const AnyArgs& p, int dtype, int64_t blocks, hipStream_t s, const
   return check_launch(what);
 }
 
+// passes of t rows that the experts have, at most
+int64_t any_passes(const AnyArgs& p, int64_t t) { return p.rows / t + std::min<int64_t>(p.El, p.rows); }
+
 // Large tiles (128 x 128) once they give two workgroups for every CU, for bf16 already where they give every second CU one: its
 // steps are mostly loads and LDS, which a large tile has half as many of (the forward, us, 64 / 128: 141 tiles, 2000 rows of 32 x
 // 300 x 300, 18.3 / 19.0; 156, 4000 of 8 x 480 x 432, 30.7 / 26.4; 186, 6000 of 16 x 440 x 360, 41.7 / 34.6; 252, 4000 of 32 x
@@ -794,32 +839,38 @@ int launch_any(const AnyArgs& p, int dtype, int64_t blocks, hipStream_t s, const
 // 600 of 16 x 512 x 800, four each, 283 / 243, 1000 of 8 x 640 x 640, two each, 229 / 205; from 2000 tokens of 16 x 640 x 1020 on the same.
 // bf16 steps are shorter and gain nothing (14 / 17 against 14 / 18, slower with more tiles).
 int row_tile(const AnyArgs& p, int dtype, int64_t El, int64_t cols, int bf16_large) {
-  auto tiles = [&](int64_t t) { return (p.rows / t + std::min(El, p.rows)) * ((cols + t - 1) / t); };
+  auto tiles = [&](int64_t t) { return any_passes(p, t) * ((cols + t - 1) / t); };
   if (dtype == MI355_F32 && (p.rows <= 64 * El || tiles(64) < 200)) return 32;
   return tiles(128) >= (dtype == MI355_F32 ? 512 : bf16_large) ? 128 : 64;
 }
 
 template <int MODE>
-int launch_rows(AnyArgs& p, int dtype, int64_t tile_capacity, int64_t El, int64_t cols, hipStream_t s, const char* what,
+int launch_rows(AnyArgs& p, int dtype, int64_t El, int64_t cols, hipStream_t s, const char* what,
                 const GateDw* gate = nullptr, const SelectBwd* select = nullptr) {
   constexpr bool GU = MODE == ANY_GATEUP;
   const int t = row_tile(p, dtype, El, cols, MODE == ANY_DH ? 512 : 150), width = GU && t == 128 ? 64 : t;
   p.col_tiles = (int)((cols + width - 1) / width);
-  const int64_t blocks = tile_capacity * (256 / t) * p.col_tiles;
+  const int64_t blocks = any_passes(p, t) * p.col_tiles;
   MI355_REQUIRE(blocks < (1ll << 30), "%s: too many tiles", what);
   if (t == 128) return launch_any<MODE, 128, 128>(p, dtype, blocks, s, what, gate, select);
   return t == 64 ? launch_any<MODE, 64, GU ? 128 : 64>(p, dtype, blocks, s, what, gate, select)
                  : launch_any<MODE, 32, GU ? 64 : 32>(p, dtype, blocks, s, what, gate, select);
 }
 
+// the weight gradients' tiles, and each one's columns of them
 int64_t dw_tiles(AnyArgs& p, int64_t El, int tile) {
-  int64_t blocks = 0;
+  int64_t tiles = 0;
   for (int d = 0; d < p.num_dw; ++d) {
     AnyDw& w = p.dw[d];
     w.nt = (w.N + tile - 1) / tile;
-    w.first = (int)blocks;
-    blocks += El * ((w.M + tile - 1) / tile) * w.nt;
+    tiles += El * ((w.M + tile - 1) / tile) * w.nt;
   }
+  return tiles;
+}
+// the workgroups of those: of each product a whole round of rows of tiles over the XCDs
+int64_t dw_blocks(const AnyArgs& p, int tile) {
+  int64_t blocks = 0;
+  for (int d = 0; d < p.num_dw; ++d) blocks += (p.El * ((p.dw[d].M + tile - 1) / tile) + 7) / 8 * 8 * static_cast<int64_t>(p.dw[d].nt);
   return blocks;
 }
 
@@ -834,12 +885,12 @@ bool any_path_ok(int dtype, int64_t D, int64_t F, int64_t R, std::initializer_li
 
 static AnyArgs any_args(const AnySeg& g, int64_t rows, const AnyFold* f = nullptr) {
   AnyArgs p{};
+  p.El = (int)g.El;
   if (f) {
     p.src = f->token_of_row; p.src_rows = (int)f->tokens; p.scale = f->row_scale;
   }
   p.rows = rows;
-  p.seg_offsets = g.seg_offsets; p.seg_counts = g.seg_counts; p.tile_expert = g.tile_expert;
-  p.tile_row0 = g.tile_row0; p.num_tiles = g.num_tiles;
+  p.seg_offsets = g.seg_offsets; p.seg_counts = g.seg_counts;
   return p;
 }
 
@@ -848,7 +899,7 @@ int any_gateup(const AnySeg& g, int dtype, const void* rows, const void* w1, con
   AnyArgs p = any_args(g, R, f);
   p.a0 = rows; p.b0 = w1; p.b1 = w3; p.c0 = gate; p.c1 = up; p.c2 = h;
   p.K = (int)D; p.N = (int)F; p.ldb = (int)D; p.w_elems = D * F;
-  return launch_rows<ANY_GATEUP>(p, dtype, g.tile_capacity, g.El, F, s, "grouped gate/up");
+  return launch_rows<ANY_GATEUP>(p, dtype, g.El, F, s, "grouped gate/up");
 }
 
 int any_linear(const AnySeg& g, int dtype, const void* x, const void* w, void* y, int64_t I, int64_t O, int64_t R,
@@ -856,7 +907,7 @@ int any_linear(const AnySeg& g, int dtype, const void* x, const void* w, void* y
   AnyArgs p = any_args(g, R);
   p.a0 = x; p.b0 = w; p.c0 = y;
   p.K = (int)I; p.N = (int)O; p.ldb = (int)I; p.w_elems = I * O;
-  return launch_rows<ANY_KC>(p, dtype, g.tile_capacity, g.El, O, s, "grouped linear");
+  return launch_rows<ANY_KC>(p, dtype, g.El, O, s, "grouped linear");
 }
 
 int any_linear_dx(const AnySeg& g, int dtype, const void* dy, const void* w, void* dx, int64_t I, int64_t O, int64_t R,
@@ -864,7 +915,7 @@ int any_linear_dx(const AnySeg& g, int dtype, const void* dy, const void* w, voi
   AnyArgs p = any_args(g, R);
   p.a0 = dy; p.b0 = w; p.c0 = dx;
   p.K = (int)O; p.N = (int)I; p.ldb = (int)I; p.w_elems = I * O;
-  return launch_rows<ANY_KS>(p, dtype, g.tile_capacity, g.El, I, s, "grouped linear dx");
+  return launch_rows<ANY_KS>(p, dtype, g.El, I, s, "grouped linear dx");
 }
 
 int any_dh(const AnySeg& g, int dtype, const void* dy, const void* w2, const void* gate, const void* up, void* dgate,
@@ -880,13 +931,12 @@ int any_dh(const AnySeg& g, int dtype, const void* dy, const void* w2, const voi
     sel = {select->logits, select->ids, nullptr, nullptr, DotPieces{}, DotRows{select->dout, select->y, select->row_of_slot, (int)D, (int)R},
            BalanceGrad{select->aux_f, select->aux_scale, select->padding}, select->dlogits, (int)f->tokens, (int)select->E,
            (int)select->K, select->score_func, select->route_norm, select->route_scale, MI355_SELECT_TOPK};
-  return launch_rows<ANY_DH>(p, dtype, g.tile_capacity, g.El, F, s, "grouped dh", router ? &job : nullptr, select ? &sel : nullptr);
+  return launch_rows<ANY_DH>(p, dtype, g.El, F, s, "grouped dh", router ? &job : nullptr, select ? &sel : nullptr);
 }
 
 namespace {
 // How a backward pass is launched: the weight gradients' tile, the input gradient's, and whether they share a launch.
 struct BackwardPlan {
-  int64_t tiles;
   bool dw_large, dw_small, one;
   int t;
 };
@@ -899,16 +949,16 @@ BackwardPlan backward_plan(const AnyArgs& p, AnyArgs& w, int dtype, int64_t El, 
   // a step of 4000 tokens of 4 x 480 x 428, four each, 192 tiles: 264 / 277).
   const bool alone = !f32 && drows && row_tile(p, dtype, El, D, 512) == 128;
   const bool dw_large = count && dw_tiles(w, El, 128) >= (f32 ? 448 : alone ? 300 : 512) && !(f32 && R < 400 * El);
-  int64_t tiles = count ? dw_tiles(w, El, dw_large ? 128 : 64) : 0;
+  const int64_t tiles = dw_tiles(w, El, dw_large ? 128 : 64);
   const bool dw_small = f32 && tiles < 160;
-  if (dw_small) tiles = dw_tiles(w, El, 32);
+  if (dw_small) dw_tiles(w, El, 32);
   const int t = row_tile(p, dtype, El, D, count && !dw_large ? 512 : 150);
-  return {tiles, dw_large, dw_small, drows && count && !dw_large && t < 128, t};
+  return {dw_large, dw_small, drows && count && !dw_large && t < 128, t};
 }
 
 void set_grads(AnyArgs& w, const AnyGrad* grads, int count) {
   for (int i = 0; i < count; ++i)
-    w.dw[i] = {grads[i].a, grads[i].b, grads[i].c, (int)grads[i].M, (int)grads[i].N, 0, 0, grads[i].through};
+    w.dw[i] = {grads[i].a, grads[i].b, grads[i].c, (int)grads[i].M, (int)grads[i].N, 0, grads[i].through};
   w.num_dw = count;
 }
 }  // namespace
@@ -929,14 +979,14 @@ int any_backward(const AnySeg& g, int dtype, const void* dgate, const void* dup,
   AnyArgs w = any_args(g, R, f);
   set_grads(w, grads, count);
   const BackwardPlan plan = backward_plan(p, w, dtype, g.El, D, drows, count, R);
-  const int64_t tiles = plan.tiles;
+  const int64_t tiles = dw_blocks(w, plan.dw_small ? 32 : plan.dw_large ? 128 : 64);
   const bool dw_large = plan.dw_large, dw_small = plan.dw_small, one = plan.one;
   const int t = plan.t;
   MI355_REQUIRE(tiles < (1ll << 30), "grouped weight gradients: too many tiles");
   MI355_REQUIRE(!router || (one && f), "grouped backward: nothing to form the gate's gradient beside");
   if (one) {
     p.col_tiles = (int)((D + t - 1) / t);
-    const int64_t dx_blocks = g.tile_capacity * (256 / t) * p.col_tiles;
+    const int64_t dx_blocks = any_passes(p, t) * p.col_tiles;
     MI355_REQUIRE(dx_blocks < (1ll << 30), "grouped drows: too many tiles");
     GateDw gate{};
     if (router) gate = gate_dw_job(router->dlogits, router->x, router->partial, f->tokens, D, router->E);
@@ -956,7 +1006,7 @@ int any_backward(const AnySeg& g, int dtype, const void* dgate, const void* dup,
     return check_launch("grouped drows and weight gradients");
   }
   if (drows)
-    if (int rc = launch_rows<ANY_DX>(p, dtype, g.tile_capacity, g.El, D, s, "grouped drows")) return rc;
+    if (int rc = launch_rows<ANY_DX>(p, dtype, g.El, D, s, "grouped drows")) return rc;
   if (!count) return MI355_OK;
   if (dw_small) return launch_any<ANY_DW, 32, 32>(w, dtype, tiles, s, "grouped weight gradients");
   return dw_large ? launch_any<ANY_DW, 128, 128>(w, dtype, tiles, s, "grouped weight gradients")
