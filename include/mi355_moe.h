@@ -452,6 +452,11 @@ int mi355_combine_fwd(const void* y, int dtype, const float* weights_TK,
 int mi355_combine_add_fwd(const void* y, int dtype, const float* weights_TK, const int32_t* row_of_slot,
                           const void* addend, void* out, int64_t T, int64_t D, int64_t K, int round_terms,
                           void* stream);
+/* The same, and totals_E[e] += counts_E[e] for E experts (fp32; NULL: nothing to add): a router's running
+ * counts.  Calls that add to the same totals are the caller's to order. */
+int mi355_combine_count_fwd(const void* y, int dtype, const float* weights_TK, const int32_t* row_of_slot,
+                            const void* addend, void* out, int64_t T, int64_t D, int64_t K, int round_terms,
+                            const int32_t* counts_E, float* totals_E, int64_t E, void* stream);
 
 
 /*

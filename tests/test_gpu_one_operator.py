@@ -423,3 +423,53 @@ def test_default_overlap_adds_the_input_gradients_in_another_order_than_the_stag
     bound = 2.0 ** -8 * (routed_gate.abs() + (routed + shared).abs() + 2 * total.abs()) * (1 + 2.0 ** -5) + 1e-30
     diff = (one[0].double() - stages[0].double()).abs()
     assert bool((diff <= bound).all()), float((diff / bound).max())
+
+
+@pytest.mark.parametrize("dtype,T,D,F", [(torch.bfloat16, 700, 512, 384), (torch.bfloat16, 3, 512, 384), (torch.float32, 300, 64, 100)])
+@pytest.mark.parametrize("padded", [False, True])
+def test_running_counts_are_added_once_whichever_launch_adds_them(dtype, T, D, F, padded):
+    """In the combine's launch, or, where a checkpoint may replay the forward and stop before its end, behind it; without gradients too, and for
+    buffers that the operator does not take."""
+    from torch.utils.checkpoint import checkpoint
+
+    from torchllmtuner_amd.moe.layer import in_checkpoint_recompute
+
+    E, K = 20, 3
+    print(f"running counts {dtype} T={T} padded={padded}", flush=True)
+    p = make_params(E, D, F, dtype, seed=T, std=0.05)
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T, D, generator=g).to(dtype).to(DEV)
+    mask = (torch.rand(T, generator=g) < 0.3).to(DEV) if padded else None
+    block = build_block(p, R.RouterSpec(E, K, score_func="softmax", route_norm=True), D, F, dtype, DEV).train()
+    with torch.no_grad():
+        ids = block._forward_as_one(x, mask)
+        want = ids[1].double()
+    assert want.sum() == K * (T if mask is None else int((~mask).sum())) and not block.tokens_per_expert_E.any()
+
+    def counted(run, times=1):
+        block.tokens_per_expert_E.fill_(5.0)
+        run()
+        assert torch.equal(block.tokens_per_expert_E.double(), 5.0 + times * want)
+
+    call = lambda: block(x.clone().requires_grad_(), padding_mask=mask)
+    assert block._totals(x) is block.tokens_per_expert_E
+    counted(call)
+    counted(lambda: (call(), call()), 2)
+    counted(lambda: torch.no_grad()(call)())
+    counted(lambda: checkpoint(call, use_reentrant=False).sum().backward())
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t):
+        assert block._totals(x) is None
+        counted(call)
+    handle = block.router.register_forward_hook(lambda *a: None)  # the stages
+    counted(call)
+    handle.remove()
+    token = in_checkpoint_recompute.set(True)
+    counted(call, 0)
+    in_checkpoint_recompute.reset(token)
+    block.eval()
+    counted(call, 0)
+    block.train()
+    for other in (torch.zeros(E, dtype=torch.float64, device=DEV), torch.zeros(E, 2, device=DEV)[:, 0]):
+        block.tokens_per_expert_E = other
+        assert block._totals(x) is None
+        counted(call)

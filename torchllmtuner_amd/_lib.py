@@ -110,6 +110,7 @@ SIGNATURES = {
          P, P, P, P, P, P, P, I, P, F, P, P],
     ),
     "mi355_combine_add_fwd": (I, [P, I, P, P, P, P, L, L, L, I, P]),
+    "mi355_combine_count_fwd": (I, [P, I, P, P, P, P, L, L, L, I, P, P, L, P]),
     "mi355_permute_rows_add_bwd": (I, [P, I, P, P, P, L, L, L, P]),
     "mi355_segments_dense": (I, [L, L, P, P, P, P, P, L, P]),
     "mi355_route_plan_covers": (I, [L, L, I, I]),

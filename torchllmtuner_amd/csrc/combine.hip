@@ -41,8 +41,12 @@ template <typename T, bool SMALL_K>
 __global__ __launch_bounds__(256) void combine_fwd_kernel(
     const T* __restrict__ y, const float* __restrict__ weights,
     const int32_t* __restrict__ row_of_slot, const T* __restrict__ addend, T* __restrict__ out, int T_, int D, int K,
-    int round_terms, int pieces) {
+    int round_terms, int pieces, const int32_t* __restrict__ counts, float* __restrict__ totals, int E) {
   const int lane = threadIdx.x & 63;
+  // A router's running counts.  As a launch behind this one, a training step, us, apart / here: 512 fp32 tokens of 8 x 256 x 512 128 / 124.5, 225 of 16 x 628 x 832 154.2 /
+  // 151.4; bf16 1000 of 16 x 1024 x 512 151.7 / 148.7, 283, 1000 and 3000 of 64 of it 184 / 181, 229 / 225.7, 345 / 342, 300 and 1000 of 128 x 2048 x 768 698 / 692, 766 / 761.
+  if (totals && blockIdx.x == 0)
+    for (int e = threadIdx.x; e < E; e += 256) totals[e] += static_cast<float>(counts[e]);
   const int tokens = blockIdx.x / pieces, piece = blockIdx.x % pieces;
   const int t = tokens * 4 + (threadIdx.x >> 6);
   if (t >= T_) return;
@@ -294,20 +298,22 @@ __global__ __launch_bounds__(256) void combine_bwd_f64_kernel(
 
 using namespace mi355;
 
-extern "C" int mi355_combine_add_fwd(const void* y, int dtype, const float* weights, const int32_t* row_of_slot,
-                                     const void* addend, void* out, int64_t T, int64_t D, int64_t K, int round_terms,
-                                     void* stream) {
+extern "C" int mi355_combine_count_fwd(const void* y, int dtype, const float* weights, const int32_t* row_of_slot,
+                                       const void* addend, void* out, int64_t T, int64_t D, int64_t K, int round_terms,
+                                       const int32_t* counts, float* totals, int64_t E, void* stream) {
   MI355_REQUIRE(T >= 0 && D >= 1 && K >= 1 && K <= 64 && T < (1ll << 31) && D < (1ll << 31),
                 "combine_fwd: bad shape (K must be <= 64)");
   if (T == 0) return MI355_OK;
   MI355_REQUIRE(weights && row_of_slot && out, "combine_fwd: null pointer");
-  MI355_REQUIRE(!addend || dtype != MI355_F64, "combine_fwd: no fp64 form with an addend");
+  MI355_REQUIRE((!addend && !totals) || dtype != MI355_F64, "combine_fwd: no fp64 form with an addend or counts");
+  MI355_REQUIRE(!totals || (counts && E >= 1 && E < (1ll << 31)), "combine_fwd: totals without counts");
   const int64_t tokens = (T + 3) / 4;  // groups of one workgroup's four
   const int64_t kib = (D * (dtype == MI355_F32 ? 4 : 2) + 1023) / 1024;  // 64 lanes of 16 bytes
   const int64_t pieces = std::max<int64_t>(1, std::min<int64_t>(kib, 0xffffff / tokens));  // a launch: below 2^32 lanes
   auto launch = [&](auto kernel, auto* yp, auto* op) {
     hipLaunchKernelGGL(kernel, dim3((unsigned)(tokens * pieces)), dim3(256), 0, as_stream(stream), yp, weights, row_of_slot,
-                       static_cast<decltype(yp)>(addend), op, (int)T, (int)D, (int)K, round_terms, (int)pieces);
+                       static_cast<decltype(yp)>(addend), op, (int)T, (int)D, (int)K, round_terms, (int)pieces, counts,
+                       totals, (int)E);
   };
   auto run = [&](auto* yp, auto* op) {
     using E = std::remove_pointer_t<decltype(op)>;
@@ -323,6 +329,12 @@ extern "C" int mi355_combine_add_fwd(const void* y, int dtype, const float* weig
   } else
     return fail(MI355_EINVAL, "combine_fwd: unknown dtype %d", dtype);
   return check_launch("combine_fwd");
+}
+
+extern "C" int mi355_combine_add_fwd(const void* y, int dtype, const float* weights, const int32_t* row_of_slot,
+                                     const void* addend, void* out, int64_t T, int64_t D, int64_t K, int round_terms,
+                                     void* stream) {
+  return mi355_combine_count_fwd(y, dtype, weights, row_of_slot, addend, out, T, D, K, round_terms, nullptr, nullptr, 0, stream);
 }
 
 extern "C" int mi355_combine_fwd(const void* y, int dtype, const float* weights,

@@ -57,6 +57,7 @@ struct Config {
 struct Stats {
   Tensor histogram, aux_acc, aux_denominator;
   double aux_coeff = 0.0;
+  Tensor totals;  // what the counts per expert are added to
 };
 
 // The block's tensors; undefined where the block has none.
@@ -227,7 +228,7 @@ bool few_choices(const Block& b, const Stats& st) {
          !st.histogram.defined() && b.T <= 4 && b.c.lo == 0 && b.c.hi == b.E && mi355_choice_covers(b.T, b.D, b.F, b.E, b.c.K, (int)b.c.num_groups);
 }
 
-std::tuple<Tensor, Tensor> choices_forward(const Block& b) {
+std::tuple<Tensor, Tensor> choices_forward(const Block& b, const Tensor& totals) {
   Launch L(b.x);
   const Config& c = b.c;
   const auto opts = b.x.options();
@@ -265,6 +266,7 @@ std::tuple<Tensor, Tensor> choices_forward(const Block& b) {
         "choice_gateup_fwd");
   if (b.Fs > 0 && !aux) shared_forward(b, k, y_shared, L.stream, false);
   shared.join();
+  if (totals.defined()) totals.add_(counts);
   check(mi355_choice_down_fwd(h, ptr(b.w2), weights, ids, y_shared, ptr(out), b.T, c.K, b.El, b.D, b.F, (int)c.round_terms,
                               L.stream),
         "choice_down_fwd");
@@ -375,8 +377,8 @@ std::tuple<Tensor, Tensor, Tensor> block_forward(const Block& b, const Stats& st
           "grouped_swiglu_fwd");
   if (b.Fs > 0 && !aux) shared_forward(b, k, y_shared, L.stream, false);
   shared.join();
-  check(mi355_combine_add_fwd(y, b.dt, k.weights, k.row_of_slot, y_shared, ptr(out), b.T, b.D, c.K, (int)c.round_terms,
-                              L.stream),
+  check(mi355_combine_count_fwd(y, b.dt, k.weights, k.row_of_slot, y_shared, ptr(out), b.T, b.D, c.K, (int)c.round_terms,
+                                iptr(counts), st.totals.defined() ? st.totals.data_ptr<float>() : nullptr, b.E, L.stream),
         "combine_fwd");
   return {out, counts, kept};
 }
@@ -598,10 +600,11 @@ OptTensor opt(const Tensor& t) { return t.defined() ? OptTensor(t) : std::nullop
       const Tensor &w3, const Tensor &w2, const OptTensor &sg, const OptTensor &su, const OptTensor &sd, int64_t K, \
       int64_t score_func, bool route_norm, double route_scale, int64_t num_groups, int64_t num_limited, int64_t lo, \
       int64_t hi, int64_t align, bool round_terms, bool overlap_shared, const OptTensor &mask,                     \
-      const OptTensor &histogram, const OptTensor &aux_denominator, double aux_coeff, const OptTensor &aux_acc
+      const OptTensor &histogram, const OptTensor &aux_denominator, double aux_coeff, const OptTensor &aux_acc,    \
+      const OptTensor &totals
 #define BLOCK_ARGS                                                                                                 \
   x, gate_w, gate_b, expert_b, w1, w3, w2, sg, su, sd, K, score_func, route_norm, route_scale, num_groups,         \
-      num_limited, lo, hi, align, round_terms, overlap_shared, mask, histogram, aux_denominator, aux_coeff, aux_acc
+      num_limited, lo, hi, align, round_terms, overlap_shared, mask, histogram, aux_denominator, aux_coeff, aux_acc, totals
 
 using BlockSig = std::tuple<Tensor, Tensor>(BLOCK_PARAMS);
 using BlockFwdSig = std::tuple<Tensor, Tensor, Tensor>(BLOCK_PARAMS);
@@ -625,7 +628,7 @@ struct MoeBlock : public torch::autograd::Function<MoeBlock> {
     return {out, counts};
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    variable_list out(26);
+    variable_list out(27);
     if (!grads[0].defined()) return out;
     const auto s = ctx->get_saved_variables();
     const auto c = ctx->saved_data["config"].toIntVector();
@@ -700,6 +703,9 @@ void check_stats(const Block& b, const Stats& st) {
                          st.histogram.dim() == 2 && st.histogram.size(0) == b.gate_w.size(0) &&
                          st.histogram.device() == b.x.device() && b.expert_b.defined()),
                     "histogram: contiguous int64 (experts, bins) beside an expert bias");
+  TORCH_CHECK_VALUE(!st.totals.defined() || (st.totals.scalar_type() == at::kFloat && st.totals.is_contiguous() &&
+                                             st.totals.numel() == b.gate_w.size(0) && st.totals.device() == b.x.device()),
+                    "totals: contiguous fp32, one per expert");
   auto scalar = [&](const Tensor& t) { return !t.defined() || (t.numel() == 1 && t.device() == b.x.device()); };
   TORCH_CHECK_VALUE(scalar(st.aux_acc) && scalar(st.aux_denominator) &&
                         (!st.aux_denominator.defined() || st.aux_denominator.scalar_type() == at::kFloat) &&
@@ -710,7 +716,7 @@ void check_stats(const Block& b, const Stats& st) {
 
 // The block of a forward call, checked.
 std::pair<Block, Stats> block_of(BLOCK_PARAMS) {
-  const Stats st{some(histogram), some(aux_acc), some(aux_denominator), aux_coeff};
+  const Stats st{some(histogram), some(aux_acc), some(aux_denominator), aux_coeff, some(totals)};
   Block b{dense(x), dense(gate_w), dense(gate_b), dense(expert_b), dense(w1), dense(w3), dense(w2), dense(sg), dense(su),
           dense(sd), dense(mask),
           Config{K, score_func, route_norm, num_groups, num_limited, lo, hi, align, round_terms, overlap_shared,
@@ -723,7 +729,7 @@ std::pair<Block, Stats> block_of(BLOCK_PARAMS) {
 
 std::tuple<Tensor, Tensor> moe_block(BLOCK_PARAMS) {
   const auto [b, st] = block_of(BLOCK_ARGS);
-  if (few_choices(b, st)) return choices_forward(b);
+  if (few_choices(b, st)) return choices_forward(b, st.totals);
   auto [out, counts, kept] = block_forward(b, st, false);
   return {out, counts};
 }
@@ -800,7 +806,7 @@ TORCH_LIBRARY_FRAGMENT(mi355_moe, m) {
       "Tensor? shared_gate, Tensor? shared_up, Tensor? shared_down, int top_k, int score_func, bool route_norm, "
       "float route_scale, int num_groups, int num_limited, int local_lo, int local_hi, int align, bool round_terms, "
       "bool overlap_shared, Tensor? padding_mask, Tensor(a!)? histogram, Tensor? aux_denominator, float aux_coeff, "
-      "Tensor(b!)? aux_acc)";
+      "Tensor(b!)? aux_acc, Tensor(c!)? totals=None)";
   m.def(("moe_block" + args + " -> (Tensor, Tensor)").c_str());
   m.def(("moe_block_fwd" + args + " -> (Tensor, Tensor, Tensor)").c_str());
   // a gradient that is not asked for is undefined (None)

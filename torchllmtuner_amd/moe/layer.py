@@ -232,7 +232,27 @@ class MoE(nn.Module):
                 stats["aux_acc"] = aux.instance_acc
         return stats
 
-    def _forward_as_one(self, tokens: torch.Tensor, padding_mask: torch.Tensor | None = None):
+    def _totals(self, tokens: torch.Tensor):
+        """The running counts where the one operator may add to them itself, else None: the addition is then the last thing of
+        ``forward``.  A checkpoint replays the forward under a hook on what it saves, and stops it before its end; the operator
+        would already have counted."""
+        if torch.compiler.is_compiling() or not self.training or in_checkpoint_recompute.get():
+            return None
+        if torch._C._autograd._top_saved_tensors_default_hooks(True) is not None:
+            return None
+        totals = self._buffers.get("tokens_per_expert_E")
+        if (
+            type(totals) is not torch.Tensor
+            or totals.dtype is not torch.float32
+            or totals.device != tokens.device
+            or totals.requires_grad
+            or not totals.is_contiguous()
+            or totals.numel() != self.router.num_experts
+        ):
+            return None
+        return totals
+
+    def _forward_as_one(self, tokens: torch.Tensor, padding_mask: torch.Tensor | None = None, totals: torch.Tensor | None = None):
         """``(output, counts per expert)`` from the one operator that computes the whole block
         (``mi355_moe::moe_block``), or None when a stage has to be visible or is not what it computes: a
         hook or an override anywhere below, an observer, another auxiliary loss, router, dispatcher,
@@ -304,7 +324,7 @@ class MoE(nn.Module):
             tokens, gate_weight, gate_bias, self.expert_bias_E, w1, w3, w2, shared,
             router.top_k, router.score_func, router.route_norm, router.route_scale, router.num_expert_groups,
             router.num_limited_groups, lo, hi, dispatcher._align(), not dispatcher.accumulate_in_fp32,
-            self.overlap_shared_experts, **stats)
+            self.overlap_shared_experts, totals=totals, **stats)
 
     def set_padding_mask(self, padding_mask: torch.Tensor | None) -> None:
         self._pending_padding_mask = padding_mask
@@ -325,10 +345,11 @@ class MoE(nn.Module):
                     f"got {tuple(padding_mask.shape)} for {tokens.shape[0]} tokens."
                 )
 
-        whole = self._forward_as_one(tokens, padding_mask)
+        totals = self._totals(tokens)
+        whole = self._forward_as_one(tokens, padding_mask, totals)
         if whole is not None:
             out_TD, num_tokens_per_expert_E = whole
-            if self.training and not in_checkpoint_recompute.get():
+            if totals is None and self.training and not in_checkpoint_recompute.get():
                 self.tokens_per_expert_E.add_(num_tokens_per_expert_E)  # (neither takes part in autograd)
             if restore_shape:
                 out_TD = out_TD.reshape(*x.shape[:-1], out_TD.shape[-1])

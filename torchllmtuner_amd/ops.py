@@ -293,7 +293,7 @@ def _(dout, x, weights, w1, w3, w2, gate, up, token_of_row, slot_of_row, row_of_
 @_fake("moe_block")
 def _(x, gate_w, gate_bias, expert_bias, w1, w3, w2, shared_gate, shared_up, shared_down, top_k, score_func, route_norm,
       route_scale, num_groups, num_limited, local_lo, local_hi, align, round_terms, overlap_shared,
-      padding_mask, histogram, aux_denominator, aux_coeff, aux_acc):
+      padding_mask, histogram, aux_denominator, aux_coeff, aux_acc, totals=None):
     return torch.empty_like(x), x.new_empty((gate_w.shape[0],), dtype=torch.int32)
 
 
@@ -695,16 +695,17 @@ def route_plan_covers(num_experts, top_k, num_groups) -> bool:
 
 def moe_block(x_TD, gate_w_ED, gate_bias_E, expert_bias_E, w1_EFD, w3_EFD, w2_EDF, shared, top_k, score_func, route_norm,
               route_scale, num_groups, num_limited, local_lo, local_hi, align, round_terms, overlap_shared,
-              padding_mask=None, histogram=None, aux_denominator=None, aux_coeff=0.0, aux_acc=None):
+              padding_mask=None, histogram=None, aux_denominator=None, aux_coeff=0.0, aux_acc=None, totals=None):
     """The block of ``moe.MoE`` as one operator: ``(output, int32 counts per expert)``, differentiable in the
     tokens and every weight.  ``shared``: the shared expert's (gate, up, down) weights or three Nones.
     ``padding_mask``: its tokens are left out of the counts, the histogram and the loss.  ``histogram``: the
     required-bias histogram to add to.  ``aux_denominator`` (fp32 on the device): inject the load-balance loss times
-    ``aux_coeff`` over it into the backward, and add the loss over it to ``aux_acc``."""
+    ``aux_coeff`` over it into the backward, and add the loss over it to ``aux_acc``.  ``totals`` (fp32, one per expert): what the
+    counts are added to."""
     return _moe_block(x_TD, gate_w_ED, gate_bias_E, expert_bias_E, w1_EFD, w3_EFD, w2_EDF, *shared, top_k,
                       SCORE_FUNCS[score_func], route_norm, route_scale, num_groups or 0, num_limited or 0, local_lo,
                       local_hi, align, round_terms, overlap_shared, padding_mask, histogram, aux_denominator, aux_coeff,
-                      aux_acc)
+                      aux_acc, totals)
 
 
 # ====================================================================== profiling hooks
