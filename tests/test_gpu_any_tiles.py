@@ -21,12 +21,16 @@ COUNTS = {
     "65": (0,) * 64 + (70,),
     "130": tuple(0 if i % 3 else 40 + i for i in range(130)),
     "most": (1400, 20, 31, 2, 50, 0, 17, 8, 64),
+    # bf16 input and weight gradients on small tiles in one launch: large ones would cover a quarter more; a product just small enough and one past it
+    "covers": (2100, 0, 1900, 2300, 1701),
+    "small": (3000, 3100, 3050, 2900),
+    "large": (4000, 3000, 3600, 3401),
 }
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("name,D,Fd", [("one", 64, 36), ("ends", 132, 200), ("few", 512, 260), ("64", 72, 100), ("65", 64, 64), ("130", 68, 132),
-                                       ("most", 324, 232)])
+                                       ("most", 324, 232), ("covers", 400, 300), ("small", 480, 428), ("large", 480, 432)])
 def test_every_tile_once(dtype, name, D, Fd):
     from torchllmtuner_amd import ops
 

@@ -947,12 +947,21 @@ BackwardPlan backward_plan(const AnyArgs& p, AnyArgs& w, int dtype, int64_t El, 
   const bool f32 = dtype == MI355_F32;
   // bf16 ones also where the input gradient is large enough for a launch of its own (16000 rows of 8 x 480 x 432, 384 tiles: 183 / 162;
   // a step of 4000 tokens of 4 x 480 x 428, four each, 192 tiles: 264 / 277).
+  // ... but with 64 x 64 tiles input and weight gradients share a launch and the selection's backward runs beside dH, which is worth more where 128 x 128
+  // ones cover a quarter more than those, and where all of it is small.  A step of bf16, us, large tiles / one launch of small ones, by R D F in 10^9 and what large tiles cover over
+  // small ones: 4096 tokens of 8 x 400 x 300, four each (2.0, 1.37) 172.7 / 158.2; 8192 of it, three each (2.9) 239.8 / 223.3; 3000 of 32 x 400 x 300 (1.4) 148.9 / 141.8; 4096 of
+  // 16 x 440 x 400 (2.9, 1.31) 214.6 / 199.9; of 32 x 320 x 300, three each (1.2, 1.44) 138.0 / 126.8; 2500 of 16 x 480 x 400 (1.9, 1.14) 154.5 / 145.2; 4096 of 32 x it, two each
+  // (1.6) 157.9 / 154.4; 3000 of 16 x 480 x 360 (2.1, 1.0) 153.5 / 152.0; 4096 of 32 x 472 x 364 (2.8, 1.0) 197.4 / 208.4; of 32 x 480 x 432 (3.4, 1.14) 223.3 / 227.4; 8192 of 16 x
+  // it (6.8) 346 / 363; 16000 of 16 x 320 x 232 (4.8, 1.2) 339 / 338.
+  auto covered = [&](int64_t t) { return (w.dw[0].M + t - 1) / t * t * ((w.dw[0].N + t - 1) / t * t); };
+  const bool together = !f32 && drows && count &&
+                        (4 * covered(128) >= 5 * covered(64) || R * w.dw[0].M * w.dw[0].N <= int64_t{2400} << 20);
   const bool alone = !f32 && drows && row_tile(p, dtype, El, D, 512) == 128;
-  const bool dw_large = count && dw_tiles(w, El, 128) >= (f32 ? 448 : alone ? 300 : 512) && !(f32 && R < 400 * El);
+  const bool dw_large = !together && count && dw_tiles(w, El, 128) >= (f32 ? 448 : alone ? 300 : 512) && !(f32 && R < 400 * El);
   const int64_t tiles = dw_tiles(w, El, dw_large ? 128 : 64);
   const bool dw_small = f32 && tiles < 160;
   if (dw_small) dw_tiles(w, El, 32);
-  const int t = row_tile(p, dtype, El, D, count && !dw_large ? 512 : 150);
+  const int t = together ? 64 : row_tile(p, dtype, El, D, count && !dw_large ? 512 : 150);
   return {dw_large, dw_small, drows && count && !dw_large && t < 128, t};
 }
 
