@@ -105,3 +105,11 @@ def test_slices_in_order_and_plan_at_the_widths_of_its_launches(T, E, K, lo, hi,
                        ("token_of_row", tor, plan.token_of_row), ("row_scale", scale, ops.combine_row_scale(w, plan)),
                        ("num_tiles", nt, plan.num_tiles), ("tile_expert", te[:n], plan.tile_expert[:n])):
         assert torch.equal(a, b), name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,E,lengths", [(1024, 64, (2, 999, 1024, 1500, 3072)), (128, 64, (33, 1023, 1025, 24576)), (2048, 64, (700, 1023, 1536))])
+def test_a_chunk_has_its_logits_up_to_the_line_of_the_wide_kernel(D, E, lengths):
+    """1024 tokens and more of few experts: the same slices as below."""
+    assert max(lengths) * E * D <= 192 << 20
+    test_a_chunk_of_the_tokens_has_their_logits(torch.bfloat16, D, E, lengths)

@@ -56,7 +56,7 @@ __global__ __launch_bounds__(256) void split_kernel(const float* __restrict__ w,
 // share, so that each lane reads whole 32- or 64-byte pieces of a row.
 // This replaces a kernel that walked the whole contraction in 128-expert tiles behind a separate
 // weight-splitting launch: 1 token of 2048 x 128 experts 34 -> 8 us, 1000 tokens 43 -> 12 us, 128
-// tokens of 7168 x 256 experts 131 -> 12 us (profiled inside the block, the weights from memory).  From 1024 tokens on, with widths on its grid, the
+// tokens of 7168 x 256 experts 131 -> 12 us (profiled inside the block, the weights from memory).  From 1024 tokens and 192 Mi products on, with widths on its grid, the
 // 128-token kernel below reads the weights four times less often and is the faster one.
 template <typename TX, int BN>
 __global__ __launch_bounds__(64 * R_WAVES) void gate_rows_kernel(const TX* __restrict__ x,
@@ -729,8 +729,12 @@ int64_t router_x3_bwd_workspace(int64_t T, int64_t D, int64_t E) {
 
 // Which forward kernel serves a gate: the 128-token one (widths on its grid and tokens enough), the
 // 32-token one (fp32 weights, rows of whole 16-byte pieces), or neither (fp64, odd widths).
+// The wide one waits for the launch that splits the weights.  Below 192 Mi products that launch is more than the other's repeated reads of the weights cost, also
+// with the split in the backward instead.  us, wide / 32 tokens: forward of 3000 tokens, 64 experts of 512 x 512 64.1 / 60.0, 2000 of 1024 x 512 84.0 / 82.0, 3000 110.3 / 108.9, 6000
+// 168.8 / 172.5, 2000 of 128 of it 134.9 / 132.8, 1500 of 128 of 2048 x 768 274.5 / 276.6; a training step with router statistics of 1024, 1500, 2000, 3000, 4000 and 6000 tokens, 64 of
+// 1024 x 512, 225.8 / 223.4, 290.6 / 282.5, 304.4 / 298.9, 351.4 / 348.5, 454.9 / 456.8, 547.5 / 549.2.
 static bool gate_wide(int x_dtype, int w_dtype, int64_t T, int64_t D, int64_t E) {
-  return T >= 1024 && router_x3_ok(x_dtype, w_dtype, D, E);
+  return T >= 1024 && T * E * D > (int64_t{192} << 20) && router_x3_ok(x_dtype, w_dtype, D, E);
 }
 int router_fwd_splits(int x_dtype, int w_dtype, int64_t T, int64_t D, int64_t E) {
   if (T < 1 || D < 1 || E < 1) return 0;
