@@ -94,6 +94,11 @@ int64_t mi355_router_gate_fwd_pieces_bytes(int x_dtype, int w_dtype, int64_t T, 
 int mi355_router_gate_fwd_partial(const void* x, int x_dtype, const float* w, const float* logit_bias,
                                   float* partial, void* pieces, int64_t T, int64_t D, int64_t E,
                                   void* stream);
+/* The same for a caller that runs the backward: pieces (mi355_router_gate_fwd_kept_bytes, 16-byte
+ * aligned; NULL if that is 0) hold the weight pieces afterwards, also where the product itself needs no such scratch. */
+int64_t mi355_router_gate_fwd_kept_bytes(int x_dtype, int w_dtype, int64_t T, int64_t D, int64_t E);
+int mi355_router_gate_fwd_keeping(const void* x, int x_dtype, const float* w, const float* logit_bias, float* partial,
+                                  void* pieces, int64_t T, int64_t D, int64_t E, void* stream);
 
 /*
  * dx[t][d] = sum_e dlogits[t][e] * w[e][d]   (written in x_dtype; NULL = skip)

@@ -82,3 +82,34 @@ def test_gate_backward_between_the_tiles(T, D, E, dtype, addend):
         finite = want.isfinite()
         assert torch.equal(got.isfinite(), finite)
         assert bool(((got.double() - want).abs() <= limit)[finite].all())
+
+
+@pytest.mark.parametrize("T,D,E", [(1, 128, 64), (33, 1024, 64), (700, 1088, 64), (1024, 512, 128), (2048, 1024, 64), (300, 192, 192), (513, 2048, 64)])
+def test_pieces_that_a_forward_keeps_are_the_backwards_own(T, D, E):
+    """mi355_router_gate_fwd_keeping leaves the weight pieces that the backward would form itself: the same gradients, bit for bit, and the same logits."""
+    from torchllmtuner_amd import _lib
+
+    print(f"kept pieces T={T} D={D} E={E}", flush=True)
+    lib, bf16, f32 = _lib.load(), 1, 0
+    g = torch.Generator(device="cuda").manual_seed(T)
+    x = torch.randn(T, D, generator=g, device="cuda").bfloat16()
+    w, dlogits = torch.randn(E, D, generator=g, device="cuda") * 0.02, torch.randn(T, E, generator=g, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    splits, kept = lib.mi355_router_gate_fwd_splits(bf16, f32, T, D, E), lib.mi355_router_gate_fwd_kept_bytes(bf16, f32, T, D, E)
+    assert kept == 4 * E * D and lib.mi355_router_gate_fwd_pieces_bytes(bf16, f32, T, D, E) == 0
+    pieces = torch.full((kept + 64,), 0xAB, dtype=torch.uint8, device="cuda")
+    logits = [torch.empty(splits, T, E, device="cuda") for _ in range(2)]
+    _lib.check(lib.mi355_router_gate_fwd_partial(x.data_ptr(), bf16, w.data_ptr(), None, logits[0].data_ptr(), None, T, D, E, stream), "partial")
+    _lib.check(lib.mi355_router_gate_fwd_keeping(x.data_ptr(), bf16, w.data_ptr(), None, logits[1].data_ptr(), pieces.data_ptr(), T, D, E, stream), "keeping")
+    assert torch.equal(*logits) and bool((pieces[kept:] == 0xAB).all())
+    hi = w.bfloat16()
+    want = torch.stack([hi, (w - hi.float()).bfloat16()])
+    assert torch.equal(pieces[:kept].view(torch.bfloat16).view(2, E, D), want)
+    work = torch.empty(lib.mi355_router_gate_bwd_workspace_bytes(T, D, E), dtype=torch.uint8, device="cuda")
+    got = []
+    for p in (None, pieces.data_ptr()):
+        dx, dw = torch.empty_like(x), torch.empty_like(w)
+        _lib.check(lib.mi355_router_gate_add_bwd(dlogits.data_ptr(), x.data_ptr(), bf16, w.data_ptr(), f32, p, None, dx.data_ptr(), dw.data_ptr(),
+                                                 work.data_ptr(), T, D, E, stream), "bwd")
+        got.append((dx, dw))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])

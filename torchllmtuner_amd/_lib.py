@@ -69,6 +69,8 @@ SIGNATURES = {
     "mi355_router_gate_fwd_splits": (I, [I, I, L, L, L]),
     "mi355_router_gate_fwd_pieces_bytes": (L, [I, I, L, L, L]),
     "mi355_router_gate_fwd_partial": (I, [P, I, P, P, P, P, L, L, L, P]),
+    "mi355_router_gate_fwd_kept_bytes": (L, [I, I, L, L, L]),
+    "mi355_router_gate_fwd_keeping": (I, [P, I, P, P, P, P, L, L, L, P]),
     "mi355_router_gate_add_bwd": (I, [P, P, I, P, I, P, P, P, P, P, L, L, L, P]),
     "mi355_router_select_dots_bwd": (I, [P, P, P, L, P, L, P, P, P, P, L, L, L, I, I, F, P]),
     "mi355_router_select_rows_bwd": (I, [P, P, P, P, I, P, L, L, P, P, P, P, L, L, L, I, I, F, P]),

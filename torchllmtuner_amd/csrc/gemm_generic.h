@@ -79,7 +79,8 @@ int router_rows_bwd(const float* dlogits, int x_dtype, const float* w, const voi
 // of that file serves the case.  `pieces` is scratch of router_fwd_pieces_bytes.
 int router_fwd_splits(int x_dtype, int w_dtype, int64_t T, int64_t D, int64_t E);
 int64_t router_fwd_pieces_bytes(int x_dtype, int w_dtype, int64_t T, int64_t D, int64_t E);
-int router_fwd_partial(const void* x, int x_dtype, const float* w, const float* bias, float* partial, void* pieces,
+int64_t router_fwd_kept_bytes(int x_dtype, int w_dtype, int64_t T, int64_t D, int64_t E);
+int router_fwd_partial(const void* x, int x_dtype, const float* w, const float* bias, float* partial, void* pieces, void* keep,
                        int64_t T, int64_t D, int64_t E, hipStream_t s);
 int router_logits_reduce(const float* partial, const float* bias, float* logits, int64_t T, int64_t E, int splits,
                          hipStream_t s);

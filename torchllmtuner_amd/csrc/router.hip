@@ -312,7 +312,7 @@ extern "C" int mi355_router_gate_fwd(const void* x, int x_dtype, const void* w, 
   const int64_t pieces = splits ? router_fwd_pieces_bytes(x_dtype, w_dtype, T, D, E) : 0;
   if (splits > 0 && (workspace || (splits == 1 && pieces == 0))) {
     float* partial = splits > 1 ? reinterpret_cast<float*>(static_cast<char*>(workspace) + pieces) : logits;
-    if (int rc = router_fwd_partial(x, x_dtype, static_cast<const float*>(w), logit_bias, partial, workspace, T, D, E,
+    if (int rc = router_fwd_partial(x, x_dtype, static_cast<const float*>(w), logit_bias, partial, workspace, nullptr, T, D, E,
                                     as_stream(stream)))
       return rc;
     return splits > 1 ? router_logits_reduce(partial, logit_bias, logits, T, E, splits, as_stream(stream)) : MI355_OK;
@@ -450,9 +450,12 @@ extern "C" int64_t mi355_router_gate_fwd_pieces_bytes(int x_dtype, int w_dtype, 
   return T >= 1 && D >= 1 && E >= 1 ? router_fwd_pieces_bytes(x_dtype, w_dtype, T, D, E) : 0;
 }
 
-extern "C" int mi355_router_gate_fwd_partial(const void* x, int x_dtype, const float* w, const float* logit_bias,
-                                             float* partial, void* pieces, int64_t T, int64_t D, int64_t E,
-                                             void* stream) {
+extern "C" int64_t mi355_router_gate_fwd_kept_bytes(int x_dtype, int w_dtype, int64_t T, int64_t D, int64_t E) {
+  return T >= 1 && D >= 1 && E >= 1 ? router_fwd_kept_bytes(x_dtype, w_dtype, T, D, E) : 0;
+}
+
+static int gate_fwd_partial(const void* x, int x_dtype, const float* w, const float* logit_bias, float* partial, void* pieces, void* keep,
+                            int64_t T, int64_t D, int64_t E, void* stream) {
   MI355_REQUIRE(T >= 1 && D >= 1 && E >= 1 && T < (1ll << 31) && D < (1ll << 31), "router_gate_fwd_partial: bad shape");
   if (router_fwd_splits(x_dtype, MI355_F32, T, D, E) < 1)
     return fail(MI355_EUNSUP, "router_gate_fwd_partial: dtype / width not covered; use mi355_router_gate_fwd");
@@ -460,7 +463,19 @@ extern "C" int mi355_router_gate_fwd_partial(const void* x, int x_dtype, const f
                 "router_gate_fwd_partial: null or misaligned pointer");
   MI355_REQUIRE(pieces || router_fwd_pieces_bytes(x_dtype, MI355_F32, T, D, E) == 0,
                 "router_gate_fwd_partial: scratch for the weight pieces required");
-  return router_fwd_partial(x, x_dtype, w, logit_bias, partial, pieces, T, D, E, as_stream(stream));
+  return router_fwd_partial(x, x_dtype, w, logit_bias, partial, pieces, keep, T, D, E, as_stream(stream));
+}
+extern "C" int mi355_router_gate_fwd_partial(const void* x, int x_dtype, const float* w, const float* logit_bias,
+                                             float* partial, void* pieces, int64_t T, int64_t D, int64_t E,
+                                             void* stream) {
+  return gate_fwd_partial(x, x_dtype, w, logit_bias, partial, pieces, nullptr, T, D, E, stream);
+}
+extern "C" int mi355_router_gate_fwd_keeping(const void* x, int x_dtype, const float* w, const float* logit_bias, float* partial,
+                                             void* pieces, int64_t T, int64_t D, int64_t E, void* stream) {
+  MI355_REQUIRE(aligned16(pieces) && (pieces || mi355_router_gate_fwd_kept_bytes(x_dtype, MI355_F32, T, D, E) == 0),
+                "router_gate_fwd_keeping: aligned room for the weight pieces required");
+  void* keep = mi355_router_gate_fwd_kept_bytes(x_dtype, MI355_F32, T, D, E) > 0 ? pieces : nullptr;
+  return gate_fwd_partial(x, x_dtype, w, logit_bias, partial, pieces, keep, T, D, E, stream);
 }
 
 #define DISPATCH_VPL(E, ...)                           \

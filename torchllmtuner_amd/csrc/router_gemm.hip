@@ -63,11 +63,11 @@ __global__ __launch_bounds__(64 * R_WAVES) void gate_rows_kernel(const TX* __res
                                                                  const float* __restrict__ w,
                                                                  const float* __restrict__ bias,
                                                                  float* __restrict__ out, int T, int D, int E,
-                                                                 int k_per_wave) {
+                                                                 int k_per_wave, uint16_t* __restrict__ keep) {
   __shared__ __attribute__((aligned(16))) float red[R_WAVES][4][64][4];
   const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, q = tid >> 6;
   const int t0 = blockIdx.x * R_BM, n0 = blockIdx.y * BN;
-  f32x4 v = gate_rows_tile<TX, BN>(x, w, T, D, E, t0, n0, blockIdx.z, k_per_wave, red);
+  f32x4 v = gate_rows_tile<TX, BN>(x, w, T, D, E, t0, n0, blockIdx.z, k_per_wave, red, blockIdx.x == 0 ? keep : nullptr);
   if (tid >= 8 * BN) return;
   const int t = t0 + (lane & 31), n = n0 + q * 8 + half * 4;
   if (t >= T || n >= E) return;
@@ -748,7 +748,16 @@ int64_t router_fwd_pieces_bytes(int x_dtype, int w_dtype, int64_t T, int64_t D, 
   return gate_wide(x_dtype, w_dtype, T, D, E) ? 3 * E * D * 2 : 0;
 }
 
-int router_fwd_partial(const void* x, int x_dtype, const float* w, const float* bias, float* partial, void* pieces,
+// ... and what a forward leaves for the backward: the 32-token kernel's first workgroups have the first two pieces in registers, and a launch of its own for
+// them in the backward is saved.  A training step with router statistics, us, apart / kept: 64 experts of 1024 x 512, 256 tokens 176.2 / 173.8, 400 187.9 / 185.8, 700 211.0 /
+// 209.1, 1000 227.9 / 222.6, 1500 287.5 / 285.1, 3000 351.9 / 353.5; 300 of 128 of 512 x 384 155.1 / 153.5.  Larger weights and more tokens have their backward beside the experts' weight
+// gradients, where the launch is hidden: 200, 500 and 1000 tokens of 128 of 2048 x 768 678.3 / 679.7, 721.3 / 723.6, 766.2 / 768.3.
+int64_t router_fwd_kept_bytes(int x_dtype, int w_dtype, int64_t T, int64_t D, int64_t E) {
+  if (const int64_t wide = router_fwd_pieces_bytes(x_dtype, w_dtype, T, D, E)) return wide;
+  return router_x3_ok(x_dtype, w_dtype, D, E) && E * D <= (1 << 17) && T * E * D <= (1 << 27) && router_fwd_splits(x_dtype, w_dtype, T, D, E) > 0 ? 2 * E * D * 2 : 0;
+}
+
+int router_fwd_partial(const void* x, int x_dtype, const float* w, const float* bias, float* partial, void* pieces, void* keep,
                        int64_t T, int64_t D, int64_t E, hipStream_t s) {
   const int splits = router_fwd_splits(x_dtype, MI355_F32, T, D, E);
   const float* in_kernel_bias = splits == 1 ? bias : nullptr;
@@ -773,7 +782,7 @@ int router_fwd_partial(const void* x, int x_dtype, const float* w, const float* 
     using TX = std::remove_const_t<std::remove_pointer_t<decltype(xp)>>;
     const dim3 grid((unsigned)t_tiles, (unsigned)((E + BN - 1) / BN), (unsigned)splits);
     hipLaunchKernelGGL((gate_rows_kernel<TX, BN>), grid, dim3(64 * R_WAVES), 0, s, xp, w, in_kernel_bias, partial, (int)T, (int)D,
-                       (int)E, k_per_wave);
+                       (int)E, k_per_wave, static_cast<uint16_t*>(keep));
   };
   auto choose = [&](auto* xp) {
     const int bn = rows_experts(t_tiles, E, splits);

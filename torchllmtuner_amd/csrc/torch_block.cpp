@@ -68,7 +68,7 @@ struct Block {
   int64_t T, D, E, F, El, N, R, Fs, tile_m, tile_cap, shared_cap;
   int dt, gate_dt;
   int splits;           // partial sums of the router's forward (0: the kernel without them)
-  int64_t piece_bytes;  // its weight pieces
+  int64_t piece_bytes, kept_bytes;  // its weight pieces: what it needs, what it leaves for the backward
   bool gather;         // the kernels of any width serve the routed part and read the tokens' rows in place
   bool folded;         // the folded kernels (token gather, combine's backward inside the experts') serve the routed part
   bool shared_folded;  // the bf16 MFMA kernels serve the shared expert
@@ -87,6 +87,7 @@ struct Block {
     shared_cap = Fs > 0 ? (T + tile_m - 1) / tile_m : 0;
     splits = mi355_router_gate_fwd_splits(dt, gate_dt, T, D, E);
     piece_bytes = splits > 0 ? mi355_router_gate_fwd_pieces_bytes(dt, gate_dt, T, D, E) : 0;
+    kept_bytes = splits > 0 ? mi355_router_gate_fwd_kept_bytes(dt, gate_dt, T, D, E) : 0;
     shared_folded = Fs > 0 && mi355_grouped_combine_bwd_slots(dt, D, Fs) > 0;
   }
 };
@@ -159,7 +160,7 @@ struct Kept {
       aux_f = c.take<float>(b.E);
       aux_scale = c.take<float>(1);
     }
-    if (b.piece_bytes > 0) pieces = c.take(b.piece_bytes, 1);
+    if (const int64_t n = save ? b.kept_bytes : b.piece_bytes) pieces = c.take(n, 1);
     if (save || !b.folded) {  // (gate and up are the other kernels' own intermediates)
       gate = c.take(b.R * b.F, item);
       up = c.take(b.R * b.F, item);
@@ -328,8 +329,8 @@ std::tuple<Tensor, Tensor, Tensor> block_forward(const Block& b, const Stats& st
   if (one_launch) {
     // (in front of the selection, below)
   } else if (b.splits > 0) {
-    check(mi355_router_gate_fwd_partial(ptr(b.x), b.dt, fptr(b.gate_w), fptr(gate_b), partial, k.pieces, b.T, b.D, b.E,
-                                        L.stream),
+    check((save ? mi355_router_gate_fwd_keeping : mi355_router_gate_fwd_partial)(ptr(b.x), b.dt, fptr(b.gate_w), fptr(gate_b), partial,
+                                                                                 k.pieces, b.T, b.D, b.E, L.stream),
           "router_gate_fwd");
   } else {
     check(mi355_router_gate_fwd(ptr(b.x), b.dt, ptr(b.gate_w), b.gate_dt, fptr(gate_b), k.logits, gate_work, b.T, b.D,
