@@ -51,8 +51,9 @@ __device__ __forceinline__ void load16_masked(const uint16_t* p, int k, int k_en
 // One slice of the contraction, by the 64 R_WAVES lanes of a workgroup (ends behind a barrier).  Lanes below 8 BN: the sum of
 // token lane & 31 and the experts q * 8 + (lane >> 5) * 4 + 0..3 of the tile, q their wave.  BN below 32: the tile's first BN experts
 // alone, the same sums in the same order (an element of the matrix instruction's result depends on its own row and column).
-// keep: where the first two pieces of the tile's bf16 weights are left, E * D apart, or null (D % 8 == 0).
-template <typename TX, int BN = R_BN>
+// KEEP: the first two pieces of the tile's weights are left at `keep`, E * D apart, unless that is null (bf16 tokens; D % 8 == 0).  (Another kernel: the test in the
+// loop took 0.3 of the 24.1 us of a forward of one token.)
+template <typename TX, int BN = R_BN, bool KEEP = false>
 __device__ __forceinline__ f32x4 gate_rows_tile(const TX* __restrict__ x, const float* __restrict__ w, int T, int D, int E,
                                                 int t0, int n0, int split, int k_per_wave, float (&red)[R_WAVES][4][64][4] /* wave, q, lane, i */,
                                                 uint16_t* keep = nullptr) {
@@ -85,7 +86,7 @@ __device__ __forceinline__ f32x4 gate_rows_tile(const TX* __restrict__ x, const 
         for (int j = 0; j < 2; ++j) {
           u32x4 hi, mid, lo;
           split8(wv[b][2 * j], wv[b][2 * j + 1], hi, mid, lo);
-          if (keep) {
+          if (KEEP && keep) {
             const int k = kb + b * R_STEP + 16 * half + 8 * j, n = n0 + (lane & 31);
             if (k < w_end && n < E) {
               uint16_t* at = keep + static_cast<int64_t>(n) * D + k;

@@ -58,7 +58,7 @@ __global__ __launch_bounds__(256) void split_kernel(const float* __restrict__ w,
 // weight-splitting launch: 1 token of 2048 x 128 experts 34 -> 8 us, 1000 tokens 43 -> 12 us, 128
 // tokens of 7168 x 256 experts 131 -> 12 us (profiled inside the block, the weights from memory).  From 1024 tokens and 192 Mi products on, with widths on its grid, the
 // 128-token kernel below reads the weights four times less often and is the faster one.
-template <typename TX, int BN>
+template <typename TX, int BN, bool KEEP>
 __global__ __launch_bounds__(64 * R_WAVES) void gate_rows_kernel(const TX* __restrict__ x,
                                                                  const float* __restrict__ w,
                                                                  const float* __restrict__ bias,
@@ -67,7 +67,7 @@ __global__ __launch_bounds__(64 * R_WAVES) void gate_rows_kernel(const TX* __res
   __shared__ __attribute__((aligned(16))) float red[R_WAVES][4][64][4];
   const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, q = tid >> 6;
   const int t0 = blockIdx.x * R_BM, n0 = blockIdx.y * BN;
-  f32x4 v = gate_rows_tile<TX, BN>(x, w, T, D, E, t0, n0, blockIdx.z, k_per_wave, red, blockIdx.x == 0 ? keep : nullptr);
+  f32x4 v = gate_rows_tile<TX, BN, KEEP>(x, w, T, D, E, t0, n0, blockIdx.z, k_per_wave, red, blockIdx.x == 0 ? keep : nullptr);
   if (tid >= 8 * BN) return;
   const int t = t0 + (lane & 31), n = n0 + q * 8 + half * 4;
   if (t >= T || n >= E) return;
@@ -781,8 +781,12 @@ int router_fwd_partial(const void* x, int x_dtype, const float* w, const float* 
     constexpr int BN = decltype(bn)::value;
     using TX = std::remove_const_t<std::remove_pointer_t<decltype(xp)>>;
     const dim3 grid((unsigned)t_tiles, (unsigned)((E + BN - 1) / BN), (unsigned)splits);
-    hipLaunchKernelGGL((gate_rows_kernel<TX, BN>), grid, dim3(64 * R_WAVES), 0, s, xp, w, in_kernel_bias, partial, (int)T, (int)D,
-                       (int)E, k_per_wave, static_cast<uint16_t*>(keep));
+    auto run = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, dim3(64 * R_WAVES), 0, s, xp, w, in_kernel_bias, partial, (int)T, (int)D, (int)E, k_per_wave,
+                         static_cast<uint16_t*>(keep));
+    };
+    if constexpr (sizeof(TX) == 2) run(keep ? gate_rows_kernel<TX, BN, true> : gate_rows_kernel<TX, BN, false>);
+    else run(gate_rows_kernel<TX, BN, false>);
   };
   auto choose = [&](auto* xp) {
     const int bn = rows_experts(t_tiles, E, splits);
