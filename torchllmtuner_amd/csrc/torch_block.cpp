@@ -617,7 +617,7 @@ using BlockBwdSig = NineTensors(const Tensor&, const Tensor&, const Tensor&, con
 
 struct MoeBlock : public torch::autograd::Function<MoeBlock> {
   static variable_list forward(AutogradContext* ctx, BLOCK_PARAMS) {
-    at::AutoDispatchBelowADInplaceOrView below;
+    at::AutoDispatchBelowAutograd below;
     static auto op = typed_op<BlockFwdSig>("mi355_moe::moe_block_fwd");
     auto [out, counts, kept] = op.call(BLOCK_ARGS);
     ctx->save_for_backward({x, gate_w, some(gate_b), w1, w3, w2, some(sg), some(su), some(sd), kept, some(mask)});
@@ -789,12 +789,29 @@ NineTensors moe_block_bwd_meta(BLOCK_BWD_PARAMS) {
           like(need.shared, b.sg),     like(need.shared, b.su),     like(need.shared, b.sd)};
 }
 
+// Under the two: the statistics are written through their pointers, so what autograd compares before it uses a saved tensor is raised here, as
+// an operator of torch's own does.
+template <typename Sig>
+auto writing(const char* name, BLOCK_PARAMS) {
+  static auto op = typed_op<Sig>(name);
+  auto r = [&] {
+    at::AutoDispatchBelowADInplaceOrView below;
+    return op.call(BLOCK_ARGS);
+  }();
+  for (const OptTensor* t : {&histogram, &aux_acc, &totals}) wrote(*t);
+  return r;
+}
+std::tuple<Tensor, Tensor> moe_block_writing(BLOCK_PARAMS) { return writing<BlockSig>("mi355_moe::moe_block", BLOCK_ARGS); }
+std::tuple<Tensor, Tensor, Tensor> moe_block_fwd_writing(BLOCK_PARAMS) {
+  return writing<BlockFwdSig>("mi355_moe::moe_block_fwd", BLOCK_ARGS);
+}
+
 std::tuple<Tensor, Tensor> moe_block_autograd(BLOCK_PARAMS) {
   if (torch::autograd::compute_requires_grad(x, gate_w, gate_b, w1, w3, w2, sg, su, sd)) {
     auto r = MoeBlock::apply(BLOCK_ARGS);
     return {r[0], r[1]};
   }
-  at::AutoDispatchBelowADInplaceOrView below;
+  at::AutoDispatchBelowAutograd below;
   static auto op = typed_op<BlockSig>("mi355_moe::moe_block");
   return op.call(BLOCK_ARGS);
 }
@@ -826,6 +843,10 @@ TORCH_LIBRARY_IMPL(mi355_moe, CUDA, m) {
 TORCH_LIBRARY_IMPL(mi355_moe, Meta, m) {
   m.impl("moe_block_fwd", moe_block_fwd_meta);
   m.impl("moe_block_bwd", moe_block_bwd_meta);
+}
+TORCH_LIBRARY_IMPL(mi355_moe, ADInplaceOrView, m) {
+  m.impl("moe_block", moe_block_writing);
+  m.impl("moe_block_fwd", moe_block_fwd_writing);
 }
 TORCH_LIBRARY_IMPL(mi355_moe, Autograd, m) {
   m.impl("moe_block", moe_block_autograd);

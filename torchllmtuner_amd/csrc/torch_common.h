@@ -74,6 +74,12 @@ auto typed_op(const char* name) {
   return c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<Sig>();
 }
 
+// An operator has written an argument through its pointer: a backward that saved its earlier value is to raise.  (An inference tensor has no
+// version, and no backward saves one.)
+inline void wrote(const OptTensor& t) {
+  if (t.has_value() && t->defined() && !t->is_inference()) t->unsafeGetTensorImpl()->bump_version();
+}
+
 // Rows that El of E experts will have of N slots, as far as the host can tell: what chooses the kernels of the forward.  A share's experts
 // have them less evenly than all experts together, the more so where tokens choose among groups of experts (128 tokens of eight, 32 of 256
 // experts: 22 have rows, one has 15, four on average), so its part is counted two and a half times.

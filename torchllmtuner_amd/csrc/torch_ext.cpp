@@ -135,6 +135,15 @@ void quantile_observe(Tensor histogram, const Tensor& scores_, const Tensor& cut
         "quantile_observe");
 }
 
+void quantile_observe_writing(Tensor histogram, const Tensor& scores, const Tensor& cutoff, const Tensor& bias, const OptTensor& pad) {
+  static auto op = typed_op<void(Tensor, const Tensor&, const Tensor&, const Tensor&, const OptTensor&)>("mi355_moe::quantile_observe");
+  {
+    at::AutoDispatchBelowADInplaceOrView below;
+    op.call(histogram, scores, cutoff, bias, pad);
+  }
+  wrote(histogram);
+}
+
 Tensor quantile_estimate(const Tensor& histogram_, const Tensor& bias_, int64_t K) {
   Launch L(histogram_);
   TORCH_CHECK_TYPE(histogram_.scalar_type() == at::kLong, "histogram_EB must be int64");
@@ -661,6 +670,7 @@ TORCH_LIBRARY(mi355_moe, m) {
       "bool need_dw) -> (Tensor, Tensor, Tensor, Tensor, Tensor)");
 }
 
+TORCH_LIBRARY_IMPL(mi355_moe, ADInplaceOrView, m) { m.impl("quantile_observe", quantile_observe_writing); }
 TORCH_LIBRARY_IMPL(mi355_moe, CUDA, m) {
   m.impl("router_gate_fwd", router_gate_fwd);
   m.impl("router_gate_bwd", router_gate_bwd);
