@@ -523,8 +523,8 @@ int mi355_grouped_swiglu_fwd_beside(const void* rows, const int32_t* token_of_ro
                                     int64_t tile_capacity, void* gate, void* up, void* h,
                                     void* y, int64_t El, int64_t D, int64_t F,
                                     int64_t row_capacity, void* stream);
-/* The same results for a caller that knows how many of the row_capacity rows to expect (padded segments, one rank's share of the
- * experts): that number, and not the capacity, chooses the kernels.  Any number up to the capacity is right. */
+/* The same results for a caller that knows how many of the row_capacity rows there can be (padded segments): that number, and not the
+ * capacity, chooses the kernels.  Any number up to the capacity is right; one that is far below the rows that come makes them slow. */
 int mi355_grouped_swiglu_fwd_expecting(const void* rows, const int32_t* token_of_row, int64_t num_tokens,
                                        const void* w1, const void* w3, const void* w2, int dtype,
                                        const int32_t* seg_offsets,
@@ -533,6 +533,15 @@ int mi355_grouped_swiglu_fwd_expecting(const void* rows, const int32_t* token_of
                                        int64_t tile_capacity, void* gate, void* up, void* h,
                                        void* y, int64_t El, int64_t D, int64_t F,
                                        int64_t row_capacity, int64_t rows_expected, void* stream);
+/* Which kernels that forward takes, for tests and measurements: rows of a pass (16, 64, 128; 256: row tiles), with the bits below; 0 where none of
+ * these serve the shape.  num_tokens: 0 for rows read in place. */
+enum {
+  MI355_FWD_PASS = 0x1ff,
+  MI355_FWD_NARROW_GATEUP = 0x200, MI355_FWD_NARROW_DOWN = 0x400,  /* row tiles of half the columns */
+  MI355_FWD_TURNED_GATEUP = 0x800, MI355_FWD_TURNED_DOWN = 0x1000  /* each tile's sums start at a step of its own */
+};
+int mi355_grouped_fwd_kernels(int dtype, int64_t El, int64_t D, int64_t F, int64_t row_capacity, int64_t rows_expected,
+                              int64_t num_tokens, int64_t tile_capacity);
 
 /*
  * Backward of the above (autograd-derived in the reference):

@@ -190,3 +190,24 @@ def test_bench_refuses_more_than_one_gpu():
     r = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2"], capture_output=True, text=True)
     assert r.returncode != 0
     assert "one GPU" in (r.stdout + r.stderr) and "{" not in r.stdout
+
+
+def test_kernels_of_the_forward_follow_the_rows_that_may_come():
+    """One rank's share of the experts may draw every token's rows: neither 16 rows a pass, which read the weights again for each, nor 64 or 128 for
+    experts that may have many of those are chosen by the rows that such a rank has on average."""
+    from torchllmtuner_amd import _lib
+
+    lib = _lib.load()
+
+    def rows_of_a_pass(T, K, El, D, F, align=1):
+        N = T * K
+        return lib.mi355_grouped_fwd_kernels(1, El, D, F, N + (El * (align - 1) if align > 1 else 0), N, T, N // 256 + El + 1) & 0x1FF
+
+    share = dict(K=8, El=32, D=7168, F=2048)
+    want = {4: 16, 32: 16, 33: 64, 64: 64, 65: 128, 100: 128, 128: 128, 129: 256, 400: 256, 4096: 256}
+    assert {T: rows_of_a_pass(T, **share) for T in want} == want
+    block = dict(K=8, El=128, D=2048, F=768)
+    want = {1: 16, 128: 16, 129: 64, 300: 64, 319: 256, 1000: 256, 8192: 256}
+    assert {T: rows_of_a_pass(T, **block) for T in want} == want
+    assert rows_of_a_pass(8, **block, align=128) == 16  # (padding is no rows)
+    assert lib.mi355_grouped_fwd_kernels(0, 8, 512, 512, 64, 64, 64, 9) == 0 == lib.mi355_grouped_fwd_kernels(1, 8, 360, 512, 64, 64, 64, 9)

@@ -22,6 +22,7 @@ int bf16_grouped_fwd(const void* rows, const int32_t* token_of_row, int64_t num_
                      const int32_t* tile_expert, const int32_t* tile_row0, const int32_t* num_tiles,
                      int64_t tile_capacity, void* gate, void* up, void* h, void* y, int64_t El, int64_t D,
                      int64_t F, int64_t row_capacity, int64_t rows_expected, int stages, hipStream_t s);
+int bf16_fwd_kernels(int64_t El, int64_t D, int64_t F, int64_t row_capacity, int64_t rows_expected, int64_t tokens, int64_t tile_capacity);
 int bf16_fused_dot_slots(int64_t F);
 int bf16_grouped_linear_dx(const void* dy, const void* w, const int32_t* seg_offsets, const int32_t* seg_counts,
                            const int32_t* tile_expert, const int32_t* tile_row0, const int32_t* num_tiles,
@@ -251,6 +252,13 @@ extern "C" int mi355_grouped_swiglu_fwd_expecting(const void* rows, const int32_
                 (long long)rows_expected, (long long)row_capacity);
   return swiglu_fwd(rows, token_of_row, num_tokens, w1, w3, w2, dtype, seg_offsets, seg_counts, tile_expert, tile_row0,
                     num_tiles, tile_capacity, gate, up, h, y, El, D, F, row_capacity, rows_expected, 3, stream);
+}
+
+extern "C" int mi355_grouped_fwd_kernels(int dtype, int64_t El, int64_t D, int64_t F, int64_t row_capacity, int64_t rows_expected,
+                                         int64_t num_tokens, int64_t tile_capacity) {
+  return dtype == MI355_BF16 && El >= 1 && bf16_fast_path_ok(D, F)
+             ? bf16_fwd_kernels(El, D, F, row_capacity, rows_expected, num_tokens, tile_capacity)
+             : 0;
 }
 
 extern "C" int mi355_grouped_swiglu_bwd(const void* dy, const void* rows,

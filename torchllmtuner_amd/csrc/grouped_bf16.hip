@@ -1170,18 +1170,29 @@ int short_rows_fwd(int stage, bool tall, const void* a, const int32_t* a_src, in
                    void* gate, void* up, void* out, const int32_t* seg_offsets, const int32_t* seg_counts, int64_t El, int64_t K,
                    int64_t N, int64_t row_capacity, bool stream, bool turn, hipStream_t s);
 
-// Up to eight rows per expert (`rows` of all: what the host expects), or 64 rows in all.
+// Up to eight rows per expert, or 64 rows in all (`rows`: as many as there may be; one rank's share of the experts may draw every token's).
 // A 16-row pass over an expert's weights costs the same for one row as for sixteen and a second pass
 // reads them again, from L2 at best.  Block forward of 128 experts of 2048 x 768, these kernels / the row tiles, us: 16 tokens (1 row on average) 133 / 147, 33 183 /
 // 200, 64 202 / 210, 100 (6) 205 / 216, 128 (8) 216 / 215; 32 of 256 experts of 7168 x 2048, 16 tokens 186 / 230, 32 245 / 254.  One dense
 // segment of 7168 x 2048 alone, gate/up and down, 60 rows 41 + 16 / 79 + 26, 128 rows 79 + 25 / 93 + 30; but beside the routed experts of that share, whose CUs it takes
 // then, 128 rows 422 / 401.  Beyond, 64-row passes (grouped_short.hip).
+//   Not by what a share's rows are on average: 16 rows a pass read the weights again for each of many (its products, us, these / 64-row passes / row tiles: 100 tokens of eight,
+// drawn evenly from the 256 experts 372 / 386 / 408, all from these 32 870 / 430 / 442, from 16 of them 812 / 230 / 228; 40 tokens 229 / 260 / 315, 422 / 413 / 427, 413 / 214 / 217).
 static bool few_rows(int64_t El, int64_t rows, int64_t R, int64_t D, int64_t F) {
   return rows <= std::max<int64_t>(8 * El, 64) && R * std::max(D, F) * 2 < (int64_t{1} << 32);
 }
 
 // Rows of a pass of grouped_short.hip, 0 for the row tiles (block forward, us, row tiles / 64 / 128 rows a pass).
-//   Up to 45 rows an expert, where hardly one needs a second pass, 64: the figures there.
+//   Up to 45 rows an expert 64, as long as a token is one row of an expert and there are no more than 64 (every pass is the only reader of its weights), or the products are
+// small; 128 for up to 128 tokens.  Beyond, the host does not know the load, and where a few experts have all rows, or a share all tokens, the passes are
+// short of matrix-core time.  The products alone, weights from memory, us, 64 / 128 / row tiles, of loads drawn evenly, by Zipf's law, from a quarter of the experts (a share: from the rank's
+// own 32), from 16, from eight: 32 of 256 of 7168 x 2048, 64 tokens 384 / 390 / 405, 261 / 271 / 315, 420 / 420 / 433, 218 / 222 / 219, 117 / 120 / 156; 100 tokens 386 / 391 / 408,
+// 306 / 312 / 355, 430 / 433 / 442, 230 / 235 / 228, 177 / 139 / 163; 128 tokens 408 / 409 / 424, 326 / 327 / 362, 442 / 446 / 449, 301 / 249 / 235, 189 / 148 / 168; 256 tokens 412 / 412 /
+// 427, 394 / 432 / 422, 607 / 497 / 475, 425 / 418 / 253, 292 / 250 / 210.  128 of 2048 x 768, 300 tokens (2400 rows, 3.8 * 10^9 of rows D F) 192 / 194 / 198, 196 / 206 / 230, 79 / 68 / 68, 63 / 60 / 62,
+// 43 / 52 / 54; 400 tokens 198 / 200 / 204, 206 / 209 / 211, 81 / 76 / 71, 70 / 67 / 68, 56 / 56 / 63; 600 tokens 211 / 215 / 215, 230 / 225 / 250, 108 / 113 / 78, 90 / 97 / 66, 79 / 72 / 67.
+//   The share's whole forward, us, row tiles from 33 tokens on / these, evenly, from its 32, from 16, from eight: 40 tokens 396 / 386, 462 / 446, 252 / 246, 188 / 144; 64 tokens 390 / 339, 472 /
+// 456, 258 / 256, 194 / 153; 128 tokens 458 / 443, 489 / 481, 270 / 280, 205 / 181 (16 rows a pass up to 102 tokens, then 64: 40 tokens 351, 454, 448, 354; 100 tokens 429, 905, 818, 793; 400 tokens, where these
+// and the row tiles are the same 483, 552, 341, 309: 467, 716, 573, 502).
 //   As many where all passes are at most two workgroups a CU, and 256-row tiles would leave most CUs without one: 16 experts of 512 x 384, four each, 90 to 300
 // rows an expert 35-41 / 31-36 / 35-39; 16 of 1024 x 512, 90 to 220 rows 44-50 / 39-44 / 45-48, 300 51 / 53 / 54, 400 56 / 64 / 56; 32 of it, 90 rows 55 / 53 /
 // 52, 130 58 / 64 / 67; one dense segment of 7168 x 2048, 129 rows 132 / 78 / 118, 512 177 / 83 / 119, 1000 179 / 115 / 126, 1400 182 / 164 / 164, 2000
@@ -1191,11 +1202,14 @@ static bool few_rows(int64_t El, int64_t rows, int64_t R, int64_t D, int64_t F) 
 // arrive as fast through row tiles then (60 of 1728 x 960, 60 rows 150 / 162 / 151; 128 of 2048 x 768 261 / 300 / 267).
 //   A dense segment beside other products leaves them more CUs in passes of 128 (one rank's share of 7168 x 2048 with a shared expert of 2048, 128 tokens
 // 365 / 347 / 348, 200 390 / 398 / 391, 300 417 / 418 / 404, 512 460 / 484 / 464).
-static int short_rows(int64_t El, int64_t rows, int64_t D, int64_t F, bool beside) {
+static int short_rows(int64_t El, int64_t rows, int64_t tokens, int64_t D, int64_t F, bool beside) {
   if (El > 256 || rows < 1) return 0;  // (what a wave there adds up)
   if (El == 1 && beside) return rows <= 400 ? 128 : 0;
   const double mean = static_cast<double>(rows) / static_cast<double>(El), sd = El == 1 ? 0.0 : std::sqrt(mean);
-  if (El > 1 && mean <= 45.0) return 64;
+  if (El > 1 && mean <= 45.0) {
+    if (tokens <= 64 || rows * D * F <= 4'000'000'000) return 64;
+    if (tokens <= 128) return 128;
+  }
   const int64_t groups = std::max((F + 63) / 64, (D + 127) / 128);
   if (pieces(mean, sd, 64) * static_cast<double>(El * groups) <= 2.0 * resident_blocks()) return 64;
   return El > 1 && mean <= 90.0 && !streamed(El, D, F) ? 128 : 0;
@@ -1209,13 +1223,31 @@ static int short_rows(int64_t El, int64_t rows, int64_t D, int64_t F, bool besid
 // an expert (and 8, grouped_few.hip) a token's bits depend on how many come with it (1000 tokens of that block: 3e-4 of the output, at most a bf16 step).
 static bool turned(int64_t El, int64_t R, int64_t K) { return El > 1 && R <= 200 * El && K * 2 % 4096 == 0; }
 
+// Rows that a pass of the forward's kernels has: 16, 64, 128 or 256.  tokens: 0 where the rows are read in place.
+static int pass_rows(int64_t El, int64_t D, int64_t F, int64_t row_capacity, int64_t rows_expected, int64_t tokens, bool beside) {
+  if (few_rows(El, rows_expected, row_capacity, D, F)) return 16;
+  const int pass = short_rows(El, rows_expected, tokens > 0 ? tokens : rows_expected, D, F, beside);
+  return pass ? pass : 256;
+}
+
+int bf16_fwd_kernels(int64_t El, int64_t D, int64_t F, int64_t row_capacity, int64_t rows_expected, int64_t tokens, int64_t tile_capacity) {
+  const int pass = pass_rows(El, D, F, row_capacity, rows_expected, tokens, false);
+  auto across = [](int64_t width, int64_t tile) { return (width + tile - 1) / tile; };
+  const bool tiles = pass == 256, turn = pass > 16;
+  return pass | (tiles && narrow(RM_GATEUP, El, across(F, 128), across(F, 64), tile_capacity) ? MI355_FWD_NARROW_GATEUP : 0) |
+         (tiles && narrow(RM_DOWN, El, across(D, 256), across(D, 128), tile_capacity) ? MI355_FWD_NARROW_DOWN : 0) |
+         (turn && (tokens > 0 || !tiles) && turned(El, row_capacity, D) ? MI355_FWD_TURNED_GATEUP : 0) |
+         (turn && turned(El, row_capacity, F) ? MI355_FWD_TURNED_DOWN : 0);
+}
+
 int bf16_grouped_fwd(const void* rows, const int32_t* token_of_row, int64_t num_tokens, const void* w1,
                      const void* w3, const void* w2, const int32_t* seg_offsets, const int32_t* seg_counts,
                      const int32_t* tile_expert, const int32_t* tile_row0, const int32_t* num_tiles,
                      int64_t tile_capacity, void* gate, void* up, void* h, void* y, int64_t El, int64_t D,
                      int64_t F, int64_t row_capacity, int64_t rows_expected, int stages, hipStream_t s) {
   const bool stream = streamed(std::min(El, row_capacity), D, F);  // (of the experts that can have rows)
-  if (few_rows(El, rows_expected, row_capacity, D, F)) {
+  const int pass = pass_rows(El, D, F, row_capacity, rows_expected, token_of_row ? num_tokens : 0, stages & STAGE_BESIDE);
+  if (pass == 16) {
     const int64_t tiles = std::min(tile_capacity, std::min(El, row_capacity) + row_capacity / 256);
     if (stages & STAGE_GATEUP)
       if (int rc = few_rows_fwd(1, rows, token_of_row, num_tokens, w1, w3, gate, up, h, seg_offsets, seg_counts,
@@ -1226,7 +1258,7 @@ int bf16_grouped_fwd(const void* rows, const int32_t* token_of_row, int64_t num_
                           num_tiles, tiles, F, D, stream, s);
     return MI355_OK;
   }
-  if (const int pass = short_rows(El, rows_expected, D, F, stages & STAGE_BESIDE)) {
+  if (pass < 256) {
     if (stages & STAGE_GATEUP)
       if (int rc = short_rows_fwd(1, pass > 64, rows, token_of_row, num_tokens, w1, w3, gate, up, h, seg_offsets, seg_counts, El,
                                   D, F, row_capacity, stream, turned(El, row_capacity, D), s))

@@ -9,6 +9,7 @@
 // are a fifth of the launch.  grouped_few.hip, 16 rows a pass, reads the weights again for every 16.
 //   An expert of more rows has as many passes, workgroups of their own that read the same weights side by side, from L2: with the passes one after the other in one
 // workgroup a router that prefers some experts made a training step of 300 tokens of the first block below 10 % longer (805 us for 735; 722 now).
+//   Where they are chosen: grouped_bf16.hip (many rows of few experts want the row tiles, which these loads do not have).
 //   Bound by HBM: block forward of three sets of weights in turn, us, row tiles / 64-row passes / 128-row passes.  128 experts of 2048 x 768, eight a
 // token, 200 tokens 219 / 214 / 212, 500 239 / 232 / 235 (1.2 GB of weights in 190), 700 250 / 245 / 249, 1000 261 / 300 / 267; 64 of 1024 x 512, six each, 300 71 / 65 / 66;
 // 60 of 1728 x 960, six each, 120 130 / 121 / 124, 300 135 / 128 / 131, 450 143 / 137 / 142; 16 of 2048 x 1024, four each, 48 68 / 60 / 60, 180 72 / 64 / 65; 16 of 512 x

@@ -244,7 +244,7 @@ std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor> rows_experts_combine_
 using GecFwdSig = std::tuple<Tensor, Tensor, Tensor>(const Tensor&, const Tensor&, const Tensor&, const Tensor&,
                                                      const Tensor&, const Tensor&, const Tensor&, const Tensor&,
                                                      const Tensor&, const Tensor&, const Tensor&, const Tensor&,
-                                                     const Tensor&, int64_t, int64_t, bool, bool, int64_t);
+                                                     const Tensor&, int64_t, int64_t, bool, bool);
 using GecBwdSig = std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor>(
     const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&,
     const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&,
@@ -255,19 +255,19 @@ struct GatherExpertsCombine : public torch::autograd::Function<GatherExpertsComb
                                const Tensor& w3, const Tensor& w2, const Tensor& tok, const Tensor& sor,
                                const Tensor& ros, const Tensor& so, const Tensor& sc, const Tensor& te,
                                const Tensor& tr, const Tensor& nt, int64_t K, int64_t cap, bool round_terms,
-                               bool save_gate_up, int64_t num_experts) {
+                               bool save_gate_up) {
     TORCH_CHECK(save_gate_up,
                 "gather_experts_combine_fwd was run without its gate / up outputs and cannot be differentiated");
     at::AutoDispatchBelowADInplaceOrView below;
     static auto op = typed_op<GecFwdSig>("mi355_moe::gather_experts_combine_fwd");
-    auto r = op.call(x, weights, w1, w3, w2, tok, sor, ros, so, sc, te, tr, nt, K, cap, round_terms, save_gate_up, num_experts);
+    auto r = op.call(x, weights, w1, w3, w2, tok, sor, ros, so, sc, te, tr, nt, K, cap, round_terms, save_gate_up);
     ctx->save_for_backward({x, weights, w1, w3, w2, std::get<1>(r), std::get<2>(r), tok, sor, ros, so, sc, te, tr, nt});
     ctx->saved_data["top_k"] = K;
     ctx->set_materialize_grads(false);
     return {std::get<0>(r), std::get<1>(r), std::get<2>(r)};
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    variable_list out(18);
+    variable_list out(17);
     if (!grads[0].defined()) return out;
     const auto s = ctx->get_saved_variables();
     const bool n0 = ctx->needs_input_grad(0), n1 = ctx->needs_input_grad(1), n2 = ctx->needs_input_grad(2),
@@ -287,14 +287,14 @@ struct GatherExpertsCombine : public torch::autograd::Function<GatherExpertsComb
 std::tuple<Tensor, Tensor, Tensor> gather_experts_combine_autograd(
     const Tensor& x, const Tensor& weights, const Tensor& w1, const Tensor& w3, const Tensor& w2, const Tensor& tok,
     const Tensor& sor, const Tensor& ros, const Tensor& so, const Tensor& sc, const Tensor& te, const Tensor& tr,
-    const Tensor& nt, int64_t K, int64_t cap, bool round_terms, bool save_gate_up, int64_t num_experts) {
+    const Tensor& nt, int64_t K, int64_t cap, bool round_terms, bool save_gate_up) {
   if (!torch::autograd::compute_requires_grad(x, weights, w1, w3, w2)) {
     at::AutoDispatchBelowADInplaceOrView below;
     static auto op = typed_op<GecFwdSig>("mi355_moe::gather_experts_combine_fwd");
-    return op.call(x, weights, w1, w3, w2, tok, sor, ros, so, sc, te, tr, nt, K, cap, round_terms, save_gate_up, num_experts);
+    return op.call(x, weights, w1, w3, w2, tok, sor, ros, so, sc, te, tr, nt, K, cap, round_terms, save_gate_up);
   }
   auto r = GatherExpertsCombine::apply(x, weights, w1, w3, w2, tok, sor, ros, so, sc, te, tr, nt, K, cap, round_terms,
-                                       save_gate_up, num_experts);
+                                       save_gate_up);
   return {r[0], r[1], r[2]};
 }
 

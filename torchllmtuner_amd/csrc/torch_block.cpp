@@ -373,8 +373,8 @@ std::tuple<Tensor, Tensor, Tensor> block_forward(const Block& b, const Stats& st
   else
     check(mi355_grouped_swiglu_fwd_expecting(b.folded ? ptr(b.x) : k.rows, b.folded ? k.token_of_row : nullptr, b.folded ? b.T : b.R,
                                              ptr(b.w1), ptr(b.w3), ptr(b.w2), b.dt, k.seg_offsets, k.seg_counts, k.tile_expert,
-                                             k.tile_row0, k.num_tiles, b.tile_cap, k.gate, k.up, h, y, b.El, b.D, b.F, b.R,
-                                             rows_expected(b.N, b.El, b.E), L.stream),
+                                             k.tile_row0, k.num_tiles, b.tile_cap, k.gate, k.up, h, y, b.El, b.D, b.F, b.R, b.N,
+                                             L.stream),
           "grouped_swiglu_fwd");
   if (b.Fs > 0 && !aux) shared_forward(b, k, y_shared, L.stream, false);
   shared.join();

@@ -8,7 +8,6 @@
 
 #include <hip/hip_runtime_api.h>
 
-#include <algorithm>
 #include <mutex>
 #include <optional>
 
@@ -79,11 +78,6 @@ auto typed_op(const char* name) {
 inline void wrote(const OptTensor& t) {
   if (t.has_value() && t->defined() && !t->is_inference()) t->unsafeGetTensorImpl()->bump_version();
 }
-
-// Rows that El of E experts will have of N slots, as far as the host can tell: what chooses the kernels of the forward.  A share's experts
-// have them less evenly than all experts together, the more so where tokens choose among groups of experts (128 tokens of eight, 32 of 256
-// experts: 22 have rows, one has 15, four on average), so its part is counted two and a half times.
-inline int64_t rows_expected(int64_t N, int64_t El, int64_t E) { return El == E ? N : std::min(N, 5 * N * El / (2 * E)); }
 
 inline int dtype_code(const Tensor& t) {
   if (t.scalar_type() == at::kFloat) return MI355_F32;

@@ -276,7 +276,7 @@ def _(dout, rows, weights, w1, w3, w2, gate, up, h, y, row_of_slot, slot_of_row,
 
 @_fake("gather_experts_combine_fwd")
 def _(x, weights, w1, w3, w2, token_of_row, slot_of_row, row_of_slot, seg_offsets, seg_counts, tile_expert,
-      tile_row0, num_tiles, top_k, row_capacity, round_terms, save_gate_up, num_experts=0):
+      tile_row0, num_tiles, top_k, row_capacity, round_terms, save_gate_up):
     F = w1.shape[1]
     rows = row_capacity if save_gate_up else 0
     return torch.empty_like(x), x.new_empty((rows, F)), x.new_empty((rows, F))
@@ -639,7 +639,7 @@ def gather_experts_combine(x_TD, weights_TK, w1_EFD, w3_EFD, w2_EDF, plan: Permu
         t.requires_grad for t in (x_TD, weights_TK, w1_EFD, w3_EFD, w2_EDF))
     out, _gate, _up = _O.gather_experts_combine_fwd(
         x_TD, weights_TK, w1_EFD, w3_EFD, w2_EDF, plan.token_of_row, plan.slot_of_row, plan.row_of_slot,
-        *plan.segments(), plan.top_k, plan.row_capacity, bool(round_terms), differentiable, plan.num_experts)
+        *plan.segments(), plan.top_k, plan.row_capacity, bool(round_terms), differentiable)
     return out
 
 
