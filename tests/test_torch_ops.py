@@ -285,3 +285,26 @@ def test_exit_hook_is_idle_without_a_gpu():
         t0 = time.perf_counter()
         ops._let_autograd_threads_finish()
         assert time.perf_counter() - t0 < 0.02
+
+
+def test_a_router_that_only_routes_serves_a_training_block():
+    """A module in the router's place needs to route and nothing else, in training as in evaluation (plain torch modules, on the CPU)."""
+
+    class Router(torch.nn.Module):
+        def forward(self, x, bias, *, padding_mask_T=None):
+            ids = torch.arange(x.shape[0] * K).remainder(E).view(-1, K)
+            return torch.full(ids.shape, 0.5), ids, torch.nn.functional.one_hot(ids, E).sum(1).bool()
+
+    class Routed(torch.nn.Module):
+        token_dispatcher = None
+
+        def forward(self, x, scores, ids, counts):
+            return x * scores.sum(1, keepdim=True)
+
+    block = moe.MoE(E, moe.RoutedExperts(moe.GroupedExperts(D, F, E), moe.LocalTokenDispatcher(E, K)),
+                    moe.TokenChoiceTopKRouter(E, D, K, score_func="softmax", route_norm=True), load_balance_coeff=None)
+    block.router, block.routed_experts = Router(), Routed()
+    x = torch.randn(T, D)
+    for steps, training in ((1, True), (1, False), (2, True)):
+        assert torch.equal(block.train(training)(x), x)
+        assert torch.equal(block.tokens_per_expert_E, torch.full((E,), steps * float(N // E)))

@@ -247,7 +247,8 @@ class MoE(nn.Module):
             or totals.device != tokens.device
             or totals.requires_grad
             or not totals.is_contiguous()
-            or totals.numel() != self.router.num_experts
+            # (a router that does not say how many experts it has is none that the operator serves)
+            or totals.numel() != getattr(self.router, "num_experts", None)
         ):
             return None
         return totals
