@@ -308,3 +308,13 @@ def test_a_router_that_only_routes_serves_a_training_block():
     for steps, training in ((1, True), (1, False), (2, True)):
         assert torch.equal(block.train(training)(x), x)
         assert torch.equal(block.tokens_per_expert_E, torch.full((E,), steps * float(N // E)))
+
+    # counts made in inference mode are refused outside it, whichever way they would be added
+    with torch.inference_mode():
+        block.tokens_per_expert_E = torch.zeros(E)
+    with pytest.raises(RuntimeError, match="InferenceMode"):
+        block.train()(x)
+    block.router = moe.TokenChoiceTopKRouter(E, D, K, score_func="softmax", route_norm=True)
+    assert block._totals(x) is None
+    block.tokens_per_expert_E = torch.zeros(E)
+    assert block._totals(x) is block.tokens_per_expert_E

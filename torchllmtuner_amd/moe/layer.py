@@ -246,6 +246,7 @@ class MoE(nn.Module):
             or totals.dtype is not torch.float32
             or totals.device != tokens.device
             or totals.requires_grad
+            or totals.is_inference()  # (what only inference mode may write: the addition behind the operator says so)
             or not totals.is_contiguous()
             # (a router that does not say how many experts it has is none that the operator serves)
             or totals.numel() != getattr(self.router, "num_experts", None)
