@@ -501,8 +501,9 @@ int mi355_combine_bwd(const void* dout, const void* y, int dtype,
  * (>= 384) those two outputs are then not written at all; for any other dtype or shape
  * that is MI355_EINVAL (the other paths use the buffers as intermediates).
  * The kernels walk the plan's tile list in tiles of mi355_grouped_tile_m(dtype) rows
- * (256), so the list must have been built with that value, or find their rows from seg_counts
- * and seg_offsets: all rows counted there are within row_capacity.
+ * (256), so the list must have been built with that value; all rows counted in seg_counts are within
+ * row_capacity.  A list may leave tiles out, whose rows' results are then not written: any tiles, or, for bf16 with D and F
+ * multiples of 64 (>= 384), whole experts.
  */
 int64_t mi355_grouped_tile_m(int dtype);
 int mi355_grouped_swiglu_fwd(const void* rows, const int32_t* token_of_row, int64_t num_tokens,

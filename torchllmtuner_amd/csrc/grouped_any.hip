@@ -27,6 +27,7 @@
 #include "grouped_any.h"
 #include "router_few.h"
 #include "select_bwd.h"
+#include "tile_list.h"
 
 namespace mi355 {
 namespace {
@@ -47,6 +48,7 @@ struct AnyArgs {
   int K, N, ldb;                  // contraction (of one half), output columns, row length of the weights
   int64_t rows, w_elems;          // rows of the buffers, elements of one expert's weights
   const int32_t *seg_offsets, *seg_counts;
+  TileList list;
   int El, col_tiles;
   AnyDw dw[3];
   int num_dw;
@@ -343,12 +345,16 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
       }
     }
   } else {
-    // Which expert, pass of TM rows and columns: every wave adds up the experts' passes itself.
+    // Which expert, pass of TM rows and columns: every wave adds up the experts' passes itself, and their tiles, to see whether the list has them all.
     auto passes_of = [&](int count) { return (count + TM - 1) / TM; };
     auto count_of = [&](int b) { return b + lane < p.El ? p.seg_counts[b + lane] : 0; };
     const int count0 = count_of(0);
-    int total = 0;
-    for (int b = 0; b < p.El; b += 64) total += __builtin_amdgcn_readlane(wave_scan(passes_of(b ? count_of(b) : count0)), 63);
+    int total = 0, unlisted = -p.list.size();
+    for (int b = 0; b < p.El; b += 64) {
+      const int c = b ? count_of(b) : count0;
+      total += __builtin_amdgcn_readlane(wave_scan(passes_of(c)), 63);
+      unlisted += __builtin_amdgcn_readlane(wave_scan(listed_tiles(c)), 63);
+    }
     if (!any_run(block, total * p.col_tiles)) return;
     const int pass_of_all = block / p.col_tiles;
     int e = 0, cnt = 0, before = 0, run = 0;
@@ -366,8 +372,11 @@ __device__ __forceinline__ void any_tile(const AnyArgs& p, int block, T* smem) {
     }
     const int q = block - before * p.col_tiles;
     const int pass = q / p.col_tiles;
-    row0 = p.seg_offsets[e] + pass * TM;
+    const int seg0 = p.seg_offsets[e];
+    int first = seg0 + pass * TM;
     m_valid = min(TM, cnt - pass * TM);
+    if (unlisted != 0 && !listed_rows(p.list, e, seg0, cnt, first, m_valid)) return;
+    row0 = first;
     n0 = (q - pass * p.col_tiles) * (MODE == ANY_GATEUP ? TN / 2 : TN);
     A0 = static_cast<const T*>(p.a0) + (ROWS_FOLD ? 0 : row0 * lda);
     a_bytes = (ROWS_FOLD ? p.src_rows : p.rows - row0) * lda * static_cast<int64_t>(sizeof(T));
@@ -891,6 +900,7 @@ static AnyArgs any_args(const AnySeg& g, int64_t rows, const AnyFold* f = nullpt
   }
   p.rows = rows;
   p.seg_offsets = g.seg_offsets; p.seg_counts = g.seg_counts;
+  p.list = {g.tile_expert, g.tile_row0, g.num_tiles, (int)std::min<int64_t>(g.tile_capacity, INT32_MAX)};
   return p;
 }
 

@@ -1167,8 +1167,9 @@ int few_rows_fwd(int stage, const void* a, const int32_t* a_src, int64_t a_rows,
 
 // grouped_short.hip
 int short_rows_fwd(int stage, bool tall, const void* a, const int32_t* a_src, int64_t a_rows, const void* b0, const void* b1,
-                   void* gate, void* up, void* out, const int32_t* seg_offsets, const int32_t* seg_counts, int64_t El, int64_t K,
-                   int64_t N, int64_t row_capacity, bool stream, bool turn, hipStream_t s);
+                   void* gate, void* up, void* out, const int32_t* seg_offsets, const int32_t* seg_counts, const int32_t* tile_expert,
+                   const int32_t* tile_row0, const int32_t* num_tiles, int64_t tile_capacity, int64_t El, int64_t K, int64_t N,
+                   int64_t row_capacity, bool stream, bool turn, hipStream_t s);
 
 // Up to eight rows per expert, or 64 rows in all (`rows`: as many as there may be; one rank's share of the experts may draw every token's).
 // A 16-row pass over an expert's weights costs the same for one row as for sixteen and a second pass
@@ -1260,11 +1261,13 @@ int bf16_grouped_fwd(const void* rows, const int32_t* token_of_row, int64_t num_
   }
   if (pass < 256) {
     if (stages & STAGE_GATEUP)
-      if (int rc = short_rows_fwd(1, pass > 64, rows, token_of_row, num_tokens, w1, w3, gate, up, h, seg_offsets, seg_counts, El,
-                                  D, F, row_capacity, stream, turned(El, row_capacity, D), s))
+      if (int rc = short_rows_fwd(1, pass > 64, rows, token_of_row, num_tokens, w1, w3, gate, up, h, seg_offsets, seg_counts,
+                                  tile_expert, tile_row0, num_tiles, tile_capacity, El, D, F, row_capacity, stream,
+                                  turned(El, row_capacity, D), s))
         return rc;
     if (stages & STAGE_DOWN)
-      return short_rows_fwd(2, pass > 64, h, nullptr, 0, w2, w2, nullptr, nullptr, y, seg_offsets, seg_counts, El, F, D, row_capacity, stream, turned(El, row_capacity, F), s);
+      return short_rows_fwd(2, pass > 64, h, nullptr, 0, w2, w2, nullptr, nullptr, y, seg_offsets, seg_counts, tile_expert, tile_row0,
+                            num_tiles, tile_capacity, El, F, D, row_capacity, stream, turned(El, row_capacity, F), s);
     return MI355_OK;
   }
   const bool beside = stages & STAGE_BESIDE;

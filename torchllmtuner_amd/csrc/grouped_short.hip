@@ -21,6 +21,7 @@
 
 #include "bf16_tiles.h"
 #include "common.h"
+#include "tile_list.h"
 
 namespace mi355 {
 namespace {
@@ -32,6 +33,7 @@ struct ShortArgs {
   const uint16_t *b0, *b1;    // (El, N, K) each; DOWN: b1 = b0
   uint16_t *gate, *up, *out;  // gate, up may be null
   const int32_t *seg_offsets, *seg_counts;
+  TileList list;
   int El, K, N, col_groups, last_row;  // last_row: of the row arrays
   int turn;    // a workgroup's contraction starts at a step of its own
   int stream;  // weights that one pass alone reads: with the non-temporal hint
@@ -55,13 +57,14 @@ __global__ __launch_bounds__(256, RB > 4 ? 2 : 3) void short_rows_kernel(ShortAr
   // Which expert, pass and columns: every wave adds up the experts' passes itself, from one load of their counts (a list in memory would be a second one behind
   // it, and both stand in front of the first weights).  An XCD has a run of (expert, column group, pass): passes that share weights are neighbours in
   // one L2, and so are an expert's column groups, which share its rows.
-  int count[4], to[4], total = 0;
+  int count[4], to[4], total = 0, unlisted = -p.list.size();
 #pragma unroll
   for (int b = 0; b < 4; ++b) count[b] = 64 * b + lane < p.El ? p.seg_counts[64 * b + lane] : 0;
 #pragma unroll
   for (int b = 0; b < 4; ++b) {
     to[b] = total + wave_scan((count[b] + ROWS - 1) / ROWS);
     total = __builtin_amdgcn_readlane(to[b], 63);
+    unlisted += __builtin_amdgcn_readlane(wave_scan(listed_tiles(count[b])), 63);
   }
   const int chunk = (total * p.col_groups + 7) >> 3, within = blockIdx.x >> 3, id = (blockIdx.x & 7) * chunk + within;
   if (within >= chunk || id >= total * p.col_groups) return;
@@ -107,7 +110,10 @@ __global__ __launch_bounds__(256, RB > 4 ? 2 : 3) void short_rows_kernel(ShortAr
       lds_load16(w1, off_hi, k, to + 3072);
     }
   };
-  const int row0 = ((const_i32)p.seg_offsets)[e] + pass * ROWS, left = min(cnt - pass * ROWS, ROWS), act = (left + 15) >> 4;
+  const int seg0 = ((const_i32)p.seg_offsets)[e];
+  int row0 = seg0 + pass * ROWS, left = min(cnt - pass * ROWS, ROWS);
+  if (unlisted != 0 && !listed_rows(p.list, e, seg0, cnt, row0, left)) return;
+  const int act = (left + 15) >> 4;
   const int l15 = lane & 15, l4 = lane >> 4;
   const uint32_t cpos = static_cast<uint32_t>((l4 ^ (l15 >> 1)) * 16);  // k 0..31; k 32..63: ^ 64
   const uint32_t ra = lds0 + l15 * 128u + cpos, rb = lds0 + B_AT + wave * 4096u + l15 * 128u + cpos;
@@ -206,13 +212,15 @@ __global__ __launch_bounds__(256, RB > 4 ? 2 : 3) void short_rows_kernel(ShortAr
 // gate/up (stage 1) or down (stage 2) of the forward; the arguments of bf16_grouped_fwd.  tall: 128 rows a pass, else 64; turn: each
 // tile's contraction starts at a step of its own (`turned` in grouped_bf16.hip).
 int short_rows_fwd(int stage, bool tall, const void* a, const int32_t* a_src, int64_t a_rows, const void* b0, const void* b1,
-                   void* gate, void* up, void* out, const int32_t* seg_offsets, const int32_t* seg_counts, int64_t El, int64_t K,
-                   int64_t N, int64_t row_capacity, bool stream, bool turn, hipStream_t s) {
+                   void* gate, void* up, void* out, const int32_t* seg_offsets, const int32_t* seg_counts, const int32_t* tile_expert,
+                   const int32_t* tile_row0, const int32_t* num_tiles, int64_t tile_capacity, int64_t El, int64_t K, int64_t N,
+                   int64_t row_capacity, bool stream, bool turn, hipStream_t s) {
   ShortArgs p{};
   p.a = (const uint16_t*)a; p.a_src = a_src; p.a_rows = (int)a_rows;
   p.b0 = (const uint16_t*)b0; p.b1 = (const uint16_t*)b1;
   p.gate = (uint16_t*)gate; p.up = (uint16_t*)up; p.out = (uint16_t*)out;
   p.seg_offsets = seg_offsets; p.seg_counts = seg_counts;
+  p.list = {tile_expert, tile_row0, num_tiles, (int)std::min<int64_t>(tile_capacity, INT32_MAX)};
   p.El = (int)El; p.K = (int)K; p.N = (int)N; p.last_row = (int)row_capacity - 1; p.turn = turn; p.stream = stream;
   const int width = stage == 1 ? 64 : 128;
   p.col_groups = (int)((N + width - 1) / width);
