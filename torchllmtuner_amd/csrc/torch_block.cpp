@@ -193,10 +193,13 @@ struct Fork {
   hipStream_t main;
   bool open = false;
   Fork(SideStream* s, hipStream_t m) : side(s), main(m) {}
-  void start() { follow(main); }
-  // the side stream waits for everything on `from`, which is behind `main` itself
-  void follow(hipStream_t from) {
-    TORCH_CHECK(side->chain(side->fork, from, side->stream), "moe_block: cannot fork to the side stream: ",
+  // in front of the call's first launch; behind one
+  void enter() { follow(main, side->entry); }
+  void start() { follow(main, side->fork); }
+  // the side stream waits for everything on `from`, another side stream with a launch of the call
+  void follow(hipStream_t from) { follow(from, side->fork); }
+  void follow(hipStream_t from, hipEvent_t event) {
+    TORCH_CHECK(side->chain(event, from, side->stream), "moe_block: cannot fork to the side stream: ",
                 hipGetErrorString(hipGetLastError()));
     open = true;
   }
@@ -256,7 +259,7 @@ std::tuple<Tensor, Tensor> choices_forward(const Block& b, const Tensor& totals)
   SideStream* aux = b.Fs > 0 && c.overlap ? side_stream(b.x.device().index(), main, 1) : nullptr;
   Fork shared(aux, main);
   if (aux) {
-    shared.start();
+    shared.enter();
     shared_forward(b, k, y_shared, aux->stream, true);
   }
   check(mi355_router_gate_fwd_partial(ptr(b.x), b.dt, fptr(b.gate_w), fptr(gate_b), partial, nullptr, b.T, b.D, b.E, L.stream),
@@ -319,7 +322,7 @@ std::tuple<Tensor, Tensor, Tensor> block_forward(const Block& b, const Stats& st
   SideStream* aux = b.Fs > 0 && c.overlap ? side_stream(b.x.device().index(), main, 1) : nullptr;
   Fork shared(aux, main);
   if (aux) {
-    shared.start();
+    shared.enter();
     shared_forward(b, k, y_shared, aux->stream, true);
   }
 
@@ -466,7 +469,7 @@ Grads block_backward(const Block& b, const Tensor& kept, const Tensor& dout_, co
   SideStream* side = routed && need.x && (beside || (b.shared_folded && aux && need.shared)) ? side_stream(device, main, 0) : nullptr;
   Fork shared(aux, main), weights(side, main);
   if (run_shared) {
-    if (aux) shared.start();
+    if (aux) shared.enter();
     void* stream = aux ? static_cast<void*>(aux->stream) : L.stream;
     if (b.shared_folded) {
       auto stage = [&](int s, void* on) {

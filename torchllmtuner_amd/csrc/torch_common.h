@@ -24,8 +24,9 @@ namespace mi355_torch {
 // nullptr means "stay on one stream".
 struct SideStream {
   hipStream_t stream = nullptr;
-  hipEvent_t fork = nullptr, join = nullptr;
-  std::mutex order;  // an event is recorded and waited for as one step: host threads share the pair
+  hipEvent_t entry = nullptr;                // a fork in front of a call's first launch
+  hipEvent_t fork = nullptr, join = nullptr;  // one behind a launch of the call, and a join
+  std::mutex order;  // an event is recorded and waited for as one step: host threads share the three
 
   // `to` waits for everything enqueued on `from` so far
   bool chain(hipEvent_t event, hipStream_t from, hipStream_t to) {
@@ -49,12 +50,15 @@ inline SideStream* side_stream(int device, hipStream_t current, int which = 0) {
     if (hipStreamIsCapturing(current, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone)
       return nullptr;  // not now: try again on a later, uncaptured call
     tried[device] = true;
-    // Without the system-scope fences of an ordinary event: what waits for these is a stream of the same device, for which the kernels' own
-    // device-scope fences are enough, and whatever later hands the data to the host or another device has fences of its own.  A step or forward with a fork and
-    // a join, us, with / without: 3000 tokens of 64 experts of 1024 x 512 364 / 359, 300 of 128 of 2048 x 768 701 / 695; one rank's share of 7168 x 2048 with its shared
-    // expert, forward of 16 and 128 tokens 182 / 178, 348 / 345, a step of 500 1492 / 1482.
+    // Without the system-scope fences of an ordinary event where what stands before it on its stream is a kernel of the same call and what waits for it one of the
+    // same device: the kernels' own device-scope fences order the two, that kernel began behind whatever a copy or another device had written for its stream (its own start
+    // drops stale lines from every L2), and whatever later hands results to the host or another device has fences of its own.  In front of a call's first launch no kernel
+    // has done that, a copy of the tokens may be the last thing on the stream: an ordinary event.  A step or forward, us, all with / all without: 3000 tokens of 64
+    // experts of 1024 x 512 364 / 359, 300 of 128 of 2048 x 768 701 / 695; one rank's share of 7168 x 2048 with its shared expert, forward of 16 and 128 tokens 182 / 178, 348 / 345,
+    // a step of 500 1492 / 1482.
     constexpr unsigned kEvent = hipEventDisableTiming | hipEventDisableSystemFence;
     if (hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking) != hipSuccess ||
+        hipEventCreateWithFlags(&s.entry, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&s.fork, kEvent) != hipSuccess ||
         hipEventCreateWithFlags(&s.join, kEvent) != hipSuccess) {
       (void)hipGetLastError();
