@@ -473,3 +473,19 @@ def test_running_counts_are_added_once_whichever_launch_adds_them(dtype, T, D, F
         block.tokens_per_expert_E = other
         assert block._totals(x) is None
         counted(call)
+
+
+@pytest.mark.parametrize("T", [0, 1, 5])
+def test_the_combine_adds_counts_with_and_without_tokens(T):
+    from torchllmtuner_amd import _lib
+
+    E, K, D = 300, 2, 16
+    p = lambda t: t.data_ptr() if t is not None else None
+    counts = torch.arange(E, dtype=torch.int32, device=DEV)
+    totals = torch.full((E,), 2.0, device=DEV)
+    y, out = torch.ones(T * K, D, device=DEV), torch.zeros(T, D, device=DEV)
+    weights, rows = torch.full((T, K), 0.5, device=DEV), torch.arange(T * K, dtype=torch.int32, device=DEV)
+    some = lambda t: p(t) if T else None
+    _lib.check(_lib.load().mi355_combine_count_fwd(some(y), 0, some(weights), some(rows), None, some(out), T, D, K, 0, p(counts), p(totals), E,
+                                                   torch.cuda.current_stream().cuda_stream), "combine_count_fwd")
+    assert torch.equal(totals, counts + 2.0) and torch.equal(out, torch.ones_like(out))

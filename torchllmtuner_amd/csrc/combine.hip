@@ -303,11 +303,11 @@ extern "C" int mi355_combine_count_fwd(const void* y, int dtype, const float* we
                                        const int32_t* counts, float* totals, int64_t E, void* stream) {
   MI355_REQUIRE(T >= 0 && D >= 1 && K >= 1 && K <= 64 && T < (1ll << 31) && D < (1ll << 31),
                 "combine_fwd: bad shape (K must be <= 64)");
-  if (T == 0) return MI355_OK;
-  MI355_REQUIRE(weights && row_of_slot && out, "combine_fwd: null pointer");
+  if (T == 0 && !totals) return MI355_OK;
+  MI355_REQUIRE(T == 0 || (weights && row_of_slot && out), "combine_fwd: null pointer");
   MI355_REQUIRE((!addend && !totals) || dtype != MI355_F64, "combine_fwd: no fp64 form with an addend or counts");
   MI355_REQUIRE(!totals || (counts && E >= 1 && E < (1ll << 31)), "combine_fwd: totals without counts");
-  const int64_t tokens = (T + 3) / 4;  // groups of one workgroup's four
+  const int64_t tokens = std::max<int64_t>(1, (T + 3) / 4);  // groups of one workgroup's four (without any: for the counts)
   const int64_t kib = (D * (dtype == MI355_F32 ? 4 : 2) + 1023) / 1024;  // 64 lanes of 16 bytes
   const int64_t pieces = std::max<int64_t>(1, std::min<int64_t>(kib, 0xffffff / tokens));  // a launch: below 2^32 lanes
   auto launch = [&](auto kernel, auto* yp, auto* op) {
