@@ -1,4 +1,5 @@
-"""Products of few experts on 128-column tiles against fp32 products, and the folded backward's pieces of the score gradient."""
+"""Backward products of few experts on 128-column tiles against fp32 products and the same on 256-column ones, and the folded backward's pieces of the score
+gradient.  Their forward, of as few rows, runs on 64-row passes (its row tiles: test_gpu_forward_tiles.py)."""
 
 from __future__ import annotations
 
@@ -66,7 +67,7 @@ def test_products(ops, counts, D, Fd):
 
 
 def wide(plan):
-    """The same plan with room for so many row tiles that no product of it runs on narrow ones."""
+    """The same plan with room for so many row tiles that no row-tiled product of it runs on narrow ones."""
     import dataclasses
 
     room = 4096 + plan.num_local_experts

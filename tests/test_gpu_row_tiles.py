@@ -16,6 +16,7 @@ DEV = "cuda:0"
 EDGES = (0, 1, 15, 16, 17, 48, 63, 64, 65, 127, 128, 129, 192, 193, 255, 256, 257, 300, 511, 512, 513, 769)
 
 
+# (the forward of the first and of the last two runs on passes of fewer rows: test_gpu_forward_tiles.py has the first's on row tiles)
 @pytest.mark.parametrize("counts,D,Fd", [(EDGES, 384, 384), (EDGES, 448, 576), (EDGES, 640, 448), (EDGES[::-1], 832, 384),
                                          ((513, 1, 255) * 24, 448, 448), ((1,), 384, 448), ((4099,), 448, 384)])
 def test_rows(counts, D, Fd):

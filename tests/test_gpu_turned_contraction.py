@@ -1,5 +1,5 @@
 """Products whose contraction starts at a K step of the tile's own (weight rows a multiple of 4 KiB apart, few rows per
-expert), against fp32 products of the same inputs."""
+expert), against fp32 products of the same inputs, on the 64-row passes (turned row tiles: test_gpu_forward_tiles.py)."""
 
 from __future__ import annotations
 
@@ -20,8 +20,8 @@ def ops():
     return o
 
 
-# one row tile an expert and several; whole output tiles and a last one that starts early (448 = 1.75 x 256, 3.5 x 128);
-# row counts on both sides of the 8 and 200 rows per expert between which the products are turned
+# one pass an expert and several; whole output tiles and a last one with columns left over (448 = 7 x 64, 3.5 x 128);
+# row counts on both sides of the 200 rows per expert up to which the products are turned
 @pytest.mark.parametrize("counts,D,Fd", [
     ((60, 0, 100, 257, 3), 2048, 512), ((60, 0, 100, 257, 3), 2048, 448), ((300, 9, 1, 17), 4096, 384),
     ((200, 200), 2048, 448), ((201, 200), 2048, 448), ((40, 30), 448, 2048), ((70, 0, 0), 640, 2048),
