@@ -1198,8 +1198,9 @@ static bool few_rows(int64_t El, int64_t rows, int64_t R, int64_t D, int64_t F) 
 // rows an expert 35-41 / 31-36 / 35-39; 16 of 1024 x 512, 90 to 220 rows 44-50 / 39-44 / 45-48, 300 51 / 53 / 54, 400 56 / 64 / 56; 32 of it, 90 rows 55 / 53 /
 // 52, 130 58 / 64 / 67; one dense segment of 7168 x 2048, 129 rows 132 / 78 / 118, 512 177 / 83 / 119, 1000 179 / 115 / 126, 1400 182 / 164 / 164, 2000
 // 187 / 238 / 185; of 2048 x 1408, 129 to 1400 rows 60-83 / 41-46 / 53-57.
-//   128 up to 90 rows where the weights stay in the memory-side cache: 16 of 2048 x 1024, 60 / 75 / 90 rows 74 / 78 / 66, 75 / 77 / 68, 76 / 77 / 70; 64 of 1024 x 512
-// 75 / 76 / 71, 77 / 81 / 74 (80 rows), 79 / 85 / 79; 64 of 640 x 704, 90 rows 80 / 79 / 75; 32 of 1280 x 640 71 / 68 / 72, 73 / 75 / 74, 75 / 77 / 78.  Weights from memory
+//   128 up to 90 rows where the passes are more and the weights stay in the memory-side cache: 64 of 1024 x 512, 60 / 75 / 90 rows
+// 75 / 76 / 71, 77 / 81 / 74 (80 rows), 79 / 85 / 79; 64 of 640 x 704, 90 rows 80 / 79 / 75; 32 of 1280 x 640 71 / 68 / 72, 73 / 75 / 74, 75 / 77 / 78.  (16 of 2048 x 1024 are
+// just two workgroups a CU and stay with 64: drawn evenly 74 / 78 / 66, 75 / 77 / 68, 76 / 77 / 70, but the products alone by Zipf's law 54 / 55 / 69, 58 / 55 / 71, 84 / 58 / 68.)  Weights from memory
 // arrive as fast through row tiles then (60 of 1728 x 960, 60 rows 150 / 162 / 151; 128 of 2048 x 768 261 / 300 / 267).
 //   A dense segment beside other products leaves them more CUs in passes of 128 (one rank's share of 7168 x 2048 with a shared expert of 2048, 128 tokens
 // 365 / 347 / 348, 200 390 / 398 / 391, 300 417 / 418 / 404, 512 460 / 484 / 464).
