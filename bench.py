@@ -369,7 +369,8 @@ def swiglu_stage_bytes(rows, experts, D, F, s, saves_gate_up=True, dh_writes_sca
     """Algorithmic HBM bytes of each grouped SwiGLU stage: every operand and every result once
     (``rows`` routed rows or tokens, ``experts`` weight sets of (F, D), element size ``s``;
     ``dh_writes_scaled_h``: the combine's backward is folded into dH, which then also writes
-    score * h for dW2)."""
+    score * h for dW2).  dW1 and dW3 as the routed experts' one launch of both, which reads the rows
+    once, and as two."""
     x, a, w = rows * D * s, rows * F * s, experts * D * F * s
     return {
         "gate_up": x + 2 * w + (3 if saves_gate_up else 1) * a,  # rows, w1, w3 -> (gate, up,) h
@@ -379,6 +380,7 @@ def swiglu_stage_bytes(rows, experts, D, F, s, saves_gate_up=True, dh_writes_sca
         "dw2": x + a + w,                                          # dy, h -> dW2
         "dw1": x + a + w,                                          # rows, dgate -> dW1
         "dw3": x + a + w,                                          # rows, dup -> dW3
+        "dw1+dw3": x + 2 * a + 2 * w,                              # rows, dgate, dup -> dW1, dW3
     }
 
 
@@ -406,7 +408,7 @@ def per_kernel_times(args, wl, block, x, gout, dev):
         logits = ops.router_gate_fwd(x, block.router.gate.weight, block.router.gate.bias)
         proj = 2.0 * R_rows * D * F
         stage_flops = {"gate_up": 2 * proj, "down": proj, "dh": proj, "drows": 2 * proj,
-                       "dw2": proj, "dw1": proj, "dw3": proj}
+                       "dw2": proj, "dw1+dw3": 2 * proj}
         if not wl.backward:
             stage_flops = {k: stage_flops[k] for k in ("gate_up", "down")}
         n_local = (wl.local_experts[1] - wl.local_experts[0]) if wl.local_experts else E
@@ -429,7 +431,7 @@ def per_kernel_times(args, wl, block, x, gout, dev):
                 buf["gate"] = buf["up"] = None
 
             def run_stage(s):
-                if s in ("dh", "dw2"):
+                if s in ("dh", "dw2", "dw1+dw3"):
                     ops.grouped_swiglu_combine_stage(s, buf, plan)
                 else:
                     ops.grouped_swiglu_stage(s, buf, plan)
@@ -615,13 +617,12 @@ def measure_workload(args, wl, steps, warmup, *, detail):
         args, wl, block, x2, g2, dev)
     peak = PEAK_BF16_TFLOPS if wl.dtype == torch.bfloat16 else PEAK_FP32_TFLOPS
 
-    # The kernel with the largest share of the step.  dW1 and dW3 are two launches of one kernel
-    # (the gathered weight gradient), so they count together; the shared expert's stages are
-    # launches of the same kernels over one dense segment and are listed under their own names.
+    # The kernel with the largest share of the step.  The routed experts' dW1 and dW3 are one launch;
+    # the shared expert's stages are launches of the same kernels over one dense segment, listed
+    # under their own names, its dW1 and dW3 two launches that count together.
     groups = {}
     for s in stage_ms:
-        key = "dw1+dw3" if s in ("dw1", "dw3") else s
-        g = groups.setdefault(f"grouped_{key}", {"ms": 0.0, "flops": 0.0, "launches": 0, "bytes": 0.0})
+        g = groups.setdefault(f"grouped_{s}", {"ms": 0.0, "flops": 0.0, "launches": 0, "bytes": 0.0})
         g["ms"] += stage_ms[s]; g["flops"] += stage_flops[s]; g["launches"] += 1; g["bytes"] += stage_bytes.get(s, 0.0)
     for s in shared_ms:
         key = "dw1+dw3" if s in ("dw1", "dw3") else s
@@ -635,9 +636,7 @@ def measure_workload(args, wl, steps, warmup, *, detail):
     traffic = traffic_commit = None
     tb, traffic_commit = measured_traffic(wl.key)
     if dominant.startswith("grouped_"):
-        parts = dominant[len("grouped_"):].split("+")
-        if parts and all(p in tb for p in parts):
-            traffic = sum(tb[p] for p in parts) / len(parts)
+        traffic = tb.get(dominant[len("grouped_"):])
     # The grouped and shared-expert products are matrix-core work: the fraction is their flops
     # (2*R*D*F per projection over real rows, padding excluded) per second against the dense
     # bf16 MFMA peak.  Their algorithmic bytes against the HBM peak, the flops per byte and the

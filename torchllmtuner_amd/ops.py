@@ -711,15 +711,16 @@ def moe_block(x_TD, gate_w_ED, gate_bias_E, expert_bias_E, w1_EFD, w3_EFD, w2_ED
 # ====================================================================== profiling hooks
 # One MFMA kernel per call on pre-allocated buffers, straight through the C ABI: for
 # profilers and per-kernel timing.  Not operators: they write into caller-owned buffers.
-STAGES = {"gate_up": 1, "down": 2, "dh": 4, "drows": 8, "dw2": 16, "dw1": 32, "dw3": 64}
+STAGES = {"gate_up": 1, "down": 2, "dh": 4, "drows": 8, "dw2": 16, "dw1": 32, "dw3": 64, "dw1+dw3": 96}
 
 
 def grouped_swiglu_combine_stage(stage: str, buf: dict, plan: PermutePlan):
-    """One backward kernel of the folded experts+combine backward on pre-allocated buffers.
+    """One launch of the folded experts+combine backward on pre-allocated buffers.
 
     ``buf`` maps dout, rows (the (T, D) tokens), row_scale, w1, w3, w2, gate, up, dgate, dup,
     hs, dot_partial, drows, dw1, dw3, dw2 to device tensors; ``stage`` is one of dh, drows,
-    dw2, dw1, dw3.
+    dw2, dw1, dw3, or dw1+dw3: both as the backward makes them, in one launch but for many experts
+    of one K step each.
     """
     x = buf["rows"]
     dev = _dev(x)
