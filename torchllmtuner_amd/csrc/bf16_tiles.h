@@ -70,17 +70,17 @@ typedef const __attribute__((address_space(3))) char* lds_cptr;
 // Requests 16 (4) bytes a lane from base + voff + soff, straight into LDS: lane l's land at byte lds + 16 l (4 l).  Written
 // out because the compiler drains the whole load counter in front of every LDS read once it knows of such a request; waited for by lds_wait.
 // (base, soff and lds are wave-uniform; byte offsets up to 4 GiB; the wait states are for scalar registers that a vector instruction wrote just before)
-__device__ __forceinline__ u32x4 lds_rsrc(uint64_t base) {
-  return u32x4{static_cast<uint32_t>(base), static_cast<uint32_t>(base >> 32), 0xffffffffu, 0x00020000u};
+__device__ __forceinline__ u32x4 lds_rsrc(uint64_t base, uint32_t bytes) {
+  return u32x4{static_cast<uint32_t>(base), static_cast<uint32_t>(base >> 32), bytes, 0x00020000u};
 }
-template <bool STREAM = false>  // with the non-temporal hint
+template <bool STREAM = false, uint32_t BYTES = 0xffffffffu>  // with the non-temporal hint; from a buffer of so many bytes, zeros for what lies past its end
 __device__ __forceinline__ void lds_load16(uint64_t base, uint32_t voff, uint32_t soff, uint32_t lds) {
   if constexpr (STREAM)
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
-                 ::"s"(lds), "v"(voff), "s"(lds_rsrc(base)), "s"(soff) : "memory");
+                 ::"s"(lds), "v"(voff), "s"(lds_rsrc(base, BYTES)), "s"(soff) : "memory");
   else
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                 ::"s"(lds), "v"(voff), "s"(lds_rsrc(base)), "s"(soff) : "memory");
+                 ::"s"(lds), "v"(voff), "s"(lds_rsrc(base, BYTES)), "s"(soff) : "memory");
 }
 // the same from a buffer of `bytes` bytes; zeros for what lies past its end
 __device__ __forceinline__ void lds_load16_within(uint64_t base, uint32_t bytes, uint32_t voff, uint32_t lds) {
@@ -95,7 +95,7 @@ __device__ __forceinline__ void lds_load4_within(uint64_t base, uint32_t bytes, 
 }
 __device__ __forceinline__ void lds_load4(uint64_t base, uint32_t voff, uint32_t soff, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dword %1, %2, %3 offen lds"
-               ::"s"(lds), "v"(voff), "s"(lds_rsrc(base)), "s"(soff) : "memory");
+               ::"s"(lds), "v"(voff), "s"(lds_rsrc(base, 0xffffffffu)), "s"(soff) : "memory");
 }
 // at most N of the wave's requests and stores are still under way
 template <int N>

@@ -50,6 +50,14 @@
 // Beside the MFMAs the loop has 48 reads and 140 other instructions a wave and K step, and they count: with addresses formed from scratch at each request (100
 // more) it took 8-10 % longer, with the row indices in scalar registers 3 %.
 //
+// Instructions count in the row tiles too.  A result's address used to be formed from scratch, with a division, a 64-bit product and a branch for rows past the
+// last (about 35 vector instructions a store, 24 stores a tile of gate/up, 3 us of its 8 us epilogue); now the tile's rows are a buffer that ends behind the
+// last of them and an address is one addition.  A request of weights used to branch on whether it carries the non-temporal hint; now the loop exists with
+// and without it (a K step's 104 scalar and 41 vector instructions are 62 and 4).  Rows past the last of a tile were read as copies of it; now they are zeros that nothing is read
+// for.  The three, us, before / with them: 128 experts of 2048 x 768, 512 rows each by Poisson draws gate/up 475 / 435, dRows 412 / 391, down 229 / 221; 16384
+// tokens of a skewed router 801 / 765, 772 / 731, 418 / 407; 64 of 1024 x 512, 281 rows 66 / 63, 56 / 53; one dense segment of 4096 rows of 7168 x 2048 178 / 172, 203 / 189, 99 / 97, dH
+// 114 / 105.
+//
 // MFMA of both: v_mfma_f32_16x16x32_bf16.  Per lane 8 bf16 of each operand (row lane%16,
 // k = 8*(lane/16)..+7), 4 fp32 of the result (column lane%16, rows 4*(lane/16) + i).
 // With random operand bits this shape sustains about 14 % more than 32x32x16 on this
@@ -83,6 +91,7 @@ typedef const int32_t __attribute__((address_space(4))) * const_i32;
 
 // LDS of the row-tiled kernels, in bytes: two stages of operands (A tile, B tile), 4 KiB a wave for its results
 constexpr uint32_t A_BYTES = 32768, STAGE_BYTES = 65536;
+constexpr uint32_t kNoRow = 0xffffff80u;  // no row of a matrix of whole 128-byte lines below 4 GiB begins there
 constexpr int R_LDS_BYTES = 2 * STAGE_BYTES + 8 * 4096;
 
 // RM_DLIN: the product of RM_DH (rows . w[e], the weight's contraction axis strided) with a plain epilogue:
@@ -120,6 +129,8 @@ struct RowArgs {
 // Row-tiled kernel: 256 rows of one expert x 64 NJ output columns, 8 waves as 4 (rows) x 2 (columns), each wave
 // 64 rows -- the 16-row blocks w, w + 4, w + 8, w + 12 for wave row w -- x 32 NJ.  GATEUP's columns are half gate and half
 // up columns of the same f range, so a wave holds gate and up of the same 16 NJ f.
+
+typedef __amdgpu_buffer_rsrc_t RowsOut;
 
 struct TileMeta {
   int e, row0, valid, n0, nt;
@@ -243,7 +254,6 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
   uint64_t gA0, gA1, gB0, gB1;  // A rows (k = 0), DX: second half of the contraction (dup); the B tile's origin in both weight stacks
   uint32_t voffA[NA];
   int k_start = 0, fk = 0;
-  bool stream = false;
   auto setup = [&](const TileMeta& m, const int (&asrc)[NA]) {
     const int64_t arow = GATHER ? 0 : static_cast<int64_t>(m.row0) * lda;
     gA0 = reinterpret_cast<uint64_t>(p.a0 + arow);
@@ -252,15 +262,16 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
     for (int i = 0; i < NA; ++i) {
       const int src = GATHER ? min(max(asrc[i], 0), p.a_rows - 1) : asrc[i];
       voffA[i] = (static_cast<uint32_t>(src) * static_cast<uint32_t>(lda) + static_cast<uint32_t>(kc_chunk * 8)) * 2u;
+      if (MODE != RM_DH && kc_row + 64 * i >= m.valid) voffA[i] = kNoRow;
     }
     // KC: the tile's first weight row is n0; KS: its first column is n0
     const int64_t borg = m.e * wsz + (B_KS ? static_cast<int64_t>(m.n0) : static_cast<int64_t>(m.n0) * ldb);
     gB0 = reinterpret_cast<uint64_t>(p.b0 + borg);
     gB1 = (MODE == RM_GATEUP || MODE == RM_DX) ? reinterpret_cast<uint64_t>(p.b1 + borg) : gB0;
     k_start = m.k_start;
-    stream = m.stream;
     fk = 0;
   };
+  // rows past the tile's last: past the end of the buffer that a request names, which makes them zeros and reads nothing
   auto tile_row = [&](const TileMeta& m, int i) { return max(min(kc_row + 64 * i, m.valid - 1), 0); };
   auto kofs = [&]() {
     if constexpr (!TURN) return fk * BK;
@@ -275,9 +286,9 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
     if constexpr (MODE == RM_DX) {
       if (k0 >= F) { k0 -= F; g = gA1; }
     }
-    lds_load16(g, voffA[i], k0 * 2, fst + wdst + i * 8192u);
+    lds_load16<false, kNoRow>(g, voffA[i], k0 * 2, fst + wdst + i * 8192u);
   };
-  auto req_b = [&](int i) {
+  auto req_b = [&](int i, auto stream) {
     int k0 = kofs();
     uint64_t g = gB0;
     uint32_t so;
@@ -299,16 +310,16 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
   };
   // the pieces of B in the order of the halves
   auto b_piece = [](int h, int j) { return MODE == RM_DOWN && NBX ? h + 2 * j : h * NBX + j; };
-  auto req_x = [&](int i) {
+  auto req_x = [&](int i, auto stream) {
     if (i < NA) req_a(i);
-    else req_b(b_piece(0, i - NA));
+    else req_b(b_piece(0, i - NA), stream);
   };
-  auto req_y = [&](int j) { req_b(b_piece(1, j)); };
-  auto issue = [&]() {
+  auto req_y = [&](int j, auto stream) { req_b(b_piece(1, j), stream); };
+  auto issue = [&](const TileMeta& cur) {
 #pragma unroll
-    for (int i = 0; i < NA + NBX; ++i) req_x(i);
+    for (int i = 0; i < NA + NBX; ++i) req_x(i, cur.stream);
 #pragma unroll
-    for (int j = 0; j < NBY; ++j) req_y(j);
+    for (int j = 0; j < NBY; ++j) req_y(j, cur.stream);
     fst ^= STAGE_BYTES;
     ++fk;
   };
@@ -352,8 +363,8 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
       asrc[i] = GATHER ? p.a_src[cur.row0 + r] : r;
     }
     setup(cur, asrc);
-    issue();
-    issue();
+    issue(cur);
+    issue(cur);
     lds_sync<VM_EPI>();
   }
 
@@ -389,7 +400,7 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
       fk = 0;
     }
   };
-  auto k_loop = [&](auto act_t) {
+  auto k_loop = [&](auto act_t, auto stream) {
     constexpr int ACT = decltype(act_t)::value;
     // A quarter of a K step's MFMAs; what else the quarter holds -- requests of the K step after the next, fragment reads of the
     // next quarter -- goes out between its 16-row blocks, where the matrix core is busy with the block before.
@@ -423,12 +434,12 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
       lds_sync<63>();
       mm(B_KS ? a0 : a1, b1, B_KS ? 1 : 0, [&](int q) {
         if (q == 0) return;
-        req_x(q - 1);
+        req_x(q - 1, stream);
 #pragma unroll
         for (int b = (q - 1) * 2; b < q * 2 && b < NJ; ++b) rd_b(b0, B_KS ? 1 : 0, B_KS ? 0 : 1, b);
       });
       mm(B_KS ? a1 : a0, b0, B_KS ? 0 : 1, [&](int q) {
-        if (q + 3 < NA + NBX) req_x(q + 3);
+        if (q + 3 < NA + NBX) req_x(q + 3, stream);
 #pragma unroll
         for (int b = q * 2; b < q * 2 + 2 && b < NJ; ++b) rd_b(b1, 1, 1, b);
       });
@@ -439,7 +450,7 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
       for (int b = 0; b < (B_KS ? 4 : 1); ++b) rb[b] ^= STAGE_BYTES;
       mm(a1, b1, 1, [&](int q) {
         if (q == 0) return;
-        if (q - 1 < NBY) req_y(q - 1);
+        if (q - 1 < NBY) req_y(q - 1, stream);
 #pragma unroll
         for (int i = (q - 1) * 2; i < q * 2 && i < 4; ++i) {
           if (i < ACT) rd_a(a0, 0, i);
@@ -450,32 +461,46 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
       ++fk;
     }
   };
-  switch (act) {
-    case 0: k_loop(std::integral_constant<int, 0>{}); break;
-    case 1: k_loop(std::integral_constant<int, 1>{}); break;
-    case 2: k_loop(std::integral_constant<int, 2>{}); break;
-    case 3: k_loop(std::integral_constant<int, 3>{}); break;
-    default: k_loop(std::integral_constant<int, 4>{});
-  }
+  // (the hint is the tile's own, also for what its loop requests of the next tile: a branch at each request cost 2 %)
+  auto with_blocks = [&](auto stream) {
+    switch (act) {
+      case 0: k_loop(std::integral_constant<int, 0>{}, stream); break;
+      case 1: k_loop(std::integral_constant<int, 1>{}, stream); break;
+      case 2: k_loop(std::integral_constant<int, 2>{}, stream); break;
+      case 3: k_loop(std::integral_constant<int, 3>{}, stream); break;
+      default: k_loop(std::integral_constant<int, 4>{}, stream);
+    }
+  };
+  if (cur.stream) with_blocks(std::true_type{});
+  else with_blocks(std::false_type{});
 
   // ---- epilogue: 16 rows at a time through the wave's own LDS, 16-byte coalesced rows ----
   // acc[mi][nj][i]: output row = wm + mi*16 + (lane&15); output column within the nj-th
   // 16-column tile = 4*(lane>>4) + i.
-  const int el = opaque(lane);
+  const uint32_t el = opaque(lane);
   constexpr int CH = 4 * NJ;  // 16-byte chunks per row of the wave's sub-tile
-  auto key = [](int m) { return CH == 16 ? m : m >> 1; };
+  auto key = [](uint32_t m) { return CH == 16 ? m : m >> 1; };
   auto put = [&](int m0, int nj, float v0, float v1, float v2, float v3) {
     const u32x2 pk = {pack2(v0, v1), pack2(v2, v3)};
-    const int c = nj * 2 + ((el >> 4) >> 1);
+    const uint32_t c = nj * 2 + ((el >> 4) >> 1);
     *reinterpret_cast<u32x2*>(reinterpret_cast<char*>(smem) + epi + (el & 15) * (CH * 16) + ((c ^ key((el & 15))) * 16) + ((el >> 4) & 1) * 8) = pk;
   };
-  auto get = [&](int m, int c) {
+  auto get = [&](uint32_t m, uint32_t c) {
     return *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(smem) + epi + m * (CH * 16) + ((c ^ key(m)) * 16));
   };
+  // The tile's rows of a matrix with rows of `pitch` bytes, as a buffer that ends behind the last of them: what a lane of the last 16-row block stores past them
+  // is dropped and what it loads is zero, so that every access is unconditional and one addition forms its address.
+  auto rows_of = [&](const auto* base, uint32_t pitch) {
+    const char* first = reinterpret_cast<const char*>(base) + static_cast<int64_t>(row0) * pitch;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(first), 0, valid * pitch, 0x00020000);
+  };
+  auto store16 = [&](RowsOut to, uint32_t offset, u32x4 v) { __builtin_amdgcn_raw_buffer_store_b128(v, to, offset, 0, 0); };
   if constexpr (MODE == RM_GATEUP) {
     // 16 rows of gate and up side by side (16 NJ columns each), then of h in the same place
     constexpr int WC = 16 * NJ, CPT = WC / 8;  // columns and chunks of one of them
-    const int f0 = n0 + wn * WC;
+    const uint32_t pitch = F * 2u, at = (wr * 16 + el / CPT) * pitch + (n0 + wn * WC) * 2u + el % CPT * 16u;
+    [[maybe_unused]] const RowsOut o0 = rows_of(p.o0, pitch), o1 = rows_of(p.o1, pitch);
+    const RowsOut o2 = rows_of(p.o2, pitch);
     lds_wait<VM_EPI>();
 #pragma unroll
     for (int mi = 0; mi < 4; ++mi) {
@@ -500,42 +525,24 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
           }
         }
         wave_lds_sync();
-        const int chunks = part == 0 ? CH : CPT;  // per row
+        // rows of one matrix, 64 / CPT an instruction
 #pragma unroll
-        for (int it = 0; it < chunks / 4; ++it) {
-          const int idx = it * 64 + el;
-          const int m = idx / chunks, rem = idx % chunks, t = rem / CPT, c = rem % CPT;
-          const int mr = mi * 64 + wr * 16 + m;
-          if (mr < valid) {
-            const u32x4 v = get(m, rem);
-            uint16_t* dst = (part == 1 ? p.o2 : (t == 0 ? p.o0 : p.o1)) + static_cast<int64_t>(row0 + mr) * F + f0 + c * 8;
-            *reinterpret_cast<u32x4*>(dst) = v;
+        for (int t = 0; t < (part == 0 ? 2 : 1); ++t)
+#pragma unroll
+          for (int it = 0; it < CPT / 4; ++it) {
+            const uint32_t m = it * (64 / CPT) + el / CPT, c = el % CPT;
+            store16(part == 1 ? o2 : t == 0 ? o0 : o1, at + (mi * 64 + it * (64 / CPT)) * pitch, get(m, t * CPT + c));
           }
-        }
         wave_lds_sync();
       }
     }
   } else if (act > 0) {
     const int c0 = n0 + wn * (32 * NJ);
-    // 64 rows x CH chunks, CH per el; a row's bytes go out contiguously; tiles never
-    // overhang in the columns.  Where the epilogue also LOADS (dH), lanes whose row lies past
-    // the tile's real rows redo the last real row instead (the same bytes to the same
-    // address), so that every load and store is unconditional: the compiler then knows how
-    // many are in flight and waits for exactly the ones it needs -- with predicated accesses
-    // every wait drains the whole queue, stores included (one counter serves both here).
-    constexpr int IPB = CH / 4;  // 16-byte pieces a el has of a block of 16 rows
-    // the u-th of them in the mi-th block: row of the block and chunk; row of the tile
-    auto chunk_at = [&](int mi, int u, int& m, int& c) {
-      const int idx = u * 64 + el;
-      m = min(idx / CH, valid - 1 - (mi * 64 + wr * 16));
-      c = idx % CH;
-    };
-    auto row_at = [&](int mi, int m) { return row0 + mi * 64 + wr * 16 + m; };
-    auto offset_at = [&](int mi, int u) -> int64_t {
-      int m, c;
-      chunk_at(mi, u, m, c);
-      return static_cast<int64_t>(row_at(mi, m)) * Ncols + c0 + c * 8;
-    };
+    // 64 rows x CH chunks, CH per lane; a row's bytes go out contiguously; tiles never overhang in the columns.
+    constexpr int IPB = CH / 4;  // 16-byte pieces a lane has of a block of 16 rows, 64 / CH rows apart
+    const uint32_t pitch = Ncols * 2u, lrow = el / CH, lc = el % CH, at = (wr * 16 + lrow) * pitch + c0 * 2u + lc * 16u;
+    auto offset_at = [&](int mi, int u) { return at + (mi * 64 + u * (64 / CH)) * pitch; };
+    const RowsOut o0 = rows_of(p.o0, pitch);
     auto stage = [&](int mi) {
 #pragma unroll
       for (int nj = 0; nj < NJ2; ++nj)
@@ -556,16 +563,17 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
       [[maybe_unused]] float* dots = reinterpret_cast<float*>(reinterpret_cast<char*>(smem) + epi + 2048);
       u32x4 gq[G], uq[G];
       float sq = 1.0f;  // lane l: the score of the block's row l % 16
+      const RowsOut o1 = rows_of(p.o1, pitch), in_gate = rows_of(p.gate, pitch), in_up = rows_of(p.up, pitch);
+      [[maybe_unused]] const RowsOut o2 = FUSE ? rows_of(p.o2, pitch) : o0, scale = FUSE ? rows_of(p.row_scale, 4) : o0,
+                                     slots = FUSE ? rows_of(p.dot_partial, p.dot_slots * 4u) : o0;
       auto request = [&](int mi, u32x4 (&g)[G], u32x4 (&u)[G], float& sc) {
 #pragma unroll
         for (int i = 0; i < G; ++i) {
-          int m, c;
-          chunk_at(mi, i, m, c);
-          const int64_t o = offset_at(mi, i);
-          g[i] = *reinterpret_cast<const u32x4*>(p.gate + o);
-          u[i] = *reinterpret_cast<const u32x4*>(p.up + o);
+          const uint32_t o = offset_at(mi, i);
+          g[i] = __builtin_amdgcn_raw_buffer_load_b128(in_gate, o, 0, 0);
+          u[i] = __builtin_amdgcn_raw_buffer_load_b128(in_up, o, 0, 0);
         }
-        if constexpr (FUSE) sc = p.row_scale[row_at(mi, min(el & 15, valid - 1 - (mi * 64 + wr * 16)))];
+        if constexpr (FUSE) sc = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(scale, (mi * 64 + wr * 16 + (el & 15)) * 4u, 0, 0));
       };
       request(0, gq, uq, sq);
       lds_wait<2 * G>();  // (2 G requests and more are younger than the next tile's operands)
@@ -579,9 +587,8 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
         stage(mi);
 #pragma unroll
         for (int u = 0; u < G; ++u) {
-          int m, c;
-          chunk_at(mi, u, m, c);
-          const u32x4 v = get(m, c);
+          const uint32_t m = u * (64 / CH) + lrow;
+          const u32x4 v = get(m, lc);
           const u32x4 gv = gq[u], uv = uq[u];
           const float sc = FUSE ? __shfl(sq, m) : 1.0f;
           float dot = 0.0f;
@@ -610,18 +617,19 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
             du[w] = pack2(r_du[0], r_du[1]);
             if constexpr (FUSE) hs[w] = pack2(r_hs[0], r_hs[1]);
           }
-          const int64_t o = offset_at(mi, u);
-          *reinterpret_cast<u32x4*>(p.o0 + o) = dg;
-          *reinterpret_cast<u32x4*>(p.o1 + o) = du;
+          const uint32_t o = offset_at(mi, u);
+          store16(o0, o, dg);
+          store16(o1, o, du);
           if constexpr (FUSE) {
-            *reinterpret_cast<u32x4*>(p.o2 + o) = hs;
+            store16(o2, o, hs);
             // columns below the tile's nominal start belong to its neighbour (a last tile
             // that would overhang starts early): they must not be counted twice
-            if (c0 + c * 8 < ntile * BNT) dot = 0.0f;
+            if (c0 + static_cast<int>(lc) * 8 < ntile * BNT) dot = 0.0f;
             const float total = row16_sum<CH>(dot);
             // all 16 lanes of the row store the same value to the same address (unconditional,
             // like every other access of this epilogue); of a narrow tile, whose 128 columns are two waves', to LDS
-            if constexpr (NJ == 4) p.dot_partial[static_cast<int64_t>(row_at(mi, m)) * p.dot_slots + ntile * WN + wn] = total;
+            if constexpr (NJ == 4)
+              __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(total), slots, ((mi * 64 + wr * 16 + m) * p.dot_slots + ntile * WN + wn) * 4u, 0, 0);
             else dots[mi * 16 + m] = total;
           }
         }
@@ -642,11 +650,7 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
         if (mi < act) {
           stage(mi);
 #pragma unroll
-          for (int u = 0; u < IPB; ++u) {
-            int m, c;
-            chunk_at(mi, u, m, c);
-            *reinterpret_cast<u32x4*>(p.o0 + offset_at(mi, u)) = get(m, c);
-          }
+          for (int u = 0; u < IPB; ++u) store16(o0, offset_at(mi, u), get(u * (64 / CH) + lrow, lc));
         }
         wave_lds_sync();
       }
@@ -657,7 +661,7 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
   if constexpr (MODE == RM_DH && GATHER && NJ == 2) {
     // a narrow tile's slot: both waves' sums; the slots past the last tile's, which a wide tile would have filled, are zero
     lds_sync<63>();
-    const int m = (el >> 4) * 64 + wr * 16 + (el & 15);  // of the tile
+    const int m = static_cast<int>((el >> 4) * 64 + wr * 16 + (el & 15));  // of the tile
     if (wn == 0 && m < valid) {
       const float* dots = reinterpret_cast<const float*>(reinterpret_cast<const char*>(smem) + epi + 2048);
       const float* other = dots + 1024;
