@@ -49,6 +49,8 @@
 // results, written at 4.6 TB/s); one dense segment of 4096 rows 116 / 102, 120 / 105; 12 or fewer rows an expert of 2048 x 768 75 / 77 (written at 5.2 TB/s).
 // Beside the MFMAs the loop has 48 reads and 140 other instructions a wave and K step, and they count: with addresses formed from scratch at each request (100
 // more) it took 8-10 % longer, with the row indices in scalar registers 3 %.
+// A gathered row's address without a branch for rows past the segment and with a 24-bit product (30 fewer), and a result's as one addition: dW2 of the first 210 / 203,
+// dW1 and dW3 409 / 402, of 250 rows each 108 / 105, 203 / 198, of the skewed router 364 / 359, 685 / 671; of 32 of 7168 x 2048, 128 rows 170 / 166.
 //
 // Instructions count in the row tiles too.  A result's address used to be formed from scratch, with a division, a 64-bit product and a branch for rows past the
 // last (about 35 vector instructions a store, 24 stores a tile of gate/up, 3 us of its 8 us epilogue); now the tile's rows are a buffer that ends behind the
@@ -834,9 +836,10 @@ __global__ __launch_bounds__(NT, 2) void wgrad_kernel(WgradArgs p) {
   };
   auto take_row = [&](int i) {
     if constexpr (INDEXED) {
+      // (rows and bytes of a row of a matrix below 4 GiB of 768 bytes a row or more both have 24 bits)
       const int r = min(max(static_cast<int>(voffG[i]), 0), p.src_rows - 1);
-      voffG[i] = static_cast<uint32_t>(r) * (GATHER ? ldB : ldA) + cc16;
-      if (left < BK && 2 * wave + (opaque(lane) >> 5) + 16 * i >= left) voffG[i] = kNowhere;
+      const uint32_t at = __umul24(static_cast<uint32_t>(r), GATHER ? ldB : ldA) + cc16;
+      voffG[i] = krow < left - 16 * i ? at : kNowhere;
     }
   };
   auto req = [&](bool is_a, int i) {
@@ -1004,9 +1007,11 @@ __global__ __launch_bounds__(NT, 2) void wgrad_kernel(WgradArgs p) {
     for (int ks = 1; ks < ksteps; ++ks) kstep(ks, std::false_type{});
 
     // the tile's results, 16 rows at a time through the wave's own LDS
-    const int el = opaque(lane);
+    const uint32_t el = opaque(lane);
     char* own = reinterpret_cast<char*>(smem) + epi;
     uint16_t* C = (t0.second ? p.c1 : p.c) + static_cast<int64_t>(t0.e) * M * N + static_cast<int64_t>(t0.m0 + wr * 64) * N + t0.n0 + wn * 128;
+    const RowsOut results = __builtin_amdgcn_make_buffer_rsrc(C, 0, 0xffffffffu, 0x00020000);
+    const uint32_t at = (el >> 4) * ldB + (el & 15) * 16u;
     if constexpr (INDEXED) {
       lds_wait<VM>();
       read_indices();
@@ -1015,20 +1020,21 @@ __global__ __launch_bounds__(NT, 2) void wgrad_kernel(WgradArgs p) {
     for (int mi = 0; mi < 4; ++mi) {
 #pragma unroll
       for (int nj = 0; nj < 8; ++nj) {
-        const int m = el & 15, c = nj * 2 + (el >> 5);
+        const uint32_t m = el & 15, c = nj * 2 + (el >> 5);
         const u32x2 pk = {pack2(acc[mi][nj][0], acc[mi][nj][1]), pack2(acc[mi][nj][2], acc[mi][nj][3])};
         *reinterpret_cast<u32x2*>(own + m * 256 + ((c ^ m) * 16) + ((el >> 4) & 1) * 8) = pk;
       }
       wave_lds_sync();
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const int m = u * 4 + (el >> 4), c = el & 15;
+        const uint32_t m = u * 4 + (el >> 4), c = el & 15;
         // (non-temporal: a weight gradient is several times the size of L2 and is read next by the
         // optimizer; written through the cache as ordinary stores, an expert's 30-60 MB of results push
         // its own operands out of L2 between two of its tiles -- with few rows per expert, where the
         // product is bound by these writes, the gathered rows were fetched from memory several times over)
-        __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(own + m * 256 + ((c ^ m) * 16)),
-                                    reinterpret_cast<u32x4*>(C + static_cast<int64_t>(mi * 16 + m) * N + c * 8));
+        constexpr int kNonTemporal = 2;
+        __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const u32x4*>(own + m * 256 + ((c ^ m) * 16)), results,
+                                               at + (mi * 16 + u * 4) * ldB, 0, kNonTemporal);
       }
       wave_lds_sync();
     }
