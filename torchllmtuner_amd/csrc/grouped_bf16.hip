@@ -76,6 +76,7 @@
 
 #include "bf16_tiles.h"
 #include "common.h"
+#include "tile_list.h"
 
 namespace mi355 {
 namespace {
@@ -126,6 +127,41 @@ struct RowArgs {
   int D, F;
   int n_tiles;
   int stream;  // weights of experts with one row tile are read with the non-temporal hint
+  int short_tiles;  // tiles of up to 128 rows may take the place of the listed ones
+  int El, tile_capacity;
+};
+
+// The tiles of up to 128 rows that the experts' rows make (at most 256 experts), found by every wave from the counts.
+struct ShortTiles {
+  int to[4];  // lane l, b: tiles of the experts up to and with 64 b + l
+  int total = 0, listed = 0, unlisted = 0;  // tiles; those of 256 rows, and how many of them the list leaves out
+  TileList list;
+  __device__ __forceinline__ void find(const RowArgs& p) {
+    const int lane = threadIdx.x & 63;
+    list = {p.tile_expert, p.tile_row0, p.num_tiles, p.tile_capacity};
+    int count[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) count[b] = 64 * b + lane < p.El ? p.seg_counts[64 * b + lane] : 0;
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+      to[b] = total + wave_scan((count[b] + 127) / 128);
+      total = __builtin_amdgcn_readlane(to[b], 63);
+      listed += __builtin_amdgcn_readlane(wave_scan(listed_tiles(count[b])), 63);
+    }
+    unlisted = listed - list.size();
+  }
+  // the expert of tile t and the tiles of those before it
+  __device__ __forceinline__ int expert(int t, int& before) const {
+    int e = 0;
+#pragma unroll
+    for (int b = 3; b >= 0; --b) {
+      const unsigned long long past = __ballot(to[b] > t);
+      if (past) e = 64 * b + __ffsll(past) - 1;
+    }
+    const int l = (e - 1) & 63, b = (e - 1) >> 6;
+    before = e == 0 ? 0 : __builtin_amdgcn_readlane(b < 2 ? (b == 0 ? to[0] : to[1]) : (b == 2 ? to[2] : to[3]), l);
+    return e;
+  }
 };
 
 // Row-tiled kernel: 256 rows of one expert x 64 NJ output columns, 8 waves as 4 (rows) x 2 (columns), each wave
@@ -160,10 +196,12 @@ __device__ __forceinline__ float row16_sum(float v) {
 // channels at a time.  The column tile counts only where the output is a whole number of tiles: a last tile
 // that would overhang computes some of its neighbour's columns again and must give the same bits, so both add up in
 // the same order.  An expert's row tiles and, where there are several, its column tiles stay in step: they share operands in L2.
-template <int MODE, int NJ, bool GATHER, bool SAVE_GU = true, bool TURN = false>
-__global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
+template <int MODE, int NJ, bool GATHER, bool SAVE_GU, bool TURN, int MB>
+__device__ __forceinline__ void row_tiles(const RowArgs& p, const ShortTiles& tiles) {
   constexpr int WM = 4, WN = 2;            // waves along the rows and along the columns
-  constexpr int TBM = 64 * WM;             // rows of the tile
+  constexpr int TBM = 16 * MB * WM;        // rows of the tile
+  constexpr bool SHORT = MB == 2;
+  constexpr uint32_t A_BYTES = TBM * 128u, STAGE_BYTES = A_BYTES + 32768u;
   constexpr int BNT = 32 * NJ * WN;        // output columns of the tile (WN waves x NJ x 32)
   constexpr int NA = TBM / 64;             // 1 KiB pieces of the A tile a wave requests per K step
   constexpr int NB = BNT / 64;             // the same for B
@@ -174,7 +212,7 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
   // is a read of the weights).  Narrow down tiles: a piece holds both halves of a wave's columns.
   constexpr int NBX = MODE == RM_DOWN && NJ == 2 ? 0 : NB / 2, NBY = NB - NBX;
   constexpr int VM = NBX ? NA + NB : NA;   // requests younger than those a barrier of the loop waits for
-  constexpr int VM_EPI = NBX ? NBY : 0;    // ... than those that the next tile's first K step needs
+  constexpr int VM_EPI = SHORT ? NA + NB : NBX ? NBY : 0;    // ... than those that the next tile's first K step needs
   static_assert(!GATHER || MODE == RM_GATEUP || MODE == RM_DH, "only gate/up and dH gather their rows");
   static_assert(!TURN || !B_KS, "only contractions that are contiguous in memory are turned");
   static_assert(!(GATHER && MODE == RM_DH) || NJ == 4 || NJ == 2, "the fused dH epilogue reduces over 16 lanes per row, or 8 and a second wave");
@@ -194,8 +232,7 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
   // Persistent workgroups: block b serves XCD b % 8 and walks that XCD's contiguous run
   // of the tile list with stride gridDim/8, the order in which the hardware dispatcher
   // would have started one-tile blocks.  Tile metadata is looked up two tiles ahead.
-  const int num_tiles = *p.num_tiles;
-  const int total = num_tiles * p.n_tiles;
+  const int total = (SHORT ? tiles.total : *p.num_tiles) * p.n_tiles;
   const int chunk = (total + 7) >> 3;
   const int stride = gridDim.x >> 3;
   const int pid_base = (blockIdx.x & 7) * chunk;
@@ -209,7 +246,8 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
     // would wait for all of those
     const int t = pid / p.n_tiles;  // some tile of the expert this work item belongs to
     TileMeta m;
-    m.e = ((const_i32)p.tile_expert)[t];
+    [[maybe_unused]] int before = 0;
+    m.e = SHORT ? tiles.expert(t, before) : ((const_i32)p.tile_expert)[t];
     const int cnt_e = ((const_i32)p.seg_counts)[m.e], off_e = ((const_i32)p.seg_offsets)[m.e];
     const int h = even_tile_rows(cnt_e, TBM);
     const int nrt = max((cnt_e + TBM - 1) / TBM, 1);  // row tiles of the expert
@@ -222,7 +260,7 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
     // column-tile-major throughout fetches the rows of an expert with many row tiles once per
     // column tile.
     constexpr int G = 3;
-    const int t0 = t - (((const_i32)p.tile_row0)[t] - off_e) / h;  // the expert's first tile
+    const int t0 = SHORT ? before : t - (((const_i32)p.tile_row0)[t] - off_e) / h;  // the expert's first tile
     const int q = pid - t0 * p.n_tiles;
     const int blk = q / (G * p.n_tiles);
     const int qb = q - blk * (G * p.n_tiles);
@@ -230,13 +268,18 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
     const int nt = qb / g, rt = blk * G + (qb - nt * g);
     m.row0 = off_e + rt * h;
     m.valid = min(h, cnt_e - rt * h);
+    if constexpr (SHORT)
+      if (tiles.unlisted != 0 && !listed_rows(tiles.list, m.e, off_e, cnt_e, m.row0, m.valid)) {
+        m.row0 = off_e;
+        m.valid = 0;
+      }
     // a last tile that would overhang starts early instead and recomputes a few columns
     // of its neighbour (same values), so no column is ever clamped
     constexpr int W = (MODE == RM_GATEUP ? BNT / 2 : BNT);
     m.n0 = min(nt * W, Ncols - W);
     m.nt = nt;
     m.stream = p.stream && nrt == 1;
-    m.k_start = TURN ? (5 * m.e + (nrt == 1 && Ncols % W == 0 ? 3 * nt : 0)) % ksteps : 0;
+    m.k_start = TURN ? (5 * m.e + (cnt_e <= 256 && Ncols % W == 0 ? 3 * nt : 0)) % ksteps : 0;
     return m;
   };
 
@@ -281,6 +324,7 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
     return (ks < ksteps ? ks : ks - ksteps) * BK;
   };
   uint32_t fst = 0;  // LDS stage (byte offset) the requests go to
+  [[maybe_unused]] uint32_t rst = 0;  // ... and, of three, the one that is read
   const uint32_t wdst = lds0 + wave * 1024u;
   auto req_a = [&](int i) {
     int k0 = kofs();
@@ -317,12 +361,16 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
     else req_b(b_piece(0, i - NA), stream);
   };
   auto req_y = [&](int j, auto stream) { req_b(b_piece(1, j), stream); };
+  auto next_stage = [](uint32_t& st) {
+    if constexpr (SHORT) st = st == 2 * STAGE_BYTES ? 0 : st + STAGE_BYTES;
+    else st ^= STAGE_BYTES;
+  };
   auto issue = [&](const TileMeta& cur) {
 #pragma unroll
     for (int i = 0; i < NA + NBX; ++i) req_x(i, cur.stream);
 #pragma unroll
     for (int j = 0; j < NBY; ++j) req_y(j, cur.stream);
-    fst ^= STAGE_BYTES;
+    next_stage(fst);
     ++fk;
   };
 
@@ -352,11 +400,13 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
   };
 
   constexpr int NJ2 = 2 * NJ;
-  f32x4 acc[4][NJ2];
+  f32x4 acc[MB][NJ2];
 
   TileMeta cur = load_meta(within);
   TileMeta nxt = load_meta(exists(within + stride) ? within + stride : within);
-  const uint32_t epi = 2 * STAGE_BYTES + wave * 4096u;  // the wave's own 4 KiB
+  // the wave's own 4 KiB for its results: of a third stage's, the one that the next tile's first step will request
+  uint32_t epi = 2 * STAGE_BYTES + wave * 4096u;
+  const uint32_t idx_at = SHORT ? 3 * STAGE_BYTES + wave * 256u : epi;  // ... 256 bytes for the next tile's row indices
   {
     int asrc[NA];
 #pragma unroll
@@ -378,11 +428,11 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
   if constexpr (GATHER) {
     // the next tile's row indices into the wave's own LDS: lane 8 i + r has that of row r of its i-th piece
     const int ol = opaque(lane), r = max(min(8 * wave + (ol & 7) + 64 * ((ol >> 3) & 3), nxt.valid - 1), 0);
-    lds_load4(reinterpret_cast<uint64_t>(p.a_src + nxt.row0), r * 4u, 0, lds0 + epi);
+    lds_load4(reinterpret_cast<uint64_t>(p.a_src + nxt.row0), r * 4u, 0, lds0 + idx_at);
   }
 
 #pragma unroll
-  for (int mi = 0; mi < 4; ++mi)
+  for (int mi = 0; mi < MB; ++mi)
 #pragma unroll
     for (int nj = 0; nj < NJ2; ++nj)
 #pragma unroll
@@ -390,19 +440,19 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
 
   // The tile's 16-row blocks are dealt to the four wave rows in turn, so that a tile that is not full keeps all waves
   // equally busy; the K loop is instantiated for the number of blocks a wave has.
-  const int act = min(max(((valid + 15) >> 4) - wr + 3, 0) >> 2, 4);
+  const int act = min(max(((valid + 15) >> 4) - wr + 3, 0) >> 2, MB);
   auto next_tile = [&]() {
     if (more) {
       int asrc[NA];
 #pragma unroll
       for (int i = 0; i < NA; ++i)
-        asrc[i] = GATHER ? lds_read_i32(lds0 + epi + (8 * i + (opaque(lane) >> 3)) * 4) : tile_row(nxt, i);
+        asrc[i] = GATHER ? lds_read_i32(lds0 + idx_at + (8 * i + (opaque(lane) >> 3)) * 4) : tile_row(nxt, i);
       setup(nxt, asrc);
     } else {
       fk = 0;
     }
   };
-  auto k_loop = [&](auto act_t, auto stream) {
+  [[maybe_unused]] auto k_loop = [&](auto act_t, auto stream) {
     constexpr int ACT = decltype(act_t)::value;
     // A quarter of a K step's MFMAs; what else the quarter holds -- requests of the K step after the next, fragment reads of the
     // next quarter -- goes out between its 16-row blocks, where the matrix core is busy with the block before.
@@ -463,18 +513,89 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
       ++fk;
     }
   };
+  [[maybe_unused]] auto k_loop_short = [&](auto act_t, auto stream) {
+    constexpr int ACT = decltype(act_t)::value;
+    // Half a K step's MFMAs: 32 k of the tile's columns, requests and the other half's fragment reads between its groups of four.
+    auto mm = [&](const bf16x8 (&af)[2], const bf16x8 (&bf)[NJ2], auto between) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        __builtin_amdgcn_sched_barrier(0);
+        between(q);
+        __builtin_amdgcn_sched_barrier(0);
+        if ((q & 1) < ACT) {
+#pragma unroll
+          for (int b = 0; b < NJ; ++b)
+            acc[q & 1][(q >> 1) * NJ + b] =
+                __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[(q >> 1) * NJ + b], af[q & 1], acc[q & 1][(q >> 1) * NJ + b], 0, 0, 0);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    bf16x8 a0[2], a1[2], b0[NJ2], b1[NJ2];
+    auto read = [&](bf16x8 (&a)[2], bf16x8 (&b)[NJ2], int kk, int q) {
+      if (q < ACT) a[q] = lds_read16((kk ? ra ^ 64u : ra) + rst + q * 8192u);
+#pragma unroll
+      for (int j = 2 * q; j < 2 * q + 2; ++j) {
+        if constexpr (!B_KS) {
+          const uint32_t base = (kk ? rb[0] ^ 64u : rb[0]) + rst;
+          b[j] = lds_read16(base + (MODE == RM_GATEUP ? (j / NJ) * (BNT / 2) * 128u + (j % NJ) * 2048u : j * 2048u));
+        } else {
+          b[j] = lds_read_tr<BNT * 2>((rb[j % NJ] ^ ((j / NJ) * 128u)) + rst + kk * 32u * (BNT * 2u));
+        }
+      }
+    };
+    auto request = [&](int i) { i < NA + NBX ? req_x(i, stream) : req_y(i - NA - NBX, stream); };
+    auto step = [&](int ks, auto first_t) {
+      constexpr bool FIRST = decltype(first_t)::value;
+      if (ks == ksteps - 2) next_tile();
+      if constexpr (!FIRST) lds_wait<NA + NB>();
+      lds_sync<63>();
+      auto between = [&](int q) {
+        read(a0, b0, 0, q);
+        if (q > 0) request(q - 1);
+      };
+      if constexpr (FIRST) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) between(q);
+      } else {
+        mm(a1, b1, between);
+      }
+      mm(a0, b0, [&](int q) {
+        read(a1, b1, 1, q);
+        if (q < 3) request(q + 3);
+      });
+      next_stage(fst);
+      next_stage(rst);
+      ++fk;
+    };
+    step(0, std::true_type{});
+    for (int ks = 1; ks < ksteps; ++ks) step(ks, std::false_type{});
+    mm(a1, b1, [](int) {});
+  };
   // (the hint is the tile's own, also for what its loop requests of the next tile: a branch at each request cost 2 %)
   auto with_blocks = [&](auto stream) {
-    switch (act) {
-      case 0: k_loop(std::integral_constant<int, 0>{}, stream); break;
-      case 1: k_loop(std::integral_constant<int, 1>{}, stream); break;
-      case 2: k_loop(std::integral_constant<int, 2>{}, stream); break;
-      case 3: k_loop(std::integral_constant<int, 3>{}, stream); break;
-      default: k_loop(std::integral_constant<int, 4>{}, stream);
+    if constexpr (SHORT) {
+      switch (act) {
+        case 0: k_loop_short(std::integral_constant<int, 0>{}, stream); break;
+        case 1: k_loop_short(std::integral_constant<int, 1>{}, stream); break;
+        default: k_loop_short(std::integral_constant<int, 2>{}, stream);
+      }
+    } else {
+      switch (act) {
+        case 0: k_loop(std::integral_constant<int, 0>{}, stream); break;
+        case 1: k_loop(std::integral_constant<int, 1>{}, stream); break;
+        case 2: k_loop(std::integral_constant<int, 2>{}, stream); break;
+        case 3: k_loop(std::integral_constant<int, 3>{}, stream); break;
+        default: k_loop(std::integral_constant<int, 4>{}, stream);
+      }
     }
   };
   if (cur.stream) with_blocks(std::true_type{});
   else with_blocks(std::false_type{});
+  if constexpr (SHORT) {
+    lds_sync<63>();  // all waves have read the stage that the results go through
+    epi = fst + wave * 4096u;
+  }
 
   // ---- epilogue: 16 rows at a time through the wave's own LDS, 16-byte coalesced rows ----
   // acc[mi][nj][i]: output row = wm + mi*16 + (lane&15); output column within the nj-th
@@ -505,7 +626,7 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
     const RowsOut o2 = rows_of(p.o2, pitch);
     lds_wait<VM_EPI>();
 #pragma unroll
-    for (int mi = 0; mi < 4; ++mi) {
+    for (int mi = 0; mi < MB; ++mi) {
       if (mi >= act) continue;
 #pragma unroll
       for (int part = SAVE_GU ? 0 : 1; part < 2; ++part) {
@@ -578,14 +699,14 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
         if constexpr (FUSE) sc = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(scale, (mi * 64 + wr * 16 + (el & 15)) * 4u, 0, 0));
       };
       request(0, gq, uq, sq);
-      lds_wait<2 * G>();  // (2 G requests and more are younger than the next tile's operands)
+      lds_wait<2 * G + (SHORT ? VM_EPI : 0)>();  // (2 G requests and more are younger than the next tile's operands)
 #pragma unroll
-      for (int mi = 0; mi < 4; ++mi) {
+      for (int mi = 0; mi < MB; ++mi) {
         if (mi >= act) break;
         u32x4 gn[G], un[G];
         float sn;
         // (the last block again past it: every load is unconditional)
-        if (mi < 3) request(min(mi + 1, act - 1), gn, un, sn);
+        if (mi < MB - 1) request(min(mi + 1, act - 1), gn, un, sn);
         stage(mi);
 #pragma unroll
         for (int u = 0; u < G; ++u) {
@@ -636,7 +757,7 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
           }
         }
         wave_lds_sync();
-        if (mi < 3) {
+        if (mi < MB - 1) {
 #pragma unroll
           for (int u = 0; u < G; ++u) {
             gq[u] = gn[u];
@@ -648,7 +769,7 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
     } else {
       lds_wait<VM_EPI>();
 #pragma unroll
-      for (int mi = 0; mi < 4; ++mi) {
+      for (int mi = 0; mi < MB; ++mi) {
         if (mi < act) {
           stage(mi);
 #pragma unroll
@@ -679,6 +800,31 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
   nxt = nxt2;
   }
   lds_wait<0>();
+}
+
+// Short tiles, of up to 128 rows with three stages of operands, where most experts have no more rows, so that the product is a read of their weights: a step's
+// requests then go out two whole steps ahead and behind one barrier.  A plain read in this pattern has 6.1 TB/s with two stages of 32 KiB and 7.0 with three; with
+// the rows and their results beside it, us, 256-row tiles / these, of Poisson loads from memory: 128 experts of 2048 x 768, 40 rows each gate/up 146 / 142, down
+// 82 / 79; 62 rows 147 / 144, 87 / 83; 100 rows 152 / 149, 92 / 89; 32 of 7168 x 2048, 60 rows 311 / 303, 176 / 173, 347 / 341; 100
+// rows 323 / 316, 182 / 178, 361 / 360; 60 of 1728 x 960, 60 and 100 rows gate/up 83 / 80, 88 / 85, down 45 / 44, 48 / 47, dRows 80 / 77, 85 / 82.  The same bits.
+//   Not where the tiles are more by a quarter, or need a round of workgroups more (115 rows of the first, one expert in nine above 128: gate/up 156 / 182, dRows
+// 155 / 171); not where the weights stay in the memory-side cache (64 experts of 1024 x 512, 100 rows: dRows 31 / 37); not dH, whose epilogue's loads
+// wait for what has been requested before them: 160 / 163; not dRows where weight rows lie a multiple of 4 KiB apart (20 rows of the first 130 / 134, 62 rows 146 / 146).  A forward
+// of 1000 tokens of the first, eight each, 257 / 252.
+template <int MODE, int NJ, bool GATHER, bool SAVE_GU = true, bool TURN = false>
+__global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
+  ShortTiles tiles;
+  if constexpr (NJ == 4 && (MODE == RM_GATEUP || MODE == RM_DOWN || MODE == RM_DX)) {
+    if (p.short_tiles) {
+      tiles.find(p);
+      auto rounds = [&](int n) { return (n * p.n_tiles + static_cast<int>(gridDim.x) - 1) / static_cast<int>(gridDim.x); };
+      if (tiles.total * 4 <= tiles.listed * 5 && rounds(tiles.total) <= rounds(tiles.listed)) {
+        row_tiles<MODE, NJ, GATHER, SAVE_GU, TURN, 2>(p, tiles);
+        return;
+      }
+    }
+  }
+  row_tiles<MODE, NJ, GATHER, SAVE_GU, TURN, 4>(p, tiles);
 }
 
 // ---- weight gradients: C[e](M,N) = sum_{r in segment e} A[r][m] * B[r][n] ----------
@@ -1146,6 +1292,9 @@ static int launch_row(RowArgs& a, int64_t width, int64_t El, int64_t tile_capaci
                       bool beside = false) {
   constexpr int div = MODE == RM_GATEUP ? 2 : 1;
   a.stream = streamed(El, a.D, a.F);
+  a.El = (int)El; a.tile_capacity = (int)std::min<int64_t>(tile_capacity, INT32_MAX);
+  // (what the kernel's waves add up; dRows' weights are read in rows of the output's width, which the two stages wait less for where they lie a multiple of 4 KiB apart)
+  a.short_tiles = a.stream && El > 1 && El <= 256 && !(MODE == RM_DX && width % 2048 == 0);
   a.n_tiles = (int)((width + 256 / div - 1) / (256 / div));
   const int64_t narrow_n = (width + 128 / div - 1) / (128 / div);
   if (narrow(MODE, El, a.n_tiles, narrow_n, tile_capacity)) {
