@@ -403,7 +403,6 @@ __device__ __forceinline__ void row_tiles(const RowArgs& p, const ShortTiles& ti
   f32x4 acc[MB][NJ2];
 
   TileMeta cur = load_meta(within);
-  TileMeta nxt = load_meta(exists(within + stride) ? within + stride : within);
   // the wave's own 4 KiB for its results: of a third stage's, the one that the next tile's first step will request
   uint32_t epi = 2 * STAGE_BYTES + wave * 4096u;
   const uint32_t idx_at = SHORT ? 3 * STAGE_BYTES + wave * 256u : epi;  // ... 256 bytes for the next tile's row indices
@@ -417,8 +416,10 @@ __device__ __forceinline__ void row_tiles(const RowArgs& p, const ShortTiles& ti
     setup(cur, asrc);
     issue(cur);
     issue(cur);
-    lds_sync<VM_EPI>();
   }
+  // (looked up with the first operands under way, not in front of them)
+  TileMeta nxt = load_meta(exists(within + stride) ? within + stride : within);
+  lds_sync<VM_EPI>();
 
   for (;;) {
   const bool more = exists(within + stride);
