@@ -423,8 +423,6 @@ __device__ __forceinline__ void row_tiles(const RowArgs& p, const ShortTiles& ti
 
   for (;;) {
   const bool more = exists(within + stride);
-  // the tile after the next: looked up now, used one tile later
-  const TileMeta nxt2 = load_meta(exists(within + 2 * stride) ? within + 2 * stride : within);
   const int row0 = cur.row0, valid = cur.valid, n0 = cur.n0, ntile = cur.nt;
   if constexpr (GATHER) {
     // the next tile's row indices into the wave's own LDS: lane 8 i + r has that of row r of its i-th piece
@@ -598,6 +596,11 @@ __device__ __forceinline__ void row_tiles(const RowArgs& p, const ShortTiles& ti
     epi = fst + wave * 4096u;
   }
 
+  // the tile after the next: looked up here, where the next one's operands are waited for in any case, used one tile later
+  TileMeta nxt2;
+  auto look_up = [&]() { nxt2 = load_meta(exists(within + 2 * stride) ? within + 2 * stride : within); };
+  if constexpr (MODE != RM_DH) look_up();
+
   // ---- epilogue: 16 rows at a time through the wave's own LDS, 16-byte coalesced rows ----
   // acc[mi][nj][i]: output row = wm + mi*16 + (lane&15); output column within the nj-th
   // 16-column tile = 4*(lane>>4) + i.
@@ -700,6 +703,7 @@ __device__ __forceinline__ void row_tiles(const RowArgs& p, const ShortTiles& ti
         if constexpr (FUSE) sc = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(scale, (mi * 64 + wr * 16 + (el & 15)) * 4u, 0, 0));
       };
       request(0, gq, uq, sq);
+      look_up();
       lds_wait<2 * G + (SHORT ? VM_EPI : 0)>();  // (2 G requests and more are younger than the next tile's operands)
 #pragma unroll
       for (int mi = 0; mi < MB; ++mi) {
@@ -780,6 +784,7 @@ __device__ __forceinline__ void row_tiles(const RowArgs& p, const ShortTiles& ti
       }
     }
   } else {
+    if constexpr (MODE == RM_DH) look_up();
     lds_wait<VM_EPI>();
   }
   if constexpr (MODE == RM_DH && GATHER && NJ == 2) {
