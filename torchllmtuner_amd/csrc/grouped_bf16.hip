@@ -99,6 +99,21 @@ constexpr int R_LDS_BYTES = 2 * STAGE_BYTES + 8 * 4096;
 
 // RM_DLIN: the product of RM_DH (rows . w[e], the weight's contraction axis strided) with a plain epilogue:
 // the input gradient of one grouped linear map
+// n / d for 0 <= n < 2^31 and a divisor that the host knows: a product instead of the thirty instructions of a division, of which a tile's lookups had five.
+// (mul = ceil(2^shift / d) with shift = 31 + ceil(log2 d) is below 2^32 and n * (mul * d - 2^shift) below 2^shift.)
+struct Divisor {
+  uint32_t mul, shift;
+};
+inline Divisor divisor(int64_t d) {
+  uint32_t log = 0;
+  while ((int64_t{1} << log) < d) ++log;
+  return {static_cast<uint32_t>(((uint64_t{1} << (31 + log)) + d - 1) / d), 31 + log};
+}
+__device__ __forceinline__ int quotient(int n, Divisor d) {
+  return static_cast<int>((static_cast<uint64_t>(static_cast<uint32_t>(n)) * d.mul) >> d.shift);
+}
+__device__ __forceinline__ int third(int n) { return static_cast<int>(__umulhi(static_cast<uint32_t>(n), 0x55555556u)); }
+
 enum RowMode { RM_GATEUP = 0, RM_DOWN = 1, RM_DH = 2, RM_DX = 3, RM_DLIN = 4 };
 
 struct RowArgs {
@@ -126,6 +141,7 @@ struct RowArgs {
   const int32_t* num_tiles;
   int D, F;
   int n_tiles;
+  Divisor by_n_tiles, by_steps;  // n_tiles; K steps
   int stream;  // weights of experts with one row tile are read with the non-temporal hint
   int short_tiles;  // tiles of up to 128 rows may take the place of the listed ones
   int El, tile_capacity;
@@ -244,13 +260,15 @@ __device__ __forceinline__ void row_tiles(const RowArgs& p, const ShortTiles& ti
     // scalar loads (constant address space): as vector loads these lookups would share the
     // counter of the operand stream and of the epilogue stores, and waiting for one of them
     // would wait for all of those
-    const int t = pid / p.n_tiles;  // some tile of the expert this work item belongs to
+    const int t = quotient(pid, p.by_n_tiles);  // some tile of the expert this work item belongs to
     TileMeta m;
     [[maybe_unused]] int before = 0;
     m.e = SHORT ? tiles.expert(t, before) : ((const_i32)p.tile_expert)[t];
     const int cnt_e = ((const_i32)p.seg_counts)[m.e], off_e = ((const_i32)p.seg_offsets)[m.e];
-    const int h = even_tile_rows(cnt_e, TBM);
     const int nrt = max((cnt_e + TBM - 1) / TBM, 1);  // row tiles of the expert
+    const bool few = nrt <= 3;
+    // (even_tile_rows, up to three tiles without a division)
+    const int h = nrt == 1 ? TBM : few ? ((nrt == 2 ? (cnt_e + 1) >> 1 : third(cnt_e + 2)) + 15) & ~15 : even_tile_rows(cnt_e, TBM);
     // Within an expert the work items run column-tile-major over groups of three row tiles:
     // the row tiles of one column tile are neighbours, so the weight tile they share -- the
     // larger operand: an expert's weights are several times its rows -- is in L2 when the next
@@ -260,12 +278,16 @@ __device__ __forceinline__ void row_tiles(const RowArgs& p, const ShortTiles& ti
     // column-tile-major throughout fetches the rows of an expert with many row tiles once per
     // column tile.
     constexpr int G = 3;
-    const int t0 = SHORT ? before : t - (((const_i32)p.tile_row0)[t] - off_e) / h;  // the expert's first tile
+    int t0 = before;  // the expert's first tile
+    if constexpr (!SHORT) {
+      const int above = ((const_i32)p.tile_row0)[t] - off_e;
+      t0 = t - (few ? (above >= h) + (above >= 2 * h) : above / h);
+    }
     const int q = pid - t0 * p.n_tiles;
-    const int blk = q / (G * p.n_tiles);
+    const int blk = few ? 0 : quotient(q, p.by_n_tiles) / G;
     const int qb = q - blk * (G * p.n_tiles);
     const int g = min(G, nrt - blk * G);  // row tiles of this group (>= 1)
-    const int nt = qb / g, rt = blk * G + (qb - nt * g);
+    const int nt = g == 1 ? qb : g == 2 ? qb >> 1 : third(qb), rt = blk * G + (qb - nt * g);
     m.row0 = off_e + rt * h;
     m.valid = min(h, cnt_e - rt * h);
     if constexpr (SHORT)
@@ -279,7 +301,11 @@ __device__ __forceinline__ void row_tiles(const RowArgs& p, const ShortTiles& ti
     m.n0 = min(nt * W, Ncols - W);
     m.nt = nt;
     m.stream = p.stream && nrt == 1;
-    m.k_start = TURN ? (5 * m.e + (cnt_e <= 256 && Ncols % W == 0 ? 3 * nt : 0)) % ksteps : 0;
+    m.k_start = 0;
+    if constexpr (TURN) {
+      m.k_start = 5 * m.e + (cnt_e <= 256 && Ncols % W == 0 ? 3 * nt : 0);
+      m.k_start -= quotient(m.k_start, p.by_steps) * ksteps;
+    }
     return m;
   };
 
@@ -849,6 +875,7 @@ struct WgradArgs {
   int El;
   int M, N;
   int m_tiles, n_tiles;
+  Divisor by_tiles, by_n_tiles;  // m_tiles * n_tiles; n_tiles
   int total;  // El * m_tiles * n_tiles
   const uint16_t* a1;  // null, or the first operand of another product with the same b, and its result
   uint16_t* c1;
@@ -904,7 +931,7 @@ __global__ __launch_bounds__(NT, 2) void wgrad_kernel(WgradArgs p) {
   auto place = [&](int w, int& rank) -> int {
     w = (exists(w) ? w : within) >> pair;
     const bool full = w < n_full;
-    const int u = full ? w : p0 + (w - n_full), r = u / per_e;
+    const int u = full ? w : p0 + (w - n_full), r = quotient(u, p.by_tiles);
     rank = full ? r * 8 + ((r & 1) ? 7 - xcd : xcd) : (El & ~7) + r;
     return u - r * per_e;
   };
@@ -918,7 +945,7 @@ __global__ __launch_bounds__(NT, 2) void wgrad_kernel(WgradArgs p) {
   // rows or columns of its neighbour -- the same values -- so every tile is whole
   auto tile_at = [&](int w, int e) -> Tile {
     int rank;
-    const int t = place(w, rank), m = t / p.n_tiles;
+    const int t = place(w, rank), m = quotient(t, p.by_n_tiles);
     return {e, seg_offsets[e], seg_counts[e], min(m * WBM, M - WBM), min((t - m * p.n_tiles) * WBN, N - WBN), (exists(w) ? w : within) & pair};
   };
   // (field by field: a choice between the structures would leave them in memory)
@@ -1298,6 +1325,7 @@ static int launch_row(RowArgs& a, int64_t width, int64_t El, int64_t tile_capaci
                       bool beside = false) {
   constexpr int div = MODE == RM_GATEUP ? 2 : 1;
   a.stream = streamed(El, a.D, a.F);
+  a.by_steps = divisor((MODE == RM_DOWN ? a.F : MODE == RM_DX ? 2 * static_cast<int64_t>(a.F) : a.D) / BK);
   a.El = (int)El; a.tile_capacity = (int)std::min<int64_t>(tile_capacity, INT32_MAX);
   // (what the kernel's waves add up; dRows' weights are read in rows of the output's width, which the two stages wait less for where they lie a multiple of 4 KiB apart)
   a.short_tiles = a.stream && El > 1 && El <= 256 && !(MODE == RM_DX && width % 2048 == 0);
@@ -1310,6 +1338,7 @@ static int launch_row(RowArgs& a, int64_t width, int64_t El, int64_t tile_capaci
       if (int rc = set_lds(row_tiled_kernel<MODE, 2, GATHER, SAVE_GU, TURN>, R_LDS_BYTES)) return rc;
       narrow_configured.done();
     }
+    a.by_n_tiles = divisor(a.n_tiles);
     const unsigned blocks = std::min(round8(tile_capacity * a.n_tiles), resident_blocks());
     hipLaunchKernelGGL((row_tiled_kernel<MODE, 2, GATHER, SAVE_GU, TURN>), dim3(blocks), dim3(NT), R_LDS_BYTES, s, a);
     return check_launch(what);
@@ -1319,6 +1348,7 @@ static int launch_row(RowArgs& a, int64_t width, int64_t El, int64_t tile_capaci
     if (int rc = set_lds(row_tiled_kernel<MODE, 4, GATHER, SAVE_GU, TURN>, R_LDS_BYTES)) return rc;
     configured.done();
   }
+  a.by_n_tiles = divisor(a.n_tiles);
   const unsigned blocks = std::min(round8(tile_capacity * a.n_tiles), beside ? beside_router_blocks(tile_capacity * a.n_tiles) : resident_blocks());
   hipLaunchKernelGGL((row_tiled_kernel<MODE, 4, GATHER, SAVE_GU, TURN>), dim3(blocks), dim3(NT), R_LDS_BYTES, s, a);
   return check_launch(what);
@@ -1535,6 +1565,8 @@ int bf16_grouped_bwd(const void* dy, const void* rows, const int32_t* token_of_r
     w.seg_offsets = seg_offsets; w.seg_counts = seg_counts; w.El = (int)El; w.M = (int)M; w.N = (int)N;
     w.m_tiles = (int)((M + WBM - 1) / WBM); w.n_tiles = (int)((N + WBN - 1) / WBN);
     w.total = (int)(El * w.m_tiles * w.n_tiles);
+    w.by_tiles = divisor(w.m_tiles * w.n_tiles);
+    w.by_n_tiles = divisor(w.n_tiles);
     w.a1 = (const uint16_t*)A1; w.c1 = (uint16_t*)C1;
     const dim3 grid(std::min(round8((int64_t)w.total * (C1 ? 2 : 1)), resident_blocks()));
     if (a_src)
