@@ -68,6 +68,13 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, mi355_bf16x2));
 }
 __device__ __forceinline__ float round_bf16(float f) { return bf16_to_f32(f32_to_bf16(f)); }
+// two values rounded at once, also as pack_bf16x2 has them: three instructions where each alone takes two
+__device__ __forceinline__ uint32_t round_bf16x2(float& a, float& b) {
+  const uint32_t p = pack_bf16x2(a, b);
+  a = __uint_as_float(p << 16);
+  b = __uint_as_float(p & 0xffff0000u);
+  return p;
+}
 
 // Height of the row tiles of a segment of `count` rows: its ceil(count / tile_m) tiles are made
 // equally tall (to a multiple of the 16-row MFMA block) instead of tile_m, tile_m, ..., rest.

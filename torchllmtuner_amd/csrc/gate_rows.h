@@ -20,18 +20,15 @@ namespace {
 
 // 8 consecutive fp32 -> three 16-byte chunks of bf16 pieces (hi, mid, lo)
 __device__ __forceinline__ void split8(const f32x4& a, const f32x4& b, u32x4& hi, u32x4& mid, u32x4& lo) {
-  float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-  float r1[8], r2[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    r1[i] = v[i] - round_bf16(v[i]);
-    r2[i] = r1[i] - round_bf16(r1[i]);
-  }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    hi[i] = pack_bf16x2(v[2 * i], v[2 * i + 1]);
-    mid[i] = pack_bf16x2(r1[2 * i], r1[2 * i + 1]);
-    lo[i] = pack_bf16x2(r2[2 * i], r2[2 * i + 1]);
+    const float v0 = i < 2 ? a[2 * i] : b[2 * i - 4], v1 = i < 2 ? a[2 * i + 1] : b[2 * i - 3];
+    float h0 = v0, h1 = v1;
+    hi[i] = round_bf16x2(h0, h1);
+    const float r0 = v0 - h0, r1 = v1 - h1;
+    h0 = r0, h1 = r1;
+    mid[i] = round_bf16x2(h0, h1);
+    lo[i] = pack_bf16x2(r0 - h0, r1 - h1);
   }
 }
 

@@ -633,8 +633,7 @@ __device__ __forceinline__ void row_tiles(const RowArgs& p, const ShortTiles& ti
   const uint32_t el = opaque(lane);
   constexpr int CH = 4 * NJ;  // 16-byte chunks per row of the wave's sub-tile
   auto key = [](uint32_t m) { return CH == 16 ? m : m >> 1; };
-  auto put = [&](int m0, int nj, float v0, float v1, float v2, float v3) {
-    const u32x2 pk = {pack2(v0, v1), pack2(v2, v3)};
+  auto put = [&](int nj, u32x2 pk) {
     const uint32_t c = nj * 2 + ((el >> 4) >> 1);
     *reinterpret_cast<u32x2*>(reinterpret_cast<char*>(smem) + epi + (el & 15) * (CH * 16) + ((c ^ key((el & 15))) * 16) + ((el >> 4) & 1) * 8) = pk;
   };
@@ -662,19 +661,21 @@ __device__ __forceinline__ void row_tiles(const RowArgs& p, const ShortTiles& ti
       for (int part = SAVE_GU ? 0 : 1; part < 2; ++part) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-          float g[4], u[4], h[4];
+          u32x2 g, u, h;
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            g[r] = round_bf16(acc[mi][j][r]);
-            u[r] = round_bf16(acc[mi][j + NJ][r]);
-            const float s = round_bf16(g[r] * fast_sigmoid(g[r]));
-            h[r] = s * u[r];
+          for (int r = 0; r < 2; ++r) {
+            float g0 = acc[mi][j][2 * r], g1 = acc[mi][j][2 * r + 1], u0 = acc[mi][j + NJ][2 * r], u1 = acc[mi][j + NJ][2 * r + 1];
+            g[r] = round_bf16x2(g0, g1);
+            u[r] = round_bf16x2(u0, u1);
+            float s0 = g0 * fast_sigmoid(g0), s1 = g1 * fast_sigmoid(g1);
+            round_bf16x2(s0, s1);
+            h[r] = pack2(s0 * u0, s1 * u1);
           }
           if (part == 0) {
-            put(mi, j, g[0], g[1], g[2], g[3]);
-            put(mi, NJ + j, u[0], u[1], u[2], u[3]);
+            put(j, g);
+            put(NJ + j, u);
           } else {
-            put(mi, j, h[0], h[1], h[2], h[3]);
+            put(j, h);
           }
         }
         wave_lds_sync();
@@ -699,7 +700,7 @@ __device__ __forceinline__ void row_tiles(const RowArgs& p, const ShortTiles& ti
     auto stage = [&](int mi) {
 #pragma unroll
       for (int nj = 0; nj < NJ2; ++nj)
-        put(mi, nj, acc[mi][nj][0], acc[mi][nj][1], acc[mi][nj][2], acc[mi][nj][3]);
+        put(nj, u32x2{pack2(acc[mi][nj][0], acc[mi][nj][1]), pack2(acc[mi][nj][2], acc[mi][nj][3])});
       wave_lds_sync();
     };
     if constexpr (MODE == RM_DH) {
@@ -749,27 +750,31 @@ __device__ __forceinline__ void row_tiles(const RowArgs& p, const ShortTiles& ti
           u32x4 dg, du, hs;
 #pragma unroll
           for (int w = 0; w < 4; ++w) {
-            float r_dg[2], r_du[2], r_hs[2];
+            float dh[2], uu[2], sl[2], slope[2], ds[2];
 #pragma unroll
             for (int hlf = 0; hlf < 2; ++hlf) {
-              float dh = __uint_as_float(hlf ? (v[w] & 0xffff0000u) : (v[w] << 16));
+              dh[hlf] = __uint_as_float(hlf ? (v[w] & 0xffff0000u) : (v[w] << 16));
               const float g = __uint_as_float(hlf ? (gv[w] & 0xffff0000u) : (gv[w] << 16));
-              const float uu = __uint_as_float(hlf ? (uv[w] & 0xffff0000u) : (uv[w] << 16));
+              uu[hlf] = __uint_as_float(hlf ? (uv[w] & 0xffff0000u) : (uv[w] << 16));
               const float sig = fast_sigmoid(g);
-              const float sl = round_bf16(g * sig);
-              if constexpr (FUSE) {
-                const float hv = round_bf16(sl * uu);  // h as the forward stored it
-                dot += dh * hv;
-                r_hs[hlf] = sc * hv;
-                dh *= sc;
-              }
-              const float ds = round_bf16(dh * uu);
-              r_du[hlf] = dh * sl;
-              r_dg[hlf] = ds * (sig * (1.0f + g * (1.0f - sig)));
+              sl[hlf] = g * sig;
+              slope[hlf] = sig * (1.0f + g * (1.0f - sig));
             }
-            dg[w] = pack2(r_dg[0], r_dg[1]);
-            du[w] = pack2(r_du[0], r_du[1]);
-            if constexpr (FUSE) hs[w] = pack2(r_hs[0], r_hs[1]);
+            round_bf16x2(sl[0], sl[1]);
+            if constexpr (FUSE) {
+              float hv[2] = {sl[0] * uu[0], sl[1] * uu[1]};
+              round_bf16x2(hv[0], hv[1]);  // h as the forward stored it
+#pragma unroll
+              for (int hlf = 0; hlf < 2; ++hlf) {
+                dot += dh[hlf] * hv[hlf];
+                dh[hlf] *= sc;
+              }
+              hs[w] = pack2(sc * hv[0], sc * hv[1]);
+            }
+            ds[0] = dh[0] * uu[0], ds[1] = dh[1] * uu[1];
+            round_bf16x2(ds[0], ds[1]);
+            dg[w] = pack2(ds[0] * slope[0], ds[1] * slope[1]);
+            du[w] = pack2(dh[0] * sl[0], dh[1] * sl[1]);
           }
           const uint32_t o = offset_at(mi, u);
           store16(o0, o, dg);
