@@ -1402,6 +1402,9 @@ static bool few_rows(int64_t El, int64_t rows, int64_t R, int64_t D, int64_t F) 
 // 75 / 76 / 71, 77 / 81 / 74 (80 rows), 79 / 85 / 79; 64 of 640 x 704, 90 rows 80 / 79 / 75; 32 of 1280 x 640 71 / 68 / 72, 73 / 75 / 74, 75 / 77 / 78.  (16 of 2048 x 1024 are
 // just two workgroups a CU and stay with 64: drawn evenly 74 / 78 / 66, 75 / 77 / 68, 76 / 77 / 70, but the products alone by Zipf's law 54 / 55 / 69, 58 / 55 / 71, 84 / 58 / 68.)  Weights from memory
 // arrive as fast through row tiles then (60 of 1728 x 960, 60 rows 150 / 162 / 151; 128 of 2048 x 768 261 / 300 / 267).
+// (These times are of row tiles whose addresses were formed from scratch, top of this file.  With the present ones gate/up and down alone, even loads, passes / row tiles: 64 of
+// 1024 x 512, 45 rows (64-row passes) 48 / 46, 60 rows 50 / 47, 85 rows 55 / 48; 20 rows 42 / 43; 128 of 2048 x 768, 12 rows 191 / 194, by Zipf's law 200 / 219; 32 of 7168 x 2048, 20
+// and 45 rows 444 / 439, 480 / 464.  The lines stand for the uneven loads, which have not been timed again above 12 rows.)
 //   A dense segment beside other products leaves them more CUs in passes of 128, up to 256 rows (one rank's share of 7168 x 2048 with a shared expert of 2048, 100 / 128 / 150 / 256 / 300 /
 // 350 / 400 tokens 378 / 385 / 372, 386 / 398 / 384, 420 / 428 / 420, 426 / 441 / 427, 418 / 432 / 423, 424 / 447 / 431, 438 / 462 / 461; 64 experts of 2048 x 1408 with one of 2816, 100 / 200 / 300 / 400 213 /
 // 209 / 208, 219 / 216 / 219, 224 / 231 / 236, 233 / 237 / 245; 16 of 64 of 4096 x 1024 with one of 1024, 100 / 300 143 / 126 / 138, 149 / 129 / 144).
