@@ -597,7 +597,7 @@ __device__ __forceinline__ void row_tiles(const RowArgs& p, const ShortTiles& ti
     for (int ks = 1; ks < ksteps; ++ks) step(ks, std::false_type{});
     mm(a1, b1, [](int) {});
   };
-  // (the hint is the tile's own, also for what its loop requests of the next tile: a branch at each request cost 2 %)
+  // (the hint is the tile's own, also for what its loop requests of the next tile: a branch at each request cost 2-5 %)
   auto with_blocks = [&](auto stream) {
     if constexpr (SHORT) {
       switch (act) {
