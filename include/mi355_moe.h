@@ -543,6 +543,10 @@ enum {
 };
 int mi355_grouped_fwd_kernels(int dtype, int64_t El, int64_t D, int64_t F, int64_t row_capacity, int64_t rows_expected,
                               int64_t num_tokens, int64_t tile_capacity);
+/* Wide row tiles of bf16 choose tiles of 128 rows by the experts' counts, on the device: the work items that these make in one product (stage 1 gate/up, 2 down, 8 drows, as
+ * in mi355_grouped_swiglu_stage), 0 where it walks the list's tiles.  For tests and measurements; counts (El) is in host memory, num_tiles the list's length. */
+int64_t mi355_grouped_short_tiles(int stage, int64_t El, int64_t D, int64_t F, int64_t row_capacity, int64_t num_tokens,
+                                  int64_t tile_capacity, const int32_t* counts, int64_t num_tiles);
 
 /*
  * Backward of the above (autograd-derived in the reference):

@@ -211,3 +211,23 @@ def test_kernels_of_the_forward_follow_the_rows_that_may_come():
     assert {T: rows_of_a_pass(T, **block) for T in want} == want
     assert rows_of_a_pass(8, **block, align=128) == 16  # (padding is no rows)
     assert lib.mi355_grouped_fwd_kernels(0, 8, 512, 512, 64, 64, 64, 9) == 0 == lib.mi355_grouped_fwd_kernels(1, 8, 360, 512, 64, 64, 64, 9)
+
+
+def test_short_tiles_serve_whole_lists():
+    """Tiles of 128 rows are found from the experts' counts: a list that leaves tiles out keeps its 256-row tiles, or the weights of what it leaves out are read."""
+    from torchllmtuner_amd import _lib
+
+    El, D, F = 128, 1344, 704
+
+    def items(stage, counts, left_out=0, El=El, D=D):
+        listed = sum(-(-c // 256) for c in counts)
+        return _lib.load().mi355_grouped_short_tiles(stage, El, D, F, sum(counts), sum(counts), sum(counts) // 256 + El + 1, (ctypes.c_int32 * El)(*counts),
+                                                     listed - left_out)
+
+    some = [60] * 127 + [700]
+    for stage in (1, 2, 8):
+        assert items(stage, some) == (127 + 6) * 6
+        assert [items(stage, some, left_out) for left_out in (1, 64, 130)] == [0, 0, 0]
+        assert items(stage, [150] * 128) == 0  # two tiles each
+        assert items(stage, [60] * 8, El=8) == 0  # their weights stay in the memory-side cache
+    assert items(2, some, D=2048) and not items(8, some, D=2048)

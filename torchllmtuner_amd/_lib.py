@@ -56,6 +56,7 @@ SIGNATURES = {
     "mi355_grouped_swiglu_fwd_beside": (I, [P, P, L, P, P, P, I, P, P, P, P, P, L, P, P, P, P, L, L, L, L, P]),
     "mi355_grouped_swiglu_fwd_expecting": (I, [P, P, L, P, P, P, I, P, P, P, P, P, L, P, P, P, P, L, L, L, L, L, P]),
     "mi355_grouped_fwd_kernels": (I, [I, L, L, L, L, L, L, L]),
+    "mi355_grouped_short_tiles": (L, [I, L, L, L, L, L, L, P, L]),
     "mi355_grouped_swiglu_stage": (
         I,
         [I, P, P, P, L, P, P, P, P, P, P, P, P, P, P, P, P, L, P, P, P, P, P, P, L, L, L, L, P],

@@ -23,6 +23,8 @@ int bf16_grouped_fwd(const void* rows, const int32_t* token_of_row, int64_t num_
                      int64_t tile_capacity, void* gate, void* up, void* h, void* y, int64_t El, int64_t D,
                      int64_t F, int64_t row_capacity, int64_t rows_expected, int stages, hipStream_t s);
 int bf16_fwd_kernels(int64_t El, int64_t D, int64_t F, int64_t row_capacity, int64_t rows_expected, int64_t tokens, int64_t tile_capacity);
+int64_t bf16_short_tiles(int stage, int64_t El, int64_t D, int64_t F, int64_t row_capacity, int64_t tokens, int64_t tile_capacity,
+                         const int32_t* counts, int64_t listed);
 int bf16_fused_dot_slots(int64_t F);
 int bf16_grouped_linear_dx(const void* dy, const void* w, const int32_t* seg_offsets, const int32_t* seg_counts,
                            const int32_t* tile_expert, const int32_t* tile_row0, const int32_t* num_tiles,
@@ -259,6 +261,12 @@ extern "C" int mi355_grouped_fwd_kernels(int dtype, int64_t El, int64_t D, int64
   return dtype == MI355_BF16 && El >= 1 && bf16_fast_path_ok(D, F)
              ? bf16_fwd_kernels(El, D, F, row_capacity, rows_expected, num_tokens, tile_capacity)
              : 0;
+}
+
+extern "C" int64_t mi355_grouped_short_tiles(int stage, int64_t El, int64_t D, int64_t F, int64_t row_capacity, int64_t num_tokens,
+                                             int64_t tile_capacity, const int32_t* counts, int64_t num_tiles) {
+  if (!counts || El < 1 || tile_capacity < 1 || !bf16_fast_path_ok(D, F) || (stage != 1 && stage != 2 && stage != 8)) return 0;
+  return bf16_short_tiles(stage, El, D, F, row_capacity, num_tokens, tile_capacity, counts, num_tiles);
 }
 
 extern "C" int mi355_grouped_swiglu_bwd(const void* dy, const void* rows,

@@ -144,27 +144,34 @@ struct RowArgs {
   Divisor by_n_tiles, by_steps;  // n_tiles; K steps
   int stream;  // weights of experts with one row tile are read with the non-temporal hint
   int short_tiles;  // tiles of up to 128 rows may take the place of the listed ones
-  int El, tile_capacity;
+  int El;
 };
+
+// Rows of a short tile, and whether short tiles (`total`, `n_tiles` of them across) take the place of the 256-row ones (`whole` of all experts' rows, `listed` in the list) on
+// `blocks` workgroups.  Not where the list leaves tiles out, which the counts know nothing of: short tiles searched the list for their rows and read the weights of all experts.
+// Half and a quarter of 128 experts of 2048 x 768 listed, 60 rows each, us, short tiles / the list's: gate/up 141 / 84, 138 / 42, down 80 / 45, 78 / 24; of 32 of 7168 x 2048 dRows
+// 322 / 165, 323 / 76.
+constexpr int kShortTile = 128;
+__host__ __device__ inline bool short_tiles_serve(int total, int whole, int listed, int n_tiles, int blocks) {
+  auto rounds = [&](int n) { return (n * n_tiles + blocks - 1) / blocks; };
+  return listed == whole && total * 4 <= whole * 5 && rounds(total) <= rounds(whole);
+}
 
 // The tiles of up to 128 rows that the experts' rows make (at most 256 experts), found by every wave from the counts.
 struct ShortTiles {
   int to[4];  // lane l, b: tiles of the experts up to and with 64 b + l
-  int total = 0, listed = 0, unlisted = 0;  // tiles; those of 256 rows, and how many of them the list leaves out
-  TileList list;
+  int total = 0, whole = 0;  // tiles; those of 256 rows
   __device__ __forceinline__ void find(const RowArgs& p) {
     const int lane = threadIdx.x & 63;
-    list = {p.tile_expert, p.tile_row0, p.num_tiles, p.tile_capacity};
     int count[4];
 #pragma unroll
     for (int b = 0; b < 4; ++b) count[b] = 64 * b + lane < p.El ? p.seg_counts[64 * b + lane] : 0;
 #pragma unroll
     for (int b = 0; b < 4; ++b) {
-      to[b] = total + wave_scan((count[b] + 127) / 128);
+      to[b] = total + wave_scan((count[b] + kShortTile - 1) / kShortTile);
       total = __builtin_amdgcn_readlane(to[b], 63);
-      listed += __builtin_amdgcn_readlane(wave_scan(listed_tiles(count[b])), 63);
+      whole += __builtin_amdgcn_readlane(wave_scan(listed_tiles(count[b])), 63);
     }
-    unlisted = listed - list.size();
   }
   // the expert of tile t and the tiles of those before it
   __device__ __forceinline__ int expert(int t, int& before) const {
@@ -290,11 +297,6 @@ __device__ __forceinline__ void row_tiles(const RowArgs& p, const ShortTiles& ti
     const int nt = g == 1 ? qb : g == 2 ? qb >> 1 : third(qb), rt = blk * G + (qb - nt * g);
     m.row0 = off_e + rt * h;
     m.valid = min(h, cnt_e - rt * h);
-    if constexpr (SHORT)
-      if (tiles.unlisted != 0 && !listed_rows(tiles.list, m.e, off_e, cnt_e, m.row0, m.valid)) {
-        m.row0 = off_e;
-        m.valid = 0;
-      }
     // a last tile that would overhang starts early instead and recomputes a few columns
     // of its neighbour (same values), so no column is ever clamped
     constexpr int W = (MODE == RM_GATEUP ? BNT / 2 : BNT);
@@ -854,8 +856,7 @@ __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
   if constexpr (NJ == 4 && (MODE == RM_GATEUP || MODE == RM_DOWN || MODE == RM_DX)) {
     if (p.short_tiles) {
       tiles.find(p);
-      auto rounds = [&](int n) { return (n * p.n_tiles + static_cast<int>(gridDim.x) - 1) / static_cast<int>(gridDim.x); };
-      if (tiles.total * 4 <= tiles.listed * 5 && rounds(tiles.total) <= rounds(tiles.listed)) {
+      if (short_tiles_serve(tiles.total, tiles.whole, *(const_i32)p.num_tiles, p.n_tiles, static_cast<int>(gridDim.x))) {
         row_tiles<MODE, NJ, GATHER, SAVE_GU, TURN, 2>(p, tiles);
         return;
       }
@@ -1310,6 +1311,12 @@ static bool narrow(int mode, int64_t El, int64_t wide_n, int64_t narrow_n, int64
 // With two row tiles or more an expert, which share the weights in L2, the hint costs 2-8 % (8192 tokens of the first block, 16384 of a skewed router).
 static bool streamed(int64_t El, int64_t D, int64_t F) { return El * D * F * 6 > (int64_t{320} << 20); }
 
+// Whether a row product on wide tiles may choose short ones by the counts (of which the kernel's waves add up 256): where the weights come from memory.  dRows' weights are read
+// in rows of the output's width, which the two stages wait less for where they lie a multiple of 4 KiB apart.
+static bool short_tiles_may(int mode, int64_t El, int64_t D, int64_t F) {
+  return streamed(El, D, F) && El > 1 && El <= 256 && !(mode == RM_DX && D % 2048 == 0);
+}
+
 // Workgroups of a gate/up product that runs beside the launches of a router (a shared expert's): a workgroup takes a CU whole until its list of tiles
 // ends, so a product that holds every CU makes each of them wait (rank and plan, 12 and 11 us alone, took 195 and 63), and the routed experts, often a
 // read of their weights, start when it has ended instead of running beside it.  An eighth of the CUs is enough to prevent that.  Block forward, us, all CUs / seven eighths /
@@ -1331,9 +1338,8 @@ static int launch_row(RowArgs& a, int64_t width, int64_t El, int64_t tile_capaci
   constexpr int div = MODE == RM_GATEUP ? 2 : 1;
   a.stream = streamed(El, a.D, a.F);
   a.by_steps = divisor((MODE == RM_DOWN ? a.F : MODE == RM_DX ? 2 * static_cast<int64_t>(a.F) : a.D) / BK);
-  a.El = (int)El; a.tile_capacity = (int)std::min<int64_t>(tile_capacity, INT32_MAX);
-  // (what the kernel's waves add up; dRows' weights are read in rows of the output's width, which the two stages wait less for where they lie a multiple of 4 KiB apart)
-  a.short_tiles = a.stream && El > 1 && El <= 256 && !(MODE == RM_DX && width % 2048 == 0);
+  a.El = (int)El;
+  a.short_tiles = short_tiles_may(MODE, El, a.D, a.F);
   a.n_tiles = (int)((width + 256 / div - 1) / (256 / div));
   const int64_t narrow_n = (width + 128 / div - 1) / (128 / div);
   if (narrow(MODE, El, a.n_tiles, narrow_n, tile_capacity)) {
@@ -1444,6 +1450,23 @@ int bf16_fwd_kernels(int64_t El, int64_t D, int64_t F, int64_t row_capacity, int
          (tiles && narrow(RM_DOWN, El, across(D, 256), across(D, 128), tile_capacity) ? MI355_FWD_NARROW_DOWN : 0) |
          (turn && (tokens > 0 || !tiles) && turned(El, row_capacity, D) ? MI355_FWD_TURNED_GATEUP : 0) |
          (turn && turned(El, row_capacity, F) ? MI355_FWD_TURNED_DOWN : 0);
+}
+
+// Work items on short tiles that a product of these counts makes (0: it walks the list's tiles); stage: one of gate/up, down, dRows.
+int64_t bf16_short_tiles(int stage, int64_t El, int64_t D, int64_t F, int64_t row_capacity, int64_t tokens, int64_t tile_capacity,
+                         const int32_t* counts, int64_t listed) {
+  const int mode = stage == STAGE_GATEUP ? RM_GATEUP : stage == STAGE_DOWN ? RM_DOWN : RM_DX;
+  const int64_t width = mode == RM_GATEUP ? F : D, tile = mode == RM_GATEUP ? 128 : 256, across = (width + tile - 1) / tile;
+  if (!short_tiles_may(mode, El, D, F) || narrow(mode, El, across, (2 * width + tile - 1) / tile, tile_capacity) ||
+      (mode != RM_DX && pass_rows(El, D, F, row_capacity, row_capacity, tokens, false) != 256))
+    return 0;
+  int total = 0, whole = 0;
+  for (int64_t e = 0; e < El; ++e) {
+    total += (counts[e] + kShortTile - 1) / kShortTile;
+    whole += (counts[e] + kListTile - 1) / kListTile;
+  }
+  const unsigned blocks = std::min(round8(tile_capacity * across), resident_blocks());
+  return short_tiles_serve(total, whole, (int)listed, (int)across, (int)blocks) ? total * across : 0;
 }
 
 int bf16_grouped_fwd(const void* rows, const int32_t* token_of_row, int64_t num_tokens, const void* w1,
