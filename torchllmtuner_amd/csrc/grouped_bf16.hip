@@ -97,8 +97,6 @@ constexpr uint32_t A_BYTES = 32768, STAGE_BYTES = 65536;
 constexpr uint32_t kNoRow = 0xffffff80u;  // no row of a matrix of whole 128-byte lines below 4 GiB begins there
 constexpr int R_LDS_BYTES = 2 * STAGE_BYTES + 8 * 4096;
 
-// RM_DLIN: the product of RM_DH (rows . w[e], the weight's contraction axis strided) with a plain epilogue:
-// the input gradient of one grouped linear map
 // n / d for 0 <= n < 2^31 and a divisor that the host knows: a product instead of the thirty instructions of a division, of which a tile's lookups had five.
 // (mul = ceil(2^shift / d) with shift = 31 + ceil(log2 d) is below 2^32 and n * (mul * d - 2^shift) below 2^shift.)
 struct Divisor {
@@ -114,6 +112,8 @@ __device__ __forceinline__ int quotient(int n, Divisor d) {
 }
 __device__ __forceinline__ int third(int n) { return static_cast<int>(__umulhi(static_cast<uint32_t>(n), 0x55555556u)); }
 
+// RM_DLIN: the product of RM_DH (rows . w[e], the weight's contraction axis strided) with a plain epilogue:
+// the input gradient of one grouped linear map
 enum RowMode { RM_GATEUP = 0, RM_DOWN = 1, RM_DH = 2, RM_DX = 3, RM_DLIN = 4 };
 
 struct RowArgs {
@@ -237,6 +237,7 @@ __device__ __forceinline__ void row_tiles(const RowArgs& p, const ShortTiles& ti
   constexpr int VM = NBX ? NA + NB : NA;   // requests younger than those a barrier of the loop waits for
   constexpr int VM_EPI = SHORT ? NA + NB : NBX ? NBY : 0;    // ... than those that the next tile's first K step needs
   static_assert(!GATHER || MODE == RM_GATEUP || MODE == RM_DH, "only gate/up and dH gather their rows");
+  static_assert(!SHORT || MODE != RM_DH, "dH's epilogue counts the requests of two stages");
   static_assert(!TURN || !B_KS, "only contractions that are contiguous in memory are turned");
   static_assert(!(GATHER && MODE == RM_DH) || NJ == 4 || NJ == 2, "the fused dH epilogue reduces over 16 lanes per row, or 8 and a second wave");
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
@@ -733,14 +734,14 @@ __device__ __forceinline__ void row_tiles(const RowArgs& p, const ShortTiles& ti
       };
       request(0, gq, uq, sq);
       look_up();
-      lds_wait<2 * G + (SHORT ? VM_EPI : 0)>();  // (2 G requests and more are younger than the next tile's operands)
+      lds_wait<2 * G>();  // (2 G requests and more are younger than the next tile's operands)
 #pragma unroll
-      for (int mi = 0; mi < MB; ++mi) {
+      for (int mi = 0; mi < 4; ++mi) {
         if (mi >= act) break;
         u32x4 gn[G], un[G];
         float sn;
         // (the last block again past it: every load is unconditional)
-        if (mi < MB - 1) request(min(mi + 1, act - 1), gn, un, sn);
+        if (mi < 3) request(min(mi + 1, act - 1), gn, un, sn);
         stage(mi);
 #pragma unroll
         for (int u = 0; u < G; ++u) {
@@ -795,7 +796,7 @@ __device__ __forceinline__ void row_tiles(const RowArgs& p, const ShortTiles& ti
           }
         }
         wave_lds_sync();
-        if (mi < MB - 1) {
+        if (mi < 3) {
 #pragma unroll
           for (int u = 0; u < G; ++u) {
             gq[u] = gn[u];
