@@ -56,9 +56,11 @@
 // last (about 35 vector instructions a store, 24 stores a tile of gate/up, 3 us of its 8 us epilogue); now the tile's rows are a buffer that ends behind the
 // last of them and an address is one addition.  A request of weights used to branch on whether it carries the non-temporal hint; now the loop exists with
 // and without it (a K step's 104 scalar and 41 vector instructions are 62 and 4).  Rows past the last of a tile were read as copies of it; now they are zeros that nothing is read
-// for.  The three, us, before / with them: 128 experts of 2048 x 768, 512 rows each by Poisson draws gate/up 475 / 435, dRows 412 / 391, down 229 / 221; 16384
+// for, but of dH.  The three, us, before / with them: 128 experts of 2048 x 768, 512 rows each by Poisson draws gate/up 475 / 435, dRows 412 / 391, down 229 / 221; 16384
 // tokens of a skewed router 801 / 765, 772 / 731, 418 / 407; 64 of 1024 x 512, 281 rows 66 / 63, 56 / 53; one dense segment of 4096 rows of 7168 x 2048 178 / 172, 203 / 189, 99 / 97, dH
-// 114 / 105.
+// (the first two) 114 / 105.  Most of it is the first's: the present code with a branch at each request instead of the second has gate/up, dRows and dH of the 512 rows in 415 / 393 / 299
+// instead of 404 / 383 / 299, of 700 dense rows 130 / 79 / 85 instead of 121 / 75 / 79, of 520 rows of the 64 experts 86 / 75 / 91 instead of 85 / 74 / 91; with copies instead of the third 405 / 385,
+// 121 / 76, 85 / 73 (369 instead of 364 in gate/up of 200 rows of 32 of 7168 x 2048).
 //
 // MFMA of both: v_mfma_f32_16x16x32_bf16.  Per lane 8 bf16 of each operand (row lane%16,
 // k = 8*(lane/16)..+7), 4 fp32 of the result (column lane%16, rows 4*(lane/16) + i).
@@ -336,6 +338,7 @@ __device__ __forceinline__ void row_tiles(const RowArgs& p, const ShortTiles& ti
     for (int i = 0; i < NA; ++i) {
       const int src = GATHER ? min(max(asrc[i], 0), p.a_rows - 1) : asrc[i];
       voffA[i] = (static_cast<uint32_t>(src) * static_cast<uint32_t>(lda) + static_cast<uint32_t>(kc_chunk * 8)) * 2u;
+      // (dH's stay copies: as zeros 79.3 us instead of 78.7 for 700 dense rows of 7168 x 2048, 34.1 instead of 33.7 for 2000 of 2048 x 2048, nothing between 60 and 520 rows an expert)
       if (MODE != RM_DH && kc_row + 64 * i >= m.valid) voffA[i] = kNoRow;
     }
     // KC: the tile's first weight row is n0; KS: its first column is n0
@@ -345,7 +348,7 @@ __device__ __forceinline__ void row_tiles(const RowArgs& p, const ShortTiles& ti
     k_start = m.k_start;
     fk = 0;
   };
-  // rows past the tile's last: past the end of the buffer that a request names, which makes them zeros and reads nothing
+  // rows past the tile's last: past the end of the buffer that a request names, which makes them zeros and reads nothing; dH: the last row again
   auto tile_row = [&](const TileMeta& m, int i) { return max(min(kc_row + 64 * i, m.valid - 1), 0); };
   auto kofs = [&]() {
     if constexpr (!TURN) return fk * BK;
@@ -600,7 +603,7 @@ __device__ __forceinline__ void row_tiles(const RowArgs& p, const ShortTiles& ti
     for (int ks = 1; ks < ksteps; ++ks) step(ks, std::false_type{});
     mm(a1, b1, [](int) {});
   };
-  // (the hint is the tile's own, also for what its loop requests of the next tile: a branch at each request cost 2-5 %)
+  // (the hint is the tile's own, also for what its loop requests of the next tile; a branch at each request instead: top of this file)
   auto with_blocks = [&](auto stream) {
     if constexpr (SHORT) {
       switch (act) {
@@ -851,6 +854,9 @@ __device__ __forceinline__ void row_tiles(const RowArgs& p, const ShortTiles& ti
 // 155 / 171); not where the weights stay in the memory-side cache (64 experts of 1024 x 512, 100 rows: dRows 31 / 37); not dH, whose epilogue's loads
 // wait for what has been requested before them: 160 / 163; not dRows where weight rows lie a multiple of 4 KiB apart (20 rows of the first 130 / 134, 62 rows 146 / 146).  A forward
 // of 1000 tokens of the first, eight each, 257 / 252.
+//   Uneven loads: of 430 products (128 of 2048 x 768 and 1344 x 704, 64 of 2048 x 1408, 60 of 1728 x 960 and 1920 x 704, 32 of 7168 x 2048; 25 to 110 rows an expert drawn evenly, by Zipf's
+// laws of 0.3 to 1.2, all from a half, a quarter or 16 of the experts, and 30 or 60 rows each beside one to six experts of 300 to 2000) that choose these, three take 1 % to 1.5 % longer than
+// on 256-row tiles (32 of 7168 x 2048, 60 rows beside one of 2000, gate/up 396 / 402), the median 4.5 % less and the best 15 %.
 template <int MODE, int NJ, bool GATHER, bool SAVE_GU = true, bool TURN = false>
 __global__ __launch_bounds__(NT, 2) void row_tiled_kernel(RowArgs p) {
   ShortTiles tiles;
